@@ -392,3 +392,29 @@ def test_residual_projection_with_norm_and_quantizer(ctx, oracle, dtype, m, n, k
         w2 = ctx.upload_weight(oracle.synth_weight(dtype, 48, 256, seed=1), dtype, 48, 256)
         ctx.gemm_preq_residual_rmsnorm_quantize(w2, d_s, d_q, 1, d_nw, 48, d_nw, eps, d_q, d_s)
     w.free(), w2.free(), d_q.free(), d_s.free(), d_nw.free()
+
+
+# ragged in rows and tokens, one per tile of the cost rule (256 x 128, 128 x 128, 128 x 64 rows x tokens; the last on one workgroup per CU)
+@pytest.mark.parametrize("m,n,k", [(8150, 2021, 2048), (3001, 1500, 256), (2050, 1990, 1024), (1000, 1999, 384)])
+def test_prompt_tiles_against_the_gemv_route(ctx, oracle, m, n, k):
+    """Every element of a prompt-sized projection on the tile its size selects: both layouts and the accumulate flag bit-equal to each
+    other, and within the f32 bar of the multi-token GEMV."""
+    with Problem(ctx, oracle, W.Q4_0, m, k, n, seed=m + n + k) as p:
+        d_y = p.alloc((n + 4) * (m + 4) * 4)
+        old = oracle.fill_normal(3, 1.0, (n + 4) * (m + 4))
+        out = {}
+        for layout, stride in ((W.LAYOUT_TOKEN_MAJOR, m + 4), (W.LAYOUT_ROW_MAJOR, n + 4)):
+            for acc in (False, True):
+                d_y.upload(old)
+                ctx.gemm_preq(p.w, p.d_s, p.d_q, n, d_y, y_stride=stride, layout=layout, accumulate=acc)
+                out[layout, acc] = fetch_gemm(d_y, m, n, stride, layout).copy()
+            was = old[:(n if layout == W.LAYOUT_TOKEN_MAJOR else m) * stride].reshape(-1, stride)
+            was = was[:, :m].T if layout == W.LAYOUT_TOKEN_MAJOR else was[:, :n]
+            assert np.array_equal(out[layout, True], was + out[layout, False])
+        assert np.array_equal(out[W.LAYOUT_TOKEN_MAJOR, False], out[W.LAYOUT_ROW_MAJOR, False])
+        ctx.set_gemm_min_n(n + 1)
+        try:
+            ctx.gemm_preq(p.w, p.d_s, p.d_q, n, d_y, y_stride=m, layout=W.LAYOUT_TOKEN_MAJOR)
+        finally:
+            ctx.set_gemm_min_n(0)
+        assert rel_l2(out[W.LAYOUT_TOKEN_MAJOR, False], fetch_gemm(d_y, m, n, m, W.LAYOUT_TOKEN_MAJOR)) < 1e-6

@@ -532,3 +532,31 @@ def test_gate_up_gemm_with_gate_and_quantizer_in_its_epilogue(ctx, ops, oracle, 
     for b in (d_xq, d_xs, d_oq, d_os, d_g, d_u):
         b.free()
     d_wg.free(), d_wu.free()
+
+
+@pytest.mark.parametrize("dtype,m,k,n", [(W.Q8_0, 4064, 2048, 2040), (W.Q4_0, 4576, 1024, 801), (W.Q4_0, 2080, 128, 1111)])
+def test_gated_prompt_tiles_equal_the_separate_launches(ctx, ops, oracle, dtype, m, k, n):
+    """The gate in the epilogue on each of the tiles the cost rule can take (256 x 128, 128 x 128, 128 x 64), ragged, with gate values
+    far outside the exponential's short branch: quants and scales bit-identical to projections + gate kernel."""
+    ws = [ctx.upload_weight(oracle.synth_weight(dtype, m, k, seed=41 + i), dtype, m, k) for i in range(2)]
+    x = oracle.fill_normal(6, 1.0, n * k).reshape(n, k)
+    x[::7] *= 400.0
+    xs, xq = oracle.quantize_q8_0_batch(x.ravel(), n, k)
+    d_xq, d_xs = ctx.to_device(xq), ctx.to_device(xs)
+    got = []
+    for fused in (True, False):
+        d_oq, d_os = ctx.to_device(np.full(n * m, 99, np.int8)), ctx.alloc(n * (m // 32) * 4)
+        if fused:
+            ops.encode_ffn_gate_up_silu_quantize(*ws, d_xs, d_xq, n, d_oq, d_os)
+        else:
+            d_g, d_u = ctx.alloc(n * m * 4), ctx.alloc(n * m * 4)
+            ctx.gemm_preq_multi(ws, d_xs, d_xq, n, [d_g, d_u], m)
+            ops.silu_mul_quantize(d_g, d_u, n, m, d_oq, d_os)
+            d_g.free(), d_u.free()
+        got.append((d_oq.download(np.int8, n * m), bits(d_os.download(np.float32, n * (m // 32)))))
+        d_oq.free(), d_os.free()
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+    for b in (d_xq, d_xs):
+        b.free()
+    for w in ws:
+        w.free()

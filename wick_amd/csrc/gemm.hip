@@ -7,18 +7,15 @@
 // blocks: every MFMA covers exactly one block (K = 32) and its i32 result is scaled
 // into f32 accumulators on the vector ALU.
 //
-// Workgroup = 512 threads = 8 waves, tile = 128 weight rows x 128 tokens, each wave
-// owns 64 rows x 32 tokens.  Two block loops exist for that wave tile:
-//   * gemm_mfma32_kernel (plain projections, the default): 2 x v_mfma_i32_32x32x32_i8 per block, one 16-register
-//     result buffer, 16-register bias tuple, 16 token scales and 2 row-scale pairs per block -- 125 VGPRs
-//     (gemm_narrow32_kernel is the same loop with one MFMA per block on the 128 x 64 tile);
-//   * gemm_mfma_kernel (the gated feed-forward launch, and plain projections on request): 4 x 2 tiles of
-//     v_mfma_i32_16x16x32_i8, four 4-register result buffers, 4-register bias -- 109 VGPRs.
-// Both stay under 128 VGPRs so that FOUR waves share a SIMD, which matters more than anything else here: a wave can
-// issue a vector-ALU instruction only every ~4.7 cycles while a SIMD retires one every ~2.2, and the kernel is bound by
-// the two scaling FMAs per result plus the matrix instructions, which a SIMD does not overlap with them.  The small
-// shape runs the matrix unit at a third of the large one's rate (1.7 vs 4.9 POP/s measured), which is what the
-// 32x32x32 loop recovers part of (3 - 8 % of a launch).
+// Two families of block loops:
+//   * gemm_tile_kernel, v_mfma_i32_32x32x32_i8: every launch of more than 48 tokens, on one of three tiles (see T32 and TileL / M / S);
+//   * gemm_narrow_kernel, v_mfma_i32_16x16x32_i8, 128 rows x 64 tokens: launches of up to 48 tokens, which skip the 16-token
+//     columns they do not have; gemm_mfma_kernel, the same shape on 128 x 128, on request (wick_rocm_set_gemm_mfma_shape).
+// The kernels are bound by the two scaling FMAs per result plus the matrix instructions, which a SIMD overlaps only in part, and by
+// feeding both from LDS.  A wave issues a vector-ALU instruction only every ~4.7 cycles while a SIMD retires one every ~2.3, so two
+// waves per SIMD at least, four where a wave has one result buffer.
+//
+// The 16x16 kernels below are described here; gemm_tile_kernel shares their data layouts and says the rest at its place.
 // One stage = 4 blocks (128 elements of K).  Both operands are copied global -> LDS directly
 // (global_load_lds_dwordx4: asynchronous, no registers, 1 KB per wave instruction):
 //   * weights from the GEMM's own copy of the matrix, made from the raw GGUF blocks when the
@@ -230,7 +227,7 @@ __device__ __forceinline__ void dma_stage(StagePtrs<NTOK>& p, StageT<NTOK>& s) {
     p.wc += 2 * kSlab;
 }
 
-template <int NTOK, bool GATED = false>
+template <int NTOK>
 __device__ __forceinline__ void init_stage_ptrs(const GemmArgs& a, uint32_t row_tile, uint32_t tok0, uint32_t kb0, StagePtrs<NTOK>& p) {
     constexpr int PER_WAVE = NTOK / 8 / kLoaderWaves;
     const uint32_t t = threadIdx.x, lane = t & 63u;
@@ -246,11 +243,8 @@ __device__ __forceinline__ void init_stage_ptrs(const GemmArgs& a, uint32_t row_
     const uint32_t granules = (a.m + GR - 1) / GR;
     {
         const uint32_t g = wave;
-        // the tile's granule g: rows 32 g .. of a plain tile; of a gated tile (64 output rows) gate, up, gate, up of its two
-        uint32_t granule = GATED ? 2u * row_tile + (g >> 1) : (BM / GR) * row_tile + g;
-        const uint8_t* w = GATED && (g & 1u) ? a.w_up : a.w;
-        granule = min(granule, granules - 1u);  // past the end of the matrix: any rows, their results are not stored
-        p.wc = w + (((size_t)(granule >> 1) * stages + kb0 / KB) * 2 + (granule & 1u)) * kSlab + 16u * lane;
+        const uint32_t granule = min((BM / GR) * row_tile + g, granules - 1u);  // past the end of the matrix: any rows, their results are not stored
+        p.wc = a.w + (((size_t)(granule >> 1) * stages + kb0 / KB) * 2 + (granule & 1u)) * kSlab + 16u * lane;
     }
     p.dx = nullptr;
     if (t < NTOK && a.xs) {  // xs is null only for the parity hook, which never scales
@@ -423,6 +417,19 @@ __device__ __forceinline__ void tile_of_block(uint32_t bid, uint32_t row_tiles, 
 template <int NTT, int NRT, int TSTEP, int RSTEP, bool ROW_MAJOR, bool CHECK, bool ACC, typename F>
 __device__ __forceinline__ void store_results(float* __restrict__ base, size_t stride, uint32_t row, uint32_t tok, uint32_t m, uint32_t n,
                                               F&& value) {
+    // accumulating inside the matrix: all old values on their way before the first is used, not one round trip per value
+    constexpr bool AHEAD = ACC && !CHECK;
+    float old[AHEAD ? NTT * NRT * 4 : 1];
+    if constexpr (AHEAD) {
+#pragma unroll
+        for (int tt = 0; tt < NTT; tt++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int rt = 0; rt < NRT; rt++)
+                    old[(tt * 4 + r) * NRT + rt] = ROW_MAJOR ? base[(size_t)(row + RSTEP * rt) * stride + tok + TSTEP * tt + r]
+                                                             : base[(size_t)(tok + TSTEP * tt + r) * stride + row + RSTEP * rt];
+    }
     if constexpr (ROW_MAJOR) {
 #pragma unroll
         for (int rt = 0; rt < NRT; rt++) {
@@ -433,7 +440,7 @@ __device__ __forceinline__ void store_results(float* __restrict__ base, size_t s
                 for (int r = 0; r < 4; r++) {
                     if (CHECK && !(row + RSTEP * rt < m && tok + TSTEP * tt + r < n)) continue;
                     const float v = value(tt, rt, r);
-                    q[TSTEP * tt + r] = ACC ? q[TSTEP * tt + r] + v : v;
+                    q[TSTEP * tt + r] = AHEAD ? old[(tt * 4 + r) * NRT + rt] + v : (ACC ? q[TSTEP * tt + r] + v : v);
                 }
         }
     } else {
@@ -446,7 +453,7 @@ __device__ __forceinline__ void store_results(float* __restrict__ base, size_t s
                 for (int rt = 0; rt < NRT; rt++) {
                     if (CHECK && !(row + RSTEP * rt < m && tok + TSTEP * tt + r < n)) continue;
                     const float v = value(tt, rt, r);
-                    q[RSTEP * rt] = ACC ? q[RSTEP * rt] + v : v;
+                    q[RSTEP * rt] = AHEAD ? old[(tt * 4 + r) * NRT + rt] + v : (ACC ? q[RSTEP * rt] + v : v);
                 }
             }
     }
@@ -463,38 +470,30 @@ __device__ __forceinline__ void store_wave_tile(const GemmArgs& a, uint32_t kspl
         if (inside) store_results<NTT, NRT, TSTEP, RSTEP, false, false, false>(base, a.m, row, tok, a.m, a.n, value);
         else store_results<NTT, NRT, TSTEP, RSTEP, false, true, false>(base, a.m, row, tok, a.m, a.n, value);
     } else if (a.y_row_major) {
-        if (a.accumulate) store_results<NTT, NRT, TSTEP, RSTEP, true, true, true>(a.y, a.y_stride, row, tok, a.m, a.n, value);
+        if (a.accumulate && inside) store_results<NTT, NRT, TSTEP, RSTEP, true, false, true>(a.y, a.y_stride, row, tok, a.m, a.n, value);
+        else if (a.accumulate) store_results<NTT, NRT, TSTEP, RSTEP, true, true, true>(a.y, a.y_stride, row, tok, a.m, a.n, value);
         else if (inside) store_results<NTT, NRT, TSTEP, RSTEP, true, false, false>(a.y, a.y_stride, row, tok, a.m, a.n, value);
         else store_results<NTT, NRT, TSTEP, RSTEP, true, true, false>(a.y, a.y_stride, row, tok, a.m, a.n, value);
     } else {
-        if (a.accumulate) store_results<NTT, NRT, TSTEP, RSTEP, false, true, true>(a.y, a.y_stride, row, tok, a.m, a.n, value);
+        if (a.accumulate && inside) store_results<NTT, NRT, TSTEP, RSTEP, false, false, true>(a.y, a.y_stride, row, tok, a.m, a.n, value);
+        else if (a.accumulate) store_results<NTT, NRT, TSTEP, RSTEP, false, true, true>(a.y, a.y_stride, row, tok, a.m, a.n, value);
         else if (inside) store_results<NTT, NRT, TSTEP, RSTEP, false, false, false>(a.y, a.y_stride, row, tok, a.m, a.n, value);
         else store_results<NTT, NRT, TSTEP, RSTEP, false, true, false>(a.y, a.y_stride, row, tok, a.m, a.n, value);
     }
 }
 
-// Maximum over the 16 lanes of a DPP row (lanes that share lane / 16); every lane of the row ends with it.
-__device__ __forceinline__ float row_max16(float v) {
-    v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, false)));   // quad_perm [1,0,3,2]
-    v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xf, 0xf, false)));   // quad_perm [2,3,0,1]
-    v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xf, 0xf, false)));  // row_half_mirror
-    v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x140, 0xf, 0xf, false)));  // row_mirror
-    return v;
-}
-
-template <int TYPE, bool DUMP, bool GATED = false>
+template <int TYPE, bool DUMP>
 __global__ __launch_bounds__(THREADS, 4) void gemm_mfma_kernel(GemmArgs a) {
-    static_assert(!(DUMP && GATED), "the parity hook dumps plain projections");
     __shared__ Smem sm;
     uint32_t row_tile, tok_tile;
     bool valid_tile;
     // K split (plain single-weight launches only): workgroup (tile, share) walks the stages [first, first + stages) of its tile
-    const uint32_t ksplit = DUMP || GATED || a.ksplit < 2 ? 1u : a.ksplit;
+    const uint32_t ksplit = DUMP || a.ksplit < 2 ? 1u : a.ksplit;
     const uint32_t split = ksplit > 1 ? blockIdx.x % ksplit : 0u;
     tile_of_block(ksplit > 1 ? blockIdx.x / ksplit : blockIdx.x, a.row_tiles, a.tok_tiles, row_tile, tok_tile, valid_tile);
     if (!valid_tile) return;  // whole workgroup leaves together
-    if constexpr (!GATED) select_weight(a, row_tile);
-    const uint32_t row0 = row_tile * (GATED ? BM / 2 : BM);  // GATED: 64 output rows per tile, see load_stage
+    select_weight(a, row_tile);
+    const uint32_t row0 = row_tile * BM;
     const uint32_t tok0 = tok_tile * BN;
 
     const uint32_t lane = threadIdx.x & 63u;
@@ -521,7 +520,7 @@ __global__ __launch_bounds__(THREADS, 4) void gemm_mfma_kernel(GemmArgs a) {
 
     StageRegs regs;
     StagePtrs<BN> ptrs;
-    init_stage_ptrs<BN, GATED>(a, row_tile, tok0, first * KB, ptrs);
+    init_stage_ptrs<BN>(a, row_tile, tok0, first * KB, ptrs);
     dma_stage(ptrs, sm.st[0]);
     load_stage(ptrs, regs);
     store_stage(sm.st[0], regs);
@@ -607,226 +606,363 @@ __global__ __launch_bounds__(THREADS, 4) void gemm_mfma_kernel(GemmArgs a) {
         __syncthreads();
     }
 
-    if constexpr (GATED) {
-        // silu(gate) * up and the Q8_0 quantizer on the wave's registers, element for element what silu_mul_quantize_kernel
-        // computes from the two float results: row tiles 0 / 1 are gate rows A / B, 2 / 3 the same rows of up; the 16 lanes
-        // of a DPP row hold the 16 rows of a tile for the same four tokens, so one row reduction gives a block's maximum.
-        static_assert(RT == 4, "two gate and two up row tiles per wave");
-        const uint32_t rbase = row0 + (wrow0 >> 1);  // first of this wave's 32 output rows = one Q8_0 block
-#pragma unroll
-        for (int tt = 0; tt < TT; tt++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const uint32_t tok = tok0 + wtok0 + 16 * tt + 4 * kq + r;
-                const float ha = silu_mul(acc[tt][0][r], acc[tt][2][r]), hb = silu_mul(acc[tt][1][r], acc[tt][3][r]);
-                const float amax = row_max16(fmaxf(fabsf(ha), fabsf(hb)));
-                float id;
-                const float scale = q8_scale_and_inverse(amax, id);
-                const int qa = (int)__builtin_rintf(__fmul_rn(ha, id)), qb = (int)__builtin_rintf(__fmul_rn(hb, id));
-                if (tok < a.n && rbase < a.m) {  // m % 32 == 0: a block is inside the matrix or not at all
-                    int8_t* dst = a.q_out + (size_t)tok * a.m + rbase;
-                    dst[l16] = (int8_t)qa;
-                    dst[16 + l16] = (int8_t)qb;
-                    if (l16 == 0) a.s_out[(size_t)tok * (a.m >> 5) + (rbase >> 5)] = scale;
-                }
-            }
-    } else if constexpr (!DUMP) {
+    if constexpr (!DUMP) {
         store_wave_tile<TT, RT>(a, ksplit, split, row0 + wrow0 + l16, tok0 + wtok0 + 4 * kq,
                                 [&](int tt, int rt, int r) { return acc[tt][rt][r]; });
     }
 }
 
 // ---------------------------------------------------------------------------------------
-// The wide tile on the large MFMA shape: same workgroup tile (128 rows x 128 tokens), same stages, copies and LDS layouts
-// as gemm_mfma_kernel, but a wave's 64 rows x 32 tokens are TWO v_mfma_i32_32x32x32_i8 per block (rows 0..31 and 32..63 of
-// the wave against its 32 tokens) instead of eight 16x16x32: the small shape runs the matrix unit at a third of its rate and
-// its time adds to the scaling FMAs' (a SIMD does not overlap the two), so a block's matrix work drops from ~160 to ~57 cycles.
-// Layout of the 32x32 result: lane l holds weight row n = l % 32 (of its row half) and the 16 tokens
-// m = 8 g + 4 (l / 32) + r, g = 0..3, r = 0..3 -- one row-scale pair per MFMA and 16 token scales per block (four 16-byte LDS
-// reads, shared by both MFMAs).  ONE result buffer: MFMA -> its 32 FMAs -> MFMA -> its 32 FMAs; the other waves of the SIMD
-// cover the MFMA's latency (measured: faster than two buffers, and 16 registers cheaper, which is what lets the 16-register
-// bias tuple, 16 token scales and 32 accumulators fit four waves per SIMD).  Operands of block b+1 are requested as soon as
-// the second MFMA of block b has been issued, token scales group by group behind their last use.
-// Plain projections only (the gated launch keeps the 16x16 kernel, whose epilogue is written for that result layout).
+// The tiles of a prompt: T32<RT, TT, WR, WT, SB> = WR x WT waves, each RT granules of 32 weight rows x TT groups of 32 tokens, on
+// v_mfma_i32_32x32x32_i8, SB blocks of K per stage.  Layout of a 32x32 result: lane l holds weight row n = l % 32 of its granule and
+// the 16 tokens m = 8 g + 4 (l / 32) + r, g = 0..3, r = 0..3 -- one row-scale pair per granule and 16 token scales per token group.
+//
+// What bounds it: a SIMD runs its matrix instructions and its scaling FMAs one after the other (32 FMAs + one MFMA per 32 x 32 block
+// result, ~124 cycles together), and every operand comes through the CU's one LDS.  A wave of 64 rows x 32 tokens reads 128 bytes per
+// lane for 64 FMAs, which with four such waves per SIMD keeps the LDS as busy as the SIMDs; 128 rows x 64 tokens reads 256 bytes for
+// 256 FMAs, half as much per FMA, and needs 2 waves per SIMD instead of 4.  The block loop alone, fed from LDS: 1217 TOP/s for 64 x 32
+// with four waves per SIMD, 1250 for 64 x 64 and 1346 for 128 x 64 with two.
+//
+// TWO result buffers: the MFMA of tile t + 1 is issued before the FMAs of tile t, so that one wave alone keeps its SIMD busy (the other
+// wave may be waiting at its stage's barrier).  Every operand register is refilled from LDS for the next block as soon as its last use
+// has been issued; all LDS addresses are immediates on four lane bases (the stage loop is written out for both buffers), so the block
+// loop holds FMAs, MFMAs, LDS reads and waits only.
 typedef int v16i __attribute__((ext_vector_type(16)));
-struct Mats32 {
-    v4i a, b0, b1;  // 16 K-bytes of this lane's token / of its row in the wave's first and second 32 rows
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+template <int RT_, int TT_, int WR_, int WT_, int SB_, int OCC_ = 2>
+struct T32 {
+    static constexpr int RT = RT_, TT = TT_, WR = WR_, WT = WT_, SB = SB_, kOcc = OCC_;
+    static constexpr int kWaves = WR * WT, kThreads = 64 * kWaves;
+    static constexpr int kGranules = WR * RT, kRows = GR * kGranules, kTokens = 32 * WT * TT;
+    static constexpr int kTiles = RT * TT;  // 32 x 32 results per wave and block
+    static_assert(kGranules % 2 == 0 && (SB == 2 || SB == 4) && (kTiles == 1 || (RT >= 2 && kTiles % 2 == 0)), "pairs of granules, half a slab or a slab per stage, alternating result buffers");
+    // One stage in LDS.  xt: [token][2 SB chunks of 16 bytes], swizzled so that consecutive tokens reading one chunk spread over all
+    // banks: position p of token t holds chunk p ^ swizzle(t).
+    struct Stage {
+        uint4 wt[kGranules][2][SB][GR];  // [granule][khalf][block][row]
+        float2 dws[kGranules][SB][GR];
+        uint4 xt[kTokens][2 * SB];
+    };
+    struct Smem {
+        Stage st[2];
+        float dxf[2][KB][kTokens];  // token scales of a slab (4 blocks), two slabs
+    };
+    static __device__ __forceinline__ uint32_t swizzle(uint32_t t) { return SB == 4 ? (t >> 1) & 7u : (t >> 2) & 3u; }
 };
-struct Scales32 {
-    float2 dw0, dw1;  // {dw, -12582912*dw} of this lane's two rows
-    v4f dx[4];        // token scales of its four token groups
+
+template <int I>
+struct Idx {
+    static constexpr int value = I;
 };
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (I < N) {
+        f(Idx<I>{});
+        static_for<N, I + 1>(f);
+    }
+}
+
 template <int OFF>
 __device__ __forceinline__ void lds_read16(uint32_t addr, v4i& dst) {
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
 }
-__device__ __forceinline__ void load_mats(const LaneAddr& la, Mats32& m) {  // 3 reads
-    lds_read16<0>(la.xt, m.a);
-    lds_read16<0>(la.wt, m.b0);
-    lds_read16<kSlabWt>(la.wt, m.b1);  // the wave's second granule
+// At most N LDS reads outstanding; ties what becomes valid with it.
+template <int N, typename V>
+__device__ __forceinline__ void lds_arrived(V& v) {
+    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(v) : "n"(N) : "memory");
 }
-template <int G>
-__device__ __forceinline__ void load_tok_scales32(const LaneAddr& la, Scales32& s) {  // 1 read
-    lds_read16<32 * G>(la.dxf, s.dx[G]);
-}
-// (the waits tie the registers that become valid, so nothing that uses them can be scheduled above)
-template <int N>
-__device__ __forceinline__ void lds_wait_a_b0(Mats32& m) {
-    asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(m.a), "+v"(m.b0) : "n"(N) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void lds_wait_phase_a(Mats32& m, Scales32& s) {
-    asm volatile("s_waitcnt lgkmcnt(%6)" : "+v"(m.b1), "+v"(s.dw0), "+v"(s.dx[0]), "+v"(s.dx[1]), "+v"(s.dx[2]), "+v"(s.dx[3]) : "n"(N) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void lds_wait_dw1(Scales32& s) {
-    asm volatile("s_waitcnt lgkmcnt(%1)" : "+v"(s.dw1) : "n"(N) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void lds_wait_all(Mats32& m, Scales32& s) {
-    asm volatile("s_waitcnt lgkmcnt(%9)"
-                 : "+v"(m.a), "+v"(m.b0), "+v"(m.b1), "+v"(s.dw0), "+v"(s.dw1), "+v"(s.dx[0]), "+v"(s.dx[1]), "+v"(s.dx[2]), "+v"(s.dx[3])
-                 : "n"(N)
-                 : "memory");
+template <typename V>
+__device__ __forceinline__ void tie(V& v) {
+    asm volatile("" : "+v"(v));
 }
 
-template <int TYPE, bool DUMP>
-__global__ __launch_bounds__(THREADS, 4) void gemm_mfma32_kernel(GemmArgs a) {
-    __shared__ Smem sm;
+template <int TYPE, bool DUMP, bool GATED, typename C>
+__global__ __launch_bounds__(C::kThreads, C::kOcc) void gemm_tile_kernel(GemmArgs a) {
+    constexpr int RT = C::RT, TT = C::TT, SB = C::SB, T = C::kTiles;
+    __shared__ __align__(16) typename C::Smem sm;
     uint32_t row_tile, tok_tile;
     bool valid_tile;
-    const uint32_t ksplit = DUMP || a.ksplit < 2 ? 1u : a.ksplit;
+    // K split (plain single-weight launches only): workgroup (tile, share) walks the slabs [first, first + slabs) of its tile
+    const uint32_t ksplit = DUMP || GATED || a.ksplit < 2 ? 1u : a.ksplit;
     const uint32_t split = ksplit > 1 ? blockIdx.x % ksplit : 0u;
     tile_of_block(ksplit > 1 ? blockIdx.x / ksplit : blockIdx.x, a.row_tiles, a.tok_tiles, row_tile, tok_tile, valid_tile);
     if (!valid_tile) return;  // whole workgroup leaves together
-    select_weight(a, row_tile);
-    const uint32_t row0 = row_tile * BM;
-    const uint32_t tok0 = tok_tile * BN;
+    if constexpr (!GATED) select_weight(a, row_tile);
+    const uint32_t row0 = row_tile * (GATED ? C::kRows / 2 : C::kRows);
+    const uint32_t tok0 = tok_tile * C::kTokens;
+    const uint32_t lane = threadIdx.x & 63u, l32 = lane & 31u, kh = lane >> 5;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t wr = wave / C::WT, wt = wave % C::WT;
+    const uint32_t nb = a.k >> 5, all_slabs = nb / KB;
+    const uint32_t first = split * all_slabs / ksplit;  // shares differ by at most one slab, none is empty
+    const uint32_t slabs = (split + 1u) * all_slabs / ksplit - first;
 
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = threadIdx.x >> 6;
-    const uint32_t l32 = lane & 31u;
-    const uint32_t kh = lane >> 5;            // which 16-byte half of the block this lane feeds
-    const uint32_t wrow0 = (wave >> 2) * 64;  // wave's rows within the tile
-    const uint32_t wtok0 = (wave & 3u) * 32;  // wave's tokens within the tile
-    const uint32_t nb = a.k >> 5;
-    const uint32_t all_stages = nb / KB;
-    const uint32_t first = split * all_stages / ksplit;  // shares differ by at most one stage, none is empty
-    const uint32_t stages = (split + 1u) * all_stages / ksplit - first;
-
-    float acc[2][16];  // [row half][4 g + r]
+    // ---- the stage's copies: global -> LDS directly, 1 KB per wave instruction, uniform bases that move one stage on per copy round ----
+    constexpr int kPairs = C::kGranules / 2, kXChunks = C::kTokens * 2 * SB / 64;
+    constexpr int kPairWaves = kPairs < C::kWaves ? kPairs : C::kWaves;  // waves that copy weights (the others: activations only)
+    constexpr int kPairsPer = kPairs / kPairWaves;
+    constexpr int kXPer = kXChunks / C::kWaves;
+    static_assert(kXChunks % C::kWaves == 0 && kPairs % kPairWaves == 0, "copies deal out evenly");
+    const uint32_t pairs_total = (a.m + 2 * GR - 1) / (2 * GR);
+    const uint8_t* wsrc[kPairsPer];
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+    for (int i = 0; i < kPairsPer; i++) {
+        const uint32_t lp = min(wave, (uint32_t)kPairWaves - 1u) * kPairsPer + i;
+        // the tile's pair lp: rows 64 lp ..; a gated tile: its pairs of gate, then the same ones of up
+        const bool up = GATED && lp >= kPairs / 2;
+        const uint32_t p = GATED ? row_tile * (kPairs / 2) + lp - (up ? kPairs / 2 : 0) : row_tile * kPairs + lp;
+        const uint8_t* w = up ? a.w_up : a.w;
+        wsrc[i] = w + ((size_t)min(p, pairs_total - 1u) * all_slabs + first) * (2 * kSlab);  // past the end: any rows, never stored
+    }
+    uint32_t woff = 16u * lane;                                               // this lane's 16 bytes of a kilobyte of operand rows
+    uint32_t soff = SB == 4 ? 16u * lane : 16u * l32 + (uint32_t)kSlab * kh;  // ... of a kilobyte of scale pairs (SB = 2: 512 B of either granule)
+    uint32_t xoff[kXPer];
 #pragma unroll
-        for (int i = 0; i < 16; i++) acc[j][i] = 0.0f;
+    for (int j = 0; j < kXPer; j++) {
+        const uint32_t tt = (64u / (2 * SB)) * (kXPer * wave + j) + lane / (2 * SB);  // token within the tile
+        const uint32_t chunk = (lane % (2 * SB)) ^ C::swizzle(tt);
+        xoff[j] = min(tt, a.n - 1u - tok0) * a.k + 16u * chunk;
+    }
+    const int8_t* xsrc = a.xq + (size_t)tok0 * a.k + (size_t)first * (KB * 32);
+    auto copy_lds = [](const void* g, void* l) {
+        __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)g, (void __attribute__((address_space(3)))*)l, 16, 0, 0);
+    };
+    // stage h (SB = 2: half a slab, SB = 4: a slab) into its buffer; then the bases move on
+    auto copy_stage = [&](uint32_t h_) {
+        typename C::Stage& s = sm.st[h_ & 1u];
+        const uint32_t half = SB == 2 ? h_ & 1u : 0u;
+        tie(woff), tie(soff);  // (opaque, or the compiler keeps a 64-bit address per copy in registers)
+        if (wave < (uint32_t)kPairWaves) {
+#pragma unroll
+            for (int i = 0; i < kPairsPer; i++) {
+                const uint32_t lp = wave * kPairsPer + i;
+#pragma unroll
+                for (int g = 0; g < 2; g++)
+#pragma unroll
+                    for (int h = 0; h < 2; h++)
+#pragma unroll
+                        for (int c = 0; c < SB / 2; c++)
+                            copy_lds(wsrc[i] + (g * kSlab + h * 2048 + (SB == 2 ? half * 1024 : c * 1024)) + woff,
+                                     reinterpret_cast<uint8_t*>(&s.wt[2 * lp + g][h][0][0]) + 1024 * c);
+                if constexpr (SB == 2) copy_lds(wsrc[i] + (kSlabWt + half * 512) + soff, &s.dws[2 * lp][0][0]);
+                else {
+                    copy_lds(wsrc[i] + kSlabWt + soff, &s.dws[2 * lp][0][0]);
+                    copy_lds(wsrc[i] + kSlab + kSlabWt + soff, &s.dws[2 * lp + 1][0][0]);
+                }
+                wsrc[i] += SB == 4 || half == 1 ? 2 * kSlab : 0;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < kXPer; j++) tie(xoff[j]), copy_lds(xsrc + xoff[j], reinterpret_cast<uint8_t*>(&s.xt[0][0]) + 1024u * (kXPer * wave + j));
+        xsrc += SB * 32;
+    };
+    // token scales of a slab (block-major in memory) through registers, one float4 per token, threads 0 .. kTokens - 1
+    static_assert(C::kTokens <= C::kThreads, "a thread per token");
+    const bool has_dx = threadIdx.x < (uint32_t)C::kTokens && a.xs;  // xs is null only for the parity hook, which never scales
+    const uint8_t* dxsrc = reinterpret_cast<const uint8_t*>(a.xs + (size_t)tok0 * nb + (size_t)first * KB);
+    uint32_t dxoff = min(threadIdx.x, a.n - 1u - tok0) * nb * (uint32_t)sizeof(float);
+    float4 dxr = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto load_dx = [&] {
+        tie(dxoff);
+        if (has_dx) dxr = *reinterpret_cast<const float4*>(dxsrc + dxoff);
+        dxsrc += KB * sizeof(float);
+    };
+    auto store_dx = [&](uint32_t buf) {
+        if (threadIdx.x < (uint32_t)C::kTokens) {
+            const uint32_t at = threadIdx.x ^ 1u;  // neighbours swapped: see the FMA that reads them
+            sm.dxf[buf][0][at] = dxr.x;
+            sm.dxf[buf][1][at] = dxr.y;
+            sm.dxf[buf][2][at] = dxr.z;
+            sm.dxf[buf][3][at] = dxr.w;
+        }
+    };
 
+    v16f acc[RT][TT];  // [granule][token group]: elements 4 g + r
+#pragma unroll
+    for (int i = 0; i < RT; i++)
+#pragma unroll
+        for (int j = 0; j < TT; j++) acc[i][j] = v16f{};
     v16i cbias;
 #pragma unroll
     for (int i = 0; i < 16; i++) cbias[i] = (int)kBiasBits;
     asm volatile("" : "+v"(cbias));  // keep it in registers (left alone, the compiler rebuilds it before every MFMA)
 
-    StageRegs regs;
-    StagePtrs<BN> ptrs;
-    init_stage_ptrs<BN, false>(a, row_tile, tok0, first * KB, ptrs);
-    dma_stage(ptrs, sm.st[0]);
-    load_stage(ptrs, regs);
-    store_stage(sm.st[0], regs);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's direct-to-LDS copies have landed
-    __syncthreads();
-
-    LaneAddr la;
-    {
-        const Stage& s = sm.st[0];
-        // this lane's token row; K-chunk 2*block + kh sits at position chunk ^ swizzle
-        const uint32_t sw = xt_swizzle(wtok0 + l32);
-        la.xsh = sw >> 1;
-        la.xbase = lds_addr(&s.xt[wtok0 + l32][0]) + (((kh ^ sw) & 1u) << 4);
-        la.xt = la.xbase + (la.xsh << 5);
-        la.wt = lds_addr(&s.wt[wrow0 / GR][kh][0][l32]);  // the wave's 64 rows are two granules
-        la.dws = lds_addr(&s.dws[wrow0 / GR][0][l32]);
-        la.dxf = lds_addr(&s.dxf[0][wtok0 + 4 * kh]);
-    }
-
-    for (uint32_t st = 0; st < stages; st++) {
-        if (st + 1 < stages) {
-            dma_stage(ptrs, sm.st[(st + 1) & 1u]);
-            load_stage(ptrs, regs);
-        }
-
-        // Reads of a block, in issue order (LDS data returns in that order): a, b0, b1, dw0, dx0..dx3, dw1.
-        Mats32 mt;
-        Scales32 sc;
-        load_mats(la, mt);                  // 3
-        lds_read8<0>(la.dws, sc.dw0);       // 1
-        load_tok_scales32<0>(la, sc);       // 4
-        load_tok_scales32<1>(la, sc);
-        load_tok_scales32<2>(la, sc);
-        load_tok_scales32<3>(la, sc);
-        lds_read8<kSlabDws>(la.dws, sc.dw1);  // 1
-#pragma unroll 1
-        for (int b = 0; b < KB; b++) {
-            next_block(la, (uint32_t)b, b + 1 < KB);  // last iteration: harmless re-read of its own block
-            const uint32_t row = row0 + wrow0 + l32, tok = tok0 + wtok0 + 4 * kh, blk = (first + st) * KB + b;
-            auto consume = [&](const v16i& d, int j, const float2 dw) {
+    // This lane's LDS bases; everything else of an address is an immediate.
+    // (granule rt of a wave: its RT consecutive ones of the tile, or its RT / 2 of gate and the same RT / 2 of up)
+    constexpr int kOwn = GATED ? RT / 2 : RT;
+    uint32_t a_wt = lds_addr(&sm.st[0].wt[kOwn * wr][kh][0][l32]);
+    uint32_t a_dws = lds_addr(&sm.st[0].dws[kOwn * wr][0][l32]);
+    uint32_t a_dxf = lds_addr(&sm.dxf[0][0][32 * TT * wt + 4 * kh]);
+    uint32_t a_xt[SB];  // chunk 2 b + kh of this lane's token sits at position chunk ^ swizzle
 #pragma unroll
-                for (int g = 0; g < 4; g++) {
+    for (int b = 0; b < SB; b++) a_xt[b] = lds_addr(&sm.st[0].xt[32 * TT * wt + l32][(2u * b + kh) ^ C::swizzle(l32)]);
+    constexpr uint32_t kBuf = sizeof(typename C::Stage);
+
+    v4i A[TT], B[RT];
+    float2 dw[RT];
+    v4f dx[4];
+    v16i D[2];
+    constexpr auto granule = [](int rt) { return rt < kOwn ? rt : C::kGranules / 2 + rt - kOwn; };
+    // LDS reads of block b of the stage
+    auto read_ab = [&](auto b) {  // TT + RT reads
+        static_for<TT>([&](auto t) { lds_read16<32 * decltype(t)::value * 32 * SB>(a_xt[decltype(b)::value], A[decltype(t)::value]); });
+        static_for<RT>([&](auto r) { lds_read16<1024 * SB * granule(decltype(r)::value) + 512 * decltype(b)::value>(a_wt, B[decltype(r)::value]); });
+    };
+    auto read_dw = [&](auto b, auto r) { lds_read8<256 * SB * granule(decltype(r)::value) + 256 * decltype(b)::value>(a_dws, dw[decltype(r)::value]); };
+    auto read_dx = [&](auto b, auto t, auto g) {
+        lds_read16<decltype(b)::value * 4 * C::kTokens + 128 * decltype(t)::value + 32 * decltype(g)::value>(a_dxf, dx[decltype(g)::value]);
+    };
+
+    // One stage: SB blocks, the first of them block blk0 of the row.
+    auto compute_stage = [&](uint32_t blk0) {
+        read_ab(Idx<0>{});
+        static_for<RT - 1>([&](auto r) { read_dw(Idx<0>{}, r); });
+        static_for<4>([&](auto g) { read_dx(Idx<0>{}, Idx<0>{}, g); });
+        read_dw(Idx<0>{}, Idx<RT - 1>{});
+        // (the reads behind the operands' may still be in flight)
+        lds_arrived<RT + 4>(A[0]);
+        static_for<TT>([&](auto t) { tie(A[decltype(t)::value]); });
+        static_for<RT>([&](auto r) { tie(B[decltype(r)::value]); });
+        D[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[0], B[0], cbias, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        static_for<SB>([&](auto b_) {
+            constexpr int b = decltype(b_)::value;
+            constexpr bool next = b + 1 < SB;
+            static_for<T>([&](auto t_) {
+                constexpr int t = decltype(t_)::value, tt = t / RT, rt = t % RT;
+                if constexpr (T == 1) {
+                    // one result per wave and block: nothing to run ahead with, the next block's MFMA goes out behind the FMAs
+                } else if constexpr (t + 1 < T) {
+                    constexpr int tt1 = (t + 1) / RT, rt1 = (t + 1) % RT;
+                    D[(t + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[tt1], B[rt1], cbias, 0, 0, 0);
+                } else if constexpr (next) {
+                    lds_arrived<1>(A[0]);  // all operands of the next block; its scale pair of granule RT - 2 may still be on its way
+                    static_for<TT>([&](auto i) { tie(A[decltype(i)::value]); });
+                    static_for<RT>([&](auto i) { tie(B[decltype(i)::value]); });
+                    D[(t + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[0], B[0], cbias, 0, 0, 0);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                constexpr bool fetch = next && (T == 1 || t == T - 2);  // all MFMAs of this block have been issued
+                if constexpr (fetch) read_ab(Idx<next ? b + 1 : 0>{});
+                constexpr int kFetched = fetch ? TT + RT : 0;  // reads that a wait below may leave outstanding on top
+                if constexpr (rt == RT - 1 && tt == 0) lds_arrived<kFetched + (TT == 1 && RT > 1 && next ? 1 : 0)>(dw[rt]);
+                static_for<4>([&](auto g_) {
+                    constexpr int g = decltype(g_)::value;
+                    if constexpr (rt == 0) {
+                        lds_arrived<(tt == 0 ? 4 : 3) - g + kFetched>(dx[g]);
+                        if constexpr (g == 0 && tt == 0) static_for<RT - 1>([&](auto i) { tie(dw[decltype(i)::value]); });
+                    }
                     if constexpr (DUMP) {
+                        const uint32_t row = row0 + GR * (RT * wr + rt) + l32, tok = tok0 + 32 * (TT * wt + tt) + 4 * kh + 8 * g;
 #pragma unroll
                         for (int r = 0; r < 4; r++) {
-                            if (row + 32 * j < a.m && tok + 8 * g + r < a.n) {
-                                int v = d[4 * g + r] - (int)kBiasBits;
+                            if (row < a.m && tok + r < a.n) {
+                                int v = D[t & 1][4 * g + r] - (int)kBiasBits;
                                 if (TYPE == 2) v >>= 4;  // weights were stored x16; exact
-                                a.dots[((size_t)(tok + 8 * g + r) * a.m + row + 32 * j) * nb + blk] = v;
+                                a.dots[((size_t)(tok + r) * a.m + row) * nb + blk0 + b] = v;
                             }
                         }
                     } else {
 #pragma unroll
                         for (int r = 0; r < 4; r++) {
-                            const float v = __builtin_fmaf(__int_as_float(d[4 * g + r]), dw.x, dw.y);
-                            acc[j][4 * g + r] = __builtin_fmaf(v, sc.dx[g][r], acc[j][4 * g + r]);
+                            const float v = __builtin_fmaf(__int_as_float(D[t & 1][4 * g + r]), dw[rt].x, dw[rt].y);
+                            acc[rt][tt][4 * g + r] = __builtin_fmaf(v, dx[g][r ^ 1], acc[rt][tt][4 * g + r]);
                         }
+                        // (without this the compiler lets the MFMAs of all tiles run ahead of their FMAs, and spills)
+                        tie(acc[rt][tt]);
                     }
-                    if (j == 1) {  // this group's token scales are done with: request the next block's
-                        if (g == 0) load_tok_scales32<0>(la, sc);
-                        if (g == 1) load_tok_scales32<1>(la, sc);
-                        if (g == 2) load_tok_scales32<2>(la, sc);
-                        if (g == 3) load_tok_scales32<3>(la, sc);
+                    // this group's token scales are done with: the next token group's, or the next block's first
+                    if constexpr (rt == RT - 1) {
+                        if constexpr (tt + 1 < TT) read_dx(Idx<b>{}, Idx<tt + 1 < TT ? tt + 1 : 0>{}, g_);
+                        else if constexpr (next) read_dx(Idx<next ? b + 1 : b>{}, Idx<0>{}, g_);
                     }
                     __builtin_amdgcn_sched_barrier(0);
+                });
+                if constexpr (tt == TT - 1 && next) read_dw(Idx<next ? b + 1 : 0>{}, Idx<rt>{});
+                if constexpr (T == 1 && next) {
+                    lds_arrived<5>(A[0]), tie(B[0]);  // (the scales behind them may still be in flight)
+                    D[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[0], B[0], cbias, 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
                 }
-            };
-            lds_wait_a_b0<7>(mt);  // the seven reads issued after a and b0 may still be in flight
-            v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(mt.a, mt.b0, cbias, 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);  // (the MFMA goes out before the wait for what only the FMAs need)
-            lds_wait_phase_a<1>(mt, sc);  // everything but dw1
-            __builtin_amdgcn_sched_barrier(0);
-            consume(d, 0, sc.dw0);
-            d = __builtin_amdgcn_mfma_i32_32x32x32_i8(mt.a, mt.b1, cbias, 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-            load_mats(la, mt);             // both MFMAs of this block have been issued
-            lds_read8<0>(la.dws, sc.dw0);  // the first row half is done
-            lds_wait_dw1<4>(sc);           // (the four reads just issued stay in flight)
-            __builtin_amdgcn_sched_barrier(0);
-            consume(d, 1, sc.dw1);
-            lds_read8<kSlabDws>(la.dws, sc.dw1);
-        }
-        lds_wait_all<0>(mt, sc);  // nothing of this stage's buffer is read past this point
-        {   // block 0 of the other buffer (the block loop left wt / dws / dxf at block KB - 1)
-            const uint32_t other = (st & 1u) ? 0u - (uint32_t)sizeof(Stage) : (uint32_t)sizeof(Stage);
-            la.xbase += other;
-            la.xt = la.xbase + (la.xsh << 5);
-            la.wt += other - (KB - 1) * kOffWt;
-            la.dws += other - (KB - 1) * kOffDws;
-            la.dxf += other - (KB - 1) * kOffDxf;
-        }
-        if (st + 1 < stages) store_stage(sm.st[(st + 1) & 1u], regs);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // direct-to-LDS copies of the next stage have landed
+            });
+        });
+    };
+    // The stage's reads are all done (nothing is outstanding past its last wait) and the next stage's copies have landed.
+    auto end_stage = [] {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
+    };
+
+    constexpr uint32_t HS = KB / SB;  // stages per slab
+    const uint32_t stages = slabs * HS;
+    load_dx();
+    copy_stage(0);
+    store_dx(0);
+    end_stage();
+    for (uint32_t h = 0; h < stages; h++) {
+        const uint32_t h1 = h + 1;
+        const bool more = h1 < stages, new_slab = more && h1 % HS == 0;
+        if (new_slab) load_dx();
+        if (more) copy_stage(h1);
+        compute_stage((first * HS + h) * SB);
+        const uint32_t other = h & 1u ? 0u - kBuf : kBuf;  // to the other buffer
+        a_wt += other, a_dws += other;
+#pragma unroll
+        for (int b = 0; b < SB; b++) a_xt[b] += other;
+        // token scales: blocks 0 .. 7 of the two slabs of dxf, then from the start
+        a_dxf += (h1 % (2 * HS) == 0 ? 0u - (2 * HS - 1) * SB : (uint32_t)SB) * (uint32_t)(sizeof(float) * C::kTokens);
+        if (new_slab) store_dx((h1 / HS) & 1u);
+        end_stage();
     }
 
-    if constexpr (!DUMP) {
-        store_wave_tile<4, 2, 8, 32>(a, ksplit, split, row0 + wrow0 + l32, tok0 + wtok0 + 4 * kh,
-                                     [&](int g, int j, int r) { return acc[j][4 * g + r]; });
+    if constexpr (GATED) {
+        // silu(gate) * up and the Q8_0 quantizer, element for element what silu_mul_quantize_kernel computes from the two float
+        // results: granules 0 .. RT / 2 - 1 of the wave are gate rows, the others the same rows of up, 32 rows = one Q8_0 block of a
+        // token.  The gated values go through a wave-private piece of LDS (the stages are done with), so that eight lanes own a block
+        // with four rows each: one scale per block and eight lanes instead of 32, and 4-byte stores.
+        constexpr int kRow = 36;  // floats per token row: 16-byte aligned, neighbouring tokens on other banks
+        static_assert(sizeof(sm) >= sizeof(float) * kRow * 32 * C::kWaves, "a 32 x 32 block of floats per wave");
+        float* const h = reinterpret_cast<float*>(&sm) + kRow * 32 * wave;
+#pragma unroll
+        for (int j = 0; j < kOwn; j++)
+#pragma unroll
+            for (int tt = 0; tt < TT; tt++) {
+                float v[16], far = 0.0f;
+#pragma unroll
+                for (int e = 0; e < 16; e++) {
+                    float n;
+                    const float ex = ggml_expf_near(-acc[j][tt][e], n);
+                    far = fmaxf(far, fabsf(n));
+                    v[e] = __fmul_rn(__fdiv_rn(acc[j][tt][e], __fadd_rn(1.0f, ex)), acc[kOwn + j][tt][e]);
+                }
+                if (__builtin_amdgcn_ballot_w64(!(far <= 126.0f)) != 0) {  // a lane outside the short branch of the exponential (or not a number)
+#pragma unroll
+                    for (int e = 0; e < 16; e++) v[e] = silu_mul(acc[j][tt][e], acc[kOwn + j][tt][e]);
+                }
+#pragma unroll
+                for (int e = 0; e < 16; e++) h[kRow * (4 * kh + 8 * (e >> 2) + (e & 3)) + l32] = v[e];
+                const uint32_t rbase = row0 + 32u * (kOwn * wr + j);
+                if (rbase < a.m) {  // m % 32 == 0: a block is inside the matrix or not at all
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const uint32_t t = 8u * i + (lane >> 3), tok = tok0 + 32 * (TT * wt + tt) + t;
+                        const float4 x = *reinterpret_cast<const float4*>(&h[kRow * t + 4u * (lane & 7u)]);
+                        float id;
+                        const float scale = q8_scale_and_inverse(group_max8(fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w)))), id);
+                        const uint32_t packed = q8_pack4(x.x, x.y, x.z, x.w, id);
+                        if (tok < a.n) {
+                            *reinterpret_cast<uint32_t*>(a.q_out + (size_t)tok * a.m + rbase + 4u * (lane & 7u)) = packed;
+                            if ((lane & 7u) == 0) a.s_out[(size_t)tok * (a.m >> 5) + (rbase >> 5)] = scale;
+                        }
+                    }
+                }
+            }
+    } else if constexpr (!DUMP) {
+#pragma unroll
+        for (int tt = 0; tt < TT; tt++)
+            store_wave_tile<4, RT, 8, 32>(a, ksplit, split, row0 + GR * RT * wr + l32, tok0 + 32 * (TT * wt + tt) + 4 * kh,
+                                          [&](int g, int rt, int r) { return acc[rt][tt][4 * g + r]; });
     }
 }
 
@@ -981,159 +1117,6 @@ __global__ __launch_bounds__(THREADS, 4) void gemm_narrow_kernel(GemmArgs a) {
     }
 }
 
-// The narrow tile (128 rows x 64 tokens) on the large MFMA shape, for launches that have tokens for the whole tile
-// (n > 48; the shorter ones keep gemm_narrow_kernel's 16-token tiles): wave w owns rows 32 (w / 2) .. of the tile (one
-// granule) against tokens 32 (w % 2) .., ONE v_mfma_i32_32x32x32_i8 per block instead of four 16x16x32, the result layout,
-// scale reads and single result buffer of gemm_mfma32_kernel.  Same stages, copies and LDS layouts as gemm_narrow_kernel.
-struct NarrowMats32 {
-    v4i a, b;
-};
-struct NarrowScales32 {
-    float2 dw;
-    v4f dx[4];
-};
-template <int N>
-__device__ __forceinline__ void lds_wait(NarrowMats32& m) {
-    asm volatile("s_waitcnt lgkmcnt(%2)" : "+v"(m.a), "+v"(m.b) : "n"(N) : "memory");
-}
-template <int N>
-__device__ __forceinline__ void lds_wait(NarrowScales32& s) {
-    asm volatile("s_waitcnt lgkmcnt(%5)" : "+v"(s.dw), "+v"(s.dx[0]), "+v"(s.dx[1]), "+v"(s.dx[2]), "+v"(s.dx[3]) : "n"(N) : "memory");
-}
-
-template <int TYPE, bool DUMP>
-__global__ __launch_bounds__(THREADS, 4) void gemm_narrow32_kernel(GemmArgs a) {
-    __shared__ SmemT<BN_NARROW> sm;
-    uint32_t row_tile, tok_tile;
-    bool valid_tile;
-    const uint32_t ksplit = DUMP || a.ksplit < 2 ? 1u : a.ksplit;
-    const uint32_t split = ksplit > 1 ? blockIdx.x % ksplit : 0u;
-    tile_of_block(ksplit > 1 ? blockIdx.x / ksplit : blockIdx.x, a.row_tiles, a.tok_tiles, row_tile, tok_tile, valid_tile);
-    if (!valid_tile) return;  // whole workgroup leaves together
-    select_weight(a, row_tile);
-    const uint32_t row0 = row_tile * BM;
-    const uint32_t tok0 = tok_tile * BN_NARROW;
-
-    const uint32_t lane = threadIdx.x & 63u;
-    const uint32_t wave = threadIdx.x >> 6;
-    const uint32_t l32 = lane & 31u;
-    const uint32_t kh = lane >> 5;             // which 16-byte half of the block this lane feeds
-    const uint32_t wrow0 = (wave >> 1) * 32;   // wave's rows within the tile: one granule
-    const uint32_t wtok0 = (wave & 1u) * 32;   // wave's tokens within the tile
-    const uint32_t nb = a.k >> 5;
-    const uint32_t all_stages = nb / KB;
-    const uint32_t first = split * all_stages / ksplit;
-    const uint32_t stages = (split + 1u) * all_stages / ksplit - first;
-
-    float acc[16];  // [4 g + r]
-#pragma unroll
-    for (int i = 0; i < 16; i++) acc[i] = 0.0f;
-    v16i cbias;
-#pragma unroll
-    for (int i = 0; i < 16; i++) cbias[i] = (int)kBiasBits;
-    asm volatile("" : "+v"(cbias));
-
-    StageRegs regs;
-    StagePtrs<BN_NARROW> ptrs;
-    init_stage_ptrs<BN_NARROW>(a, row_tile, tok0, first * KB, ptrs);
-    dma_stage(ptrs, sm.st[0]);
-    load_stage(ptrs, regs);
-    store_stage(sm.st[0], regs);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's direct-to-LDS copies have landed
-    __syncthreads();
-
-    LaneAddr la;  // block 0 of buffer 0; moved on as in the wide kernel
-    {
-        const StageT<BN_NARROW>& s = sm.st[0];
-        const uint32_t sw = xt_swizzle(wtok0 + l32);
-        la.xsh = sw >> 1;
-        la.xbase = lds_addr(&s.xt[wtok0 + l32][0]) + (((kh ^ sw) & 1u) << 4);
-        la.xt = la.xbase + (la.xsh << 5);
-        la.wt = lds_addr(&s.wt[wrow0 / GR][kh][0][l32]);
-        la.dws = lds_addr(&s.dws[wrow0 / GR][0][l32]);
-        la.dxf = lds_addr(&s.dxf[0][wtok0 + 4 * kh]);
-    }
-
-    for (uint32_t st = 0; st < stages; st++) {
-        if (st + 1 < stages) {
-            dma_stage(ptrs, sm.st[(st + 1) & 1u]);
-            load_stage(ptrs, regs);
-        }
-
-        // Reads of a block, in issue order: a, b, dx0..dx3, dw.
-        NarrowMats32 mt;
-        NarrowScales32 sc;
-        lds_read16<0>(la.xt, mt.a);
-        lds_read16<0>(la.wt, mt.b);
-        lds_read16<0>(la.dxf, sc.dx[0]);
-        lds_read16<32>(la.dxf, sc.dx[1]);
-        lds_read16<64>(la.dxf, sc.dx[2]);
-        lds_read16<96>(la.dxf, sc.dx[3]);
-        lds_read8<0>(la.dws, sc.dw);
-#pragma unroll 1
-        for (int b = 0; b < KB; b++) {
-            const bool adv = b + 1 < KB;  // last iteration: harmless re-read of its own block
-            la.xt = la.xbase + ((((uint32_t)(adv ? b + 1 : b)) ^ la.xsh) << 5);
-            la.wt += adv ? kOffWt : 0;
-            la.dws += adv ? kOffDws : 0;
-            la.dxf += adv ? kOffDxfNarrow : 0;
-            const uint32_t row = row0 + wrow0 + l32, tok = tok0 + wtok0 + 4 * kh, blk = (first + st) * KB + b;
-            lds_wait<5>(mt);  // the five scale reads issued after a and b may still be in flight
-            const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(mt.a, mt.b, cbias, 0, 0, 0);
-            __builtin_amdgcn_sched_barrier(0);
-            lds_read16<0>(la.xt, mt.a);  // the MFMA that reads block b's operands has been issued
-            lds_read16<0>(la.wt, mt.b);
-            lds_wait<2>(sc);  // (the two reads just issued stay in flight)
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int g = 0; g < 4; g++) {
-                if constexpr (DUMP) {
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        if (row < a.m && tok + 8 * g + r < a.n) {
-                            int v = d[4 * g + r] - (int)kBiasBits;
-                            if (TYPE == 2) v >>= 4;  // weights were stored x16; exact
-                            a.dots[((size_t)(tok + 8 * g + r) * a.m + row) * nb + blk] = v;
-                        }
-                    }
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; r++) {
-                        const float v = __builtin_fmaf(__int_as_float(d[4 * g + r]), sc.dw.x, sc.dw.y);
-                        acc[4 * g + r] = __builtin_fmaf(v, sc.dx[g][r], acc[4 * g + r]);
-                    }
-                }
-                // this group's token scales are done with: request the next block's
-                if (g == 0) lds_read16<0>(la.dxf, sc.dx[0]);
-                if (g == 1) lds_read16<32>(la.dxf, sc.dx[1]);
-                if (g == 2) lds_read16<64>(la.dxf, sc.dx[2]);
-                if (g == 3) lds_read16<96>(la.dxf, sc.dx[3]);
-                __builtin_amdgcn_sched_barrier(0);
-            }
-            lds_read8<0>(la.dws, sc.dw);
-        }
-        asm volatile("s_waitcnt lgkmcnt(0)"
-                     : "+v"(mt.a), "+v"(mt.b), "+v"(sc.dw), "+v"(sc.dx[0]), "+v"(sc.dx[1]), "+v"(sc.dx[2]), "+v"(sc.dx[3])
-                     :
-                     : "memory");  // nothing of this stage's buffer is read past this point
-        {
-            const uint32_t other = (st & 1u) ? 0u - (uint32_t)sizeof(StageT<BN_NARROW>) : (uint32_t)sizeof(StageT<BN_NARROW>);
-            la.xbase += other;
-            la.xt = la.xbase + (la.xsh << 5);
-            la.wt += other - (KB - 1) * kOffWt;
-            la.dws += other - (KB - 1) * kOffDws;
-            la.dxf += other - (KB - 1) * kOffDxfNarrow;
-        }
-        if (st + 1 < stages) store_stage(sm.st[(st + 1) & 1u], regs);
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // direct-to-LDS copies of the next stage have landed
-        __syncthreads();
-    }
-
-    if constexpr (!DUMP) {
-        store_wave_tile<4, 1, 8, 32>(a, ksplit, split, row0 + wrow0 + l32, tok0 + wtok0 + 4 * kh, [&](int g, int, int r) { return acc[4 * g + r]; });
-    }
-}
-
 // y (+)= partial[0] + partial[1] + ... in that order, element by element (token-major partials [split][n][m]).
 // (S a template parameter: all of an element's loads are in flight together instead of one round trip per share.)
 template <int S>
@@ -1167,12 +1150,14 @@ uint32_t wide_split_factor(uint32_t m, uint32_t n, uint32_t k, uint32_t max_spli
     return s_;
 }
 
+// Launches of few 128 x 128 tiles (at most one per CU): the ones that may be split over K.
+bool narrow_tiles(uint64_t row_tiles, uint32_t n) { return n <= BN_NARROW || row_tiles * ((n + BN - 1) / BN) <= 256; }
+
 uint32_t split_k_factor(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits) {
     const uint32_t ws = wide_split_factor(m, n, k, max_splits);
     if (ws > 1) return ws;
     const uint32_t row_tiles = (m + BM - 1) / BM;
-    const bool narrow = n <= BN_NARROW || row_tiles * ((n + BN - 1) / BN) <= 256;
-    if (!narrow) return 1;
+    if (!narrow_tiles(row_tiles, n)) return 1;
     const uint32_t tiles = row_tiles * ((n + BN_NARROW - 1) / BN_NARROW), stages = (k >> 5) / KB;
     if (stages < 8) return 1;
     uint32_t s_ = 1;
@@ -1193,64 +1178,90 @@ hipError_t launch_reduce(const GemmArgs& a, const Launch& L) {
     return hipErrorInvalidValue;  // split_k_factor makes 2, 4 or 8 shares
 }
 
+// The three tiles of a prompt (rows x tokens) and when each is taken.  A CU works through its share of the launch's tiles two
+// workgroups at a time, so a launch takes about ceil(tiles / 256) x (what a tile costs the CU): per 256 x 128 results and 2048
+// elements of K 34 / 40 / 46 us on the large / medium / small tile -- the larger a wave's tile, the fewer operand bytes per FMA --
+// plus 5 / 1.4 / 3 us for filling, draining and storing it, and a third more when the CU has only one workgroup.  Measured (large /
+// medium / small, us): 6912 x 2048 over 2002 tokens 82 / 85 / 95, 13824 x 2048 over 4096 266 / 285 / 317, 9216 x 1024 over 2048
+// 69 / 57 / 59, 2048 x 2048 over 2002 53 / 29 / 27, 1024 x 4608 over 2048 109 / 50 / 38.  With the gate in the epilogue the fixed part
+// is 6 / 6.3 / 5 us: 2 x 4608 x 1024 over 2048 tokens 76 / 69 / 68, over 555 35 / 28 / 26, 2 x 6912 x 2048 over 2002 159 / 164 / 169.
+using TileL = T32<4, 2, 2, 2, 2>;     // 256 x 128, 4 waves of 128 x 64
+using TileM = T32<2, 1, 2, 4, 4, 4>;  // 128 x 128, 8 waves of 64 x 32
+using TileS = T32<2, 1, 2, 2, 4>;     // 128 x 64, 4 waves of 64 x 32
+using TileN = T32<1, 1, 4, 2, 4, 4>;  // 128 x 64, 8 waves of 32 x 32: where a CU gets one workgroup at most, its waves are all there is
+template <typename C>
+float tile_cost(uint64_t row_tiles, uint32_t n, uint32_t k, bool gated = false) {
+    const uint64_t tiles = row_tiles * ((n + C::kTokens - 1) / C::kTokens), rounds = (tiles + 255) / 256;
+    const float per_k = C::kRows == 256 ? 34.0f : (C::kTokens == 128 ? 40.0f : 46.0f);
+    const float fixed = C::kRows == 256 ? (gated ? 6.0f : 5.0f) : (C::kTokens == 128 ? (gated ? 6.3f : 1.4f) : (gated ? 5.0f : 3.0f));
+    return (float)rounds * (rounds == 1 ? 1.35f : 1.0f) * ((float)(C::kRows * C::kTokens) / (256.0f * 128.0f)) * (per_k * (float)k / 2048.0f + fixed);
+}
+
+template <typename Cost, typename Go>
+hipError_t cheapest_tile(Cost&& cost, Go&& go) {
+    const float l = cost(TileL{}), m = cost(TileM{}), s_ = cost(TileS{});
+    if (l <= m && l <= s_) return go(TileL{});
+    return m <= s_ ? go(TileM{}) : go(TileS{});
+}
+
 template <bool DUMP>
 hipError_t launch(int type, GemmArgs& a, const Launch& L, uint32_t more = 0, bool defer_reduce = false) {
     if (a.m == 0 || a.n == 0) return hipSuccess;
-    a.row_tiles = (a.m + BM - 1) / BM;
-    a.tile_start[0] = a.tile_start[1] = UINT32_MAX;
-    for (uint32_t i = 0; i < more; i++) {
-        a.tile_start[i] = a.row_tiles;
-        a.row_tiles += (a.m_more[i] + BM - 1) / BM;
-    }
-    // The narrow tile also serves small problems that would leave more than half of the
-    // 512 resident workgroup slots (2 per CU) empty with the wide tile: twice the tiles.
+    const auto tile_rows = [&](uint32_t rows) {  // row tiles of `rows` rows over the launch's weights
+        uint64_t t = (a.m + (uint64_t)rows - 1) / rows;
+        for (uint32_t i = 0; i < more; i++) t += (a.m_more[i] + (uint64_t)rows - 1) / rows;
+        return t;
+    };
     const bool wide_split = !DUMP && more == 0 && a.ksplit > 1 && wide_split_factor(a.m, a.n, a.k, a.ksplit) == a.ksplit;
-    const bool narrow = !wide_split && (a.n <= BN_NARROW || a.row_tiles * ((a.n + BN - 1) / BN) <= 256);
-    a.tok_tiles = narrow ? (a.n + BN_NARROW - 1) / BN_NARROW : (a.n + BN - 1) / BN;
-    if ((uint64_t)a.row_tiles * a.tok_tiles > 0x7fffff00ull) return hipErrorInvalidValue;  // beyond a launch's grid
-    const uint32_t tiles = a.row_tiles * a.tok_tiles;
-    const uint32_t blocks = ((tiles + 7u) / 8u) * 8u;  // every XCD gets the same number of slots
-    if (narrow) {
+    if (DUMP || (!wide_split && !narrow_tiles(tile_rows(BM), a.n))) a.ksplit = 1;  // only few-tile launches carry a split
+    const auto go = [&](auto kernel, uint32_t rows, uint32_t tokens, uint32_t threads) {
+        a.row_tiles = (a.m + rows - 1) / rows;
+        a.tile_start[0] = a.tile_start[1] = UINT32_MAX;
+        for (uint32_t i = 0; i < more; i++) {
+            a.tile_start[i] = a.row_tiles;
+            a.row_tiles += (a.m_more[i] + rows - 1) / rows;
+        }
+        a.tok_tiles = (a.n + tokens - 1) / tokens;
+        const uint32_t shares = a.ksplit > 1 ? a.ksplit : 1u;
+        if ((uint64_t)a.row_tiles * a.tok_tiles * shares > 0x7fffff00ull) return hipErrorInvalidValue;  // beyond a launch's grid
+        // every XCD gets the same number of slots of the tile map; tile id = blockIdx.x / shares runs over all of them
+        const uint32_t grid = (a.row_tiles * a.tok_tiles + 7u) / 8u * 8u * shares;
+        hipError_t e = launch_kernel(L, kFamGemm, kernel, dim3(grid), dim3(threads), a);
+        if (e != hipSuccess || shares == 1 || defer_reduce) return e;  // deferred: the caller's next kernel adds the shares up itself
+        return launch_reduce(a, L);
+    };
+    // (The product kernels do not depend on the weight type: the copy they read is the same for both.  The parity hook's do.)
+    const bool q8 = DUMP && type != kTypeQ4_0;
+    const auto tile = [&](auto cfg) {
+        using C = decltype(cfg);
+        if constexpr (DUMP)
+            if (q8) return go(gemm_tile_kernel<8, true, false, C>, C::kRows, C::kTokens, C::kThreads);
+        return go(gemm_tile_kernel<2, DUMP, false, C>, C::kRows, C::kTokens, C::kThreads);
+    };
+    const bool narrow = !wide_split && narrow_tiles(tile_rows(BM), a.n);
+    if (narrow && (a.n <= 48 || L.gemm_mfma16)) {
         // a launch of at most 16 / 32 / 48 tokens computes one / two / three of the tile's four 16-token MFMA tiles (the parity
         // hook: all four).  These launches are bound by their block loop, not by memory: 65536 x 16 x 2048 40 -> 34 us.
-        const auto narrow_launch = [&](uint32_t grid) {
-            if constexpr (!DUMP) {
-                if (a.n <= 16) return launch_kernel(L, kFamGemm, gemm_narrow_kernel<2, false, 1>, dim3(grid), dim3(THREADS), a);
-                if (a.n <= 32) return launch_kernel(L, kFamGemm, gemm_narrow_kernel<2, false, 2>, dim3(grid), dim3(THREADS), a);
-                if (a.n <= 48) return launch_kernel(L, kFamGemm, gemm_narrow_kernel<2, false, 3>, dim3(grid), dim3(THREADS), a);
-            }
-            // (the product kernels do not depend on the weight type any more: the copy they read is the same for both)
-            if (!L.gemm_mfma16 && a.n > 48)
-                return type == kTypeQ4_0 ? launch_kernel(L, kFamGemm, gemm_narrow32_kernel<2, DUMP>, dim3(grid), dim3(THREADS), a)
-                                         : launch_kernel(L, kFamGemm, gemm_narrow32_kernel<8, DUMP>, dim3(grid), dim3(THREADS), a);
-            return type == kTypeQ4_0 ? launch_kernel(L, kFamGemm, gemm_narrow_kernel<2, DUMP>, dim3(grid), dim3(THREADS), a)
-                                     : launch_kernel(L, kFamGemm, gemm_narrow_kernel<8, DUMP>, dim3(grid), dim3(THREADS), a);
-        };
-        if (!DUMP && a.ksplit > 1) {
-            // tile id = blockIdx.x / ksplit must run over all `blocks` slots of the tile map
-            hipError_t e = narrow_launch(blocks * a.ksplit);
-            if (e != hipSuccess || defer_reduce) return e;  // deferred: the caller's next kernel adds the shares up itself
-            return launch_reduce(a, L);
+        if constexpr (!DUMP) {
+            if (a.n <= 16) return go(gemm_narrow_kernel<2, false, 1>, BM, BN_NARROW, THREADS);
+            if (a.n <= 32) return go(gemm_narrow_kernel<2, false, 2>, BM, BN_NARROW, THREADS);
+            if (a.n <= 48) return go(gemm_narrow_kernel<2, false, 3>, BM, BN_NARROW, THREADS);
         }
-        return narrow_launch(blocks);
+        if constexpr (DUMP)
+            if (q8) return go(gemm_narrow_kernel<8, true>, BM, BN_NARROW, THREADS);
+        return go(gemm_narrow_kernel<2, DUMP>, BM, BN_NARROW, THREADS);
     }
-    if (wide_split) {
-        hipError_t e = !L.gemm_mfma16
-                           ? (type == kTypeQ4_0 ? launch_kernel(L, kFamGemm, gemm_mfma32_kernel<2, DUMP>, dim3(blocks * a.ksplit), dim3(THREADS), a)
-                                                : launch_kernel(L, kFamGemm, gemm_mfma32_kernel<8, DUMP>, dim3(blocks * a.ksplit), dim3(THREADS), a))
-                           : (type == kTypeQ4_0 ? launch_kernel(L, kFamGemm, gemm_mfma_kernel<2, DUMP>, dim3(blocks * a.ksplit), dim3(THREADS), a)
-                                                : launch_kernel(L, kFamGemm, gemm_mfma_kernel<8, DUMP>, dim3(blocks * a.ksplit), dim3(THREADS), a));
-        if (e != hipSuccess || defer_reduce) return e;
-        return launch_reduce(a, L);
+    if (L.gemm_mfma16) {
+        if constexpr (DUMP)
+            if (q8) return go(gemm_mfma_kernel<8, true>, BM, BN, THREADS);
+        return go(gemm_mfma_kernel<2, DUMP>, BM, BN, THREADS);
     }
-    a.ksplit = 1;  // an unsplit launch of the wide kernel
-    if (!L.gemm_mfma16) {
-        if (type == kTypeQ4_0) return launch_kernel(L, kFamGemm, gemm_mfma32_kernel<2, DUMP>, dim3(blocks), dim3(THREADS), a);
-        return launch_kernel(L, kFamGemm, gemm_mfma32_kernel<8, DUMP>, dim3(blocks), dim3(THREADS), a);
-    }
-    if (type == kTypeQ4_0)
-        return launch_kernel(L, kFamGemm, gemm_mfma_kernel<2, DUMP>, dim3(blocks), dim3(THREADS), a);
-    return launch_kernel(L, kFamGemm, gemm_mfma_kernel<8, DUMP>, dim3(blocks), dim3(THREADS), a);
+    if (wide_split) return tile(TileM{});
+    const uint64_t small = tile_rows(BM) * ((a.n + BN_NARROW - 1) / BN_NARROW) * (a.ksplit > 1 ? a.ksplit : 1u);
+    if (narrow && small <= 256) return tile(TileN{});  // (1024 x 1024 over 555 tokens 10.9 us on TileS, 10.6 here; 512 tiles: 27 / 29.5)
+    if (a.n <= BN_NARROW || a.ksplit > 1) return tile(TileS{});
+    const auto cost = [&](auto cfg) { return tile_cost<decltype(cfg)>(tile_rows(decltype(cfg)::kRows), a.n, a.k); };
+    return cheapest_tile(cost, tile);
 }
 
 }  // namespace
@@ -1311,20 +1322,25 @@ bool gemm_gated_applies(uint32_t m, uint32_t n, uint32_t k) {
     return m % 32u == 0 && k % 128u == 0 && n > BN_NARROW && (uint64_t)((m + 63u) / 64u) * ((n + BN - 1) / BN) > 256u;
 }
 
-hipError_t launch_gemm_mfma_gated(int type, const uint8_t* d_w_gate, const uint8_t* d_w_up, uint32_t m, uint32_t k, const int8_t* d_q,
+hipError_t launch_gemm_mfma_gated(int /*type: the copies are the same for both*/, const uint8_t* d_w_gate, const uint8_t* d_w_up, uint32_t m, uint32_t k, const int8_t* d_q,
                                   const float* d_scales, uint32_t n, int8_t* d_out_q, float* d_out_scales, const Launch& L) {
     if (m == 0 || n == 0) return hipSuccess;
     if (!gemm_gated_applies(m, n, k)) return hipErrorInvalidValue;
     GemmArgs a{};
     a.w = d_w_gate, a.w_up = d_w_up, a.xq = d_q, a.xs = d_scales, a.q_out = d_out_q, a.s_out = d_out_scales;
     a.m = m, a.n = n, a.k = k;
-    a.row_tiles = (m + 63u) / 64u;
-    a.tok_tiles = (n + BN - 1) / BN;
     a.tile_start[0] = a.tile_start[1] = UINT32_MAX;
-    if ((uint64_t)a.row_tiles * a.tok_tiles > 0x7fffff00ull) return hipErrorInvalidValue;
-    const uint32_t blocks = ((a.row_tiles * a.tok_tiles + 7u) / 8u) * 8u;
-    if (type == kTypeQ4_0) return launch_kernel(L, kFamGemm, gemm_mfma_kernel<2, false, true>, dim3(blocks), dim3(THREADS), a);
-    return launch_kernel(L, kFamGemm, gemm_mfma_kernel<8, false, true>, dim3(blocks), dim3(THREADS), a);
+    const auto tile = [&](auto cfg) {
+        using C = decltype(cfg);
+        a.row_tiles = (m + C::kRows / 2 - 1) / (C::kRows / 2), a.tok_tiles = (n + C::kTokens - 1) / C::kTokens;
+        if ((uint64_t)a.row_tiles * a.tok_tiles > 0x7fffff00ull) return hipErrorInvalidValue;
+        return launch_kernel(L, kFamGemm, gemm_tile_kernel<2, false, true, C>, dim3((a.row_tiles * a.tok_tiles + 7u) / 8u * 8u), dim3(C::kThreads), a);
+    };
+    const auto cost = [&](auto cfg) {
+        using C = decltype(cfg);
+        return tile_cost<C>((m + C::kRows / 2 - 1) / (C::kRows / 2), n, k, true);
+    };
+    return cheapest_tile(cost, tile);
 }
 
 // Parity hook through the matrix-core path: the same loads, unpack, LDS layout and

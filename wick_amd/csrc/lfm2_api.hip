@@ -623,11 +623,9 @@ int enqueue_prompt_pass(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, uint32_t n, uint3
         // the out projection's input: already Q8_0 blocks when its producer wrote them itself
         if (!quantized && (rc = wick_rocm_quantize_q8_0(ctx, m->pG, n, hs, hs, m->pQ, m->pS))) break;
         if ((rc = project_and_norm(L.n_kv == 0 ? L.out_proj : L.o, m->pQ, m->pS, L.ffn_norm))) break;  // hidden += out projection; FFN norm
-        if (L.gate->type == kTypeQ4_0 && L.gate->k <= 1024 && wick_rocm_ffn_gate_up_silu_quantize_applies(L.gate, L.up, n)) {
+        if (wick_rocm_ffn_gate_up_silu_quantize_applies(L.gate, L.up, n)) {
             // gate, up, SiLU gate and the down projection's quantizer in one launch; its output cannot overwrite its own input.
-            // (Where it pays, measured on one GPU against GEMM + gate kernel: Q4_0 with k = 1024 6-7 % faster; k = 2048 2-8 %
-            // slower -- the epilogue's exp / divide work sits on the vector ALU that bounds the GEMM; Q8_0, whose kernel is
-            // two registers over its budget, 11 % slower.)
+            // (Against GEMM + gate kernel: 4608 x 1024 over 2048 tokens 75 -> 68 us, over 555 32 -> 26; 6912 x 2048 over 2002 174 -> 159.)
             if ((rc = wick_rocm_ffn_gate_up_silu_quantize_q8(ctx, L.gate, L.up, m->pQ, m->pS, n, m->pQ2, m->pS2))) break;
             rc = next_norm ? project_and_norm(L.down, m->pQ2, m->pS2, next_norm)
                            : wick_rocm_gemm_q8(ctx, L.down, m->pQ2, m->pS2, n, m->pX, hs, WICK_ROCM_LAYOUT_TOKEN_MAJOR, 1);

@@ -244,7 +244,11 @@ __device__ __forceinline__ unsigned long long argmax_key(float f, uint32_t index
 __device__ __forceinline__ float bits_f(uint32_t u) { return __uint_as_float(u); }
 
 // ggml_expf (wick/src/backend/cpu.rs:604-652), operation for operation: bit-exact.
-__device__ __forceinline__ float ggml_expf(float x) {
+struct GgmlExp {
+    float n, j, k;
+    uint32_t e;
+};
+__device__ __forceinline__ GgmlExp ggml_expf_parts(float x) {
     const float R = bits_f(0x4B400000u), LOG2E = bits_f(0x3FB8AA3Bu);
     const float LN2_HI = bits_f(0x3F317200u), LN2_LO = bits_f(0x35BFBE8Eu);
     const float C1 = bits_f(0x3F7FFFF6u), C2 = bits_f(0x3EFFFEDBu), C3 = bits_f(0x3E2AAF33u);
@@ -257,13 +261,23 @@ __device__ __forceinline__ float ggml_expf(float x) {
     const float u = __fmul_rn(b, b);
     const float inner = __fadd_rn(__fadd_rn(C2, __fmul_rn(C3, b)), __fmul_rn(__fadd_rn(C4, __fmul_rn(C5, b)), u));
     const float j = __fadd_rn(__fmul_rn(C1, b), __fmul_rn(inner, u));
-    const float abs_n = fabsf(n);
-    if (abs_n <= 126.0f) return __fadd_rn(k, __fmul_rn(j, k));
-    if (abs_n > 192.0f) return n > 0.0f ? __builtin_inff() : 0.0f;
-    const uint32_t d = n <= 0.0f ? 0x82000000u : 0u;
+    return {n, j, k, e};
+}
+__device__ __forceinline__ float ggml_expf(float x) {
+    const GgmlExp p = ggml_expf_parts(x);
+    const float abs_n = fabsf(p.n);
+    if (abs_n <= 126.0f) return __fadd_rn(p.k, __fmul_rn(p.j, p.k));
+    if (abs_n > 192.0f) return p.n > 0.0f ? __builtin_inff() : 0.0f;
+    const uint32_t d = p.n <= 0.0f ? 0x82000000u : 0u;
     const float s1 = bits_f(d + 0x7f000000u);
-    const float s2 = bits_f(e - d);
-    return __fmul_rn(__fadd_rn(s2, __fmul_rn(s2, j)), s1);
+    const float s2 = bits_f(p.e - d);
+    return __fmul_rn(__fadd_rn(s2, __fmul_rn(s2, p.j)), s1);
+}
+// Its first branch alone: the value where |n| <= 126.  For code that takes many of them and branches once on the largest |n|.
+__device__ __forceinline__ float ggml_expf_near(float x, float& n) {
+    const GgmlExp p = ggml_expf_parts(x);
+    n = p.n;
+    return __fadd_rn(p.k, __fmul_rn(p.j, p.k));
 }
 
 // silu_mul_inplace's element (wick/src/backend/cpu.rs:668-673): g / (1 + expf(-g)) * u, bit-exact.
