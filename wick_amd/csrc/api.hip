@@ -5,11 +5,14 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
 #include <new>
 #include <string>
+#include <thread>
+#include <vector>
 
 #include "wick_rocm_ctx.h"
 #include "../../include/wick_gguf.h"
@@ -48,6 +51,30 @@ void noalloc_release(wick_rocm_ctx* ctx) {
     if (ctx->device < 0 || ctx->device >= kNoallocMaxDevices) return;
     std::lock_guard<std::mutex> lk(g_noalloc_mu);
     if (g_noalloc_owner[ctx->device] == ctx) g_noalloc_owner[ctx->device] = nullptr;
+}
+
+void free_stage(wick_rocm_ctx* ctx) {
+    for (hipEvent_t& e : ctx->stage_ev)
+        if (e) (void)hipEventDestroy(e), e = nullptr;
+    if (ctx->stage) (void)hipHostFree(ctx->stage);
+    ctx->stage = nullptr, ctx->stage_slots = 0;
+}
+
+// At least `slots` staging slots: two serve small copies, a context that never makes a large one pins 4 MB only.
+bool make_stage(wick_rocm_ctx* ctx, int slots) {
+    if (ctx->stage_slots >= slots) return true;
+    free_stage(ctx);  // (every copy has waited: nothing is in flight)
+    void* p = nullptr;
+    bool ok = hipHostMalloc(&p, slots * kStageSlotBytes, hipHostMallocDefault) == hipSuccess;
+    ctx->stage = static_cast<char*>(p);
+    for (int i = 0; ok && slots > 2 && i < slots; i++) ok = hipEventCreateWithFlags(&ctx->stage_ev[i], hipEventDisableTiming) == hipSuccess;
+    if (!ok) {
+        (void)hipGetLastError();
+        free_stage(ctx);
+        return false;
+    }
+    ctx->stage_slots = slots;
+    return true;
 }
 
 int check_weight(wick_rocm_ctx* ctx, const wick_rocm_weight* w) {
@@ -134,6 +161,91 @@ int gemm_locked(wick_rocm_ctx* ctx, const wick_rocm_weight* w, const int8_t* d_q
 
 }  // namespace
 
+// Host memory of the callers is pageable, and the runtime's own way with it costs 110 us for 256 KB of logits and 5 - 30 GB/s for
+// large copies (one thread, first-touch page faults included).  Through pinned slots: 12 us + 6 us of memcpy for the logits; a large
+// copy is dealt out to several threads that each fill or empty one slot while their other one is on the bus (2 MB pieces keep the bus
+// at 46 - 50 of its 57 GB/s; eight threads fault in and fill fresh pages at 57 GB/s, one at 5 - 15).
+int copy_pieces(wick_rocm_ctx* ctx, const HostPiece* pieces, size_t count, bool to_host) {
+    size_t total = 0;
+    for (size_t i = 0; i < count; i++) total += pieces[i].bytes;
+    if (total == 0) return WICK_ROCM_OK;
+    const auto issue = [&](char* dev, char* host, size_t n) {
+        return to_host ? hipMemcpyAsync(host, dev, n, hipMemcpyDeviceToHost, ctx->stream) : hipMemcpyAsync(dev, host, n, hipMemcpyHostToDevice, ctx->stream);
+    };
+    if (!make_stage(ctx, total <= 2 * kStageSlotBytes ? 2 : kStageSlots)) {  // no pinned memory left: the runtime's way
+        for (size_t i = 0; i < count; i++) WR_HIP(ctx, issue(static_cast<char*>(pieces[i].dev), static_cast<char*>(pieces[i].host), pieces[i].bytes));
+        WR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        return WICK_ROCM_OK;
+    }
+    if (total <= 2 * kStageSlotBytes) {  // small: all pieces side by side in the staging memory, one wait
+        size_t at = 0;
+        for (size_t i = 0; i < count; i++) {
+            if (!to_host) std::memcpy(ctx->stage + at, pieces[i].host, pieces[i].bytes);
+            WR_HIP(ctx, issue(static_cast<char*>(pieces[i].dev), ctx->stage + at, pieces[i].bytes));
+            at += pieces[i].bytes;
+        }
+        WR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        at = 0;
+        for (size_t i = 0; to_host && i < count; i++) {
+            std::memcpy(pieces[i].host, ctx->stage + at, pieces[i].bytes);
+            at += pieces[i].bytes;
+        }
+        return WICK_ROCM_OK;
+    }
+    std::vector<HostPiece> chunks;
+    chunks.reserve(total / kStageSlotBytes + count);
+    for (size_t i = 0; i < count; i++)
+        for (size_t o = 0; o < pieces[i].bytes; o += kStageSlotBytes)
+            chunks.push_back({static_cast<char*>(pieces[i].dev) + o, static_cast<char*>(pieces[i].host) + o,
+                              pieces[i].bytes - o < kStageSlotBytes ? pieces[i].bytes - o : kStageSlotBytes});
+    std::atomic<size_t> next{0};
+    std::atomic<int> failed{(int)hipSuccess};
+    const auto work = [&](int w) {
+        const auto ok = [&](hipError_t e) {
+            int none = (int)hipSuccess;
+            if (e != hipSuccess) failed.compare_exchange_strong(none, (int)e);
+            return e == hipSuccess;
+        };
+        if (!ok(hipSetDevice(ctx->device))) return;
+        size_t busy[2];  // the chunk on its way in each of this worker's slots
+        bool has[2] = {false, false};
+        const auto settle = [&](int k) {
+            if (!has[k]) return true;
+            has[k] = false;
+            if (!ok(hipEventSynchronize(ctx->stage_ev[2 * w + k]))) return false;
+            if (to_host) std::memcpy(chunks[busy[k]].host, ctx->stage + (2 * w + k) * kStageSlotBytes, chunks[busy[k]].bytes);
+            return true;
+        };
+        for (int k = 0; failed.load(std::memory_order_relaxed) == (int)hipSuccess; k ^= 1) {
+            const size_t i = next.fetch_add(1, std::memory_order_relaxed);
+            if (i >= chunks.size()) break;
+            if (!settle(k)) return;
+            char* slot = ctx->stage + (2 * w + k) * kStageSlotBytes;
+            if (!to_host) std::memcpy(slot, chunks[i].host, chunks[i].bytes);
+            if (!ok(issue(static_cast<char*>(chunks[i].dev), slot, chunks[i].bytes)) || !ok(hipEventRecord(ctx->stage_ev[2 * w + k], ctx->stream))) return;
+            busy[k] = i, has[k] = true;
+        }
+        settle(0), settle(1);
+    };
+    const unsigned cores = std::thread::hardware_concurrency();
+    size_t workers = cores >= 2 * kStageWorkers ? kStageWorkers : (cores > 3 ? cores / 2 : 1);
+    if (workers > (chunks.size() + 1) / 2) workers = (chunks.size() + 1) / 2;
+    std::vector<std::thread> threads;
+    for (size_t w = 1; w < workers; w++) {
+        try {
+            threads.emplace_back(work, (int)w);
+        } catch (...) {  // no thread to be had: those that run share the rest
+            break;
+        }
+    }
+    work(0);
+    for (std::thread& t : threads) t.join();
+    const hipError_t e = (hipError_t)failed.load(), drained = hipStreamSynchronize(ctx->stream);  // after an error too: the slots are free again
+    if (e != hipSuccess) return fail_hip(ctx, e, "host copy");
+    if (drained != hipSuccess) return fail_hip(ctx, drained, "host copy");
+    return WICK_ROCM_OK;
+}
+
 extern "C" {
 
 const char* wick_rocm_version(void) { return "wick-rocm 0.1 (gfx950)"; }
@@ -195,6 +307,7 @@ void wick_rocm_ctx_destroy(wick_rocm_ctx* ctx) {
         if (ctx->scratch_s) (void)hipFree(ctx->scratch_s);
         if (ctx->scratch_f) (void)hipFree(ctx->scratch_f);
         if (ctx->argmax_partial) (void)hipFree(ctx->argmax_partial);
+        free_stage(ctx);
         for (auto* v : {&ctx->timer.recs, &ctx->timer.spares})
             for (KernelTimer::Rec& r : *v) {
                 (void)hipEventDestroy(r.start);
@@ -245,9 +358,8 @@ int wick_rocm_upload(wick_rocm_ctx* ctx, void* d_dst, const void* src, size_t nb
     if (nbytes == 0) return WICK_ROCM_OK;
     if (!d_dst || !src) return fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "upload: null pointer");
     if (ctx->capturing) return fail(ctx, WICK_ROCM_ERR_STATE, "upload during graph capture");
-    WR_HIP(ctx, hipMemcpyAsync(d_dst, src, nbytes, hipMemcpyHostToDevice, ctx->stream));
-    WR_HIP(ctx, hipStreamSynchronize(ctx->stream));  // the host buffer may be reused on return
-    return WICK_ROCM_OK;
+    const HostPiece p{d_dst, const_cast<void*>(src), nbytes};
+    return copy_pieces(ctx, &p, 1, false);  // waits: the host buffer may be reused on return
 }
 
 int wick_rocm_download(wick_rocm_ctx* ctx, void* dst, const void* d_src, size_t nbytes) {
@@ -255,8 +367,8 @@ int wick_rocm_download(wick_rocm_ctx* ctx, void* dst, const void* d_src, size_t 
     if (nbytes == 0) return WICK_ROCM_OK;
     if (!dst || !d_src) return fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "download: null pointer");
     if (ctx->capturing) return fail(ctx, WICK_ROCM_ERR_STATE, "download during graph capture");
-    WR_HIP(ctx, hipMemcpyAsync(dst, d_src, nbytes, hipMemcpyDeviceToHost, ctx->stream));
-    WR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    const HostPiece p{const_cast<void*>(d_src), dst, nbytes};
+    if (int rc = copy_pieces(ctx, &p, 1, true)) return rc;
     noalloc_release(ctx);
     return WICK_ROCM_OK;
 }
@@ -326,7 +438,14 @@ int wick_rocm_weight_upload(wick_rocm_ctx* ctx, const void* host_blocks, size_t 
     if (!w) return fail(ctx, WICK_ROCM_ERR_HIP, "out of host memory");
     // (+64: the Q6_K kernel reads its last 16-byte piece whole)
     hipError_t e = hipMalloc(&w->d, nbytes + 64);
-    if (e == hipSuccess) e = hipMemcpyAsync(w->d, host_blocks, nbytes, hipMemcpyHostToDevice, ctx->stream);
+    if (e == hipSuccess) {
+        const HostPiece p{w->d, const_cast<void*>(host_blocks), nbytes};
+        if (int rc = copy_pieces(ctx, &p, 1, false)) {
+            (void)hipFree(w->d);
+            delete w;
+            return rc;
+        }
+    }
     // The prefill GEMM reads its own layout of the weight (see gemm.hip): made here, once, on the device.  Weights the GEMM does
     // not take (Q6_K, k % 128 != 0) or uploaded with packing switched off keep the raw blocks only and run as GEMVs for any n.
     if (e == hipSuccess && ctx->gemm_packing && ggml_type != kTypeQ6_K && k % 128u == 0) {

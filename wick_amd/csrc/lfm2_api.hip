@@ -354,7 +354,9 @@ struct wick_rocm_lfm2 {
     uint32_t prefill_cap = 0;
     float *pX = nullptr, *pA = nullptr, *pG = nullptr, *pGate = nullptr, *pUp = nullptr, *pS = nullptr, *pS2 = nullptr, *pAttn = nullptr;
     int8_t *pQ = nullptr, *pQ2 = nullptr;
-    uint32_t* pTokens = nullptr;
+    uint32_t* h_tokens = nullptr;    // pinned: a prompt's tokens, read by the embedding lookup where they are (max_seq_len)
+    float* conv_states = nullptr;    // the gated-conv layers' rolling states
+    size_t conv_floats = 0;
     void* shift_stage = nullptr;   // staging rows of a context shift, allocated by the first one
     bool kv_f16 = false;           // the KV caches hold f16 rows (wick_rocm_lfm2_load_kv); f32 otherwise
     size_t kv_elem() const { return kv_f16 ? 2 : 4; }
@@ -419,6 +421,7 @@ void release(wick_rocm_ctx* ctx, wick_rocm_lfm2* m) {
         if (g) wick_rocm_graph_destroy(ctx, g);
     for (wick_rocm_weight* w : m->weights) wick_rocm_weight_free(ctx, w);
     for (void* b : m->buffers) wick_rocm_buffer_free(ctx, b);
+    if (m->h_tokens) (void)hipHostFree(m->h_tokens);
     delete m;
 }
 
@@ -533,8 +536,7 @@ int ensure_prefill_buffers(wick_rocm_ctx* ctx, wick_rocm_lfm2* m) {
         (rc = alloc_t(ctx, m, P * hs, &m->pG)) || (rc = alloc_t(ctx, m, P * inter, &m->pGate)) || (rc = alloc_t(ctx, m, P * inter, &m->pUp)) ||
         (rc = alloc_t(ctx, m, P * wide, &m->pQ)) || (rc = alloc_t(ctx, m, P * (wide / 32), &m->pS)) ||
         (rc = alloc_t(ctx, m, P * inter, &m->pQ2)) || (rc = alloc_t(ctx, m, P * (inter / 32), &m->pS2)) ||
-        (rc = alloc_t(ctx, m, attention_prefill_scratch_floats((uint32_t)P, c.n_heads, (uint32_t)hd), &m->pAttn)) ||
-        (rc = alloc_t(ctx, m, P, &m->pTokens)))
+        (rc = alloc_t(ctx, m, attention_prefill_scratch_floats((uint32_t)P, c.n_heads, (uint32_t)hd), &m->pAttn)))
         return rc;
     // room for the K shares of a split projection, once: no prompt then regrows the context's scratch (a regrow waits for the
     // stream and makes every captured step graph stale)
@@ -560,11 +562,11 @@ int gemm_group(wick_rocm_ctx* ctx, std::initializer_list<const wick_rocm_weight*
     return WICK_ROCM_OK;
 }
 
-// One pass of a prompt: n <= prefill_cap tokens (already in pTokens) at positions pos0 .. pos0 + n - 1.  The batched form
+// One pass of a prompt: n <= prefill_cap tokens (device-readable; null: their rows are in pX already) at positions pos0 .. pos0 + n - 1.  The batched form
 // of enqueue_step (prefill_layers_and_logits, wick/src/model/lfm2.rs:1139-2109): projections as GEMMs over the tokens,
 // the short conv per (token, channel) with the rolling state behind it, the KV append per token, causal attention per
 // (head, token).
-int enqueue_prompt_pass(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, uint32_t n, uint32_t pos0, bool lookup = true) {
+int enqueue_prompt_pass(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, uint32_t n, uint32_t pos0, const uint32_t* tokens) {
     const wick_rocm_lfm2_config& c = m->cfg;
     const uint32_t hs = c.hidden_size, hd = hs / c.n_heads, inter = c.intermediate_size;
     const float scale = 1.0f / sqrtf((float)hd);
@@ -574,8 +576,8 @@ int enqueue_prompt_pass(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, uint32_t n, uint3
         return e == hipSuccess ? WICK_ROCM_OK : fail_hip(ctx, e, what);
     };
     // the pass's input rows: the tokens' embedding rows, or what the caller put into pX (a prompt given as embeddings)
-    int rc = !lookup ? WICK_ROCM_OK
-                     : locked([&] { return launch_embed_rows(static_cast<const uint8_t*>(m->embd->d), m->embd->type, m->embd->m, hs, m->pTokens, n, m->pX, ctx->launch()); },
+    int rc = !tokens ? WICK_ROCM_OK
+                     : locked([&] { return launch_embed_rows(static_cast<const uint8_t*>(m->embd->d), m->embd->type, m->embd->m, hs, tokens, n, m->pX, ctx->launch()); },
                               "embed_rows launch");
     // A residual projection and the norm + quantizer behind it go out as one call (a split projection's shares are then added
     // up by the norm's kernel): the out projection with the FFN norm, the down projection with the NEXT layer's first norm.
@@ -668,6 +670,19 @@ int for_each_state_piece(const wick_rocm_lfm2* model, uint32_t seq_len, F&& piec
     return WICK_ROCM_OK;
 }
 
+// The state of seq_len positions to or from `host`, all pieces in one copy.
+int copy_state(wick_rocm_ctx* ctx, const wick_rocm_lfm2* model, uint32_t seq_len, uint8_t* host, bool to_host) {
+    WR_ENTER(ctx);
+    if (ctx->capturing) return fail(ctx, WICK_ROCM_ERR_STATE, to_host ? "download during graph capture" : "upload during graph capture");
+    std::vector<HostPiece> pieces;
+    for_each_state_piece(model, seq_len, [&](void* d, size_t n) {
+        pieces.push_back({d, host, n});
+        host += n;
+        return WICK_ROCM_OK;
+    });
+    return copy_pieces(ctx, pieces.data(), pieces.size(), to_host);
+}
+
 }  // namespace
 
 extern "C" {
@@ -726,6 +741,11 @@ int wick_rocm_lfm2_load_kv(wick_rocm_ctx* ctx, const wick_gguf* g, uint32_t cont
     };
     m->layers.resize(c.n_layers);
     int rc = 0;
+    // the layers' rolling conv states in one piece (each on its own 256 bytes): a reset clears them in one launch
+    const size_t conv_floats = ((size_t)(c.conv_kernel_size - 1) * hs + 63) / 64 * 64;
+    size_t n_conv = 0;
+    m->conv_floats = conv_floats * c.n_layers;
+    if (conv_floats && (rc = alloc_t(ctx, m, m->conv_floats, &m->conv_states))) return bail(rc);
     // block types from tensor presence, wick/src/model/lfm2.rs:151-170
     for (uint32_t i = 0; i < c.n_layers; i++) {
         const std::string p = "blk." + std::to_string(i) + ".";
@@ -755,7 +775,7 @@ int wick_rocm_lfm2_load_kv(wick_rocm_ctx* ctx, const wick_gguf* g, uint32_t cont
             if ((rc = upload_f32(ctx, m, g, p + "shortconv.conv.weight", (uint64_t)hs * c.conv_kernel_size, &L.conv_w))) return bail(rc);
             if ((rc = upload_weight(ctx, m, g, p + "shortconv.in_proj.weight", 3 * hs, hs, &L.in_proj))) return bail(rc);
             if ((rc = upload_weight(ctx, m, g, p + "shortconv.out_proj.weight", hs, hs, &L.out_proj))) return bail(rc);
-            if (c.conv_kernel_size > 1 && (rc = alloc_t(ctx, m, (size_t)(c.conv_kernel_size - 1) * hs, &L.conv_state))) return bail(rc);
+            if (c.conv_kernel_size > 1) L.conv_state = m->conv_states + n_conv++ * conv_floats;
         }
         if ((rc = upload_weight(ctx, m, g, p + "ffn_gate.weight", inter, hs, &L.gate))) return bail(rc);
         if ((rc = upload_weight(ctx, m, g, p + "ffn_up.weight", inter, hs, &L.up))) return bail(rc);
@@ -817,13 +837,10 @@ int wick_rocm_lfm2_reset(wick_rocm_ctx* ctx, wick_rocm_lfm2* model) {
     if (!ctx || !model) return WICK_ROCM_ERR_INVALID_ARG;
     std::lock_guard<std::mutex> lk(model->mu);
     std::lock_guard<std::recursive_mutex> whole_step(ctx->mu);  // nothing else gets onto the context's stream (or into a capture) in between
-    const size_t state_floats = (size_t)(model->cfg.conv_kernel_size - 1) * model->cfg.hidden_size;
-    if (state_floats) {
-        const std::vector<float> zeros(state_floats, 0.0f);
-        for (const LayerWeights& L : model->layers)
-            if (L.conv_state)
-                if (int rc = wick_rocm_upload(ctx, L.conv_state, zeros.data(), state_floats * sizeof(float))) return rc;
-    }
+    if (ctx->capturing) return fail(ctx, WICK_ROCM_ERR_STATE, "lfm2_reset during graph capture");
+    Guard device(ctx);
+    const hipError_t e = launch_fill_zero(model->conv_states, model->conv_floats, ctx->launch());  // in stream order, like the steps around it
+    if (e != hipSuccess) return fail_hip(ctx, e, "reset launch");
     return WICK_ROCM_OK;
 }
 
@@ -872,11 +889,15 @@ static int prefill_locked(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, const uint3
     for (uint32_t done = 0; done < n; done += model->prefill_cap) {
         last = n - done < model->prefill_cap ? n - done : model->prefill_cap;
         if (tokens) {
-            if (int rc = wick_rocm_upload(ctx, model->pTokens, tokens + done, (size_t)last * sizeof(uint32_t))) return rc;
+            if (!model->h_tokens) {
+                Guard device(ctx);
+                WR_HIP(ctx, hipHostMalloc(reinterpret_cast<void**>(&model->h_tokens), (size_t)c.max_seq_len * sizeof(uint32_t), hipHostMallocDefault));
+            }
+            memcpy(model->h_tokens + done, tokens + done, (size_t)last * sizeof(uint32_t));  // (the previous prompt's call has waited for its passes)
         } else {  // frame j of the prompt is row j of the pass's input (wick/src/model/lfm2.rs:2452-2487)
             if (int rc = wick_rocm_upload(ctx, model->pX, embeddings + (size_t)done * c.hidden_size, (size_t)last * c.hidden_size * sizeof(float))) return rc;
         }
-        if (int rc = enqueue_prompt_pass(ctx, model, last, start_pos + done, tokens != nullptr)) return rc;
+        if (int rc = enqueue_prompt_pass(ctx, model, last, start_pos + done, tokens ? model->h_tokens + done : nullptr)) return rc;
     }
     // output norm + tied LM head on the last token only (wick/src/model/lfm2.rs:2080-2109)
     const float* h_last = model->pX + (size_t)(last - 1) * c.hidden_size;
@@ -1006,12 +1027,7 @@ int wick_rocm_lfm2_snapshot_state(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uin
     if (seq_len > model->cfg.max_seq_len) return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2 snapshot: seq_len beyond the context size");
     if (nbytes != wick_rocm_lfm2_state_bytes(model, seq_len) || (!out && nbytes))
         return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2 snapshot: the buffer must hold exactly wick_rocm_lfm2_state_bytes(model, seq_len) bytes");
-    uint8_t* at = static_cast<uint8_t*>(out);
-    return for_each_state_piece(model, seq_len, [&](const void* d, size_t n) {
-        const int rc = wick_rocm_download(ctx, at, d, n);
-        at += n;
-        return rc;
-    });
+    return copy_state(ctx, model, seq_len, static_cast<uint8_t*>(out), true);
 }
 
 int wick_rocm_lfm2_restore_state(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uint32_t seq_len, const void* in, size_t nbytes) {
@@ -1021,12 +1037,7 @@ int wick_rocm_lfm2_restore_state(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uint
     if (seq_len > model->cfg.max_seq_len) return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2 restore: seq_len beyond the context size");
     if (nbytes != wick_rocm_lfm2_state_bytes(model, seq_len) || (!in && nbytes))
         return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2 restore: the snapshot must hold exactly wick_rocm_lfm2_state_bytes(model, seq_len) bytes");
-    const uint8_t* at = static_cast<const uint8_t*>(in);
-    return for_each_state_piece(model, seq_len, [&](void* d, size_t n) {
-        const int rc = wick_rocm_upload(ctx, d, at, n);
-        at += n;
-        return rc;
-    });
+    return copy_state(ctx, model, seq_len, static_cast<uint8_t*>(const_cast<void*>(in)), false);
 }
 
 int wick_rocm_lfm2_shift_kv(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uint32_t seq_len, uint32_t n_keep, uint32_t shift) {
@@ -1039,14 +1050,22 @@ int wick_rocm_lfm2_shift_kv(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uint32_t 
         return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2 shift_kv: shift range out of bounds (n_keep + shift > seq_len)");
     if (seq_len - n_keep - shift == 0) return WICK_ROCM_OK;  // nothing behind the dropped rows: only the caller's seq_len changes
     const uint32_t hd = c.hidden_size / c.n_heads;
-    if (!model->shift_stage && c.n_kv_heads)
+    std::vector<KvShiftLayer> layers;  // conv layers keep their rolling buffer (wick/src/kv_cache.rs:584-590)
+    for (const LayerWeights& L : model->layers)
+        if (L.n_kv) layers.push_back({L.k_cache, L.v_cache, L.n_kv});
+    if (layers.empty()) return WICK_ROCM_OK;
+    const bool in_place = hd % 8u == 0 && kv_shift_in_place_applies(seq_len, n_keep, shift);
+    if (!in_place && !model->shift_stage)
         if (int rc = alloc(ctx, model, 2 * (size_t)c.max_seq_len * c.n_kv_heads * hd * model->kv_elem(), &model->shift_stage)) return rc;
-    for (const LayerWeights& L : model->layers)  // conv layers keep their rolling buffer (wick/src/kv_cache.rs:584-590)
-        if (L.n_kv) {
-            const hipError_t e = launch_kv_shift(L.k_cache, L.v_cache, model->shift_stage, seq_len, n_keep, shift, L.n_kv, hd, model->theta_scale,
-                                                 ctx->launch(), model->kv_f16);
-            if (e != hipSuccess) return fail_hip(ctx, e, "kv_shift launch");
-        }
+    hipError_t e = hipSuccess;
+    if (in_place) {
+        e = launch_kv_shift_in_place(layers.data(), (uint32_t)layers.size(), seq_len, n_keep, shift, hd, model->theta_scale, ctx->launch(), model->kv_f16);
+    } else {
+        for (size_t i = 0; e == hipSuccess && i < layers.size(); i++)
+            e = launch_kv_shift(layers[i].k_cache, layers[i].v_cache, model->shift_stage, seq_len, n_keep, shift, layers[i].n_kv_heads, hd,
+                                model->theta_scale, ctx->launch(), model->kv_f16);
+    }
+    if (e != hipSuccess) return fail_hip(ctx, e, "kv_shift launch");
     return wick_rocm_sync(ctx);
 }
 

@@ -298,6 +298,57 @@ __global__ __launch_bounds__(256) void kv_shift_stage_kernel(KvShiftArgs a) {
     }
 }
 
+// The same rows moved in place, for up to kShiftLayers layers of one launch (blockIdx.y): rows [dst0, dst0 + rows) receive the rows
+// `shift` further on, rows <= shift, so no row is both read and written.  Bound by HBM: one read and one write of what moves, where
+// staging and copying back makes two of each and three launches per layer (2136 rows of 512 keys and values, six layers: 320 us
+// staged, 3 launches of ~10 us here).  Four elements per lane: the pairs of a head are (i, i + half).
+constexpr uint32_t kShiftLayers = 16;
+struct KvShiftInPlaceArgs {
+    KvShiftLayer layer[kShiftLayers];
+    uint32_t dst0, rows, shift, head_dim;
+    float theta_scale;
+};
+template <typename KV>
+__device__ __forceinline__ void kv_store4(KV* p, float4 v) {
+    if constexpr (std::is_same<KV, float>::value) {
+        *reinterpret_cast<float4*>(p) = v;
+    } else {
+        const kv_h4 h = {(_Float16)v.x, (_Float16)v.y, (_Float16)v.z, (_Float16)v.w};
+        *reinterpret_cast<kv_h4*>(p) = h;
+    }
+}
+template <typename KV>
+__global__ __launch_bounds__(256) void kv_shift_in_place_kernel(KvShiftInPlaceArgs a) {
+    __shared__ __align__(16) float sn_tab[kRopeTableMax], cs_tab[kRopeTableMax];
+    const KvShiftLayer l = a.layer[blockIdx.y];
+    const uint32_t hd = a.head_dim, half = hd >> 1, kv_dim = l.n_kv_heads * hd;
+    for (uint32_t i = threadIdx.x; i < half; i += 256) {
+        float theta = -(float)a.shift;
+        for (uint32_t j = 0; j < i; j++) theta = __fmul_rn(theta, a.theta_scale);
+        sincosf(theta, &sn_tab[i], &cs_tab[i]);
+    }
+    __syncthreads();
+    const uint32_t r0 = a.dst0 + blockIdx.x * kShiftRows, r1 = min(r0 + kShiftRows, a.dst0 + a.rows);
+    KV* const k = static_cast<KV*>(l.k_cache);
+    KV* const v = static_cast<KV*>(l.v_cache);
+    const uint32_t q = half >> 2, per_row = l.n_kv_heads * q;  // quads of pairs of a head / a row (head_dim % 8 == 0)
+    for (uint32_t e = threadIdx.x; e < (r1 - r0) * per_row; e += 256) {
+        const uint32_t row = r0 + e / per_row, w = e % per_row, i = 4u * (w % q), at = (w / q) * hd + i;
+        const size_t src = (size_t)(row + a.shift) * kv_dim + at, dst = (size_t)row * kv_dim + at;
+        const float4 x0 = kv_load4(k + src), x1 = kv_load4(k + src + half), y0 = kv_load4(v + src), y1 = kv_load4(v + src + half);
+        const float4 sn = *reinterpret_cast<const float4*>(&sn_tab[i]), cs = *reinterpret_cast<const float4*>(&cs_tab[i]);
+        kv_store4(k + dst, make_float4(__fsub_rn(__fmul_rn(x0.x, cs.x), __fmul_rn(x1.x, sn.x)), __fsub_rn(__fmul_rn(x0.y, cs.y), __fmul_rn(x1.y, sn.y)),
+                                       __fsub_rn(__fmul_rn(x0.z, cs.z), __fmul_rn(x1.z, sn.z)), __fsub_rn(__fmul_rn(x0.w, cs.w), __fmul_rn(x1.w, sn.w))));
+        kv_store4(k + dst + half, make_float4(__fadd_rn(__fmul_rn(x0.x, sn.x), __fmul_rn(x1.x, cs.x)), __fadd_rn(__fmul_rn(x0.y, sn.y), __fmul_rn(x1.y, cs.y)),
+                                              __fadd_rn(__fmul_rn(x0.z, sn.z), __fmul_rn(x1.z, cs.z)), __fadd_rn(__fmul_rn(x0.w, sn.w), __fmul_rn(x1.w, cs.w))));
+        kv_store4(v + dst, y0), kv_store4(v + dst + half, y1);
+    }
+}
+
+__global__ __launch_bounds__(256) void fill_zero_kernel(float* d, size_t n) {
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) d[i] = 0.0f;
+}
+
 // ---- decode attention -----------------------------------------------------------------
 // forward_attn_block's tail (wick/src/model/lfm2.rs:984-1006) = attn_scores -> softmax_inplace -> attn_values
 // (cpu.rs:1346-1355, 715-731, 1391-1401), one 256-thread block per query head over positions [0, seq_len).
@@ -1449,6 +1500,36 @@ hipError_t launch_kv_shift(void* d_k_cache, void* d_v_cache, void* d_stage, uint
     e = hipMemcpyAsync(static_cast<uint8_t*>(d_k_cache) + (size_t)n_keep * kv_dim * esize, a.k_stage, elems * esize, hipMemcpyDeviceToDevice, L.stream);
     if (e != hipSuccess) return e;
     return hipMemcpyAsync(static_cast<uint8_t*>(d_v_cache) + (size_t)n_keep * kv_dim * esize, a.v_stage, elems * esize, hipMemcpyDeviceToDevice, L.stream);
+}
+
+// A launch costs about what moving 100 rows of six layers does; staging costs three launches per layer and the rows twice over.
+constexpr uint32_t kShiftMaxSteps = 16;
+bool kv_shift_in_place_applies(uint32_t seq_len, uint32_t n_keep, uint32_t shift) {
+    return shift != 0 && (uint64_t)n_keep + shift < seq_len && (seq_len - n_keep - shift + shift - 1) / shift <= kShiftMaxSteps;
+}
+hipError_t launch_kv_shift_in_place(const KvShiftLayer* layers, uint32_t n_layers, uint32_t seq_len, uint32_t n_keep, uint32_t shift, uint32_t head_dim,
+                                    float theta_scale, const Launch& L, bool kv_f16) {
+    if (head_dim % 8u != 0 || !kv_shift_in_place_applies(seq_len, n_keep, shift)) return hipErrorInvalidValue;
+    const uint32_t end = seq_len - shift;  // rows [n_keep, end) are written
+    for (uint32_t l0 = 0; l0 < n_layers; l0 += kShiftLayers) {
+        KvShiftInPlaceArgs a{};
+        const uint32_t n = n_layers - l0 < kShiftLayers ? n_layers - l0 : kShiftLayers;
+        for (uint32_t i = 0; i < n; i++) a.layer[i] = layers[l0 + i];
+        a.shift = shift, a.head_dim = head_dim, a.theta_scale = theta_scale;
+        for (a.dst0 = n_keep; a.dst0 < end; a.dst0 += shift) {
+            a.rows = end - a.dst0 < shift ? end - a.dst0 : shift;
+            hipError_t e = with_kv_type(kv_f16, [&](auto kv) {
+                return launch_kernel(L, kFamOther, kv_shift_in_place_kernel<decltype(kv)>, dim3((a.rows + kShiftRows - 1) / kShiftRows, n), dim3(256), a);
+            });
+            if (e != hipSuccess) return e;
+        }
+    }
+    return hipSuccess;
+}
+
+hipError_t launch_fill_zero(float* d, size_t n, const Launch& L) {
+    if (n == 0) return hipSuccess;
+    return launch_kernel(L, kFamOther, fill_zero_kernel, dim3((uint32_t)(n < 64u * 256u ? (n + 255) / 256 : 64)), dim3(256), d, n);
 }
 
 hipError_t launch_attention_decode(const float* d_q, const void* d_k_cache, const void* d_v_cache, float* d_out, float* d_scores,

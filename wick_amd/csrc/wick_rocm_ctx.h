@@ -10,6 +10,10 @@
 
 using namespace wick_rocm;
 
+constexpr int kStageWorkers = 8;                     // most host threads a large copy uses
+constexpr int kStageSlots = 2 * kStageWorkers;       // a worker copies one slot while the other is on its way
+constexpr size_t kStageSlotBytes = 2u << 20;
+
 struct wick_rocm_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -46,6 +50,10 @@ struct wick_rocm_ctx {
     int64_t gemv_direct_max_bytes = -1;
     bool gemm_mfma16 = false;  // wick_rocm_set_gemm_mfma_shape(ctx, 16)
     unsigned long long* argmax_partial = nullptr;  // kArgmaxPartials keys for wick_rocm_argmax
+    // Pinned staging of host <-> device copies (copy_pieces), made by the first one: 2 or kStageSlots slots of kStageSlotBytes.
+    char* stage = nullptr;
+    int stage_slots = 0;
+    hipEvent_t stage_ev[kStageSlots] = {};
     Launch launch() { return Launch{stream, &timer, gemv_direct_max_bytes, gemm_mfma16}; }
 };
 
@@ -95,6 +103,15 @@ inline int fail_hip(wick_rocm_ctx* ctx, hipError_t e, const char* where) {
         hipError_t e_ = (call);                                \
         if (e_ != hipSuccess) return fail_hip(ctx, e_, #call); \
     } while (0)
+
+// One piece of a copy between device and (pageable) host memory.
+struct HostPiece {
+    void* dev;
+    void* host;
+    size_t bytes;
+};
+// Copies the pieces in stream order and waits (lock held, not capturing).  api.hip.
+int copy_pieces(wick_rocm_ctx* ctx, const HostPiece* pieces, size_t count, bool to_host);
 
 // Takes the context lock and makes its device current for the calling thread.
 struct Guard {

@@ -175,6 +175,17 @@ hipError_t launch_qk_norm_rope(float* d_q, float* d_k, const float* d_v, const f
 // 2 * (seq_len - n_keep - shift) * n_kv_heads * head_dim cache elements.
 hipError_t launch_kv_shift(void* d_k_cache, void* d_v_cache, void* d_stage, uint32_t seq_len, uint32_t n_keep, uint32_t shift,
                            uint32_t n_kv_heads, uint32_t head_dim, float theta_scale, const Launch& L, bool kv_f16 = false);
+// The same without a staging buffer, for several layers at once: the kept rows move down `shift` rows at a time, so that source and
+// destination of one launch never overlap.  Applies where that takes few launches.
+struct KvShiftLayer {
+    void* k_cache;
+    void* v_cache;
+    uint32_t n_kv_heads;
+};
+bool kv_shift_in_place_applies(uint32_t seq_len, uint32_t n_keep, uint32_t shift);
+hipError_t launch_kv_shift_in_place(const KvShiftLayer* layers, uint32_t n_layers, uint32_t seq_len, uint32_t n_keep, uint32_t shift, uint32_t head_dim,
+                                    float theta_scale, const Launch& L, bool kv_f16 = false);
+hipError_t launch_fill_zero(float* d, size_t n, const Launch& L);
 // A prompt of n tokens at once (token j at position pos + j): embedding rows [n][k], the short conv of every (token, channel), causal attention over caches that already hold the prompt's K / V rows (head_dim 32 / 64 / 128 / 256;
 // scratch: attention_prefill_scratch_floats).
 hipError_t launch_embed_rows(const uint8_t* d_w, int type, uint32_t m, uint32_t k, const uint32_t* d_tokens, uint32_t n, float* d_out,
