@@ -53,6 +53,20 @@ void noalloc_release(wick_rocm_ctx* ctx) {
     if (g_noalloc_owner[ctx->device] == ctx) g_noalloc_owner[ctx->device] = nullptr;
 }
 
+// A chunk between device memory and a pinned slot (either may be the source), 16-byte aligned, n pieces of 16 bytes.
+__global__ __launch_bounds__(256) void stage_copy_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, uint32_t n) {
+    const uint32_t step = gridDim.x * 256u;
+    for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n; i += 4u * step) {
+        uint4 v[4];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++)
+            if (i + j * step < n) v[j] = src[i + j * step];
+#pragma unroll
+        for (uint32_t j = 0; j < 4; j++)
+            if (i + j * step < n) dst[i + j * step] = v[j];
+    }
+}
+
 void free_stage(wick_rocm_ctx* ctx) {
     for (hipEvent_t& e : ctx->stage_ev)
         if (e) (void)hipEventDestroy(e), e = nullptr;
@@ -161,10 +175,11 @@ int gemm_locked(wick_rocm_ctx* ctx, const wick_rocm_weight* w, const int8_t* d_q
 
 }  // namespace
 
-// Host memory of the callers is pageable, and the runtime's own way with it costs 110 us for 256 KB of logits and 5 - 30 GB/s for
-// large copies (one thread, first-touch page faults included).  Through pinned slots: 12 us + 6 us of memcpy for the logits; a large
-// copy is dealt out to several threads that each fill or empty one slot while their other one is on the bus (2 MB pieces keep the bus
-// at 46 - 50 of its 57 GB/s; eight threads fault in and fill fresh pages at 57 GB/s, one at 5 - 15).
+// Host memory of the callers is pageable, and large copies the runtime's way run at 5 - 30 GB/s (one thread, first-touch page faults
+// included).  Here a large copy is dealt out to several threads that each fill or empty one pinned slot while their other one is on the
+// bus (57 GB/s); one thread faults in and fills fresh pages at 5 - 15 GB/s, eight at 57.  2 MB slots and six threads: 74 MB up in
+// 1.78 ms, 54 MB down in 1.5 (touched) - 1.8 ms (fresh); 1 MB slots 2.0 / 1.6, eight threads no faster.  A copy of up to two slots
+// goes through one of them, all pieces together, with one wait.
 int copy_pieces(wick_rocm_ctx* ctx, const HostPiece* pieces, size_t count, bool to_host) {
     size_t total = 0;
     for (size_t i = 0; i < count; i++) total += pieces[i].bytes;
@@ -198,6 +213,13 @@ int copy_pieces(wick_rocm_ctx* ctx, const HostPiece* pieces, size_t count, bool 
         for (size_t o = 0; o < pieces[i].bytes; o += kStageSlotBytes)
             chunks.push_back({static_cast<char*>(pieces[i].dev) + o, static_cast<char*>(pieces[i].host) + o,
                               pieces[i].bytes - o < kStageSlotBytes ? pieces[i].bytes - o : kStageSlotBytes});
+    // The chunks go over the bus in a kernel: a copy engine's transfers and the events between them wait for each other across queues
+    // (2 MB chunks with an event behind each: 30 - 35 GB/s by copy engine, ~48 by kernel).
+    const auto issue_chunk = [&](char* dev, char* host, size_t n) {
+        if (reinterpret_cast<uintptr_t>(dev) % 16u != 0 || n % 16u != 0) return issue(dev, host, n);
+        return launch_kernel(Launch{ctx->stream, nullptr}, kFamOther, stage_copy_kernel, dim3(64), dim3(256), reinterpret_cast<const uint4*>(to_host ? dev : host),
+                             reinterpret_cast<uint4*>(to_host ? host : dev), (uint32_t)(n / 16u));
+    };
     std::atomic<size_t> next{0};
     std::atomic<int> failed{(int)hipSuccess};
     const auto work = [&](int w) {
@@ -222,7 +244,7 @@ int copy_pieces(wick_rocm_ctx* ctx, const HostPiece* pieces, size_t count, bool 
             if (!settle(k)) return;
             char* slot = ctx->stage + (2 * w + k) * kStageSlotBytes;
             if (!to_host) std::memcpy(slot, chunks[i].host, chunks[i].bytes);
-            if (!ok(issue(static_cast<char*>(chunks[i].dev), slot, chunks[i].bytes)) || !ok(hipEventRecord(ctx->stage_ev[2 * w + k], ctx->stream))) return;
+            if (!ok(issue_chunk(static_cast<char*>(chunks[i].dev), slot, chunks[i].bytes)) || !ok(hipEventRecord(ctx->stage_ev[2 * w + k], ctx->stream))) return;
             busy[k] = i, has[k] = true;
         }
         settle(0), settle(1);

@@ -10,7 +10,7 @@
 
 using namespace wick_rocm;
 
-constexpr int kStageWorkers = 8;                     // most host threads a large copy uses
+constexpr int kStageWorkers = 6;                     // most host threads a large copy uses
 constexpr int kStageSlots = 2 * kStageWorkers;       // a worker copies one slot while the other is on its way
 constexpr size_t kStageSlotBytes = 2u << 20;
 
