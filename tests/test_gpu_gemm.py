@@ -418,3 +418,33 @@ def test_prompt_tiles_against_the_gemv_route(ctx, oracle, m, n, k):
         finally:
             ctx.set_gemm_min_n(0)
         assert rel_l2(out[W.LAYOUT_TOKEN_MAJOR, False], fetch_gemm(d_y, m, n, m, W.LAYOUT_TOKEN_MAJOR)) < 1e-6
+
+
+@pytest.mark.parametrize("dtype", [W.Q4_0, W.Q8_0])
+@pytest.mark.parametrize("m,n,k", [(33, 9, 128), (32, 32, 1024), (100, 33, 1152), (64, 64, 4608), (1000, 31, 6912), (2080, 37, 1664)])
+def test_few_token_launches(ctx, oracle, dtype, m, n, k):
+    """Granule-per-workgroup launches at their edges: one row past a granule, one / two token groups full and one short, fewer slabs
+    than waves, slabs that do not deal out evenly over waves and shares; split over K with the shares added inside the launch (repeated:
+    the arrival counters must be back at zero) and unsplit; both layouts, accumulate, block dots."""
+    with Problem(ctx, oracle, dtype, m, k, n, seed=m + 3 * n + k + dtype) as p:
+        ref = oracle.gemm_q8(dtype, p.wb, p.s, p.q, m, n, k)
+        first = {}
+        for splits in (0, 1, 0, 2, 8, 0):
+            ctx.set_gemm_max_k_splits(splits)
+            try:
+                for layout, stride in ((W.LAYOUT_ROW_MAJOR, n + 3), (W.LAYOUT_TOKEN_MAJOR, m + 5)):
+                    rows = m if layout == W.LAYOUT_ROW_MAJOR else n
+                    d_y = p.to_device(np.full(rows * stride, 2.5, np.float32))
+                    ctx.gemm_preq(p.w, p.d_s, p.d_q, n, d_y, y_stride=stride, layout=layout)
+                    y = fetch_gemm(d_y, m, n, stride, layout).copy()
+                    assert_f32_parity(y, ref, f"few {dtype} {m}x{n}x{k} splits {splits} layout {layout}")
+                    assert np.array_equal(y, first.setdefault(splits, y))  # same bits in either layout and every time
+                    full = d_y.download(np.float32, rows * stride).reshape(rows, stride)
+                    assert np.all(full[:, n if layout == W.LAYOUT_ROW_MAJOR else m:] == 2.5)
+                    ctx.gemm_preq(p.w, p.d_s, p.d_q, n, d_y, y_stride=stride, layout=layout, accumulate=True)
+                    assert np.array_equal(fetch_gemm(d_y, m, n, stride, layout), y + y)
+            finally:
+                ctx.set_gemm_max_k_splits(0)
+        d_d = p.alloc(n * m * (k // 32) * 4)
+        ctx.block_dots_i32(p.w, p.d_q, n, d_d)
+        assert np.array_equal(d_d.download(np.int32, n * m * (k // 32)).reshape(n, m, k // 32), oracle.block_dots_i32(dtype, p.wb, p.q, m, n, k))

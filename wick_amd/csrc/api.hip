@@ -157,14 +157,15 @@ int gemm_locked(wick_rocm_ctx* ctx, const wick_rocm_weight* w, const int8_t* d_q
     hipError_t e;
     if (n >= ctx->min_n_for(w->nbytes) && mfma_ok) {
         uint32_t splits = may_split && ctx->gemm_max_splits > 1 ? gemm_split_k(w->m, n, w->k, ctx->gemm_max_splits) : 1u;
-        if (splits > 1) {
+        const bool in_launch = !ctx->gemm_mfma16 && gemm_split_in_launch(w->m, n, w->k);  // needs no scratch
+        if (splits > 1 && !in_launch) {
             const size_t floats = (size_t)splits * n * w->m;
             if (ctx->capturing && floats > ctx->scratch_f_cap) splits = 1;  // no room reserved: the unsplit launch, same result to the f32 bar
             else if (int rc = ensure_scratch(ctx, 0, 0, floats)) return rc;
         }
-        const bool defer = deferred && splits > 1;
+        const bool defer = deferred && splits > 1 && !in_launch;
         e = launch_gemm_mfma(w->type, static_cast<const uint8_t*>(w->d_gemm), w->m, w->k, d_q, d_s, n, d_y, y_stride,
-                             y_layout, accumulate, ctx->launch(), splits, splits > 1 ? ctx->scratch_f : nullptr, defer);
+                             y_layout, accumulate, ctx->launch(), splits, splits > 1 && !in_launch ? ctx->scratch_f : nullptr, defer);
         if (defer && e == hipSuccess) *deferred = splits;
     } else
         e = launch_gemv_tokens(w->type, static_cast<const uint8_t*>(w->d), w->m, w->k, d_q, d_s, n, d_y, y_stride,

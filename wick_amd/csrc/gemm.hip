@@ -1117,6 +1117,139 @@ __global__ __launch_bounds__(THREADS, 4) void gemm_narrow_kernel(GemmArgs a) {
     }
 }
 
+// ---------------------------------------------------------------------------------------
+// Few tokens (n <= 64: a chat turn, the tail of a prompt).  Such a launch is one latency after the other: with 128-row tiles a
+// 1024-row projection occupied 8 to 64 CUs, and every stage of K cost a barrier and the block loop of a lone workgroup.  Here a
+// workgroup takes ONE granule of 32 rows x all tokens (TG groups of 32), and K in rounds of one slab per wave and token group:
+//   * a wave multiplies its slab -- operands straight from memory into registers, a slab is in operand order already -- and leaves
+//     v = isum * dw of every (block, row, token) in LDS;
+//   * then every thread walks its elements through the round's blocks in order, acc = fma(v, dx, acc): the one part of a row's sum
+//     that is sequential is two LDS reads and an FMA per block instead of a whole block loop, and the bits are those of the tiles.
+// The next round's operands are requested before the walk.  Shares of K (split_k_factor) are walked one after the other and added up in
+// the same order as elsewhere, in the same workgroup: no scratch and no second launch.
+// Measured back to back, 23 tokens: 1024 x 1024 split in 4 6.7 -> 4.9 us, 2048 x 1024 (Q | K | V) 8.8 -> 4.9, 9216 x 1024 (gate | up)
+// 9.1 -> 6.5.
+template <int TYPE, bool DUMP, int TG, int WV>
+__global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(GemmArgs a) {
+    constexpr int SL = WV / TG, NB = SL * KB;              // slabs and blocks of a round
+    constexpr int EP = 16 * TG / WV, TPR = 32 * TG / EP;   // elements (consecutive tokens of a row) per thread, threads per row
+    constexpr int kRow = 36;                               // floats of a row of 32 tokens: 16-byte aligned, rows spread over the banks
+    __shared__ __align__(16) float vs[NB * TG][GR][kRow];
+    __shared__ __align__(16) float dxs[NB][32 * TG];
+    const uint32_t shares = DUMP || a.ksplit < 2 ? 1u : a.ksplit;
+    if (blockIdx.x >= a.row_tiles) return;  // (grids are rounded up)
+    uint32_t granule = blockIdx.x;  // within the launch's weights
+    select_weight(a, granule);
+    const uint32_t lane = threadIdx.x & 63u, l32 = lane & 31u, kh = lane >> 5;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const uint32_t sl = wave / TG, tg = wave % TG;
+    const uint32_t nb = a.k >> 5, slabs = nb / KB;
+
+    struct Regs {
+        v4i w[KB], x[KB];
+        float2 dw[KB];
+        float4 dx;
+    };
+    const uint8_t* const slab0 = a.w + ((size_t)(granule >> 1) * slabs * 2 + (granule & 1u)) * kSlab;
+    const int8_t* const xbase = a.xq + (size_t)min(32u * tg + l32, a.n - 1u) * a.k + 16 * kh;
+    // token scales: thread t < 32 WV fetches the four of token t / SL and slab t % SL of the round
+    const uint32_t dtok = threadIdx.x / SL, dsl = threadIdx.x % SL;
+    const float* const sbase = DUMP ? nullptr : a.xs + (size_t)min(dtok, a.n - 1u) * nb;
+    const auto fetch = [&](uint32_t s0, Regs& r) {
+        const uint32_t s = s0 + sl;
+        if (s < slabs) {
+            const uint8_t* p = slab0 + (size_t)s * (2 * kSlab);
+#pragma unroll
+            for (int b = 0; b < KB; b++) {
+                r.w[b] = *reinterpret_cast<const v4i*>(p + 2048 * kh + 512 * b + 16 * l32);
+                r.x[b] = *reinterpret_cast<const v4i*>(xbase + (size_t)s * (32 * KB) + 32 * b);
+                r.dw[b] = *reinterpret_cast<const float2*>(p + kSlabWt + 256 * b + 8 * l32);
+            }
+        }
+        if (!DUMP && threadIdx.x < 32u * WV && s0 + dsl < slabs) r.dx = *reinterpret_cast<const float4*>(sbase + (s0 + dsl) * KB);
+    };
+
+    v16i cbias;
+#pragma unroll
+    for (int i = 0; i < 16; i++) cbias[i] = (int)kBiasBits;
+    asm volatile("" : "+v"(cbias));
+    const uint32_t row = threadIdx.x / TPR, tok0 = EP * (threadIdx.x % TPR);  // this thread's elements
+    float acc[EP], total[EP];
+#pragma unroll
+    for (int e = 0; e < EP; e++) acc[e] = total[e] = 0.0f;
+    uint32_t share = 0, share_end = slabs / shares;
+
+    Regs r{};
+    fetch(0, r);
+    for (uint32_t s0 = 0; s0 < slabs; s0 += SL) {
+        if (s0 + sl < slabs) {
+#pragma unroll
+            for (int b = 0; b < KB; b++) {
+                const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(r.x[b], r.w[b], cbias, 0, 0, 0);
+                if constexpr (DUMP) {
+#pragma unroll
+                    for (int e = 0; e < 16; e++) {
+                        const uint32_t rw = GR * granule + l32, t = 32u * tg + 4u * kh + 8u * (e >> 2) + (e & 3);
+                        if (rw < a.m && t < a.n) {
+                            int v = d[e] - (int)kBiasBits;
+                            if (TYPE == 2) v >>= 4;  // weights were stored x16; exact
+                            a.dots[((size_t)t * a.m + rw) * nb + (s0 + sl) * KB + b] = v;
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int g = 0; g < 4; g++) {
+                        v4f v;
+#pragma unroll
+                        for (int q = 0; q < 4; q++) v[q] = __builtin_fmaf(__int_as_float(d[4 * g + q]), r.dw[b].x, r.dw[b].y);
+                        *reinterpret_cast<v4f*>(&vs[(sl * KB + b) * TG + tg][l32][8 * g + 4 * kh]) = v;
+                    }
+                }
+            }
+        }
+        if constexpr (!DUMP) {
+            if (threadIdx.x < 32u * WV) {
+                dxs[KB * dsl][dtok] = r.dx.x, dxs[KB * dsl + 1][dtok] = r.dx.y;
+                dxs[KB * dsl + 2][dtok] = r.dx.z, dxs[KB * dsl + 3][dtok] = r.dx.w;
+            }
+            __syncthreads();
+        }
+        if (s0 + SL < slabs) fetch(s0 + SL, r);
+        if constexpr (!DUMP) {
+#pragma unroll
+            for (uint32_t q = 0; q < (uint32_t)SL; q++) {
+                if (s0 + q < slabs) {
+                    if (s0 + q == share_end) {  // the next share of K starts
+                        share++;
+                        share_end = (share + 1u) * slabs / shares;
+#pragma unroll
+                        for (int e = 0; e < EP; e++) total[e] = share == 1 ? acc[e] : total[e] + acc[e], acc[e] = 0.0f;
+                    }
+#pragma unroll
+                    for (int b = 0; b < KB; b++) {
+                        const float* const v = &vs[(q * KB + b) * TG + tok0 / 32][row][tok0 % 32];
+                        const float* const dx = &dxs[q * KB + b][tok0];
+#pragma unroll
+                        for (int e = 0; e < EP; e++) acc[e] = __builtin_fmaf(v[e], dx[e], acc[e]);
+                    }
+                }
+            }
+            if (s0 + SL < slabs) __syncthreads();  // the planes are written again
+        }
+    }
+    if constexpr (!DUMP) {
+#pragma unroll
+        for (int e = 0; e < EP; e++) {
+            const uint32_t rw = GR * granule + row, t = tok0 + e;
+            const float v = shares == 1 ? acc[e] : total[e] + acc[e];
+            if (rw < a.m && t < a.n) {
+                float* const y = a.y_row_major ? a.y + (size_t)rw * a.y_stride + t : a.y + (size_t)t * a.y_stride + rw;
+                *y = a.accumulate ? *y + v : v;
+            }
+        }
+    }
+}
+
 // y (+)= partial[0] + partial[1] + ... in that order, element by element (token-major partials [split][n][m]).
 // (S a template parameter: all of an element's loads are in flight together instead of one round trip per share.)
 template <int S>
@@ -1152,6 +1285,16 @@ uint32_t wide_split_factor(uint32_t m, uint32_t n, uint32_t k, uint32_t max_spli
 
 // Launches of few 128 x 128 tiles (at most one per CU): the ones that may be split over K.
 bool narrow_tiles(uint64_t row_tiles, uint32_t n) { return n <= BN_NARROW || row_tiles * ((n + BN - 1) / BN) <= 256; }
+
+// Launches of gemm_few_kernel: up to 64 tokens and few enough granules that latency and not the chip's throughput is what they cost
+// (every workgroup fetches all tokens' activations for its 32 rows; beyond, the 128-row tiles are the cheaper readers).  A round of K
+// takes it ~2 us, so a long K that the tiles may split into shares side by side stays with them.  Tiles / here, us:  unsplit 2048 x
+// 1024 over 23 tokens 8.8 / 4.9, 1024 x 4608 29 / 14; split 1024 x 1024 over 23 6.7 / 4.9, 9216 x 2048 12.1 / 10.1, 1024 x 4608
+// 8.9 / 14.3, 2048 x 2048 over 40 8.2 / 11.5; 65536 x 2048 over 16 27 / 40.
+bool few_applies(uint64_t rows, uint32_t n, uint32_t k, bool split) {
+    const uint64_t units = (rows + GR - 1) / GR, slabs = k / (KB * 32);
+    return n <= 64 && units <= 512 && units * slabs <= (n <= 32 ? 12288u : 4096u) && (!split || slabs <= (n <= 32 ? 16u : 8u));
+}
 
 uint32_t split_k_factor(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits) {
     const uint32_t ws = wide_split_factor(m, n, k, max_splits);
@@ -1214,7 +1357,7 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, uint32_t more = 0, boo
     };
     const bool wide_split = !DUMP && more == 0 && a.ksplit > 1 && wide_split_factor(a.m, a.n, a.k, a.ksplit) == a.ksplit;
     if (DUMP || (!wide_split && !narrow_tiles(tile_rows(BM), a.n))) a.ksplit = 1;  // only few-tile launches carry a split
-    const auto go = [&](auto kernel, uint32_t rows, uint32_t tokens, uint32_t threads) {
+    const auto go = [&](auto kernel, uint32_t rows, uint32_t tokens, uint32_t threads, bool whole = false) {
         a.row_tiles = (a.m + rows - 1) / rows;
         a.tile_start[0] = a.tile_start[1] = UINT32_MAX;
         for (uint32_t i = 0; i < more; i++) {
@@ -1225,9 +1368,9 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, uint32_t more = 0, boo
         const uint32_t shares = a.ksplit > 1 ? a.ksplit : 1u;
         if ((uint64_t)a.row_tiles * a.tok_tiles * shares > 0x7fffff00ull) return hipErrorInvalidValue;  // beyond a launch's grid
         // every XCD gets the same number of slots of the tile map; tile id = blockIdx.x / shares runs over all of them
-        const uint32_t grid = (a.row_tiles * a.tok_tiles + 7u) / 8u * 8u * shares;
+        const uint32_t grid = (a.row_tiles * a.tok_tiles + 7u) / 8u * 8u * (whole ? 1u : shares);  // whole: a workgroup takes all shares of its rows
         hipError_t e = launch_kernel(L, kFamGemm, kernel, dim3(grid), dim3(threads), a);
-        if (e != hipSuccess || shares == 1 || defer_reduce) return e;  // deferred: the caller's next kernel adds the shares up itself
+        if (e != hipSuccess || shares == 1 || defer_reduce || whole) return e;  // deferred: the caller's next kernel adds the shares up itself
         return launch_reduce(a, L);
     };
     // (The product kernels do not depend on the weight type: the copy they read is the same for both.  The parity hook's do.)
@@ -1238,7 +1381,18 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, uint32_t more = 0, boo
             if (q8) return go(gemm_tile_kernel<8, true, false, C>, C::kRows, C::kTokens, C::kThreads);
         return go(gemm_tile_kernel<2, DUMP, false, C>, C::kRows, C::kTokens, C::kThreads);
     };
-    const bool narrow = !wide_split && narrow_tiles(tile_rows(BM), a.n);
+    const bool few = !L.gemm_mfma16 && few_applies(GR * tile_rows(GR), a.n, a.k, a.ksplit > 1), narrow = !wide_split && narrow_tiles(tile_rows(BM), a.n);
+    if (few) {
+        // Eight waves and 151 KB of LDS while every CU gets one workgroup at most, else four and half of it.
+        const auto waves = [&](auto tg, auto wv) {
+            constexpr int TG = decltype(tg)::value, WV = decltype(wv)::value;
+            if constexpr (DUMP)
+                if (q8) return go(gemm_few_kernel<8, true, TG, WV>, GR, 64, 64 * WV, true);
+            return go(gemm_few_kernel<2, DUMP, TG, WV>, GR, 64, 64 * WV, true);
+        };
+        if (tile_rows(GR) <= 256) return a.n <= 32 ? waves(Idx<1>{}, Idx<8>{}) : waves(Idx<2>{}, Idx<8>{});
+        return a.n <= 32 ? waves(Idx<1>{}, Idx<4>{}) : waves(Idx<2>{}, Idx<4>{});
+    }
     if (narrow && (a.n <= 48 || L.gemm_mfma16)) {
         // a launch of at most 16 / 32 / 48 tokens computes one / two / three of the tile's four 16-token MFMA tiles (the parity
         // hook: all four).  These launches are bound by their block loop, not by memory: 65536 x 16 x 2048 40 -> 34 us.
@@ -1267,6 +1421,7 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, uint32_t more = 0, boo
 }  // namespace
 
 uint32_t gemm_split_k(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits) { return split_k_factor(m, n, k, max_splits); }
+bool gemm_split_in_launch(uint32_t m, uint32_t n, uint32_t k) { return few_applies(m, n, k, true); }
 
 // The GEMM's own copy of a weight (slabs, see StageT): its size, and the kernel that makes it from the raw blocks.
 size_t gemm_packed_bytes(uint32_t m, uint32_t k) { return (size_t)((m + 2 * GR - 1) / (2 * GR)) * 2 * ((k >> 5) / KB) * kSlab; }
@@ -1290,8 +1445,8 @@ hipError_t launch_gemm_mfma(int type, const uint8_t* d_w, uint32_t m, uint32_t k
     a.m = m, a.n = n, a.k = k, a.y_stride = y_stride;
     a.y_row_major = (y_layout == 1);
     a.accumulate = accumulate;
-    if (splits > 1 && d_partial) {
-        if (splits != split_k_factor(m, n, k, splits)) return hipErrorInvalidValue;  // the shape does not carry that split
+    if (splits > 1 && (d_partial || gemm_split_in_launch(m, n, k))) {
+        if (splits != split_k_factor(m, n, k, splits) || (defer_reduce && gemm_split_in_launch(m, n, k))) return hipErrorInvalidValue;  // the shape does not carry that split
         a.ksplit = splits, a.partial = d_partial;
     } else if (defer_reduce) {
         return hipErrorInvalidValue;  // nothing to defer on an unsplit launch
