@@ -6,6 +6,7 @@ import pytest
 import wick_amd as W
 from conftest import assert_f32_parity
 from gpu_util import Problem
+from wick_amd.lfm2 import Lfm2Ops
 
 pytestmark = pytest.mark.gpu
 
@@ -183,3 +184,27 @@ def test_block_dots_through_the_product_kernel_at_full_size(ctx, oracle, dtype):
         with pytest.raises(W.RocmError) as e:
             ctx.block_dots_f32_i32(p6.w, p6.d_q, p6.d_q)
         assert e.value.status == -2
+
+
+@pytest.mark.parametrize("dtype", [W.Q4_0, W.Q8_0])
+@pytest.mark.parametrize("k", [192, 1024, 1088, 2048, 2112, 3136, 4096, 4160, 5184, 7232, 8192])
+def test_fused_quantizer_at_the_edges_of_its_rounds(ctx, oracle, dtype, k):
+    """f32 activations normed (or gated) and quantized inside the launch, at the lengths where the prologue takes another round
+    of quads or the last round is nearly empty: bit for bit the separate norm / gate, quantizer and GEMV."""
+    ops, m, eps = Lfm2Ops(ctx), 70, float(np.float32(1e-5))
+    w = ctx.upload_weight(oracle.synth_weight(dtype, m, k, 5 + k), dtype, m, k)
+    x, nw, y0 = oracle.fill_normal(k, 1.0, k), 1 + 0.2 * oracle.fill_normal(k + 1, 1.0, k), oracle.fill_normal(k + 2, 1.0, m)
+    d_x, d_nw, d_n, d_q, d_s = ctx.to_device(x), ctx.to_device(nw), ctx.alloc(k * 4), ctx.alloc(k), ctx.alloc(k // 32 * 4)
+    d_a, d_b = ctx.to_device(y0), ctx.to_device(y0)
+    for fused, separate in ((lambda: ctx.encode_gemv_rmsnorm_fused([w], d_x, d_nw, eps, [d_a], accumulate=True), lambda: ops.encode_rmsnorm(d_x, d_nw, d_n, k, eps)),
+                            (lambda: ctx.encode_gemv_silu_mul(w, d_x, d_nw, d_a, accumulate=True), lambda: (d_n.upload(x), ops.silu_mul_inplace(d_n, d_nw, k))),
+                            (lambda: ctx.encode_gemv(w, d_x, 0, d_a, 0, accumulate=True), lambda: d_n.upload(x))):
+        d_a.upload(y0), d_b.upload(y0)
+        fused(), separate()
+        ctx.quantize_q8_0(d_n, 1, k, k, d_q, d_s)
+        ctx.gemv_with_preq(w, d_s, d_q, d_b, accumulate=True)
+        a, b = d_a.download(np.float32, m), d_b.download(np.float32, m)
+        assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    for b in (d_x, d_nw, d_n, d_q, d_s, d_a, d_b):
+        b.free()
+    w.free()

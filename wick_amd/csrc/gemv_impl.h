@@ -45,6 +45,7 @@ struct GemvArgs {
     const float* conv_proj;
     uint32_t conv_hidden, conv_kernel;
     float eps;          // RMSNorm epsilon
+    double inv_k;       // 1 / k
     int32_t* dots;      // parity hook (DUMP variants): raw i32 block dots, [token][row][block], instead of y
     int xform;          // kXformNone / kXformRmsNorm / kXformSiluMul (host-side selector of the kernel variant)
     int gated;          // host-side selector of the GATED variant: batch.w[0] = gate, batch.w[1] = up, y[0][r] = silu(gate_r) * up_r
@@ -69,7 +70,7 @@ struct ActRegs {
 // FUSEQ workgroups have four waves that quantize the activation vector together.
 constexpr int kFusedWaves = 4;
 constexpr int kFusedMaxK = 8192;
-constexpr int kConvMaxK = 2048;  // kXformShortConv: eight operands per quad instead of two
+constexpr int kConvMaxK = 2048;
 
 // How a lane gets its pair (MODE):
 //   kDirect    each lane loads its own 36 / 68 bytes (two / four 16-byte loads + one dword);
@@ -96,7 +97,7 @@ enum { kDirect = 0, kDirectNT = 1, kSpan = 2 };
 // launch of its own.
 
 // The leading scalar parameters repeat fields of `a` (x = a.xf for the fused variant, a.xq
-// otherwise; w0 / y0 / rows0 = weight 0 of the batch).  Passed on their own, at the front,
+// otherwise; w0 / rows0 = weight 0 of the batch; aux / aux2 = a.xaux / a.xaux2, the transform's operands).  Passed on their own, at the front,
 // they are the kernel arguments the hardware preloads into SGPRs at wave launch (the build
 // asks for that, -amdgpu-kernarg-preload-count): everything needed to issue the activation
 // and weight loads of a single-weight launch is there at the first instruction, instead of
@@ -115,10 +116,9 @@ enum { kDirect = 0, kDirectNT = 1, kSpan = 2 };
 // timestamps, wick/src/model/metal_lfm2.rs:3367-4116, for launches inside a graph replay, which carry no events).
 template <int TYPE, int LPR, int NCHUNK, int U, int NT, bool FUSEQ, bool MULTI, int MODE, int XF = kXformNone, bool GATED = false, bool DUMP = false,
           bool SPAN = false>
-__global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kernel(const void* p_x, const uint8_t* p_w0, float* p_y0,
-                                                                                  uint32_t p_k, uint32_t p_rows0,
-                                                                                  uint32_t p_rows_per_wave, uint32_t p_total_waves,
-                                                                                  int p_accumulate, GemvArgs a) {
+__global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kernel(const void* p_x, const uint8_t* p_w0, const float* p_aux,
+                                                                                  const float* p_aux2, uint32_t p_k, uint32_t p_rows0,
+                                                                                  uint32_t p_rows_per_wave, uint32_t p_total_waves, GemvArgs a) {
     static_assert(XF == kXformNone || FUSEQ, "activation transforms belong to the fused-quantizer variant");
     static_assert(!GATED || (FUSEQ && !MULTI && NT == 1 && U % 2 == 0), "the gated variant pairs lane slots");
     static_assert(!DUMP || (!MULTI && !GATED && XF == kXformNone), "the parity hook runs the plain single-weight variants");
@@ -139,8 +139,12 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
         FUSEQ ? blockIdx.x * kFusedWaves + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)) : blockIdx.x;
     // The f32 activations are requested first of all (fused variant): they need only two
     // scalars of the argument block, and everything below overlaps with their latency.
-    constexpr int kQuadRounds = XF == kXformShortConv ? kConvMaxK / 4 / (64 * kFusedWaves)  // 2: eight operands per quad
-                                                      : kFusedMaxK / 4 / (64 * kFusedWaves);  // 8
+    // A round: one quad of the vector per thread.  LPR and NCHUNK say how long the vector can be (64 LPR NCHUNK, and more than
+    // half of it), so their number is known here and only rounds past the middle need a test.  (With eight rounds and a test
+    // of each in every kernel a 1024-long vector -- one round -- took two dozen taken branches: in_proj of a decode step
+    // 2.25 -> 1.6 us from its first to its last instruction.)
+    constexpr int kQuadRounds = LPR * NCHUNK <= 16 ? 1 : LPR * NCHUNK / 16;
+    const auto past = [&](int i) { return i > kQuadRounds / 2 && (uint32_t)i * 64u * kFusedWaves >= (p_k >> 2); };
     float4 xv[FUSEQ ? kQuadRounds : 1];
     float4 av[XF != kXformNone && XF != kXformShortConv ? kQuadRounds : 1];  // the transform's second operand, same quads
     float4 cv[XF == kXformShortConv ? kQuadRounds : 1][7];  // conv operands: c, x', state 0, state 1, three quads of the kernel (xv holds b)
@@ -149,50 +153,33 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
 #pragma unroll
         for (int i = 0; i < kQuadRounds; i++) {
             const uint32_t quad = threadIdx.x + i * 64 * kFusedWaves;
-            // whole rounds past the end of the vector are skipped (uniform, one taken branch);
-            // within a round: clamped
-            if (i > 0 && i * 64 * kFusedWaves >= quads) break;
+            // whole rounds past the end of the vector are skipped; within a round: clamped
+            if (past(i)) break;
             xv[i] = reinterpret_cast<const float4*>(p_x)[min(quad, quads - 1)];
         }
         if constexpr (XF == kXformShortConv) {
-            const float4 *px = reinterpret_cast<const float4*>(p_x), *st = reinterpret_cast<const float4*>(a.xaux2),
-                         *cw = reinterpret_cast<const float4*>(a.xaux);
+            const float4 *px = reinterpret_cast<const float4*>(p_x), *st = reinterpret_cast<const float4*>(p_aux2),
+                         *cw = reinterpret_cast<const float4*>(p_aux);
 #pragma unroll
             for (int i = 0; i < kQuadRounds; i++) {
-                if (i > 0 && i * 64 * kFusedWaves >= quads) break;
+                if (past(i)) break;
                 const uint32_t quad = min(threadIdx.x + i * 64 * kFusedWaves, quads - 1);
                 cv[i][0] = px[quads + quad], cv[i][1] = px[2 * quads + quad];
                 cv[i][2] = st[quad], cv[i][3] = st[quads + quad];
                 cv[i][4] = cw[3 * quad], cv[i][5] = cw[3 * quad + 1], cv[i][6] = cw[3 * quad + 2];  // [channel][tap] of four channels
             }
         } else if constexpr (XF != kXformNone) {
-            const float4* aux = reinterpret_cast<const float4*>(a.xaux);
+            const float4* aux = reinterpret_cast<const float4*>(p_aux);
 #pragma unroll
             for (int i = 0; i < kQuadRounds; i++) {
                 const uint32_t quad = threadIdx.x + i * 64 * kFusedWaves;
-                if (i > 0 && i * 64 * kFusedWaves >= quads) break;
+                if (past(i)) break;
                 av[i] = aux[min(quad, quads - 1)];
             }
         }
         // keep the compiler from moving the weight loads in front of these
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
-    }
-
-    if constexpr (GATED) {
-        // Side job of the FFN's gate / up launch in a gated-conv layer: advance the layer's rolling conv state.  The out
-        // projection before this launch has read the old state; nothing reads it again before the next token.  One thread
-        // per four channels, slots ascending, exactly what shortconv_step_kernel does to the state.
-        if (a.conv_state != nullptr && blockIdx.x * (64u * kFusedWaves) < (a.conv_hidden >> 2)) {
-            const uint32_t cq = a.conv_hidden >> 2, d_conv = a.conv_kernel - 1;
-            const float4* pj = reinterpret_cast<const float4*>(a.conv_proj);
-            float4* st = reinterpret_cast<float4*>(a.conv_state);
-            for (uint32_t q = blockIdx.x * (64u * kFusedWaves) + threadIdx.x; q < cq; q += gridDim.x * (64u * kFusedWaves)) {  // any grid covers every channel
-                const float4 b = pj[q], x = pj[2 * cq + q];
-                for (uint32_t s_ = 1; s_ < d_conv; s_++) st[(size_t)(s_ - 1) * cq + q] = st[(size_t)s_ * cq + q];
-                st[(size_t)(d_conv - 1) * cq + q] = make_float4(__fmul_rn(b.x, x.x), __fmul_rn(b.y, x.y), __fmul_rn(b.z, x.z), __fmul_rn(b.w, x.w));
-            }
-        }
     }
 
     // Which weight of the batch this wave works on.  Every per-weight field is copied out of
@@ -202,7 +189,7 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
     // wave_end[] entries past the batch are UINT32_MAX (set_wave_ends).
     uint32_t widx = 0;
     const uint8_t* wbase = p_w0;
-    float* ybase = p_y0;
+    float* ybase = a.batch.y[0];
     uint32_t row_hi = p_rows0, row_lo = 0, wave_lo = 0;
     if constexpr (MULTI) {
         uint64_t w0 = (uint64_t)a.batch.w[0], w1 = (uint64_t)a.batch.w[1], w2 = (uint64_t)a.batch.w[2], w3 = (uint64_t)a.batch.w[3];
@@ -246,6 +233,9 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
     uint32_t span_tail[U][NCHUNK];  // kSpan: where the dword remainder of the span starts
     bool rvalid[U];
     uint32_t lrow[U];
+    // Decode launches that add to y ask for the old values with the weights instead of at the end, behind everything.
+    constexpr bool kEarlyY = NT == 1 && !GATED && !DUMP;
+    float yold[kEarlyY ? U : 1];
     __shared__ __align__(16) uint8_t span_lds[MODE == kSpan ? (FUSEQ ? kFusedWaves : 1) * 64 * PT::BYTES : 16];
     // Loads are unconditional (row and pair indices clamped into range) so that the number
     // of outstanding loads is known at every wait; a clamped load's data is neutralised by
@@ -291,6 +281,14 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
             }
         }
     };
+    auto issue_y = [&] {
+        if constexpr (kEarlyY) {
+            if (a.accumulate) {
+#pragma unroll
+                for (int u = 0; u < U; u++) yold[u] = ybase[min(lrow[u], rows - 1)];
+            }
+        }
+    };
     // kSpan: the span pieces in w[u][c] go through this wave's LDS slot and come back as
     // this lane's own pair (position rsel * ppr + sub of the span, or sub for a row chunk).
     auto own_pair = [&](uint32_t (&piece)[WREGS], uint32_t tail) {
@@ -313,12 +311,32 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
     //   1. (fused) this thread's share of the f32 activation vector,
     //   2. the weight loads of the first pass (the long pole, HBM),
     //   3. wait for (1) only, quantize into LDS, barrier -- all under the latency of (2).
-    __shared__ __align__(16) uint32_t fq[FUSEQ ? kFusedMaxK / 4 : 4];
-    __shared__ float fs[FUSEQ ? kFusedMaxK / 32 : 1];
+    __shared__ __align__(16) uint32_t fq[FUSEQ ? kQuadRounds * 64 * kFusedWaves : 4];
+    __shared__ __align__(16) float2 fs[FUSEQ ? kQuadRounds * 8 * kFusedWaves : 2];  // a block's scale and sum of quants
     issue_pass(wave_row0);
+    issue_y();
     if constexpr (FUSEQ) {
         asm volatile("" ::: "memory");
         __builtin_amdgcn_sched_barrier(0);
+    }
+
+    if constexpr (GATED) {
+        // Side job of the FFN's gate / up launch in a gated-conv layer: advance the layer's rolling conv state.  The out
+        // projection before this launch has read the old state; nothing reads it again before the next token.  One thread
+        // per four channels, slots ascending, exactly what shortconv_step_kernel does to the state.  A workgroup of its own,
+        // the last one, does it: in a workgroup with rows the loads and stores came before its own work and held the whole
+        // launch up (3.7 -> 2.6 us).
+        if (a.conv_state != nullptr && blockIdx.x == gridDim.x - 1u) {
+            const uint32_t cq = a.conv_hidden >> 2, d_conv = a.conv_kernel - 1;
+            const float4* pj = reinterpret_cast<const float4*>(a.conv_proj);
+            float4* st = reinterpret_cast<float4*>(a.conv_state);
+            for (uint32_t q = threadIdx.x; q < cq; q += blockDim.x) {
+                const float4 b = pj[q], x = pj[2 * cq + q];
+                for (uint32_t s_ = 1; s_ < d_conv; s_++) st[(size_t)(s_ - 1) * cq + q] = st[(size_t)s_ * cq + q];
+                st[(size_t)(d_conv - 1) * cq + q] = make_float4(__fmul_rn(b.x, x.x), __fmul_rn(b.y, x.y), __fmul_rn(b.z, x.z), __fmul_rn(b.w, x.w));
+            }
+            return;
+        }
     }
 
     // Fused variant: the workgroup quantizes the f32 activation vector ONCE, together,
@@ -329,7 +347,7 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
         if constexpr (XF == kXformSiluMul) {
 #pragma unroll
             for (int i = 0; i < kQuadRounds; i++) {
-                if (i * 64 * kFusedWaves < quads) {
+                if (!past(i)) {
                     xv[i].x = silu_mul(xv[i].x, av[i].x), xv[i].y = silu_mul(xv[i].y, av[i].y);
                     xv[i].z = silu_mul(xv[i].z, av[i].z), xv[i].w = silu_mul(xv[i].w, av[i].w);
                 }
@@ -339,7 +357,7 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
             // per channel, the operations and their order are shortconv_step_kernel's: bit-identical
 #pragma unroll
             for (int i = 0; i < kQuadRounds; i++) {
-                if (i * 64 * kFusedWaves < quads) {
+                if (!past(i)) {
                     const float w[12] = {cv[i][4].x, cv[i][4].y, cv[i][4].z, cv[i][4].w, cv[i][5].x, cv[i][5].y,
                                          cv[i][5].z, cv[i][5].w, cv[i][6].x, cv[i][6].y, cv[i][6].z, cv[i][6].w};
                     const float b[4] = {xv[i].x, xv[i].y, xv[i].z, xv[i].w}, c[4] = {cv[i][0].x, cv[i][0].y, cv[i][0].z, cv[i][0].w};
@@ -363,20 +381,19 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
             double part = 0.0;
 #pragma unroll
             for (int i = 0; i < kQuadRounds; i++) {
-                const uint32_t quad = threadIdx.x + i * 64 * kFusedWaves;
-                if (i * 64 * kFusedWaves < quads && quad < quads) {
-                    const double x0 = xv[i].x, x1 = xv[i].y, x2 = xv[i].z, x3 = xv[i].w;
-                    part += (x0 * x0 + x1 * x1) + (x2 * x2 + x3 * x3);
-                }
+                if (past(i)) break;
+                const double x0 = xv[i].x, x1 = xv[i].y, x2 = xv[i].z, x3 = xv[i].w;
+                const double p4 = (x0 * x0 + x1 * x1) + (x2 * x2 + x3 * x3);
+                part += threadIdx.x + i * 64 * kFusedWaves < quads ? p4 : 0.0;
             }
             part = wave_sum_f64(part);
             if (lane == 0) sq[threadIdx.x >> 6] = part;
             __syncthreads();
             const double total = (sq[0] + sq[1]) + (sq[2] + sq[3]);
-            const float inv_rms = (float)(1.0 / sqrt(total / (double)p_k + (double)a.eps));
+            const float inv_rms = rms_inverse(total, a.inv_k, a.eps);
 #pragma unroll
             for (int i = 0; i < kQuadRounds; i++) {
-                if (i * 64 * kFusedWaves < quads) {
+                if (!past(i)) {
                     xv[i].x = __fmul_rn(__fmul_rn(xv[i].x, inv_rms), av[i].x), xv[i].y = __fmul_rn(__fmul_rn(xv[i].y, inv_rms), av[i].y);
                     xv[i].z = __fmul_rn(__fmul_rn(xv[i].z, inv_rms), av[i].z), xv[i].w = __fmul_rn(__fmul_rn(xv[i].w, inv_rms), av[i].w);
                 }
@@ -385,15 +402,18 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
 #pragma unroll
         for (int i = 0; i < kQuadRounds; i++) {
             const uint32_t quad = threadIdx.x + i * 64 * kFusedWaves;
-            if (i * 64 * kFusedWaves < quads) {  // uniform: whole rounds only differ in their tail
+            if (!past(i)) {
                 const float4 v = xv[i];
                 float amax = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
                 amax = group_max8(amax);
                 float id;
                 const float scale = q8_scale_and_inverse(amax, id);
+                const uint32_t packed = q8_pack4(v.x, v.y, v.z, v.w, id);
+                int xsum = 0;
+                if constexpr (TYPE == 2) xsum = group_sum8_i32(__builtin_amdgcn_sdot4(0x01010101, (int)packed, 0, false));
                 if (quad < quads) {
-                    fq[quad] = q8_pack4(v.x, v.y, v.z, v.w, id);
-                    if ((quad & 7u) == 0) fs[quad >> 3] = scale;
+                    fq[quad] = packed;
+                    if ((quad & 7u) == 0) fs[quad >> 3] = make_float2(scale, __builtin_bit_cast(float, xsum));
                 }
             }
         }
@@ -411,17 +431,16 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
             const uint32_t tok = ok ? tok0 + t : 0;
             const uint32_t pp = ok ? p : 0;
             if constexpr (FUSEQ) {
-                // This lane's two blocks, from the copy the workgroup quantized into LDS.
+                // This lane's two blocks, from the copy the workgroup quantized into LDS (a pair out of range: scales of zero).
+                const float4 both = *reinterpret_cast<const float4*>(&fs[2 * pp]);
+                act[c].s[t][0] = ok ? both.x : 0.0f, act[c].sum[t][0] = __builtin_bit_cast(int, both.y);
+                act[c].s[t][1] = ok ? both.z : 0.0f, act[c].sum[t][1] = __builtin_bit_cast(int, both.w);
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
                     const uint4 lo = *reinterpret_cast<const uint4*>(&fq[pp * 16 + h * 8]);
                     const uint4 hi = *reinterpret_cast<const uint4*>(&fq[pp * 16 + h * 8 + 4]);
-                    act[c].q[t][h][0] = ok ? lo.x : 0, act[c].q[t][h][1] = ok ? lo.y : 0;
-                    act[c].q[t][h][2] = ok ? lo.z : 0, act[c].q[t][h][3] = ok ? lo.w : 0;
-                    act[c].q[t][h][4] = ok ? hi.x : 0, act[c].q[t][h][5] = ok ? hi.y : 0;
-                    act[c].q[t][h][6] = ok ? hi.z : 0, act[c].q[t][h][7] = ok ? hi.w : 0;
-                    act[c].sum[t][h] = (TYPE == 2) ? block_xsum(act[c].q[t][h]) : 0;
-                    act[c].s[t][h] = ok ? fs[2 * pp + h] : 0.0f;
+                    act[c].q[t][h][0] = lo.x, act[c].q[t][h][1] = lo.y, act[c].q[t][h][2] = lo.z, act[c].q[t][h][3] = lo.w;
+                    act[c].q[t][h][4] = hi.x, act[c].q[t][h][5] = hi.y, act[c].q[t][h][6] = hi.z, act[c].q[t][h][7] = hi.w;
                 }
             } else {
                 const uint4* src = reinterpret_cast<const uint4*>(static_cast<const int8_t*>(p_x) + (size_t)tok * p_k + (size_t)pp * 64);
@@ -440,7 +459,7 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
     }
 
     for (uint32_t base = wave_row0; base < wave_row1; base += RPW * UR) {
-        if (base != wave_row0) issue_pass(base);
+        if (base != wave_row0) issue_pass(base), issue_y();
         // Consume.
         float gate_sum = 0.0f;  // GATED: the row sum of the even slot, waiting for its odd partner
 #pragma unroll
@@ -479,7 +498,8 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
                 } else if (sub == 0 && rvalid[u] && tok0 + t < a.n) {
                     float* dst = a.y_row_major ? ybase + (size_t)lrow[u] * a.y_stride + (tok0 + t)
                                                : ybase + (size_t)(tok0 + t) * a.y_stride + lrow[u];
-                    *dst = p_accumulate ? *dst + tot : tot;
+                    if constexpr (kEarlyY) *dst = a.accumulate ? yold[u] + tot : tot;
+                    else *dst = a.accumulate ? *dst + tot : tot;
                 }
             }
         }
@@ -589,7 +609,9 @@ hipError_t launch_pairs_u(GemvArgs& a, uint32_t total_rows, int num_cus, const L
     if (passes_per_wave == 0) passes_per_wave = 1;
     a.rows_per_wave = passes_per_wave * pass_rows;
     const uint32_t waves = set_wave_ends(a);
-    const dim3 grid = FUSEQ ? dim3((waves + kFusedWaves - 1) / kFusedWaves, 1) : dim3(waves, (a.n + NT - 1) / NT);
+    const uint32_t side = a.gated && a.conv_state ? 1u : 0u;  // the side job's workgroup
+    a.inv_k = 1.0 / (double)a.k;
+    const dim3 grid = FUSEQ ? dim3((waves + kFusedWaves - 1) / kFusedWaves + side, 1) : dim3(waves, (a.n + NT - 1) / NT);
     const dim3 block(FUSEQ ? 64 * kFusedWaves : 64);
     const uint64_t bytes = (uint64_t)total_rows * (a.k >> 5) * (TYPE == 2 ? 18u : 34u) * (a.gated ? 2u : 1u);
     constexpr int kSmall = TYPE == 2 ? kDirectNT : kDirect;
@@ -603,7 +625,7 @@ hipError_t launch_pairs_u(GemvArgs& a, uint32_t total_rows, int num_cus, const L
     // hot scalars first (preloaded into SGPRs), then the whole argument block
     auto go = [&](auto kernel) {
         return launch_kernel(L, kFamGemv, kernel, grid, block, FUSEQ ? static_cast<const void*>(a.xf) : static_cast<const void*>(a.xq),
-                             a.batch.w[0], a.batch.y[0], a.k, a.batch.row_end[0], a.rows_per_wave, a.total_waves, a.accumulate, a);
+                             a.batch.w[0], a.xaux, a.xaux2, a.k, a.batch.row_end[0], a.rows_per_wave, a.total_waves, a);
     };
     if constexpr (DUMP) {  // the parity hook: plain single-weight variants, same fetch mode as the product launch of this size
         if constexpr (NT == 1) {

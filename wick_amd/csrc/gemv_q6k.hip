@@ -152,7 +152,7 @@ __global__ __launch_bounds__(64) void gemv_q6k_kernel(Q6kArgs a) {
         double total = 0.0;
 #pragma unroll
         for (int v = 0; v < 4; v++) total += wave_sum_f64(part[v]);
-        const float inv_rms = (float)(1.0 / sqrt(total / (double)a.k + (double)a.eps));
+        const float inv_rms = rms_inverse(total, 1.0 / (double)a.k, a.eps);
         const uint32_t quads = a.k >> 2;
 #pragma unroll
         for (int j = 0; j < XQ; j++) {

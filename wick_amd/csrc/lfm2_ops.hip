@@ -104,13 +104,14 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* __restrict__ 
     __shared__ double slots[16];
     const float* xr = x + (size_t)blockIdx.x * x_stride;
     float* yr = y + (size_t)blockIdx.x * y_stride;
+    const double inv_dim = 1.0 / (double)dim;  // while the loads are under way
     double s = 0.0;
     for (uint32_t i = threadIdx.x; i < dim; i += blockDim.x) {
         const double v = (double)xr[i];
         s += v * v;
     }
     const double total = block_sum_f64(s, slots);
-    const float inv_rms = (float)(1.0 / sqrt(total / (double)dim + (double)eps));
+    const float inv_rms = rms_inverse(total, inv_dim, eps);
     for (uint32_t i = threadIdx.x; i < dim; i += blockDim.x) yr[i] = __fmul_rn(__fmul_rn(xr[i], inv_rms), weight[i]);
 }
 
@@ -153,7 +154,7 @@ __device__ __forceinline__ void norm_rope_head(const float* src, const float* w,
         const double v = (double)src[i];
         s += v * v;
     }
-    const float inv_rms = (float)(1.0 / sqrt(wave_sum_f64(s) / (double)hd + (double)eps));
+    const float inv_rms = rms_inverse(wave_sum_f64(s), 1.0 / (double)hd, eps);
     for (uint32_t i = lane; i < half; i += 64) {
         float sn, cs;
         if (sn_tab) sn = sn_tab[i], cs = cs_tab[i];
@@ -238,7 +239,7 @@ __global__ __launch_bounds__(256) void qk_norm_rope_tokens64_kernel(QkNormRopeAr
             if (hh >= heads) break;
             const bool is_q = hh < a.n_heads;
             const double sq = (double)v[t] * (double)v[t];
-            const float inv_rms = (float)(1.0 / sqrt(wave_sum_f64(sq) / (double)HD + (double)a.eps));
+            const float inv_rms = rms_inverse(wave_sum_f64(sq), 1.0 / (double)HD, a.eps);
             const float xn = __fmul_rn(__fmul_rn(v[t], inv_rms), is_q ? wq : wk);
             const float other = __shfl_xor(xn, 32);
             // lanes 0-31 hold x0 and write r0 = x0 cs - x1 sn; lanes 32-63 hold x1 and write r1 = x0 sn + x1 cs
@@ -1204,6 +1205,7 @@ __global__ __launch_bounds__(256) void rmsnorm_quantize_kernel(const float* __re
                                                                float* __restrict__ scales, uint32_t dim, uint32_t x_stride, float eps) {
     __shared__ double slots[16];
     const float* xr = x + (size_t)blockIdx.x * x_stride;
+    const double inv_dim = 1.0 / (double)dim;  // while the loads are under way
     double s = 0.0;
     for (uint32_t i0 = threadIdx.x; i0 < dim; i0 += 4u * 256u) {  // four loads in flight; elements t, t + 256, .. in order, as rmsnorm_kernel sums them
         float xv[4];
@@ -1218,7 +1220,7 @@ __global__ __launch_bounds__(256) void rmsnorm_quantize_kernel(const float* __re
         }
     }
     const double total = block_sum_f64(s, slots);
-    const float inv_rms = (float)(1.0 / sqrt(total / (double)dim + (double)eps));
+    const float inv_rms = rms_inverse(total, inv_dim, eps);
     const uint32_t quads = dim >> 2;
     for (uint32_t quad0 = 0; quad0 < quads; quad0 += blockDim.x) {  // groups of 8 lanes stay together: quads % 8 == 0
         const uint32_t quad = quad0 + threadIdx.x;
@@ -1252,6 +1254,7 @@ __global__ __launch_bounds__(256) void residual_rmsnorm_quantize_kernel(float* _
     __shared__ __align__(16) float row[kResidualNormMaxDim];
     float* xr = x + (size_t)blockIdx.x * x_stride;
     const float* pr = partial + (size_t)blockIdx.x * dim;
+    const double inv_dim = 1.0 / (double)dim;  // while the loads are under way
     double s = 0.0;
     for (uint32_t i0 = threadIdx.x; i0 < dim; i0 += 4u * 256u) {  // four elements' loads (S + 1 each) in flight together
         float xv[4], pv[4][S];
@@ -1277,7 +1280,7 @@ __global__ __launch_bounds__(256) void residual_rmsnorm_quantize_kernel(float* _
         }
     }
     const double total = block_sum_f64(s, slots);  // its barriers also publish row[]
-    const float inv_rms = (float)(1.0 / sqrt(total / (double)dim + (double)eps));
+    const float inv_rms = rms_inverse(total, inv_dim, eps);
     const uint32_t quads = dim >> 2;
     for (uint32_t quad0 = 0; quad0 < quads; quad0 += blockDim.x) {
         const uint32_t quad = quad0 + threadIdx.x;

@@ -177,6 +177,14 @@ __device__ __forceinline__ float group_max8(float v) {
     return v;
 }
 
+// Sum over the same groups of 8 lanes.
+__device__ __forceinline__ int group_sum8_i32(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0xB1, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x4E, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, false);
+    return v;
+}
+
 template <int WIDTH>
 __device__ __forceinline__ float group_sum(float v) {
     if constexpr (WIDTH >= 2) v = dpp_add<0xB1>(v);   // quad_perm [1,0,3,2]
@@ -208,6 +216,18 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
     const double r2 = __hiloint2double(__builtin_amdgcn_readlane(hi, 32), __builtin_amdgcn_readlane(lo, 32));
     const double r3 = __hiloint2double(__builtin_amdgcn_readlane(hi, 48), __builtin_amdgcn_readlane(lo, 48));
     return (r0 + r1) + (r2 + r3);
+}
+
+// 1 / sqrt(total / k + eps) of an RMSNorm (rmsnorm, wick/src/backend/cpu.rs:577-594) in f64, rounded to f32 once.  The hardware's
+// reciprocal root (22 bits and more) and one step of third order, y (1 + e / 2 + 3 e^2 / 8) with e = 1 - s y^2: the error is
+// of order e^3, below f64's own rounding, in ten instructions where a division, a root and a division are a serial chain of
+// some eighty in front of every projection of a decode step.
+__device__ __forceinline__ float rms_inverse(double total, double inv_k, float eps) {
+    const double s = __builtin_fma(total, inv_k, (double)eps);
+    const double y = __builtin_amdgcn_rsq(s);
+    const double e = __builtin_fma(-(s * y), y, 1.0);
+    const double r = __builtin_fma(y * e, __builtin_fma(0.375, e, 0.5), y);
+    return (float)(__builtin_amdgcn_class(y, 0x100) ? r : y);  // positive normal; else 1 / sqrt of 0, inf or NaN as it stands
 }
 
 // f32 sum / maximum over the whole wave, every lane gets the result: DPP inside the rows, row results through scalar
