@@ -393,6 +393,13 @@ def test_attention_block_equals_the_separate_launches(ctx, ops, oracle, n_heads,
         b.free()
 
 
+@pytest.mark.parametrize("n_heads,n_kv,hd,max_seq,steps", [(8, 2, 64, 4500, [0, 63, 64, 4095, 4096, 4480, 4499]), (6, 2, 64, 330, [1, 319, 320, 329]),
+                                                           (8, 1, 32, 300, [0, 64, 299]), (8, 2, 128, 270, [0, 127, 269]), (4, 1, 256, 258, [0, 256])])
+def test_attention_block_of_grouped_query_heads(ctx, ops, oracle, n_heads, n_kv, hd, max_seq, steps):
+    """One, two and four query heads per workgroup, new rows at the edges of chunks and of the cache, contexts past one round of splits."""
+    test_attention_block_equals_the_separate_launches(ctx, ops, oracle, n_heads, n_kv, hd, max_seq, steps)
+
+
 def test_argmax_rules(ctx, ops):
     """cpu_argmax (wick/src/sampler.rs:7-19): last of equal maxima, NaN = -inf, -0.0 < +0.0."""
     cases = [[1.0, 3.0, 2.0], [3.0, 1.0, 3.0, 2.0], [np.nan, 1.0, np.nan], [np.nan, np.nan], [np.nan, -np.inf], [0.0, -0.0], [-0.0, 0.0, -0.0],

@@ -195,7 +195,8 @@ size_t wick_rocm_attention_block_scratch_bytes(uint32_t max_seq, uint32_t n_head
 // f32-cache form).
 static int attention_block_kv(wick_rocm_ctx* ctx, float* d_q, float* d_k, const float* d_v, const float* d_q_norm, const float* d_k_norm,
                               void* d_k_cache, void* d_v_cache, float* d_out, void* d_scratch, uint32_t pos, const uint32_t* d_pos,
-                              uint32_t max_seq, uint32_t head_dim, uint32_t n_heads, uint32_t n_kv_heads, float eps, float theta_scale, bool kv_f16) {
+                              uint32_t max_seq, uint32_t head_dim, uint32_t n_heads, uint32_t n_kv_heads, float eps, float theta_scale, bool kv_f16,
+                              const float* d_rope = nullptr) {
     WR_ENTER(ctx);
     if (!d_q || !d_k || !d_v || !d_q_norm || !d_k_norm || !d_k_cache || !d_v_cache || !d_out || !d_scratch)
         return fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "attention_block: null device pointer");
@@ -209,7 +210,7 @@ static int attention_block_kv(wick_rocm_ctx* ctx, float* d_q, float* d_k, const 
     hipError_t e;
     if (attention_layer_applies(head_dim)) {
         e = launch_attention_layer(d_q, d_k, d_v, d_q_norm, d_k_norm, d_k_cache, d_v_cache, d_out, partials, pos, d_pos, max_seq, n_heads,
-                                   n_kv_heads, head_dim, eps, theta_scale, scale, ctx->launch(), kv_f16);
+                                   n_kv_heads, head_dim, eps, theta_scale, scale, ctx->launch(), kv_f16, d_rope);
     } else {
         e = launch_qk_norm_rope(d_q, d_k, d_v, d_q_norm, d_k_norm, d_k_cache, d_v_cache, pos, d_pos, max_seq, head_dim, n_heads, n_kv_heads, eps,
                                 theta_scale, ctx->launch(), 1, 0, 0, kv_f16);
@@ -289,17 +290,17 @@ namespace {
 // extras of launch_argmax (may be null).
 int lm_head_greedy_locked(wick_rocm_ctx* ctx, const wick_rocm_weight* w, const float* d_x, const float* d_norm_weight, float eps, float* d_logits,
                           unsigned long long* d_partial, uint32_t* d_out, uint32_t* d_token, uint32_t* d_pos, uint32_t* d_history,
-                          uint32_t history_len, float* d_emb_out) {
+                          uint32_t history_len, float* d_emb_out, RopeTable rope = {}) {
     const uint8_t* wd = static_cast<const uint8_t*>(w->d);
     const uint32_t waves = w->type == kTypeQ6_K ? gemv_q6k_waves(w->m, w->k, ctx->num_cus) : 0u;
     if (waves != 0 && waves <= kArgmaxPartials && !misaligned(d_x, 16) && !misaligned(d_norm_weight, 16)) {
         hipError_t e = launch_gemv_q6k_rmsnorm(wd, w->m, w->k, d_x, d_norm_weight, eps, d_logits, 0, ctx->num_cus, ctx->launch(), d_partial);
         if (e != hipSuccess) return fail_hip(ctx, e, "Q6_K gemv launch");
-        e = launch_argmax_final(d_partial, waves, w->m, d_out, d_token, d_pos, d_history, history_len, ctx->launch(), wd, w->type, w->m, w->k, d_emb_out);
+        e = launch_argmax_final(d_partial, waves, w->m, d_out, d_token, d_pos, d_history, history_len, ctx->launch(), wd, w->type, w->m, w->k, d_emb_out, rope);
         return e == hipSuccess ? WICK_ROCM_OK : fail_hip(ctx, e, "argmax launch");
     }
     if (int rc = wick_rocm_gemv_rmsnorm_f32_multi(ctx, &w, &d_logits, 1, d_x, d_norm_weight, eps, 0)) return rc;
-    hipError_t e = launch_argmax(d_logits, w->m, d_partial, d_out, d_token, d_pos, d_history, history_len, ctx->launch(), wd, w->type, w->m, w->k, d_emb_out);
+    hipError_t e = launch_argmax(d_logits, w->m, d_partial, d_out, d_token, d_pos, d_history, history_len, ctx->launch(), wd, w->type, w->m, w->k, d_emb_out, rope);
     return e == hipSuccess ? WICK_ROCM_OK : fail_hip(ctx, e, "argmax launch");
 }
 
@@ -349,6 +350,8 @@ struct wick_rocm_lfm2 {
     float *hidden = nullptr, *proj = nullptr, *gated = nullptr, *q = nullptr, *k = nullptr, *v = nullptr, *attn = nullptr,
           *gate = nullptr, *scores = nullptr, *logits = nullptr;
     uint32_t *d_token = nullptr, *d_pos = nullptr, *d_pick = nullptr, *d_history = nullptr;
+    float* rope = nullptr;  // the current position's sines and cosines, kept by set_step and the greedy pick
+    RopeTable rope_table() const { return {reinterpret_cast<float2*>(rope), cfg.hidden_size / cfg.n_heads / 2u, theta_scale}; }
     unsigned long long* d_argmax_partial = nullptr;
     // prompt (prefill) buffers for up to `prefill_cap` tokens, allocated by the first prefill
     uint32_t prefill_cap = 0;
@@ -465,7 +468,7 @@ int enqueue_step(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, StepMode mode) {
         } else {
             if ((rc = gemv_normed(ctx, {L.q, L.k, L.v}, {m->q, m->k, m->v}, m->hidden, L.attn_norm, c.rms_norm_eps))) break;
             if ((rc = attention_block_kv(ctx, m->q, m->k, m->v, L.q_norm, L.k_norm, L.k_cache, L.v_cache, m->attn, m->scores, 0, m->d_pos,
-                                         c.max_seq_len, hd, c.n_heads, L.n_kv, c.rms_norm_eps, m->theta_scale, m->kv_f16)))
+                                         c.max_seq_len, hd, c.n_heads, L.n_kv, c.rms_norm_eps, m->theta_scale, m->kv_f16, m->rope)))
                 break;
             if ((rc = gemv_residual(ctx, L.o, m->hidden, m->attn))) break;
         }
@@ -483,7 +486,7 @@ int enqueue_step(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, StepMode mode) {
     if (mode != kStepGreedy) return gemv_normed(ctx, {m->embd}, {m->logits}, m->hidden, m->out_norm, c.rms_norm_eps);
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     return lm_head_greedy_locked(ctx, m->embd, m->hidden, m->out_norm, c.rms_norm_eps, m->logits, m->d_argmax_partial, m->d_pick, m->d_token, m->d_pos,
-                                 m->d_history, c.max_seq_len, m->hidden);
+                                 m->d_history, c.max_seq_len, m->hidden, m->rope_table());
 }
 
 int step_graph(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, StepMode mode, wick_rocm_graph** out) {
@@ -643,7 +646,7 @@ int enqueue_prompt_pass(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, uint32_t n, uint3
 int set_step(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, uint32_t token, uint32_t pos) {
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
     hipError_t e = launch_set_step(m->d_token, token, m->d_pos, pos, ctx->launch(), static_cast<const uint8_t*>(m->embd->d), m->embd->type, m->embd->m,
-                                   m->cfg.hidden_size, m->hidden);
+                                   m->cfg.hidden_size, m->hidden, m->rope_table());
     return e == hipSuccess ? WICK_ROCM_OK : fail_hip(ctx, e, "set_step launch");
 }
 
@@ -799,7 +802,7 @@ int wick_rocm_lfm2_load_kv(wick_rocm_ctx* ctx, const wick_gguf* g, uint32_t cont
     if ((rc = alloc_t(ctx, m, hs, &m->hidden)) || (rc = alloc_t(ctx, m, 3 * (size_t)hs, &m->proj)) ||
         (rc = alloc_t(ctx, m, hs, &m->gated)) || (rc = alloc_t(ctx, m, hs, &m->q)) || (rc = alloc_t(ctx, m, kv_max, &m->k)) ||
         (rc = alloc_t(ctx, m, kv_max, &m->v)) || (rc = alloc_t(ctx, m, hs, &m->attn)) || (rc = alloc_t(ctx, m, inter, &m->gate)) ||
-        (rc = alloc_t(ctx, m, attention_scratch_floats(c.max_seq_len, c.n_heads, hd), &m->scores)) ||
+        (rc = alloc_t(ctx, m, attention_scratch_floats(c.max_seq_len, c.n_heads, hd), &m->scores)) || (rc = alloc_t(ctx, m, hd, &m->rope)) ||
         (rc = alloc_t(ctx, m, c.vocab_size, &m->logits)) || (rc = alloc_t(ctx, m, 1, &m->d_token)) ||
         (rc = alloc_t(ctx, m, 1, &m->d_pos)) || (rc = alloc_t(ctx, m, 1, &m->d_pick)) || (rc = alloc_t(ctx, m, kArgmaxPartials, &m->d_argmax_partial)) || (rc = alloc_t(ctx, m, c.max_seq_len, &m->d_history)))
         return bail(rc);
@@ -875,7 +878,7 @@ static int prefill_locked(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, const uint3
             if (tokens) {
                 if (int rc = set_step(ctx, model, tokens[j], start_pos + j)) return rc;
             } else {
-                const hipError_t e = launch_set_step(nullptr, 0, model->d_pos, start_pos + j, ctx->launch());
+                const hipError_t e = launch_set_step(nullptr, 0, model->d_pos, start_pos + j, ctx->launch(), nullptr, 0, 0, 0, nullptr, model->rope_table());
                 if (e != hipSuccess) return fail_hip(ctx, e, "set_step launch");
                 if (int rc = wick_rocm_upload(ctx, model->hidden, embeddings + (size_t)j * c.hidden_size, (size_t)c.hidden_size * sizeof(float))) return rc;
             }
@@ -967,7 +970,7 @@ static int step_locked(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uint32_t token
     if (embedding) {  // position only; the input vector goes where the lookup would have put the row
         {
             std::lock_guard<std::recursive_mutex> lk(ctx->mu);
-            const hipError_t e = launch_set_step(nullptr, 0, model->d_pos, pos, ctx->launch());
+            const hipError_t e = launch_set_step(nullptr, 0, model->d_pos, pos, ctx->launch(), nullptr, 0, 0, 0, nullptr, model->rope_table());
             if (e != hipSuccess) return fail_hip(ctx, e, "set_step launch");
         }
         if (int rc = wick_rocm_upload(ctx, model->hidden, embedding, (size_t)c.hidden_size * sizeof(float))) return rc;

@@ -143,6 +143,16 @@ __device__ __forceinline__ void rope_sincos(uint32_t pos, uint32_t i, float thet
     sincosf(theta, &sn, &cs);
 }
 
+// A position's table of them, {sin, cos} of pair i: filled once per decode step by the kernel that sets the position, read by every
+// attention layer of the step.
+__device__ __forceinline__ void rope_table_fill(const RopeTable& t, uint32_t pos, uint32_t first, uint32_t step) {
+    for (uint32_t i = first; i < t.half; i += step) {
+        float2 v;
+        rope_sincos(pos, i, t.theta_scale, v.x, v.y);
+        t.tab[i] = v;
+    }
+}
+
 // RMSNorm + RoPE of one head by the calling wave: dst[] (and dst2[], when given) receive the result; src may equal dst.
 // sn_tab / cs_tab: the position's sines and cosines per pair when the caller has them already (else computed here).
 template <typename D1, typename D2>
@@ -594,15 +604,24 @@ __global__ __launch_bounds__(256) void attention_combine_kernel(AttentionArgs a,
     attention_merge<HD>(a, splits, blockIdx.x, attention_seq(a));
 }
 
-// The attention block between the Q/K/V projections and the output projection with QK-norm, RoPE and the KV append
-// folded into the sequence-split kernel (wick/src/model/lfm2.rs:783-1006): every workgroup (head, split) norms and
-// rotates its own query head into LDS (same arithmetic as qk_norm_rope_kernel); the workgroups whose chunk holds the
-// new position norm and rotate the key head, append it and the value row to the caches (query heads that share a KV
-// head write identical bytes) and read them back after a barrier.  No workgroup depends on another; the partials are
-// merged by attention_combine_kernel as before.  Results are bit-identical to qk_norm_rope + attention_split +
-// attention_combine, one launch less.  (Merging in the last workgroup to finish, behind a ticket counter, was built
-// and measured: the device-scope fences it needs write back and invalidate the L2 per workgroup and cost far more
-// than the launch they save.)
+// The attention block between the Q/K/V projections and the output projection with QK-norm, RoPE and the KV append folded
+// into the sequence-split kernel (wick/src/model/lfm2.rs:783-1006); the partials are merged by attention_combine_kernel.  A
+// workgroup takes NH query heads that share a KV head, and the chunks split, split + splits, .. of 64 positions.  Arithmetic per
+// head is that of qk_norm_rope_kernel and attention_chunks, bit for bit.
+//
+// What bounds it: at short contexts the chain of round trips and of vector instructions between them, at long ones the bytes
+// in flight.  So
+//   * everything that does not depend on the position is requested first, then the first chunk's K and V rows; the norm and
+//     the rotation run meanwhile, the latter from a table of the position's sines and cosines when there is one (the chain of
+//     powers and the range reduction took 0.8 us of every launch).  The new position's own row takes part from LDS and
+//     from the projection's output; the cache gets it on the side;
+//   * one set of loads serves NH heads; the next chunk's are issued as soon as the registers of this one are free; the softmax
+//     of head i is wave i's alone and leaves the weights in LDS in the order the value sum reads them (16 bytes at a time):
+//     two barriers per chunk instead of four, the exponentials once instead of in every wave.
+// First to last instruction in a step of the 350M model (16 heads, 8 KV heads): 4.2 -> 3.0 us at position 30, 15.6 -> 11.0 at
+// 20000 (f16; 41 MB).
+// (Merging in the last workgroup to finish, by a ticket, with partials written and read past the L2 by relaxed atomics so that
+// no fence is needed: the three round trips in a row cost what the second launch costs, 5 - 15 us per step more at 1500 positions.)
 struct AttentionLayerArgs {
     AttentionArgs at;     // q unused; caches as read
     const float* q_raw;   // [n_heads * HD] projection output, left unchanged
@@ -610,32 +629,210 @@ struct AttentionLayerArgs {
     const float* v;       // [n_kv_heads * HD]
     const float* q_norm;
     const float* k_norm;
+    const float2* rope;   // the position's {sin, cos} per pair, or null
     void* k_cache;        // the same caches, writable
     void* v_cache;
     float eps, theta_scale;
 };
 
-template <int HD, typename KV>
-__global__ __launch_bounds__(256) void attention_layer_kernel(AttentionLayerArgs f, uint32_t splits) {
-    __shared__ __align__(16) float qh[HD];
-    const AttentionArgs& a = f.at;
-    const uint32_t h = blockIdx.x / splits, split = blockIdx.x % splits, tid = threadIdx.x;
-    const uint32_t seq = attention_seq(a);
-    if (seq == 0 || split * kAttnChunk >= seq) return;
-    const uint32_t pos = seq - 1u, kv_dim = a.n_kv_heads * HD, kvh = h / (a.n_heads / a.n_kv_heads);
-    if (tid < 64) norm_rope_head(f.q_raw + (size_t)h * HD, f.q_norm, HD, pos, f.eps, f.theta_scale, qh, static_cast<float*>(nullptr));
-    if ((pos / kAttnChunk) % splits == split) {  // this workgroup's chunks include the new position
-        if (tid >= 64 && tid < 128)
-            norm_rope_head(f.k_raw + (size_t)kvh * HD, f.k_norm, HD, pos, f.eps, f.theta_scale,
-                           static_cast<KV*>(f.k_cache) + (size_t)pos * kv_dim + (size_t)kvh * HD, static_cast<float*>(nullptr));
-        if (tid >= 128) {
-            const float* vh = f.v + (size_t)kvh * HD;
-            KV* vc = static_cast<KV*>(f.v_cache) + (size_t)pos * kv_dim + (size_t)kvh * HD;
-            for (uint32_t i = tid - 128; i < HD; i += 128) kv_store(vc + i, vh[i]);
+// norm_rope_head with its operands requested ahead: load() when nothing else is known, finish() when the rest is there.
+template <int HD>
+struct NormRope {
+    static constexpr uint32_t E = (HD + 63) / 64, P = (HD / 2 + 63) / 64;
+    float x[E], x0[P], x1[P], w0[P], w1[P];
+    __device__ __forceinline__ void load(const float* src, const float* w, uint32_t lane) {
+#pragma unroll
+        for (uint32_t e = 0; e < E; e++) x[e] = src[HD < 64 ? lane % HD : lane + 64u * e];
+#pragma unroll
+        for (uint32_t p = 0; p < P; p++) {
+            const uint32_t i = (lane + 64u * p) % (HD / 2);
+            x0[p] = src[i], x1[p] = src[i + HD / 2], w0[p] = w[i], w1[p] = w[i + HD / 2];
         }
     }
-    __syncthreads();  // qh[] and this workgroup's cache rows are complete
-    attention_chunks<HD, KV>(a, splits, h, split, seq, qh);
+    __device__ __forceinline__ void finish(const float2 (&sc)[P], float eps, float* dst, uint32_t lane) const {
+        double s = 0.0;
+#pragma unroll
+        for (uint32_t e = 0; e < E; e++) {
+            const double v = (double)x[e];
+            if (HD >= 64 || lane < HD) s += v * v;
+        }
+        const float inv_rms = rms_inverse(wave_sum_f64(s), 1.0 / (double)HD, eps);
+#pragma unroll
+        for (uint32_t p = 0; p < P; p++) {
+            const float a = __fmul_rn(__fmul_rn(x0[p], inv_rms), w0[p]), b = __fmul_rn(__fmul_rn(x1[p], inv_rms), w1[p]);
+            const uint32_t i = lane + 64u * p;
+            if (i < HD / 2) {
+                dst[i] = __fsub_rn(__fmul_rn(a, sc[p].y), __fmul_rn(b, sc[p].x));
+                dst[i + HD / 2] = __fadd_rn(__fmul_rn(a, sc[p].x), __fmul_rn(b, sc[p].y));
+            }
+        }
+    }
+};
+
+// A key row's four elements as loaded, widened when they are used.
+template <typename KV>
+struct KvQuad {
+    using T = typename std::conditional<std::is_same<KV, float>::value, float4, kv_h4>::type;
+    T v;
+    __device__ __forceinline__ void load(const KV* p) { v = *reinterpret_cast<const T*>(p); }
+    __device__ __forceinline__ void set(const float4& f) {
+        if constexpr (std::is_same<KV, float>::value) v = f;
+        else v = kv_h4{(KV)f.x, (KV)f.y, (KV)f.z, (KV)f.w};
+    }
+    __device__ __forceinline__ float4 get() const {
+        if constexpr (std::is_same<KV, float>::value) return v;
+        else return make_float4((float)v[0], (float)v[1], (float)v[2], (float)v[3]);
+    }
+};
+
+template <int HD, typename KV, int NH>
+__global__ __launch_bounds__(256) void attention_layer_kernel(AttentionLayerArgs f, uint32_t splits) {
+    constexpr uint32_t LR = HD / 4, RPP = 256 / LR, KROWS = kAttnChunk / RPP;  // lanes per key row, rows per pass, key rows per thread
+    constexpr uint32_t VG = 256 / HD, VROWS = kAttnChunk / VG;                  // position groups of the value sum, rows of each
+    using NR = NormRope<HD>;
+    __shared__ __align__(16) float qh[NH][HD];
+    __shared__ __align__(16) float kh[HD];  // the new key row
+    __shared__ float sc[2][NH][kAttnChunk];
+    __shared__ __align__(16) float ew[2][NH][kAttnChunk];  // weight of position p at (p % VG) * VROWS + p / VG
+    __shared__ float cor[2][NH];
+    __shared__ float red[NH][256];
+    const AttentionArgs& a = f.at;
+    const uint32_t hg = blockIdx.x / splits, split = blockIdx.x % splits, tid = threadIdx.x, lane = tid & 63u;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
+    const uint32_t kv_dim = a.n_kv_heads * HD, h0 = hg * NH, kvh = h0 / (a.n_heads / a.n_kv_heads);
+    const uint32_t quad = tid % LR, prow = tid / LR, d = tid % HD, g = tid / HD;
+    // job `wave` of NH + 1: query head h0 + job, or the key head (with NH = 4 that is wave 0's second)
+    const auto job_src = [&](uint32_t job) { return job < NH ? f.q_raw + (size_t)(h0 + job) * HD : f.k_raw + (size_t)kvh * HD; };
+    NR nr;
+    nr.load(job_src(wave), wave < NH ? f.q_norm : f.k_norm, lane);
+    float2 sincos[NR::P];
+    if (f.rope) {
+#pragma unroll
+        for (uint32_t p = 0; p < NR::P; p++) sincos[p] = f.rope[(lane + 64u * p) % (HD / 2)];
+    }
+    const float v_new = f.v[(size_t)kvh * HD + d];
+    const uint32_t seq = attention_seq(a);
+    if (seq == 0 || split * kAttnChunk >= seq) return;
+    const uint32_t pos = seq - 1u;
+
+    KvQuad<KV> kv[KROWS];
+    KV vv[VROWS];
+    // Rows past the position are read as they are (the cache has max_seq rows; past those: clamped) and replaced or masked.
+    const auto fetch = [&](uint32_t t0, bool k) {
+        const KV* p = static_cast<const KV*>(k ? a.k_cache : a.v_cache) + (size_t)t0 * kv_dim + (size_t)kvh * HD;
+        const uint32_t lim = a.max_seq - 1u - t0;
+        if (lim >= kAttnChunk - 1u) {
+            if (k) {
+#pragma unroll
+                for (uint32_t j = 0; j < KROWS; j++) kv[j].load(p + (size_t)(j * RPP) * kv_dim + (prow * kv_dim + 4u * quad));
+            } else {
+#pragma unroll
+                for (uint32_t j = 0; j < VROWS; j++) vv[j] = p[(size_t)(j * VG) * kv_dim + (g * kv_dim + d)];
+            }
+        } else if (k) {
+#pragma unroll
+            for (uint32_t j = 0; j < KROWS; j++) kv[j].load(p + (min(prow + j * RPP, lim) * kv_dim + 4u * quad));
+        } else {
+#pragma unroll
+            for (uint32_t j = 0; j < VROWS; j++) vv[j] = p[min(g + j * VG, lim) * kv_dim + d];
+        }
+    };
+    fetch(split * kAttnChunk, true);
+    fetch(split * kAttnChunk, false);
+
+    const uint32_t new_chunk = pos / kAttnChunk;
+    const bool appends = new_chunk % splits == split;  // this workgroup's chunks include the new position
+    if (!f.rope) {
+#pragma unroll
+        for (uint32_t p = 0; p < NR::P; p++) rope_sincos(pos, (lane + 64u * p) % (HD / 2), f.theta_scale, sincos[p].x, sincos[p].y);
+    }
+    if (wave <= NH) nr.finish(sincos, f.eps, wave < NH ? qh[wave] : kh, lane);
+    if (NH == 4 && wave == 0) {
+        nr.load(job_src(4), f.k_norm, lane);
+        nr.finish(sincos, f.eps, kh, lane);
+    }
+    __syncthreads();
+    if (appends && h0 % (a.n_heads / a.n_kv_heads) == 0) {  // the KV head's first query heads write its row
+        const size_t at = (size_t)pos * kv_dim + (size_t)kvh * HD;
+        if (tid < HD) {
+            kv_store(static_cast<KV*>(f.k_cache) + at + tid, kh[tid]);
+            kv_store(static_cast<KV*>(f.v_cache) + at + tid, v_new);
+        }
+    }
+
+    float4 q4[NH];
+#pragma unroll
+    for (int i = 0; i < NH; i++) q4[i] = reinterpret_cast<const float4*>(qh[i])[quad];
+    float acc[NH];
+#pragma unroll
+    for (int i = 0; i < NH; i++) acc[i] = 0.0f;
+    float m_run = -__builtin_inff(), l_run = 0.0f;  // of head `wave`, in that wave
+    int b = 0;
+    for (uint32_t c = split; c * kAttnChunk < seq; c += splits, b ^= 1) {
+        const uint32_t t0 = c * kAttnChunk;
+        const uint32_t nt = seq - t0 < kAttnChunk ? seq - t0 : kAttnChunk;
+        const bool more = (c + splits) * kAttnChunk < seq;
+        if (c == new_chunk) {  // rows at (and past) the position: the new row
+            KvQuad<KV> k4;
+            k4.set(*reinterpret_cast<const float4*>(&kh[4 * quad]));
+#pragma unroll
+            for (uint32_t j = 0; j < KROWS; j++)
+                if (prow + j * RPP >= nt - 1u) kv[j] = k4;
+#pragma unroll
+            for (uint32_t j = 0; j < VROWS; j++) vv[j] = g + j * VG >= nt - 1u ? (KV)v_new : vv[j];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < KROWS; j++) {
+            const uint32_t r = prow + j * RPP;
+            const float4 k4 = kv[j].get();
+#pragma unroll
+            for (int i = 0; i < NH; i++) {
+                float p = q4[i].x * k4.x + q4[i].y * k4.y + q4[i].z * k4.z + q4[i].w * k4.w;
+                p = group_sum<LR>(p);  // DPP adds inside 16 lanes: no trip through the LDS crossbar
+                if (quad == 0) sc[b][i][r] = r < nt ? p * a.scale : -__builtin_inff();
+            }
+        }
+        if (more) fetch(t0 + splits * kAttnChunk, true);
+        __syncthreads();
+        if (wave < NH) {  // one lane per position
+            const float s = sc[b][wave][lane];
+            const float m_new = fmaxf(m_run, wave_max_f32(s));
+            const float e = lane < nt ? ggml_expf(s - m_new) : 0.0f;  // positions past the end weigh 0
+            const float l_chunk = wave_sum_f32(e);
+            const float corr = ggml_expf(m_run - m_new);  // 0 on the first chunk (m_run = -inf)
+            l_run = l_run * corr + l_chunk;
+            m_run = m_new;
+            ew[b][wave][(lane % VG) * VROWS + lane / VG] = e;
+            if (lane == 0) cor[b][wave] = corr;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NH; i++) acc[i] *= cor[b][i];
+#pragma unroll
+        for (uint32_t j = 0; j < VROWS; j += 4) {
+            const float v0 = (float)vv[j], v1 = (float)vv[j + 1], v2 = (float)vv[j + 2], v3 = (float)vv[j + 3];
+#pragma unroll
+            for (int i = 0; i < NH; i++) {
+                const float4 w4 = *reinterpret_cast<const float4*>(&ew[b][i][g * VROWS + j]);
+                acc[i] += w4.x * v0, acc[i] += w4.y * v1, acc[i] += w4.z * v2, acc[i] += w4.w * v3;
+            }
+        }
+        if (more) fetch(t0 + splits * kAttnChunk, false);
+    }
+#pragma unroll
+    for (int i = 0; i < NH; i++) red[i][tid] = acc[i];
+    __syncthreads();
+    for (uint32_t t = tid; t < NH * HD; t += 256u) {
+        const uint32_t i = t / HD, dd = t % HD;
+        float r = red[i][dd];
+#pragma unroll
+        for (uint32_t p = 1; p < VG; p++) r += red[i][p * HD + dd];
+        a.scores[((size_t)(h0 + i) * splits + split) * (HD + 2) + 2 + dd] = r;
+    }
+    if (wave < NH && lane == 0) {
+        float* part = a.scores + ((size_t)(h0 + wave) * splits + split) * (HD + 2);
+        part[0] = m_run, part[1] = l_run;
+    }
 }
 
 // Causal attention for the n tokens of a prompt whose K / V rows are already in the caches (pass B of the reference's
@@ -1401,7 +1598,7 @@ __device__ __forceinline__ void embed_row_batched(const EmbedArgs& emb, uint32_t
 
 __global__ __launch_bounds__(256) void argmax_final_kernel(const unsigned long long* __restrict__ partial, uint32_t blocks, uint32_t n,
                                                            uint32_t* __restrict__ out, uint32_t* __restrict__ d_token, uint32_t* __restrict__ d_pos,
-                                                           uint32_t* __restrict__ d_history, uint32_t history_len, EmbedArgs emb) {
+                                                           uint32_t* __restrict__ d_history, uint32_t history_len, EmbedArgs emb, RopeTable rope) {
     __shared__ uint32_t picked;
     __shared__ unsigned long long red[4];
     const uint32_t waves = blockDim.x >> 6;  // 1 (at most 64 partial keys) or 4
@@ -1416,6 +1613,8 @@ __global__ __launch_bounds__(256) void argmax_final_kernel(const unsigned long l
 #pragma unroll
         for (int j = 0; j < 8; j++) best = k[j] > best ? k[j] : best;
     }
+    // the next position's table, under the keys' latency; before the position is advanced below (behind a barrier or in this wave)
+    if (rope.tab && d_pos && threadIdx.x >= blockDim.x - 64u) rope_table_fill(rope, *d_pos + 1u, threadIdx.x & 63u, 64u);
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
         const unsigned long long o = __shfl_xor(best, off, 64);
@@ -1448,16 +1647,13 @@ __global__ __launch_bounds__(256) void argmax_final_kernel(const unsigned long l
 
 // Sets the device-side token / position of the next step (either may be null) and, when an embedding is given, looks
 // the token's row up as that step's input.
-__global__ __launch_bounds__(256) void set_step_kernel(uint32_t* d_token, uint32_t token, uint32_t* d_pos, uint32_t pos, EmbedArgs emb) {
+__global__ __launch_bounds__(256) void set_step_kernel(uint32_t* d_token, uint32_t token, uint32_t* d_pos, uint32_t pos, EmbedArgs emb, RopeTable rope) {
+    if (rope.tab && threadIdx.x >= 192u) rope_table_fill(rope, pos, threadIdx.x - 192u, 64u);
     if (threadIdx.x == 0) {
         if (d_token) *d_token = token;
         if (d_pos) *d_pos = pos;
     }
     if (emb.w && token < emb.m) embed_row_batched(emb, token);
-}
-
-__global__ void advance_pos_kernel(uint32_t* d_pos) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *d_pos = *d_pos + 1u;
 }
 
 }  // namespace
@@ -1567,16 +1763,29 @@ bool attention_layer_applies(uint32_t head_dim) { return head_dim == 32 || head_
 hipError_t launch_attention_layer(const float* d_q, const float* d_k, const float* d_v, const float* d_q_norm, const float* d_k_norm,
                                   void* d_k_cache, void* d_v_cache, float* d_out, float* d_scratch, uint32_t pos,
                                   const uint32_t* d_pos, uint32_t max_seq, uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, float eps,
-                                  float theta_scale, float scale, const Launch& L, bool kv_f16) {
+                                  float theta_scale, float scale, const Launch& L, bool kv_f16, const float* d_rope) {
     AttentionLayerArgs f{};
     f.at = AttentionArgs{nullptr, d_k_cache, d_v_cache, d_out, d_scratch, d_pos, pos + 1u, max_seq, n_heads, n_kv_heads, head_dim, scale};
     f.q_raw = d_q, f.k_raw = d_k, f.v = d_v, f.q_norm = d_q_norm, f.k_norm = d_k_norm;
-    f.k_cache = d_k_cache, f.v_cache = d_v_cache, f.eps = eps, f.theta_scale = theta_scale;
-    const uint32_t splits = attention_splits(max_seq);
-    const dim3 grid(n_heads * splits), block(256);
+    f.k_cache = d_k_cache, f.v_cache = d_v_cache, f.eps = eps, f.theta_scale = theta_scale, f.rope = reinterpret_cast<const float2*>(d_rope);
+    const uint32_t splits = attention_splits(max_seq), group = n_heads / n_kv_heads;
+    const dim3 block(256);
     auto run = [&](auto hd) -> hipError_t {
         constexpr int HD = decltype(hd)::value;
-        hipError_t e = with_kv_type(kv_f16, [&](auto kv) { return launch_kernel(L, kFamOther, attention_layer_kernel<HD, decltype(kv)>, grid, block, f, splits); });
+        const auto go = [&](auto nh) {
+            constexpr int NH = decltype(nh)::value;
+            return with_kv_type(kv_f16, [&](auto kv) {
+                return launch_kernel(L, kFamOther, attention_layer_kernel<HD, decltype(kv), NH>, dim3(n_heads / NH * splits), block, f, splits);
+            });
+        };
+        // As many query heads per workgroup as share a KV head and as their accumulators leave registers for.  One head each is as
+        // fast while everything fits the L2s and the launch is latency; at 20000 positions of f32 rows two heads (16 over 8) take
+        // 367 us a step against 397, four (32 over 8) 194 against 210.
+        constexpr int kMax = 256 / HD < 4 ? 256 / HD : 4;
+        hipError_t e;
+        if (kMax >= 4 && group % 4u == 0) e = go(std::integral_constant<int, kMax>{});
+        else if (kMax >= 2 && group % 2u == 0) e = go(std::integral_constant<int, kMax < 2 ? kMax : 2>{});
+        else e = go(std::integral_constant<int, 1>{});
         if (e != hipSuccess) return e;
         return launch_kernel(L, kFamOther, attention_combine_kernel<HD>, dim3(n_heads), block, f.at, splits);
     };
@@ -1720,29 +1929,25 @@ hipError_t launch_silu_mul(float* d_gate, const float* d_up, uint32_t n, const L
 
 hipError_t launch_argmax(const float* d_x, uint32_t n, unsigned long long* d_partial, uint32_t* d_out, uint32_t* d_token, uint32_t* d_pos,
                          uint32_t* d_history, uint32_t history_len, const Launch& L, const uint8_t* d_embd, int embd_type, uint32_t embd_m,
-                         uint32_t embd_k, float* d_embd_out) {
+                         uint32_t embd_k, float* d_embd_out, RopeTable rope) {
     const uint32_t blocks = n >= 4096u ? kArgmaxBlocks : 1u;
     hipError_t e = launch_kernel(L, kFamOther, argmax_partial_kernel, dim3(blocks), dim3(256), d_x, n, d_partial);
     if (e != hipSuccess) return e;
-    return launch_argmax_final(d_partial, blocks, n, d_out, d_token, d_pos, d_history, history_len, L, d_embd, embd_type, embd_m, embd_k, d_embd_out);
+    return launch_argmax_final(d_partial, blocks, n, d_out, d_token, d_pos, d_history, history_len, L, d_embd, embd_type, embd_m, embd_k, d_embd_out, rope);
 }
 
 hipError_t launch_argmax_final(const unsigned long long* d_partial, uint32_t n_partials, uint32_t n, uint32_t* d_out, uint32_t* d_token, uint32_t* d_pos,
                                uint32_t* d_history, uint32_t history_len, const Launch& L, const uint8_t* d_embd, int embd_type, uint32_t embd_m,
-                               uint32_t embd_k, float* d_embd_out) {
+                               uint32_t embd_k, float* d_embd_out, RopeTable rope) {
     const EmbedArgs emb{d_embd_out ? d_embd : nullptr, d_embd_out, embd_type, embd_m, embd_k};
     return launch_kernel(L, kFamOther, argmax_final_kernel, dim3(1), dim3(emb.w || n_partials > 64u ? 256 : 64), d_partial, n_partials, n, d_out, d_token,
-                         d_pos, d_history, history_len, emb);
+                         d_pos, d_history, history_len, emb, rope);
 }
 
 hipError_t launch_set_step(uint32_t* d_token, uint32_t token, uint32_t* d_pos, uint32_t pos, const Launch& L, const uint8_t* d_embd, int embd_type,
-                           uint32_t embd_m, uint32_t embd_k, float* d_embd_out) {
+                           uint32_t embd_m, uint32_t embd_k, float* d_embd_out, RopeTable rope) {
     const EmbedArgs emb{d_embd_out ? d_embd : nullptr, d_embd_out, embd_type, embd_m, embd_k};
-    return launch_kernel(L, kFamOther, set_step_kernel, dim3(1), dim3(256), d_token, token, d_pos, pos, emb);
-}
-
-hipError_t launch_advance_pos(uint32_t* d_pos, const Launch& L) {
-    return launch_kernel(L, kFamOther, advance_pos_kernel, dim3(1), dim3(64), d_pos);
+    return launch_kernel(L, kFamOther, set_step_kernel, dim3(1), dim3(256), d_token, token, d_pos, pos, emb, rope);
 }
 
 }  // namespace wick_rocm

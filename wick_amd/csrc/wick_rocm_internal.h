@@ -212,12 +212,12 @@ hipError_t launch_attention_decode(const float* d_q, const void* d_k_cache, cons
                                    uint32_t seq_len, const uint32_t* d_pos, uint32_t max_seq, uint32_t n_heads, uint32_t n_kv_heads,
                                    uint32_t head_dim, float scale, const Launch& L, bool kv_f16 = false);
 // QK-norm + RoPE + KV append folded into the sequence-split attention kernel, then the merge (head_dim 32 / 64 / 128 / 256).
-// d_scratch as for launch_attention_decode.
+// d_scratch as for launch_attention_decode.  d_rope: the position's table (RopeTable) when there is one.
 bool attention_layer_applies(uint32_t head_dim);
 hipError_t launch_attention_layer(const float* d_q, const float* d_k, const float* d_v, const float* d_q_norm, const float* d_k_norm,
                                   void* d_k_cache, void* d_v_cache, float* d_out, float* d_scratch, uint32_t pos,
                                   const uint32_t* d_pos, uint32_t max_seq, uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, float eps,
-                                  float theta_scale, float scale, const Launch& L, bool kv_f16 = false);
+                                  float theta_scale, float scale, const Launch& L, bool kv_f16 = false, const float* d_rope = nullptr);
 hipError_t launch_shortconv_step(const float* d_proj, float* d_buffer, const float* d_conv_w, float* d_out, uint32_t hidden,
                                  uint32_t kernel_size, const Launch& L);
 hipError_t launch_rmsnorm_quantize(const float* d_x, const float* d_weight, uint32_t rows, uint32_t dim, uint32_t x_stride, float eps, int8_t* d_q,
@@ -230,20 +230,26 @@ hipError_t launch_residual_rmsnorm_quantize(float* d_x, const float* d_partial, 
                                             uint32_t x_stride, float eps, int8_t* d_q, float* d_scales, const Launch& L);
 hipError_t launch_silu_mul_quantize(const float* d_gate, const float* d_up, uint32_t n, uint32_t dim, int8_t* d_q, float* d_scales, const Launch& L);
 hipError_t launch_silu_mul(float* d_gate, const float* d_up, uint32_t n, const Launch& L);
+// The sines and cosines of a position's RoPE angles, {sin, cos} of head_dim / 2 pairs (head_dim floats, 8-byte aligned), filled by
+// the launch that sets or advances the position.  tab null: none.
+struct RopeTable {
+    float2* tab = nullptr;
+    uint32_t half = 0;
+    float theta_scale = 0.0f;
+};
 // d_history[pos] = pick (pos = *d_pos before it is advanced), when given.  d_partial: scratch of kArgmaxPartials keys, 8-byte aligned;
 // d_x 16-byte aligned.
 constexpr uint32_t kArgmaxPartials = 4096;  // 64 for the two-stage pick; up to one key per wave of a Q6_K LM head that leaves its own
 // d_embd_out non-null: the pick's row of the embedding (d_embd, type, m x k) is written there as the next step's input.
 hipError_t launch_argmax(const float* d_x, uint32_t n, unsigned long long* d_partial, uint32_t* d_out, uint32_t* d_token, uint32_t* d_pos,
                          uint32_t* d_history, uint32_t history_len, const Launch& L, const uint8_t* d_embd = nullptr, int embd_type = 0,
-                         uint32_t embd_m = 0, uint32_t embd_k = 0, float* d_embd_out = nullptr);
+                         uint32_t embd_m = 0, uint32_t embd_k = 0, float* d_embd_out = nullptr, RopeTable rope = {});
 // The second stage on its own, over n_partials keys that a producer has left in d_partial (n = the number of candidates; 0: pick 0).
 hipError_t launch_argmax_final(const unsigned long long* d_partial, uint32_t n_partials, uint32_t n, uint32_t* d_out, uint32_t* d_token, uint32_t* d_pos,
                                uint32_t* d_history, uint32_t history_len, const Launch& L, const uint8_t* d_embd = nullptr, int embd_type = 0,
-                               uint32_t embd_m = 0, uint32_t embd_k = 0, float* d_embd_out = nullptr);
+                               uint32_t embd_m = 0, uint32_t embd_k = 0, float* d_embd_out = nullptr, RopeTable rope = {});
 hipError_t launch_set_step(uint32_t* d_token, uint32_t token, uint32_t* d_pos, uint32_t pos, const Launch& L, const uint8_t* d_embd = nullptr,
-                           int embd_type = 0, uint32_t embd_m = 0, uint32_t embd_k = 0, float* d_embd_out = nullptr);
-hipError_t launch_advance_pos(uint32_t* d_pos, const Launch& L);
+                           int embd_type = 0, uint32_t embd_m = 0, uint32_t embd_k = 0, float* d_embd_out = nullptr, RopeTable rope = {});
 
 // n at and above which gemm_q8 uses the MFMA kernel (when k % 128 == 0): the counterpart of GEMM_MIN_N = 16
 // (wick/src/model/metal_lfm2.rs:18-21), set where the two routes cross on this GPU.  The multi-token GEMV streams the weight
