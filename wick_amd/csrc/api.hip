@@ -53,9 +53,10 @@ void noalloc_release(wick_rocm_ctx* ctx) {
     if (g_noalloc_owner[ctx->device] == ctx) g_noalloc_owner[ctx->device] = nullptr;
 }
 
-// A chunk between device memory and a pinned slot (either may be the source), 16-byte aligned, n pieces of 16 bytes.
-__global__ __launch_bounds__(256) void stage_copy_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, uint32_t n) {
-    const uint32_t step = gridDim.x * 256u;
+// A chunk between device memory and a pinned slot (either may be the source), 16-byte aligned at both ends.
+__global__ __launch_bounds__(256) void stage_copy_kernel(const uint4* __restrict__ src, uint4* __restrict__ dst, uint32_t bytes) {
+    const uint32_t step = gridDim.x * 256u, n = bytes / 16u;
+    if (blockIdx.x == 0 && threadIdx.x < bytes % 16u) reinterpret_cast<uint8_t*>(dst + n)[threadIdx.x] = reinterpret_cast<const uint8_t*>(src + n)[threadIdx.x];
     for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n; i += 4u * step) {
         uint4 v[4];
 #pragma unroll
@@ -182,11 +183,21 @@ int gemm_locked(wick_rocm_ctx* ctx, const wick_rocm_weight* w, const int8_t* d_q
 // 1.78 ms, 54 MB down in 1.5 (touched) - 1.8 ms (fresh); 1 MB slots 2.0 / 1.6, eight threads no faster.  A copy of up to two slots
 // goes through one of them, all pieces together, with one wait.
 int copy_pieces(wick_rocm_ctx* ctx, const HostPiece* pieces, size_t count, bool to_host) {
+    const auto padded = [](size_t n) { return (n + 15u) & ~size_t{15}; };
     size_t total = 0;
-    for (size_t i = 0; i < count; i++) total += pieces[i].bytes;
+    for (size_t i = 0; i < count; i++) total += padded(pieces[i].bytes);
     if (total == 0) return WICK_ROCM_OK;
     const auto issue = [&](char* dev, char* host, size_t n) {
         return to_host ? hipMemcpyAsync(host, dev, n, hipMemcpyDeviceToHost, ctx->stream) : hipMemcpyAsync(dev, host, n, hipMemcpyHostToDevice, ctx->stream);
+    };
+    // Copies go over the bus in a kernel where the device address allows it (the slots do): a copy engine's transfer takes 9 us
+    // longer to start and to be seen finished (256 KB of logits behind a step: 14.6 -> 6 us), and large copies' transfers and the
+    // events between them wait for each other across queues (2 MB chunks with an event behind each: 30 - 35 GB/s, ~48 by kernel).
+    const auto issue_chunk = [&](char* dev, char* host, size_t n) {
+        if (reinterpret_cast<uintptr_t>(dev) % 16u != 0) return issue(dev, host, n);
+        const uint32_t blocks = (uint32_t)((n + 4095u) / 4096u);
+        return launch_kernel(Launch{ctx->stream, nullptr}, kFamOther, stage_copy_kernel, dim3(blocks < 64u ? blocks : 64u), dim3(256),
+                             reinterpret_cast<const uint4*>(to_host ? dev : host), reinterpret_cast<uint4*>(to_host ? host : dev), (uint32_t)n);
     };
     if (!make_stage(ctx, total <= 2 * kStageSlotBytes ? 2 : kStageSlots)) {  // no pinned memory left: the runtime's way
         for (size_t i = 0; i < count; i++) WR_HIP(ctx, issue(static_cast<char*>(pieces[i].dev), static_cast<char*>(pieces[i].host), pieces[i].bytes));
@@ -197,14 +208,14 @@ int copy_pieces(wick_rocm_ctx* ctx, const HostPiece* pieces, size_t count, bool 
         size_t at = 0;
         for (size_t i = 0; i < count; i++) {
             if (!to_host) std::memcpy(ctx->stage + at, pieces[i].host, pieces[i].bytes);
-            WR_HIP(ctx, issue(static_cast<char*>(pieces[i].dev), ctx->stage + at, pieces[i].bytes));
-            at += pieces[i].bytes;
+            if (pieces[i].bytes) WR_HIP(ctx, issue_chunk(static_cast<char*>(pieces[i].dev), ctx->stage + at, pieces[i].bytes));
+            at += padded(pieces[i].bytes);
         }
         WR_HIP(ctx, hipStreamSynchronize(ctx->stream));
         at = 0;
         for (size_t i = 0; to_host && i < count; i++) {
             std::memcpy(pieces[i].host, ctx->stage + at, pieces[i].bytes);
-            at += pieces[i].bytes;
+            at += padded(pieces[i].bytes);
         }
         return WICK_ROCM_OK;
     }
@@ -214,13 +225,6 @@ int copy_pieces(wick_rocm_ctx* ctx, const HostPiece* pieces, size_t count, bool 
         for (size_t o = 0; o < pieces[i].bytes; o += kStageSlotBytes)
             chunks.push_back({static_cast<char*>(pieces[i].dev) + o, static_cast<char*>(pieces[i].host) + o,
                               pieces[i].bytes - o < kStageSlotBytes ? pieces[i].bytes - o : kStageSlotBytes});
-    // The chunks go over the bus in a kernel: a copy engine's transfers and the events between them wait for each other across queues
-    // (2 MB chunks with an event behind each: 30 - 35 GB/s by copy engine, ~48 by kernel).
-    const auto issue_chunk = [&](char* dev, char* host, size_t n) {
-        if (reinterpret_cast<uintptr_t>(dev) % 16u != 0 || n % 16u != 0) return issue(dev, host, n);
-        return launch_kernel(Launch{ctx->stream, nullptr}, kFamOther, stage_copy_kernel, dim3(64), dim3(256), reinterpret_cast<const uint4*>(to_host ? dev : host),
-                             reinterpret_cast<uint4*>(to_host ? host : dev), (uint32_t)(n / 16u));
-    };
     std::atomic<size_t> next{0};
     std::atomic<int> failed{(int)hipSuccess};
     const auto work = [&](int w) {
