@@ -78,6 +78,22 @@ def test_forward_matches_the_oracle_step_by_step(ctx, oracle, tmp_path, name):
     model.free()
 
 
+@pytest.mark.parametrize("hidden,wtype", [(256, W.Q4_0), (512, W.Q8_0), (1024, W.Q4_0), (1024, W.Q8_0), (2048, W.Q4_0)])
+def test_step_at_positions_around_the_split_edges(ctx, oracle, tmp_path, hidden, wtype):
+    """One record per head, a second split's first key, a partial last group of splits, both sides of the position up to which
+    the output projection merges the records itself (1024) -- for head counts 4 to 32, on a restored random state."""
+    model, ref, cfg = load(ctx, oracle, tmp_path, context=1100, n_layers=1, hidden=hidden, inter=256, n_heads=hidden // 64, kv_heads=(hidden // 128,),
+                           vocab=256, wtype=wtype, embd_type=W.Q8_0, seed=7)
+    kvd, rng = hidden // 2, np.random.default_rng(hidden)
+    for pos in (0, 1, 63, 64, 300, 1022, 1023, 1024):
+        k, v = rng.standard_normal((2, pos, kvd)).astype(np.float32)
+        if pos:
+            model.restore_state(np.concatenate([k.ravel(), v.ravel()]).view(np.uint8), pos)
+        state = {"seq_len": pos, "layers": [{"k": list(k), "v": list(v)}]}
+        check_step(model.forward(pos % 256, pos), ref.forward(pos % 256, pos, state), ref.min_margin, f"hidden {hidden} pos {pos}")
+    model.free()
+
+
 def test_larger_model_longer_sequence(ctx, oracle, tmp_path):
     """Six layers, 24 positions: strict until the oracle reports the first near-tie, bounded afterwards."""
     model, ref, cfg = load(ctx, oracle, tmp_path, n_layers=6, hidden=512, inter=1024, n_heads=8, kv_heads=(0, 0, 4, 0, 8, 2), vocab=1000,

@@ -49,6 +49,24 @@ hipError_t launch_gemv_shortconv_f32(int type, const uint8_t* d_w, uint32_t m, u
     return type == kTypeQ4_0 ? dispatch<2, 1, true>(a, num_cus, L) : dispatch<8, 1, true>(a, num_cus, L);
 }
 
+bool attn_merge_kernel_applies(const uint8_t* d_w, uint32_t k, uint32_t head_dim) {
+    return head_dim == 64 && k <= 1024u && k % 64u == 0 && reinterpret_cast<uintptr_t>(d_w) % 4u == 0;
+}
+
+hipError_t launch_gemv_attn_merge(int type, const uint8_t* d_w, uint32_t m, uint32_t k, const float* d_partials, const uint32_t* d_pos, uint32_t splits,
+                                  uint32_t max_seq, float* d_y, int accumulate, int num_cus, const Launch& L) {
+    GemvArgs a{};
+    a.batch.w[0] = d_w, a.batch.y[0] = d_y, a.batch.row_end[0] = m, a.batch.count = 1;
+    a.xf = d_partials;
+    a.xform = kXformAttnMerge, a.xaux = reinterpret_cast<const float*>(d_pos);
+    a.splits = splits, a.max_seq = max_seq;
+    a.x_stride = k;
+    a.k = k;
+    a.n = 1;
+    a.accumulate = accumulate;
+    return type == kTypeQ4_0 ? dispatch<2, 1, true>(a, num_cus, L) : dispatch<8, 1, true>(a, num_cus, L);
+}
+
 hipError_t launch_gemv_gated_f32(int type, const uint8_t* d_w_gate, const uint8_t* d_w_up, uint32_t m, uint32_t k, const float* d_x,
                                  float* d_out, int num_cus, const Launch& L, int xform, const float* d_aux, float eps, float* conv_state,
                                  const float* conv_proj, uint32_t conv_hidden, uint32_t conv_kernel) {

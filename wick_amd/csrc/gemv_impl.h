@@ -49,6 +49,7 @@ struct GemvArgs {
     int32_t* dots;      // parity hook (DUMP variants): raw i32 block dots, [token][row][block], instead of y
     int xform;          // kXformNone / kXformRmsNorm / kXformSiluMul (host-side selector of the kernel variant)
     int gated;          // host-side selector of the GATED variant: batch.w[0] = gate, batch.w[1] = up, y[0][r] = silu(gate_r) * up_r
+    uint32_t splits, max_seq;  // kXformAttnMerge: partial records per head and the cache's rows
     uint32_t x_stride;
     uint32_t k;
     uint32_t n;         // tokens (1 for decode)
@@ -93,8 +94,21 @@ enum { kDirect = 0, kDirectNT = 1, kSpan = 2 };
 //                  in front of its out projection: x = [b | c | x'] (3k floats), out = c * (s0 w0 + s1 w1 + (b x') w2)
 //                  with the rolling state s0, s1 READ ONLY -- many workgroups read it, so it is advanced by a later
 //                  launch (the side job of the gate / up kernel).  Kernel size 3, k <= 2048.
+//   kXformAttnMerge  the merge of a decode step's attention partials (attention_merge, bit for bit; head_dim 64) in front of the
+//                  output projection: x = the partial records {max, sum, acc[64]} of [head][split], aux = the position.  The
+//                  first 16 splits' records are requested with everything else (enqueue_step uses it up to there).
+//                  Against a merge launch: a step of the 350M shape (6 attention layers) 251 -> 244 us at position 30,
+//                  260 -> 253 at 600, 268 -> 263 at 980, 278 -> 276 at 1500, 286 -> 294 at 2500.  For k = 2048 every
+//                  workgroup reads twice the records: 160 -> 165 us at 980 and nothing gained at 30, hence k <= 1024.
 // Every workgroup redoes the transform on the whole vector (k <= 8192 floats, a few per thread): cheaper than a
 // launch of its own.
+
+// A quad of head quad / 16's weighted value sum of one split (records are 8-byte aligned).
+__device__ __forceinline__ float4 merge_quad(const float* rec, uint32_t splits, uint32_t split, uint32_t quad) {
+    const float2* p = reinterpret_cast<const float2*>(rec + ((size_t)(quad >> 4) * splits + split) * 66u + 2u + 4u * (quad & 15u));
+    const float2 a = p[0], b = p[1];
+    return make_float4(a.x, a.y, b.x, b.y);
+}
 
 // The leading scalar parameters repeat fields of `a` (x = a.xf for the fused variant, a.xq
 // otherwise; w0 / rows0 = weight 0 of the batch; aux / aux2 = a.xaux / a.xaux2, the transform's operands).  Passed on their own, at the front,
@@ -146,10 +160,33 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
     constexpr int kQuadRounds = LPR * NCHUNK <= 16 ? 1 : LPR * NCHUNK / 16;
     const auto past = [&](int i) { return i > kQuadRounds / 2 && (uint32_t)i * 64u * kFusedWaves >= (p_k >> 2); };
     float4 xv[FUSEQ ? kQuadRounds : 1];
-    float4 av[XF != kXformNone && XF != kXformShortConv ? kQuadRounds : 1];  // the transform's second operand, same quads
+    // kXformAttnMerge: this wave's heads' {max, sum} per split (one lane each), this thread's quads of the first splits
+    constexpr int kMergeHeads = XF == kXformAttnMerge ? LPR * NCHUNK / kFusedWaves : 1, kMergeAhead = 16, kRecord = 66;
+    float m_part[kMergeHeads], l_part[kMergeHeads];
+    float4 o_part[XF == kXformAttnMerge ? kQuadRounds : 1][XF == kXformAttnMerge ? kMergeAhead : 1];
+    uint32_t active = 0;  // splits with a record
+    float4 av[XF == kXformRmsNorm || XF == kXformSiluMul ? kQuadRounds : 1];  // the transform's second operand, same quads
     float4 cv[XF == kXformShortConv ? kQuadRounds : 1][7];  // conv operands: c, x', state 0, state 1, three quads of the kernel (xv holds b)
     if constexpr (FUSEQ) {
         const uint32_t quads = p_k >> 2;
+        if constexpr (XF == kXformAttnMerge) {
+            const float* rec = static_cast<const float*>(p_x);
+            const uint32_t seq = min(*reinterpret_cast<const uint32_t*>(p_aux) + 1u, a.max_seq);
+            active = min((seq + 63u) / 64u, a.splits);
+#pragma unroll
+            for (int t = 0; t < kMergeHeads; t++) {
+                const uint32_t h = min((threadIdx.x >> 6) + kFusedWaves * t, (p_k >> 6) - 1u);
+                const float* r = rec + ((size_t)h * a.splits + min(lane, active - 1u)) * kRecord;
+                m_part[t] = r[0], l_part[t] = r[1];
+            }
+#pragma unroll
+            for (int i = 0; i < kQuadRounds; i++) {
+                if (past(i)) break;
+                const uint32_t quad = min(threadIdx.x + i * 64 * kFusedWaves, quads - 1);
+#pragma unroll
+                for (int j = 0; j < kMergeAhead; j++) o_part[i][j] = merge_quad(rec, a.splits, min((uint32_t)j, active - 1u), quad);
+            }
+        } else
 #pragma unroll
         for (int i = 0; i < kQuadRounds; i++) {
             const uint32_t quad = threadIdx.x + i * 64 * kFusedWaves;
@@ -168,7 +205,7 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
                 cv[i][2] = st[quad], cv[i][3] = st[quads + quad];
                 cv[i][4] = cw[3 * quad], cv[i][5] = cw[3 * quad + 1], cv[i][6] = cw[3 * quad + 2];  // [channel][tap] of four channels
             }
-        } else if constexpr (XF != kXformNone) {
+        } else if constexpr (XF != kXformNone && XF != kXformAttnMerge) {
             const float4* aux = reinterpret_cast<const float4*>(p_aux);
 #pragma unroll
             for (int i = 0; i < kQuadRounds; i++) {
@@ -351,6 +388,53 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
                     xv[i].x = silu_mul(xv[i].x, av[i].x), xv[i].y = silu_mul(xv[i].y, av[i].y);
                     xv[i].z = silu_mul(xv[i].z, av[i].z), xv[i].w = silu_mul(xv[i].w, av[i].w);
                 }
+            }
+        }
+        if constexpr (XF == kXformAttnMerge) {
+            __shared__ __align__(16) float wts[LPR * NCHUNK * 64], tot[LPR * NCHUNK];  // heads: k / 64 <= LPR NCHUNK
+#pragma unroll
+            for (int t = 0; t < kMergeHeads; t++) {
+                const uint32_t h = (threadIdx.x >> 6) + kFusedWaves * t;
+                const bool on = lane < active;
+                const float m_i = on ? m_part[t] : -__builtin_inff(), l_i = on ? l_part[t] : 0.0f;
+                const float m = wave_max_f32(m_i);
+                const float w = on ? ggml_expf(m_i - m) : 0.0f;
+                const float l = wave_sum_f32(l_i * w);
+                wts[h * 64u + lane] = w;
+                if (lane == 0) tot[h] = l;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < kQuadRounds; i++) {
+                if (past(i)) break;
+                const uint32_t quad = min(threadIdx.x + i * 64 * kFusedWaves, quads - 1), h = quad >> 4;
+                float o[4][4] = {};  // [split % 4][dim]: the four groups of attention_merge's threads
+                const auto four = [&](const float4 (&v)[4], uint32_t i0) {
+                    const float4 w4 = *reinterpret_cast<const float4*>(&wts[h * 64u + i0]);
+                    const float w[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const bool on = i0 + j < active;
+                        o[j][0] = __fadd_rn(o[j][0], on ? __fmul_rn(v[j].x, w[j]) : 0.0f), o[j][1] = __fadd_rn(o[j][1], on ? __fmul_rn(v[j].y, w[j]) : 0.0f);
+                        o[j][2] = __fadd_rn(o[j][2], on ? __fmul_rn(v[j].z, w[j]) : 0.0f), o[j][3] = __fadd_rn(o[j][3], on ? __fmul_rn(v[j].w, w[j]) : 0.0f);
+                    }
+                };
+#pragma unroll
+                for (int j = 0; j < kMergeAhead; j += 4) {
+                    if ((uint32_t)j >= active) break;
+                    const float4 v[4] = {o_part[i][j], o_part[i][j + 1], o_part[i][j + 2], o_part[i][j + 3]};
+                    four(v, j);
+                }
+                for (uint32_t j = kMergeAhead; j < active; j += 4) {
+                    float4 v[4];
+#pragma unroll
+                    for (int e = 0; e < 4; e++) v[e] = merge_quad(static_cast<const float*>(p_x), a.splits, min(j + e, active - 1u), quad);
+                    four(v, j);
+                }
+                float r[4];
+#pragma unroll
+                for (int d = 0; d < 4; d++) r[d] = __fdiv_rn(__fadd_rn(__fadd_rn(__fadd_rn(o[0][d], o[1][d]), o[2][d]), o[3][d]), tot[h]);
+                xv[i] = make_float4(r[0], r[1], r[2], r[3]);
             }
         }
         if constexpr (XF == kXformShortConv) {
@@ -662,6 +746,14 @@ hipError_t launch_pairs_u(GemvArgs& a, uint32_t total_rows, int num_cus, const L
                 return go(gemv_pairs_kernel<TYPE, LPR, NCHUNK, U, NT, FUSEQ, false, kSmall, kXformShortConv>);
             } else {
                 return hipErrorInvalidValue;  // shortconv_kernel_applies() keeps such shapes away
+            }
+        }
+        if (a.xform == kXformAttnMerge) {  // one weight, k <= 2048 (attn_merge_kernel_applies)
+            if constexpr (LPR >= 4 && LPR <= 32 && NCHUNK == 1) {
+                if (mode == kSpan) return go(gemv_pairs_kernel<TYPE, LPR, NCHUNK, U, NT, FUSEQ, false, kSpan, kXformAttnMerge>);
+                return go(gemv_pairs_kernel<TYPE, LPR, NCHUNK, U, NT, FUSEQ, false, kSmall, kXformAttnMerge>);
+            } else {
+                return hipErrorInvalidValue;
             }
         }
         if (a.xform == kXformRmsNorm) return with_xform(std::integral_constant<int, kXformRmsNorm>{});

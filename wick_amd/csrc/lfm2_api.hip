@@ -196,7 +196,7 @@ size_t wick_rocm_attention_block_scratch_bytes(uint32_t max_seq, uint32_t n_head
 static int attention_block_kv(wick_rocm_ctx* ctx, float* d_q, float* d_k, const float* d_v, const float* d_q_norm, const float* d_k_norm,
                               void* d_k_cache, void* d_v_cache, float* d_out, void* d_scratch, uint32_t pos, const uint32_t* d_pos,
                               uint32_t max_seq, uint32_t head_dim, uint32_t n_heads, uint32_t n_kv_heads, float eps, float theta_scale, bool kv_f16,
-                              const float* d_rope = nullptr) {
+                              const float* d_rope = nullptr, bool merge = true) {
     WR_ENTER(ctx);
     if (!d_q || !d_k || !d_v || !d_q_norm || !d_k_norm || !d_k_cache || !d_v_cache || !d_out || !d_scratch)
         return fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "attention_block: null device pointer");
@@ -210,7 +210,7 @@ static int attention_block_kv(wick_rocm_ctx* ctx, float* d_q, float* d_k, const 
     hipError_t e;
     if (attention_layer_applies(head_dim)) {
         e = launch_attention_layer(d_q, d_k, d_v, d_q_norm, d_k_norm, d_k_cache, d_v_cache, d_out, partials, pos, d_pos, max_seq, n_heads,
-                                   n_kv_heads, head_dim, eps, theta_scale, scale, ctx->launch(), kv_f16, d_rope);
+                                   n_kv_heads, head_dim, eps, theta_scale, scale, ctx->launch(), kv_f16, d_rope, merge);
     } else {
         e = launch_qk_norm_rope(d_q, d_k, d_v, d_q_norm, d_k_norm, d_k_cache, d_v_cache, pos, d_pos, max_seq, head_dim, n_heads, n_kv_heads, eps,
                                 theta_scale, ctx->launch(), 1, 0, 0, kv_f16);
@@ -363,7 +363,7 @@ struct wick_rocm_lfm2 {
     void* shift_stage = nullptr;   // staging rows of a context shift, allocated by the first one
     bool kv_f16 = false;           // the KV caches hold f16 rows (wick_rocm_lfm2_load_kv); f32 otherwise
     size_t kv_elem() const { return kv_f16 ? 2 : 4; }
-    wick_rocm_graph* g_step[3] = {nullptr, nullptr, nullptr};  // one captured step per StepMode
+    wick_rocm_graph* g_step[2][3] = {};  // captured steps: [position below kFoldMergeBelow][StepMode]
     bool use_graph = true;
     std::mutex mu;
 };
@@ -420,8 +420,9 @@ int upload_weight(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, const wick_gguf* g, con
 
 void release(wick_rocm_ctx* ctx, wick_rocm_lfm2* m) {
     wick_rocm_sync(ctx);
-    for (wick_rocm_graph* g : m->g_step)
-        if (g) wick_rocm_graph_destroy(ctx, g);
+    for (auto& modes : m->g_step)
+        for (wick_rocm_graph* g : modes)
+            if (g) wick_rocm_graph_destroy(ctx, g);
     for (wick_rocm_weight* w : m->weights) wick_rocm_weight_free(ctx, w);
     for (void* b : m->buffers) wick_rocm_buffer_free(ctx, b);
     if (m->h_tokens) (void)hipHostFree(m->h_tokens);
@@ -448,9 +449,14 @@ int gemv_residual(wick_rocm_ctx* ctx, const wick_rocm_weight* w, float* y, const
     return wick_rocm_matmul_f32(ctx, w, x, 0, 1, w->k, y, 0, w->m, 1);
 }
 
+// Positions up to which the output projection merges the attention partials itself (16 splits, read in one round trip); beyond, the
+// records of all heads that each of its workgroups then reads cost what the launch costs.
+constexpr uint32_t kFoldMergeBelow = 1024;  // (measured: kXformAttnMerge, gemv_impl.h)
+
 // Enqueues one decode step that reads token / pos from the device: run_layers + the tied LM head
 // (wick/src/model/lfm2.rs:1020-1124, 2258-2289), optionally the greedy pick.
-int enqueue_step(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, StepMode mode) {
+// near_start: the position is below kFoldMergeBelow.
+int enqueue_step(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, StepMode mode, bool near_start) {
     const wick_rocm_lfm2_config& c = m->cfg;
     const uint32_t hs = c.hidden_size, hd = hs / c.n_heads;
     // m->hidden already holds the token's embedding row: set_step (or the previous step's greedy pick) looked it up
@@ -466,11 +472,20 @@ int enqueue_step(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, StepMode mode) {
                 if ((rc = gemv_residual(ctx, L.out_proj, m->hidden, m->gated))) break;
             }
         } else {
+            const bool fold = near_start && L.o->type != kTypeQ6_K && attn_merge_kernel_applies(static_cast<const uint8_t*>(L.o->d), L.o->k, hd);
             if ((rc = gemv_normed(ctx, {L.q, L.k, L.v}, {m->q, m->k, m->v}, m->hidden, L.attn_norm, c.rms_norm_eps))) break;
             if ((rc = attention_block_kv(ctx, m->q, m->k, m->v, L.q_norm, L.k_norm, L.k_cache, L.v_cache, m->attn, m->scores, 0, m->d_pos,
-                                         c.max_seq_len, hd, c.n_heads, L.n_kv, c.rms_norm_eps, m->theta_scale, m->kv_f16, m->rope)))
+                                         c.max_seq_len, hd, c.n_heads, L.n_kv, c.rms_norm_eps, m->theta_scale, m->kv_f16, m->rope, !fold)))
                 break;
-            if ((rc = gemv_residual(ctx, L.o, m->hidden, m->attn))) break;
+            if (!fold) {
+                if ((rc = gemv_residual(ctx, L.o, m->hidden, m->attn))) break;
+            } else {  // the partials' merge in the output projection's prologue
+                std::lock_guard<std::recursive_mutex> lk(ctx->mu);
+                const hipError_t e = launch_gemv_attn_merge(L.o->type, static_cast<const uint8_t*>(L.o->d), L.o->m, L.o->k, m->scores, m->d_pos,
+                                                            attention_splits(c.max_seq_len), c.max_seq_len, m->hidden, 1, ctx->num_cus, ctx->launch());
+                if (e != hipSuccess) rc = fail_hip(ctx, e, "output projection launch");
+                if (rc) break;
+            }
         }
         // gate = silu(W_gate n(hidden)) * (W_up n(hidden)); hidden += W_down gate
         if (L.conv_fused)
@@ -489,15 +504,15 @@ int enqueue_step(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, StepMode mode) {
                                  m->d_history, c.max_seq_len, m->hidden, m->rope_table());
 }
 
-int step_graph(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, StepMode mode, wick_rocm_graph** out) {
-    wick_rocm_graph*& g = m->g_step[mode];
+int step_graph(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, StepMode mode, bool near_start, wick_rocm_graph** out) {
+    wick_rocm_graph*& g = m->g_step[near_start][mode];
     if (g && graph_is_stale(ctx, g)) {  // the context's scratch moved since the capture (another model, a wider matmul): capture again
         wick_rocm_graph_destroy(ctx, g);
         g = nullptr;
     }
     if (!g) {
         if (int rc = wick_rocm_graph_begin(ctx)) return rc;
-        const int rc = enqueue_step(ctx, m, mode);
+        const int rc = enqueue_step(ctx, m, mode, near_start);
         wick_rocm_graph* captured = nullptr;
         const int rc_end = wick_rocm_graph_end(ctx, &captured);  // always end the capture
         if (rc) {
@@ -512,16 +527,17 @@ int step_graph(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, StepMode mode, wick_rocm_g
 }
 
 // One step on the context's stream: a replay of the captured graph, or the same launches enqueued one by one.
-int run_step(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, StepMode mode) {
+int run_step(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, StepMode mode, uint32_t pos) {
+    const bool near_start = pos < kFoldMergeBelow;
     // per-dispatch timing cannot see inside a graph: while it is on, steps are enqueued launch by launch
     bool timing;
     {
         std::lock_guard<std::recursive_mutex> lk(ctx->mu);
         timing = ctx->timer.enabled;
     }
-    if (!m->use_graph || timing) return enqueue_step(ctx, m, mode);
+    if (!m->use_graph || timing) return enqueue_step(ctx, m, mode, near_start);
     wick_rocm_graph* g = nullptr;
-    if (int rc = step_graph(ctx, m, mode, &g)) return rc;
+    if (int rc = step_graph(ctx, m, mode, near_start, &g)) return rc;
     return wick_rocm_graph_launch(ctx, g);
 }
 
@@ -860,7 +876,7 @@ int wick_rocm_lfm2_forward(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uint32_t t
     std::lock_guard<std::recursive_mutex> whole_step(ctx->mu);  // nothing else gets onto the context's stream (or into a capture) in between
     if (int rc = check_step(ctx, model, token, pos, 1)) return rc;
     if (int rc = set_step(ctx, model, token, pos)) return rc;
-    if (int rc = run_step(ctx, model, kStepLogits)) return rc;
+    if (int rc = run_step(ctx, model, kStepLogits, pos)) return rc;
     if (logits) return wick_rocm_download(ctx, logits, model->logits, (size_t)model->cfg.vocab_size * sizeof(float));
     return wick_rocm_sync(ctx);
 }
@@ -882,7 +898,7 @@ static int prefill_locked(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, const uint3
                 if (e != hipSuccess) return fail_hip(ctx, e, "set_step launch");
                 if (int rc = wick_rocm_upload(ctx, model->hidden, embeddings + (size_t)j * c.hidden_size, (size_t)c.hidden_size * sizeof(float))) return rc;
             }
-            if (int rc = run_step(ctx, model, mode)) return rc;
+            if (int rc = run_step(ctx, model, mode, start_pos + j)) return rc;
         }
         if (logits) return wick_rocm_download(ctx, logits, model->logits, (size_t)c.vocab_size * sizeof(float));
         return wick_rocm_sync(ctx);
@@ -959,7 +975,7 @@ int wick_rocm_lfm2_generate_greedy(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, ui
     if (int rc = check_step(ctx, model, token, pos, n)) return rc;
     if (int rc = set_step(ctx, model, token, pos)) return rc;
     for (uint32_t i = 0; i < n; i++)  // the pick of step i is written to the device-side token and position pos + i of the history
-        if (int rc = run_step(ctx, model, kStepGreedy)) return rc;
+        if (int rc = run_step(ctx, model, kStepGreedy, pos + i)) return rc;
     return wick_rocm_download(ctx, out_tokens, model->d_history + pos, (size_t)n * sizeof(uint32_t));
 }
 
@@ -977,7 +993,7 @@ static int step_locked(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uint32_t token
     } else if (int rc = set_step(ctx, model, token, pos)) {
         return rc;
     }
-    if (int rc = run_step(ctx, model, mode)) return rc;
+    if (int rc = run_step(ctx, model, mode, pos)) return rc;
     if (!out) return wick_rocm_sync(ctx);
     return mode == kStepHidden ? wick_rocm_download(ctx, out, model->gated, (size_t)c.hidden_size * sizeof(float))
                                : wick_rocm_download(ctx, out, model->logits, (size_t)c.vocab_size * sizeof(float));

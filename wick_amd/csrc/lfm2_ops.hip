@@ -1763,7 +1763,7 @@ bool attention_layer_applies(uint32_t head_dim) { return head_dim == 32 || head_
 hipError_t launch_attention_layer(const float* d_q, const float* d_k, const float* d_v, const float* d_q_norm, const float* d_k_norm,
                                   void* d_k_cache, void* d_v_cache, float* d_out, float* d_scratch, uint32_t pos,
                                   const uint32_t* d_pos, uint32_t max_seq, uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, float eps,
-                                  float theta_scale, float scale, const Launch& L, bool kv_f16, const float* d_rope) {
+                                  float theta_scale, float scale, const Launch& L, bool kv_f16, const float* d_rope, bool merge) {
     AttentionLayerArgs f{};
     f.at = AttentionArgs{nullptr, d_k_cache, d_v_cache, d_out, d_scratch, d_pos, pos + 1u, max_seq, n_heads, n_kv_heads, head_dim, scale};
     f.q_raw = d_q, f.k_raw = d_k, f.v = d_v, f.q_norm = d_q_norm, f.k_norm = d_k_norm;
@@ -1786,7 +1786,7 @@ hipError_t launch_attention_layer(const float* d_q, const float* d_k, const floa
         if (kMax >= 4 && group % 4u == 0) e = go(std::integral_constant<int, kMax>{});
         else if (kMax >= 2 && group % 2u == 0) e = go(std::integral_constant<int, kMax < 2 ? kMax : 2>{});
         else e = go(std::integral_constant<int, 1>{});
-        if (e != hipSuccess) return e;
+        if (e != hipSuccess || !merge) return e;
         return launch_kernel(L, kFamOther, attention_combine_kernel<HD>, dim3(n_heads), block, f.at, splits);
     };
     switch (head_dim) {

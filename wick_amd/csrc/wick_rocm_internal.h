@@ -88,7 +88,7 @@ hipError_t launch_gemv(int type, const GemvBatch& batch, uint32_t k, const int8_
 // kernel).  Only when pairs_kernel_applies() and d_x is 16-byte aligned.
 bool pairs_kernel_applies(const GemvBatch& batch, uint32_t k);
 // xform: what is done to x before it is quantized (d_aux: the RMSNorm weights / the "up" vector, k floats, 16-byte aligned).
-enum { kXformNone = 0, kXformRmsNorm = 1, kXformSiluMul = 2, kXformShortConv = 3 };
+enum { kXformNone = 0, kXformRmsNorm = 1, kXformSiluMul = 2, kXformShortConv = 3, kXformAttnMerge = 4 };
 hipError_t launch_gemv_f32(int type, const GemvBatch& batch, uint32_t k, const float* d_x, int accumulate, int num_cus,
                            const Launch& L, int xform = kXformNone, const float* d_aux = nullptr, float eps = 0.0f);
 
@@ -96,6 +96,11 @@ hipError_t launch_gemv_f32(int type, const GemvBatch& batch, uint32_t k, const f
 // x' = xform(x) quantized to Q8_0 (xform: none or RMSNorm).  Only when gated_kernel_applies() (even block count,
 // k <= 4096, 4-byte aligned weights) and d_x / d_aux are 16-byte aligned.
 bool gated_kernel_applies(const uint8_t* d_w_gate, const uint8_t* d_w_up, uint32_t k);
+// y (+)= W * quantize(merge of the heads' partials): the output projection behind launch_attention_layer(merge = false), whose partial
+// records [k / 64 heads][splits][66] d_partials holds; the position is *d_pos.  Only when attn_merge_kernel_applies().
+bool attn_merge_kernel_applies(const uint8_t* d_w, uint32_t k, uint32_t head_dim);
+hipError_t launch_gemv_attn_merge(int type, const uint8_t* d_w, uint32_t m, uint32_t k, const float* d_partials, const uint32_t* d_pos, uint32_t splits,
+                                  uint32_t max_seq, float* d_y, int accumulate, int num_cus, const Launch& L);
 // conv_state non-null: the first workgroups also advance that rolling short-conv state by one token (slot s <- slot s + 1, last
 // slot <- b * x of conv_proj = [b | c | x], conv_hidden floats each, conv_hidden % 4 == 0, 16-byte aligned): what
 // launch_shortconv_step does to the state, for a layer whose conv output went through launch_gemv_shortconv_f32.
@@ -212,12 +217,13 @@ hipError_t launch_attention_decode(const float* d_q, const void* d_k_cache, cons
                                    uint32_t seq_len, const uint32_t* d_pos, uint32_t max_seq, uint32_t n_heads, uint32_t n_kv_heads,
                                    uint32_t head_dim, float scale, const Launch& L, bool kv_f16 = false);
 // QK-norm + RoPE + KV append folded into the sequence-split attention kernel, then the merge (head_dim 32 / 64 / 128 / 256).
-// d_scratch as for launch_attention_decode.  d_rope: the position's table (RopeTable) when there is one.
+// d_scratch as for launch_attention_decode.  d_rope: the position's table (RopeTable) when there is one.  merge false: the
+// partials stay in d_scratch, d_out is not written.
 bool attention_layer_applies(uint32_t head_dim);
 hipError_t launch_attention_layer(const float* d_q, const float* d_k, const float* d_v, const float* d_q_norm, const float* d_k_norm,
                                   void* d_k_cache, void* d_v_cache, float* d_out, float* d_scratch, uint32_t pos,
                                   const uint32_t* d_pos, uint32_t max_seq, uint32_t n_heads, uint32_t n_kv_heads, uint32_t head_dim, float eps,
-                                  float theta_scale, float scale, const Launch& L, bool kv_f16 = false, const float* d_rope = nullptr);
+                                  float theta_scale, float scale, const Launch& L, bool kv_f16 = false, const float* d_rope = nullptr, bool merge = true);
 hipError_t launch_shortconv_step(const float* d_proj, float* d_buffer, const float* d_conv_w, float* d_out, uint32_t hidden,
                                  uint32_t kernel_size, const Launch& L);
 hipError_t launch_rmsnorm_quantize(const float* d_x, const float* d_weight, uint32_t rows, uint32_t dim, uint32_t x_stride, float eps, int8_t* d_q,
