@@ -148,6 +148,47 @@ def test_accumulate(ctx, oracle, dtype, n):
         assert_f32_parity(fetch_gemm(d_y, m, n, m, W.LAYOUT_TOKEN_MAJOR), ref, "gemm accumulate")
 
 
+@pytest.mark.parametrize("dtype", [W.Q4_0, W.Q8_0])
+@pytest.mark.parametrize("layout", [W.LAYOUT_ROW_MAJOR, W.LAYOUT_TOKEN_MAJOR])
+@pytest.mark.parametrize("ms,k", [
+    ((100, 33, 7), 512),       # ragged rows, per-lane loads
+    ((1500, 500, 12), 1024),   # span loads
+    ((70, 64, 1), 4608),       # two chunks of pairs per row
+    ((140001, 3, 1), 64),      # several passes per wave
+    ((65, 40, 2), 96),         # odd block count: the generic kernel
+])
+def test_one_token_accumulates_into_a_column(ctx, oracle, dtype, layout, ms, k):
+    """y += W x of ONE token into a column of a [rows][N] matrix (row-major, a stride that is no extent) and into a strided
+    token-major row, by wick_rocm_gemm_q8 per weight and by wick_rocm_gemm_q8_multi: every other element stays."""
+    rm = layout == W.LAYOUT_ROW_MAJOR
+    col, stride = 2, 5 if rm else sum(ms) + 9
+    with Problem(ctx, oracle, dtype, ms[0], k, 1, seed=ms[0] + k + dtype) as p:
+        wbs = [p.wb] + [oracle.synth_weight(dtype, m, k, 50 + i, 0.02) for i, m in enumerate(ms[1:])]
+        ws = [p.w] + [ctx.upload_weight(wb, dtype, m, k) for wb, m in zip(wbs[1:], ms[1:])]
+        offs = np.concatenate([[0], np.cumsum(ms)[:-1]])
+        elem = [int(o) * stride + col if rm else int(o) for o in offs]
+        y0 = oracle.fill_normal(21, 1.0, sum(ms) * stride if rm else stride)
+        step, want, touched = stride if rm else 1, y0.copy(), np.zeros(y0.size, bool)
+        for wb, m, e in zip(wbs, ms, elem):
+            at = slice(e, e + (m - 1) * step + 1, step)
+            want[at] += oracle.gemv_q8(dtype, wb, p.s[0], p.q[0], m, k)
+            touched[at] = True
+        for multi in (False, True):
+            d_y = ctx.to_device(y0)
+            ys = [d_y.ptr + 4 * e for e in elem]
+            if multi:
+                ctx.gemm_preq_multi(ws, p.d_s, p.d_q, 1, ys, stride, layout=layout, accumulate=True)
+            else:
+                for w, y in zip(ws, ys):
+                    ctx.gemm_preq(w, p.d_s, p.d_q, 1, y, y_stride=stride, layout=layout, accumulate=True)
+            y = d_y.download(np.float32, y0.size)
+            assert np.array_equal(y[~touched], y0[~touched])
+            assert_f32_parity(y[touched], want[touched], f"one token, {'multi' if multi else 'single'}")
+            d_y.free()
+        for w in ws[1:]:
+            w.free()
+
+
 def test_weight_free_releases_both_copies(ctx, oracle):
     """Uploading and freeing a weight over and over leaves the device's free memory where it was: the raw blocks and the
     GEMM's copy both go (read through hipMemGetInfo of the HIP runtime the library itself is linked against)."""

@@ -270,7 +270,11 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
     uint32_t span_tail[U][NCHUNK];  // kSpan: where the dword remainder of the span starts
     bool rvalid[U];
     uint32_t lrow[U];
-    // Decode launches that add to y ask for the old values with the weights instead of at the end, behind everything.
+    // Where the sum of row `row` and token `tok` goes.  (The early load below and the store both take it from here.)
+    const auto y_at = [&](uint32_t row, uint32_t tok) {
+        return a.y_row_major ? ybase + (size_t)row * a.y_stride + tok : ybase + (size_t)tok * a.y_stride + row;
+    };
+    // Single-token launches that add to y ask for the old values with the weights instead of at the end, behind everything.
     constexpr bool kEarlyY = NT == 1 && !GATED && !DUMP;
     float yold[kEarlyY ? U : 1];
     __shared__ __align__(16) uint8_t span_lds[MODE == kSpan ? (FUSEQ ? kFusedWaves : 1) * 64 * PT::BYTES : 16];
@@ -322,7 +326,7 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
         if constexpr (kEarlyY) {
             if (a.accumulate) {
 #pragma unroll
-                for (int u = 0; u < U; u++) yold[u] = ybase[min(lrow[u], rows - 1)];
+                for (int u = 0; u < U; u++) yold[u] = *y_at(min(lrow[u], rows - 1), tok0);
             }
         }
     };
@@ -580,8 +584,7 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
                     if ((u & 1) == 0) gate_sum = tot;
                     else if (sub == 0 && rvalid[u]) ybase[lrow[u]] = silu_mul(gate_sum, tot);
                 } else if (sub == 0 && rvalid[u] && tok0 + t < a.n) {
-                    float* dst = a.y_row_major ? ybase + (size_t)lrow[u] * a.y_stride + (tok0 + t)
-                                               : ybase + (size_t)(tok0 + t) * a.y_stride + lrow[u];
+                    float* const dst = y_at(lrow[u], tok0 + t);
                     if constexpr (kEarlyY) *dst = a.accumulate ? yold[u] + tot : tot;
                     else *dst = a.accumulate ? *dst + tot : tot;
                 }
