@@ -148,47 +148,6 @@ def test_accumulate(ctx, oracle, dtype, n):
         assert_f32_parity(fetch_gemm(d_y, m, n, m, W.LAYOUT_TOKEN_MAJOR), ref, "gemm accumulate")
 
 
-@pytest.mark.parametrize("dtype", [W.Q4_0, W.Q8_0])
-@pytest.mark.parametrize("layout", [W.LAYOUT_ROW_MAJOR, W.LAYOUT_TOKEN_MAJOR])
-@pytest.mark.parametrize("ms,k", [
-    ((100, 33, 7), 512),       # ragged rows, per-lane loads
-    ((1500, 500, 12), 1024),   # span loads
-    ((70, 64, 1), 4608),       # two chunks of pairs per row
-    ((140001, 3, 1), 64),      # several passes per wave
-    ((65, 40, 2), 96),         # odd block count: the generic kernel
-])
-def test_one_token_accumulates_into_a_column(ctx, oracle, dtype, layout, ms, k):
-    """y += W x of ONE token into a column of a [rows][N] matrix (row-major, a stride that is no extent) and into a strided
-    token-major row, by wick_rocm_gemm_q8 per weight and by wick_rocm_gemm_q8_multi: every other element stays."""
-    rm = layout == W.LAYOUT_ROW_MAJOR
-    col, stride = 2, 5 if rm else sum(ms) + 9
-    with Problem(ctx, oracle, dtype, ms[0], k, 1, seed=ms[0] + k + dtype) as p:
-        wbs = [p.wb] + [oracle.synth_weight(dtype, m, k, 50 + i, 0.02) for i, m in enumerate(ms[1:])]
-        ws = [p.w] + [ctx.upload_weight(wb, dtype, m, k) for wb, m in zip(wbs[1:], ms[1:])]
-        offs = np.concatenate([[0], np.cumsum(ms)[:-1]])
-        elem = [int(o) * stride + col if rm else int(o) for o in offs]
-        y0 = oracle.fill_normal(21, 1.0, sum(ms) * stride if rm else stride)
-        step, want, touched = stride if rm else 1, y0.copy(), np.zeros(y0.size, bool)
-        for wb, m, e in zip(wbs, ms, elem):
-            at = slice(e, e + (m - 1) * step + 1, step)
-            want[at] += oracle.gemv_q8(dtype, wb, p.s[0], p.q[0], m, k)
-            touched[at] = True
-        for multi in (False, True):
-            d_y = ctx.to_device(y0)
-            ys = [d_y.ptr + 4 * e for e in elem]
-            if multi:
-                ctx.gemm_preq_multi(ws, p.d_s, p.d_q, 1, ys, stride, layout=layout, accumulate=True)
-            else:
-                for w, y in zip(ws, ys):
-                    ctx.gemm_preq(w, p.d_s, p.d_q, 1, y, y_stride=stride, layout=layout, accumulate=True)
-            y = d_y.download(np.float32, y0.size)
-            assert np.array_equal(y[~touched], y0[~touched])
-            assert_f32_parity(y[touched], want[touched], f"one token, {'multi' if multi else 'single'}")
-            d_y.free()
-        for w in ws[1:]:
-            w.free()
-
-
 def test_weight_free_releases_both_copies(ctx, oracle):
     """Uploading and freeing a weight over and over leaves the device's free memory where it was: the raw blocks and the
     GEMM's copy both go (read through hipMemGetInfo of the HIP runtime the library itself is linked against)."""
@@ -386,16 +345,29 @@ def test_gemm_split_over_k(ctx, oracle, dtype, m, n, k, layout, accumulate):
     w.free(), d_q.free(), d_s.free()
 
 
+@pytest.mark.parametrize("shape", [32, 16])
 @pytest.mark.parametrize("dtype,m,n,k,pad", [
     (W.Q4_0, 1024, 512, 4608, 0),   # the down projection of a 512-token prompt: split, the norm's kernel adds the shares up
     (W.Q8_0, 1024, 100, 1024, 8),   # an out projection of a short prompt: split in 4, padded rows
     (W.Q4_0, 256, 300, 1024, 0),    # 10 tiles
     (W.Q4_0, 1024, 2002, 4608, 0),  # 256 tiles: unsplit, the plain norm kernel
     (W.Q8_0, 512, 7, 256, 4),       # below the MFMA hand-off: multi-token GEMV, then the norm
+    (W.Q4_0, 1024, 23, 1024, 0),    # few tokens, split in 4: the shares added inside the launch, or by the norm on the 16x16x32 loop
+    (W.Q8_0, 512, 64, 1024, 4),     # the same at the most tokens such a launch has
+    (W.Q4_0, 1024, 40, 4608, 0),    # few tokens, K too long for that: shares side by side either way
 ])
-def test_residual_projection_with_norm_and_quantizer(ctx, oracle, dtype, m, n, k, pad):
+def test_residual_projection_with_norm_and_quantizer(ctx, oracle, dtype, m, n, k, pad, shape):
     """x += W a, then Q8_0(rmsnorm(x)): one call == wick_rocm_gemm_q8 (accumulate) + wick_rocm_rmsnorm_quantize_q8_0, bit for bit -- the
-    residual rows, the quants and the scales -- whether or not the projection is split over K; and x against the oracle."""
+    residual rows, the quants and the scales -- whether or not the projection is split over K, on either block loop; and x against
+    the oracle."""
+    ctx.set_gemm_mfma_shape(shape)
+    try:
+        residual_projection_with_norm_and_quantizer(ctx, oracle, dtype, m, n, k, pad)
+    finally:
+        ctx.set_gemm_mfma_shape(0)
+
+
+def residual_projection_with_norm_and_quantizer(ctx, oracle, dtype, m, n, k, pad):
     from wick_amd.lfm2 import Lfm2Ops
     ops, eps, stride = Lfm2Ops(ctx), 1e-5, m + pad
     wb = oracle.synth_weight(dtype, m, k, seed=31)
@@ -489,3 +461,44 @@ def test_few_token_launches(ctx, oracle, dtype, m, n, k):
         d_d = p.alloc(n * m * (k // 32) * 4)
         ctx.block_dots_i32(p.w, p.d_q, n, d_d)
         assert np.array_equal(d_d.download(np.int32, n * m * (k // 32)).reshape(n, m, k // 32), oracle.block_dots_i32(dtype, p.wb, p.q, m, n, k))
+
+
+@pytest.mark.parametrize("dtype", [W.Q4_0, W.Q8_0])
+@pytest.mark.parametrize("layout", [W.LAYOUT_ROW_MAJOR, W.LAYOUT_TOKEN_MAJOR])
+@pytest.mark.parametrize("ms,k", [
+    ((100, 33, 7), 512),       # ragged rows, per-lane loads
+    ((1500, 500, 12), 1024),   # span loads
+    ((70, 64, 1), 4608),       # two chunks of pairs per row
+    ((140001, 3, 1), 64),      # several passes per wave
+    ((65, 40, 2), 96),         # odd block count: the generic kernel
+])
+def test_one_token_accumulates_into_a_column(ctx, oracle, dtype, layout, ms, k):
+    """y += W x of ONE token into a column of a [rows][N] matrix (row-major, a stride that is no extent) and into a strided
+    token-major row, by wick_rocm_gemm_q8 per weight and by wick_rocm_gemm_q8_multi: every other element stays."""
+    rm = layout == W.LAYOUT_ROW_MAJOR
+    col, stride = 2, 5 if rm else sum(ms) + 9
+    with Problem(ctx, oracle, dtype, ms[0], k, 1, seed=ms[0] + k + dtype) as p:
+        wbs = [p.wb] + [oracle.synth_weight(dtype, m, k, 50 + i, 0.02) for i, m in enumerate(ms[1:])]
+        ws = [p.w] + [ctx.upload_weight(wb, dtype, m, k) for wb, m in zip(wbs[1:], ms[1:])]
+        offs = np.concatenate([[0], np.cumsum(ms)[:-1]])
+        elem = [int(o) * stride + col if rm else int(o) for o in offs]
+        y0 = oracle.fill_normal(21, 1.0, sum(ms) * stride if rm else stride)
+        step, want, touched = stride if rm else 1, y0.copy(), np.zeros(y0.size, bool)
+        for wb, m, e in zip(wbs, ms, elem):
+            at = slice(e, e + (m - 1) * step + 1, step)
+            want[at] += oracle.gemv_q8(dtype, wb, p.s[0], p.q[0], m, k)
+            touched[at] = True
+        for multi in (False, True):
+            d_y = ctx.to_device(y0)
+            ys = [d_y.ptr + 4 * e for e in elem]
+            if multi:
+                ctx.gemm_preq_multi(ws, p.d_s, p.d_q, 1, ys, stride, layout=layout, accumulate=True)
+            else:
+                for w, y in zip(ws, ys):
+                    ctx.gemm_preq(w, p.d_s, p.d_q, 1, y, y_stride=stride, layout=layout, accumulate=True)
+            y = d_y.download(np.float32, y0.size)
+            assert np.array_equal(y[~touched], y0[~touched])
+            assert_f32_parity(y[touched], want[touched], f"one token, {'multi' if multi else 'single'}")
+            d_y.free()
+        for w in ws[1:]:
+            w.free()

@@ -158,7 +158,7 @@ int gemm_locked(wick_rocm_ctx* ctx, const wick_rocm_weight* w, const int8_t* d_q
     hipError_t e;
     if (n >= ctx->min_n_for(w->nbytes) && mfma_ok) {
         uint32_t splits = may_split && ctx->gemm_max_splits > 1 ? gemm_split_k(w->m, n, w->k, ctx->gemm_max_splits) : 1u;
-        const bool in_launch = !ctx->gemm_mfma16 && gemm_split_in_launch(w->m, n, w->k);  // needs no scratch
+        const bool in_launch = gemm_split_in_launch(w->m, n, w->k, ctx->launch());  // needs no scratch
         if (splits > 1 && !in_launch) {
             const size_t floats = (size_t)splits * n * w->m;
             if (ctx->capturing && floats > ctx->scratch_f_cap) splits = 1;  // no room reserved: the unsplit launch, same result to the f32 bar

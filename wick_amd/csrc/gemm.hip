@@ -1421,7 +1421,7 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, uint32_t more = 0, boo
 }  // namespace
 
 uint32_t gemm_split_k(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits) { return split_k_factor(m, n, k, max_splits); }
-bool gemm_split_in_launch(uint32_t m, uint32_t n, uint32_t k) { return few_applies(m, n, k, true); }
+bool gemm_split_in_launch(uint32_t m, uint32_t n, uint32_t k, const Launch& L) { return !L.gemm_mfma16 && few_applies(m, n, k, true); }
 
 // The GEMM's own copy of a weight (slabs, see StageT): its size, and the kernel that makes it from the raw blocks.
 size_t gemm_packed_bytes(uint32_t m, uint32_t k) { return (size_t)((m + 2 * GR - 1) / (2 * GR)) * 2 * ((k >> 5) / KB) * kSlab; }
@@ -1445,8 +1445,9 @@ hipError_t launch_gemm_mfma(int type, const uint8_t* d_w, uint32_t m, uint32_t k
     a.m = m, a.n = n, a.k = k, a.y_stride = y_stride;
     a.y_row_major = (y_layout == 1);
     a.accumulate = accumulate;
-    if (splits > 1 && (d_partial || gemm_split_in_launch(m, n, k))) {
-        if (splits != split_k_factor(m, n, k, splits) || (defer_reduce && gemm_split_in_launch(m, n, k))) return hipErrorInvalidValue;  // the shape does not carry that split
+    const bool in_launch = gemm_split_in_launch(m, n, k, L);
+    if (splits > 1 && (d_partial || in_launch)) {
+        if (splits != split_k_factor(m, n, k, splits) || (defer_reduce && in_launch)) return hipErrorInvalidValue;  // the shape does not carry that split
         a.ksplit = splits, a.partial = d_partial;
     } else if (defer_reduce) {
         return hipErrorInvalidValue;  // nothing to defer on an unsplit launch
