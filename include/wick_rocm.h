@@ -89,7 +89,9 @@ int wick_rocm_device_info(wick_rocm_ctx *ctx, char *name_buf, size_t name_len, i
 void *wick_rocm_ctx_stream(wick_rocm_ctx *ctx);
 
 /* ---- device buffers (activation / output storage the caller owns) ---------
- * Counterpart of MetalContext::create_buffer / read_f32 (wick/src/backend/metal.rs). */
+ * Counterpart of MetalContext::create_buffer / read_f32 (wick/src/backend/metal.rs).
+ * upload / download wait for the copy.  A device range that runs past the end of its allocation is WICK_ROCM_ERR_HIP and nothing
+ * is copied. */
 int wick_rocm_buffer_alloc(wick_rocm_ctx *ctx, size_t nbytes, void **d_ptr);
 int wick_rocm_buffer_free(wick_rocm_ctx *ctx, void *d_ptr);
 int wick_rocm_upload(wick_rocm_ctx *ctx, void *d_dst, const void *src, size_t nbytes);   /* H2D, ordered on the stream */

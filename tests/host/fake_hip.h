@@ -1,0 +1,17 @@
+// A HIP runtime for the CPU tests of the library's host code: what is enqueued on a stream is done when the stream (or an
+// event) is waited for and not before, device memory is host memory, and calls can be made to fail.  No kernel runs, but the
+// one that copies between device memory and a pinned slot, whose accesses are checked against the allocations.
+#pragma once
+#include <cstddef>
+
+namespace fake_hip {
+
+extern thread_local int inside;  // this thread is in the runtime, not in the library's code
+extern long launches;      // kernels enqueued so far
+extern long out_of_range;  // accesses of the copy kernel outside every allocation (they are left out)
+size_t pending();          // enqueued and not done
+size_t allocations();      // device allocations that are not freed
+void fail_launch(long n);  // the n-th kernel launch from now fails (n = 1: the next one; 0: none)
+void fail_copy(long n);    // the same for hipMemcpyAsync
+
+}  // namespace fake_hip

@@ -1,0 +1,73 @@
+// What the library's host code does when something goes wrong, on a runtime that only pretends (fake_hip.h): one case per
+// run, named on the command line, with a GGUF file of a small model where one is needed.  Prints what fails; 0: nothing did.
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <vector>
+
+#include "../../include/wick_gguf.h"
+#include "../../include/wick_rocm.h"
+#include "../../include/wick_rocm_lfm2.h"
+#include "fake_hip.h"
+
+namespace {
+
+int failures = 0;
+#define CHECK(cond, ...)                                   \
+    do {                                                   \
+        if (!(cond)) {                                     \
+            failures++;                                    \
+            std::printf("line %d: %s: ", __LINE__, #cond); \
+            std::printf(__VA_ARGS__);                      \
+            std::printf("\n");                             \
+        }                                                  \
+    } while (0)
+
+struct Ctx {
+    wick_rocm_ctx* c = nullptr;
+    Ctx() {
+        if (wick_rocm_ctx_create(0, &c) != WICK_ROCM_OK) std::abort();
+    }
+    ~Ctx() { wick_rocm_ctx_destroy(c); }
+    operator wick_rocm_ctx*() const { return c; }
+};
+
+// wick_rocm_upload / wick_rocm_download of a range that does not lie in its allocation, or of no device memory at all.
+void ranges() {
+    Ctx ctx;
+    constexpr size_t kSize = 8192;
+    void* d = nullptr;
+    CHECK(wick_rocm_buffer_alloc(ctx, kSize, &d) == WICK_ROCM_OK, "alloc");
+    char* const dev = static_cast<char*>(d);
+    std::vector<char> host(16u << 20, 1), back(16u << 20);
+    for (size_t off : {0, 16, 4096})
+        for (size_t n : {size_t{8208}, size_t{65536}, size_t{5u << 20}}) {  // past the end by one piece; one slot; many slots
+            CHECK(wick_rocm_upload(ctx, dev + off, host.data(), n) < 0, "%zu bytes at %zu", n, off);
+            CHECK(wick_rocm_download(ctx, back.data(), dev + off, n) < 0, "%zu bytes at %zu", n, off);
+        }
+    CHECK(fake_hip::pending() == 0, "%zu", fake_hip::pending());
+    // not device memory: whatever the runtime makes of it, no kernel of ours gets the address
+    const long before = fake_hip::launches;
+    alignas(16) static char plain[4096];
+    wick_rocm_upload(ctx, plain, host.data(), sizeof plain);
+    wick_rocm_download(ctx, back.data(), plain, sizeof plain);
+    CHECK(fake_hip::launches == before, "%ld launches", fake_hip::launches - before);
+    CHECK(fake_hip::out_of_range == 0, "%ld accesses", fake_hip::out_of_range);
+    // and a range inside, up to its last byte, is copied
+    for (size_t off : {0, 16, 4096}) {
+        for (size_t i = 0; i < kSize; i++) host[i] = (char)(i * 7 + off);
+        CHECK(wick_rocm_upload(ctx, dev + off, host.data(), kSize - off) == WICK_ROCM_OK, "at %zu", off);
+        CHECK(wick_rocm_download(ctx, back.data(), dev + off, kSize - off) == WICK_ROCM_OK, "at %zu", off);
+        CHECK(std::memcmp(host.data(), back.data(), kSize - off) == 0, "at %zu", off);
+    }
+    wick_rocm_buffer_free(ctx, d);
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    const char* name = argc > 1 ? argv[1] : "";
+    if (!std::strcmp(name, "ranges")) ranges();
+    else CHECK(false, "no case '%s'", name);
+    return failures ? 1 : 0;
+}

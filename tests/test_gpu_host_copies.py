@@ -54,3 +54,33 @@ def test_model_shift_in_place_equals_the_staged_one(ctx, oracle, n, keep, shift,
         assert np.array_equal(got[at:at + want.size], want)
         at += want.size
     assert at == got.size
+
+
+@pytest.mark.parametrize("nbytes", [8192 + 16, 3 * SLOT])
+def test_a_range_past_its_allocation_is_refused(ctx, nbytes):
+    """The library's own check, in front of the copy kernel (what it does with other addresses: tests/test_host_faults.py)."""
+    import wick_amd as W
+
+    buf, host = ctx.alloc(8192), np.zeros(nbytes, np.uint8)
+    for off in (0, 16):
+        for call in (lambda: ctx._lib.wick_rocm_upload(ctx._h, buf.ptr + off, host.ctypes.data, nbytes),
+                     lambda: ctx._lib.wick_rocm_download(ctx._h, host.ctypes.data, buf.ptr + off, nbytes)):
+            with pytest.raises(W.RocmError, match="range"):
+                ctx._check(call())
+    buf.free()
+
+
+@pytest.mark.parametrize("pinned", [False, True])
+def test_memory_of_other_allocators(ctx, pinned):
+    """A pointer into the middle of an allocation that the caller made, on the device or (pinned) on the host."""
+    import ctypes
+
+    hip = ctypes.CDLL("libamdhip64.so")
+    src, p = np.random.default_rng(3).integers(0, 256, 100_000, dtype=np.uint8), ctypes.c_void_p()
+    assert (hip.hipHostMalloc(ctypes.byref(p), ctypes.c_size_t(150_000), 0) if pinned else hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(150_000))) == 0
+    for off in (4096, 4099):
+        back = np.empty_like(src)
+        ctx._check(ctx._lib.wick_rocm_upload(ctx._h, p.value + off, src.ctypes.data, src.nbytes))
+        ctx._check(ctx._lib.wick_rocm_download(ctx._h, back.ctypes.data, p.value + off, src.nbytes))
+        assert np.array_equal(back, src)
+    assert (hip.hipHostFree(p) if pinned else hip.hipFree(p)) == 0

@@ -175,6 +175,34 @@ int gemm_locked(wick_rocm_ctx* ctx, const wick_rocm_weight* w, const int8_t* d_q
     return WICK_ROCM_OK;
 }
 
+// The copy as the runtime does it.
+int copy_by_runtime(wick_rocm_ctx* ctx, const HostPiece* pieces, size_t count, bool to_host) {
+    for (size_t i = 0; i < count; i++) {
+        const HostPiece& p = pieces[i];
+        WR_HIP(ctx, to_host ? hipMemcpyAsync(p.host, p.dev, p.bytes, hipMemcpyDeviceToHost, ctx->stream)
+                            : hipMemcpyAsync(p.dev, p.host, p.bytes, hipMemcpyHostToDevice, ctx->stream));
+    }
+    WR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+    return WICK_ROCM_OK;
+}
+
+// A copy of one piece whose device address the caller of the library gave.  copy_pieces hands addresses to a kernel, where a
+// range that is too short is a fault of the GPU: its end is looked up first (0.4 us, and 0.3 for whose memory it is), and what is
+// not this GPU's memory (pinned, managed, a peer's) is left to the runtime.
+int copy_checked(wick_rocm_ctx* ctx, const HostPiece& p, bool to_host) {
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    hipPointerAttribute_t attr{};
+    if (hipMemGetAddressRange(&base, &size, p.dev) != hipSuccess || hipPointerGetAttributes(&attr, p.dev) != hipSuccess) {
+        (void)hipGetLastError();
+        return copy_by_runtime(ctx, &p, 1, to_host);
+    }
+    const size_t offset = (size_t)(static_cast<char*>(p.dev) - static_cast<char*>(base));
+    if (offset > size || p.bytes > size - offset) return fail_hip(ctx, hipErrorInvalidValue, to_host ? "download: source range" : "upload: destination range");
+    if (attr.type != hipMemoryTypeDevice || attr.device != ctx->device) return copy_by_runtime(ctx, &p, 1, to_host);
+    return copy_pieces(ctx, &p, 1, to_host);
+}
+
 }  // namespace
 
 // Host memory of the callers is pageable, and large copies the runtime's way run at 5 - 30 GB/s (one thread, first-touch page faults
@@ -199,11 +227,7 @@ int copy_pieces(wick_rocm_ctx* ctx, const HostPiece* pieces, size_t count, bool 
         return launch_kernel(Launch{ctx->stream, nullptr}, kFamOther, stage_copy_kernel, dim3(blocks < 64u ? blocks : 64u), dim3(256),
                              reinterpret_cast<const uint4*>(to_host ? dev : host), reinterpret_cast<uint4*>(to_host ? host : dev), (uint32_t)n);
     };
-    if (!make_stage(ctx, total <= 2 * kStageSlotBytes ? 2 : kStageSlots)) {  // no pinned memory left: the runtime's way
-        for (size_t i = 0; i < count; i++) WR_HIP(ctx, issue(static_cast<char*>(pieces[i].dev), static_cast<char*>(pieces[i].host), pieces[i].bytes));
-        WR_HIP(ctx, hipStreamSynchronize(ctx->stream));
-        return WICK_ROCM_OK;
-    }
+    if (!make_stage(ctx, total <= 2 * kStageSlotBytes ? 2 : kStageSlots)) return copy_by_runtime(ctx, pieces, count, to_host);  // no pinned memory left
     if (total <= 2 * kStageSlotBytes) {  // small: all pieces side by side in the staging memory, one wait
         size_t at = 0;
         for (size_t i = 0; i < count; i++) {
@@ -386,7 +410,7 @@ int wick_rocm_upload(wick_rocm_ctx* ctx, void* d_dst, const void* src, size_t nb
     if (!d_dst || !src) return fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "upload: null pointer");
     if (ctx->capturing) return fail(ctx, WICK_ROCM_ERR_STATE, "upload during graph capture");
     const HostPiece p{d_dst, const_cast<void*>(src), nbytes};
-    return copy_pieces(ctx, &p, 1, false);  // waits: the host buffer may be reused on return
+    return copy_checked(ctx, p, false);  // waits: the host buffer may be reused on return
 }
 
 int wick_rocm_download(wick_rocm_ctx* ctx, void* dst, const void* d_src, size_t nbytes) {
@@ -395,7 +419,7 @@ int wick_rocm_download(wick_rocm_ctx* ctx, void* dst, const void* d_src, size_t 
     if (!dst || !d_src) return fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "download: null pointer");
     if (ctx->capturing) return fail(ctx, WICK_ROCM_ERR_STATE, "download during graph capture");
     const HostPiece p{const_cast<void*>(d_src), dst, nbytes};
-    if (int rc = copy_pieces(ctx, &p, 1, true)) return rc;
+    if (int rc = copy_checked(ctx, p, true)) return rc;
     noalloc_release(ctx);
     return WICK_ROCM_OK;
 }

@@ -110,7 +110,8 @@ struct HostPiece {
     void* host;
     size_t bytes;
 };
-// Copies the pieces in stream order and waits (lock held, not capturing).  api.hip.
+// Copies the pieces in stream order and waits (lock held, not capturing).  The device addresses are the library's own: they go
+// to a kernel unchecked.  api.hip.
 int copy_pieces(wick_rocm_ctx* ctx, const HostPiece* pieces, size_t count, bool to_host);
 
 // Takes the context lock and makes its device current for the calling thread.
