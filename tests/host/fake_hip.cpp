@@ -26,6 +26,7 @@ struct State {  // (in a function: kernels are registered by other files' static
     std::deque<std::function<void()>> queue;
     bool capturing = false;
     long launch_fails = 0, copy_fails = 0;
+    bool pinned_fails = false;
 };
 State& st() {
     static State* s = new State;
@@ -135,6 +136,10 @@ void fail_copy(long n) {
     Lock lk;
     st().copy_fails = n;
 }
+void fail_pinned(bool on) {
+    Lock lk;
+    st().pinned_fails = on;
+}
 }  // namespace fake_hip
 
 extern "C" {
@@ -182,7 +187,7 @@ hipError_t hipGetSymbolAddress(void** p, const void* symbol) {
 
 hipError_t hipMalloc(void** p, size_t n) { return allocate(st().device, p, n); }
 hipError_t hipFree(void* p) { return release(st().device, p); }
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return allocate(st().pinned, p, n); }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return st().pinned_fails ? done(hipErrorOutOfMemory) : allocate(st().pinned, p, n); }
 hipError_t hipHostFree(void* p) { return release(st().pinned, p); }
 // As the runtime does: a range that starts in an allocation has to end in it; two addresses it does not know are a copy on the host.
 hipError_t hipMemcpyAsync(void* dst, const void* src, size_t n, hipMemcpyKind, hipStream_t) {

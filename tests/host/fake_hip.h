@@ -13,5 +13,6 @@ size_t pending();          // enqueued and not done
 size_t allocations();      // device allocations that are not freed
 void fail_launch(long n);  // the n-th kernel launch from now fails (n = 1: the next one; 0: none)
 void fail_copy(long n);    // the same for hipMemcpyAsync
+void fail_pinned(bool on); // no pinned memory is to be had
 
 }  // namespace fake_hip

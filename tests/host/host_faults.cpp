@@ -3,6 +3,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <utility>
 #include <vector>
 
 #include "../../include/wick_gguf.h"
@@ -63,11 +64,73 @@ void ranges() {
     wick_rocm_buffer_free(ctx, d);
 }
 
+struct Gguf {
+    wick_gguf* g = nullptr;
+    explicit Gguf(const char* path) {
+        if (wick_gguf_open(path, &g) != 0) std::abort();
+    }
+    ~Gguf() { wick_gguf_close(g); }
+};
+
+struct Model {
+    wick_rocm_ctx* ctx;
+    wick_rocm_lfm2* m = nullptr;
+    Model(wick_rocm_ctx* c, const char* path) : ctx(c) {
+        Gguf g(path);
+        if (wick_rocm_lfm2_load(c, g.g, 64, &m) != WICK_ROCM_OK) std::abort();
+    }
+    ~Model() { wick_rocm_lfm2_free(ctx, m); }
+    operator wick_rocm_lfm2*() const { return m; }
+};
+
+// A copy of several pieces whose second, third, .. piece fails: nothing may be on its way in the staging memory (or in the
+// caller's) when the call returns, since the next copy fills it again.
+void copies(const char* path) {
+    Ctx ctx;
+    Model m(ctx, path);
+    constexpr uint32_t kPos = 40;
+    std::vector<unsigned char> in(wick_rocm_lfm2_state_bytes(m, kPos)), out(in.size());
+    for (size_t i = 0; i < in.size(); i++) in[i] = (unsigned char)(i * 13 + 1);
+    const auto restore = [&] { return wick_rocm_lfm2_restore_state(ctx, m, kPos, in.data(), in.size()); };
+    const auto snapshot = [&] { return wick_rocm_lfm2_snapshot_state(ctx, m, kPos, out.data(), out.size()); };
+    for (bool pinned : {true, false}) {  // without pinned memory the pieces are the runtime's copies, of the caller's memory
+        if (!pinned) {
+            fake_hip::fail_pinned(true);
+            wick_rocm_ctx* other = nullptr;  // (this context has its staging memory; the model's copies on another one)
+            CHECK(wick_rocm_ctx_create(0, &other) == WICK_ROCM_OK, "context");
+            std::swap(ctx.c, other);
+            wick_rocm_ctx_destroy(other);
+            m.ctx = ctx;
+        }
+        for (long n = 1; n <= 6; n++)  // two conv states, two layers' keys and values
+            for (bool up : {true, false}) {
+                (pinned ? fake_hip::fail_launch : fake_hip::fail_copy)(n);
+                CHECK((up ? restore() : snapshot()) < 0, "piece %ld, up %d, pinned %d", n, up, pinned);
+                CHECK(fake_hip::pending() == 0, "%zu on their way behind piece %ld, up %d, pinned %d", fake_hip::pending(), n, up, pinned);
+            }
+        CHECK(restore() == WICK_ROCM_OK && snapshot() == WICK_ROCM_OK, "pinned %d", pinned);
+        CHECK(in == out, "pinned %d", pinned);
+    }
+    fake_hip::fail_pinned(false);
+    // and one of many slots, dealt out to several threads
+    void* d = nullptr;
+    std::vector<char> host(27u << 20, 3);
+    CHECK(wick_rocm_buffer_alloc(ctx, host.size(), &d) == WICK_ROCM_OK, "alloc");
+    for (long n : {1, 2, 5, 14}) {
+        fake_hip::fail_launch(n);
+        CHECK(wick_rocm_upload(ctx, d, host.data(), host.size()) < 0 && fake_hip::pending() == 0, "up, chunk %ld", n);
+        fake_hip::fail_launch(n);
+        CHECK(wick_rocm_download(ctx, host.data(), d, host.size()) < 0 && fake_hip::pending() == 0, "down, chunk %ld", n);
+    }
+    wick_rocm_buffer_free(ctx, d);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const char* name = argc > 1 ? argv[1] : "";
     if (!std::strcmp(name, "ranges")) ranges();
+    else if (!std::strcmp(name, "copies") && argc > 2) copies(argv[2]);
     else CHECK(false, "no case '%s'", name);
     return failures ? 1 : 0;
 }

@@ -26,5 +26,18 @@ def host_faults(tmp_path_factory):
     return run
 
 
+@pytest.fixture(scope="session")
+def model_file(oracle, tmp_path_factory):
+    import lfm2_synth
+
+    path = tmp_path_factory.mktemp("model") / "small.gguf"
+    path.write_bytes(bytes(lfm2_synth.build(oracle, seed=5)[0]))
+    return str(path)
+
+
 def test_copies_out_of_range_are_refused_before_anything_is_enqueued(host_faults):
     host_faults("ranges")
+
+
+def test_a_copy_that_fails_leaves_nothing_on_its_way(host_faults, model_file):
+    host_faults("copies", model_file)

@@ -175,15 +175,23 @@ int gemm_locked(wick_rocm_ctx* ctx, const wick_rocm_weight* w, const int8_t* d_q
     return WICK_ROCM_OK;
 }
 
+// The end of a host copy: waits for what was enqueued, after an error (e) too, since the staging slots are filled again by the next
+// copy and the host memory is the caller's again on return.
+int finish_copy(wick_rocm_ctx* ctx, hipError_t e) {
+    const hipError_t drained = hipStreamSynchronize(ctx->stream);
+    if (e == hipSuccess) e = drained;
+    return e == hipSuccess ? WICK_ROCM_OK : fail_hip(ctx, e, "host copy");
+}
+
 // The copy as the runtime does it.
 int copy_by_runtime(wick_rocm_ctx* ctx, const HostPiece* pieces, size_t count, bool to_host) {
-    for (size_t i = 0; i < count; i++) {
+    hipError_t e = hipSuccess;
+    for (size_t i = 0; e == hipSuccess && i < count; i++) {
         const HostPiece& p = pieces[i];
-        WR_HIP(ctx, to_host ? hipMemcpyAsync(p.host, p.dev, p.bytes, hipMemcpyDeviceToHost, ctx->stream)
-                            : hipMemcpyAsync(p.dev, p.host, p.bytes, hipMemcpyHostToDevice, ctx->stream));
+        e = to_host ? hipMemcpyAsync(p.host, p.dev, p.bytes, hipMemcpyDeviceToHost, ctx->stream)
+                    : hipMemcpyAsync(p.dev, p.host, p.bytes, hipMemcpyHostToDevice, ctx->stream);
     }
-    WR_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    return WICK_ROCM_OK;
+    return finish_copy(ctx, e);
 }
 
 // A copy of one piece whose device address the caller of the library gave.  copy_pieces hands addresses to a kernel, where a
@@ -230,12 +238,13 @@ int copy_pieces(wick_rocm_ctx* ctx, const HostPiece* pieces, size_t count, bool 
     if (!make_stage(ctx, total <= 2 * kStageSlotBytes ? 2 : kStageSlots)) return copy_by_runtime(ctx, pieces, count, to_host);  // no pinned memory left
     if (total <= 2 * kStageSlotBytes) {  // small: all pieces side by side in the staging memory, one wait
         size_t at = 0;
-        for (size_t i = 0; i < count; i++) {
+        hipError_t e = hipSuccess;
+        for (size_t i = 0; e == hipSuccess && i < count; i++) {
             if (!to_host) std::memcpy(ctx->stage + at, pieces[i].host, pieces[i].bytes);
-            if (pieces[i].bytes) WR_HIP(ctx, issue_chunk(static_cast<char*>(pieces[i].dev), ctx->stage + at, pieces[i].bytes));
+            if (pieces[i].bytes) e = issue_chunk(static_cast<char*>(pieces[i].dev), ctx->stage + at, pieces[i].bytes);
             at += padded(pieces[i].bytes);
         }
-        WR_HIP(ctx, hipStreamSynchronize(ctx->stream));
+        if (int rc = finish_copy(ctx, e)) return rc;
         at = 0;
         for (size_t i = 0; to_host && i < count; i++) {
             std::memcpy(pieces[i].host, ctx->stage + at, pieces[i].bytes);
@@ -291,10 +300,7 @@ int copy_pieces(wick_rocm_ctx* ctx, const HostPiece* pieces, size_t count, bool 
     }
     work(0);
     for (std::thread& t : threads) t.join();
-    const hipError_t e = (hipError_t)failed.load(), drained = hipStreamSynchronize(ctx->stream);  // after an error too: the slots are free again
-    if (e != hipSuccess) return fail_hip(ctx, e, "host copy");
-    if (drained != hipSuccess) return fail_hip(ctx, drained, "host copy");
-    return WICK_ROCM_OK;
+    return finish_copy(ctx, (hipError_t)failed.load());
 }
 
 extern "C" {
