@@ -125,12 +125,35 @@ void copies(const char* path) {
     wick_rocm_buffer_free(ctx, d);
 }
 
+// A prompt whose n-th launch fails: its first kernel reads the tokens from the model's pinned copy, which the next prompt
+// overwrites, so nothing may be pending when the call returns.
+void prompts(const char* path) {
+    Ctx ctx;
+    Model m(ctx, path);
+    uint32_t tokens[20];
+    for (uint32_t i = 0; i < 20; i++) tokens[i] = i;
+    const auto prompt = [&] { return wick_rocm_lfm2_forward_prefill(ctx, m, tokens, 20, 0, nullptr); };
+    CHECK(prompt() == WICK_ROCM_OK, "prompt");
+    const long before = fake_hip::launches;
+    CHECK(prompt() == WICK_ROCM_OK, "prompt");
+    const long launches = fake_hip::launches - before;
+    CHECK(launches > 20, "%ld launches", launches);
+    for (long n = 1; n <= launches; n++) {
+        fake_hip::fail_launch(n);
+        CHECK(prompt() < 0, "launch %ld", n);
+        CHECK(fake_hip::pending() == 0, "%zu pending behind launch %ld", fake_hip::pending(), n);
+        wick_rocm_sync(ctx);
+    }
+    CHECK(prompt() == WICK_ROCM_OK, "prompt");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const char* name = argc > 1 ? argv[1] : "";
     if (!std::strcmp(name, "ranges")) ranges();
     else if (!std::strcmp(name, "copies") && argc > 2) copies(argv[2]);
+    else if (!std::strcmp(name, "prompts") && argc > 2) prompts(argv[2]);
     else CHECK(false, "no case '%s'", name);
     return failures ? 1 : 0;
 }

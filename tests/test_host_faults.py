@@ -41,3 +41,7 @@ def test_copies_out_of_range_are_refused_before_anything_is_enqueued(host_faults
 
 def test_a_copy_that_fails_leaves_nothing_on_its_way(host_faults, model_file):
     host_faults("copies", model_file)
+
+
+def test_a_prompt_that_fails_leaves_nothing_pending(host_faults, model_file):
+    host_faults("prompts", model_file)

@@ -881,8 +881,8 @@ int wick_rocm_lfm2_forward(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uint32_t t
     return wick_rocm_sync(ctx);
 }
 
-// Shared body of the two prompt entry points: exactly one of tokens / embeddings is given.
-static int prefill_locked(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, const uint32_t* tokens, const float* embeddings, uint32_t n, uint32_t start_pos,
+// The passes of a prompt and the last token's logits: exactly one of tokens / embeddings is given.
+static int prefill_passes(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, const uint32_t* tokens, const float* embeddings, uint32_t n, uint32_t start_pos,
                           float* logits) {
     const wick_rocm_lfm2_config& c = model->cfg;
     if ((uint64_t)start_pos + n > c.max_seq_len) return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2: position beyond the context size");
@@ -912,7 +912,7 @@ static int prefill_locked(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, const uint3
                 Guard device(ctx);
                 WR_HIP(ctx, hipHostMalloc(reinterpret_cast<void**>(&model->h_tokens), (size_t)c.max_seq_len * sizeof(uint32_t), hipHostMallocDefault));
             }
-            memcpy(model->h_tokens + done, tokens + done, (size_t)last * sizeof(uint32_t));  // (the previous prompt's call has waited for its passes)
+            memcpy(model->h_tokens + done, tokens + done, (size_t)last * sizeof(uint32_t));  // (no earlier prompt's pass is under way: prefill_locked)
         } else {  // frame j of the prompt is row j of the pass's input (wick/src/model/lfm2.rs:2452-2487)
             if (int rc = wick_rocm_upload(ctx, model->pX, embeddings + (size_t)done * c.hidden_size, (size_t)last * c.hidden_size * sizeof(float))) return rc;
         }
@@ -923,6 +923,15 @@ static int prefill_locked(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, const uint3
     if (int rc = gemv_normed(ctx, {model->embd}, {model->logits}, h_last, model->out_norm, c.rms_norm_eps)) return rc;
     if (logits) return wick_rocm_download(ctx, logits, model->logits, (size_t)c.vocab_size * sizeof(float));
     return wick_rocm_sync(ctx);
+}
+
+// Shared body of the two prompt entry points.  A pass reads the tokens from h_tokens, which the next prompt overwrites: when
+// this returns no pass is under way, after an error either.
+static int prefill_locked(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, const uint32_t* tokens, const float* embeddings, uint32_t n, uint32_t start_pos,
+                          float* logits) {
+    const int rc = prefill_passes(ctx, model, tokens, embeddings, n, start_pos, logits);  // (without an error it has waited)
+    if (rc && !ctx->capturing) (void)hipStreamSynchronize(ctx->stream);
+    return rc;
 }
 
 int wick_rocm_lfm2_forward_prefill(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, const uint32_t* tokens, uint32_t n, uint32_t start_pos, float* logits) {
