@@ -1,8 +1,10 @@
 // What the library's host code does when something goes wrong, on a runtime that only pretends (fake_hip.h): one case per
 // run, named on the command line, with a GGUF file of a small model where one is needed.  Prints what fails; 0: nothing did.
+#include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <new>
 #include <utility>
 #include <vector>
 
@@ -14,6 +16,8 @@
 namespace {
 
 int failures = 0;
+std::atomic<long> memory_left{-1};  // allocations until the one that fails (in the library and in libstdc++ alike); < 0: none does
+
 #define CHECK(cond, ...)                                   \
     do {                                                   \
         if (!(cond)) {                                     \
@@ -147,13 +151,131 @@ void prompts(const char* path) {
     CHECK(prompt() == WICK_ROCM_OK, "prompt");
 }
 
+// Every allocation of every call fails once: the call answers with an error (or does without), nothing is thrown through the C
+// entry point, nothing is left on the device, and the same call then works.
+template <typename F>
+void every_allocation(const char* what, F&& call) {
+    for (long n = 0;; n++) {
+        if (n > 100000) {
+            CHECK(false, "%s", what);
+            return;
+        }
+        const size_t before = fake_hip::allocations();
+        bool threw = false;
+        int rc = 0;
+        memory_left = n;
+        try {
+            rc = call();
+        } catch (...) {
+            threw = true;
+        }
+        const bool failed = memory_left < 0;
+        memory_left = -1;
+        CHECK(!threw, "%s: an exception at allocation %ld", what, n);
+        CHECK(fake_hip::pending() == 0 && (rc == 0 || fake_hip::allocations() == before), "%s: allocation %ld", what, n);
+        if (threw) return;  // (its locks may be held)
+        if (!failed) {
+            CHECK(rc == 0 && n > 0, "%s: %d after %ld allocations", what, rc, n);
+            return;
+        }
+    }
+}
+
+void memory(const char* path) {
+    std::vector<char> host(27u << 20, 3);
+    std::vector<unsigned char> file(1u << 22);
+    FILE* f = std::fopen(path, "rb");
+    file.resize(std::fread(file.data(), 1, file.size(), f));
+    std::fclose(f);
+    every_allocation("context", [] {
+        wick_rocm_ctx* c = nullptr;
+        const int rc = wick_rocm_ctx_create(0, &c);
+        wick_rocm_ctx_destroy(c);
+        return rc;
+    });
+    Ctx ctx;
+    Gguf gguf(path);
+    const auto opened = [](int rc, wick_gguf* g) {
+        wick_gguf_close(g);
+        return rc;
+    };
+    every_allocation("gguf file", [&] {
+        wick_gguf* g = nullptr;
+        const int rc = wick_gguf_open(path, &g);
+        return opened(rc, g);
+    });
+    every_allocation("gguf bytes", [&] {
+        wick_gguf* g = nullptr;
+        const int rc = wick_gguf_from_bytes(file.data(), file.size(), &g);
+        return opened(rc, g);
+    });
+    every_allocation("load", [&] {
+        wick_rocm_lfm2* m = nullptr;
+        const int rc = wick_rocm_lfm2_load(ctx, gguf.g, 64, &m);
+        if (m) wick_rocm_lfm2_free(ctx, m);
+        return rc;
+    });
+    every_allocation("weight", [&] {
+        wick_rocm_weight* w = nullptr;
+        const int rc = wick_rocm_weight_from_gguf(ctx, gguf.g, "blk.0.ffn_down.weight", &w);
+        if (w) wick_rocm_weight_free(ctx, w);
+        return rc;
+    });
+    void* d = nullptr;
+    CHECK(wick_rocm_buffer_alloc(ctx, host.size(), &d) == WICK_ROCM_OK, "alloc");
+    every_allocation("upload", [&] { return wick_rocm_upload(ctx, d, host.data(), host.size()); });
+    every_allocation("refused upload", [&] { return wick_rocm_upload(ctx, d, host.data(), host.size() + 16) < 0 ? 0 : -1; });
+    Model m(ctx, path);
+    constexpr uint32_t kPos = 40;
+    std::vector<unsigned char> state(wick_rocm_lfm2_state_bytes(m, kPos), 1);
+    uint32_t tokens[20] = {}, picks[4];
+    every_allocation("restore", [&] { return wick_rocm_lfm2_restore_state(ctx, m, kPos, state.data(), state.size()); });
+    every_allocation("snapshot", [&] { return wick_rocm_lfm2_snapshot_state(ctx, m, kPos, state.data(), state.size()); });
+    every_allocation("shift", [&] { return wick_rocm_lfm2_shift_kv(ctx, m, kPos, 8, 10); });
+    every_allocation("greedy", [&] {
+        const int rc = wick_rocm_lfm2_generate_greedy(ctx, m, 1, 5, 4, picks);
+        if (rc) wick_rocm_sync(ctx);  // (steps may be under way: they touch the model's own memory only)
+        return rc;
+    });
+    Model fresh(ctx, path);  // (its prompt buffers are still to be made)
+    memory_left = 0;
+    CHECK(wick_rocm_lfm2_forward_prefill(ctx, fresh, tokens, 20, 0, nullptr) < 0, "prompt");
+    memory_left = -1;
+    CHECK(wick_rocm_lfm2_forward_prefill(ctx, fresh, tokens, 20, 0, nullptr) == WICK_ROCM_OK, "prompt");
+    CHECK(wick_rocm_lfm2_forward_prefill(ctx, m, tokens, 20, 0, nullptr) == WICK_ROCM_OK, "prompt");
+    every_allocation("timing", [&] {
+        double ms[4];
+        uint64_t launches[4];
+        if (int rc = wick_rocm_kernel_timing_begin(ctx)) return rc;
+        const int rc = wick_rocm_lfm2_forward_prefill(ctx, m, tokens, 20, 0, nullptr), end = wick_rocm_kernel_timing_end(ctx, ms, launches, 4);
+        return rc ? rc : end;
+    });
+    wick_rocm_buffer_free(ctx, d);
+}
+
 }  // namespace
+
+void* operator new(size_t n) {
+    if (fake_hip::inside == 0 && memory_left >= 0 && memory_left-- == 0) throw std::bad_alloc();
+    if (void* p = std::malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void* operator new(size_t n, const std::nothrow_t&) noexcept {
+    try {
+        return operator new(n);
+    } catch (...) {
+        return nullptr;
+    }
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 int main(int argc, char** argv) {
     const char* name = argc > 1 ? argv[1] : "";
     if (!std::strcmp(name, "ranges")) ranges();
     else if (!std::strcmp(name, "copies") && argc > 2) copies(argv[2]);
     else if (!std::strcmp(name, "prompts") && argc > 2) prompts(argv[2]);
+    else if (!std::strcmp(name, "memory") && argc > 2) memory(argv[2]);
     else CHECK(false, "no case '%s'", name);
     return failures ? 1 : 0;
 }

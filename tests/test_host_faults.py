@@ -45,3 +45,7 @@ def test_a_copy_that_fails_leaves_nothing_on_its_way(host_faults, model_file):
 
 def test_a_prompt_that_fails_leaves_nothing_pending(host_faults, model_file):
     host_faults("prompts", model_file)
+
+
+def test_no_exception_leaves_an_entry_point_when_host_memory_runs_out(host_faults, model_file):
+    host_faults("memory", model_file)

@@ -253,7 +253,7 @@ int copy_pieces(wick_rocm_ctx* ctx, const HostPiece* pieces, size_t count, bool 
         return WICK_ROCM_OK;
     }
     std::vector<HostPiece> chunks;
-    chunks.reserve(total / kStageSlotBytes + count);
+    if (!make_room(chunks, total / kStageSlotBytes + count)) return fail_host_memory(ctx);
     for (size_t i = 0; i < count; i++)
         for (size_t o = 0; o < pieces[i].bytes; o += kStageSlotBytes)
             chunks.push_back({static_cast<char*>(pieces[i].dev) + o, static_cast<char*>(pieces[i].host) + o,
@@ -332,7 +332,12 @@ int wick_rocm_ctx_create(int device_id, wick_rocm_ctx** out) {
     wick_rocm_ctx* ctx = new (std::nothrow) wick_rocm_ctx();
     if (!ctx) return WICK_ROCM_ERR_HIP;
     ctx->device = device_id;
-    ctx->name = std::string(prop.gcnArchName) + " " + prop.name;
+    try {
+        ctx->name = std::string(prop.gcnArchName) + " " + prop.name;
+    } catch (...) {
+        delete ctx;
+        return WICK_ROCM_ERR_HIP;
+    }
     ctx->num_cus = prop.multiProcessorCount;
     ctx->hbm_bytes = prop.totalGlobalMem;
     if (hipSetDevice(device_id) != hipSuccess || hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) {
@@ -492,7 +497,7 @@ int wick_rocm_weight_upload(wick_rocm_ctx* ctx, const void* host_blocks, size_t 
     }
     if (ctx->capturing) return fail(ctx, WICK_ROCM_ERR_STATE, "weight_upload during graph capture");
     wick_rocm_weight* w = new (std::nothrow) wick_rocm_weight();
-    if (!w) return fail(ctx, WICK_ROCM_ERR_HIP, "out of host memory");
+    if (!w) return fail_host_memory(ctx);
     // (+64: the Q6_K kernel reads its last 16-byte piece whole)
     hipError_t e = hipMalloc(&w->d, nbytes + 64);
     if (e == hipSuccess) {
@@ -536,8 +541,11 @@ int wick_rocm_weight_from_gguf(wick_rocm_ctx* ctx, const wick_gguf* gguf, const 
     const void* bytes = nullptr;
     size_t nbytes = 0;
     if (wick_gguf_tensor_meta(gguf, tensor_name, &offset, &rows, &cols, &type) != 0 ||
-        wick_gguf_tensor_data(gguf, tensor_name, &bytes, &nbytes) != 0)
-        return fail(ctx, WICK_ROCM_ERR_INVALID_ARG, (std::string("weight_from_gguf: ") + wick_gguf_last_error()).c_str());
+        wick_gguf_tensor_data(gguf, tensor_name, &bytes, &nbytes) != 0) {
+        char what[600];
+        std::snprintf(what, sizeof what, "weight_from_gguf: %s", wick_gguf_last_error());
+        return fail(ctx, WICK_ROCM_ERR_INVALID_ARG, what);
+    }
     if (rows > UINT32_MAX || cols > UINT32_MAX) return fail(ctx, WICK_ROCM_ERR_BAD_SHAPE, "weight_from_gguf: dimension exceeds 32 bits");
     return wick_rocm_weight_upload(ctx, bytes, nbytes, type, (uint32_t)rows, (uint32_t)cols, out);
 }
@@ -987,7 +995,7 @@ int wick_rocm_graph_end(wick_rocm_ctx* ctx, wick_rocm_graph** out) {
     wick_rocm_graph* g = e == hipSuccess ? new (std::nothrow) wick_rocm_graph() : nullptr;
     if (e == hipSuccess && !g) {
         (void)hipGraphDestroy(graph);
-        return fail(ctx, WICK_ROCM_ERR_HIP, "out of host memory");
+        return fail_host_memory(ctx);
     }
     if (e == hipSuccess) {
         g->graph = graph;
@@ -1032,7 +1040,7 @@ int wick_rocm_event_create(wick_rocm_ctx* ctx, wick_rocm_event** out) {
     WR_ENTER(ctx);
     if (!out) return fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "event_create: null out pointer");
     wick_rocm_event* e = new (std::nothrow) wick_rocm_event();
-    if (!e) return fail(ctx, WICK_ROCM_ERR_HIP, "out of host memory");
+    if (!e) return fail_host_memory(ctx);
     hipError_t he = hipEventCreate(&e->ev);
     if (he != hipSuccess) {
         delete e;
@@ -1082,7 +1090,11 @@ int wick_rocm_kernel_timing_end(wick_rocm_ctx* ctx, double* total_ms, uint64_t* 
             if (total_ms) total_ms[r.family] += (double)ms;
             if (launches) launches[r.family] += 1;
         }
-        ctx->timer.spares.push_back(r);
+        try {
+            ctx->timer.spares.push_back(r);
+        } catch (...) {
+            (void)hipEventDestroy(r.start), (void)hipEventDestroy(r.stop);
+        }
     }
     ctx->timer.recs.clear();
     if (first != hipSuccess) return fail_hip(ctx, first, "kernel_timing_end");

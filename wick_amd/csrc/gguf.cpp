@@ -13,6 +13,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <new>
 #include <string>
 #include <unordered_map>
 #include <vector>
@@ -27,8 +28,22 @@ int fail(int code, const char* fmt, ...) {
     va_start(ap, fmt);
     vsnprintf(buf, sizeof buf, fmt, ap);
     va_end(ap);
-    g_error = buf;
+    try {
+        g_error = buf;
+    } catch (...) {
+        g_error.clear();
+    }
     return code;
+}
+
+// No exception leaves a C entry point.
+template <typename F>
+int no_throw(F&& f) {
+    try {
+        return f();
+    } catch (...) {
+        return fail(WICK_GGUF_ERR_IO, "out of host memory");
+    }
 }
 
 constexpr uint32_t kMagic = 0x46554747u;  // "GGUF" little-endian, wick/src/gguf.rs:18
@@ -318,22 +333,26 @@ int parse(wick_gguf& g) {
 // Looks a key up; type < 0 accepts any stored type.
 int find_value(const wick_gguf* g, const char* key, int type, const Value** out) {
     if (!g || !key) return fail(WICK_GGUF_ERR_INVALID_ARG, "null handle or key");
-    auto it = g->metadata.find(key);
-    if (it == g->metadata.end()) return fail(WICK_GGUF_ERR_NOT_FOUND, "metadata key %s not found", key);
-    if (type >= 0 && it->second.type != type) return fail(WICK_GGUF_ERR_NOT_FOUND, "metadata key %s has another type", key);
-    *out = &it->second;
-    return WICK_GGUF_OK;
+    return no_throw([&] {
+        auto it = g->metadata.find(key);
+        if (it == g->metadata.end()) return fail(WICK_GGUF_ERR_NOT_FOUND, "metadata key %s not found", key);
+        if (type >= 0 && it->second.type != type) return fail(WICK_GGUF_ERR_NOT_FOUND, "metadata key %s has another type", key);
+        *out = &it->second;
+        return (int)WICK_GGUF_OK;
+    });
 }
 
 int find_tensor(const wick_gguf* g, const char* name, bool need_data, const TensorRec** out) {
     if (!g || !name) return fail(WICK_GGUF_ERR_INVALID_ARG, "null handle or tensor name");
-    auto it = g->tensor_index.find(name);
-    if (it == g->tensor_index.end()) return fail(WICK_GGUF_ERR_NOT_FOUND, "tensor not found: %s", name);
-    const TensorRec* t = &g->tensors[it->second];
-    if (need_data && t->size_bytes == 0)  // tensor_range, wick/src/gguf.rs:612-617
-        return fail(WICK_GGUF_ERR_UNSUPPORTED, "tensor %s has unsupported GGML type %d (%s)", name, t->type, wick_gguf_type_name(t->type));
-    *out = t;
-    return WICK_GGUF_OK;
+    return no_throw([&] {
+        auto it = g->tensor_index.find(name);
+        if (it == g->tensor_index.end()) return fail(WICK_GGUF_ERR_NOT_FOUND, "tensor not found: %s", name);
+        const TensorRec* t = &g->tensors[it->second];
+        if (need_data && t->size_bytes == 0)  // tensor_range, wick/src/gguf.rs:612-617
+            return fail(WICK_GGUF_ERR_UNSUPPORTED, "tensor %s has unsupported GGML type %d (%s)", name, t->type, wick_gguf_type_name(t->type));
+        *out = t;
+        return (int)WICK_GGUF_OK;
+    });
 }
 
 }  // namespace
@@ -361,9 +380,13 @@ int wick_gguf_open(const char* path, wick_gguf** out) {
     const int e = errno;
     ::close(fd);
     if (p == MAP_FAILED) return fail(WICK_GGUF_ERR_IO, "mmap %s: %s", path, strerror(e));
-    wick_gguf* g = new wick_gguf;
+    wick_gguf* g = new (std::nothrow) wick_gguf;
+    if (!g) {
+        munmap(p, (size_t)st.st_size);
+        return fail(WICK_GGUF_ERR_IO, "out of host memory");
+    }
     g->data = static_cast<const uint8_t*>(p), g->size = (size_t)st.st_size, g->mapped = true;
-    const int rc = parse(*g);
+    const int rc = no_throw([&] { return parse(*g); });
     if (rc != 0) {
         delete g;
         return rc;
@@ -375,10 +398,13 @@ int wick_gguf_open(const char* path, wick_gguf** out) {
 int wick_gguf_from_bytes(const void* bytes, size_t nbytes, wick_gguf** out) {
     if (!out || (!bytes && nbytes)) return fail(WICK_GGUF_ERR_INVALID_ARG, "from_bytes: null bytes or out pointer");
     *out = nullptr;
-    wick_gguf* g = new wick_gguf;
-    g->owned.assign(static_cast<const uint8_t*>(bytes), static_cast<const uint8_t*>(bytes) + nbytes);
-    g->data = g->owned.data(), g->size = nbytes;
-    const int rc = parse(*g);
+    wick_gguf* g = new (std::nothrow) wick_gguf;
+    if (!g) return fail(WICK_GGUF_ERR_IO, "out of host memory");
+    const int rc = no_throw([&] {
+        g->owned.assign(static_cast<const uint8_t*>(bytes), static_cast<const uint8_t*>(bytes) + nbytes);
+        g->data = g->owned.data(), g->size = nbytes;
+        return parse(*g);
+    });
     if (rc != 0) {
         delete g;
         return rc;

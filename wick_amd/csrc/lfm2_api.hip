@@ -374,12 +374,14 @@ namespace {
 // output norm (forward_embedding / forward_hidden_from_embedding, wick/src/model/lfm2.rs:2325-2349).
 enum StepMode { kStepLogits = 0, kStepGreedy = 1, kStepHidden = 2 };
 
-int ctx_fail(wick_rocm_ctx* ctx, int code, const std::string& what) {
+int ctx_fail(wick_rocm_ctx* ctx, int code, const char* what) {
     std::lock_guard<std::recursive_mutex> lk(ctx->mu);
-    return fail(ctx, code, what.c_str());
+    return fail(ctx, code, what);
 }
+int ctx_fail(wick_rocm_ctx* ctx, int code, const std::string& what) { return ctx_fail(ctx, code, what.c_str()); }
 
 int alloc(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, size_t nbytes, void** out) {
+    if (!make_room(m->buffers, m->buffers.size() + 1)) return fail_host_memory(ctx);
     if (int rc = wick_rocm_buffer_alloc(ctx, nbytes, out)) return rc;
     m->buffers.push_back(*out);
     m->bytes += nbytes;
@@ -410,6 +412,7 @@ int upload_f32(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, const wick_gguf* g, const 
 
 int upload_weight(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, const wick_gguf* g, const std::string& name, uint32_t rows, uint32_t cols,
                   wick_rocm_weight** out) {
+    if (!make_room(m->weights, m->weights.size() + 1)) return fail_host_memory(ctx);
     if (int rc = wick_rocm_weight_from_gguf(ctx, g, name.c_str(), out)) return rc;
     m->weights.push_back(*out);
     m->bytes += (*out)->nbytes + (*out)->gemm_bytes;
@@ -694,6 +697,7 @@ int copy_state(wick_rocm_ctx* ctx, const wick_rocm_lfm2* model, uint32_t seq_len
     WR_ENTER(ctx);
     if (ctx->capturing) return fail(ctx, WICK_ROCM_ERR_STATE, to_host ? "download during graph capture" : "upload during graph capture");
     std::vector<HostPiece> pieces;
+    if (!make_room(pieces, 2 * model->layers.size())) return fail_host_memory(ctx);
     for_each_state_piece(model, seq_len, [&](void* d, size_t n) {
         pieces.push_back({d, host, n});
         host += n;
@@ -712,8 +716,7 @@ int wick_rocm_lfm2_load(wick_rocm_ctx* ctx, const wick_gguf* g, uint32_t context
 
 int wick_rocm_lfm2_kv_dtype(const wick_rocm_lfm2* model) { return model && model->kv_f16 ? WICK_ROCM_KV_F16 : WICK_ROCM_KV_F32; }
 
-int wick_rocm_lfm2_load_kv(wick_rocm_ctx* ctx, const wick_gguf* g, uint32_t context_size, int kv_dtype, wick_rocm_lfm2** out) {
-    if (!ctx) return WICK_ROCM_ERR_INVALID_ARG;
+static int load_model(wick_rocm_ctx* ctx, const wick_gguf* g, uint32_t context_size, int kv_dtype, wick_rocm_lfm2** out) {
     if (!g || !out) return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2_load: null argument");
     *out = nullptr;
     if (kv_dtype != WICK_ROCM_KV_F32 && kv_dtype != WICK_ROCM_KV_F16)
@@ -751,20 +754,17 @@ int wick_rocm_lfm2_load_kv(wick_rocm_ctx* ctx, const wick_gguf* g, uint32_t cont
     const uint32_t hs = c.hidden_size, hd = hs / c.n_heads, inter = c.intermediate_size;
     if (hd % 4u != 0 || hd > 256u) return ctx_fail(ctx, WICK_ROCM_ERR_BAD_SHAPE, "lfm2_load: head_dim must be a multiple of 4 and <= 256");
 
-    std::unique_ptr<wick_rocm_lfm2> holder(new wick_rocm_lfm2);
+    const auto drop = [ctx](wick_rocm_lfm2* unfinished) { release(ctx, unfinished); };
+    std::unique_ptr<wick_rocm_lfm2, decltype(drop)> holder(new wick_rocm_lfm2, drop);
     wick_rocm_lfm2* m = holder.get();
     m->kv_f16 = kv_dtype == WICK_ROCM_KV_F16;
-    auto bail = [&](int rc) {
-        release(ctx, holder.release());
-        return rc;
-    };
     m->layers.resize(c.n_layers);
     int rc = 0;
     // the layers' rolling conv states in one piece (each on its own 256 bytes): a reset clears them in one launch
     const size_t conv_floats = ((size_t)(c.conv_kernel_size - 1) * hs + 63) / 64 * 64;
     size_t n_conv = 0;
     m->conv_floats = conv_floats * c.n_layers;
-    if (conv_floats && (rc = alloc_t(ctx, m, m->conv_floats, &m->conv_states))) return bail(rc);
+    if (conv_floats && (rc = alloc_t(ctx, m, m->conv_floats, &m->conv_states))) return rc;
     // block types from tensor presence, wick/src/model/lfm2.rs:151-170
     for (uint32_t i = 0; i < c.n_layers; i++) {
         const std::string p = "blk." + std::to_string(i) + ".";
@@ -774,44 +774,47 @@ int wick_rocm_lfm2_load_kv(wick_rocm_ctx* ctx, const wick_gguf* g, uint32_t cont
             int32_t n_kv;
             memcpy(&n_kv, static_cast<const uint8_t*>(kv_data) + 4 * i, 4);
             if (n_kv <= 0 || c.n_heads % (uint32_t)n_kv != 0)
-                return bail(ctx_fail(ctx, WICK_ROCM_ERR_BAD_SHAPE, "lfm2_load: layer " + std::to_string(i) + ": n_kv_heads must be > 0 and divide n_heads"));
+                return ctx_fail(ctx, WICK_ROCM_ERR_BAD_SHAPE, "lfm2_load: layer " + std::to_string(i) + ": n_kv_heads must be > 0 and divide n_heads");
             L.n_kv = (uint32_t)n_kv;
             c.n_kv_heads = L.n_kv > c.n_kv_heads ? L.n_kv : c.n_kv_heads;
         }
-        if ((rc = upload_f32(ctx, m, g, p + "attn_norm.weight", hs, &L.attn_norm))) return bail(rc);
-        if ((rc = upload_f32(ctx, m, g, p + "ffn_norm.weight", hs, &L.ffn_norm))) return bail(rc);
+        if ((rc = upload_f32(ctx, m, g, p + "attn_norm.weight", hs, &L.attn_norm))) return rc;
+        if ((rc = upload_f32(ctx, m, g, p + "ffn_norm.weight", hs, &L.ffn_norm))) return rc;
         if (is_attn) {
             const uint32_t kv_dim = L.n_kv * hd;
-            if ((rc = upload_f32(ctx, m, g, p + "attn_q_norm.weight", hd, &L.q_norm))) return bail(rc);
-            if ((rc = upload_f32(ctx, m, g, p + "attn_k_norm.weight", hd, &L.k_norm))) return bail(rc);
-            if ((rc = upload_weight(ctx, m, g, p + "attn_q.weight", hs, hs, &L.q))) return bail(rc);
-            if ((rc = upload_weight(ctx, m, g, p + "attn_k.weight", kv_dim, hs, &L.k))) return bail(rc);
-            if ((rc = upload_weight(ctx, m, g, p + "attn_v.weight", kv_dim, hs, &L.v))) return bail(rc);
-            if ((rc = upload_weight(ctx, m, g, p + "attn_output.weight", hs, hs, &L.o))) return bail(rc);
-            if ((rc = alloc(ctx, m, (size_t)c.max_seq_len * kv_dim * m->kv_elem(), &L.k_cache))) return bail(rc);
-            if ((rc = alloc(ctx, m, (size_t)c.max_seq_len * kv_dim * m->kv_elem(), &L.v_cache))) return bail(rc);
+            if ((rc = upload_f32(ctx, m, g, p + "attn_q_norm.weight", hd, &L.q_norm))) return rc;
+            if ((rc = upload_f32(ctx, m, g, p + "attn_k_norm.weight", hd, &L.k_norm))) return rc;
+            if ((rc = upload_weight(ctx, m, g, p + "attn_q.weight", hs, hs, &L.q))) return rc;
+            if ((rc = upload_weight(ctx, m, g, p + "attn_k.weight", kv_dim, hs, &L.k))) return rc;
+            if ((rc = upload_weight(ctx, m, g, p + "attn_v.weight", kv_dim, hs, &L.v))) return rc;
+            if ((rc = upload_weight(ctx, m, g, p + "attn_output.weight", hs, hs, &L.o))) return rc;
+            if ((rc = alloc(ctx, m, (size_t)c.max_seq_len * kv_dim * m->kv_elem(), &L.k_cache))) return rc;
+            if ((rc = alloc(ctx, m, (size_t)c.max_seq_len * kv_dim * m->kv_elem(), &L.v_cache))) return rc;
         } else {
-            if ((rc = upload_f32(ctx, m, g, p + "shortconv.conv.weight", (uint64_t)hs * c.conv_kernel_size, &L.conv_w))) return bail(rc);
-            if ((rc = upload_weight(ctx, m, g, p + "shortconv.in_proj.weight", 3 * hs, hs, &L.in_proj))) return bail(rc);
-            if ((rc = upload_weight(ctx, m, g, p + "shortconv.out_proj.weight", hs, hs, &L.out_proj))) return bail(rc);
+            if ((rc = upload_f32(ctx, m, g, p + "shortconv.conv.weight", (uint64_t)hs * c.conv_kernel_size, &L.conv_w))) return rc;
+            if ((rc = upload_weight(ctx, m, g, p + "shortconv.in_proj.weight", 3 * hs, hs, &L.in_proj))) return rc;
+            if ((rc = upload_weight(ctx, m, g, p + "shortconv.out_proj.weight", hs, hs, &L.out_proj))) return rc;
             if (c.conv_kernel_size > 1) L.conv_state = m->conv_states + n_conv++ * conv_floats;
         }
-        if ((rc = upload_weight(ctx, m, g, p + "ffn_gate.weight", inter, hs, &L.gate))) return bail(rc);
-        if ((rc = upload_weight(ctx, m, g, p + "ffn_up.weight", inter, hs, &L.up))) return bail(rc);
-        if ((rc = upload_weight(ctx, m, g, p + "ffn_down.weight", hs, inter, &L.down))) return bail(rc);
+        if ((rc = upload_weight(ctx, m, g, p + "ffn_gate.weight", inter, hs, &L.gate))) return rc;
+        if ((rc = upload_weight(ctx, m, g, p + "ffn_up.weight", inter, hs, &L.up))) return rc;
+        if ((rc = upload_weight(ctx, m, g, p + "ffn_down.weight", hs, inter, &L.down))) return rc;
         L.conv_fused = L.n_kv == 0 && L.conv_state && reinterpret_cast<uintptr_t>(L.conv_state) % 16u == 0 && reinterpret_cast<uintptr_t>(L.conv_w) % 16u == 0 &&
                        wick_rocm_shortconv_fusable(L.out_proj, L.gate, L.up, c.conv_kernel_size) != 0;
     }
-    if ((rc = upload_f32(ctx, m, g, "token_embd_norm.weight", hs, &m->out_norm))) return bail(rc);
+    if ((rc = upload_f32(ctx, m, g, "token_embd_norm.weight", hs, &m->out_norm))) return rc;
     {
         // The tied embedding serves row lookups and the LM head over ONE token (a prompt pass takes the last token's logits only,
         // wick/src/model/lfm2.rs:2190-2212): it never runs as a batched GEMM, so it keeps its raw blocks only.
+        const std::string name = "token_embd.weight";
         std::lock_guard<std::recursive_mutex> lk(ctx->mu);
-        const bool packing = ctx->gemm_packing;
+        struct Unpacked {
+            bool& flag;
+            const bool was = flag;
+            ~Unpacked() { flag = was; }
+        } unpacked{ctx->gemm_packing};
         ctx->gemm_packing = false;
-        rc = upload_weight(ctx, m, g, "token_embd.weight", c.vocab_size, hs, &m->embd);
-        ctx->gemm_packing = packing;
-        if (rc) return bail(rc);
+        if ((rc = upload_weight(ctx, m, g, name, c.vocab_size, hs, &m->embd))) return rc;
     }
 
     const uint32_t kv_max = (c.n_kv_heads ? c.n_kv_heads : 1) * hd;
@@ -821,15 +824,24 @@ int wick_rocm_lfm2_load_kv(wick_rocm_ctx* ctx, const wick_gguf* g, uint32_t cont
         (rc = alloc_t(ctx, m, attention_scratch_floats(c.max_seq_len, c.n_heads, hd), &m->scores)) || (rc = alloc_t(ctx, m, hd, &m->rope)) ||
         (rc = alloc_t(ctx, m, c.vocab_size, &m->logits)) || (rc = alloc_t(ctx, m, 1, &m->d_token)) ||
         (rc = alloc_t(ctx, m, 1, &m->d_pos)) || (rc = alloc_t(ctx, m, 1, &m->d_pick)) || (rc = alloc_t(ctx, m, kArgmaxPartials, &m->d_argmax_partial)) || (rc = alloc_t(ctx, m, c.max_seq_len, &m->d_history)))
-        return bail(rc);
+        return rc;
     // GEMVs that cannot take the fused-quantizer kernel quantize into the context's scratch: size it before any capture
-    if ((rc = wick_rocm_reserve_scratch(ctx, 1, hs > inter ? hs : inter))) return bail(rc);
+    if ((rc = wick_rocm_reserve_scratch(ctx, 1, hs > inter ? hs : inter))) return rc;
     m->cfg = c;
     m->theta_scale = wick_rocm_rope_theta_scale(hd, c.rope_theta);
-    if ((rc = wick_rocm_lfm2_reset(ctx, m))) return bail(rc);
-    if ((rc = wick_rocm_sync(ctx))) return bail(rc);  // uploads read the GGUF image: done before the caller may close it
+    if ((rc = wick_rocm_lfm2_reset(ctx, m))) return rc;
+    if ((rc = wick_rocm_sync(ctx))) return rc;  // uploads read the GGUF image: done before the caller may close it
     *out = holder.release();
     return WICK_ROCM_OK;
+}
+
+int wick_rocm_lfm2_load_kv(wick_rocm_ctx* ctx, const wick_gguf* g, uint32_t context_size, int kv_dtype, wick_rocm_lfm2** out) {
+    if (!ctx) return WICK_ROCM_ERR_INVALID_ARG;
+    try {
+        return load_model(ctx, g, context_size, kv_dtype, out);  // (what it had made goes with its holder)
+    } catch (...) {
+        return ctx_fail(ctx, WICK_ROCM_ERR_HIP, "out of host memory");
+    }
 }
 
 int wick_rocm_lfm2_free(wick_rocm_ctx* ctx, wick_rocm_lfm2* model) {
@@ -1079,6 +1091,7 @@ int wick_rocm_lfm2_shift_kv(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uint32_t 
     if (seq_len - n_keep - shift == 0) return WICK_ROCM_OK;  // nothing behind the dropped rows: only the caller's seq_len changes
     const uint32_t hd = c.hidden_size / c.n_heads;
     std::vector<KvShiftLayer> layers;  // conv layers keep their rolling buffer (wick/src/kv_cache.rs:584-590)
+    if (!make_room(layers, model->layers.size())) return fail_host_memory(ctx);
     for (const LayerWeights& L : model->layers)
         if (L.n_kv) layers.push_back({L.k_cache, L.v_cache, L.n_kv});
     if (layers.empty()) return WICK_ROCM_OK;

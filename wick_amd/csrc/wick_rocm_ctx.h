@@ -4,6 +4,7 @@
 
 #include <mutex>
 #include <string>
+#include <vector>
 
 #include "../../include/wick_rocm.h"
 #include "wick_rocm_internal.h"
@@ -86,16 +87,37 @@ struct wick_rocm_event {
 };
 
 
+// No exception leaves a C entry point: what allocates on the host is caught where it does, and an error whose message finds no
+// memory is returned without one.
 inline int fail(wick_rocm_ctx* ctx, int code, const char* what) {
-    if (ctx) ctx->err = what;
+    try {
+        if (ctx) ctx->err = what;
+    } catch (...) {
+        ctx->err.clear();
+    }
     return code;
 }
 
 inline int fail_hip(wick_rocm_ctx* ctx, hipError_t e, const char* where) {
-    if (ctx) {
-        ctx->err = std::string(where) + ": " + hipGetErrorString(e);
+    try {
+        if (ctx) ctx->err = std::string(where) + ": " + hipGetErrorString(e);
+    } catch (...) {
+        ctx->err.clear();
     }
     return WICK_ROCM_ERR_HIP;
+}
+
+inline int fail_host_memory(wick_rocm_ctx* ctx) { return fail(ctx, WICK_ROCM_ERR_HIP, "out of host memory"); }
+
+// Room for n elements (push_back then does not allocate); false: there is no memory.
+template <typename T>
+inline bool make_room(std::vector<T>& v, size_t n) {
+    try {
+        v.reserve(n);
+        return true;
+    } catch (...) {
+        return false;
+    }
 }
 
 #define WR_HIP(ctx, call)                                      \

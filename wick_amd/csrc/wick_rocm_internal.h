@@ -66,8 +66,13 @@ inline hipError_t launch_kernel(const Launch& L, int family, void (*kernel)(KArg
             if (e != hipSuccess) return e;
         }
         r.family = family;
+        try {
+            L.timer->recs.push_back(r);
+        } catch (...) {
+            (void)hipEventDestroy(r.start), (void)hipEventDestroy(r.stop);
+            return hipErrorOutOfMemory;
+        }
         hipExtLaunchKernelGGL(kernel, grid, block, 0, L.stream, r.start, r.stop, 0, args...);
-        L.timer->recs.push_back(r);
     } else {
         hipLaunchKernelGGL(kernel, grid, block, 0, L.stream, args...);
     }
