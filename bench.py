@@ -580,9 +580,11 @@ def bench_prefill_sites(ctx, W, O, n=4096, dtype=8):
     return res
 
 
-def bench_gate_up_fused(ctx, W, O, dtype, m, k, n, wg=None, wu=None, reps=5):
+def bench_gate_up_fused(ctx, W, O, dtype, m, k, n, wg=None, wu=None, reps=20, warmup=60):
     """gate | up of a prompt pass up to the down projection's Q8_0 input: one GEMM launch over both weights + the SiLU gate /
-    quantizer kernel, against the GEMM whose epilogue gates and quantizes (same bits).  Per-dispatch timestamps, median."""
+    quantizer kernel, against the GEMM whose epilogue gates and quantizes (same bits).  Per-dispatch timestamps, medians; the two
+    are run in turn, warm-up included: a GPU that has just become busy runs the first few dozen launches up to a fifth slower, and
+    whichever side is timed first would carry all of that."""
     from wick_amd.lfm2 import Lfm2Ops
     ops = Lfm2Ops(ctx)
     wg = O.synth_weight(dtype, m, k, seed=41) if wg is None else wg
@@ -600,16 +602,18 @@ def bench_gate_up_fused(ctx, W, O, dtype, m, k, n, wg=None, wu=None, reps=5):
         ops.encode_ffn_gate_up_silu_quantize(d_wg, d_wu, d_s, d_q, n, d_oq, d_os)
 
     out = {"dtype": dtype, "m": m, "k": k, "n": n}
-    for name, fn in (("separate_us", separate), ("fused_us", fused)):
-        fn()
-        ts = []
-        for _ in range(reps):
+    sides = {"separate": separate, "fused": fused}
+    for _ in range(warmup):
+        separate(), fused()
+    ts = {name: [] for name in sides}
+    for _ in range(reps):
+        for name, fn in sides.items():
             ctx.kernel_timing_begin()
             fn()
             kt = ctx.kernel_timing_end()
-            ts.append(sum(ms for ms, cnt in kt.values()) * 1e3)
-            out[name.replace("_us", "_gemm_us")] = kt["gemm"][0] * 1e3
-        out[name] = float(np.median(ts))
+            ts[name].append((kt["gemm"][0] * 1e3, sum(ms for ms, cnt in kt.values()) * 1e3))
+    for name in sides:
+        out[name + "_gemm_us"], out[name + "_us"] = (float(v) for v in np.median(np.array(ts[name]), axis=0))
     for b in (d_q, d_s, d_g, d_u, d_oq, d_os):
         b.free()
     d_wg.free(), d_wu.free()

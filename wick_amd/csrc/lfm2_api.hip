@@ -649,7 +649,10 @@ int enqueue_prompt_pass(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, uint32_t n, uint3
         if ((rc = project_and_norm(L.n_kv == 0 ? L.out_proj : L.o, m->pQ, m->pS, L.ffn_norm))) break;  // hidden += out projection; FFN norm
         if (wick_rocm_ffn_gate_up_silu_quantize_applies(L.gate, L.up, n)) {
             // gate, up, SiLU gate and the down projection's quantizer in one launch; its output cannot overwrite its own input.
-            // (Against GEMM + gate kernel: 4608 x 1024 over 2048 tokens 75 -> 68 us, over 555 32 -> 26; 6912 x 2048 over 2002 174 -> 159.)
+            // (GEMM + gate kernel against this, us inside a prompt pass: 4608 x 1024 over 2002 tokens 75.0 / 68.4, over 555 31.5 / 25.9;
+            // 6912 x 2048 over 2002 173.8 / 162.8, over 1024 95.2 / 86.2, over 1400 122.1 / 124.5 -- the one length found where it loses.
+            // Whole prompts of 400 .. 4096 tokens through the 350M shape are 1.02 - 1.09 times as fast with it; through six layers of the
+            // 1.2B shape 1.04 at 300 .. 1024, 0.99 at 1400, 1.01 at 2002, 1.02 at 4096.)
             if ((rc = wick_rocm_ffn_gate_up_silu_quantize_q8(ctx, L.gate, L.up, m->pQ, m->pS, n, m->pQ2, m->pS2))) break;
             rc = next_norm ? project_and_norm(L.down, m->pQ2, m->pS2, next_norm)
                            : wick_rocm_gemm_q8(ctx, L.down, m->pQ2, m->pS2, n, m->pX, hs, WICK_ROCM_LAYOUT_TOKEN_MAJOR, 1);
