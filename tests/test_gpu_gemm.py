@@ -437,8 +437,8 @@ def test_prompt_tiles_against_the_gemv_route(ctx, oracle, m, n, k):
 @pytest.mark.parametrize("m,n,k", [(33, 9, 128), (32, 32, 1024), (100, 33, 1152), (64, 64, 4608), (1000, 31, 6912), (2080, 37, 1664)])
 def test_few_token_launches(ctx, oracle, dtype, m, n, k):
     """Granule-per-workgroup launches at their edges: one row past a granule, one / two token groups full and one short, fewer slabs
-    than waves, slabs that do not deal out evenly over waves and shares; split over K with the shares added inside the launch (repeated:
-    the arrival counters must be back at zero) and unsplit; both layouts, accumulate, block dots."""
+    than waves, slabs that do not deal out evenly over waves and shares; split over K with the shares walked and added up by one
+    workgroup (repeated: the same bits every time) and unsplit; both layouts, accumulate, block dots."""
     with Problem(ctx, oracle, dtype, m, k, n, seed=m + 3 * n + k + dtype) as p:
         ref = oracle.gemm_q8(dtype, p.wb, p.s, p.q, m, n, k)
         first = {}

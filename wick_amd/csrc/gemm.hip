@@ -62,11 +62,14 @@ namespace {
 
 constexpr int BM = 128;       // weight rows per workgroup
 constexpr int BN = 128;       // tokens per workgroup
-constexpr int BN_NARROW = 64;  // ... of the narrow kernel (n <= 64)
+constexpr int BN_NARROW = 64;  // ... of the narrow kernel
 constexpr int KB = 4;         // blocks per stage
 constexpr int THREADS = 512;  // 8 waves: 2 (rows) x 4 (tokens)
 constexpr int TT = 2;          // 16-token MFMA tiles per wave
 constexpr int RT = 4;          // 16-row MFMA tiles per wave
+// The rules that choose tile and split count in CUs of the whole chip (the constants in them were fitted on it), two workgroups
+// each.  On a partition of it they still choose launches that are right, not the fastest ones.
+constexpr uint32_t kCus = 256;
 constexpr uint32_t kBiasBits = 0x4B400000u;  // 12582912.0f
 constexpr float kBias = 12582912.0f;
 
@@ -967,12 +970,11 @@ __global__ __launch_bounds__(C::kThreads, C::kOcc) void gemm_tile_kernel(GemmArg
 }
 
 // ---------------------------------------------------------------------------------------
-// Narrow variant for 16 <= n <= 64 (an LM head or a projection over a short prompt): tile =
-// 128 weight rows x 64 tokens, every one of the 8 waves owns 16 rows x all 64 tokens (one
-// row tile x four token tiles), so no matrix or scaling work is spent on token columns that
-// do not exist beyond the 64, and the weights -- the only large operand -- are streamed
-// exactly once.  Same staging, LDS layouts and arithmetic as the wide kernel; 60 KB of LDS,
-// two workgroups per CU.  TTN (1 .. 4): how many of the four token tiles the launch has tokens
+// Narrow variant for launches of up to 48 tokens that gemm_few_kernel does not take (an LM head, or a long K, over a short
+// prompt; up to 64 tokens, and few tiles of more, where the 16x16x32 loop is asked for): tile = 128 weight rows x 64 tokens,
+// every one of the 8 waves owns 16 rows x all 64 tokens (one row tile x four token tiles), so no matrix or scaling work is
+// spent on token columns that do not exist beyond the 64, and the weights -- the only large operand -- are streamed exactly
+// once per 64 tokens.  Same staging, LDS layouts and arithmetic as the wide kernel; 60 KB of LDS, two workgroups per CU.  TTN (1 .. 4): how many of the four token tiles the launch has tokens
 // for -- a launch of n <= 16 / 32 / 48 tokens reads and multiplies only those (these launches
 // are bound by their block loop, so the unused tiles were a third to three quarters of their time).
 struct NarrowMats {
@@ -1277,14 +1279,14 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
 // instead of one narrow tile per CU.  Shares of >= 8 stages.
 uint32_t wide_split_factor(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits) {
     const uint32_t tiles = ((m + BM - 1) / BM) * ((n + BN - 1) / BN), stages = (k >> 5) / KB;
-    if (n <= BN_NARROW || tiles < 64 || tiles > 256 || stages < 32) return 1;
+    if (n <= BN_NARROW || tiles < kCus / 4 || tiles > kCus || stages < 32) return 1;
     uint32_t s_ = 1;
-    while (2 * s_ <= max_splits && tiles * 2 * s_ <= 512 && stages / (2 * s_) >= 8) s_ *= 2;
+    while (2 * s_ <= max_splits && tiles * 2 * s_ <= 2 * kCus && stages / (2 * s_) >= 8) s_ *= 2;
     return s_;
 }
 
 // Launches of few 128 x 128 tiles (at most one per CU): the ones that may be split over K.
-bool narrow_tiles(uint64_t row_tiles, uint32_t n) { return n <= BN_NARROW || row_tiles * ((n + BN - 1) / BN) <= 256; }
+bool narrow_tiles(uint64_t row_tiles, uint32_t n) { return n <= BN_NARROW || row_tiles * ((n + BN - 1) / BN) <= kCus; }
 
 // Launches of gemm_few_kernel: up to 64 tokens and few enough granules that latency and not the chip's throughput is what they cost
 // (every workgroup fetches all tokens' activations for its 32 rows; beyond, the 128-row tiles are the cheaper readers).  A round of K
@@ -1293,7 +1295,7 @@ bool narrow_tiles(uint64_t row_tiles, uint32_t n) { return n <= BN_NARROW || row
 // 8.9 / 14.3, 2048 x 2048 over 40 8.2 / 11.5; 65536 x 2048 over 16 27 / 40.
 bool few_applies(uint64_t rows, uint32_t n, uint32_t k, bool split) {
     const uint64_t units = (rows + GR - 1) / GR, slabs = k / (KB * 32);
-    return n <= 64 && units <= 512 && units * slabs <= (n <= 32 ? 12288u : 4096u) && (!split || slabs <= (n <= 32 ? 16u : 8u));
+    return n <= 64 && units <= 2 * kCus && units * slabs <= (n <= 32 ? 12288u : 4096u) && (!split || slabs <= (n <= 32 ? 16u : 8u));
 }
 
 uint32_t split_k_factor(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits) {
@@ -1304,7 +1306,7 @@ uint32_t split_k_factor(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits)
     const uint32_t tiles = row_tiles * ((n + BN_NARROW - 1) / BN_NARROW), stages = (k >> 5) / KB;
     if (stages < 8) return 1;
     uint32_t s_ = 1;
-    while (2 * s_ <= max_splits && tiles * 2 * s_ <= 256 && stages / (2 * s_) >= 2) s_ *= 2;
+    while (2 * s_ <= max_splits && tiles * 2 * s_ <= kCus && stages / (2 * s_) >= 2) s_ *= 2;
     return s_;
 }
 
@@ -1334,7 +1336,7 @@ using TileS = T32<2, 1, 2, 2, 4>;     // 128 x 64, 4 waves of 64 x 32
 using TileN = T32<1, 1, 4, 2, 4, 4>;  // 128 x 64, 8 waves of 32 x 32: where a CU gets one workgroup at most, its waves are all there is
 template <typename C>
 float tile_cost(uint64_t row_tiles, uint32_t n, uint32_t k, bool gated = false) {
-    const uint64_t tiles = row_tiles * ((n + C::kTokens - 1) / C::kTokens), rounds = (tiles + 255) / 256;
+    const uint64_t tiles = row_tiles * ((n + C::kTokens - 1) / C::kTokens), rounds = (tiles + kCus - 1) / kCus;
     const float per_k = C::kRows == 256 ? 34.0f : (C::kTokens == 128 ? 40.0f : 46.0f);
     const float fixed = C::kRows == 256 ? (gated ? 6.0f : 5.0f) : (C::kTokens == 128 ? (gated ? 6.3f : 1.4f) : (gated ? 5.0f : 3.0f));
     return (float)rounds * (rounds == 1 ? 1.35f : 1.0f) * ((float)(C::kRows * C::kTokens) / (256.0f * 128.0f)) * (per_k * (float)k / 2048.0f + fixed);
@@ -1390,7 +1392,7 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, uint32_t more = 0, boo
                 if (q8) return go(gemm_few_kernel<8, true, TG, WV>, GR, 64, 64 * WV, true);
             return go(gemm_few_kernel<2, DUMP, TG, WV>, GR, 64, 64 * WV, true);
         };
-        if (tile_rows(GR) <= 256) return a.n <= 32 ? waves(Idx<1>{}, Idx<8>{}) : waves(Idx<2>{}, Idx<8>{});
+        if (tile_rows(GR) <= kCus) return a.n <= 32 ? waves(Idx<1>{}, Idx<8>{}) : waves(Idx<2>{}, Idx<8>{});
         return a.n <= 32 ? waves(Idx<1>{}, Idx<4>{}) : waves(Idx<2>{}, Idx<4>{});
     }
     if (narrow && (a.n <= 48 || L.gemm_mfma16)) {
@@ -1412,7 +1414,7 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, uint32_t more = 0, boo
     }
     if (wide_split) return tile(TileM{});
     const uint64_t small = tile_rows(BM) * ((a.n + BN_NARROW - 1) / BN_NARROW) * (a.ksplit > 1 ? a.ksplit : 1u);
-    if (narrow && small <= 256) return tile(TileN{});  // (1024 x 1024 over 555 tokens 10.9 us on TileS, 10.6 here; 512 tiles: 27 / 29.5)
+    if (narrow && small <= kCus) return tile(TileN{});  // (1024 x 1024 over 555 tokens 10.9 us on TileS, 10.6 here; 512 tiles: 27 / 29.5)
     if (a.n <= BN_NARROW || a.ksplit > 1) return tile(TileS{});
     const auto cost = [&](auto cfg) { return tile_cost<decltype(cfg)>(tile_rows(decltype(cfg)::kRows), a.n, a.k); };
     return cheapest_tile(cost, tile);
@@ -1475,7 +1477,7 @@ hipError_t launch_gemm_mfma_multi(int type, const uint8_t* const* d_w, const uin
 // projections + silu_mul_quantize_kernel.  The float projections (2 * n * m * 4 bytes) are never written.
 bool gemm_gated_applies(uint32_t m, uint32_t n, uint32_t k) {
     // wide tiles only (the narrow kernel's waves own 16 rows: no block in one wave), and enough of them to fill the chip
-    return m % 32u == 0 && k % 128u == 0 && n > BN_NARROW && (uint64_t)((m + 63u) / 64u) * ((n + BN - 1) / BN) > 256u;
+    return m % 32u == 0 && k % 128u == 0 && n > BN_NARROW && (uint64_t)((m + 63u) / 64u) * ((n + BN - 1) / BN) > kCus;
 }
 
 hipError_t launch_gemm_mfma_gated(int /*type: the copies are the same for both*/, const uint8_t* d_w_gate, const uint8_t* d_w_up, uint32_t m, uint32_t k, const int8_t* d_q,

@@ -39,7 +39,7 @@ struct GemvArgs {
     const float* xf;    // [n][x_stride] f32 activations, quantized in-kernel (FUSEQ variants)
     const float* xaux;  // FUSEQ with a transform: RMSNorm weights [k] / the "up" vector [k] / the conv kernel [k][3]
     const float* xaux2; // kXformShortConv: the rolling conv state [2][k] (read only)
-    // GATED with a side job: the rolling state of the layer's short convolution is advanced by the first workgroups
+    // GATED with a side job: the rolling state of the layer's short convolution is advanced by a workgroup of its own, the last
     // (conv_state[s] <- conv_state[s + 1], last slot <- b * x of conv_proj = [b | c | x]); null: no side job
     float* conv_state;
     const float* conv_proj;
@@ -47,7 +47,7 @@ struct GemvArgs {
     float eps;          // RMSNorm epsilon
     double inv_k;       // 1 / k
     int32_t* dots;      // parity hook (DUMP variants): raw i32 block dots, [token][row][block], instead of y
-    int xform;          // kXformNone / kXformRmsNorm / kXformSiluMul (host-side selector of the kernel variant)
+    int xform;          // kXformNone, kXformRmsNorm, .. (host-side selector of the kernel variant)
     int gated;          // host-side selector of the GATED variant: batch.w[0] = gate, batch.w[1] = up, y[0][r] = silu(gate_r) * up_r
     uint32_t splits, max_seq;  // kXformAttnMerge: partial records per head and the cache's rows
     uint32_t x_stride;
@@ -70,7 +70,6 @@ struct ActRegs {
 
 // FUSEQ workgroups have four waves that quantize the activation vector together.
 constexpr int kFusedWaves = 4;
-constexpr int kFusedMaxK = 8192;
 constexpr int kConvMaxK = 2048;
 
 // How a lane gets its pair (MODE):
@@ -96,7 +95,8 @@ enum { kDirect = 0, kDirectNT = 1, kSpan = 2 };
 //                  launch (the side job of the gate / up kernel).  Kernel size 3, k <= 2048.
 //   kXformAttnMerge  the merge of a decode step's attention partials (attention_merge, bit for bit; head_dim 64) in front of the
 //                  output projection: x = the partial records {max, sum, acc[64]} of [head][split], aux = the position.  The
-//                  first 16 splits' records are requested with everything else (enqueue_step uses it up to there).
+//                  records of all splits, at most kAttnMergeMaxSplits, are requested with everything else (enqueue_step uses it at
+//                  positions that have no more).
 //                  Against a merge launch: a step of the 350M shape (6 attention layers) 251 -> 244 us at position 30,
 //                  260 -> 253 at 600, 268 -> 263 at 980, 278 -> 276 at 1500, 286 -> 294 at 2500.  For k = 2048 every
 //                  workgroup reads twice the records: 160 -> 165 us at 980 and nothing gained at 30, hence k <= 1024.
@@ -160,10 +160,10 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
     constexpr int kQuadRounds = LPR * NCHUNK <= 16 ? 1 : LPR * NCHUNK / 16;
     const auto past = [&](int i) { return i > kQuadRounds / 2 && (uint32_t)i * 64u * kFusedWaves >= (p_k >> 2); };
     float4 xv[FUSEQ ? kQuadRounds : 1];
-    // kXformAttnMerge: this wave's heads' {max, sum} per split (one lane each), this thread's quads of the first splits
-    constexpr int kMergeHeads = XF == kXformAttnMerge ? LPR * NCHUNK / kFusedWaves : 1, kMergeAhead = 16, kRecord = 66;
+    // kXformAttnMerge: this wave's heads' {max, sum} per split (one lane each), this thread's quads of the splits
+    constexpr int kMergeHeads = XF == kXformAttnMerge ? LPR * NCHUNK / kFusedWaves : 1, kMergeSplits = kAttnMergeMaxSplits, kRecord = 66;
     float m_part[kMergeHeads], l_part[kMergeHeads];
-    float4 o_part[XF == kXformAttnMerge ? kQuadRounds : 1][XF == kXformAttnMerge ? kMergeAhead : 1];
+    float4 o_part[XF == kXformAttnMerge ? kQuadRounds : 1][XF == kXformAttnMerge ? kMergeSplits : 1];
     uint32_t active = 0;  // splits with a record
     float4 av[XF == kXformRmsNorm || XF == kXformSiluMul ? kQuadRounds : 1];  // the transform's second operand, same quads
     float4 cv[XF == kXformShortConv ? kQuadRounds : 1][7];  // conv operands: c, x', state 0, state 1, three quads of the kernel (xv holds b)
@@ -172,7 +172,7 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
         if constexpr (XF == kXformAttnMerge) {
             const float* rec = static_cast<const float*>(p_x);
             const uint32_t seq = min(*reinterpret_cast<const uint32_t*>(p_aux) + 1u, a.max_seq);
-            active = min((seq + 63u) / 64u, a.splits);
+            active = min(min((seq + 63u) / 64u, a.splits), (uint32_t)kMergeSplits);
 #pragma unroll
             for (int t = 0; t < kMergeHeads; t++) {
                 const uint32_t h = min((threadIdx.x >> 6) + kFusedWaves * t, (p_k >> 6) - 1u);
@@ -184,7 +184,7 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
                 if (past(i)) break;
                 const uint32_t quad = min(threadIdx.x + i * 64 * kFusedWaves, quads - 1);
 #pragma unroll
-                for (int j = 0; j < kMergeAhead; j++) o_part[i][j] = merge_quad(rec, a.splits, min((uint32_t)j, active - 1u), quad);
+                for (int j = 0; j < kMergeSplits; j++) o_part[i][j] = merge_quad(rec, a.splits, min((uint32_t)j, active - 1u), quad);
             }
         } else
 #pragma unroll
@@ -413,27 +413,18 @@ __global__ __launch_bounds__(FUSEQ ? 64 * kFusedWaves : 64) void gemv_pairs_kern
                 if (past(i)) break;
                 const uint32_t quad = min(threadIdx.x + i * 64 * kFusedWaves, quads - 1), h = quad >> 4;
                 float o[4][4] = {};  // [split % 4][dim]: the four groups of attention_merge's threads
-                const auto four = [&](const float4 (&v)[4], uint32_t i0) {
+#pragma unroll
+                for (int i0 = 0; i0 < kMergeSplits; i0 += 4) {
+                    if ((uint32_t)i0 >= active) break;
                     const float4 w4 = *reinterpret_cast<const float4*>(&wts[h * 64u + i0]);
                     const float w[4] = {w4.x, w4.y, w4.z, w4.w};
 #pragma unroll
                     for (int j = 0; j < 4; j++) {
-                        const bool on = i0 + j < active;
-                        o[j][0] = __fadd_rn(o[j][0], on ? __fmul_rn(v[j].x, w[j]) : 0.0f), o[j][1] = __fadd_rn(o[j][1], on ? __fmul_rn(v[j].y, w[j]) : 0.0f);
-                        o[j][2] = __fadd_rn(o[j][2], on ? __fmul_rn(v[j].z, w[j]) : 0.0f), o[j][3] = __fadd_rn(o[j][3], on ? __fmul_rn(v[j].w, w[j]) : 0.0f);
+                        const bool on = (uint32_t)(i0 + j) < active;
+                        const float4 v = o_part[i][i0 + j];
+                        o[j][0] = __fadd_rn(o[j][0], on ? __fmul_rn(v.x, w[j]) : 0.0f), o[j][1] = __fadd_rn(o[j][1], on ? __fmul_rn(v.y, w[j]) : 0.0f);
+                        o[j][2] = __fadd_rn(o[j][2], on ? __fmul_rn(v.z, w[j]) : 0.0f), o[j][3] = __fadd_rn(o[j][3], on ? __fmul_rn(v.w, w[j]) : 0.0f);
                     }
-                };
-#pragma unroll
-                for (int j = 0; j < kMergeAhead; j += 4) {
-                    if ((uint32_t)j >= active) break;
-                    const float4 v[4] = {o_part[i][j], o_part[i][j + 1], o_part[i][j + 2], o_part[i][j + 3]};
-                    four(v, j);
-                }
-                for (uint32_t j = kMergeAhead; j < active; j += 4) {
-                    float4 v[4];
-#pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = merge_quad(static_cast<const float*>(p_x), a.splits, min(j + e, active - 1u), quad);
-                    four(v, j);
                 }
                 float r[4];
 #pragma unroll
@@ -751,12 +742,12 @@ hipError_t launch_pairs_u(GemvArgs& a, uint32_t total_rows, int num_cus, const L
                 return hipErrorInvalidValue;  // shortconv_kernel_applies() keeps such shapes away
             }
         }
-        if (a.xform == kXformAttnMerge) {  // one weight, k <= 2048 (attn_merge_kernel_applies)
-            if constexpr (LPR >= 4 && LPR <= 32 && NCHUNK == 1) {
+        if (a.xform == kXformAttnMerge) {  // one weight, k <= 1024: rows of at most 16 pairs
+            if constexpr (LPR <= 16 && NCHUNK == 1) {
                 if (mode == kSpan) return go(gemv_pairs_kernel<TYPE, LPR, NCHUNK, U, NT, FUSEQ, false, kSpan, kXformAttnMerge>);
                 return go(gemv_pairs_kernel<TYPE, LPR, NCHUNK, U, NT, FUSEQ, false, kSmall, kXformAttnMerge>);
             } else {
-                return hipErrorInvalidValue;
+                return hipErrorInvalidValue;  // attn_merge_kernel_applies() keeps such shapes away
             }
         }
         if (a.xform == kXformRmsNorm) return with_xform(std::integral_constant<int, kXformRmsNorm>{});

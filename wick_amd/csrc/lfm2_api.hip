@@ -453,8 +453,8 @@ int gemv_residual(wick_rocm_ctx* ctx, const wick_rocm_weight* w, float* y, const
 }
 
 // Positions up to which the output projection merges the attention partials itself (16 splits, read in one round trip); beyond, the
-// records of all heads that each of its workgroups then reads cost what the launch costs.
-constexpr uint32_t kFoldMergeBelow = 1024;  // (measured: kXformAttnMerge, gemv_impl.h)
+// records of all heads that each of its workgroups then reads cost what the launch costs (measured: kXformAttnMerge, gemv_impl.h).
+constexpr uint32_t kFoldMergeBelow = kAttnMergeMaxSplits * 64u;
 
 // Enqueues one decode step that reads token / pos from the device: run_layers + the tied LM head
 // (wick/src/model/lfm2.rs:1020-1124, 2258-2289), optionally the greedy pick.

@@ -102,11 +102,13 @@ hipError_t launch_gemv_f32(int type, const GemvBatch& batch, uint32_t k, const f
 // k <= 4096, 4-byte aligned weights) and d_x / d_aux are 16-byte aligned.
 bool gated_kernel_applies(const uint8_t* d_w_gate, const uint8_t* d_w_up, uint32_t k);
 // y (+)= W * quantize(merge of the heads' partials): the output projection behind launch_attention_layer(merge = false), whose partial
-// records [k / 64 heads][splits][66] d_partials holds; the position is *d_pos.  Only when attn_merge_kernel_applies().
+// records [k / 64 heads][splits][66] d_partials holds; the position is *d_pos, and has at most kAttnMergeMaxSplits records of 64
+// positions.  Only when attn_merge_kernel_applies().
+constexpr uint32_t kAttnMergeMaxSplits = 16;
 bool attn_merge_kernel_applies(const uint8_t* d_w, uint32_t k, uint32_t head_dim);
 hipError_t launch_gemv_attn_merge(int type, const uint8_t* d_w, uint32_t m, uint32_t k, const float* d_partials, const uint32_t* d_pos, uint32_t splits,
                                   uint32_t max_seq, float* d_y, int accumulate, int num_cus, const Launch& L);
-// conv_state non-null: the first workgroups also advance that rolling short-conv state by one token (slot s <- slot s + 1, last
+// conv_state non-null: one more workgroup advances that rolling short-conv state by one token (slot s <- slot s + 1, last
 // slot <- b * x of conv_proj = [b | c | x], conv_hidden floats each, conv_hidden % 4 == 0, 16-byte aligned): what
 // launch_shortconv_step does to the state, for a layer whose conv output went through launch_gemv_shortconv_f32.
 hipError_t launch_gemv_gated_f32(int type, const uint8_t* d_w_gate, const uint8_t* d_w_up, uint32_t m, uint32_t k, const float* d_x,
