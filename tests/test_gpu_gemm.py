@@ -502,3 +502,88 @@ def test_one_token_accumulates_into_a_column(ctx, oracle, dtype, layout, ms, k):
             d_y.free()
         for w in ws[1:]:
             w.free()
+
+
+# Pairs of launches on the two sides of each rule that chooses a GEMM kernel, a tile or a number of shares: (m, n, k), the rule's
+# quantity at its limit and one step past it.
+EDGES = [
+    (16384, 9, 128), (16416, 9, 128),      # 512 granules of rows: one workgroup per granule
+    (16384, 32, 3072), (16384, 32, 3200),  # 12288 slabs, up to 32 tokens
+    (16384, 33, 1024), (16384, 33, 1152),  # 4096 slabs, 33 tokens and more
+    (512, 64, 512), (512, 65, 512),        # 64 tokens
+    (256, 32, 2048), (256, 32, 2176),      # 16 slabs of a split launch, up to 32 tokens
+    (256, 33, 1024), (256, 33, 1152),      # 8 slabs, 33 tokens and more
+    (8192, 33, 256), (8224, 33, 256),      # 256 granules: eight waves or four
+    (16416, 48, 128), (16416, 49, 128),    # 48 tokens on the 128-row tiles; 49 .. 64 on the 32x32x32 loop
+    (64, 40, 896), (64, 40, 1024),         # 8 stages: split over K
+    (4096, 1024, 128), (4096, 1025, 128),  # 256 tiles of 128 x 128
+    (2048, 1024, 128), (2048, 1025, 128),  # 256 tiles of 128 x 64: a workgroup per CU
+    (1024, 1024, 4096), (1024, 896, 4096), (1024, 1024, 3968),  # 64 wide tiles, 32 stages: shares on the wide tile
+    (4096, 1024, 4096), (4096, 1025, 4096),                     # 256 wide tiles
+]
+
+
+@pytest.mark.parametrize("m,n,k", EDGES)
+def test_both_sides_of_every_launch_rule(ctx, oracle, m, n, k):
+    """Either side of a rule gives the multi-token GEMV's result (another kernel, other sums: within 1e-6), in both layouts, added to
+    what is there, and leaves the padding alone; split over K as the library does it, and unsplit."""
+    dtype = W.Q4_0 if (m + n + k) % 2 == 0 else W.Q8_0
+    rows = 256 if m % 256 == 0 else 32  # of the weight, repeated: making 16384 of them takes the oracle seconds
+    wb = np.tile(oracle.synth_weight(dtype, rows, k, 7, 0.02).reshape(rows, -1), (m // rows, 1))
+    s, q = oracle.quantize_q8_0_batch(oracle.fill_normal(5, 1.0, n * k), n, k)
+    w, d_q, d_s = ctx.upload_weight(wb, dtype, m, k), ctx.to_device(q), ctx.to_device(s)
+    old = oracle.fill_normal(6, 1.0, (n + 3) * (m + 5))
+    d_ref = ctx.alloc(n * m * 4)
+    ctx.set_gemm_min_n(n + 1)
+    try:
+        ctx.gemm_preq(w, d_s, d_q, n, d_ref, y_stride=m, layout=W.LAYOUT_TOKEN_MAJOR)
+    finally:
+        ctx.set_gemm_min_n(0)
+    ref = fetch_gemm(d_ref, m, n, m, W.LAYOUT_TOKEN_MAJOR)
+    for splits in (0, 1):  # (a limit on unsplit launches is met by launches over several weights, or with the split switched off)
+        got = {}
+        ctx.set_gemm_max_k_splits(splits)
+        try:
+            for layout, stride in ((W.LAYOUT_TOKEN_MAJOR, m + 5), (W.LAYOUT_ROW_MAJOR, n + 3)):
+                outer, inner = (n, m) if layout == W.LAYOUT_TOKEN_MAJOR else (m, n)
+                d_y = ctx.to_device(old)
+                ctx.gemm_preq(w, d_s, d_q, n, d_y, y_stride=stride, layout=layout)
+                got[layout] = fetch_gemm(d_y, m, n, stride, layout).copy()
+                assert rel_l2(got[layout], ref) < 1e-6
+                d_y.upload(old)
+                ctx.gemm_preq(w, d_s, d_q, n, d_y, y_stride=stride, layout=layout, accumulate=True)
+                y, was = d_y.download(np.float32, outer * stride).reshape(outer, stride), old[:outer * stride].reshape(outer, stride)
+                assert np.array_equal(y[:, inner:], was[:, inner:])
+                assert np.array_equal(y[:, :inner], was[:, :inner] + (got[layout].T if layout == W.LAYOUT_TOKEN_MAJOR else got[layout]))
+                d_y.free()
+        finally:
+            ctx.set_gemm_max_k_splits(0)
+        assert np.array_equal(got[W.LAYOUT_TOKEN_MAJOR], got[W.LAYOUT_ROW_MAJOR])
+    w.free(), d_q.free(), d_s.free(), d_ref.free()
+
+
+@pytest.mark.parametrize("m,n,k", [(2048, 1025, 128), (2080, 1024, 128), (2048, 1024, 128), (8224, 65, 128), (8224, 64, 128), (96, 64, 256)])
+def test_the_gated_launch_starts_past_256_tiles(ctx, oracle, m, n, k):
+    """Where the gate | up launch with the gate in its epilogue applies: more than 256 tiles of 64 rows x 128 tokens and more than 64
+    tokens; on the first shapes it takes, the same bits as the separate launches."""
+    from wick_amd.lfm2 import Lfm2Ops
+
+    ops = Lfm2Ops(ctx)
+    ws = [ctx.upload_weight(oracle.synth_weight(W.Q4_0, m, k, seed=41 + i), W.Q4_0, m, k) for i in range(2)]
+    tiles = (m + 63) // 64 * ((n + 127) // 128)
+    assert ops.ffn_gate_up_silu_quantize_applies(ws[0], ws[1], n) == (tiles > 256 and n > 64)
+    if tiles > 256 and n > 64:
+        s, q = oracle.quantize_q8_0_batch(oracle.fill_normal(9, 1.0, n * k), n, k)
+        d_q, d_s, out = ctx.to_device(q), ctx.to_device(s), []
+        d_g, d_u, d_oq, d_os = ctx.alloc(n * m * 4), ctx.alloc(n * m * 4), ctx.alloc(n * m), ctx.alloc(n * (m // 32) * 4)
+        for gated in (True, False):
+            if gated:
+                ops.encode_ffn_gate_up_silu_quantize(ws[0], ws[1], d_s, d_q, n, d_oq, d_os)
+            else:
+                ctx.gemm_preq_multi(ws, d_s, d_q, n, [d_g, d_u], m)
+                ops.silu_mul_quantize(d_g, d_u, n, m, d_oq, d_os)
+            out.append((d_oq.download(np.uint8, n * m), d_os.download(np.uint32, n * (m // 32))))
+        assert all(np.array_equal(a, b) for a, b in zip(*out))
+        for b in (d_q, d_s, d_g, d_u, d_oq, d_os):
+            b.free()
+    ws[0].free(), ws[1].free()

@@ -59,6 +59,39 @@ def test_rmsnorm(ctx, ops, oracle, rows, dim):
         b.free()
 
 
+@pytest.mark.parametrize("eps", [0.0, 1e-5, 1e-30])
+@pytest.mark.parametrize("dim", [1, 7, 32, 100, 1024, 2048, 5000, 6912])
+def test_rmsnorm_inverse_root_against_the_exact_value(ctx, ops, dim, eps):
+    """1 / sqrt(sum / dim + eps), which every norm takes from the hardware's reciprocal root and one step of correction in f64, over
+    sums from the square of the smallest subnormal to beyond the largest f32: the f32 it is rounded to belongs to a value within
+    2^-46 of the exact one (f64 sums of up to 27 terms a thread and eleven more, a product with 1 / dim, the root: under 50 f64
+    roundings).  And zero, infinite and NaN sums."""
+    rng, eps = np.random.default_rng(dim), np.float32(eps)
+    exps = np.arange(-149, 125)
+    x = (rng.standard_normal((exps.size, dim)) * 2.0 ** exps[:, None]).astype(np.float32)
+    x[:, 0] = 2.0 ** exps
+    special = np.zeros((4, dim), np.float32)
+    special[1, dim // 2], special[2, 0], special[3, -1] = np.inf, np.nan, -np.inf
+    special[1:, dim // 3] += np.float32(0.5)
+    rows = np.concatenate([x, special])
+    d_x, d_w, d_y = ctx.to_device(rows), ctx.to_device(np.ones(dim, np.float32)), ctx.alloc(rows.size * 4)
+    ops.encode_rmsnorm(d_x, d_w, d_y, dim, float(eps), rows=len(rows))
+    y = d_y.download(np.float32, rows.size).reshape(rows.shape)
+    for b in (d_x, d_w, d_y):
+        b.free()
+    big, bound = x.astype(np.longdouble), np.longdouble(2.0) ** -46
+    with np.errstate(over="ignore", invalid="ignore", divide="ignore"):
+        inv = 1 / np.sqrt((big * big).sum(1) / dim + np.longdouble(eps))
+        lo, hi = (inv * (1 - bound)).astype(np.float32), (inv * (1 + bound)).astype(np.float32)
+        for j in (0, dim // 2, dim - 1):  # (a product of two f32: monotonous in the second)
+            a, b = x[:, j] * lo, x[:, j] * hi
+            assert np.all((np.minimum(a, b) <= y[:exps.size, j]) & (y[:exps.size, j] <= np.maximum(a, b)) | (np.isnan(a) & np.isnan(y[:exps.size, j])))
+        assert np.mean(lo == hi) > 0.99  # (the interval is one value nearly everywhere)
+        zero = np.float32(np.inf) if eps == 0 else np.float32(1 / np.sqrt(np.float64(eps)))
+        want = np.concatenate([special[:1] * zero, special[1:2] * np.float32(0), special[2:3] * np.float32(np.nan), special[3:] * np.float32(0)])
+    assert np.array_equal(y[exps.size:], want, equal_nan=True)
+
+
 def test_rmsnorm_reference_closed_forms(ctx, ops):
     d_x, d_w, d_y = ctx.to_device(np.array([1, 2, 3, 4], np.float32)), ctx.to_device(np.ones(4, np.float32)), ctx.alloc(16)
     ops.encode_rmsnorm(d_x, d_w, d_y, 4, 1e-5)  # wick/src/backend/cpu.rs:2278-2295

@@ -219,9 +219,9 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
 }
 
 // 1 / sqrt(total / k + eps) of an RMSNorm (rmsnorm, wick/src/backend/cpu.rs:577-594) in f64, rounded to f32 once.  The hardware's
-// reciprocal root (22 bits and more) and one step of third order, y (1 + e / 2 + 3 e^2 / 8) with e = 1 - s y^2: the error is
-// of order e^3, below f64's own rounding, in ten instructions where a division, a root and a division are a serial chain of
-// some eighty in front of every projection of a decode step.
+// reciprocal root (22 bits and more) and one step of Halley's iteration for 1 / sqrt(s), y (1 + e / 2 + 3 e^2 / 8) with
+// e = 1 - s y^2: the error is of order e^3, below f64's own rounding, in ten instructions where a division, a root and a
+// division are a serial chain of some eighty in front of every projection of a decode step.
 __device__ __forceinline__ float rms_inverse(double total, double inv_k, float eps) {
     const double s = __builtin_fma(total, inv_k, (double)eps);
     const double y = __builtin_amdgcn_rsq(s);
