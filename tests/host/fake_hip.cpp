@@ -12,7 +12,7 @@
 #include <string>
 
 namespace fake_hip {
-long launches = 0, out_of_range = 0;
+long launches = 0, other_device = 0, out_of_range = 0;
 thread_local int inside = 0;
 }
 
@@ -44,6 +44,7 @@ struct Config {
     hipStream_t stream;
 };
 thread_local Config config;
+thread_local int current = 0;  // the thread's GPU; the streams' handles are one past theirs
 
 hipError_t done(hipError_t e) {
     if (e != hipSuccess) last = e;
@@ -78,8 +79,9 @@ void enqueue(std::function<void()> f) {
     if (!st().capturing) st().queue.push_back(std::move(f));
 }
 
-hipError_t launch(const void* f, void** args) {
+hipError_t launch(const void* f, void** args, hipStream_t stream) {
     Lock lk;
+    if (reinterpret_cast<uintptr_t>(stream) != (uintptr_t)current + 1) fake_hip::other_device++;
     if (due(st().launch_fails)) return done(hipErrorLaunchFailure);
     fake_hip::launches++;
     if (st().kernels[f].find("stage_copy_kernel") == std::string::npos) {
@@ -159,14 +161,17 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shared, hi
     *grid = config.grid, *block = config.block, *shared = config.shared, *stream = config.stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t) { return launch(f, args); }
-hipError_t hipExtLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t, hipEvent_t, hipEvent_t, int) { return launch(f, args); }
+hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t s) { return launch(f, args, s); }
+hipError_t hipExtLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t s, hipEvent_t, hipEvent_t, int) { return launch(f, args, s); }
 
 hipError_t hipGetDeviceCount(int* n) {
-    *n = 1;
+    *n = 2;
     return hipSuccess;
 }
-hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipSetDevice(int d) {
+    current = d;
+    return hipSuccess;
+}
 hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) {
     std::memset(p, 0, sizeof *p);
     std::strcpy(p->gcnArchName, "gfx950");
@@ -217,7 +222,7 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void* p) {
 }
 
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
-    *s = handle<hipStream_t>();
+    *s = reinterpret_cast<hipStream_t>((uintptr_t)current + 1);
     return hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }

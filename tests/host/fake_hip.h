@@ -8,6 +8,7 @@ namespace fake_hip {
 
 extern thread_local int inside;  // this thread is in the runtime, not in the library's code
 extern long launches;      // kernels enqueued so far
+extern long other_device;  // kernels on a stream of another GPU than the calling thread's (there are two)
 extern long out_of_range;  // accesses of the copy kernel outside every allocation (they are left out)
 size_t pending();          // enqueued and not done
 size_t allocations();      // device allocations that are not freed

@@ -253,6 +253,47 @@ void memory(const char* path) {
     wick_rocm_buffer_free(ctx, d);
 }
 
+// A model on the second GPU, called from a thread whose current one is the first: every launch of every call goes to the model's.
+void devices(const char* path) {
+    wick_rocm_ctx *first = nullptr, *ctx = nullptr;
+    CHECK(wick_rocm_ctx_create(1, &ctx) == WICK_ROCM_OK && wick_rocm_ctx_create(0, &first) == WICK_ROCM_OK, "contexts");
+    Gguf g(path);
+    wick_rocm_lfm2* m = nullptr;
+    CHECK(wick_rocm_lfm2_load(ctx, g.g, 64, &m) == WICK_ROCM_OK, "load");
+    wick_rocm_lfm2_config cfg;
+    wick_rocm_lfm2_get_config(m, &cfg);
+    std::vector<float> logits(cfg.vocab_size), frame(3 * cfg.hidden_size);
+    std::vector<unsigned char> state(wick_rocm_lfm2_state_bytes(m, 20));
+    uint32_t tokens[20] = {}, picks[4], consumed;
+    const auto each = [&](const char* what, auto&& call) {
+        wick_rocm_sync(first);  // makes the first GPU current, as work of the caller's on it does
+        fake_hip::other_device = 0;
+        const int rc = call();
+        CHECK(rc == WICK_ROCM_OK && fake_hip::other_device == 0, "%s: %d, %ld launches beside the model's GPU", what, rc, fake_hip::other_device);
+    };
+    for (int replay : {0, 1}) {
+        wick_rocm_lfm2_set_graph_replay(m, replay);
+        each("reset", [&] { return wick_rocm_lfm2_reset(ctx, m); });
+        each("step", [&] { return wick_rocm_lfm2_forward(ctx, m, 1, 0, logits.data()); });
+        each("prompt", [&] { return wick_rocm_lfm2_forward_prefill(ctx, m, tokens, 20, 0, logits.data()); });
+        each("short prompt", [&] { return wick_rocm_lfm2_forward_prefill(ctx, m, tokens, 2, 0, logits.data()); });
+        each("chunked prompt", [&] { return wick_rocm_lfm2_forward_prefill_chunked(ctx, m, tokens, 20, 0, 7, nullptr, &consumed, logits.data()); });
+        each("embedded prompt", [&] { return wick_rocm_lfm2_forward_prefill_from_embeddings(ctx, m, frame.data(), 3, 0, logits.data()); });
+        each("short embedded prompt", [&] { return wick_rocm_lfm2_forward_prefill_from_embeddings(ctx, m, frame.data(), 1, 0, logits.data()); });
+        each("greedy", [&] { return wick_rocm_lfm2_generate_greedy(ctx, m, 1, 5, 4, picks); });
+        each("greedy step", [&] { return wick_rocm_lfm2_forward_greedy(ctx, m, 1, 5, picks); });
+        each("embedded step", [&] { return wick_rocm_lfm2_forward_from_embedding(ctx, m, frame.data(), 5, logits.data()); });
+        each("hidden state", [&] { return wick_rocm_lfm2_forward_embedding(ctx, m, 1, 5, frame.data()); });
+        each("hidden state of a frame", [&] { return wick_rocm_lfm2_forward_hidden_from_embedding(ctx, m, frame.data(), 5, frame.data()); });
+        each("snapshot", [&] { return wick_rocm_lfm2_snapshot_state(ctx, m, 20, state.data(), state.size()); });
+        each("restore", [&] { return wick_rocm_lfm2_restore_state(ctx, m, 20, state.data(), state.size()); });
+        each("shift in place", [&] { return wick_rocm_lfm2_shift_kv(ctx, m, 20, 2, 6); });
+        each("staged shift", [&] { return wick_rocm_lfm2_shift_kv(ctx, m, 40, 2, 1); });
+    }
+    wick_rocm_lfm2_free(ctx, m);
+    wick_rocm_ctx_destroy(ctx), wick_rocm_ctx_destroy(first);
+}
+
 }  // namespace
 
 void* operator new(size_t n) {
@@ -276,6 +317,7 @@ int main(int argc, char** argv) {
     else if (!std::strcmp(name, "copies") && argc > 2) copies(argv[2]);
     else if (!std::strcmp(name, "prompts") && argc > 2) prompts(argv[2]);
     else if (!std::strcmp(name, "memory") && argc > 2) memory(argv[2]);
+    else if (!std::strcmp(name, "devices") && argc > 2) devices(argv[2]);
     else CHECK(false, "no case '%s'", name);
     return failures ? 1 : 0;
 }

@@ -49,3 +49,7 @@ def test_a_prompt_that_fails_leaves_nothing_pending(host_faults, model_file):
 
 def test_no_exception_leaves_an_entry_point_when_host_memory_runs_out(host_faults, model_file):
     host_faults("memory", model_file)
+
+
+def test_every_launch_of_a_model_goes_to_its_own_gpu(host_faults, model_file):
+    host_faults("devices", model_file)

@@ -870,9 +870,8 @@ size_t wick_rocm_lfm2_gpu_memory_bytes(const wick_rocm_lfm2* model) { return mod
 int wick_rocm_lfm2_reset(wick_rocm_ctx* ctx, wick_rocm_lfm2* model) {
     if (!ctx || !model) return WICK_ROCM_ERR_INVALID_ARG;
     std::lock_guard<std::mutex> lk(model->mu);
-    std::lock_guard<std::recursive_mutex> whole_step(ctx->mu);  // nothing else gets onto the context's stream (or into a capture) in between
+    WR_ENTER(ctx);  // held to the end: nothing else gets onto the context's stream (or into a capture) in between
     if (ctx->capturing) return fail(ctx, WICK_ROCM_ERR_STATE, "lfm2_reset during graph capture");
-    Guard device(ctx);
     const hipError_t e = launch_fill_zero(model->conv_states, model->conv_floats, ctx->launch());  // in stream order, like the steps around it
     if (e != hipSuccess) return fail_hip(ctx, e, "reset launch");
     return WICK_ROCM_OK;
@@ -888,7 +887,7 @@ int wick_rocm_lfm2_set_graph_replay(wick_rocm_lfm2* model, int enabled) {
 int wick_rocm_lfm2_forward(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uint32_t token, uint32_t pos, float* logits) {
     if (!ctx || !model) return WICK_ROCM_ERR_INVALID_ARG;
     std::lock_guard<std::mutex> lk(model->mu);
-    std::lock_guard<std::recursive_mutex> whole_step(ctx->mu);  // nothing else gets onto the context's stream (or into a capture) in between
+    WR_ENTER(ctx);  // held to the end: nothing else gets onto the context's stream (or into a capture) in between
     if (int rc = check_step(ctx, model, token, pos, 1)) return rc;
     if (int rc = set_step(ctx, model, token, pos)) return rc;
     if (int rc = run_step(ctx, model, kStepLogits, pos)) return rc;
@@ -923,10 +922,8 @@ static int prefill_passes(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, const uint3
     for (uint32_t done = 0; done < n; done += model->prefill_cap) {
         last = n - done < model->prefill_cap ? n - done : model->prefill_cap;
         if (tokens) {
-            if (!model->h_tokens) {
-                Guard device(ctx);
+            if (!model->h_tokens)
                 WR_HIP(ctx, hipHostMalloc(reinterpret_cast<void**>(&model->h_tokens), (size_t)c.max_seq_len * sizeof(uint32_t), hipHostMallocDefault));
-            }
             memcpy(model->h_tokens + done, tokens + done, (size_t)last * sizeof(uint32_t));  // (no earlier prompt's pass is under way: prefill_locked)
         } else {  // frame j of the prompt is row j of the pass's input (wick/src/model/lfm2.rs:2452-2487)
             if (int rc = wick_rocm_upload(ctx, model->pX, embeddings + (size_t)done * c.hidden_size, (size_t)last * c.hidden_size * sizeof(float))) return rc;
@@ -953,7 +950,7 @@ int wick_rocm_lfm2_forward_prefill(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, co
     if (!ctx || !model) return WICK_ROCM_ERR_INVALID_ARG;
     if (!tokens || n == 0) return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2 prefill: empty prompt");
     std::lock_guard<std::mutex> lk(model->mu);
-    std::lock_guard<std::recursive_mutex> whole_step(ctx->mu);  // nothing else gets onto the context's stream (or into a capture) in between
+    WR_ENTER(ctx);  // held to the end: nothing else gets onto the context's stream (or into a capture) in between
     for (uint32_t j = 0; j < n; j++)
         if (tokens[j] >= model->cfg.vocab_size) return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2: token_id out of range");
     return prefill_locked(ctx, model, tokens, nullptr, n, start_pos, logits);
@@ -964,7 +961,7 @@ int wick_rocm_lfm2_forward_prefill_from_embeddings(wick_rocm_ctx* ctx, wick_rocm
     if (!ctx || !model) return WICK_ROCM_ERR_INVALID_ARG;
     if (!embeddings || n == 0) return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2 prefill: at least one frame is required");
     std::lock_guard<std::mutex> lk(model->mu);
-    std::lock_guard<std::recursive_mutex> whole_step(ctx->mu);
+    WR_ENTER(ctx);
     return prefill_locked(ctx, model, nullptr, embeddings, n, start_pos, logits);
 }
 
@@ -995,7 +992,7 @@ int wick_rocm_lfm2_generate_greedy(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, ui
     if (!out_tokens) return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2: null output pointer");
     if (n == 0) return WICK_ROCM_OK;
     std::lock_guard<std::mutex> lk(model->mu);
-    std::lock_guard<std::recursive_mutex> whole_step(ctx->mu);  // nothing else gets onto the context's stream (or into a capture) in between
+    WR_ENTER(ctx);  // held to the end: nothing else gets onto the context's stream (or into a capture) in between
     if (int rc = check_step(ctx, model, token, pos, n)) return rc;
     if (int rc = set_step(ctx, model, token, pos)) return rc;
     for (uint32_t i = 0; i < n; i++)  // the pick of step i is written to the device-side token and position pos + i of the history
@@ -1027,14 +1024,14 @@ int wick_rocm_lfm2_forward_from_embedding(wick_rocm_ctx* ctx, wick_rocm_lfm2* mo
     if (!ctx || !model) return WICK_ROCM_ERR_INVALID_ARG;
     if (!embedding) return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2: null embedding pointer");
     std::lock_guard<std::mutex> lk(model->mu);
-    std::lock_guard<std::recursive_mutex> whole_step(ctx->mu);
+    WR_ENTER(ctx);
     return step_locked(ctx, model, 0, embedding, pos, kStepLogits, logits);
 }
 
 int wick_rocm_lfm2_forward_embedding(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uint32_t token, uint32_t pos, float* hidden) {
     if (!ctx || !model) return WICK_ROCM_ERR_INVALID_ARG;
     std::lock_guard<std::mutex> lk(model->mu);
-    std::lock_guard<std::recursive_mutex> whole_step(ctx->mu);
+    WR_ENTER(ctx);
     return step_locked(ctx, model, token, nullptr, pos, kStepHidden, hidden);
 }
 
@@ -1042,7 +1039,7 @@ int wick_rocm_lfm2_forward_hidden_from_embedding(wick_rocm_ctx* ctx, wick_rocm_l
     if (!ctx || !model) return WICK_ROCM_ERR_INVALID_ARG;
     if (!embedding) return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2: null embedding pointer");
     std::lock_guard<std::mutex> lk(model->mu);
-    std::lock_guard<std::recursive_mutex> whole_step(ctx->mu);
+    WR_ENTER(ctx);
     return step_locked(ctx, model, 0, embedding, pos, kStepHidden, hidden);
 }
 
@@ -1066,7 +1063,7 @@ size_t wick_rocm_lfm2_state_bytes(const wick_rocm_lfm2* model, uint32_t seq_len)
 int wick_rocm_lfm2_snapshot_state(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uint32_t seq_len, void* out, size_t nbytes) {
     if (!ctx || !model) return WICK_ROCM_ERR_INVALID_ARG;
     std::lock_guard<std::mutex> lk(model->mu);
-    std::lock_guard<std::recursive_mutex> whole(ctx->mu);
+    WR_ENTER(ctx);
     if (seq_len > model->cfg.max_seq_len) return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2 snapshot: seq_len beyond the context size");
     if (nbytes != wick_rocm_lfm2_state_bytes(model, seq_len) || (!out && nbytes))
         return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2 snapshot: the buffer must hold exactly wick_rocm_lfm2_state_bytes(model, seq_len) bytes");
@@ -1076,7 +1073,7 @@ int wick_rocm_lfm2_snapshot_state(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uin
 int wick_rocm_lfm2_restore_state(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uint32_t seq_len, const void* in, size_t nbytes) {
     if (!ctx || !model) return WICK_ROCM_ERR_INVALID_ARG;
     std::lock_guard<std::mutex> lk(model->mu);
-    std::lock_guard<std::recursive_mutex> whole(ctx->mu);
+    WR_ENTER(ctx);
     if (seq_len > model->cfg.max_seq_len) return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2 restore: seq_len beyond the context size");
     if (nbytes != wick_rocm_lfm2_state_bytes(model, seq_len) || (!in && nbytes))
         return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2 restore: the snapshot must hold exactly wick_rocm_lfm2_state_bytes(model, seq_len) bytes");
@@ -1086,7 +1083,7 @@ int wick_rocm_lfm2_restore_state(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uint
 int wick_rocm_lfm2_shift_kv(wick_rocm_ctx* ctx, wick_rocm_lfm2* model, uint32_t seq_len, uint32_t n_keep, uint32_t shift) {
     if (!ctx || !model) return WICK_ROCM_ERR_INVALID_ARG;
     std::lock_guard<std::mutex> lk(model->mu);
-    std::lock_guard<std::recursive_mutex> whole(ctx->mu);
+    WR_ENTER(ctx);
     const wick_rocm_lfm2_config& c = model->cfg;
     if (shift == 0) return ctx_fail(ctx, WICK_ROCM_ERR_INVALID_ARG, "lfm2 shift_kv: shift must be > 0");
     if (seq_len > c.max_seq_len || (uint64_t)n_keep + shift > seq_len)
