@@ -17,7 +17,8 @@
  *     its stream and uploaded weights.
  *   - All hot-path calls only ENQUEUE work on the context's stream (like encoding
  *     into a Metal command encoder, wick/src/model/metal_lfm2.rs:1-4); nothing
- *     synchronises except wick_rocm_sync / wick_rocm_download / event queries.
+ *     synchronises except wick_rocm_sync, host copies (wick_rocm_upload,
+ *     wick_rocm_download, uploads of weights) and event queries.
  *   - Calls on one context serialise on an internal mutex, the counterpart of the
  *     GPU models' `infer_lock` (wick/src/model/metal_lfm2.rs:254-267).
  *   - Weight bytes keep the GGUF block layout verbatim (wick/src/quant.rs:13-34):
@@ -190,17 +191,21 @@ size_t wick_rocm_weight_device_bytes(const wick_rocm_weight *w);
  * WICK_SPLITS switches (wick/src/backend/cpu.rs:23-27). */
 int wick_rocm_set_gemm_min_n(wick_rocm_ctx *ctx, uint32_t min_n);
 
-/* A GEMM launch that would leave at least half of the CUs without a tile while walking a long K (few tokens x few rows x
- * k >= 2048: the down projection of a short prompt) is split over K in up to max_splits shares (1, 2, 4, 8): the shares' sums go
- * to context scratch and a second small launch adds them up in a fixed order -- deterministic, but not the same low-order bits
- * as the unsplit sum (both inside the f32 bar).  max_splits = 1 switches it off, 0 restores the default (8).  A tuning knob like
- * the one above; wick_rocm_matmul_f32_noalloc never splits. */
+/* A single-weight GEMM launch that would leave at least half of the CUs without a tile (few tokens x few rows, k >= 1024), or that
+ * has 64 .. 256 tiles of 128 x 128 and k >= 4096 (the down projection of a long prompt), is split over K in up to max_splits
+ * shares (1, 2, 4, 8), which are added up in a fixed order -- deterministic, but not the same low-order bits as the unsplit sum
+ * (both inside the f32 bar).  The shares' sums go to context scratch and a second small launch adds them up (or the norm behind a
+ * wick_rocm_gemm_q8_residual_rmsnorm_quantize); launches of up to 64 tokens with a K that is not long (at most 16 stages of 128
+ * up to 32 tokens, 8 above) walk the shares one after the other in each workgroup and need neither.  max_splits = 1 switches it
+ * off, 0 restores the default (8).  A tuning knob like the one above; wick_rocm_matmul_f32_noalloc never splits. */
 int wick_rocm_set_gemm_max_k_splits(wick_rocm_ctx *ctx, uint32_t max_splits);
 
-/* Which matrix-core instruction the GEMM's block loops are built on: 32 (the default, also 0) = v_mfma_i32_32x32x32_i8
- * (two per block and wave on the wide tile, one on the narrow tile when the launch has more than 48 tokens), 16 = eight / four
- * v_mfma_i32_16x16x32_i8 (what the gated feed-forward launch and narrow launches of up to 48 tokens always use).  Block dots are bit-identical either way, f32 sums agree to the last bit or two (the order in
- * which a row's blocks are added is the same, the lanes that hold them differ).  A tuning knob like the ones above. */
+/* Which matrix-core instruction the GEMM's block loops are built on: 32 (the default, also 0) = v_mfma_i32_32x32x32_i8, on the tile
+ * and for the number of tokens that each launch's size selects; 16 = v_mfma_i32_16x16x32_i8 on 128 rows x 64 tokens where the
+ * launch has few tiles and on 128 x 128 elsewhere.  Two kinds of launch do not ask: few tokens over more rows or a longer K than
+ * the 32x32x32 loop has a kernel for (up to 48) always use the 16x16x32 one, the gated feed-forward launch
+ * (wick_rocm_ffn_gate_up_silu_quantize_q8) always the other.  Block dots are bit-identical either way, f32 sums agree to the last
+ * bit or two.  A tuning knob like the ones above. */
 int wick_rocm_set_gemm_mfma_shape(wick_rocm_ctx *ctx, int shape);
 
 /* How the single-token GEMV fetches its weights, by bytes of weights in one launch: below
@@ -224,8 +229,7 @@ int wick_rocm_matmul_f32(wick_rocm_ctx *ctx, const wick_rocm_weight *w, const fl
  * forbid allocation.  Same arguments and same kernels, but the Q8_0-quantized activations go into a fixed array in device
  * memory that is part of the library's image (4.5 MiB per GPU, held until the process ends) instead of context scratch that
  * grows on demand.  Results are bit-identical to wick_rocm_matmul_f32 wherever that call does not split its launch over K
- * (wick_rocm_set_gemm_max_k_splits: always with max_splits = 1; with the default only prompts of few tokens over a long K
- * split) and within the f32 bar of it otherwise: this entry point never splits, the shares would need scratch of their own.
+ * (wick_rocm_set_gemm_max_k_splits says which launches split; none with max_splits = 1) and within the f32 bar of it otherwise: this entry point never splits, the shares would need scratch of their own.
  * Limits and rules:
  *   - n * k <= 4194304 elements (e.g. 2048 tokens x 2048, 512 x 8192); larger calls return WICK_ROCM_ERR_BAD_SHAPE;
  *   - no hipMalloc, hipFree or other allocating call is made, on any path; with per-dispatch kernel timing on

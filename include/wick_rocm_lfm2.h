@@ -103,8 +103,8 @@ int wick_rocm_attention_prefill_quantize_q8_0(wick_rocm_ctx *ctx, const float *d
 
 /* The attention block between the Q/K/V projections and the output projection: what wick_rocm_qk_norm_rope followed
  * by wick_rocm_attention_decode compute (wick/src/model/lfm2.rs:783-1006), bit for bit, with the norm, the rotation and
- * the KV append folded into the attention kernel (workgroups norm and rotate their own query head; those that own the
- * new position norm, rotate and append K and V themselves), one launch less.  d_scratch:
+ * the KV append folded into the attention kernel (every workgroup norms and rotates its own query heads and the new key, one
+ * workgroup per KV head appends the new rows), one launch less.  d_scratch:
  * wick_rocm_attention_block_scratch_bytes(...) bytes, contents need not be kept.  d_q / d_k may be overwritten (head
  * dims without a fused kernel run the separate launches, which work in place). */
 size_t wick_rocm_attention_block_scratch_bytes(uint32_t max_seq, uint32_t n_heads, uint32_t head_dim);
@@ -132,7 +132,7 @@ int wick_rocm_shortconv_seq_quantize_q8_0(wick_rocm_ctx *ctx, const float *d_pro
  *   wick_rocm_shortconv_out_proj_f32        y (+)= W_out * quantize(c * conv(b * x)): the out projection computes the gated
  *                                           convolution in its prologue from d_proj, the conv weight and the rolling state,
  *                                           which it only READS (every workgroup needs the old state);
- *   wick_rocm_ffn_gate_up_conv_advance_f32  wick_rocm_ffn_gate_up_f32 of the same layer, whose first workgroups also advance
+ *   wick_rocm_ffn_gate_up_conv_advance_f32  wick_rocm_ffn_gate_up_f32 of the same layer, with one more workgroup that advances
  *                                           the rolling state by this token (slot s <- slot s + 1, last slot <- b * x).
  * Called in this order, y, d_act and the state are bit-identical to wick_rocm_shortconv_step + wick_rocm_matmul_f32(accumulate)
  * + wick_rocm_ffn_gate_up_f32.  Shapes: kernel size 3, hidden <= 2048 (even block count), Q4_0 / Q8_0 weights the one-launch
@@ -223,7 +223,10 @@ int wick_rocm_lfm2_reset(wick_rocm_ctx *ctx, wick_rocm_lfm2 *model);
  * With enabled = 0 the same launches are enqueued one by one instead, which per-dispatch timing
  * (wick_rocm_kernel_timing_begin) and kernel tracers need; results are identical.  While per-dispatch timing is on,
  * steps are enqueued one by one whatever this switch says.  The counterpart of the
- * reference's profiled encode path (encode_layers_profiled, wick/src/model/metal_lfm2.rs:4559-4712). */
+ * reference's profiled encode path (encode_layers_profiled, wick/src/model/metal_lfm2.rs:4559-4712).
+ * A graph is captured when it is first needed: one per kind of step (logits, greedy pick, hidden state) and side of position
+ * 1024, below which the output projections merge the attention partials.  The first step of a kind takes 0.3 - 1.5 ms longer for
+ * it, the first one past 1024 -- in the middle of a run, if the run passes there -- 0.15 - 0.35 ms. */
 int wick_rocm_lfm2_set_graph_replay(wick_rocm_lfm2 *model, int enabled);
 
 /* Model::forward (wick/src/model/lfm2.rs:2258-2289): one token at position `pos` (= tokens seen so far) ->
@@ -277,8 +280,9 @@ int wick_rocm_lfm2_snapshot_state(wick_rocm_ctx *ctx, wick_rocm_lfm2 *model, uin
 int wick_rocm_lfm2_restore_state(wick_rocm_ctx *ctx, wick_rocm_lfm2 *model, uint32_t seq_len, const void *in, size_t nbytes);
 
 /* Model::shift_kv (wick/src/model/lfm2.rs:2507-2516, wick/src/model/metal_lfm2.rs:2473-2531; supports_kv_shift is true for
- * this backend): wick_rocm_kv_shift on every attention layer of a state of seq_len positions; gated-conv layers keep their
- * rolling buffer.  The next step's position is seq_len - shift.  Waits for the shift. */
+ * this backend): what wick_rocm_kv_shift does, on every attention layer of a state of seq_len positions (in place, several layers
+ * to a launch, where head_dim % 8 == 0 and the moved rows are at most 16 times `shift`; through a staging buffer otherwise: the
+ * same bytes); gated-conv layers keep their rolling buffer.  The next step's position is seq_len - shift.  Waits for the shift. */
 int wick_rocm_lfm2_shift_kv(wick_rocm_ctx *ctx, wick_rocm_lfm2 *model, uint32_t seq_len, uint32_t n_keep, uint32_t shift);
 
 /* The logits of the last step on the device ([vocab_size] floats). */

@@ -487,3 +487,18 @@ def test_cpp_host_mirror_runs_the_model(ctx, oracle, tmp_path):
     assert got == want
     a, b = lines["prefill"].split()
     assert a == b
+
+
+def test_greedy_run_across_the_change_of_step_graphs(ctx, oracle, tmp_path):
+    """A run that passes the position from which the merge of the attention partials is a launch of its own: the second graph of the
+    step is captured between two of its tokens (first run) or is there already (second), and the picks are those of steps
+    enqueued launch by launch."""
+    model, _, cfg = load(ctx, oracle, tmp_path, context=1100, n_layers=2, hidden=512, inter=512, n_heads=8, kv_heads=(4, 0), vocab=320, seed=8)
+    start = np.random.default_rng(3).standard_normal(model.snapshot_state(1018).size // 4).astype(np.float32).view(np.uint8)
+    picks = []
+    for graphs in (True, True, False):
+        model.set_graph_replay(graphs)
+        model.restore_state(start, 1018)
+        picks.append(model.generate_greedy(7, 1018, 12))
+    assert np.array_equal(picks[0], picks[2]) and np.array_equal(picks[1], picks[2])
+    model.free()
