@@ -195,8 +195,8 @@ int wick_rocm_set_gemm_min_n(wick_rocm_ctx *ctx, uint32_t min_n);
  * has 64 .. 256 tiles of 128 x 128 and k >= 4096 (the down projection of a long prompt), is split over K in up to max_splits
  * shares (1, 2, 4, 8), which are added up in a fixed order -- deterministic, but not the same low-order bits as the unsplit sum
  * (both inside the f32 bar).  The shares' sums go to context scratch and a second small launch adds them up (or the norm behind a
- * wick_rocm_gemm_q8_residual_rmsnorm_quantize); launches of up to 64 tokens with a K that is not long (at most 16 stages of 128
- * up to 32 tokens, 8 above) walk the shares one after the other in each workgroup and need neither.  max_splits = 1 switches it
+ * wick_rocm_gemm_q8_residual_rmsnorm_quantize); launches of up to 64 tokens with a K that is not long (at most 2048 up to 32
+ * tokens, 1024 above) may walk the shares one after the other in each workgroup instead, which gives the same bits.  max_splits = 1 switches it
  * off, 0 restores the default (8).  A tuning knob like the one above; wick_rocm_matmul_f32_noalloc never splits. */
 int wick_rocm_set_gemm_max_k_splits(wick_rocm_ctx *ctx, uint32_t max_splits);
 

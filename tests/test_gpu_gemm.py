@@ -352,9 +352,12 @@ def test_gemm_split_over_k(ctx, oracle, dtype, m, n, k, layout, accumulate):
     (W.Q4_0, 256, 300, 1024, 0),    # 10 tiles
     (W.Q4_0, 1024, 2002, 4608, 0),  # 256 tiles: unsplit, the plain norm kernel
     (W.Q8_0, 512, 7, 256, 4),       # below the MFMA hand-off: multi-token GEMV, then the norm
-    (W.Q4_0, 1024, 23, 1024, 0),    # few tokens, split in 4: the shares added inside the launch, or by the norm on the 16x16x32 loop
-    (W.Q8_0, 512, 64, 1024, 4),     # the same at the most tokens such a launch has
-    (W.Q4_0, 1024, 40, 4608, 0),    # few tokens, K too long for that: shares side by side either way
+    (W.Q4_0, 1024, 23, 1024, 0),    # few tokens, split in 4: the shares walked inside the launch (by the norm on the 16x16x32 loop)
+    (W.Q8_0, 768, 32, 1024, 4), (W.Q8_0, 736, 32, 1024, 4),   # 24 granules: inside the launch; fewer: the norm adds them up
+    (W.Q4_0, 2304, 20, 1536, 0), (W.Q4_0, 2272, 20, 1536, 0),  # 72 granules, 12 slabs: the same
+    (W.Q4_0, 3840, 33, 1024, 0), (W.Q4_0, 3808, 64, 1024, 0),  # 120 granules, 33 tokens and more: the same
+    (W.Q8_0, 512, 64, 1024, 4),     # the norm adds them up; the plain call walks them inside the launch
+    (W.Q4_0, 1024, 40, 4608, 0),    # K too long for that: shares side by side either way
 ])
 def test_residual_projection_with_norm_and_quantizer(ctx, oracle, dtype, m, n, k, pad, shape):
     """x += W a, then Q8_0(rmsnorm(x)): one call == wick_rocm_gemm_q8 (accumulate) + wick_rocm_rmsnorm_quantize_q8_0, bit for bit -- the
@@ -511,7 +514,8 @@ EDGES = [
     (16384, 32, 3072), (16384, 32, 3200),  # 12288 slabs, up to 32 tokens
     (16384, 33, 1024), (16384, 33, 1152),  # 4096 slabs, 33 tokens and more
     (512, 64, 512), (512, 65, 512),        # 64 tokens
-    (256, 32, 2048), (256, 32, 2176),      # 16 slabs of a split launch, up to 32 tokens
+    (256, 32, 1920), (256, 32, 2048),      # 15 slabs of a split launch, up to 32 tokens and under 96 granules
+    (3040, 9, 2048), (3072, 9, 2048), (3072, 9, 2176),  # 16 slabs from 96 granules on
     (256, 33, 1024), (256, 33, 1152),      # 8 slabs, 33 tokens and more
     (8192, 33, 256), (8224, 33, 256),      # 256 granules: eight waves or four
     (16416, 48, 128), (16416, 49, 128),    # 48 tokens on the 128-row tiles; 49 .. 64 on the 32x32x32 loop

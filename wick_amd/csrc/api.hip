@@ -158,11 +158,16 @@ int gemm_locked(wick_rocm_ctx* ctx, const wick_rocm_weight* w, const int8_t* d_q
     hipError_t e;
     if (n >= ctx->min_n_for(w->nbytes) && mfma_ok) {
         uint32_t splits = may_split && ctx->gemm_max_splits > 1 ? gemm_split_k(w->m, n, w->k, ctx->gemm_max_splits) : 1u;
-        const bool in_launch = gemm_split_in_launch(w->m, n, w->k, ctx->launch());  // needs no scratch
+        bool in_launch = gemm_split_in_launch(w->m, n, w->k, ctx->launch(), deferred != nullptr);  // needs no scratch
         if (splits > 1 && !in_launch) {
             const size_t floats = (size_t)splits * n * w->m;
-            if (ctx->capturing && floats > ctx->scratch_f_cap) splits = 1;  // no room reserved: the unsplit launch, same result to the f32 bar
-            else if (int rc = ensure_scratch(ctx, 0, 0, floats)) return rc;
+            if (ctx->capturing && floats > ctx->scratch_f_cap) {
+                // no room reserved: the shares inside the launch where it can (the same bits), else unsplit (the same to the f32 bar)
+                in_launch = gemm_split_in_launch(w->m, n, w->k, ctx->launch(), false);
+                if (!in_launch) splits = 1;
+            } else if (int rc = ensure_scratch(ctx, 0, 0, floats)) {
+                return rc;
+            }
         }
         const bool defer = deferred && splits > 1 && !in_launch;
         e = launch_gemm_mfma(w->type, static_cast<const uint8_t*>(w->d_gemm), w->m, w->k, d_q, d_s, n, d_y, y_stride,
@@ -953,7 +958,7 @@ int wick_rocm_block_dots_i32(wick_rocm_ctx* ctx, const wick_rocm_weight* w, cons
         return WICK_ROCM_OK;
     }
     const bool mfma = w->d_gemm && n >= ctx->min_n_for(w->nbytes) && (w->k % 128u == 0) && (reinterpret_cast<uintptr_t>(d_quants) % 16u == 0);
-    hipError_t e = mfma ? launch_block_dots_mfma(w->type, static_cast<const uint8_t*>(w->d_gemm), w->m, w->k, d_quants, n, d_out, ctx->launch())
+    hipError_t e = mfma ? launch_block_dots_mfma(w->type, static_cast<const uint8_t*>(w->d_gemm), w->m, w->k, d_quants, n, d_out, ctx->gemm_max_splits, ctx->launch())
                         : launch_block_dots_gemv(w->type, static_cast<const uint8_t*>(w->d), w->m, w->k, d_quants, n, d_out, ctx->num_cus, ctx->launch());
     if (e != hipSuccess) return fail_hip(ctx, e, "block_dots launch");
     return WICK_ROCM_OK;

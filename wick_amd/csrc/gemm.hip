@@ -1289,13 +1289,27 @@ uint32_t wide_split_factor(uint32_t m, uint32_t n, uint32_t k, uint32_t max_spli
 bool narrow_tiles(uint64_t row_tiles, uint32_t n) { return n <= BN_NARROW || row_tiles * ((n + BN - 1) / BN) <= kCus; }
 
 // Launches of gemm_few_kernel: up to 64 tokens and few enough granules that latency and not the chip's throughput is what they cost
-// (every workgroup fetches all tokens' activations for its 32 rows; beyond, the 128-row tiles are the cheaper readers).  A round of K
-// takes it ~2 us, so a long K that the tiles may split into shares side by side stays with them.  Tiles / here, us:  unsplit 2048 x
-// 1024 over 23 tokens 8.8 / 4.9, 1024 x 4608 29 / 14; split 1024 x 1024 over 23 6.7 / 4.9, 9216 x 2048 12.1 / 10.1, 1024 x 4608
-// 8.9 / 14.3, 2048 x 2048 over 40 8.2 / 11.5; 65536 x 2048 over 16 27 / 40.
-bool few_applies(uint64_t rows, uint32_t n, uint32_t k, bool split) {
+// (every workgroup fetches all tokens' activations for its 32 rows; beyond, the 128-row tiles are the cheaper readers).  Tiles / here,
+// us: 2048 x 1024 over 23 tokens 8.8 / 4.9, 1024 x 4608 29 / 14; 65536 x 2048 over 16 27 / 40.
+bool few_applies(uint64_t rows, uint32_t n, uint32_t k) {
     const uint64_t units = (rows + GR - 1) / GR, slabs = k / (KB * 32);
-    return n <= 64 && units <= 2 * kCus && units * slabs <= (n <= 32 ? 12288u : 4096u) && (!split || slabs <= (n <= 32 ? 16u : 8u));
+    return n <= 64 && units <= 2 * kCus && units * slabs <= (n <= 32 ? 12288u : 4096u);
+}
+
+// The same for launches that the tiles may split into shares of K side by side, where this kernel walks the shares one after the
+// other: ~0.3 us a slab up to 32 tokens, twice that above.  What the tiles' shares cost instead is a launch that adds them up, or,
+// with `deferrable`, the additions in the norm's kernel behind the projection: nothing at 512 rows, as much as the launch at 4096.
+// Shares side by side / here, us:
+//   plain, 9 tokens:        1024 x 1024 6.3 / 4.5, x 1792 7.5 / 6.5, x 2048 (8 shares, not 4) 6.7 / 7.1; 4096 x 2048 7.0 / 7.3
+//   plain, 24:              1024 x 1024 6.6 / 4.9, x 1792 8.0 / 6.8, x 2048 7.0 / 7.4; 3072 x 2048 7.6 / 7.5, 4096 x 2048 8.5 / 7.5
+//   plain, 40:              1024 x 1024 7.2 / 7.0, 4096 x 1024 8.2 / 7.1; 2048 x 2048 8.2 / 11.5
+//   with the norm, 24:      512 x 1024 8.0 / 7.9, x 2048 7.9 / 10.2; 1024 x 1024 8.1 / 7.8, x 1536 8.8 / 9.3; 2048 x 1152 9.9 / 9.4,
+//                           x 2048 9.8 / 11.2; 3072 x 1792 11.9 / 11.2, 4096 x 2048 13.3 / 12.5
+//   with the norm, 40:      1024 x 1024 8.5 / 10.2, 2048 x 1024 10.0 / 10.8, 3072 x 1024 11.3 / 11.6, 4096 x 1024 12.9 / 12.3
+bool few_applies_split(uint64_t rows, uint32_t n, uint32_t k, bool deferrable) {
+    const uint64_t units = (rows + GR - 1) / GR, slabs = k / (KB * 32), cost = n <= 32 ? 1u : 2u;
+    if (!few_applies(rows, n, k) || slabs * cost > (cost == 1 && units < 96 ? 15u : 16u)) return false;
+    return !deferrable || 12 * slabs * cost <= 72 + units;
 }
 
 uint32_t split_k_factor(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits) {
@@ -1349,16 +1363,20 @@ hipError_t cheapest_tile(Cost&& cost, Go&& go) {
     return m <= s_ ? go(TileM{}) : go(TileS{});
 }
 
+// in_launch: the launch walks its shares of K itself (gemm_split_in_launch).  The parity hook comes with the product launch's share
+// count and in_launch, runs its kernel, and walks K whole.
 template <bool DUMP>
-hipError_t launch(int type, GemmArgs& a, const Launch& L, uint32_t more = 0, bool defer_reduce = false) {
+hipError_t launch(int type, GemmArgs& a, const Launch& L, bool in_launch, uint32_t more = 0, bool defer_reduce = false) {
     if (a.m == 0 || a.n == 0) return hipSuccess;
     const auto tile_rows = [&](uint32_t rows) {  // row tiles of `rows` rows over the launch's weights
         uint64_t t = (a.m + (uint64_t)rows - 1) / rows;
         for (uint32_t i = 0; i < more; i++) t += (a.m_more[i] + (uint64_t)rows - 1) / rows;
         return t;
     };
-    const bool wide_split = !DUMP && more == 0 && a.ksplit > 1 && wide_split_factor(a.m, a.n, a.k, a.ksplit) == a.ksplit;
-    if (DUMP || (!wide_split && !narrow_tiles(tile_rows(BM), a.n))) a.ksplit = 1;  // only few-tile launches carry a split
+    uint32_t ksplit = a.ksplit > 1 ? a.ksplit : 1u;
+    const bool wide_split = more == 0 && ksplit > 1 && wide_split_factor(a.m, a.n, a.k, ksplit) == ksplit;
+    if (!wide_split && !narrow_tiles(tile_rows(BM), a.n)) ksplit = 1;  // only few-tile launches carry a split
+    a.ksplit = DUMP ? 1u : ksplit;
     const auto go = [&](auto kernel, uint32_t rows, uint32_t tokens, uint32_t threads, bool whole = false) {
         a.row_tiles = (a.m + rows - 1) / rows;
         a.tile_start[0] = a.tile_start[1] = UINT32_MAX;
@@ -1367,7 +1385,7 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, uint32_t more = 0, boo
             a.row_tiles += (a.m_more[i] + rows - 1) / rows;
         }
         a.tok_tiles = (a.n + tokens - 1) / tokens;
-        const uint32_t shares = a.ksplit > 1 ? a.ksplit : 1u;
+        const uint32_t shares = a.ksplit;
         if ((uint64_t)a.row_tiles * a.tok_tiles * shares > 0x7fffff00ull) return hipErrorInvalidValue;  // beyond a launch's grid
         // every XCD gets the same number of slots of the tile map; tile id = blockIdx.x / shares runs over all of them
         const uint32_t grid = (a.row_tiles * a.tok_tiles + 7u) / 8u * 8u * (whole ? 1u : shares);  // whole: a workgroup takes all shares of its rows
@@ -1383,7 +1401,8 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, uint32_t more = 0, boo
             if (q8) return go(gemm_tile_kernel<8, true, false, C>, C::kRows, C::kTokens, C::kThreads);
         return go(gemm_tile_kernel<2, DUMP, false, C>, C::kRows, C::kTokens, C::kThreads);
     };
-    const bool few = !L.gemm_mfma16 && few_applies(GR * tile_rows(GR), a.n, a.k, a.ksplit > 1), narrow = !wide_split && narrow_tiles(tile_rows(BM), a.n);
+    const bool few = !L.gemm_mfma16 && (ksplit > 1 ? in_launch : few_applies(GR * tile_rows(GR), a.n, a.k));
+    const bool narrow = !wide_split && narrow_tiles(tile_rows(BM), a.n);
     if (few) {
         // Eight waves and 151 KB of LDS while every CU gets one workgroup at most, else four and half of it.
         const auto waves = [&](auto tg, auto wv) {
@@ -1413,9 +1432,9 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, uint32_t more = 0, boo
         return go(gemm_mfma_kernel<2, DUMP>, BM, BN, THREADS);
     }
     if (wide_split) return tile(TileM{});
-    const uint64_t small = tile_rows(BM) * ((a.n + BN_NARROW - 1) / BN_NARROW) * (a.ksplit > 1 ? a.ksplit : 1u);
+    const uint64_t small = tile_rows(BM) * ((a.n + BN_NARROW - 1) / BN_NARROW) * ksplit;
     if (narrow && small <= kCus) return tile(TileN{});  // (1024 x 1024 over 555 tokens 10.9 us on TileS, 10.6 here; 512 tiles: 27 / 29.5)
-    if (a.n <= BN_NARROW || a.ksplit > 1) return tile(TileS{});
+    if (a.n <= BN_NARROW || ksplit > 1) return tile(TileS{});
     const auto cost = [&](auto cfg) { return tile_cost<decltype(cfg)>(tile_rows(decltype(cfg)::kRows), a.n, a.k); };
     return cheapest_tile(cost, tile);
 }
@@ -1423,7 +1442,9 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, uint32_t more = 0, boo
 }  // namespace
 
 uint32_t gemm_split_k(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits) { return split_k_factor(m, n, k, max_splits); }
-bool gemm_split_in_launch(uint32_t m, uint32_t n, uint32_t k, const Launch& L) { return !L.gemm_mfma16 && few_applies(m, n, k, true); }
+bool gemm_split_in_launch(uint32_t m, uint32_t n, uint32_t k, const Launch& L, bool deferrable) {
+    return !L.gemm_mfma16 && few_applies_split(m, n, k, deferrable);
+}
 
 // The GEMM's own copy of a weight (slabs, see StageT): its size, and the kernel that makes it from the raw blocks.
 size_t gemm_packed_bytes(uint32_t m, uint32_t k) { return (size_t)((m + 2 * GR - 1) / (2 * GR)) * 2 * ((k >> 5) / KB) * kSlab; }
@@ -1438,7 +1459,8 @@ hipError_t launch_gemm_pack(int type, const uint8_t* d_raw, uint32_t m, uint32_t
     return hipErrorInvalidValue;
 }
 
-// splits > 1 (= gemm_split_k(m, n, k, ...)) with d_partial holding splits * n * m floats: the K-split launch pair.
+// splits > 1 (= gemm_split_k(m, n, k, ...)): d_partial holds splits * n * m floats, or is null and the launch walks the shares itself
+// (only where gemm_split_in_launch says so).
 hipError_t launch_gemm_mfma(int type, const uint8_t* d_w, uint32_t m, uint32_t k, const int8_t* d_q,
                             const float* d_scales, uint32_t n, float* d_y, uint32_t y_stride, int y_layout,
                             int accumulate, const Launch& L, uint32_t splits, float* d_partial, bool defer_reduce) {
@@ -1447,14 +1469,14 @@ hipError_t launch_gemm_mfma(int type, const uint8_t* d_w, uint32_t m, uint32_t k
     a.m = m, a.n = n, a.k = k, a.y_stride = y_stride;
     a.y_row_major = (y_layout == 1);
     a.accumulate = accumulate;
-    const bool in_launch = gemm_split_in_launch(m, n, k, L);
-    if (splits > 1 && (d_partial || in_launch)) {
-        if (splits != split_k_factor(m, n, k, splits) || (defer_reduce && in_launch)) return hipErrorInvalidValue;  // the shape does not carry that split
+    const bool in_launch = splits > 1 && !d_partial;
+    if (splits > 1) {
+        if (splits != split_k_factor(m, n, k, splits) || (in_launch && !gemm_split_in_launch(m, n, k, L, false)))
+            return hipErrorInvalidValue;  // the shape does not carry that split
         a.ksplit = splits, a.partial = d_partial;
-    } else if (defer_reduce) {
-        return hipErrorInvalidValue;  // nothing to defer on an unsplit launch
     }
-    return launch<false>(type, a, L, 0, defer_reduce);
+    if (defer_reduce && (splits <= 1 || in_launch)) return hipErrorInvalidValue;  // nothing to defer
+    return launch<false>(type, a, L, in_launch, 0, defer_reduce);
 }
 
 // The same launch over up to three weights of one type and k that share the activations: outputs y[i] (same stride,
@@ -1469,7 +1491,7 @@ hipError_t launch_gemm_mfma_multi(int type, const uint8_t* const* d_w, const uin
     a.y_row_major = (y_layout == 1);
     a.accumulate = accumulate;
     for (uint32_t i = 1; i < count; i++) a.w_more[i - 1] = d_w[i], a.y_more[i - 1] = d_y[i], a.m_more[i - 1] = m[i];
-    return launch<false>(type, a, L, count - 1);
+    return launch<false>(type, a, L, false, count - 1);
 }
 
 // Gate and up projection of a feed-forward block over n tokens in one launch whose epilogue applies the SiLU gate and
@@ -1504,11 +1526,12 @@ hipError_t launch_gemm_mfma_gated(int /*type: the copies are the same for both*/
 // Parity hook through the matrix-core path: the same loads, unpack, LDS layout and
 // MFMA as the GEMM, writing the raw i32 block dots instead of scaling them.
 hipError_t launch_block_dots_mfma(int type, const uint8_t* d_w, uint32_t m, uint32_t k, const int8_t* d_q, uint32_t n,
-                                  int32_t* d_out, const Launch& L) {
+                                  int32_t* d_out, uint32_t max_splits, const Launch& L) {
     GemmArgs a{};
     a.w = d_w, a.xq = d_q, a.xs = nullptr, a.y = nullptr, a.dots = d_out;
     a.m = m, a.n = n, a.k = k, a.y_stride = 0;
-    return launch<true>(type, a, L);
+    a.ksplit = split_k_factor(m, n, k, max_splits);
+    return launch<true>(type, a, L, gemm_split_in_launch(m, n, k, L, false));
 }
 
 }  // namespace wick_rocm

@@ -153,8 +153,9 @@ hipError_t launch_gemm_mfma(int type, const uint8_t* d_w, uint32_t m, uint32_t k
 // up in ascending order onto y itself (launch_residual_rmsnorm_quantize).
 // Ways (1, 2, 4 or 8, at most max_splits) the launch above may be split over K: > 1 only for launches of few tiles and long K.
 uint32_t gemm_split_k(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits);
-// Whether the launch, on the block loop that L asks for, adds its shares up itself (few tokens): no scratch, nothing to defer.
-bool gemm_split_in_launch(uint32_t m, uint32_t n, uint32_t k, const Launch& L);
+// Whether the launch, on the block loop that L asks for, should walk its shares itself (few tokens): no scratch, nothing to defer.
+// deferrable: the caller's next kernel would add the shares up.  (With deferrable: a part of what there is without.)
+bool gemm_split_in_launch(uint32_t m, uint32_t n, uint32_t k, const Launch& L, bool deferrable);
 hipError_t launch_gemm_mfma_multi(int type, const uint8_t* const* d_w, const uint32_t* m, uint32_t count, uint32_t k, const int8_t* d_q,
                                   const float* d_scales, uint32_t n, float* const* d_y, uint32_t y_stride, int y_layout, int accumulate,
                                   const Launch& L);
@@ -171,7 +172,7 @@ hipError_t launch_block_dots_gemv(int type, const uint8_t* d_w, uint32_t m, uint
 hipError_t launch_block_dots_gemv_f32(int type, const uint8_t* d_w, uint32_t m, uint32_t k, const float* d_x, int32_t* d_out, int num_cus,
                                       const Launch& L);
 hipError_t launch_block_dots_mfma(int type, const uint8_t* d_w, uint32_t m, uint32_t k, const int8_t* d_q, uint32_t n,
-                                  int32_t* d_out, const Launch& L);
+                                  int32_t* d_out, uint32_t max_splits, const Launch& L);
 
 // The non-matmul operations of an LFM2 decode step (lfm2_ops.hip).  d_pos / d_token, when non-null, are read on the
 // device in place of the by-value pos / token.
