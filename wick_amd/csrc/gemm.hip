@@ -7,9 +7,10 @@
 // blocks: every MFMA covers exactly one block (K = 32) and its i32 result is scaled
 // into f32 accumulators on the vector ALU.
 //
-// Two families of block loops:
-//   * gemm_tile_kernel, v_mfma_i32_32x32x32_i8: every launch of more than 48 tokens, on one of three tiles (see T32 and TileL / M / S);
-//   * gemm_narrow_kernel, v_mfma_i32_16x16x32_i8, 128 rows x 64 tokens: launches of up to 48 tokens, which skip the 16-token
+// Three families of block loops:
+//   * gemm_tile_kernel, v_mfma_i32_32x32x32_i8: prompts, on one of four tiles (see T32 and TileL / M / S / N);
+//   * gemm_few_kernel, the same instruction, 32 rows x all of up to 64 tokens: where latency is what a launch costs (few_applies);
+//   * gemm_narrow_kernel, v_mfma_i32_16x16x32_i8, 128 rows x 64 tokens: the other launches of up to 48 tokens, which skip the 16-token
 //     columns they do not have; gemm_mfma_kernel, the same shape on 128 x 128, on request (wick_rocm_set_gemm_mfma_shape).
 // The kernels are bound by the two scaling FMAs per result plus the matrix instructions, which a SIMD overlaps only in part, and by
 // feeding both from LDS.  A wave issues a vector-ALU instruction only every ~4.7 cycles while a SIMD retires one every ~2.3, so two
