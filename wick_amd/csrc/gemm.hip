@@ -634,9 +634,13 @@ __global__ __launch_bounds__(THREADS, 4) void gemm_mfma_kernel(GemmArgs a) {
 typedef int v16i __attribute__((ext_vector_type(16)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 
-template <int RT_, int TT_, int WR_, int WT_, int SB_, int OCC_ = 2>
+// WAVES: per SIMD, what the registers have to leave room for.  SCALE_FIRST: a result's 16 FMAs with the row scale go out ahead of its 16
+// with the token scales, in the result's registers, so that no FMA waits for the one before it: with two waves per SIMD the register-only
+// block loop runs at 1.52 instead of 1.32 POP/s (1.60 either way with four); smaller tiles have not the registers for it.
+template <int RT_, int TT_, int WR_, int WT_, int SB_, int WAVES, bool SCALE_FIRST = false>
 struct T32 {
-    static constexpr int RT = RT_, TT = TT_, WR = WR_, WT = WT_, SB = SB_, kOcc = OCC_;
+    static constexpr int RT = RT_, TT = TT_, WR = WR_, WT = WT_, SB = SB_, kOcc = WAVES;
+    static constexpr bool kScaleFirst = SCALE_FIRST;
     static constexpr int kWaves = WR * WT, kThreads = 64 * kWaves;
     static constexpr int kGranules = WR * RT, kRows = GR * kGranules, kTokens = 32 * WT * TT;
     static constexpr int kTiles = RT * TT;  // 32 x 32 results per wave and block
@@ -851,11 +855,21 @@ __global__ __launch_bounds__(C::kThreads, C::kOcc) void gemm_tile_kernel(GemmArg
                 if constexpr (fetch) read_ab(Idx<next ? b + 1 : 0>{});
                 constexpr int kFetched = fetch ? TT + RT : 0;  // reads that a wait below may leave outstanding on top
                 if constexpr (rt == RT - 1 && tt == 0) lds_arrived<kFetched + (TT == 1 && RT > 1 && next ? 1 : 0)>(dw[rt]);
+                if constexpr (!DUMP && C::kScaleFirst) {
+                    static_assert(RT > 1, "the granules' scale pairs come ahead of the token scales");
+                    if constexpr (rt == 0 && tt == 0) {
+                        lds_arrived<5 + kFetched>(dw[0]);  // (behind them: the token scales and the last granule's pair)
+                        static_for<RT - 1>([&](auto i) { tie(dw[decltype(i)::value]); });
+                    }
+#pragma unroll
+                    for (int e = 0; e < 16; e++) D[t & 1][e] = __float_as_int(__builtin_fmaf(__int_as_float(D[t & 1][e]), dw[rt].x, dw[rt].y));
+                    __builtin_amdgcn_sched_barrier(0);
+                }
                 static_for<4>([&](auto g_) {
                     constexpr int g = decltype(g_)::value;
                     if constexpr (rt == 0) {
                         lds_arrived<(tt == 0 ? 4 : 3) - g + kFetched>(dx[g]);
-                        if constexpr (g == 0 && tt == 0) static_for<RT - 1>([&](auto i) { tie(dw[decltype(i)::value]); });
+                        if constexpr (!(!DUMP && C::kScaleFirst) && g == 0 && tt == 0) static_for<RT - 1>([&](auto i) { tie(dw[decltype(i)::value]); });
                     }
                     if constexpr (DUMP) {
                         const uint32_t row = row0 + GR * (RT * wr + rt) + l32, tok = tok0 + 32 * (TT * wt + tt) + 4 * kh + 8 * g;
@@ -870,11 +884,12 @@ __global__ __launch_bounds__(C::kThreads, C::kOcc) void gemm_tile_kernel(GemmArg
                     } else {
 #pragma unroll
                         for (int r = 0; r < 4; r++) {
-                            const float v = __builtin_fmaf(__int_as_float(D[t & 1][4 * g + r]), dw[rt].x, dw[rt].y);
+                            float v = __int_as_float(D[t & 1][4 * g + r]);
+                            if constexpr (!C::kScaleFirst) v = __builtin_fmaf(v, dw[rt].x, dw[rt].y);
                             acc[rt][tt][4 * g + r] = __builtin_fmaf(v, dx[g][r ^ 1], acc[rt][tt][4 * g + r]);
                         }
                         // (without this the compiler lets the MFMAs of all tiles run ahead of their FMAs, and spills)
-                        tie(acc[rt][tt]);
+                        if constexpr (!C::kScaleFirst || g == 3) tie(acc[rt][tt]);
                     }
                     // this group's token scales are done with: the next token group's, or the next block's first
                     if constexpr (rt == RT - 1) {
@@ -1338,30 +1353,59 @@ hipError_t launch_reduce(const GemmArgs& a, const Launch& L) {
     return hipErrorInvalidValue;  // split_k_factor makes 2, 4 or 8 shares
 }
 
-// The three tiles of a prompt (rows x tokens) and when each is taken.  A CU works through its share of the launch's tiles two
-// workgroups at a time, so a launch takes about ceil(tiles / 256) x (what a tile costs the CU): per 256 x 128 results and 2048
-// elements of K 34 / 40 / 46 us on the large / medium / small tile -- the larger a wave's tile, the fewer operand bytes per FMA --
-// plus 5 / 1.4 / 3 us for filling, draining and storing it, and a third more when the CU has only one workgroup.  Measured (large /
-// medium / small, us): 6912 x 2048 over 2002 tokens 82 / 85 / 95, 13824 x 2048 over 4096 266 / 285 / 317, 9216 x 1024 over 2048
-// 69 / 57 / 59, 2048 x 2048 over 2002 53 / 29 / 27, 1024 x 4608 over 2048 109 / 50 / 38.  With the gate in the epilogue the fixed part
-// is 6 / 6.3 / 5 us: 2 x 4608 x 1024 over 2048 tokens 76 / 69 / 68, over 555 35 / 28 / 26, 2 x 6912 x 2048 over 2002 159 / 164 / 169.
-using TileL = T32<4, 2, 2, 2, 2>;     // 256 x 128, 4 waves of 128 x 64
-using TileM = T32<2, 1, 2, 4, 4, 4>;  // 128 x 128, 8 waves of 64 x 32
-using TileS = T32<2, 1, 2, 2, 4>;     // 128 x 64, 4 waves of 64 x 32
-using TileN = T32<1, 1, 4, 2, 4, 4>;  // 128 x 64, 8 waves of 32 x 32: where a CU gets one workgroup at most, its waves are all there is
+// The tiles of a launch over a prompt, and what each costs: us per slab (128 elements of K) of a share with 1 .. kPerCu workgroups on a CU, and us
+// per workgroup for filling, draining and storing it -- plain launches first, those with the gate in the epilogue second (0: not
+// built).  Fitted to 130 launches (3072, 2048, 1024 x 1024, 1024 x 4608, 6144, 3072, 2048 x 2048, 2048 x 6912 and gate | up 4608 x 1024,
+// 6912 x 2048, each over 80 .. 2048 tokens, weights and activations of random bits: a launch that keeps the chip busy runs at the
+// power limit), which they meet to 4 % rms; the tile they choose is 1 % behind the best of all.  A launch is workgroups on 256 CUs, kPerCu
+// at a time, and what the last round leaves idle is what separates the tiles: large ones do more per operand byte, small ones leave
+// less over, and a CU with a single workgroup on it wants that one's waves to be many.
+struct TileCost {
+    float slab[4], fixed;
+};
+struct TileL : T32<4, 2, 2, 2, 2, 2, true> {  // 256 x 128, 4 waves of 128 x 64
+    static constexpr int kPerCu = 2;
+    static constexpr TileCost kCost[2] = {{{3.07f, 3.81f}, 5.15f}, {{3.14f, 3.88f}, 4.76f}};
+};
+struct TileX : T32<2, 2, 2, 2, 2, 3> {  // 128 x 128, 4 waves of 64 x 64
+    static constexpr int kPerCu = 3;
+    static constexpr TileCost kCost[2] = {{{1.79f, 2.31f, 3.30f}, 1.50f}, {{1.47f, 2.25f, 3.32f}, 2.30f}};
+};
+struct TileS : T32<2, 1, 2, 2, 4, 2> {  // 128 x 64, 4 waves of 64 x 32
+    static constexpr int kPerCu = 2;
+    static constexpr TileCost kCost[2] = {{{0.94f, 1.30f}, 1.22f}, {{0.89f, 1.31f}, 1.70f}};
+};
+struct TileQ : T32<2, 1, 2, 2, 2, 4> {  // the same with half a slab per stage: four of them on a CU
+    static constexpr int kPerCu = 4;
+    static constexpr TileCost kCost[2] = {{{1.29f, 1.62f, 1.97f, 2.47f}, 1.41f}, {{1.14f, 1.66f, 1.95f, 2.53f}, 1.13f}};
+};
+struct TileN : T32<1, 1, 4, 2, 4, 4> {  // 128 x 64, 8 waves of 32 x 32
+    static constexpr int kPerCu = 2;
+    static constexpr TileCost kCost[2] = {{{0.80f, 1.31f}, 1.37f}, {}};
+};
+struct TileH : T32<1, 1, 2, 2, 4, 4> {  // 64 x 64, 4 waves of 32 x 32
+    static constexpr int kPerCu = 4;
+    static constexpr TileCost kCost[2] = {{{0.68f, 0.82f, 1.10f, 1.42f}, 0.64f}, {}};
+};
 template <typename C>
-float tile_cost(uint64_t row_tiles, uint32_t n, uint32_t k, bool gated = false) {
-    const uint64_t tiles = row_tiles * ((n + C::kTokens - 1) / C::kTokens), rounds = (tiles + kCus - 1) / kCus;
-    const float per_k = C::kRows == 256 ? 34.0f : (C::kTokens == 128 ? 40.0f : 46.0f);
-    const float fixed = C::kRows == 256 ? (gated ? 6.0f : 5.0f) : (C::kTokens == 128 ? (gated ? 6.3f : 1.4f) : (gated ? 5.0f : 3.0f));
-    return (float)rounds * (rounds == 1 ? 1.35f : 1.0f) * ((float)(C::kRows * C::kTokens) / (256.0f * 128.0f)) * (per_k * (float)k / 2048.0f + fixed);
+float tile_cost(uint64_t row_tiles, uint32_t n, uint32_t k, uint32_t shares, bool gated = false) {
+    const uint64_t tiles = row_tiles * ((n + C::kTokens - 1) / C::kTokens) * shares, per_cu = (tiles + kCus - 1) / kCus;
+    const TileCost& c = C::kCost[gated];
+    const uint32_t rest = (uint32_t)(per_cu % C::kPerCu);
+    const float per_slab = (float)(per_cu / C::kPerCu) * c.slab[C::kPerCu - 1] + (rest ? c.slab[rest - 1] : 0.0f);
+    return per_slab * (float)k / (float)(KB * 32 * shares) + (float)per_cu * c.fixed;
 }
-
-template <typename Cost, typename Go>
+// go(tile) for the one of them that cost(tile) is lowest for.
+template <typename... Tiles, typename Cost, typename Go>
 hipError_t cheapest_tile(Cost&& cost, Go&& go) {
-    const float l = cost(TileL{}), m = cost(TileM{}), s_ = cost(TileS{});
-    if (l <= m && l <= s_) return go(TileL{});
-    return m <= s_ ? go(TileM{}) : go(TileS{});
+    const float costs[] = {cost(Tiles{})...};
+    uint32_t best = 0;
+    for (uint32_t i = 1; i < sizeof...(Tiles); i++)
+        if (costs[i] < costs[best]) best = i;
+    hipError_t e = hipErrorInvalidValue;
+    uint32_t i = 0;
+    (void)((i++ == best ? (e = go(Tiles{}), true) : false) || ...);
+    return e;
 }
 
 // in_launch: the launch walks its shares of K itself (gemm_split_in_launch).  The parity hook comes with the product launch's share
@@ -1432,12 +1476,8 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, bool in_launch, uint32
             if (q8) return go(gemm_mfma_kernel<8, true>, BM, BN, THREADS);
         return go(gemm_mfma_kernel<2, DUMP>, BM, BN, THREADS);
     }
-    if (wide_split) return tile(TileM{});
-    const uint64_t small = tile_rows(BM) * ((a.n + BN_NARROW - 1) / BN_NARROW) * ksplit;
-    if (narrow && small <= kCus) return tile(TileN{});  // (1024 x 1024 over 555 tokens 10.9 us on TileS, 10.6 here; 512 tiles: 27 / 29.5)
-    if (a.n <= BN_NARROW || ksplit > 1) return tile(TileS{});
-    const auto cost = [&](auto cfg) { return tile_cost<decltype(cfg)>(tile_rows(decltype(cfg)::kRows), a.n, a.k); };
-    return cheapest_tile(cost, tile);
+    const auto cost = [&](auto cfg) { return tile_cost<decltype(cfg)>(tile_rows(decltype(cfg)::kRows), a.n, a.k, ksplit); };
+    return cheapest_tile<TileL, TileX, TileS, TileQ, TileN, TileH>(cost, tile);
 }
 
 }  // namespace
@@ -1519,9 +1559,9 @@ hipError_t launch_gemm_mfma_gated(int /*type: the copies are the same for both*/
     };
     const auto cost = [&](auto cfg) {
         using C = decltype(cfg);
-        return tile_cost<C>((m + C::kRows / 2 - 1) / (C::kRows / 2), n, k, true);
+        return tile_cost<C>((m + C::kRows / 2 - 1) / (C::kRows / 2), n, k, 1, true);
     };
-    return cheapest_tile(cost, tile);
+    return cheapest_tile<TileL, TileX, TileS, TileQ>(cost, tile);
 }
 
 // Parity hook through the matrix-core path: the same loads, unpack, LDS layout and
