@@ -174,6 +174,27 @@ def test_shortconv_of_a_prompt(ctx, ops, oracle, hidden, kernel, n, start):
         b.free()
 
 
+@pytest.mark.parametrize("hidden,n", [(32, 1), (32, 2), (96, 3), (64, 4), (1056, 33), (1024, 1023), (1024, 1024), (1024, 1025), (2048, 513), (2048, 514)])
+def test_shortconv_of_a_prompt_writes_the_state_in_its_own_launch(ctx, ops, oracle, hidden, n):
+    """Kernel size 3: a thread takes two tokens, or four from 262144 (token, four channels) pairs on, and the threads of the first tokens
+    write the new state.  == the float form + the Q8_0 quantizer, whose state a launch of its own writes, bit for bit; twice in a row,
+    so that the second call starts from a state that the first one left."""
+    w, state = oracle.fill_normal(3, 0.5, hidden * 3), oracle.fill_normal(4, 1.0, 2 * hidden)
+    d_w, d_buf, d_ref = ctx.to_device(w), ctx.to_device(state), ctx.to_device(state)
+    d_out, d_q, d_s = ctx.alloc(n * hidden * 4), ctx.alloc(n * hidden), ctx.alloc(n * (hidden // 32) * 4)
+    for seed in (5, 6):
+        d_projs = ctx.to_device(oracle.fill_normal(seed, 1.0, n * 3 * hidden))
+        ops.encode_conv1d_seq_quantize(d_projs, d_buf, d_w, d_q, d_s, hidden, 3, n)
+        q, s = d_q.download(np.int8, n * hidden), d_s.download(np.float32, n * (hidden // 32))
+        ops.encode_conv1d_seq(d_projs, d_ref, d_w, d_out, hidden, 3, n)
+        ctx.quantize_q8_0(d_out, n, hidden, hidden, d_q, d_s)
+        assert np.array_equal(q, d_q.download(np.int8, n * hidden)) and np.array_equal(bits(s), bits(d_s.download(np.float32, n * (hidden // 32))))
+        assert np.array_equal(bits(d_buf.download(np.float32, 2 * hidden)), bits(d_ref.download(np.float32, 2 * hidden)))
+        d_projs.free()
+    for b in (d_w, d_buf, d_ref, d_out, d_q, d_s):
+        b.free()
+
+
 @pytest.mark.parametrize("n_heads,n_kv,hd,pos", [(4, 2, 64, 0), (16, 8, 64, 5), (8, 8, 32, 300), (4, 1, 128, 4095), (2, 2, 256, 17)])
 def test_qk_norm_rope_and_append(ctx, ops, oracle, n_heads, n_kv, hd, pos):
     max_seq, eps, base = 4096, 1e-5, 1_000_000.0

@@ -1314,17 +1314,87 @@ __global__ __launch_bounds__(256) void shortconv_seq_kernel(const float* __restr
     out[(size_t)j * hidden + ch] = __fmul_rn(p[hidden + ch], sum);
 }
 
-// shortconv_seq_kernel followed by the Q8_0 quantizer, bit for bit: a thread takes four consecutive channels of one
-// token (16-byte loads), eight threads one 32-channel block, and the gated convolution goes straight into Q8_0 blocks
-// for the out projection -- the f32 result never touches memory.  hidden % 32 == 0, 16-byte aligned buffers.
-// KS: the kernel size when known at compile time (3, the reference's default: the taps unroll and all of a thread's loads are
-// issued together), 0: read from kernel_size.
-template <int KS>
+// shortconv_seq_kernel followed by the Q8_0 quantizer, bit for bit: a thread takes four consecutive channels (16-byte loads) of T
+// consecutive tokens, eight threads one 32-channel block, and the gated convolution goes straight into Q8_0 blocks for the out
+// projection -- the f32 result never touches memory.  Kernel size 3; hidden % 32 == 0, 16-byte aligned buffers.
+// Bound by its loads: all of a thread's are issued together, and a token's gated input b*x serves the T taps it takes part in from one load
+// (a thread per token fetched it three times over).  The old state is read by the threads of the first tokens alone (T >= 2), so they write
+// the new one too, b*x of the last two tokens: no launch of its own behind this one.
+// Before, with that launch, and now, us (kernel trace): 23 tokens x 1024 channels 3.0 + 2.2 / 3.1, 555 5.1 + 4.4 / 5.1, 2002 x 2048 17.8 + 4.9 / 12.1.
+typedef float f4_dword_aligned __attribute__((ext_vector_type(4), aligned(4)));
+template <int T>
+__global__ __launch_bounds__(256) void shortconv3_seq_quantize_kernel(const float* __restrict__ proj, float* __restrict__ buffer,
+                                                                      const float* __restrict__ conv_w, int8_t* __restrict__ q,
+                                                                      float* __restrict__ scales, uint32_t hidden, uint32_t n, uint32_t total_threads) {
+    static_assert(T >= 2, "the tokens that see the old state are one thread's");
+    const uint32_t t = blockIdx.x * 256u + threadIdx.x, qpr = hidden >> 2;
+    const bool live = t < total_threads;
+    const uint32_t j0 = live ? t / qpr * T : 0u, c0 = 4u * (live ? t % qpr : 0u);
+    const size_t row = (size_t)3 * hidden;
+    const float* const base = proj + c0;
+    const auto at = [&](uint32_t token, uint32_t part) { return *reinterpret_cast<const float4*>(base + token * row + part * hidden); };
+    const auto clamped = [&](uint32_t token) { return token < n ? token : n - 1u; };
+    float4 b[T + 2], x[T + 2], c[T];  // of tokens j0 - 2 ..; at the start of the prompt the first two are the old state's slots (x unused)
+    if (j0 == 0) {
+        b[0] = *reinterpret_cast<const float4*>(buffer + c0), b[1] = *reinterpret_cast<const float4*>(buffer + hidden + c0);
+        x[0] = x[1] = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
+    } else {
+        b[0] = at(j0 - 2u, 0), x[0] = at(j0 - 2u, 2), b[1] = at(j0 - 1u, 0), x[1] = at(j0 - 1u, 2);
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < (uint32_t)T; i++) {
+        const uint32_t token = clamped(j0 + i);
+        b[i + 2] = at(token, 0), x[i + 2] = at(token, 2), c[i] = at(token, 1);
+    }
+    float w[12];  // [channel][tap]
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        const f4_dword_aligned v = *reinterpret_cast<const f4_dword_aligned*>(conv_w + (size_t)c0 * 3u + 4 * i);
+        w[4 * i] = v.x, w[4 * i + 1] = v.y, w[4 * i + 2] = v.z, w[4 * i + 3] = v.w;
+    }
+    float bx[T + 2][4];  // (an old slot times one is the slot, to the bit)
+#pragma unroll
+    for (int i = 0; i < T + 2; i++) {
+        bx[i][0] = __fmul_rn(b[i].x, x[i].x), bx[i][1] = __fmul_rn(b[i].y, x[i].y);
+        bx[i][2] = __fmul_rn(b[i].z, x[i].z), bx[i][3] = __fmul_rn(b[i].w, x[i].w);
+    }
+    if (live && j0 == 0) {  // the new state: b*x of tokens n - 2 and n - 1, or the old second slot and b*x of the only one
+        const uint32_t last = n - 1u;
+        const float4 lb = at(last, 0), lx = at(last, 2);
+        float4 s0 = make_float4(bx[1][0], bx[1][1], bx[1][2], bx[1][3]);
+        if (n > 1u) {
+            const float4 pb = at(last - 1u, 0), px = at(last - 1u, 2);
+            s0 = make_float4(__fmul_rn(pb.x, px.x), __fmul_rn(pb.y, px.y), __fmul_rn(pb.z, px.z), __fmul_rn(pb.w, px.w));
+        }
+        *reinterpret_cast<float4*>(buffer + c0) = s0;
+        *reinterpret_cast<float4*>(buffer + hidden + c0) = make_float4(__fmul_rn(lb.x, lx.x), __fmul_rn(lb.y, lx.y), __fmul_rn(lb.z, lx.z), __fmul_rn(lb.w, lx.w));
+    }
+#pragma unroll
+    for (int i = 0; i < T; i++) {
+        const float cc[4] = {c[i].x, c[i].y, c[i].z, c[i].w};
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            float sum = __fadd_rn(0.0f, __fmul_rn(bx[i][e], w[3 * e]));  // (0 + -0 is +0, as the loop over the taps has it)
+            sum = __fadd_rn(sum, __fmul_rn(bx[i + 1][e], w[3 * e + 1]));
+            v[e] = __fmul_rn(cc[e], __fadd_rn(sum, __fmul_rn(bx[i + 2][e], w[3 * e + 2])));
+        }
+        const float amax = group_max8(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+        float id;
+        const float scale = q8_scale_and_inverse(amax, id);
+        const uint32_t packed = q8_pack4(v[0], v[1], v[2], v[3], id), token = j0 + i;
+        if (live && token < n) {
+            *reinterpret_cast<uint32_t*>(q + (size_t)token * hidden + c0) = packed;
+            if ((c0 & 31u) == 0) scales[(size_t)token * (hidden >> 5) + (c0 >> 5)] = scale;
+        }
+    }
+}
+
+// The same for any kernel size, a token per thread; the state is left to shortconv_state_kernel.
 __global__ __launch_bounds__(256) void shortconv_seq_quantize_kernel(const float* __restrict__ proj, const float* __restrict__ buffer,
                                                                      const float* __restrict__ conv_w, int8_t* __restrict__ q,
-                                                                     float* __restrict__ scales, uint32_t hidden, uint32_t kernel_size_arg,
+                                                                     float* __restrict__ scales, uint32_t hidden, uint32_t kernel_size,
                                                                      uint64_t total_quads) {
-    const uint32_t kernel_size = KS ? (uint32_t)KS : kernel_size_arg;
     const uint64_t t = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const bool live = t < total_quads;
     const uint64_t tt = live ? t : 0;
@@ -1836,17 +1906,26 @@ bool shortconv_seq_quantize_applies(const float* d_proj, const float* d_buffer, 
     return hidden % 32u == 0 && ((uintptr_t)d_proj | (uintptr_t)d_buffer) % 16u == 0;
 }
 
+constexpr uint64_t kShortconvFour = 256u * 1024u;  // (token, four channels) pairs from which a thread takes four tokens
+
 // The convolution of n tokens written as Q8_0 blocks ([n][hidden] quants, [n][hidden / 32] scales), then the state.
 hipError_t launch_shortconv_seq_quantize(const float* d_proj, float* d_buffer, const float* d_conv_w, int8_t* d_q, float* d_scales, uint32_t hidden,
                                          uint32_t kernel_size, uint32_t n, const Launch& L) {
     if (n == 0) return hipSuccess;
     if (!shortconv_seq_quantize_applies(d_proj, d_buffer, hidden)) return hipErrorInvalidValue;
     const uint64_t total = (uint64_t)n * (hidden >> 2);
-    const auto go = [&](auto kernel) {
-        return launch_kernel(L, kFamQuantize, kernel, dim3((uint32_t)((total + 255) / 256)), dim3(256), d_proj, static_cast<const float*>(d_buffer),
-                             d_conv_w, d_q, d_scales, hidden, kernel_size, total);
-    };
-    hipError_t e = kernel_size == 3 ? go(shortconv_seq_quantize_kernel<3>) : go(shortconv_seq_quantize_kernel<0>);
+    if (kernel_size == 3) {
+        // two tokens per thread while that leaves the chip work to do, then four
+        const auto go = [&](auto kernel, uint32_t tokens) {
+            const uint64_t threads = (uint64_t)((n + tokens - 1u) / tokens) * (hidden >> 2);
+            if (threads > 0xffffff00ull) return hipErrorInvalidValue;
+            return launch_kernel(L, kFamQuantize, kernel, dim3((uint32_t)((threads + 255) / 256)), dim3(256), d_proj, d_buffer, d_conv_w, d_q, d_scales,
+                                 hidden, n, (uint32_t)threads);
+        };
+        return total < kShortconvFour ? go(shortconv3_seq_quantize_kernel<2>, 2) : go(shortconv3_seq_quantize_kernel<4>, 4);
+    }
+    hipError_t e = launch_kernel(L, kFamQuantize, shortconv_seq_quantize_kernel, dim3((uint32_t)((total + 255) / 256)), dim3(256), d_proj,
+                                 static_cast<const float*>(d_buffer), d_conv_w, d_q, d_scales, hidden, kernel_size, total);
     if (e != hipSuccess || kernel_size < 2) return e;
     return launch_kernel(L, kFamOther, shortconv_state_kernel, dim3((hidden + 255u) / 256u), dim3(256), d_proj, d_buffer, hidden, kernel_size, n);
 }
