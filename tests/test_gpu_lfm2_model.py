@@ -502,3 +502,24 @@ def test_greedy_run_across_the_change_of_step_graphs(ctx, oracle, tmp_path):
         picks.append(model.generate_greedy(7, 1018, 12))
     assert np.array_equal(picks[0], picks[2]) and np.array_equal(picks[1], picks[2])
     model.free()
+
+
+@pytest.mark.parametrize("wtype", [W.Q4_0, W.Q8_0])
+def test_a_prompt_is_the_same_on_either_block_loop(ctx, oracle, tmp_path, wtype):
+    """Prompts on both sides of the token counts at which a pass takes other launches (gate | up with the gate in its epilogue, one granule
+    per workgroup or on tiles; K shares side by side, on one granule per workgroup, 64-row or 128-row tiles): logits and state are bit for
+    bit those of the 16x16x32 kernels, which take the separate launches throughout."""
+    model, _, _ = load(ctx, oracle, tmp_path, context=320, n_layers=2, hidden=512, inter=2304, n_heads=8, kv_heads=(0, 2), vocab=256, wtype=wtype, embd_type=W.Q8_0)
+    tokens = np.random.default_rng(3).integers(0, 256, 300).astype(np.uint32)
+    try:
+        for n in (9, 16, 17, 32, 33, 48, 49, 64, 65, 129, 300):
+            got = []
+            for shape in (32, 16):
+                ctx.set_gemm_mfma_shape(shape)
+                model.reset()
+                got.append((model.forward_prefill(tokens[:n], 0), model.snapshot_state(n)))
+            assert np.array_equal(got[0][0].view(np.uint32), got[1][0].view(np.uint32)), f"{n} tokens: logits"
+            assert np.array_equal(got[0][1], got[1][1]), f"{n} tokens: state"
+    finally:
+        ctx.set_gemm_mfma_shape(32)
+        model.free()

@@ -54,6 +54,8 @@
 //     12582912*dw is exact because dw has an 11-bit significand);
 //     acc = fma(t, dx, acc), both plain v_fma_f32 (v_fma_mix_f32 with an f16 scale
 //     operand would save registers but issues at half the rate).
+#include <algorithm>
+
 #include "wick_rocm_device.h"
 #include "wick_rocm_internal.h"
 
@@ -1147,32 +1149,43 @@ __global__ __launch_bounds__(THREADS, 4) void gemm_narrow_kernel(GemmArgs a) {
 // the same order as elsewhere, in the same workgroup: no scratch and no second launch.
 // Measured back to back, 23 tokens: 1024 x 1024 split in 4 6.7 -> 4.9 us, 2048 x 1024 (Q | K | V) 8.8 -> 4.9, 9216 x 1024 (gate | up)
 // 9.1 -> 6.5.
-template <int TYPE, bool DUMP, int TG, int WV>
+//
+// GATED: gate | up over few tokens with the SiLU gate and the down projection's quantizer behind it.  A workgroup takes a granule of gate
+// rows and the same one of up, half of the waves each; a granule is one Q8_0 block of every token, so the gated values are exchanged
+// through LDS and leave as blocks, element for element what the two projections and silu_mul_quantize_kernel compute.
+template <int TYPE, bool DUMP, bool GATED, int TG, int WV>
 __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(GemmArgs a) {
-    constexpr int SL = WV / TG, NB = SL * KB;              // slabs and blocks of a round
-    constexpr int EP = 16 * TG / WV, TPR = 32 * TG / EP;   // elements (consecutive tokens of a row) per thread, threads per row
+    static_assert(!(GATED && DUMP), "the parity hook runs the plain launch");
+    constexpr int MS = GATED ? 2 : 1;                      // weights
+    constexpr int SL = WV / TG / MS, NB = SL * KB;         // slabs and blocks of a round
+    constexpr int EP = 16 * TG / WV, TPR = 32 * TG / EP;   // elements (consecutive tokens of a row) per thread and weight, threads per row
     constexpr int kRow = 36;                               // floats of a row of 32 tokens: 16-byte aligned, rows spread over the banks
-    __shared__ __align__(16) float vs[NB * TG][GR][kRow];
+    __shared__ __align__(16) float vs[MS][NB * TG][GR][kRow];
     __shared__ __align__(16) float dxs[NB][32 * TG];
-    const uint32_t shares = DUMP || a.ksplit < 2 ? 1u : a.ksplit;
-    if (blockIdx.x >= a.row_tiles) return;  // (grids are rounded up)
-    uint32_t granule = blockIdx.x;  // within the launch's weights
-    select_weight(a, granule);
+    // shares of K: side by side, a workgroup each, into a.partial; or (no partial) one after the other in this one
+    const uint32_t ksplit = DUMP || GATED || a.ksplit < 2 ? 1u : a.ksplit;
+    const bool side = ksplit > 1 && a.partial;
+    const uint32_t shares = side ? 1u : ksplit, my_share = side ? blockIdx.x % ksplit : 0u;
+    uint32_t granule = side ? blockIdx.x / ksplit : blockIdx.x;  // within the launch's weights
+    if (granule >= a.row_tiles) return;                          // (grids are rounded up)
+    if constexpr (!GATED) select_weight(a, granule);
     const uint32_t lane = threadIdx.x & 63u, l32 = lane & 31u, kh = lane >> 5;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const uint32_t sl = wave / TG, tg = wave % TG;
-    const uint32_t nb = a.k >> 5, slabs = nb / KB;
+    const uint32_t mat = wave / (WV / MS), sl = wave % (WV / MS) / TG, tg = wave % TG;
+    const uint32_t nb = a.k >> 5, all_slabs = nb / KB;
+    const uint32_t first = side ? my_share * all_slabs / ksplit : 0u;  // this workgroup's slabs; shares differ by at most one
+    const uint32_t slabs = side ? (my_share + 1u) * all_slabs / ksplit - first : all_slabs;
 
     struct Regs {
         v4i w[KB], x[KB];
         float2 dw[KB];
         float4 dx;
     };
-    const uint8_t* const slab0 = a.w + ((size_t)(granule >> 1) * slabs * 2 + (granule & 1u)) * kSlab;
-    const int8_t* const xbase = a.xq + (size_t)min(32u * tg + l32, a.n - 1u) * a.k + 16 * kh;
-    // token scales: thread t < 32 WV fetches the four of token t / SL and slab t % SL of the round
+    const uint8_t* const slab0 = (GATED && mat ? a.w_up : a.w) + (((size_t)(granule >> 1) * all_slabs + first) * 2 + (granule & 1u)) * kSlab;
+    const int8_t* const xbase = a.xq + (size_t)min(32u * tg + l32, a.n - 1u) * a.k + (size_t)first * (32 * KB) + 16 * kh;
+    // token scales: thread t < 32 TG SL fetches the four of token t / SL and slab t % SL of the round
     const uint32_t dtok = threadIdx.x / SL, dsl = threadIdx.x % SL;
-    const float* const sbase = DUMP ? nullptr : a.xs + (size_t)min(dtok, a.n - 1u) * nb;
+    const float* const sbase = DUMP ? nullptr : a.xs + (size_t)min(dtok, a.n - 1u) * nb + (size_t)first * KB;
     const auto fetch = [&](uint32_t s0, Regs& r) {
         const uint32_t s = s0 + sl;
         if (s < slabs) {
@@ -1184,7 +1197,7 @@ __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(GemmArgs a) {
                 r.dw[b] = *reinterpret_cast<const float2*>(p + kSlabWt + 256 * b + 8 * l32);
             }
         }
-        if (!DUMP && threadIdx.x < 32u * WV && s0 + dsl < slabs) r.dx = *reinterpret_cast<const float4*>(sbase + (s0 + dsl) * KB);
+        if (!DUMP && threadIdx.x < 32u * TG * SL && s0 + dsl < slabs) r.dx = *reinterpret_cast<const float4*>(sbase + (s0 + dsl) * KB);
     };
 
     v16i cbias;
@@ -1192,9 +1205,13 @@ __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(GemmArgs a) {
     for (int i = 0; i < 16; i++) cbias[i] = (int)kBiasBits;
     asm volatile("" : "+v"(cbias));
     const uint32_t row = threadIdx.x / TPR, tok0 = EP * (threadIdx.x % TPR);  // this thread's elements
-    float acc[EP], total[EP];
+    float acc[MS][EP], total[EP];
 #pragma unroll
-    for (int e = 0; e < EP; e++) acc[e] = total[e] = 0.0f;
+    for (int e = 0; e < EP; e++) {
+        total[e] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < MS; i++) acc[i][e] = 0.0f;
+    }
     uint32_t share = 0, share_end = slabs / shares;
 
     Regs r{};
@@ -1220,13 +1237,13 @@ __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(GemmArgs a) {
                         v4f v;
 #pragma unroll
                         for (int q = 0; q < 4; q++) v[q] = __builtin_fmaf(__int_as_float(d[4 * g + q]), r.dw[b].x, r.dw[b].y);
-                        *reinterpret_cast<v4f*>(&vs[(sl * KB + b) * TG + tg][l32][8 * g + 4 * kh]) = v;
+                        *reinterpret_cast<v4f*>(&vs[mat][(sl * KB + b) * TG + tg][l32][8 * g + 4 * kh]) = v;
                     }
                 }
             }
         }
         if constexpr (!DUMP) {
-            if (threadIdx.x < 32u * WV) {
+            if (threadIdx.x < 32u * TG * SL) {
                 dxs[KB * dsl][dtok] = r.dx.x, dxs[KB * dsl + 1][dtok] = r.dx.y;
                 dxs[KB * dsl + 2][dtok] = r.dx.z, dxs[KB * dsl + 3][dtok] = r.dx.w;
             }
@@ -1237,30 +1254,54 @@ __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(GemmArgs a) {
 #pragma unroll
             for (uint32_t q = 0; q < (uint32_t)SL; q++) {
                 if (s0 + q < slabs) {
-                    if (s0 + q == share_end) {  // the next share of K starts
+                    if (!GATED && s0 + q == share_end) {  // the next share of K starts
                         share++;
                         share_end = (share + 1u) * slabs / shares;
 #pragma unroll
-                        for (int e = 0; e < EP; e++) total[e] = share == 1 ? acc[e] : total[e] + acc[e], acc[e] = 0.0f;
+                        for (int e = 0; e < EP; e++) total[e] = share == 1 ? acc[0][e] : total[e] + acc[0][e], acc[0][e] = 0.0f;
                     }
 #pragma unroll
                     for (int b = 0; b < KB; b++) {
-                        const float* const v = &vs[(q * KB + b) * TG + tok0 / 32][row][tok0 % 32];
                         const float* const dx = &dxs[q * KB + b][tok0];
 #pragma unroll
-                        for (int e = 0; e < EP; e++) acc[e] = __builtin_fmaf(v[e], dx[e], acc[e]);
+                        for (int i = 0; i < MS; i++) {
+                            const float* const v = &vs[i][(q * KB + b) * TG + tok0 / 32][row][tok0 % 32];
+#pragma unroll
+                            for (int e = 0; e < EP; e++) acc[i][e] = __builtin_fmaf(v[e], dx[e], acc[i][e]);
+                        }
                     }
                 }
             }
-            if (s0 + SL < slabs) __syncthreads();  // the planes are written again
+            if (GATED || s0 + SL < slabs) __syncthreads();  // the planes are written again
         }
     }
-    if constexpr (!DUMP) {
+    if constexpr (GATED) {
+        static_assert(WV * 8 >= 32 * TG && sizeof(vs) >= sizeof(float) * 32 * TG * kRow, "eight threads and a row of LDS per token");
+        float* const h = &vs[0][0][0][0];  // [token][row]
+#pragma unroll
+        for (int e = 0; e < EP; e++) h[kRow * (tok0 + e) + row] = silu_mul(acc[0][e], acc[MS - 1][e]);
+        __syncthreads();
+        const uint32_t tok = threadIdx.x >> 3, quad = threadIdx.x & 7u;
+        if (tok < 32u * TG) {
+            const float4 x = *reinterpret_cast<const float4*>(&h[kRow * tok + 4u * quad]);
+            float id;
+            const float scale = q8_scale_and_inverse(group_max8(fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w)))), id);
+            const uint32_t packed = q8_pack4(x.x, x.y, x.z, x.w, id);
+            if (tok < a.n) {
+                *reinterpret_cast<uint32_t*>(a.q_out + (size_t)tok * a.m + GR * granule + 4u * quad) = packed;
+                if (quad == 0) a.s_out[(size_t)tok * (a.m >> 5) + granule] = scale;
+            }
+        }
+    } else if constexpr (!DUMP) {
 #pragma unroll
         for (int e = 0; e < EP; e++) {
             const uint32_t rw = GR * granule + row, t = tok0 + e;
-            const float v = shares == 1 ? acc[e] : total[e] + acc[e];
+            const float v = shares == 1 ? acc[0][e] : total[e] + acc[0][e];
             if (rw < a.m && t < a.n) {
+                if (side) {
+                    a.partial[((size_t)my_share * a.n + t) * a.m + rw] = v;
+                    continue;
+                }
                 float* const y = a.y_row_major ? a.y + (size_t)rw * a.y_stride + t : a.y + (size_t)t * a.y_stride + rw;
                 *y = a.accumulate ? *y + v : v;
             }
@@ -1305,23 +1346,28 @@ uint32_t wide_split_factor(uint32_t m, uint32_t n, uint32_t k, uint32_t max_spli
 bool narrow_tiles(uint64_t row_tiles, uint32_t n) { return n <= BN_NARROW || row_tiles * ((n + BN - 1) / BN) <= kCus; }
 
 // Launches of gemm_few_kernel: up to 64 tokens and few enough granules that latency and not the chip's throughput is what they cost
-// (every workgroup fetches all tokens' activations for its 32 rows; beyond, the 128-row tiles are the cheaper readers).  Tiles / here,
-// us: 2048 x 1024 over 23 tokens 8.8 / 4.9, 1024 x 4608 29 / 14; 65536 x 2048 over 16 27 / 40.
+// (every workgroup fetches all tokens' activations for its 32 rows; beyond, the 128-row tiles are the cheaper readers, and above 32
+// tokens, where a round of K is half as long, the 64-row ones from a second workgroup per CU on).  Tiles / here, us: 2048 x 1024 over 23
+// tokens 8.8 / 4.9, 1024 x 4608 29 / 14; 9216 x 1024 over 32 9.1 / 7.5, over 48 9.5 / 10.6; 65536 x 2048 over 16 27 / 40.
 bool few_applies(uint64_t rows, uint32_t n, uint32_t k) {
     const uint64_t units = (rows + GR - 1) / GR, slabs = k / (KB * 32);
-    return n <= 64 && units <= 2 * kCus && units * slabs <= (n <= 32 ? 12288u : 4096u);
+    return n <= 64 && units <= (n <= 32 ? 2 * kCus : kCus) && units * slabs <= (n <= 32 ? 12288u : 4096u);
 }
 
-// The same for launches that the tiles may split into shares of K side by side, where this kernel walks the shares one after the
-// other: ~0.3 us a slab up to 32 tokens, twice that above.  What the tiles' shares cost instead is a launch that adds them up, or,
-// with `deferrable`, the additions in the norm's kernel behind the projection: nothing at 512 rows, as much as the launch at 4096.
-// Shares side by side / here, us:
+// Shares of K side by side on the same kernel, a workgroup each: while the chip holds them all at once (one workgroup of eight waves per CU,
+// or two of four).  128-row or 64-row tiles / here, us: 1024 x 4608 in 8 over 23 tokens 6.7 / 4.7, over 48 6.9 / 6.3; 2048 x 6912 over 23 8.5 / 7.1,
+// over 37 8.7 / 9.9 (not taken); 2048 x 2048 over 23 4.8 / 4.3; 4096 x 4096 7.2 / 8.9 (not taken).
+bool few_side_applies(uint64_t rows, uint32_t n, uint32_t shares) {
+    return n <= 64 && (rows + GR - 1) / GR * shares <= (n <= 32 ? 2 * kCus : kCus);
+}
+
+// Shares of K one after the other in one launch of that kernel: ~0.3 us a slab up to 32 tokens, twice that above, against shares side by side and
+// the launch that adds them up, or, with `deferrable`, the additions in the norm's kernel behind the projection.  With the norm, side by
+// side is the faster way wherever few_side_applies (1024 x 1024 in 4 over 23 tokens 3.5 and 0.4 more in the norm, here 4.7); beyond, and plain:
 //   plain, 9 tokens:        1024 x 1024 6.3 / 4.5, x 1792 7.5 / 6.5, x 2048 (8 shares, not 4) 6.7 / 7.1; 4096 x 2048 7.0 / 7.3
 //   plain, 24:              1024 x 1024 6.6 / 4.9, x 1792 8.0 / 6.8, x 2048 7.0 / 7.4; 3072 x 2048 7.6 / 7.5, 4096 x 2048 8.5 / 7.5
 //   plain, 40:              1024 x 1024 7.2 / 7.0, 4096 x 1024 8.2 / 7.1; 2048 x 2048 8.2 / 11.5
-//   with the norm, 24:      512 x 1024 8.0 / 7.9, x 2048 7.9 / 10.2; 1024 x 1024 8.1 / 7.8, x 1536 8.8 / 9.3; 2048 x 1152 9.9 / 9.4,
-//                           x 2048 9.8 / 11.2; 3072 x 1792 11.9 / 11.2, 4096 x 2048 13.3 / 12.5
-//   with the norm, 40:      1024 x 1024 8.5 / 10.2, 2048 x 1024 10.0 / 10.8, 3072 x 1024 11.3 / 11.6, 4096 x 1024 12.9 / 12.3
+//   with the norm, 24:      4096 x 2048 13.3 / 12.5; over 40 tokens 3072 x 1024 11.3 / 11.6, 4096 x 1024 12.9 / 12.3
 bool few_applies_split(uint64_t rows, uint32_t n, uint32_t k, bool deferrable) {
     const uint64_t units = (rows + GR - 1) / GR, slabs = k / (KB * 32), cost = n <= 32 ? 1u : 2u;
     if (!few_applies(rows, n, k) || slabs * cost > (cost == 1 && units < 96 ? 15u : 16u)) return false;
@@ -1446,22 +1492,24 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, bool in_launch, uint32
             if (q8) return go(gemm_tile_kernel<8, true, false, C>, C::kRows, C::kTokens, C::kThreads);
         return go(gemm_tile_kernel<2, DUMP, false, C>, C::kRows, C::kTokens, C::kThreads);
     };
-    const bool few = !L.gemm_mfma16 && (ksplit > 1 ? in_launch : few_applies(GR * tile_rows(GR), a.n, a.k));
+    const bool few = !L.gemm_mfma16 && (ksplit > 1 ? in_launch || few_side_applies(a.m, a.n, ksplit) : few_applies(GR * tile_rows(GR), a.n, a.k));
     const bool narrow = !wide_split && narrow_tiles(tile_rows(BM), a.n);
     if (few) {
         // Eight waves and 151 KB of LDS while every CU gets one workgroup at most, else four and half of it.
+        const bool whole = DUMP || ksplit == 1 || in_launch;
         const auto waves = [&](auto tg, auto wv) {
             constexpr int TG = decltype(tg)::value, WV = decltype(wv)::value;
             if constexpr (DUMP)
-                if (q8) return go(gemm_few_kernel<8, true, TG, WV>, GR, 64, 64 * WV, true);
-            return go(gemm_few_kernel<2, DUMP, TG, WV>, GR, 64, 64 * WV, true);
+                if (q8) return go(gemm_few_kernel<8, true, false, TG, WV>, GR, 64, 64 * WV, whole);
+            return go(gemm_few_kernel<2, DUMP, false, TG, WV>, GR, 64, 64 * WV, whole);
         };
-        if (tile_rows(GR) <= kCus) return a.n <= 32 ? waves(Idx<1>{}, Idx<8>{}) : waves(Idx<2>{}, Idx<8>{});
+        if (tile_rows(GR) * (whole ? 1u : ksplit) <= kCus) return a.n <= 32 ? waves(Idx<1>{}, Idx<8>{}) : waves(Idx<2>{}, Idx<8>{});
         return a.n <= 32 ? waves(Idx<1>{}, Idx<4>{}) : waves(Idx<2>{}, Idx<4>{});
     }
-    if (narrow && (a.n <= 48 || L.gemm_mfma16)) {
+    if (narrow && (a.n <= (ksplit > 1 ? 32u : 48u) || L.gemm_mfma16)) {
         // a launch of at most 16 / 32 / 48 tokens computes one / two / three of the tile's four 16-token MFMA tiles (the parity
         // hook: all four).  These launches are bound by their block loop, not by memory: 65536 x 16 x 2048 40 -> 34 us.
+        // (33 .. 48 tokens in shares of K: the 64-row tile.  2048 x 6912 in 8 over 37 9.6 / 8.7 us.)
         if constexpr (!DUMP) {
             if (a.n <= 16) return go(gemm_narrow_kernel<2, false, 1>, BM, BN_NARROW, THREADS);
             if (a.n <= 32) return go(gemm_narrow_kernel<2, false, 2>, BM, BN_NARROW, THREADS);
@@ -1483,8 +1531,9 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, bool in_launch, uint32
 }  // namespace
 
 uint32_t gemm_split_k(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits) { return split_k_factor(m, n, k, max_splits); }
-bool gemm_split_in_launch(uint32_t m, uint32_t n, uint32_t k, const Launch& L, bool deferrable) {
-    return !L.gemm_mfma16 && few_applies_split(m, n, k, deferrable);
+bool gemm_split_in_launch(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits, const Launch& L, bool deferrable) {
+    if (L.gemm_mfma16 || !few_applies_split(m, n, k, deferrable)) return false;
+    return !deferrable || !few_side_applies(m, n, split_k_factor(m, n, k, max_splits));
 }
 
 // The GEMM's own copy of a weight (slabs, see StageT): its size, and the kernel that makes it from the raw blocks.
@@ -1512,7 +1561,7 @@ hipError_t launch_gemm_mfma(int type, const uint8_t* d_w, uint32_t m, uint32_t k
     a.accumulate = accumulate;
     const bool in_launch = splits > 1 && !d_partial;
     if (splits > 1) {
-        if (splits != split_k_factor(m, n, k, splits) || (in_launch && !gemm_split_in_launch(m, n, k, L, false)))
+        if (splits != split_k_factor(m, n, k, splits) || (in_launch && !gemm_split_in_launch(m, n, k, splits, L, false)))
             return hipErrorInvalidValue;  // the shape does not carry that split
         a.ksplit = splits, a.partial = d_partial;
     }
@@ -1543,25 +1592,51 @@ bool gemm_gated_applies(uint32_t m, uint32_t n, uint32_t k) {
     return m % 32u == 0 && k % 128u == 0 && n > BN_NARROW && (uint64_t)((m + 63u) / 64u) * ((n + BN - 1) / BN) > kCus;
 }
 
+namespace {
+// The few-token form of the launch: one workgroup per granule and CU.
+bool gated_few_applies(uint32_t m, uint32_t n) { return n <= 32 && m / GR <= kCus; }
+
+template <typename C>
+float gated_tile_cost(uint32_t m, uint32_t n, uint32_t k) { return tile_cost<C>((m + C::kRows / 2 - 1) / (C::kRows / 2), n, k, 1, true); }
+}  // namespace
+
+// Where the launch is expected to be faster than the two projections in one launch and the gate kernel behind it (2.7 us and the floats'
+// round trip).  In one launch / two, us: 4608 x 1024 over 9 .. 32 tokens 7.0 .. 7.8 / 9.5 .. 10.2, over 48 11.9 / 12.4, 128 12.2 / 13.1, 300 14.8 / 17.9;
+// 6912 x 2048 over 23 12.4 / 14.1, over 64 19.5 / 18.1 (not taken), 200 25.0 / 28.4.
+bool gemm_gated_faster(uint32_t m, uint32_t n, uint32_t k, const Launch& L) {
+    if (gemm_gated_applies(m, n, k)) return true;
+    if (L.gemm_mfma16 || m % GR != 0 || k % (KB * 32) != 0 || m == 0 || n == 0) return false;
+    if (gated_few_applies(m, n)) return true;
+    if (n <= 48 && (uint64_t)2 * m / GR > 2 * kCus) return false;  // the narrow kernel's
+    const auto plain = [&](auto cfg) {
+        using C = decltype(cfg);
+        return tile_cost<C>(2 * (uint64_t)((m + C::kRows - 1) / C::kRows), n, k, 1);
+    };
+    const float separate = std::min({plain(TileL{}), plain(TileX{}), plain(TileS{}), plain(TileQ{}), plain(TileN{}), plain(TileH{})});
+    const float gated = std::min({gated_tile_cost<TileL>(m, n, k), gated_tile_cost<TileX>(m, n, k), gated_tile_cost<TileS>(m, n, k), gated_tile_cost<TileQ>(m, n, k)});
+    return !few_applies(2 * (uint64_t)m, n, k) && gated < separate + 2.7f + (float)n * (float)m * 3e-6f;
+}
+
+// Any n; d_out_* as for gemm_gated_applies.
 hipError_t launch_gemm_mfma_gated(int /*type: the copies are the same for both*/, const uint8_t* d_w_gate, const uint8_t* d_w_up, uint32_t m, uint32_t k, const int8_t* d_q,
                                   const float* d_scales, uint32_t n, int8_t* d_out_q, float* d_out_scales, const Launch& L) {
     if (m == 0 || n == 0) return hipSuccess;
-    if (!gemm_gated_applies(m, n, k)) return hipErrorInvalidValue;
+    if (m % GR != 0 || k % (KB * 32) != 0) return hipErrorInvalidValue;
     GemmArgs a{};
     a.w = d_w_gate, a.w_up = d_w_up, a.xq = d_q, a.xs = d_scales, a.q_out = d_out_q, a.s_out = d_out_scales;
     a.m = m, a.n = n, a.k = k;
     a.tile_start[0] = a.tile_start[1] = UINT32_MAX;
+    if (gated_few_applies(m, n)) {
+        a.row_tiles = m / GR, a.tok_tiles = 1;
+        return launch_kernel(L, kFamGemm, gemm_few_kernel<2, false, true, 1, 8>, dim3(a.row_tiles), dim3(512), a);
+    }
     const auto tile = [&](auto cfg) {
         using C = decltype(cfg);
         a.row_tiles = (m + C::kRows / 2 - 1) / (C::kRows / 2), a.tok_tiles = (n + C::kTokens - 1) / C::kTokens;
         if ((uint64_t)a.row_tiles * a.tok_tiles > 0x7fffff00ull) return hipErrorInvalidValue;
         return launch_kernel(L, kFamGemm, gemm_tile_kernel<2, false, true, C>, dim3((a.row_tiles * a.tok_tiles + 7u) / 8u * 8u), dim3(C::kThreads), a);
     };
-    const auto cost = [&](auto cfg) {
-        using C = decltype(cfg);
-        return tile_cost<C>((m + C::kRows / 2 - 1) / (C::kRows / 2), n, k, 1, true);
-    };
-    return cheapest_tile<TileL, TileX, TileS, TileQ>(cost, tile);
+    return cheapest_tile<TileL, TileX, TileS, TileQ>([&](auto cfg) { return gated_tile_cost<decltype(cfg)>(m, n, k); }, tile);
 }
 
 // Parity hook through the matrix-core path: the same loads, unpack, LDS layout and
@@ -1572,7 +1647,7 @@ hipError_t launch_block_dots_mfma(int type, const uint8_t* d_w, uint32_t m, uint
     a.w = d_w, a.xq = d_q, a.xs = nullptr, a.y = nullptr, a.dots = d_out;
     a.m = m, a.n = n, a.k = k, a.y_stride = 0;
     a.ksplit = split_k_factor(m, n, k, max_splits);
-    return launch<true>(type, a, L, gemm_split_in_launch(m, n, k, L, false));
+    return launch<true>(type, a, L, gemm_split_in_launch(m, n, k, max_splits, L, false));
 }
 
 }  // namespace wick_rocm

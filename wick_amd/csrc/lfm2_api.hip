@@ -584,6 +584,12 @@ int gemm_group(wick_rocm_ctx* ctx, std::initializer_list<const wick_rocm_weight*
     return WICK_ROCM_OK;
 }
 
+// Whether a pass's gate and up projections go out in one launch with the gate and the down projection's quantizer (the same bits).
+bool gate_up_in_one_launch(wick_rocm_ctx* ctx, const wick_rocm_weight* gate, const wick_rocm_weight* up, uint32_t n) {
+    return gate->d_gemm && up->d_gemm && gate->type == up->type && gate->m == up->m && gate->k == up->k && n >= ctx->min_n_for(gate->nbytes + up->nbytes) &&
+           gemm_gated_faster(gate->m, n, gate->k, ctx->launch());
+}
+
 // One pass of a prompt: n <= prefill_cap tokens (device-readable; null: their rows are in pX already) at positions pos0 .. pos0 + n - 1.  The batched form
 // of enqueue_step (prefill_layers_and_logits, wick/src/model/lfm2.rs:1139-2109): projections as GEMMs over the tokens,
 // the short conv per (token, channel) with the rolling state behind it, the KV append per token, causal attention per
@@ -647,13 +653,13 @@ int enqueue_prompt_pass(wick_rocm_ctx* ctx, wick_rocm_lfm2* m, uint32_t n, uint3
         // the out projection's input: already Q8_0 blocks when its producer wrote them itself
         if (!quantized && (rc = wick_rocm_quantize_q8_0(ctx, m->pG, n, hs, hs, m->pQ, m->pS))) break;
         if ((rc = project_and_norm(L.n_kv == 0 ? L.out_proj : L.o, m->pQ, m->pS, L.ffn_norm))) break;  // hidden += out projection; FFN norm
-        if (wick_rocm_ffn_gate_up_silu_quantize_applies(L.gate, L.up, n)) {
-            // gate, up, SiLU gate and the down projection's quantizer in one launch; its output cannot overwrite its own input.
-            // (GEMM + gate kernel against this, us inside a prompt pass: 4608 x 1024 over 2002 tokens 75.0 / 68.4, over 555 31.5 / 25.9;
-            // 6912 x 2048 over 2002 173.8 / 162.8, over 1024 95.2 / 86.2, over 1400 122.1 / 124.5 -- the one length found where it loses.
-            // Whole prompts of 400 .. 4096 tokens through the 350M shape are 1.02 - 1.09 times as fast with it; through six layers of the
-            // 1.2B shape 1.04 at 300 .. 1024, 0.99 at 1400, 1.01 at 2002, 1.02 at 4096.)
-            if ((rc = wick_rocm_ffn_gate_up_silu_quantize_q8(ctx, L.gate, L.up, m->pQ, m->pS, n, m->pQ2, m->pS2))) break;
+        if (gate_up_in_one_launch(ctx, L.gate, L.up, n)) {
+            // gate, up, SiLU gate and the down projection's quantizer; the output cannot overwrite the input
+            if ((rc = locked([&] {
+                     return launch_gemm_mfma_gated(L.gate->type, static_cast<const uint8_t*>(L.gate->d_gemm), static_cast<const uint8_t*>(L.up->d_gemm), L.gate->m,
+                                                   L.gate->k, m->pQ, m->pS, n, m->pQ2, m->pS2, ctx->launch());
+                 }, "gate / up launch")))
+                break;
             rc = next_norm ? project_and_norm(L.down, m->pQ2, m->pS2, next_norm)
                            : wick_rocm_gemm_q8(ctx, L.down, m->pQ2, m->pS2, n, m->pX, hs, WICK_ROCM_LAYOUT_TOKEN_MAJOR, 1);
             continue;

@@ -155,12 +155,14 @@ hipError_t launch_gemm_mfma(int type, const uint8_t* d_w, uint32_t m, uint32_t k
 uint32_t gemm_split_k(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits);
 // Whether the launch, on the block loop that L asks for, should walk its shares itself (few tokens): no scratch, nothing to defer.
 // deferrable: the caller's next kernel would add the shares up.  (With deferrable: a part of what there is without.)
-bool gemm_split_in_launch(uint32_t m, uint32_t n, uint32_t k, const Launch& L, bool deferrable);
+bool gemm_split_in_launch(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits, const Launch& L, bool deferrable);
 hipError_t launch_gemm_mfma_multi(int type, const uint8_t* const* d_w, const uint32_t* m, uint32_t count, uint32_t k, const int8_t* d_q,
                                   const float* d_scales, uint32_t n, float* const* d_y, uint32_t y_stride, int y_layout, int accumulate,
                                   const Launch& L);
-// out = Q8_0(silu(W_gate x) * (W_up x)) over n tokens in one launch (wide tiles only: gemm_gated_applies).
+// out = Q8_0(silu(W_gate x) * (W_up x)) over n tokens in one launch (m % 32 == 0, k % 128 == 0).  gemm_gated_applies: what the entry point for it
+// takes; gemm_gated_faster: where a caller that may as well take two launches should take it.
 bool gemm_gated_applies(uint32_t m, uint32_t n, uint32_t k);
+bool gemm_gated_faster(uint32_t m, uint32_t n, uint32_t k, const Launch& L);
 hipError_t launch_gemm_mfma_gated(int type, const uint8_t* d_w_gate, const uint8_t* d_w_up, uint32_t m, uint32_t k, const int8_t* d_q,
                                   const float* d_scales, uint32_t n, int8_t* d_out_q, float* d_out_scales, const Launch& L);
 
