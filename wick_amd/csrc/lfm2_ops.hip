@@ -1016,12 +1016,20 @@ template <int HALVES, typename KV>
 __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(AttentionArgs a, uint32_t pos0, uint32_t n, uint32_t q_stride, uint32_t out_stride,
                                                                                 int8_t* q_out, float* s_out) {
     constexpr bool LO = std::is_same<KV, float>::value;  // the caches' values have low halves
+    constexpr int PLANES = LO ? 2 : 1;                   // hi | lo
     constexpr int HD = 64, KT = 64, NT = 512 * HALVES;
     constexpr int LDH = 72;  // f16 per K row: 64 + 8 (144 bytes: 16-byte aligned rows, conflict-free 16-byte operand reads)
-    constexpr int LDV = 68;  // f16 per V^T row: 64 + 4 (136 bytes: 8-byte aligned rows; 64 rows' 8-byte writes cover all banks twice)
     constexpr float kPScale = 4096.0f;
-    __shared__ __align__(16) _Float16 kbuf[2][2][KT][LDH];  // [buffer][hi | lo][key][dim]
-    __shared__ __align__(16) _Float16 vbuf[2][2][HD][LDV];  // [buffer][hi | lo][dim][key]
+    // Two tiles: K [plane][key][LDH], V [plane][key][dim] with 16-byte piece p of a row at p ^ (key & 7), so that the 16 rows that a
+    // transposing read touches spread over the banks.  At the end the partner states, kStates floats per lane.
+    constexpr int kStates = 18;
+    struct Tile {
+        _Float16 k[PLANES][KT][LDH];
+        _Float16 v[PLANES][KT][HD];
+    };
+    constexpr size_t kTilesBytes = 2 * sizeof(Tile), kStateBytes = sizeof(float) * kStates * 64 * 4 * HALVES;
+    __shared__ __align__(16) uint8_t smem[kTilesBytes > kStateBytes ? kTilesBytes : kStateBytes];
+    Tile* const tiles = reinterpret_cast<Tile*>(smem);
     const uint32_t h = blockIdx.x;
     const uint32_t qblocks = (n + 63u) / 64u;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, l16 = lane & 15u, g = lane >> 4;
@@ -1040,7 +1048,7 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(A
     const uint32_t pq = base + jl;
     uint32_t wg_last = base + (qb_long * 64u + 63u < n ? qb_long * 64u + 63u : n - 1u);
     if (wg_last >= a.max_seq) wg_last = a.max_seq - 1u;
-    const uint32_t wave_last = min(base + min(j0 + 16u * wave + 15u, n - 1u), wg_last);
+    const uint32_t wave_first = base + min(j0 + 16u * wave, n - 1u), wave_last = min(base + min(j0 + 16u * wave + 15u, n - 1u), wg_last);
 
     // this lane's query, dims 32 s + 8 g .. + 7 of slab s, scaled and split
     h8 qh[2], ql[2];
@@ -1063,144 +1071,173 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(A
     for (int c = 0; c < 4; c++) o[c] = v4f{0.f, 0.f, 0.f, 0.f};
     float m_run = -__builtin_inff(), l_run = 0.0f;
 
-    constexpr int C4 = HD / 4, RPP = NT / C4, NR = KT / RPP;
-    const uint32_t c4 = tid % C4, r0 = tid / C4;
-    float4 kk[NR], vv[NR];
-    auto fetch_tile = [&](uint32_t t0) {
+    // A tile's pieces of 16 bytes -- of f32 rows four values, which become 8 bytes of each plane; of f16 rows eight, which go to LDS as they
+    // are -- dealt out to the threads: kk of K and as many of V, or (f16, 1024 threads) one of either.
+    constexpr int PPR = LO ? 16 : 8, kPieces = KT * PPR, kBoth = 2 * kPieces / NT, NR = kBoth > 1 ? kBoth / 2 : 1;
+    static_assert(kBoth >= 1 && (kBoth == 1 || kBoth % 2 == 0), "every thread moves the same number of pieces");
+    using Piece = typename std::conditional<LO, float4, h8>::type;
+    struct Regs {
+        Piece k[NR], v[NR];  // (v unused where a thread moves one piece)
+    };
+    const uint32_t piece = tid % PPR, row0 = tid / PPR % KT;
+    const bool moves_v = kBoth == 1 && tid >= (uint32_t)kPieces;
+    // Rows past the last position any query sees repeat it (their weights are zero); tiles past the last one are never looked at.
+    auto fetch = [&](uint32_t t0, Regs& r) {
 #pragma unroll
         for (int i = 0; i < NR; i++) {
-            const uint32_t key = min(t0 + r0 + i * RPP, wg_last);
-            kk[i] = kv_load4(kbase + (size_t)key * kv_dim + 4u * c4);
-            vv[i] = kv_load4(vbase + (size_t)key * kv_dim + 4u * c4);
+            const size_t at = (size_t)min(t0 + row0 + i * (NT / PPR), wg_last) * kv_dim + (16u / sizeof(KV)) * piece;
+            if constexpr (kBoth == 1) {
+                r.k[0] = *reinterpret_cast<const Piece*>((moves_v ? vbase : kbase) + at);
+            } else {
+                r.k[i] = *reinterpret_cast<const Piece*>(kbase + at);
+                r.v[i] = *reinterpret_cast<const Piece*>(vbase + at);
+            }
         }
     };
-    // A thread holds one key x four dims of K and of V.  K rows go to LDS as they are; V is transposed on the way: the four
-    // lane groups of a wave hold four consecutive keys of the same dims, so a 4 x 4 transpose across them (two rounds of
-    // row / half swaps on {hi, lo} pairs packed into one register) leaves every lane with four keys of one dim = one
-    // 8-byte write per half, instead of eight conflicting 2-byte writes.
-    auto store_tile = [&](int buf) {
+    auto store = [&](Tile& t, const Regs& r) {
 #pragma unroll
         for (int i = 0; i < NR; i++) {
-            const uint32_t key = r0 + i * RPP;
-            const float kf[4] = {kk[i].x, kk[i].y, kk[i].z, kk[i].w}, vf[4] = {vv[i].x, vv[i].y, vv[i].z, vv[i].w};
-            h4 khi, klo;
-            uint32_t vp[4];  // V of this key: dim j as {hi, lo}
+            const uint32_t key = row0 + i * (NT / PPR);
+            if constexpr (LO) {
+                const uint32_t vat = 8u * ((piece >> 1) ^ (key & 7u)) + 4u * (piece & 1u);
+                const float kf[4] = {r.k[i].x, r.k[i].y, r.k[i].z, r.k[i].w}, vf[4] = {r.v[i].x, r.v[i].y, r.v[i].z, r.v[i].w};
+                h4 khi, klo, vhi, vlo;
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                _Float16 hi, lo;
-                split_f16(kf[j], hi, lo);
-                khi[j] = hi, klo[j] = lo;
-                split_f16(vf[j], hi, lo);
-                vp[j] = (uint32_t)__builtin_bit_cast(uint16_t, hi) | ((uint32_t)__builtin_bit_cast(uint16_t, lo) << 16);
-            }
-            *reinterpret_cast<h4*>(&kbuf[buf][0][key][4 * c4]) = khi;
-            if constexpr (LO) *reinterpret_cast<h4*>(&kbuf[buf][1][key][4 * c4]) = klo;
-            // transpose M[g][j] (g = lane group = key, j = register = dim) in 2 x 2 blocks, then the blocks themselves
-            auto s01 = __builtin_amdgcn_permlane16_swap(vp[0], vp[1], false, false);
-            auto s23 = __builtin_amdgcn_permlane16_swap(vp[2], vp[3], false, false);
-            auto t02 = __builtin_amdgcn_permlane32_swap(s01[0], s23[0], false, false);
-            auto t13 = __builtin_amdgcn_permlane32_swap(s01[1], s23[1], false, false);
-            const uint32_t w[4] = {t02[0], t13[0], t02[1], t13[1]};  // this lane's dim 4 c4 + g, keys (key & ~3) + 0 .. 3
-            uint2 vhi, vlo;
-            vhi.x = __builtin_amdgcn_perm(w[1], w[0], 0x05040100u), vhi.y = __builtin_amdgcn_perm(w[3], w[2], 0x05040100u);
-            vlo.x = __builtin_amdgcn_perm(w[1], w[0], 0x07060302u), vlo.y = __builtin_amdgcn_perm(w[3], w[2], 0x07060302u);
-            const uint32_t key4 = key & ~3u;
-            *reinterpret_cast<uint2*>(&vbuf[buf][0][4 * c4 + g][key4]) = vhi;
-            if constexpr (LO) *reinterpret_cast<uint2*>(&vbuf[buf][1][4 * c4 + g][key4]) = vlo;
-        }
-    };
-    fetch_tile(0);
-    store_tile(0);
-    if (KT <= wg_last) fetch_tile(KT);
-    __syncthreads();
-    int cur = 0;
-    for (uint32_t t0 = 0; t0 <= wg_last; t0 += KT, cur ^= 1) {
-        const uint32_t key0 = t0 + 32u * ksp;  // this wave's 32 keys of the tile
-        if (active && key0 <= wave_last) {
-            // scores: 2 sub-tiles of 16 keys x 2 slabs of 32 dims x 3 products
-            v4f sc[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
-            h8 kh[2][2], kl[2][2];  // [slab][sub-tile]
-#pragma unroll
-            for (int s = 0; s < 2; s++)
-#pragma unroll
-                for (int u = 0; u < 2; u++) {
-                    kh[s][u] = *reinterpret_cast<const h8*>(&kbuf[cur][0][32u * ksp + 16 * u + l16][32 * s + 8 * g]);
-                    if constexpr (LO) kl[s][u] = *reinterpret_cast<const h8*>(&kbuf[cur][1][32u * ksp + 16 * u + l16][32 * s + 8 * g]);
-                }
-#pragma unroll
-            for (int s = 0; s < 2; s++) {
-                if constexpr (LO) {
-#pragma unroll
-                    for (int u = 0; u < 2; u++) sc[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl[s][u], qh[s], sc[u], 0, 0, 0);
-                }
-#pragma unroll
-                for (int u = 0; u < 2; u++) sc[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[s][u], ql[s], sc[u], 0, 0, 0);
-#pragma unroll
-                for (int u = 0; u < 2; u++) sc[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[s][u], qh[s], sc[u], 0, 0, 0);
-            }
-            // the V operands of the second product are on their way while the softmax runs
-            h8 vh[4], vl[4];
-#pragma unroll
-            for (int c = 0; c < 4; c++) {
-                const h4 a0 = *reinterpret_cast<const h4*>(&vbuf[cur][0][16 * c + l16][32u * ksp + 4 * g]);
-                const h4 a1 = *reinterpret_cast<const h4*>(&vbuf[cur][0][16 * c + l16][32u * ksp + 16 + 4 * g]);
-                vh[c] = h8{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
-                if constexpr (LO) {
-                    const h4 b0 = *reinterpret_cast<const h4*>(&vbuf[cur][1][16 * c + l16][32u * ksp + 4 * g]);
-                    const h4 b1 = *reinterpret_cast<const h4*>(&vbuf[cur][1][16 * c + l16][32u * ksp + 16 + 4 * g]);
-                    vl[c] = h8{b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
-                }
-            }
-            float tmax = -__builtin_inff();
-            const bool masked_tile = key0 + 31u > base + min(j0 + 16u * wave, n - 1u);
-#pragma unroll
-            for (int u = 0; u < 2; u++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    if (masked_tile && key0 + 16u * u + 4u * g + r > pq) sc[u][r] = -__builtin_inff();
-                    tmax = fmaxf(tmax, sc[u][r]);
-                }
-            tmax = groups_max(tmax);
-            const float m_new = fmaxf(m_run, tmax);
-            const float m_sub = m_new == -__builtin_inff() ? 0.0f : m_new;
-            const float alpha = exp_nonpos_hw(m_run - m_sub);
-            m_run = m_new;
-            float psum = 0.0f;
-            h8 ph, pl;
-#pragma unroll
-            for (int u = 0; u < 2; u++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const float pw = exp_nonpos_hw(sc[u][r] - m_sub);
-                    psum += pw;
+                for (int e = 0; e < 4; e++) {
                     _Float16 hi, lo;
-                    split_f16(pw * kPScale, hi, lo);
-                    ph[4 * u + r] = hi, pl[4 * u + r] = lo;
+                    split_f16(kf[e], hi, lo);
+                    khi[e] = hi, klo[e] = lo;
+                    split_f16(vf[e], hi, lo);
+                    vhi[e] = hi, vlo[e] = lo;
                 }
-            l_run = l_run * alpha + psum;
+                *reinterpret_cast<h4*>(&t.k[0][key][4 * piece]) = khi;
+                *reinterpret_cast<h4*>(&t.k[PLANES - 1][key][4 * piece]) = klo;
+                *reinterpret_cast<h4*>(&t.v[0][key][vat]) = vhi;
+                *reinterpret_cast<h4*>(&t.v[PLANES - 1][key][vat]) = vlo;
+            } else {
+                _Float16* const kd = &t.k[0][key][8 * piece];
+                _Float16* const vd = &t.v[0][key][8u * (piece ^ (key & 7u))];
+                if constexpr (kBoth == 1) {
+                    *reinterpret_cast<h8*>(moves_v ? vd : kd) = r.k[0];
+                } else {
+                    *reinterpret_cast<h8*>(kd) = r.k[i];
+                    *reinterpret_cast<h8*>(vd) = r.v[i];
+                }
+            }
+        }
+    };
+    // V^T rows (dims) 16 c + l16, keys 32 ksp + 16 u + 4 g ..: the 16 lanes of a lane group point at 4 keys x 16 dims, lane i at key i / 4 and dims
+    // 4 (i % 4) .. of them, and the read hands every lane four keys of one dim.
+    const uint32_t vkey = 32u * ksp + 4u * g + (l16 >> 2);
+    uint32_t v_at[4];
 #pragma unroll
-            for (int c = 0; c < 4; c++) o[c] *= alpha;
+    for (uint32_t c = 0; c < 4; c++) v_at[c] = vkey * HD + 8u * ((2u * c + ((l16 >> 1) & 1u)) ^ (vkey & 7u)) + 4u * (l16 & 1u);
+    auto read_v = [&](const Tile& t, int plane, int c) {
+        typedef short s4 __attribute__((ext_vector_type(4)));
+        typedef __attribute__((address_space(3))) s4* lds_s4;
+        const _Float16* const p = &t.v[plane][0][0] + v_at[c];  // (keys 16 apart swizzle alike)
+        const h4 a0 = __builtin_bit_cast(h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)p));
+        const h4 a1 = __builtin_bit_cast(h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(p + 16 * HD)));
+        return h8{a0[0], a0[1], a0[2], a0[3], a1[0], a1[1], a1[2], a1[3]};
+    };
+    auto attend = [&](const Tile& t, uint32_t t0) {
+        const uint32_t key0 = t0 + 32u * ksp;  // this wave's 32 keys of the tile
+        if (!active || key0 > wave_last) return;
+        // scores: 2 sub-tiles of 16 keys x 2 slabs of 32 dims x 3 products
+        v4f sc[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
+        h8 kh[2][2], kl[2][2];  // [slab][sub-tile]
+#pragma unroll
+        for (int s = 0; s < 2; s++)
+#pragma unroll
+            for (int u = 0; u < 2; u++) {
+                kh[s][u] = *reinterpret_cast<const h8*>(&t.k[0][32u * ksp + 16 * u + l16][32 * s + 8 * g]);
+                if constexpr (LO) kl[s][u] = *reinterpret_cast<const h8*>(&t.k[PLANES - 1][32u * ksp + 16 * u + l16][32 * s + 8 * g]);
+            }
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
             if constexpr (LO) {
 #pragma unroll
-                for (int c = 0; c < 4; c++) o[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl[c], ph, o[c], 0, 0, 0);
+                for (int u = 0; u < 2; u++) sc[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kl[s][u], qh[s], sc[u], 0, 0, 0);
             }
 #pragma unroll
-            for (int c = 0; c < 4; c++) o[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[c], pl, o[c], 0, 0, 0);
+            for (int u = 0; u < 2; u++) sc[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[s][u], ql[s], sc[u], 0, 0, 0);
 #pragma unroll
-            for (int c = 0; c < 4; c++) o[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[c], ph, o[c], 0, 0, 0);
+            for (int u = 0; u < 2; u++) sc[u] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kh[s][u], qh[s], sc[u], 0, 0, 0);
         }
-        if (t0 + KT <= wg_last) {
-            store_tile(cur ^ 1);
-            if (t0 + 2 * KT <= wg_last) fetch_tile(t0 + 2 * KT);
+        // the V operands of the second product are on their way while the softmax runs
+        h8 vh[4], vl[4];
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            vh[c] = read_v(t, 0, c);
+            if constexpr (LO) vl[c] = read_v(t, PLANES - 1, c);
         }
+        if (key0 + 31u > wave_first) {  // some query does not see all of the keys
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int r = 0; r < 4; r++)
+                    if (key0 + 16u * u + 4u * g + r > pq) sc[u][r] = -__builtin_inff();
+        }
+        float tmax = -__builtin_inff();
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) tmax = fmaxf(tmax, sc[u][r]);
+        tmax = groups_max(tmax);
+        const float m_new = fmaxf(m_run, tmax);
+        const float m_sub = m_new == -__builtin_inff() ? 0.0f : m_new;
+        float alpha = 1.0f;
+        if (__builtin_amdgcn_ballot_w64(m_new > m_run) != 0) {  // else every factor is one (or acts on zeros)
+            alpha = exp_nonpos_hw(m_run - m_sub);
+            m_run = m_new;
+#pragma unroll
+            for (int c = 0; c < 4; c++) o[c] *= alpha;
+        }
+        float psum = 0.0f;
+        h8 ph, pl;
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const float pw = exp_nonpos_hw(sc[u][r] - m_sub);
+                psum += pw;
+                _Float16 hi, lo;
+                split_f16(pw * kPScale, hi, lo);
+                ph[4 * u + r] = hi, pl[4 * u + r] = lo;
+            }
+        l_run = __builtin_fmaf(l_run, alpha, psum);
+        if constexpr (LO) {
+#pragma unroll
+            for (int c = 0; c < 4; c++) o[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vl[c], ph, o[c], 0, 0, 0);
+        }
+#pragma unroll
+        for (int c = 0; c < 4; c++) o[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[c], pl, o[c], 0, 0, 0);
+#pragma unroll
+        for (int c = 0; c < 4; c++) o[c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vh[c], ph, o[c], 0, 0, 0);
+    };
+    // Tile t sits in LDS, t + 1 and t + 2 are on their way in registers: behind the arithmetic of tile t the first goes into the buffer that tile
+    // t - 1 left and t + 3 is requested in its place.  One barrier per tile.
+    Regs r0, r1;
+    fetch(0, r0);
+    fetch(KT, r1);
+    store(tiles[0], r0);
+    fetch(2 * KT, r0);
+    __syncthreads();
+    for (uint32_t t0 = 0; t0 <= wg_last; t0 += 2 * KT) {
+        attend(tiles[0], t0);
+        store(tiles[1], r1);
+        fetch(t0 + 3 * KT, r1);
+        __syncthreads();
+        if (t0 + KT > wg_last) break;
+        attend(tiles[1], t0 + KT);
+        store(tiles[0], r0);
+        fetch(t0 + 4 * KT, r0);
         __syncthreads();
     }
     l_run = groups_sum(l_run);
     {
-        // the upper-key waves hand (maximum, weight sum, weighted values) to their partners through the K buffers
-        constexpr int NS = 18;
-        static_assert(sizeof(kbuf) >= sizeof(float) * NS * 64 * 4 * HALVES, "K buffers hold the partner states");
-        float* xch = reinterpret_cast<float*>(&kbuf[0][0][0][0]) + (size_t)(half * 4u + wave) * NS * 64u + lane;
+        // the upper-key waves hand (maximum, weight sum, weighted values) to their partners through LDS
+        float* xch = reinterpret_cast<float*>(smem) + (size_t)(half * 4u + wave) * kStates * 64u + lane;
         if (ksp == 1) {
             xch[0] = m_run, xch[64] = l_run;
 #pragma unroll
