@@ -980,9 +980,17 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ void split_f16(float x, _Float16& hi, _Float16& lo) {
-    hi = (_Float16)x;
-    lo = (_Float16)(x - (float)hi);
+// Four values at a time: two conversions of a pair, not one of each value and one of the pair.
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void split_f16(const v4f& x, h4& hi, h4& lo) {
+#pragma unroll
+    for (int i = 0; i < 4; i += 2) {
+        h2 h = __builtin_convertvector((v2f{x[i], x[i + 1]}), h2);
+        asm("" : "+v"(h));
+        const h2 l = __builtin_convertvector((v2f{x[i] - (float)h[0], x[i + 1] - (float)h[1]}), h2);
+        hi[i] = h[0], hi[i + 1] = h[1], lo[i] = l[0], lo[i + 1] = l[1];
+    }
 }
 
 // Reductions over the four lane groups of a query (lanes l, l ^ 16, l ^ 32, l ^ 48) with gfx950's row / half swaps: swapping a
@@ -1030,17 +1038,19 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(A
     constexpr size_t kTilesBytes = 2 * sizeof(Tile), kStateBytes = sizeof(float) * kStates * 64 * 4 * HALVES;
     __shared__ __align__(16) uint8_t smem[kTilesBytes > kStateBytes ? kTilesBytes : kStateBytes];
     Tile* const tiles = reinterpret_cast<Tile*>(smem);
-    const uint32_t h = blockIdx.x;
+    // Workgroups go to the eight XCDs in turn: the heads of a KV head to the same one, whose L2 then holds that head's rows once.
+    const uint32_t kvh = blockIdx.x % a.n_kv_heads, h = kvh * (a.n_heads / a.n_kv_heads) + blockIdx.x / a.n_kv_heads;
     const uint32_t qblocks = (n + 63u) / 64u;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, l16 = lane & 15u, g = lane >> 4;
     const uint32_t wave_id = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
-    const uint32_t wave = wave_id & 3u, ksp = (wave_id >> 2) & 1u, half = wave_id >> 3;
+    // (consecutive waves sit on different SIMDs: a block with few queries keeps as many of them busy as it can)
+    const uint32_t wave = (wave_id >> 1) & 3u, ksp = wave_id & 1u, half = wave_id >> 3;
     const uint32_t qb_long = qblocks - 1u - blockIdx.y;
     const uint32_t qb = half == 0 ? qb_long : blockIdx.y;
-    const bool active = half == 0 || qb != qb_long;
     const uint32_t j0 = qb * 64u;
+    const bool active = (half == 0 || qb != qb_long) && j0 + 16u * wave < n;  // the wave has queries
     const uint32_t base = a.d_pos ? *a.d_pos : pos0;
-    const uint32_t kv_dim = a.n_kv_heads * HD, kvh = h / (a.n_heads / a.n_kv_heads);
+    const uint32_t kv_dim = a.n_kv_heads * HD;
     const KV* kbase = static_cast<const KV*>(a.k_cache) + (size_t)kvh * HD;
     const KV* vbase = static_cast<const KV*>(a.v_cache) + (size_t)kvh * HD;
     const uint32_t jq = j0 + 16u * wave + l16;
@@ -1057,13 +1067,10 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(A
 #pragma unroll
         for (int s = 0; s < 2; s++) {
             const float4 v0 = *reinterpret_cast<const float4*>(qp + 32 * s), v1 = *reinterpret_cast<const float4*>(qp + 32 * s + 4);
-            const float f[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                _Float16 hi, lo;
-                split_f16(f[i] * a.scale, hi, lo);
-                qh[s][i] = hi, ql[s][i] = lo;
-            }
+            h4 h0, l0, h1, l1;  // (the scale, 1 / 8, is exact)
+            split_f16(v4f{v0.x * a.scale, v0.y * a.scale, v0.z * a.scale, v0.w * a.scale}, h0, l0);
+            split_f16(v4f{v1.x * a.scale, v1.y * a.scale, v1.z * a.scale, v1.w * a.scale}, h1, l1);
+            qh[s] = __builtin_shufflevector(h0, h1, 0, 1, 2, 3, 4, 5, 6, 7), ql[s] = __builtin_shufflevector(l0, l1, 0, 1, 2, 3, 4, 5, 6, 7);
         }
     }
     v4f o[4];
@@ -1075,7 +1082,7 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(A
     // are -- dealt out to the threads: kk of K and as many of V, or (f16, 1024 threads) one of either.
     constexpr int PPR = LO ? 16 : 8, kPieces = KT * PPR, kBoth = 2 * kPieces / NT, NR = kBoth > 1 ? kBoth / 2 : 1;
     static_assert(kBoth >= 1 && (kBoth == 1 || kBoth % 2 == 0), "every thread moves the same number of pieces");
-    using Piece = typename std::conditional<LO, float4, h8>::type;
+    using Piece = typename std::conditional<LO, v4f, h8>::type;
     struct Regs {
         Piece k[NR], v[NR];  // (v unused where a thread moves one piece)
     };
@@ -1094,22 +1101,21 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(A
             }
         }
     };
-    auto store = [&](Tile& t, const Regs& r) {
+    auto store = [&](Tile& t, Regs& r) {
+        // (Opaque from here on: the compiler would convert the values as soon as it has requested them, and wait for them there.)
+#pragma unroll
+        for (int i = 0; i < NR; i++) {
+            asm volatile("" : "+v"(r.k[i]));
+            if constexpr (kBoth > 1) asm volatile("" : "+v"(r.v[i]));
+        }
 #pragma unroll
         for (int i = 0; i < NR; i++) {
             const uint32_t key = row0 + i * (NT / PPR);
             if constexpr (LO) {
                 const uint32_t vat = 8u * ((piece >> 1) ^ (key & 7u)) + 4u * (piece & 1u);
-                const float kf[4] = {r.k[i].x, r.k[i].y, r.k[i].z, r.k[i].w}, vf[4] = {r.v[i].x, r.v[i].y, r.v[i].z, r.v[i].w};
                 h4 khi, klo, vhi, vlo;
-#pragma unroll
-                for (int e = 0; e < 4; e++) {
-                    _Float16 hi, lo;
-                    split_f16(kf[e], hi, lo);
-                    khi[e] = hi, klo[e] = lo;
-                    split_f16(vf[e], hi, lo);
-                    vhi[e] = hi, vlo[e] = lo;
-                }
+                split_f16(r.k[i], khi, klo);
+                split_f16(r.v[i], vhi, vlo);
                 *reinterpret_cast<h4*>(&t.k[0][key][4 * piece]) = khi;
                 *reinterpret_cast<h4*>(&t.k[PLANES - 1][key][4 * piece]) = klo;
                 *reinterpret_cast<h4*>(&t.v[0][key][vat]) = vhi;
@@ -1194,17 +1200,18 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(A
             for (int c = 0; c < 4; c++) o[c] *= alpha;
         }
         float psum = 0.0f;
-        h8 ph, pl;
+        h4 p_hi[2], p_lo[2];
 #pragma unroll
-        for (int u = 0; u < 2; u++)
+        for (int u = 0; u < 2; u++) {
+            v4f pw;
 #pragma unroll
             for (int r = 0; r < 4; r++) {
-                const float pw = exp_nonpos_hw(sc[u][r] - m_sub);
-                psum += pw;
-                _Float16 hi, lo;
-                split_f16(pw * kPScale, hi, lo);
-                ph[4 * u + r] = hi, pl[4 * u + r] = lo;
+                pw[r] = exp_nonpos_hw(sc[u][r] - m_sub);
+                psum += pw[r];
             }
+            split_f16(pw * kPScale, p_hi[u], p_lo[u]);
+        }
+        const h8 ph = __builtin_shufflevector(p_hi[0], p_hi[1], 0, 1, 2, 3, 4, 5, 6, 7), pl = __builtin_shufflevector(p_lo[0], p_lo[1], 0, 1, 2, 3, 4, 5, 6, 7);
         l_run = __builtin_fmaf(l_run, alpha, psum);
         if constexpr (LO) {
 #pragma unroll
@@ -1218,22 +1225,31 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(A
     // Tile t sits in LDS, t + 1 and t + 2 are on their way in registers: behind the arithmetic of tile t the first goes into the buffer that tile
     // t - 1 left and t + 3 is requested in its place.  One barrier per tile.
     Regs r0, r1;
-    fetch(0, r0);
-    fetch(KT, r1);
-    store(tiles[0], r0);
-    fetch(2 * KT, r0);
+    // (The requests stay in their order, or the waits for one tile would be for all.)
+    const auto request = [&](uint32_t t0, Regs& r) {
+        fetch(t0, r);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const auto next_tile = [&](Tile& t, Regs& r, uint32_t then) {
+        store(t, r);
+        __builtin_amdgcn_sched_barrier(0);
+        request(then, r);
+    };
+    request(0, r0);
+    request(KT, r1);
+    next_tile(tiles[0], r0, 2 * KT);
     __syncthreads();
-    for (uint32_t t0 = 0; t0 <= wg_last; t0 += 2 * KT) {
+    uint32_t t0 = 0;
+    for (; t0 + KT <= wg_last; t0 += 2 * KT) {  // (no way out in the middle: it would make the waits for one tile waits for both)
         attend(tiles[0], t0);
-        store(tiles[1], r1);
-        fetch(t0 + 3 * KT, r1);
+        next_tile(tiles[1], r1, t0 + 3 * KT);
         __syncthreads();
-        if (t0 + KT > wg_last) break;
         attend(tiles[1], t0 + KT);
-        store(tiles[0], r0);
-        fetch(t0 + 4 * KT, r0);
+        next_tile(tiles[0], r0, t0 + 4 * KT);
         __syncthreads();
     }
+    if (t0 <= wg_last) attend(tiles[0], t0);
+    __syncthreads();
     l_run = groups_sum(l_run);
     {
         // the upper-key waves hand (maximum, weight sum, weighted values) to their partners through LDS
