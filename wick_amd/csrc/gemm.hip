@@ -677,6 +677,20 @@ template <int OFF>
 __device__ __forceinline__ void lds_read16(uint32_t addr, v4i& dst) {
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
 }
+template <int OFF>
+__device__ __forceinline__ void lds_read4(uint32_t addr, float& dst) {
+    asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
+}
+// sum += x of lane E of this lane's row of 16, times v. A DPP source is read two wait states after a VALU instruction wrote it at the earliest,
+// which the compiler does not see to in inline code; x is read by a run of these, of which the first, E == 0, waits.
+template <int E>
+__device__ __forceinline__ void fmac_row_lane(float& sum, float x, float v) {
+    if constexpr (E == 0) {
+        asm("s_nop 1\n\tv_fmac_f32_dpp %0, %1, %2 row_newbcast:0 row_mask:0xf bank_mask:0xf" : "+v"(sum) : "v"(x), "v"(v));
+    } else {
+        asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%c3 row_mask:0xf bank_mask:0xf" : "+v"(sum) : "v"(x), "v"(v), "n"(E));
+    }
+}
 // At most N LDS reads outstanding; ties what becomes valid with it.
 template <int N, typename V>
 __device__ __forceinline__ void lds_arrived(V& v) {
@@ -780,7 +794,7 @@ __global__ __launch_bounds__(C::kThreads, C::kOcc) void gemm_tile_kernel(GemmArg
     };
     auto store_dx = [&](uint32_t buf) {
         if (threadIdx.x < (uint32_t)C::kTokens) {
-            const uint32_t at = threadIdx.x ^ 1u;  // neighbours swapped: see the FMA that reads them
+            const uint32_t at = T == 1 ? threadIdx.x : threadIdx.x ^ 1u;  // neighbours swapped: see the FMA that reads them
             sm.dxf[buf][0][at] = dxr.x;
             sm.dxf[buf][1][at] = dxr.y;
             sm.dxf[buf][2][at] = dxr.z;
@@ -803,111 +817,155 @@ __global__ __launch_bounds__(C::kThreads, C::kOcc) void gemm_tile_kernel(GemmArg
     constexpr int kOwn = GATED ? RT / 2 : RT;
     uint32_t a_wt = lds_addr(&sm.st[0].wt[kOwn * wr][kh][0][l32]);
     uint32_t a_dws = lds_addr(&sm.st[0].dws[kOwn * wr][0][l32]);
-    uint32_t a_dxf = lds_addr(&sm.dxf[0][0][32 * TT * wt + 4 * kh]);
+    // token scales: the first of the lane's four groups of four, or (T == 1) the lane of every 16 that holds the scale of their result e reads
+    // that one, 8 (e / 4) + 4 kh + e % 4
+    uint32_t a_dxf = lds_addr(&sm.dxf[0][0][32 * TT * wt + 4 * kh + (T == 1 ? 8 * ((lane & 15u) >> 2) + (lane & 3u) : 0u)]);
     uint32_t a_xt[SB];  // chunk 2 b + kh of this lane's token sits at position chunk ^ swizzle
 #pragma unroll
     for (int b = 0; b < SB; b++) a_xt[b] = lds_addr(&sm.st[0].xt[32 * TT * wt + l32][(2u * b + kh) ^ C::swizzle(l32)]);
     constexpr uint32_t kBuf = sizeof(typename C::Stage);
 
-    v4i A[TT], B[RT];
-    float2 dw[RT];
-    v4f dx[4];
-    v16i D[2];
     constexpr auto granule = [](int rt) { return rt < kOwn ? rt : C::kGranules / 2 + rt - kOwn; };
     // LDS reads of block b of the stage
-    auto read_ab = [&](auto b) {  // TT + RT reads
+    auto read_ab = [&](auto b, v4i (&A)[TT], v4i (&B)[RT]) {  // TT + RT reads
         static_for<TT>([&](auto t) { lds_read16<32 * decltype(t)::value * 32 * SB>(a_xt[decltype(b)::value], A[decltype(t)::value]); });
         static_for<RT>([&](auto r) { lds_read16<1024 * SB * granule(decltype(r)::value) + 512 * decltype(b)::value>(a_wt, B[decltype(r)::value]); });
     };
-    auto read_dw = [&](auto b, auto r) { lds_read8<256 * SB * granule(decltype(r)::value) + 256 * decltype(b)::value>(a_dws, dw[decltype(r)::value]); };
-    auto read_dx = [&](auto b, auto t, auto g) {
-        lds_read16<decltype(b)::value * 4 * C::kTokens + 128 * decltype(t)::value + 32 * decltype(g)::value>(a_dxf, dx[decltype(g)::value]);
+    auto read_dw = [&](auto b, auto r, float2& dw) { lds_read8<256 * SB * granule(decltype(r)::value) + 256 * decltype(b)::value>(a_dws, dw); };
+    [[maybe_unused]] auto read_dx = [&](auto b, auto t, auto g, v4f& dx) {
+        lds_read16<decltype(b)::value * 4 * C::kTokens + 128 * decltype(t)::value + 32 * decltype(g)::value>(a_dxf, dx);
+    };
+    // (parity checks) dot of element e of one result
+    [[maybe_unused]] auto dump = [&](int d, uint32_t rt, uint32_t tt, uint32_t e, uint32_t blk) {
+        const uint32_t row = row0 + GR * (RT * wr + rt) + l32, tok = tok0 + 32 * (TT * wt + tt) + 4 * kh + 8 * (e >> 2) + (e & 3u);
+        if (row < a.m && tok < a.n) {
+            const int v = d - (int)kBiasBits;
+            a.dots[((size_t)tok * a.m + row) * nb + blk] = TYPE == 2 ? v >> 4 : v;  // (type 2: weights were stored x16; exact)
+        }
     };
 
     // One stage: SB blocks, the first of them block blk0 of the row.
     auto compute_stage = [&](uint32_t blk0) {
-        read_ab(Idx<0>{});
-        static_for<RT - 1>([&](auto r) { read_dw(Idx<0>{}, r); });
-        static_for<4>([&](auto g) { read_dx(Idx<0>{}, Idx<0>{}, g); });
-        read_dw(Idx<0>{}, Idx<RT - 1>{});
-        // (the reads behind the operands' may still be in flight)
-        lds_arrived<RT + 4>(A[0]);
-        static_for<TT>([&](auto t) { tie(A[decltype(t)::value]); });
-        static_for<RT>([&](auto r) { tie(B[decltype(r)::value]); });
-        D[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[0], B[0], cbias, 0, 0, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        static_for<SB>([&](auto b_) {
-            constexpr int b = decltype(b_)::value;
-            constexpr bool next = b + 1 < SB;
-            static_for<T>([&](auto t_) {
-                constexpr int t = decltype(t_)::value, tt = t / RT, rt = t % RT;
-                if constexpr (T == 1) {
-                    // one result per wave and block: nothing to run ahead with, the next block's MFMA goes out behind the FMAs
-                } else if constexpr (t + 1 < T) {
-                    constexpr int tt1 = (t + 1) / RT, rt1 = (t + 1) % RT;
-                    D[(t + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[tt1], B[rt1], cbias, 0, 0, 0);
-                } else if constexpr (next) {
-                    lds_arrived<1>(A[0]);  // all operands of the next block; its scale pair of granule RT - 2 may still be on its way
-                    static_for<TT>([&](auto i) { tie(A[decltype(i)::value]); });
-                    static_for<RT>([&](auto i) { tie(B[decltype(i)::value]); });
-                    D[(t + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[0], B[0], cbias, 0, 0, 0);
+        v16i D[2];
+        if constexpr (T == 1) {
+            // One result per wave and block: the operands are read two blocks ahead, the next block's MFMA goes out before this one's FMAs. A
+            // small tile is bound by what it reads from the LDS, 104 bytes per lane and block, 64 of them token scales, which every lane reads
+            // alike: here each lane reads the scale of one of its row's sixteen tokens, 4 bytes, and the FMAs take it from there.
+            v4i A[2][1], B[2][1];
+            float2 dw[2];
+            float xs[2];
+            const auto read_scales = [&](auto b) {
+                constexpr int at = decltype(b)::value;
+                read_dw(b, Idx<0>{}, dw[at & 1]);
+                lds_read4<at * 4 * C::kTokens>(a_dxf, xs[at & 1]);
+            };
+            read_ab(Idx<0>{}, A[0], B[0]), read_scales(Idx<0>{});
+            read_ab(Idx<1>{}, A[1], B[1]), read_scales(Idx<1>{});
+            lds_arrived<6>(A[0][0]), tie(B[0][0]);
+            D[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[0][0], B[0][0], cbias, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            static_for<SB>([&](auto b_) {
+                constexpr int b = decltype(b_)::value, at = b & 1, ahead = b + 2 < SB ? b + 2 : 0;
+                // requested and not waited for yet, in order: scales of b (b == 0), operands of b + 1, scales of b + 1; (b > 0) scales of b first
+                if constexpr (b + 1 < SB) {
+                    lds_arrived<2>(A[at ^ 1][0]), tie(B[at ^ 1][0]), tie(dw[at]), tie(xs[at]);
+                    D[at ^ 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[at ^ 1][0], B[at ^ 1][0], cbias, 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                } else {
+                    lds_arrived<0>(dw[at]), tie(xs[at]);
+                }
+                if constexpr (b + 2 < SB) read_ab(Idx<ahead>{}, A[at], B[at]);
+                v16i& d = D[at];
+                if constexpr (DUMP) {
+#pragma unroll
+                    for (int e = 0; e < 16; e++) dump(d[e], 0, 0, e, blk0 + b);
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 16; e++) d[e] = __float_as_int(__builtin_fmaf(__int_as_float(d[e]), dw[at].x, dw[at].y));
+                    __builtin_amdgcn_sched_barrier(0);
+                    static_for<16>([&](auto e_) {
+                        constexpr int e = decltype(e_)::value;
+                        float sum = acc[0][0][e];
+                        fmac_row_lane<e>(sum, xs[at], __int_as_float(d[e]));
+                        acc[0][0][e] = sum;
+                    });
+                    tie(acc[0][0]);
                 }
                 __builtin_amdgcn_sched_barrier(0);
-                constexpr bool fetch = next && (T == 1 || t == T - 2);  // all MFMAs of this block have been issued
-                if constexpr (fetch) read_ab(Idx<next ? b + 1 : 0>{});
-                constexpr int kFetched = fetch ? TT + RT : 0;  // reads that a wait below may leave outstanding on top
-                if constexpr (rt == RT - 1 && tt == 0) lds_arrived<kFetched + (TT == 1 && RT > 1 && next ? 1 : 0)>(dw[rt]);
-                if constexpr (!DUMP && C::kScaleFirst) {
-                    static_assert(RT > 1, "the granules' scale pairs come ahead of the token scales");
-                    if constexpr (rt == 0 && tt == 0) {
-                        lds_arrived<5 + kFetched>(dw[0]);  // (behind them: the token scales and the last granule's pair)
-                        static_for<RT - 1>([&](auto i) { tie(dw[decltype(i)::value]); });
-                    }
-#pragma unroll
-                    for (int e = 0; e < 16; e++) D[t & 1][e] = __float_as_int(__builtin_fmaf(__int_as_float(D[t & 1][e]), dw[rt].x, dw[rt].y));
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-                static_for<4>([&](auto g_) {
-                    constexpr int g = decltype(g_)::value;
-                    if constexpr (rt == 0) {
-                        lds_arrived<(tt == 0 ? 4 : 3) - g + kFetched>(dx[g]);
-                        if constexpr (!(!DUMP && C::kScaleFirst) && g == 0 && tt == 0) static_for<RT - 1>([&](auto i) { tie(dw[decltype(i)::value]); });
-                    }
-                    if constexpr (DUMP) {
-                        const uint32_t row = row0 + GR * (RT * wr + rt) + l32, tok = tok0 + 32 * (TT * wt + tt) + 4 * kh + 8 * g;
-#pragma unroll
-                        for (int r = 0; r < 4; r++) {
-                            if (row < a.m && tok + r < a.n) {
-                                int v = D[t & 1][4 * g + r] - (int)kBiasBits;
-                                if (TYPE == 2) v >>= 4;  // weights were stored x16; exact
-                                a.dots[((size_t)(tok + r) * a.m + row) * nb + blk0 + b] = v;
-                            }
-                        }
-                    } else {
-#pragma unroll
-                        for (int r = 0; r < 4; r++) {
-                            float v = __int_as_float(D[t & 1][4 * g + r]);
-                            if constexpr (!C::kScaleFirst) v = __builtin_fmaf(v, dw[rt].x, dw[rt].y);
-                            acc[rt][tt][4 * g + r] = __builtin_fmaf(v, dx[g][r ^ 1], acc[rt][tt][4 * g + r]);
-                        }
-                        // (without this the compiler lets the MFMAs of all tiles run ahead of their FMAs, and spills)
-                        if constexpr (!C::kScaleFirst || g == 3) tie(acc[rt][tt]);
-                    }
-                    // this group's token scales are done with: the next token group's, or the next block's first
-                    if constexpr (rt == RT - 1) {
-                        if constexpr (tt + 1 < TT) read_dx(Idx<b>{}, Idx<tt + 1 < TT ? tt + 1 : 0>{}, g_);
-                        else if constexpr (next) read_dx(Idx<next ? b + 1 : b>{}, Idx<0>{}, g_);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                });
-                if constexpr (tt == TT - 1 && next) read_dw(Idx<next ? b + 1 : 0>{}, Idx<rt>{});
-                if constexpr (T == 1 && next) {
-                    lds_arrived<5>(A[0]), tie(B[0]);  // (the scales behind them may still be in flight)
-                    D[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[0], B[0], cbias, 0, 0, 0);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
+                if constexpr (b + 2 < SB) read_scales(Idx<ahead>{});
             });
-        });
+        } else {
+            v4i A[TT], B[RT];
+            float2 dw[RT];
+            v4f dx[4];
+            read_ab(Idx<0>{}, A, B);
+            static_for<RT - 1>([&](auto r) { read_dw(Idx<0>{}, r, dw[decltype(r)::value]); });
+            static_for<4>([&](auto g) { read_dx(Idx<0>{}, Idx<0>{}, g, dx[decltype(g)::value]); });
+            read_dw(Idx<0>{}, Idx<RT - 1>{}, dw[RT - 1]);
+            // (the reads behind the operands' may still be in flight)
+            lds_arrived<RT + 4>(A[0]);
+            static_for<TT>([&](auto t) { tie(A[decltype(t)::value]); });
+            static_for<RT>([&](auto r) { tie(B[decltype(r)::value]); });
+            D[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[0], B[0], cbias, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            static_for<SB>([&](auto b_) {
+                constexpr int b = decltype(b_)::value;
+                constexpr bool next = b + 1 < SB;
+                static_for<T>([&](auto t_) {
+                    constexpr int t = decltype(t_)::value, tt = t / RT, rt = t % RT;
+                    if constexpr (t + 1 < T) {
+                        constexpr int tt1 = (t + 1) / RT, rt1 = (t + 1) % RT;
+                        D[(t + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[tt1], B[rt1], cbias, 0, 0, 0);
+                    } else if constexpr (next) {
+                        lds_arrived<1>(A[0]);  // all operands of the next block; its scale pair of granule RT - 2 may still be on its way
+                        static_for<TT>([&](auto i) { tie(A[decltype(i)::value]); });
+                        static_for<RT>([&](auto i) { tie(B[decltype(i)::value]); });
+                        D[(t + 1) & 1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(A[0], B[0], cbias, 0, 0, 0);
+                    }
+                    __builtin_amdgcn_sched_barrier(0);
+                    constexpr bool fetch = next && t == T - 2;  // all MFMAs of this block have been issued
+                    if constexpr (fetch) read_ab(Idx<next ? b + 1 : 0>{}, A, B);
+                    constexpr int kFetched = fetch ? TT + RT : 0;  // reads that a wait below may leave outstanding on top
+                    if constexpr (rt == RT - 1 && tt == 0) lds_arrived<kFetched + (TT == 1 && next ? 1 : 0)>(dw[rt]);
+                    if constexpr (!DUMP && C::kScaleFirst) {
+                        if constexpr (rt == 0 && tt == 0) {
+                            lds_arrived<5 + kFetched>(dw[0]);  // (behind them: the token scales and the last granule's pair)
+                            static_for<RT - 1>([&](auto i) { tie(dw[decltype(i)::value]); });
+                        }
+#pragma unroll
+                        for (int e = 0; e < 16; e++) D[t & 1][e] = __float_as_int(__builtin_fmaf(__int_as_float(D[t & 1][e]), dw[rt].x, dw[rt].y));
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    static_for<4>([&](auto g_) {
+                        constexpr int g = decltype(g_)::value;
+                        if constexpr (rt == 0) {
+                            lds_arrived<(tt == 0 ? 4 : 3) - g + kFetched>(dx[g]);
+                            if constexpr (!(!DUMP && C::kScaleFirst) && g == 0 && tt == 0) static_for<RT - 1>([&](auto i) { tie(dw[decltype(i)::value]); });
+                        }
+                        if constexpr (DUMP) {
+#pragma unroll
+                            for (int r = 0; r < 4; r++) dump(D[t & 1][4 * g + r], rt, tt, 4 * g + r, blk0 + b);
+                        } else {
+#pragma unroll
+                            for (int r = 0; r < 4; r++) {
+                                float v = __int_as_float(D[t & 1][4 * g + r]);
+                                if constexpr (!C::kScaleFirst) v = __builtin_fmaf(v, dw[rt].x, dw[rt].y);
+                                acc[rt][tt][4 * g + r] = __builtin_fmaf(v, dx[g][r ^ 1], acc[rt][tt][4 * g + r]);
+                            }
+                            // (without this the compiler lets the MFMAs of all tiles run ahead of their FMAs, and spills)
+                            if constexpr (!C::kScaleFirst || g == 3) tie(acc[rt][tt]);
+                        }
+                        // this group's token scales are done with: the next token group's, or the next block's first
+                        if constexpr (rt == RT - 1) {
+                            if constexpr (tt + 1 < TT) read_dx(Idx<b>{}, Idx<tt + 1 < TT ? tt + 1 : 0>{}, g_, dx[g]);
+                            else if constexpr (next) read_dx(Idx<next ? b + 1 : b>{}, Idx<0>{}, g_, dx[g]);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
+                    });
+                    if constexpr (tt == TT - 1 && next) read_dw(Idx<next ? b + 1 : 0>{}, Idx<rt>{}, dw[rt]);
+                });
+            });
+        }
     };
     // The stage's reads are all done (nothing is outstanding past its last wait) and the next stage's copies have landed.
     auto end_stage = [] {
@@ -1400,10 +1458,10 @@ hipError_t launch_reduce(const GemmArgs& a, const Launch& L) {
 }
 
 // The tiles of a launch over a prompt, and what each costs: us per slab (128 elements of K) of a share with 1 .. kPerCu workgroups on a CU, and us
-// per workgroup for filling, draining and storing it -- plain launches first, those with the gate in the epilogue second (0: not
-// built).  Fitted to 130 launches (3072, 2048, 1024 x 1024, 1024 x 4608, 6144, 3072, 2048 x 2048, 2048 x 6912 and gate | up 4608 x 1024,
+// per workgroup for filling, draining and storing it (and 3 us a launch, the same for all) -- plain launches first, those with the gate
+// in the epilogue second (0: not built).  Fitted to 130 launches (3072, 2048, 1024 x 1024, 1024 x 4608, 6144, 3072, 2048 x 2048, 2048 x 6912 and gate | up 4608 x 1024,
 // 6912 x 2048, each over 80 .. 2048 tokens, weights and activations of random bits: a launch that keeps the chip busy runs at the
-// power limit), which they meet to 4 % rms; the tile they choose is 1 % behind the best of all.  A launch is workgroups on 256 CUs, kPerCu
+// power limit), which they meet to 5 % rms; the tile they choose is 0.3 % behind the best of the six.  A launch is workgroups on 256 CUs, kPerCu
 // at a time, and what the last round leaves idle is what separates the tiles: large ones do more per operand byte, small ones leave
 // less over, and a CU with a single workgroup on it wants that one's waves to be many.
 struct TileCost {
@@ -1411,27 +1469,27 @@ struct TileCost {
 };
 struct TileL : T32<4, 2, 2, 2, 2, 2, true> {  // 256 x 128, 4 waves of 128 x 64
     static constexpr int kPerCu = 2;
-    static constexpr TileCost kCost[2] = {{{3.07f, 3.81f}, 5.15f}, {{3.14f, 3.88f}, 4.76f}};
+    static constexpr TileCost kCost[2] = {{{3.10f, 4.36f}, 2.10f}, {{3.11f, 4.04f}, 6.63f}};
 };
 struct TileX : T32<2, 2, 2, 2, 2, 3> {  // 128 x 128, 4 waves of 64 x 64
     static constexpr int kPerCu = 3;
-    static constexpr TileCost kCost[2] = {{{1.79f, 2.31f, 3.30f}, 1.50f}, {{1.47f, 2.25f, 3.32f}, 2.30f}};
+    static constexpr TileCost kCost[2] = {{{1.79f, 2.38f, 3.42f}, 1.43f}, {{1.83f, 2.24f, 3.26f}, 2.59f}};
 };
 struct TileS : T32<2, 1, 2, 2, 4, 2> {  // 128 x 64, 4 waves of 64 x 32
     static constexpr int kPerCu = 2;
-    static constexpr TileCost kCost[2] = {{{0.94f, 1.30f}, 1.22f}, {{0.89f, 1.31f}, 1.70f}};
+    static constexpr TileCost kCost[2] = {{{0.94f, 1.32f}, 1.25f}, {{0.99f, 1.35f}, 1.25f}};
 };
 struct TileQ : T32<2, 1, 2, 2, 2, 4> {  // the same with half a slab per stage: four of them on a CU
     static constexpr int kPerCu = 4;
-    static constexpr TileCost kCost[2] = {{{1.29f, 1.62f, 1.97f, 2.47f}, 1.41f}, {{1.14f, 1.66f, 1.95f, 2.53f}, 1.13f}};
+    static constexpr TileCost kCost[2] = {{{1.28f, 1.64f, 2.04f, 2.56f}, 1.32f}, {{1.32f, 1.62f, 2.07f, 2.55f}, 1.48f}};
 };
 struct TileN : T32<1, 1, 4, 2, 4, 4> {  // 128 x 64, 8 waves of 32 x 32
     static constexpr int kPerCu = 2;
-    static constexpr TileCost kCost[2] = {{{0.80f, 1.31f}, 1.37f}, {}};
+    static constexpr TileCost kCost[2] = {{{0.70f, 1.25f}, 1.53f}, {}};
 };
 struct TileH : T32<1, 1, 2, 2, 4, 4> {  // 64 x 64, 4 waves of 32 x 32
     static constexpr int kPerCu = 4;
-    static constexpr TileCost kCost[2] = {{{0.68f, 0.82f, 1.10f, 1.42f}, 0.64f}, {}};
+    static constexpr TileCost kCost[2] = {{{0.53f, 0.76f, 1.06f, 1.32f}, 0.73f}, {}};
 };
 template <typename C>
 float tile_cost(uint64_t row_tiles, uint32_t n, uint32_t k, uint32_t shares, bool gated = false) {
