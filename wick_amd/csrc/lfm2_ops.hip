@@ -1518,98 +1518,77 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(float* __restrict__ gate,
 
 // ---- normalise / gate and quantize in one pass (prompt passes) -----------------------------------
 // What rmsnorm_kernel followed by the Q8_0 quantizer compute (wick/src/backend/cpu.rs:577-594, wick/src/backend/simd.rs:255-323),
-// bit for bit, without the f32 round trip through memory: the sum of squares is taken over the same elements per thread
-// and in the same order as rmsnorm_kernel does, the normalised values are formed by the same two products, and eight
-// lanes own one 32-element block exactly as in the quantizer.  One block per row; dim % 32 == 0, rows 16-byte aligned.
-__global__ __launch_bounds__(256) void rmsnorm_quantize_kernel(const float* __restrict__ x, const float* __restrict__ weight, int8_t* __restrict__ q,
+// bit for bit, without the f32 round trip through memory: thread t sums the squares of elements t, t + 256, .. in order, as
+// rmsnorm_kernel does, the normalised values are formed by the same two products, and eight lanes own one 32-element block exactly as in
+// the quantizer.  One workgroup per row; dim % 32 == 0, rows 16-byte aligned.
+//
+// S > 0: the S K shares of a split projection ([S][rows][dim]) are added onto the residual row first, which is written back: what
+// gemm_splitk_reduce_kernel (accumulating) leaves, the shares summed in ascending order and then added to x.
+//
+// Q: the row has at most 1024 Q elements and is kept in LDS for the quantizer, four elements of it and their weights per thread and
+// 1024.  Latency bounds it: everything is requested in one go, so that a row is one round trip to memory and not two (three with the
+// weights), and the LDS holds no more than the row, so that eight rows fit a CU and 2048 are one round.  Q = 0: rows of any length, read
+// a second time from memory.
+template <int S, int Q>
+__global__ __launch_bounds__(256) void rmsnorm_quantize_kernel(typename std::conditional<S != 0, float*, const float*>::type __restrict__ x,
+                                                               const float* __restrict__ partial, size_t share_stride,
+                                                               const float* __restrict__ weight, int8_t* __restrict__ q,
                                                                float* __restrict__ scales, uint32_t dim, uint32_t x_stride, float eps) {
-    __shared__ double slots[16];
-    const float* xr = x + (size_t)blockIdx.x * x_stride;
-    const double inv_dim = 1.0 / (double)dim;  // while the loads are under way
-    double s = 0.0;
-    for (uint32_t i0 = threadIdx.x; i0 < dim; i0 += 4u * 256u) {  // four loads in flight; elements t, t + 256, .. in order, as rmsnorm_kernel sums them
-        float xv[4];
-#pragma unroll
-        for (int j = 0; j < 4; j++) xv[j] = xr[i0 + 256u * j < dim ? i0 + 256u * j : i0];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            if (i0 + 256u * j < dim) {
-                const double v = (double)xv[j];
-                s += v * v;
-            }
-        }
-    }
-    const double total = block_sum_f64(s, slots);
-    const float inv_rms = rms_inverse(total, inv_dim, eps);
-    const uint32_t quads = dim >> 2;
-    for (uint32_t quad0 = 0; quad0 < quads; quad0 += blockDim.x) {  // groups of 8 lanes stay together: quads % 8 == 0
-        const uint32_t quad = quad0 + threadIdx.x;
-        const bool live = quad < quads;
-        const uint32_t qd = live ? quad : 0;
-        const float4 v = reinterpret_cast<const float4*>(xr)[qd];
-        const float4 w = reinterpret_cast<const float4*>(weight)[qd];
-        const float v0 = __fmul_rn(__fmul_rn(v.x, inv_rms), w.x), v1 = __fmul_rn(__fmul_rn(v.y, inv_rms), w.y);
-        const float v2 = __fmul_rn(__fmul_rn(v.z, inv_rms), w.z), v3 = __fmul_rn(__fmul_rn(v.w, inv_rms), w.w);
-        float amax = fmaxf(fmaxf(fabsf(v0), fabsf(v1)), fmaxf(fabsf(v2), fabsf(v3)));
-        amax = group_max8(amax);
-        float id;
-        const float scale = q8_scale_and_inverse(amax, id);
-        const uint32_t packed = q8_pack4(v0, v1, v2, v3, id);
-        if (live) {
-            *reinterpret_cast<uint32_t*>(q + (size_t)blockIdx.x * dim + 4u * quad) = packed;
-            if ((quad & 7u) == 0) scales[(size_t)blockIdx.x * (dim >> 5) + (quad >> 3)] = scale;
-        }
-    }
-}
-
-// The K shares of a split projection added onto the residual rows, then rmsnorm_quantize_kernel of the updated rows, bit for bit
-// what gemm_splitk_reduce_kernel (accumulating) followed by rmsnorm_quantize_kernel leave: the shares are summed in ascending
-// order and then added to x; thread t covers the same elements t, t + 256, .. in the same order for the f64 sum of squares.  The
-// updated row is written back and kept in LDS for the quantizer's pass.  partial: [splits][rows][dim].
-template <int S>
-__global__ __launch_bounds__(256) void residual_rmsnorm_quantize_kernel(float* __restrict__ x, const float* __restrict__ partial, size_t share_stride,
-                                                                        const float* __restrict__ weight, int8_t* __restrict__ q,
-                                                                        float* __restrict__ scales, uint32_t dim, uint32_t x_stride, float eps) {
-    __shared__ double slots[16];
-    __shared__ __align__(16) float row[kResidualNormMaxDim];
-    float* xr = x + (size_t)blockIdx.x * x_stride;
+    static_assert(S == 0 || Q > 0, "the updated row is kept");
+    __shared__ double slots[4];
+    __shared__ __align__(16) float row[Q ? 1024 * Q : 4];
+    auto* const xr = x + (size_t)blockIdx.x * x_stride;
     const float* pr = partial + (size_t)blockIdx.x * dim;
+    const uint32_t quads = dim >> 2;
+    constexpr int W = Q == 1 || Q == 2 ? Q : 1;  // quads of weights requested ahead
+    float4 w[W];
+    if constexpr (Q == 1 || Q == 2) {
+#pragma unroll
+        for (int j = 0; j < W; j++) w[j] = reinterpret_cast<const float4*>(weight)[min(threadIdx.x + 256u * j, quads - 1u)];
+    }
     const double inv_dim = 1.0 / (double)dim;  // while the loads are under way
     double s = 0.0;
-    for (uint32_t i0 = threadIdx.x; i0 < dim; i0 += 4u * 256u) {  // four elements' loads (S + 1 each) in flight together
-        float xv[4], pv[4][S];
+    // four elements' loads (S + 1 each) in flight together, eight of a row kept in eight
+    constexpr uint32_t E = Q == 2 ? 8 : 4;
+    for (uint32_t i0 = threadIdx.x; i0 < dim; i0 += E * 256u) {
+        float xv[E], pv[E][S ? S : 1];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (uint32_t j = 0; j < E; j++) {
             const uint32_t i = i0 + 256u * j < dim ? i0 + 256u * j : i0;
             xv[j] = xr[i];
 #pragma unroll
             for (int p = 0; p < S; p++) pv[j][p] = pr[(size_t)p * share_stride + i];
         }
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
+        for (uint32_t j = 0; j < E; j++) {
             const uint32_t i = i0 + 256u * j;
             if (i < dim) {
-                float sum = pv[j][0];
+                float h = xv[j];
+                if constexpr (S != 0) {
+                    float sum = pv[j][0];
 #pragma unroll
-                for (int p = 1; p < S; p++) sum += pv[j][p];
-                const float h = xv[j] + sum;
-                xr[i] = h, row[i] = h;
+                    for (int p = 1; p < S; p++) sum += pv[j][p];
+                    h += sum;
+                    xr[i] = h;
+                }
+                if constexpr (Q != 0) row[i] = h;
                 const double v = (double)h;
                 s += v * v;
             }
         }
     }
-    const double total = block_sum_f64(s, slots);  // its barriers also publish row[]
+    s = wave_sum_f64(s);
+    if ((threadIdx.x & 63u) == 0) slots[threadIdx.x >> 6] = s;
+    __syncthreads();  // publishes row[] as well
+    double total = 0.0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) total += slots[i];
     const float inv_rms = rms_inverse(total, inv_dim, eps);
-    const uint32_t quads = dim >> 2;
-    for (uint32_t quad0 = 0; quad0 < quads; quad0 += blockDim.x) {
-        const uint32_t quad = quad0 + threadIdx.x;
+    const auto quantize = [&](uint32_t quad, const float4& w4) {  // groups of 8 lanes stay together: quads % 8 == 0
         const bool live = quad < quads;
-        const uint32_t qd = live ? quad : 0;
-        const float4 v = reinterpret_cast<const float4*>(row)[qd];
-        const float4 w = reinterpret_cast<const float4*>(weight)[qd];
-        const float v0 = __fmul_rn(__fmul_rn(v.x, inv_rms), w.x), v1 = __fmul_rn(__fmul_rn(v.y, inv_rms), w.y);
-        const float v2 = __fmul_rn(__fmul_rn(v.z, inv_rms), w.z), v3 = __fmul_rn(__fmul_rn(v.w, inv_rms), w.w);
+        const float4 v = reinterpret_cast<const float4*>(Q ? row : xr)[live ? quad : 0];
+        const float v0 = __fmul_rn(__fmul_rn(v.x, inv_rms), w4.x), v1 = __fmul_rn(__fmul_rn(v.y, inv_rms), w4.y);
+        const float v2 = __fmul_rn(__fmul_rn(v.z, inv_rms), w4.z), v3 = __fmul_rn(__fmul_rn(v.w, inv_rms), w4.w);
         float amax = fmaxf(fmaxf(fabsf(v0), fabsf(v1)), fmaxf(fabsf(v2), fabsf(v3)));
         amax = group_max8(amax);
         float id;
@@ -1619,6 +1598,12 @@ __global__ __launch_bounds__(256) void residual_rmsnorm_quantize_kernel(float* _
             *reinterpret_cast<uint32_t*>(q + (size_t)blockIdx.x * dim + 4u * quad) = packed;
             if ((quad & 7u) == 0) scales[(size_t)blockIdx.x * (dim >> 5) + (quad >> 3)] = scale;
         }
+    };
+    if constexpr (Q == 1 || Q == 2) {
+#pragma unroll
+        for (int j = 0; j < W; j++) quantize(threadIdx.x + 256u * j, w[j]);
+    } else {
+        for (uint32_t quad0 = 0; quad0 < quads; quad0 += 256u) quantize(quad0 + threadIdx.x, reinterpret_cast<const float4*>(weight)[min(quad0 + threadIdx.x, quads - 1u)]);
     }
 }
 
@@ -2029,22 +2014,39 @@ hipError_t launch_attention_prefill(const float* d_q, const void* d_k_cache, con
     });
 }
 
+// go(Q) for rows of dim elements (rmsnorm_quantize_kernel); 0: longer than it keeps
+template <typename Go>
+hipError_t with_row_quads(uint32_t dim, Go&& go) {
+    if (dim <= 1024u) return go(std::integral_constant<int, 1>{});
+    if (dim <= 2048u) return go(std::integral_constant<int, 2>{});
+    if (dim <= kResidualNormMaxDim) return go(std::integral_constant<int, (int)(kResidualNormMaxDim / 1024u)>{});
+    return go(std::integral_constant<int, 0>{});
+}
+
 hipError_t launch_rmsnorm_quantize(const float* d_x, const float* d_weight, uint32_t rows, uint32_t dim, uint32_t x_stride, float eps, int8_t* d_q,
                                    float* d_scales, const Launch& L) {
     if (rows == 0) return hipSuccess;
-    return launch_kernel(L, kFamQuantize, rmsnorm_quantize_kernel, dim3(rows), dim3(256), d_x, d_weight, d_q, d_scales, dim, x_stride, eps);
+    return with_row_quads(dim, [&](auto quads) {
+        return launch_kernel(L, kFamQuantize, rmsnorm_quantize_kernel<0, decltype(quads)::value>, dim3(rows), dim3(256), d_x, (const float*)nullptr, (size_t)0,
+                             d_weight, d_q, d_scales, dim, x_stride, eps);
+    });
 }
 
 hipError_t launch_residual_rmsnorm_quantize(float* d_x, const float* d_partial, uint32_t splits, const float* d_weight, uint32_t rows, uint32_t dim,
                                             uint32_t x_stride, float eps, int8_t* d_q, float* d_scales, const Launch& L) {
     if (rows == 0) return hipSuccess;
-    if (dim > kResidualNormMaxDim) return hipErrorInvalidValue;
-    const auto go = [&](auto kernel) {
-        return launch_kernel(L, kFamQuantize, kernel, dim3(rows), dim3(256), d_x, d_partial, (size_t)rows * dim, d_weight, d_q, d_scales, dim, x_stride, eps);
+    const auto go = [&](auto shares) {
+        return with_row_quads(dim, [&](auto quads) -> hipError_t {
+            constexpr int S = decltype(shares)::value, Q = decltype(quads)::value;
+            if constexpr (Q == 0) return hipErrorInvalidValue;
+            else
+                return launch_kernel(L, kFamQuantize, rmsnorm_quantize_kernel<S, Q>, dim3(rows), dim3(256), d_x, d_partial, (size_t)rows * dim, d_weight, d_q,
+                                     d_scales, dim, x_stride, eps);
+        });
     };
-    if (splits == 2) return go(residual_rmsnorm_quantize_kernel<2>);
-    if (splits == 4) return go(residual_rmsnorm_quantize_kernel<4>);
-    if (splits == 8) return go(residual_rmsnorm_quantize_kernel<8>);
+    if (splits == 2) return go(std::integral_constant<int, 2>{});
+    if (splits == 4) return go(std::integral_constant<int, 4>{});
+    if (splits == 8) return go(std::integral_constant<int, 8>{});
     return hipErrorInvalidValue;  // the K split makes 2, 4 or 8 shares
 }
 
