@@ -290,6 +290,13 @@ def test_qk_norm_rope_of_a_prompt(ctx, ops, oracle, n_heads, n_kv, hd, pos0, n, 
     d_qn.free(), d_kn.free()
 
 
+@pytest.mark.parametrize("n_heads,n_kv,pos0,n,pad", [(6, 3, 5, 7, 4),     # 9 heads: fours of heads that hold both kinds, one of a single head; odd tokens
+                                                     (30, 10, 4089, 2, 0),  # more heads than a workgroup has in flight; up to the cache's last row
+                                                     (4, 2, 0, 3, 2)])      # rows not 16-byte aligned: the kernel of other head sizes
+def test_qk_norm_rope_of_a_prompt_64(ctx, ops, oracle, n_heads, n_kv, pos0, n, pad):
+    test_qk_norm_rope_of_a_prompt(ctx, ops, oracle, n_heads, n_kv, 64, pos0, n, pad)
+
+
 # contexts of <= 256 positions (and head_dim 96) run the one-workgroup kernel, longer ones the sequence-split kernel;
 # 20000 positions make every workgroup walk several chunks
 @pytest.mark.parametrize("n_heads,n_kv,hd,seq", [(4, 2, 64, 1), (16, 8, 64, 10), (16, 8, 64, 253), (16, 8, 64, 257), (8, 2, 64, 1500), (4, 4, 32, 33),
