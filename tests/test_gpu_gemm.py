@@ -591,3 +591,33 @@ def test_the_gated_launch_starts_past_256_tiles(ctx, oracle, m, n, k):
         for b in (d_q, d_s, d_g, d_u, d_oq, d_os):
             b.free()
     ws[0].free(), ws[1].free()
+
+
+@pytest.mark.parametrize("dtype", [W.Q4_0, W.Q8_0])
+def test_the_gate_in_the_launch_over_all_magnitudes(ctx, oracle, dtype):
+    """The launch's own silu takes gates of 2^-60 .. 41 in a shorter way than the others: groups of 32 tokens whose gates lie inside, across
+    either end and outside (tiny, subnormal, zero, huge, infinite), the same bits as the separate launches."""
+    from wick_amd.lfm2 import Lfm2Ops
+
+    m, n, k = 2112, 1030, 128
+    ops = Lfm2Ops(ctx)
+    ws = [ctx.upload_weight(oracle.synth_weight(dtype, m, k, seed=51 + i), dtype, m, k) for i in range(2)]
+    assert ops.ffn_gate_up_silu_quantize_applies(ws[0], ws[1], n)
+    s, q = oracle.quantize_q8_0_batch(oracle.fill_normal(10, 1.0, n * k), n, k)
+    unit = oracle.gemm_q8(dtype, oracle.synth_weight(dtype, m, k, seed=51), s, q, m, n, k).std()  # a gate of factor 1 is one of this size
+    factors = np.array([1, 3, 9, 13, 20, 45, 1e3, 1e-2, 1e-6, 1e-12, 1e-17, 1e-18, 1e-19, 1e-22, 1e-30, 1e-38, 0, 1e20, 1e30, 3e38], np.float32)
+    s = np.minimum(s.reshape(n, -1) * (factors[np.arange(n) // 32 % factors.size].astype(np.float64) / unit)[:, None], 3e38).astype(np.float32)
+    d_q, d_s, out = ctx.to_device(q), ctx.to_device(s), []
+    d_g, d_u, d_oq, d_os = ctx.alloc(n * m * 4), ctx.alloc(n * m * 4), ctx.alloc(n * m), ctx.alloc(n * (m // 32) * 4)
+    for gated in (True, False):
+        if gated:
+            ops.encode_ffn_gate_up_silu_quantize(ws[0], ws[1], d_s, d_q, n, d_oq, d_os)
+        else:
+            ctx.gemm_preq_multi(ws, d_s, d_q, n, [d_g, d_u], m)
+            ops.silu_mul_quantize(d_g, d_u, n, m, d_oq, d_os)
+        out.append((d_oq.download(np.uint8, n * m), d_os.download(np.uint32, n * (m // 32))))
+    g = np.abs(d_g.download(np.float32, n * m).reshape(n, m))
+    assert (g[:32] < 41).all() and (g == 0).any() and np.isinf(g[~np.isnan(g)]).any()
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
+    for b in (d_q, d_s, d_g, d_u, d_oq, d_os, *ws):
+        b.free()

@@ -999,7 +999,9 @@ __global__ __launch_bounds__(C::kThreads, C::kOcc) void gemm_tile_kernel(GemmArg
         // silu(gate) * up and the Q8_0 quantizer, element for element what silu_mul_quantize_kernel computes from the two float
         // results: granules 0 .. RT / 2 - 1 of the wave are gate rows, the others the same rows of up, 32 rows = one Q8_0 block of a
         // token.  The gated values go through a wave-private piece of LDS (the stages are done with), so that eight lanes own a block
-        // with four rows each: one scale per block and eight lanes instead of 32, and 4-byte stores.
+        // with four rows each: one scale per block and eight lanes instead of 32, and 4-byte stores.  It is bound by its instructions: with
+        // the shorter silu (silu_mul_near) and a quarter of the scales' divisions per lane, 4608 x 1024 over 555 tokens 24.8 -> 23.0 us,
+        // 6912 x 2048 over 2002 155 -> 152.5.
         constexpr int kRow = 36;  // floats per token row: 16-byte aligned, neighbouring tokens on other banks
         static_assert(sizeof(sm) >= sizeof(float) * kRow * 32 * C::kWaves, "a 32 x 32 block of floats per wave");
         float* const h = reinterpret_cast<float*>(&sm) + kRow * 32 * wave;
@@ -1007,15 +1009,10 @@ __global__ __launch_bounds__(C::kThreads, C::kOcc) void gemm_tile_kernel(GemmArg
         for (int j = 0; j < kOwn; j++)
 #pragma unroll
             for (int tt = 0; tt < TT; tt++) {
-                float v[16], far = 0.0f;
+                float v[16], far = 0.0f, small = 1.0f;
 #pragma unroll
-                for (int e = 0; e < 16; e++) {
-                    float n;
-                    const float ex = ggml_expf_near(-acc[j][tt][e], n);
-                    far = fmaxf(far, fabsf(n));
-                    v[e] = __fmul_rn(__fdiv_rn(acc[j][tt][e], __fadd_rn(1.0f, ex)), acc[kOwn + j][tt][e]);
-                }
-                if (__builtin_amdgcn_ballot_w64(!(far <= 126.0f)) != 0) {  // a lane outside the short branch of the exponential (or not a number)
+                for (int e = 0; e < 16; e++) v[e] = silu_mul_near(acc[j][tt][e], acc[kOwn + j][tt][e], far, small);
+                if (__builtin_amdgcn_ballot_w64(!silu_mul_was_near(far, small)) != 0) {  // some lane outside what that takes
 #pragma unroll
                     for (int e = 0; e < 16; e++) v[e] = silu_mul(acc[j][tt][e], acc[kOwn + j][tt][e]);
                 }
@@ -1023,18 +1020,24 @@ __global__ __launch_bounds__(C::kThreads, C::kOcc) void gemm_tile_kernel(GemmArg
                 for (int e = 0; e < 16; e++) h[kRow * (4 * kh + 8 * (e >> 2) + (e & 3)) + l32] = v[e];
                 const uint32_t rbase = row0 + 32u * (kOwn * wr + j);
                 if (rbase < a.m) {  // m % 32 == 0: a block is inside the matrix or not at all
+                    // Eight lanes have four tokens' blocks: each lane works out the scale of one of the four and hands its inverse round.
+                    float4 x[4];
+                    float amax[4];
 #pragma unroll
                     for (int i = 0; i < 4; i++) {
-                        const uint32_t t = 8u * i + (lane >> 3), tok = tok0 + 32 * (TT * wt + tt) + t;
-                        const float4 x = *reinterpret_cast<const float4*>(&h[kRow * t + 4u * (lane & 7u)]);
-                        float id;
-                        const float scale = q8_scale_and_inverse(group_max8(fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w)))), id);
-                        const uint32_t packed = q8_pack4(x.x, x.y, x.z, x.w, id);
-                        if (tok < a.n) {
-                            *reinterpret_cast<uint32_t*>(a.q_out + (size_t)tok * a.m + rbase + 4u * (lane & 7u)) = packed;
-                            if ((lane & 7u) == 0) a.s_out[(size_t)tok * (a.m >> 5) + (rbase >> 5)] = scale;
-                        }
+                        x[i] = *reinterpret_cast<const float4*>(&h[kRow * (8u * i + (lane >> 3)) + 4u * (lane & 7u)]);
+                        amax[i] = group_max8(fmaxf(fmaxf(fabsf(x[i].x), fabsf(x[i].y)), fmaxf(fabsf(x[i].z), fabsf(x[i].w))));
                     }
+                    const uint32_t mine = lane & 3u, tok = tok0 + 32 * (TT * wt + tt) + (lane >> 3);
+                    float id;
+                    const float scale = q8_scale_and_inverse(mine < 2u ? (mine == 0u ? amax[0] : amax[1]) : (mine == 2u ? amax[2] : amax[3]), id);
+                    if ((lane & 7u) < 4u && tok + 8u * mine < a.n) a.s_out[(size_t)(tok + 8u * mine) * (a.m >> 5) + (rbase >> 5)] = scale;
+                    static_for<4>([&](auto i_) {
+                        constexpr int i = decltype(i_)::value;
+                        const float idi = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(id), 0x55 * i, 0xf, 0xf, false));  // of lane i of the four
+                        const uint32_t packed = q8_pack4(x[i].x, x[i].y, x[i].z, x[i].w, idi);
+                        if (tok + 8u * i < a.n) *reinterpret_cast<uint32_t*>(a.q_out + (size_t)(tok + 8u * i) * a.m + rbase + 4u * (lane & 7u)) = packed;
+                    });
                 }
             }
     } else if constexpr (!DUMP) {
@@ -1469,19 +1472,19 @@ struct TileCost {
 };
 struct TileL : T32<4, 2, 2, 2, 2, 2, true> {  // 256 x 128, 4 waves of 128 x 64
     static constexpr int kPerCu = 2;
-    static constexpr TileCost kCost[2] = {{{3.10f, 4.36f}, 2.10f}, {{3.11f, 4.04f}, 6.63f}};
+    static constexpr TileCost kCost[2] = {{{3.10f, 4.36f}, 2.10f}, {{3.06f, 4.00f}, 6.15f}};
 };
 struct TileX : T32<2, 2, 2, 2, 2, 3> {  // 128 x 128, 4 waves of 64 x 64
     static constexpr int kPerCu = 3;
-    static constexpr TileCost kCost[2] = {{{1.79f, 2.38f, 3.42f}, 1.43f}, {{1.83f, 2.24f, 3.26f}, 2.59f}};
+    static constexpr TileCost kCost[2] = {{{1.79f, 2.38f, 3.42f}, 1.43f}, {{1.79f, 2.23f, 3.27f}, 2.24f}};
 };
 struct TileS : T32<2, 1, 2, 2, 4, 2> {  // 128 x 64, 4 waves of 64 x 32
     static constexpr int kPerCu = 2;
-    static constexpr TileCost kCost[2] = {{{0.94f, 1.32f}, 1.25f}, {{0.99f, 1.35f}, 1.25f}};
+    static constexpr TileCost kCost[2] = {{{0.94f, 1.32f}, 1.25f}, {{0.99f, 1.37f}, 0.92f}};
 };
 struct TileQ : T32<2, 1, 2, 2, 2, 4> {  // the same with half a slab per stage: four of them on a CU
     static constexpr int kPerCu = 4;
-    static constexpr TileCost kCost[2] = {{{1.28f, 1.64f, 2.04f, 2.56f}, 1.32f}, {{1.32f, 1.62f, 2.07f, 2.55f}, 1.48f}};
+    static constexpr TileCost kCost[2] = {{{1.28f, 1.64f, 2.04f, 2.56f}, 1.32f}, {{1.31f, 1.66f, 2.03f, 2.61f}, 0.93f}};
 };
 struct TileN : T32<1, 1, 4, 2, 4, 4> {  // 128 x 64, 8 waves of 32 x 32
     static constexpr int kPerCu = 2;

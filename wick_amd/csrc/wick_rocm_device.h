@@ -293,14 +293,28 @@ __device__ __forceinline__ float ggml_expf(float x) {
     const float s2 = bits_f(p.e - d);
     return __fmul_rn(__fadd_rn(s2, __fmul_rn(s2, p.j)), s1);
 }
-// Its first branch alone: the value where |n| <= 126.  For code that takes many of them and branches once on the largest |n|.
-__device__ __forceinline__ float ggml_expf_near(float x, float& n) {
-    const GgmlExp p = ggml_expf_parts(x);
-    n = p.n;
-    return __fadd_rn(p.k, __fmul_rn(p.j, p.k));
-}
-
 // silu_mul_inplace's element (wick/src/backend/cpu.rs:668-673): g / (1 + expf(-g)) * u, bit-exact.
 __device__ __forceinline__ float silu_mul(float g, float u) { return __fmul_rn(__fdiv_rn(g, __fadd_rn(1.0f, ggml_expf(-g))), u); }
+
+// The same bits in some thirty instructions instead of forty, for 2^-60 <= |g| and |n| <= 60 (|g| < 41) alone: for code that takes many of
+// them and asks once, by far and small over all of them (0 and 1 at first), whether they were.  There
+//   n LN2_HI (6 + 15 bits) and j k (k a power of two) are exact, so that a fused operation rounds as the separate ones do, and
+//   g / (1 + e^-g) needs neither scaling nor special cases: a Newton step on the hardware's reciprocal and two corrections by the exact
+//   remainder, the last of which rounds correctly (Markstein 1990).
+__device__ __forceinline__ float silu_mul_near(float g, float u, float& far, float& small) {
+    const float x = -g, R = bits_f(0x4B400000u);
+    const float z = __fadd_rn(R, __fmul_rn(x, bits_f(0x3FB8AA3Bu)));
+    const float n = __fsub_rn(z, R);
+    const float b = __fsub_rn(__builtin_fmaf(-n, bits_f(0x3F317200u), x), __fmul_rn(n, bits_f(0x35BFBE8Eu)));
+    const float k = bits_f((__float_as_uint(z) << 23) + 0x3F800000u), b2 = __fmul_rn(b, b);
+    const float lo = __fadd_rn(bits_f(0x3EFFFEDBu), __fmul_rn(bits_f(0x3E2AAF33u), b)), hi = __fadd_rn(bits_f(0x3D2B9F17u), __fmul_rn(bits_f(0x3C072010u), b));
+    const float j = __fadd_rn(__fmul_rn(bits_f(0x3F7FFFF6u), b), __fmul_rn(__fadd_rn(lo, __fmul_rn(hi, b2)), b2));
+    const float d = __fadd_rn(1.0f, __builtin_fmaf(j, k, k));
+    const float y0 = __builtin_amdgcn_rcpf(d), y = __builtin_fmaf(__builtin_fmaf(-d, y0, 1.0f), y0, y0);
+    const float q0 = __fmul_rn(g, y), q1 = __builtin_fmaf(__builtin_fmaf(-d, q0, g), y, q0);
+    far = fmaxf(far, fabsf(n)), small = fminf(small, fabsf(g));
+    return __fmul_rn(__builtin_fmaf(__builtin_fmaf(-d, q1, g), y, q1), u);
+}
+__device__ __forceinline__ bool silu_mul_was_near(float far, float small) { return far <= 60.0f && small >= 0x1p-60f; }
 
 }  // namespace wick_rocm
