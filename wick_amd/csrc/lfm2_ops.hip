@@ -990,24 +990,31 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // a_hi b_hi + a_hi b_lo + a_lo b_hi, each an exact f16 x f16 product accumulated in f32 by v_mfma_f32_16x16x32_f16 (the
 // dropped a_lo b_lo term is below 2^-22 of the product).  Three MFMAs of K = 32 in 16 cycles each replace eight f32 MFMAs
 // of K = 4 in 32 cycles each: the matrix time drops by a factor of five and the kernel becomes bound by the softmax's
-// vector work.  K tiles sit in LDS as f16 hi / lo rows, V tiles transposed ([dim][key]) so that the second product's A
-// operand (V^T: 8 keys of one dim per lane) is two 8-byte reads; the softmax weights are scaled by 2^12 before the
-// split (exact, undone at the end) so that small weights keep their bits in f16.  Slot j of lane group g stands for
+// vector work.  K and V tiles sit in LDS as f16 hi / lo rows; the second product's A operand (V^T: 8 keys of one dim per lane) is two
+// reads that transpose on the way (ds_read_b64_tr_b16); the softmax weights are scaled by 2^12 before the
+// split (exact, undone at the end) so that small weights keep their bits in f16.  What a tile costs is spread evenly: of 88 us a launch
+// (2048 tokens behind 0 .. 6144 on f16 rows) the second product is 12, the exponentials, the split of the weights and the tile's copy 7
+// each -- all of it instructions, which is why each of them is counted here.  Slot j of lane group g stands for
 // key 4 g + j of the wave's first 16-key sub-tile (j < 4) or of its second (j >= 4) in both operands of the second
 // product, which is again exactly how the first product leaves the weights in the registers.
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 
-// Four values at a time: two conversions of a pair, not one of each value and one of the pair.
+// hi = f16(x), lo = f16(x - hi) of four values x = y * SCALE (a power of two).  The product and the difference are exact, so that each half
+// is one fused multiply-add that rounds to f16: two instructions a value (1.5 where nothing is scaled and pairs are converted together)
+// instead of four and a half.
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef float v2f __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ void split_f16(const v4f& x, h4& hi, h4& lo) {
+template <int SCALE = 1>
+__device__ __forceinline__ void split_f16(const v4f& y, h4& hi, h4& lo) {
 #pragma unroll
     for (int i = 0; i < 4; i += 2) {
-        h2 h = __builtin_convertvector((v2f{x[i], x[i + 1]}), h2);
+        h2 h;
+        if constexpr (SCALE == 1) h = __builtin_convertvector((v2f{y[i], y[i + 1]}), h2);
+        else h[0] = (_Float16)(y[i] * (float)SCALE), h[1] = (_Float16)(y[i + 1] * (float)SCALE);
         asm("" : "+v"(h));
-        const h2 l = __builtin_convertvector((v2f{x[i] - (float)h[0], x[i + 1] - (float)h[1]}), h2);
-        hi[i] = h[0], hi[i + 1] = h[1], lo[i] = l[0], lo[i + 1] = l[1];
+        hi[i] = h[0], hi[i + 1] = h[1];
+        lo[i] = (_Float16)__builtin_fmaf(y[i], (float)SCALE, -(float)h[0]), lo[i + 1] = (_Float16)__builtin_fmaf(y[i + 1], (float)SCALE, -(float)h[1]);
     }
 }
 
@@ -1045,7 +1052,7 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(A
     constexpr int PLANES = LO ? 2 : 1;                   // hi | lo
     constexpr int HD = 64, KT = 64, NT = 512 * HALVES;
     constexpr int LDH = 72;  // f16 per K row: 64 + 8 (144 bytes: 16-byte aligned rows, conflict-free 16-byte operand reads)
-    constexpr float kPScale = 4096.0f;
+    constexpr int kPScale = 4096;
     // Two tiles: K [plane][key][LDH], V [plane][key][dim] with 16-byte piece p of a row at p ^ (key & 7), so that the 16 rows that a
     // transposing read touches spread over the banks.  At the end the partner states, kStates floats per lane.
     constexpr int kStates = 18;
@@ -1105,17 +1112,21 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(A
         Piece k[NR], v[NR];  // (v unused where a thread moves one piece)
     };
     const uint32_t piece = tid % PPR, row0 = tid / PPR % KT;
-    const bool moves_v = kBoth == 1 && tid >= (uint32_t)kPieces;
+    const bool moves_v = kBoth == 1 && 64u * wave_id >= (uint32_t)kPieces;
     // Rows past the last position any query sees repeat it (their weights are zero); tiles past the last one are never looked at.
     auto fetch = [&](uint32_t t0, Regs& r) {
+        // (bytes: a uniform base per tile and 32 bits within it)
+        const uint32_t from = min(t0, wg_last), stride = kv_dim * (uint32_t)sizeof(KV), lim = min(wg_last - from, KT - 1u) * stride;
+        const char* const kt = reinterpret_cast<const char*>(kbase + (size_t)from * kv_dim);
+        const char* const vt = reinterpret_cast<const char*>(vbase + (size_t)from * kv_dim);
 #pragma unroll
         for (int i = 0; i < NR; i++) {
-            const size_t at = (size_t)min(t0 + row0 + i * (NT / PPR), wg_last) * kv_dim + (16u / sizeof(KV)) * piece;
+            const uint32_t at = min(row0 * stride + i * (NT / PPR) * stride, lim) + 16u * piece;
             if constexpr (kBoth == 1) {
-                r.k[0] = *reinterpret_cast<const Piece*>((moves_v ? vbase : kbase) + at);
+                r.k[0] = *reinterpret_cast<const Piece*>((moves_v ? vt : kt) + at);
             } else {
-                r.k[i] = *reinterpret_cast<const Piece*>(kbase + at);
-                r.v[i] = *reinterpret_cast<const Piece*>(vbase + at);
+                r.k[i] = *reinterpret_cast<const Piece*>(kt + at);
+                r.v[i] = *reinterpret_cast<const Piece*>(vt + at);
             }
         }
     };
@@ -1227,7 +1238,7 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(A
                 pw[r] = exp_nonpos_hw(sc[u][r] - m_sub);
                 psum += pw[r];
             }
-            split_f16(pw * kPScale, p_hi[u], p_lo[u]);
+            split_f16<kPScale>(pw, p_hi[u], p_lo[u]);
         }
         const h8 ph = __builtin_shufflevector(p_hi[0], p_hi[1], 0, 1, 2, 3, 4, 5, 6, 7), pl = __builtin_shufflevector(p_lo[0], p_lo[1], 0, 1, 2, 3, 4, 5, 6, 7);
         l_run = __builtin_fmaf(l_run, alpha, psum);
@@ -1288,7 +1299,7 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(A
 #pragma unroll
         for (int c = 0; c < 4; c++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) o[c][r] = (o[c][r] * fa + xch[(2 + 4 * c + r) * 64] * fb) * (1.0f / kPScale);
+            for (int r = 0; r < 4; r++) o[c][r] = (o[c][r] * fa + xch[(2 + 4 * c + r) * 64] * fb) * (1.0f / (float)kPScale);
     }
     // register r of tile c holds dim 16 c + 4 g + r of query l16
     if (q_out) {
