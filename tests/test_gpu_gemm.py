@@ -370,6 +370,12 @@ def test_residual_projection_with_norm_and_quantizer(ctx, oracle, dtype, m, n, k
         ctx.set_gemm_mfma_shape(0)
 
 
+@pytest.mark.parametrize("m,n,k,pad", [(1056, 150, 1024, 4), (2048, 40, 2048, 0), (2016, 100, 4608, 0)])
+def test_residual_projection_over_row_lengths(ctx, oracle, m, n, k, pad):
+    """Rows of 1025 .. 2048 elements, whose shares the norm's kernel adds up with eight elements per thread on their way."""
+    residual_projection_with_norm_and_quantizer(ctx, oracle, W.Q4_0, m, n, k, pad)
+
+
 def residual_projection_with_norm_and_quantizer(ctx, oracle, dtype, m, n, k, pad):
     from wick_amd.lfm2 import Lfm2Ops
     ops, eps, stride = Lfm2Ops(ctx), 1e-5, m + pad
@@ -591,6 +597,39 @@ def test_the_gated_launch_starts_past_256_tiles(ctx, oracle, m, n, k):
         for b in (d_q, d_s, d_g, d_u, d_oq, d_os):
             b.free()
     ws[0].free(), ws[1].free()
+
+
+# A launch with a last tile of 32 rows and of few tokens on each of the tiles that launch costs choose from.
+@pytest.mark.parametrize("m,n,k", [(96, 67, 256), (5472, 131, 1024), (5408, 643, 128), (4832, 1027, 512), (6176, 451, 128), (6944, 1669, 128)])
+def test_ragged_launches_on_every_tile(ctx, oracle, m, n, k):
+    """Partly filled tiles give the multi-token GEMV's result, in both layouts, added to what is there, and leave the padding alone."""
+    test_both_sides_of_every_launch_rule(ctx, oracle, m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k", [(5472, 259, 128), (6560, 259, 128), (6176, 451, 512), (6752, 1031, 1024)])
+def test_ragged_gated_launches_on_every_tile(ctx, oracle, m, n, k):
+    """The same of the launches with the gate in the epilogue, against the separate ones, bit for bit."""
+    from wick_amd.lfm2 import Lfm2Ops
+
+    ops = Lfm2Ops(ctx)
+    wb = [np.tile(oracle.synth_weight(W.Q4_0, 32, k, seed=61 + i).reshape(32, -1), (m // 32, 1)) for i in range(2)]
+    ws = [ctx.upload_weight(b, W.Q4_0, m, k) for b in wb]
+    assert ops.ffn_gate_up_silu_quantize_applies(ws[0], ws[1], n)
+    s, q = oracle.quantize_q8_0_batch(oracle.fill_normal(12, 1.0, n * k), n, k)
+    d_q, d_s, out = ctx.to_device(q), ctx.to_device(s), []
+    d_g, d_u = ctx.alloc(n * m * 4), ctx.alloc(n * m * 4)
+    d_oq, d_os = ctx.to_device(np.full(n * m + 64, 77, np.int8)), ctx.to_device(np.full(n * (m // 32) + 16, 77.0, np.float32))
+    for gated in (True, False):
+        if gated:
+            ops.encode_ffn_gate_up_silu_quantize(ws[0], ws[1], d_s, d_q, n, d_oq, d_os)
+        else:
+            ctx.gemm_preq_multi(ws, d_s, d_q, n, [d_g, d_u], m)
+            ops.silu_mul_quantize(d_g, d_u, n, m, d_oq, d_os)
+        out.append((d_oq.download(np.uint8, n * m + 64), d_os.download(np.uint32, n * (m // 32) + 16)))
+    assert all(np.array_equal(a, b) for a, b in zip(*out))
+    assert (out[0][0][n * m:] == 77).all() and (out[0][1][n * (m // 32):].view(np.float32) == 77.0).all()
+    for b in (d_q, d_s, d_g, d_u, d_oq, d_os, *ws):
+        b.free()
 
 
 @pytest.mark.parametrize("dtype", [W.Q4_0, W.Q8_0])

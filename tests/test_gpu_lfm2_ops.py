@@ -507,6 +507,12 @@ def test_rmsnorm_quantize_equals_the_two_launches(ctx, ops, oracle, rows, dim, p
         b.free()
 
 
+@pytest.mark.parametrize("rows,dim,pad", [(2, 1056, 0), (3, 2048, 4), (2, 8192, 0), (2, 8224, 0)])
+def test_rmsnorm_quantize_over_row_lengths(ctx, ops, oracle, rows, dim, pad):
+    """Rows kept in 4, 8 or 32 KB of LDS, and longer ones, which are read twice: either side of each."""
+    test_rmsnorm_quantize_equals_the_two_launches(ctx, ops, oracle, rows, dim, pad)
+
+
 @pytest.mark.parametrize("rows,dim", [(1, 32), (4, 256), (9, 4608), (33, 1024)])
 def test_silu_mul_quantize_equals_the_two_launches(ctx, ops, oracle, rows, dim):
     g, u = oracle.fill_normal(rows + dim, 2.0, rows * dim), oracle.fill_normal(rows + dim + 1, 1.0, rows * dim)
