@@ -8,7 +8,7 @@
 // into f32 accumulators on the vector ALU.
 //
 // Three families of block loops:
-//   * gemm_tile_kernel, v_mfma_i32_32x32x32_i8: prompts, on one of four tiles (see T32 and TileL / M / S / N);
+//   * gemm_tile_kernel, v_mfma_i32_32x32x32_i8: prompts, on the cheapest of six tiles for the launch (see T32 and TileL .. TileH);
 //   * gemm_few_kernel, the same instruction, 32 rows x all of up to 64 tokens: where latency is what a launch costs (few_applies);
 //   * gemm_narrow_kernel, v_mfma_i32_16x16x32_i8, 128 rows x 64 tokens: the other launches of up to 48 tokens, which skip the 16-token
 //     columns they do not have; gemm_mfma_kernel, the same shape on 128 x 128, on request (wick_rocm_set_gemm_mfma_shape).
@@ -1392,9 +1392,9 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const float* __
 // How many ways a single-weight launch is split over K: only narrow launches that leave at least half of the CUs without
 // a tile, with K long enough (>= 8 stages) that the shorter walk pays for the second launch, every share >= 2 stages (a stage
 // of a launch with few tiles costs a whole memory round trip, 1.2 - 1.4 us: nothing else is there to hide it).
-// The same on the wide tile: a long-K launch of 64 .. 256 wide tiles (the down projection of a long prompt: 1024 x 2002 x 4608 is
-// 128 of them) fills the chip's 512 workgroup slots with (tile, share) pairs of the wide kernel, whose block loop is the faster one,
-// instead of one narrow tile per CU.  Shares of >= 8 stages.
+// Also a long-K launch of 64 .. 256 tiles of 128 x 128 (the down projection of a long prompt: 1024 x 2002 x 4608 is 128 of them), up to two
+// (tile, share) pairs per CU: the large tiles' block loops are the faster ones, and without shares they would leave half of the chip
+// idle.  Shares of >= 8 stages.  (The shares fix the order of a row's sum, so they follow from the shape alone, whichever tile then runs.)
 uint32_t wide_split_factor(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits) {
     const uint32_t tiles = ((m + BM - 1) / BM) * ((n + BN - 1) / BN), stages = (k >> 5) / KB;
     if (n <= BN_NARROW || tiles < kCus / 4 || tiles > kCus || stages < 32) return 1;
