@@ -344,3 +344,38 @@ def test_a_graph_that_only_quantizes_survives_a_larger_partial_sum_buffer(oracle
         b.free()
     w.free(), w2.free()
     ctx.close()
+
+
+def test_a_graph_of_a_short_residual_projection_needs_no_scratch(oracle):
+    """K shares that a launch can walk itself stay inside it in a capture, though an eager call takes them side by side where the scratch has
+    room: the graph survives a regrow, with the bits of the eager call and of a context that has no room."""
+    n, m, eps = 23, 1024, 1e-5
+    wb = oracle.synth_weight(W.Q4_0, m, m, 11)
+    s, q = oracle.quantize_q8_0_batch(oracle.fill_normal(4, 1.0, n * m), n, m)
+    x = oracle.fill_normal(6, 1.0, n * m)
+    got = []
+    for room in (True, False):
+        ctx = W.RocmContext(0)
+        w = ctx.upload_weight(wb, W.Q4_0, m, m)
+        d_s, d_q, d_nw = ctx.to_device(s), ctx.to_device(q), ctx.to_device(np.ones(m, np.float32))
+        d_x, d_oq, d_os = ctx.to_device(x), ctx.alloc(n * m), ctx.alloc(n * (m // 32) * 4)
+        if room:
+            ctx.reserve_scratch(64, m)
+        args = (w, d_s, d_q, n, d_x, m, d_nw, eps, d_oq, d_os)
+        ctx.graph_begin()
+        ctx.gemm_preq_residual_rmsnorm_quantize(*args)
+        g = ctx.graph_end()
+        for launch in (lambda: ctx.graph_launch(g), lambda: ctx.gemm_preq_residual_rmsnorm_quantize(*args)):
+            d_x.upload(x)
+            launch()
+            got.append((d_x.download(np.uint32, n * m), d_oq.download(np.int8, n * m), d_os.download(np.uint32, n * (m // 32))))
+        ctx.reserve_scratch(1, 1 << 23)  # every buffer moves
+        d_x.upload(x)
+        ctx.graph_launch(g)
+        got.append((d_x.download(np.uint32, n * m), d_oq.download(np.int8, n * m), d_os.download(np.uint32, n * (m // 32))))
+        ctx.graph_destroy(g)
+        for b in (d_s, d_q, d_nw, d_x, d_oq, d_os, w):
+            b.free()
+        ctx.close()
+    for other in got[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(got[0], other))

@@ -158,12 +158,14 @@ int gemm_locked(wick_rocm_ctx* ctx, const wick_rocm_weight* w, const int8_t* d_q
     hipError_t e;
     if (n >= ctx->min_n_for(w->nbytes) && mfma_ok) {
         uint32_t splits = may_split && ctx->gemm_max_splits > 1 ? gemm_split_k(w->m, n, w->k, ctx->gemm_max_splits) : 1u;
-        bool in_launch = gemm_split_in_launch(w->m, n, w->k, ctx->gemm_max_splits, ctx->launch(), deferred != nullptr);  // needs no scratch
+        const size_t floats = (size_t)splits * n * w->m;
+        // (A graph does not come to depend on the scratch, nor the scratch grow, for shares that can do without.)
+        bool in_launch = gemm_split_in_launch(w->m, n, w->k, ctx->gemm_max_splits, ctx->launch(), deferred != nullptr,
+                                              !ctx->capturing && floats <= ctx->scratch_f_cap);
         if (splits > 1 && !in_launch) {
-            const size_t floats = (size_t)splits * n * w->m;
             if (ctx->capturing && floats > ctx->scratch_f_cap) {
                 // no room reserved: the shares inside the launch where it can (the same bits), else unsplit (the same to the f32 bar)
-                in_launch = gemm_split_in_launch(w->m, n, w->k, ctx->gemm_max_splits, ctx->launch(), false);
+                in_launch = gemm_split_in_launch(w->m, n, w->k, ctx->gemm_max_splits, ctx->launch(), false, false);
                 if (!in_launch) splits = 1;
             } else if (int rc = ensure_scratch(ctx, 0, 0, floats)) {
                 return rc;

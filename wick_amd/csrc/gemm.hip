@@ -1429,10 +1429,12 @@ bool few_side_applies(uint64_t rows, uint32_t n, uint32_t shares) {
 //   plain, 24:              1024 x 1024 6.6 / 4.9, x 1792 8.0 / 6.8, x 2048 7.0 / 7.4; 3072 x 2048 7.6 / 7.5, 4096 x 2048 8.5 / 7.5
 //   plain, 40:              1024 x 1024 7.2 / 7.0, 4096 x 1024 8.2 / 7.1; 2048 x 2048 8.2 / 11.5
 //   with the norm, 24:      4096 x 2048 13.3 / 12.5; over 40 tokens 3072 x 1024 11.3 / 11.6, 4096 x 1024 12.9 / 12.3
-bool few_applies_split(uint64_t rows, uint32_t n, uint32_t k, bool deferrable) {
+// Without room for shares side by side: all that needs none, the faster way or not.
+bool few_applies_split(uint64_t rows, uint32_t n, uint32_t k, uint32_t shares, bool deferrable, bool room) {
     const uint64_t units = (rows + GR - 1) / GR, slabs = k / (KB * 32), cost = n <= 32 ? 1u : 2u;
-    if (!few_applies(rows, n, k) || slabs * cost > (cost == 1 && units < 96 ? 15u : 16u)) return false;
-    return !deferrable || 12 * slabs * cost <= 72 + units;
+    if (n > 64 || units > 2 * kCus || units * slabs > (cost == 1 ? 12288u : 4096u) || slabs * cost > (cost == 1 && units < 96 ? 15u : 16u)) return false;
+    if (deferrable && 12 * slabs * cost > 72 + units) return false;
+    return !room || (few_applies(rows, n, k) && !(deferrable && few_side_applies(rows, n, shares)));
 }
 
 uint32_t split_k_factor(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits) {
@@ -1592,9 +1594,8 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, bool in_launch, uint32
 }  // namespace
 
 uint32_t gemm_split_k(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits) { return split_k_factor(m, n, k, max_splits); }
-bool gemm_split_in_launch(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits, const Launch& L, bool deferrable) {
-    if (L.gemm_mfma16 || !few_applies_split(m, n, k, deferrable)) return false;
-    return !deferrable || !few_side_applies(m, n, split_k_factor(m, n, k, max_splits));
+bool gemm_split_in_launch(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits, const Launch& L, bool deferrable, bool room) {
+    return !L.gemm_mfma16 && few_applies_split(m, n, k, split_k_factor(m, n, k, max_splits), deferrable, room);
 }
 
 // The GEMM's own copy of a weight (slabs, see StageT): its size, and the kernel that makes it from the raw blocks.
@@ -1622,7 +1623,7 @@ hipError_t launch_gemm_mfma(int type, const uint8_t* d_w, uint32_t m, uint32_t k
     a.accumulate = accumulate;
     const bool in_launch = splits > 1 && !d_partial;
     if (splits > 1) {
-        if (splits != split_k_factor(m, n, k, splits) || (in_launch && !gemm_split_in_launch(m, n, k, splits, L, false)))
+        if (splits != split_k_factor(m, n, k, splits) || (in_launch && !gemm_split_in_launch(m, n, k, splits, L, false, false)))
             return hipErrorInvalidValue;  // the shape does not carry that split
         a.ksplit = splits, a.partial = d_partial;
     }
@@ -1708,7 +1709,7 @@ hipError_t launch_block_dots_mfma(int type, const uint8_t* d_w, uint32_t m, uint
     a.w = d_w, a.xq = d_q, a.xs = nullptr, a.y = nullptr, a.dots = d_out;
     a.m = m, a.n = n, a.k = k, a.y_stride = 0;
     a.ksplit = split_k_factor(m, n, k, max_splits);
-    return launch<true>(type, a, L, gemm_split_in_launch(m, n, k, max_splits, L, false));
+    return launch<true>(type, a, L, gemm_split_in_launch(m, n, k, max_splits, L, false, true));
 }
 
 }  // namespace wick_rocm

@@ -154,8 +154,9 @@ hipError_t launch_gemm_mfma(int type, const uint8_t* d_w, uint32_t m, uint32_t k
 // Ways (1, 2, 4 or 8, at most max_splits) the launch above may be split over K: > 1 only for launches of few tiles and long K.
 uint32_t gemm_split_k(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits);
 // Whether the launch, on the block loop that L asks for, should walk its shares itself (few tokens): no scratch, nothing to defer.
-// deferrable: the caller's next kernel would add the shares up.  (With deferrable: a part of what there is without.)
-bool gemm_split_in_launch(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits, const Launch& L, bool deferrable);
+// deferrable: the caller's next kernel would add the shares up.  (With deferrable: a part of what there is without.)  room: there is scratch for
+// shares side by side that the call may use; some launches are faster with it that can do without.
+bool gemm_split_in_launch(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits, const Launch& L, bool deferrable, bool room);
 hipError_t launch_gemm_mfma_multi(int type, const uint8_t* const* d_w, const uint32_t* m, uint32_t count, uint32_t k, const int8_t* d_q,
                                   const float* d_scales, uint32_t n, float* const* d_y, uint32_t y_stride, int y_layout, int accumulate,
                                   const Launch& L);
