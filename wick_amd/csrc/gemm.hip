@@ -701,8 +701,9 @@ __device__ __forceinline__ void tie(V& v) {
     asm volatile("" : "+v"(v));
 }
 
+// (DUMP, the parity hook: all registers that there are, which it would otherwise take from scratch, up to 840 bytes a lane.)
 template <int TYPE, bool DUMP, bool GATED, typename C>
-__global__ __launch_bounds__(C::kThreads, C::kOcc) void gemm_tile_kernel(GemmArgs a) {
+__global__ __launch_bounds__(C::kThreads, DUMP ? 1 : C::kOcc) void gemm_tile_kernel(GemmArgs a) {
     constexpr int RT = C::RT, TT = C::TT, SB = C::SB, T = C::kTiles;
     __shared__ __align__(16) typename C::Smem sm;
     uint32_t row_tile, tok_tile;
