@@ -634,7 +634,6 @@ __global__ __launch_bounds__(THREADS, 4) void gemm_mfma_kernel(GemmArgs a) {
 // has been issued; all LDS addresses are immediates on four lane bases (the stage loop is written out for both buffers), so the block
 // loop holds FMAs, MFMAs, LDS reads and waits only.
 typedef int v16i __attribute__((ext_vector_type(16)));
-typedef float v16f __attribute__((ext_vector_type(16)));
 
 // WAVES: per SIMD, what the registers have to leave room for.  SCALE_FIRST: a result's 16 FMAs with the row scale go out ahead of its 16
 // with the token scales, in the result's registers, so that no FMA waits for the one before it: with two waves per SIMD the register-only
@@ -680,16 +679,6 @@ __device__ __forceinline__ void lds_read16(uint32_t addr, v4i& dst) {
 template <int OFF>
 __device__ __forceinline__ void lds_read4(uint32_t addr, float& dst) {
     asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(dst) : "v"(addr), "n"(OFF));
-}
-// sum += x of lane E of this lane's row of 16, times v. A DPP source is read two wait states after a VALU instruction wrote it at the earliest,
-// which the compiler does not see to in inline code; x is read by a run of these, of which the first, E == 0, waits.
-template <int E>
-__device__ __forceinline__ void fmac_row_lane(float& sum, float x, float v) {
-    if constexpr (E == 0) {
-        asm("s_nop 1\n\tv_fmac_f32_dpp %0, %1, %2 row_newbcast:0 row_mask:0xf bank_mask:0xf" : "+v"(sum) : "v"(x), "v"(v));
-    } else {
-        asm("v_fmac_f32_dpp %0, %1, %2 row_newbcast:%c3 row_mask:0xf bank_mask:0xf" : "+v"(sum) : "v"(x), "v"(v), "n"(E));
-    }
 }
 // At most N LDS reads outstanding; ties what becomes valid with it.
 template <int N, typename V>
@@ -884,12 +873,7 @@ __global__ __launch_bounds__(C::kThreads, DUMP ? 1 : C::kOcc) void gemm_tile_ker
 #pragma unroll
                     for (int e = 0; e < 16; e++) d[e] = __float_as_int(__builtin_fmaf(__int_as_float(d[e]), dw[at].x, dw[at].y));
                     __builtin_amdgcn_sched_barrier(0);
-                    static_for<16>([&](auto e_) {
-                        constexpr int e = decltype(e_)::value;
-                        float sum = acc[0][0][e];
-                        fmac_row_lane<e>(sum, xs[at], __int_as_float(d[e]));
-                        acc[0][0][e] = sum;
-                    });
+                    fmac_row_lanes(acc[0][0], xs[at], __builtin_bit_cast(v16f, d));
                     tie(acc[0][0]);
                 }
                 __builtin_amdgcn_sched_barrier(0);

@@ -196,6 +196,27 @@ __device__ __forceinline__ float group_sum(float v) {
     return v;
 }
 
+// sums[e] += x of lane e of this lane's row of 16, times v[e].  A source of another lane is read two wait states after a vector instruction
+// wrote it at the earliest, which the compiler does not see to in inline code.  Hence ONE piece of it, the wait and all that reads x: sixteen
+// pieces of which the first waits may be put in another order (they write different sums), and x may be copied in front of any of them.
+typedef float v16f __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ void fmac_row_lanes(v16f& sums, float x, const v16f& v) {
+    float s[16];
+#pragma unroll
+    for (int e = 0; e < 16; e++) s[e] = sums[e];
+#define WICK_FMAC_LANE(e) "v_fmac_f32_dpp %" #e ", %16, %[v" #e "] row_newbcast:" #e " row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 1\n\t" WICK_FMAC_LANE(0) WICK_FMAC_LANE(1) WICK_FMAC_LANE(2) WICK_FMAC_LANE(3) WICK_FMAC_LANE(4) WICK_FMAC_LANE(5)
+        WICK_FMAC_LANE(6) WICK_FMAC_LANE(7) WICK_FMAC_LANE(8) WICK_FMAC_LANE(9) WICK_FMAC_LANE(10) WICK_FMAC_LANE(11) WICK_FMAC_LANE(12)
+        WICK_FMAC_LANE(13) WICK_FMAC_LANE(14) WICK_FMAC_LANE(15)
+        : "+&v"(s[0]), "+&v"(s[1]), "+&v"(s[2]), "+&v"(s[3]), "+&v"(s[4]), "+&v"(s[5]), "+&v"(s[6]), "+&v"(s[7]), "+&v"(s[8]), "+&v"(s[9]),
+          "+&v"(s[10]), "+&v"(s[11]), "+&v"(s[12]), "+&v"(s[13]), "+&v"(s[14]), "+&v"(s[15])
+        : "v"(x), [v0] "v"(v[0]), [v1] "v"(v[1]), [v2] "v"(v[2]), [v3] "v"(v[3]), [v4] "v"(v[4]), [v5] "v"(v[5]), [v6] "v"(v[6]), [v7] "v"(v[7]),
+          [v8] "v"(v[8]), [v9] "v"(v[9]), [v10] "v"(v[10]), [v11] "v"(v[11]), [v12] "v"(v[12]), [v13] "v"(v[13]), [v14] "v"(v[14]), [v15] "v"(v[15]));
+#undef WICK_FMAC_LANE
+#pragma unroll
+    for (int e = 0; e < 16; e++) sums[e] = s[e];
+}
+
 // The same for a double over the whole wave, every lane gets the total: four DPP steps inside the rows of 16 lanes
 // (each moves the two halves of the double), then the four row totals through scalar registers.  A butterfly of
 // 64-bit shuffles costs twelve trips through the LDS crossbar, which is most of an RMSNorm prologue.
