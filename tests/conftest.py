@@ -1,4 +1,5 @@
 import os
+import subprocess
 import sys
 
 import numpy as np
@@ -33,6 +34,24 @@ def ctx():
     c = W.RocmContext(0)
     yield c
     c.close()
+
+
+@pytest.fixture(scope="session")
+def host_faults(tmp_path_factory):
+    """Runs a case of tests/host/host_faults.cpp, the library's objects linked against a pretended HIP runtime, and gives its output."""
+    here, lib = os.path.join(ROOT, "tests", "host"), os.path.join(ROOT, "wick_amd", "lib", "libwick_rocm.a")
+    exe = str(tmp_path_factory.mktemp("host") / "host_faults")
+    cmd = ["g++", "-std=c++17", "-O1", "-g", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", os.path.join(here, "host_faults.cpp"),
+           os.path.join(here, "fake_hip.cpp"), lib, "-lpthread", "-o", exe]
+    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert r.returncode == 0, r.stdout
+
+    def run(case, *args):
+        r = subprocess.run([exe, case, *args], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+        assert r.returncode == 0, f"{case}: status {r.returncode}\n{r.stdout}"
+        return r.stdout
+
+    return run
 
 
 def rel_l2(a, b) -> float:

@@ -1,5 +1,6 @@
 #include "fake_hip.h"
 
+#include <cxxabi.h>
 #include <hip/hip_runtime_api.h>
 
 #include <cstdint>
@@ -24,6 +25,7 @@ struct State {  // (in a function: kernels are registered by other files' static
     std::map<const void*, std::string> kernels;
     std::map<const void*, void*> symbols;
     std::deque<std::function<void()>> queue;
+    std::vector<std::string> enqueued;  // kernels, mangled
     bool capturing = false;
     long launch_fails = 0, copy_fails = 0;
     bool pinned_fails = false;
@@ -84,6 +86,7 @@ hipError_t launch(const void* f, void** args, hipStream_t stream) {
     if (reinterpret_cast<uintptr_t>(stream) != (uintptr_t)current + 1) fake_hip::other_device++;
     if (due(st().launch_fails)) return done(hipErrorLaunchFailure);
     fake_hip::launches++;
+    st().enqueued.push_back(st().kernels[f]);
     if (st().kernels[f].find("stage_copy_kernel") == std::string::npos) {
         enqueue([] {});
         return hipSuccess;
@@ -129,6 +132,17 @@ size_t pending() {
 size_t allocations() {
     Lock lk;
     return st().device.size();
+}
+std::vector<std::string> kernels() {
+    Lock lk;
+    std::vector<std::string> names;
+    for (const std::string& mangled : st().enqueued) {
+        char* const plain = abi::__cxa_demangle(mangled.c_str(), nullptr, nullptr, nullptr);
+        names.push_back(plain ? plain : mangled);
+        std::free(plain);
+    }
+    st().enqueued.clear();
+    return names;
 }
 void fail_launch(long n) {
     Lock lk;

@@ -1,10 +1,12 @@
 // What the library's host code does when something goes wrong, on a runtime that only pretends (fake_hip.h): one case per
 // run, named on the command line, with a GGUF file of a small model where one is needed.  Prints what fails; 0: nothing did.
+// And which kernels a call enqueues ("routes").
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <new>
+#include <string>
 #include <utility>
 #include <vector>
 
@@ -294,6 +296,49 @@ void devices(const char* path) {
     wick_rocm_ctx_destroy(ctx), wick_rocm_ctx_destroy(first);
 }
 
+// The kernels of each call, a line a kernel behind a line with the call itself: "norm rows dim", "gemm m n k splits" (splits: most shares of K),
+// "residual m n k", "gate_up m n k", "prompt file n".
+void routes(int count, char** calls) {
+    Ctx ctx;
+    void* d = nullptr;  // (no kernel runs: one buffer is every operand)
+    CHECK(wick_rocm_buffer_alloc(ctx, 4096, &d) == WICK_ROCM_OK, "alloc");
+    const auto f = static_cast<float*>(d);
+    const auto q = static_cast<int8_t*>(d);
+    for (int i = 0; i < count; i++) {
+        char kind[16] = "", path[512] = "";
+        unsigned a[4] = {};
+        int rc = -1;
+        const auto weight = [&](uint32_t m, uint32_t k) {
+            wick_rocm_weight* w = nullptr;
+            const std::vector<char> blocks((size_t)m * k / 32 * 18);
+            CHECK(wick_rocm_weight_upload(ctx, blocks.data(), blocks.size(), 2, m, k, &w) == WICK_ROCM_OK, "%s: weight", calls[i]);
+            fake_hip::kernels();
+            return w;
+        };
+        if (std::sscanf(calls[i], "prompt %511s %u", path, a) == 2) {
+            Model m(ctx, path);
+            const std::vector<uint32_t> tokens(a[0]);
+            fake_hip::kernels();
+            rc = wick_rocm_lfm2_forward_prefill(ctx, m, tokens.data(), a[0], 0, nullptr);
+        } else if (std::sscanf(calls[i], "%15s %u %u %u %u", kind, a, a + 1, a + 2, a + 3) >= 3) {
+            if (!std::strcmp(kind, "norm")) {
+                rc = wick_rocm_rmsnorm_quantize_q8_0(ctx, f, f, a[0], a[1], a[1], 1e-5f, q, f);
+            } else {
+                wick_rocm_weight *const w = weight(a[0], a[2]), *const up = weight(a[0], a[2]);
+                wick_rocm_set_gemm_max_k_splits(ctx, a[3]);
+                if (!std::strcmp(kind, "gemm")) rc = wick_rocm_gemm_q8(ctx, w, q, f, a[1], f, a[0], WICK_ROCM_LAYOUT_TOKEN_MAJOR, 0);
+                if (!std::strcmp(kind, "residual")) rc = wick_rocm_gemm_q8_residual_rmsnorm_quantize(ctx, w, q, f, a[1], f, a[0], f, 1e-5f, q, f);
+                if (!std::strcmp(kind, "gate_up")) rc = wick_rocm_ffn_gate_up_silu_quantize_q8(ctx, w, up, q, f, a[1], q, f);
+                wick_rocm_weight_free(ctx, w), wick_rocm_weight_free(ctx, up);
+            }
+        }
+        CHECK(rc == WICK_ROCM_OK, "%s: %d", calls[i], rc);
+        std::printf("%s\n", calls[i]);
+        for (const std::string& name : fake_hip::kernels()) std::printf("\t%s\n", name.c_str());
+    }
+    wick_rocm_buffer_free(ctx, d);
+}
+
 }  // namespace
 
 void* operator new(size_t n) {
@@ -318,6 +363,7 @@ int main(int argc, char** argv) {
     else if (!std::strcmp(name, "prompts") && argc > 2) prompts(argv[2]);
     else if (!std::strcmp(name, "memory") && argc > 2) memory(argv[2]);
     else if (!std::strcmp(name, "devices") && argc > 2) devices(argv[2]);
+    else if (!std::strcmp(name, "routes")) routes(argc - 2, argv + 2);
     else CHECK(false, "no case '%s'", name);
     return failures ? 1 : 0;
 }

@@ -1,29 +1,6 @@
 """The library's host code when something goes wrong: its objects linked against a pretended HIP runtime (tests/host/fake_hip.cpp),
 so that a refused call, a failed launch or memory that runs out is seen on the CPU and nothing is done to a GPU."""
-import os
-import subprocess
-
 import pytest
-
-from conftest import ROOT
-
-HERE = os.path.join(ROOT, "tests", "host")
-LIB = os.path.join(ROOT, "wick_amd", "lib", "libwick_rocm.a")
-
-
-@pytest.fixture(scope="session")
-def host_faults(tmp_path_factory):
-    exe = str(tmp_path_factory.mktemp("host") / "host_faults")
-    cmd = ["g++", "-std=c++17", "-O1", "-g", "-Wall", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", os.path.join(HERE, "host_faults.cpp"),
-           os.path.join(HERE, "fake_hip.cpp"), LIB, "-lpthread", "-o", exe]
-    r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    assert r.returncode == 0, r.stdout
-
-    def run(case, *args):
-        r = subprocess.run([exe, case, *args], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
-        assert r.returncode == 0, f"{case}: status {r.returncode}\n{r.stdout}"
-
-    return run
 
 
 @pytest.fixture(scope="session")

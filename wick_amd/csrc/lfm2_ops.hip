@@ -1554,10 +1554,14 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(float* __restrict__ gate,
 // S > 0: the S K shares of a split projection ([S][rows][dim]) are added onto the residual row first, which is written back: what
 // gemm_splitk_reduce_kernel (accumulating) leaves, the shares summed in ascending order and then added to x.
 //
-// Q: the row has at most 1024 Q elements and is kept in LDS for the quantizer, four elements of it and their weights per thread and
-// 1024.  Latency bounds it: everything is requested in one go, so that a row is one round trip to memory and not two (three with the
-// weights), and the LDS holds no more than the row, so that eight rows fit a CU and 2048 are one round.  Q = 0: rows of any length, read
-// a second time from memory.
+// Q: the row has at most 1024 Q elements and is kept in LDS for the quantizer.  Latency bounds it.  Q = 1, 2: four elements of the row and
+// their weights per thread and 1024, everything requested in one go, so that a row is one round trip to memory and not two (three with
+// the weights); the LDS holds no more than the row, so that eight rows fit a CU and 2048 are one round.  Q = 0: rows of any length, read
+// a second time, which the caches serve: no LDS to speak of and few registers, eight rows a CU whatever their length.  Q = 8, 32 KB and
+// five rows a CU by its LDS: where the row is a sum that is not in memory yet.
+// Without shares, a row past 2048 elements kept / read twice, us: 23 rows of 2304 3.7 / 3.5, of 4096 4.4 / 3.9, 2002 of 2304 10.2 / 8.1, of
+// 4096 13.6 / 12.1, of 8192 24.5 / 23.2 (16 KB for rows up to 4096: 3.7, 4.4, 8.5, 12.7); up to 2048 the two are within 4 % of each other
+// (555 of 1024 3.0 / 2.9, 2002 of 1024 4.4 / 4.4, 128 of 2048 3.0 / 3.2).
 template <int S, int Q>
 __global__ __launch_bounds__(256) void rmsnorm_quantize_kernel(typename std::conditional<S != 0, float*, const float*>::type __restrict__ x,
                                                                const float* __restrict__ partial, size_t share_stride,
@@ -2046,19 +2050,18 @@ hipError_t launch_attention_prefill(const float* d_q, const void* d_k_cache, con
     });
 }
 
-// go(Q) for rows of dim elements (rmsnorm_quantize_kernel); 0: longer than it keeps
-template <typename Go>
+// go(Q) for rows of dim elements (rmsnorm_quantize_kernel): LONGER for those past 2048
+template <int LONGER, typename Go>
 hipError_t with_row_quads(uint32_t dim, Go&& go) {
     if (dim <= 1024u) return go(std::integral_constant<int, 1>{});
     if (dim <= 2048u) return go(std::integral_constant<int, 2>{});
-    if (dim <= kResidualNormMaxDim) return go(std::integral_constant<int, (int)(kResidualNormMaxDim / 1024u)>{});
-    return go(std::integral_constant<int, 0>{});
+    return go(std::integral_constant<int, LONGER>{});
 }
 
 hipError_t launch_rmsnorm_quantize(const float* d_x, const float* d_weight, uint32_t rows, uint32_t dim, uint32_t x_stride, float eps, int8_t* d_q,
                                    float* d_scales, const Launch& L) {
     if (rows == 0) return hipSuccess;
-    return with_row_quads(dim, [&](auto quads) {
+    return with_row_quads<0>(dim, [&](auto quads) {
         return launch_kernel(L, kFamQuantize, rmsnorm_quantize_kernel<0, decltype(quads)::value>, dim3(rows), dim3(256), d_x, (const float*)nullptr, (size_t)0,
                              d_weight, d_q, d_scales, dim, x_stride, eps);
     });
@@ -2067,13 +2070,11 @@ hipError_t launch_rmsnorm_quantize(const float* d_x, const float* d_weight, uint
 hipError_t launch_residual_rmsnorm_quantize(float* d_x, const float* d_partial, uint32_t splits, const float* d_weight, uint32_t rows, uint32_t dim,
                                             uint32_t x_stride, float eps, int8_t* d_q, float* d_scales, const Launch& L) {
     if (rows == 0) return hipSuccess;
+    if (dim > kResidualNormMaxDim) return hipErrorInvalidValue;
     const auto go = [&](auto shares) {
-        return with_row_quads(dim, [&](auto quads) -> hipError_t {
-            constexpr int S = decltype(shares)::value, Q = decltype(quads)::value;
-            if constexpr (Q == 0) return hipErrorInvalidValue;
-            else
-                return launch_kernel(L, kFamQuantize, rmsnorm_quantize_kernel<S, Q>, dim3(rows), dim3(256), d_x, d_partial, (size_t)rows * dim, d_weight, d_q,
-                                     d_scales, dim, x_stride, eps);
+        return with_row_quads<(int)(kResidualNormMaxDim / 1024u)>(dim, [&](auto quads) {
+            return launch_kernel(L, kFamQuantize, rmsnorm_quantize_kernel<decltype(shares)::value, decltype(quads)::value>, dim3(rows), dim3(256), d_x, d_partial,
+                                 (size_t)rows * dim, d_weight, d_q, d_scales, dim, x_stride, eps);
         });
     };
     if (splits == 2) return go(std::integral_constant<int, 2>{});
