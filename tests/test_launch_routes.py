@@ -2,7 +2,11 @@
 runtime (tests/host/fake_hip.cpp), so that it is seen on the CPU."""
 import re
 
+import numpy as np
 import pytest
+
+import lfm2_synth
+from lfm2_synth import Q4_0, Q8_0
 
 
 @pytest.fixture(scope="session")
@@ -27,3 +31,32 @@ def routes(host_faults):
 def test_the_norm_keeps_short_rows_only(routes, dim, quads):
     """Rows past 2048 elements are read a second time: kept, they would leave the CU four workgroups."""
     assert routes(f"norm 30 {dim}") == [[f"rmsnorm_quantize_kernel<0, {quads}>"]]
+
+
+class Zeros:
+    """Weights for a model whose kernels do not run."""
+
+    @staticmethod
+    def synth_weight(ggml_type, m, k, seed, sigma):
+        per, size = {Q4_0: (32, 18), Q8_0: (32, 34)}[ggml_type]
+        return np.zeros(m * k // per * size, np.uint8)
+
+
+@pytest.mark.parametrize("inter,hidden,tokens,gated", [
+    (1024, 1024, 23, True), (1024, 1152, 23, False),   # 8 slabs of K
+    (2048, 1152, 32, True), (2048, 1280, 32, False),   # 9
+    (4096, 1280, 9, True), (4096, 1408, 9, False),     # 10: 128 workgroups against 256
+    (4128, 1408, 9, True),                             # past 256 granules of both
+    (4128, 3584, 24, True), (4128, 3712, 24, False),   # 28 slabs
+    (4128, 2816, 25, True), (4128, 2944, 25, False),   # 22
+    (8192, 3200, 32, True),                            # 512 x 25 slabs: the projections alone are the 128-row tiles'
+    (8224, 1024, 23, False),                           # 257 granules
+    (4608, 1024, 32, True), (4608, 1024, 33, False),   # 32 tokens
+])
+def test_few_tokens_take_the_gate_into_the_launch_while_k_is_short(routes, tmp_path, inter, hidden, tokens, gated):
+    """A prompt's gate | up over up to 32 tokens: one launch, or the projections and the gate behind them."""
+    path = tmp_path / "model.gguf"
+    path.write_bytes(bytes(lfm2_synth.build(Zeros, n_layers=1, hidden=hidden, inter=inter, n_heads=hidden // 64, kv_heads=(0,), embd_type=Q8_0)[0]))
+    kernels, = routes(f"prompt {path} {tokens}")
+    assert ("gemm_few_kernel<2, false, true, 1, 8>" in kernels) == gated
+    assert ("silu_mul_quantize_kernel" not in kernels) == gated or tokens == 33  # (33 tokens: the tiles' costs decide)

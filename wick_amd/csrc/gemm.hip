@@ -1643,6 +1643,21 @@ namespace {
 // The few-token form of the launch: one workgroup per granule and CU.
 bool gated_few_applies(uint32_t m, uint32_t n) { return n <= 32 && m / GR <= kCus; }
 
+// Where that form is the faster way.  Half of a workgroup's waves have a weight each, so that a round is half as many slabs of K as in the
+// projections alone (gemm_few_kernel as well where few_applies), on half as many workgroups: it saves a launch and the floats, once, and
+// loses time with every slab.  With a CU for every granule of both, 8 to 10 slabs of K; beyond, where the projections alone run on four
+// waves too, two to three times as many, fewer with more tokens to walk.  One launch / two, us, over 23 or 24 tokens:
+//   1024 x 512 5.0 / 6.2, x 1024 7.0 / 7.0, x 1536 8 % slower, x 2048 11.1 / 9.5, x 4096 21.0 / 15.6, x 8192 38.8 / 25.9
+//   2048 x 1024 7.0 / 7.2, x 1280 0.2 % slower, x 2048 12.1 / 10.5;  4096 x 1024 7 % faster, x 1280 4 %, x 1408 0.2 % slower, x 1792 6 %
+//   4608 x 1024 7.8 / 9.8, x 2048 12.4 / 13.3, x 3584 3 % faster, x 4096 1 % slower;  6912 x 2048 13.0 / 13.7, x 3584 0.2 % faster
+// and over 32: 4608 x 2816 0.5 % faster, x 3328 3 % slower, x 4096 6 %;  8192 x 2816 3 % faster.
+// Where the projections alone are more than few_applies takes, on the 128-row tiles, it always is: 6912 x 4096 24 / 34, 2048 x 16384 83 / 115.
+bool gated_few_faster(uint32_t m, uint32_t n, uint32_t k) {
+    if (!few_applies(2 * (uint64_t)m, n, k)) return true;
+    const uint32_t slabs = k / (KB * 32);
+    return 2 * m / GR <= kCus ? slabs <= 8 + m / 2048 : slabs <= (n <= 24 ? 28u : 22u);
+}
+
 template <typename C>
 float gated_tile_cost(uint32_t m, uint32_t n, uint32_t k) { return tile_cost<C>((m + C::kRows / 2 - 1) / (C::kRows / 2), n, k, 1, true); }
 }  // namespace
@@ -1653,7 +1668,7 @@ float gated_tile_cost(uint32_t m, uint32_t n, uint32_t k) { return tile_cost<C>(
 bool gemm_gated_faster(uint32_t m, uint32_t n, uint32_t k, const Launch& L) {
     if (gemm_gated_applies(m, n, k)) return true;
     if (L.gemm_mfma16 || m % GR != 0 || k % (KB * 32) != 0 || m == 0 || n == 0) return false;
-    if (gated_few_applies(m, n)) return true;
+    if (gated_few_applies(m, n)) return gated_few_faster(m, n, k);
     if (n <= 48 && (uint64_t)2 * m / GR > 2 * kCus) return false;  // the narrow kernel's
     const auto plain = [&](auto cfg) {
         using C = decltype(cfg);
