@@ -416,8 +416,11 @@ def residual_projection_with_norm_and_quantizer(ctx, oracle, dtype, m, n, k, pad
     w.free(), w2.free(), d_q.free(), d_s.free(), d_nw.free()
 
 
-# ragged in rows and tokens, one per tile of the cost rule (256 x 128, 128 x 128, 128 x 64 rows x tokens; the last on one workgroup per CU)
-@pytest.mark.parametrize("m,n,k", [(8150, 2021, 2048), (3001, 1500, 256), (2050, 1990, 1024), (1000, 1999, 384)])
+# ragged in rows and tokens, and the tile that their costs choose
+PROMPT_TILES = {(8150, 2021, 2048): "TileL", (3001, 1500, 256): "TileH", (2050, 1990, 1024): "TileH", (1000, 1999, 384): "TileN"}
+
+
+@pytest.mark.parametrize("m,n,k", list(PROMPT_TILES))
 def test_prompt_tiles_against_the_gemv_route(ctx, oracle, m, n, k):
     """Every element of a prompt-sized projection on the tile its size selects: both layouts and the accumulate flag bit-equal to each
     other, and within the f32 bar of the multi-token GEMV."""
@@ -514,26 +517,60 @@ def test_one_token_accumulates_into_a_column(ctx, oracle, dtype, layout, ms, k):
 
 
 # Pairs of launches on the two sides of each rule that chooses a GEMM kernel, a tile or a number of shares: (m, n, k), the rule's
-# quantity at its limit and one step past it.
-EDGES = [
-    (16384, 9, 128), (16416, 9, 128),      # 512 granules of rows: one workgroup per granule
-    (16384, 32, 3072), (16384, 32, 3200),  # 12288 slabs, up to 32 tokens
-    (16384, 33, 1024), (16384, 33, 1152),  # 4096 slabs, 33 tokens and more
-    (512, 64, 512), (512, 65, 512),        # 64 tokens
-    (256, 32, 1920), (256, 32, 2048),      # 15 slabs of a split launch, up to 32 tokens and under 96 granules
-    (3040, 9, 2048), (3072, 9, 2048), (3072, 9, 2176),  # 16 slabs from 96 granules on
-    (256, 33, 1024), (256, 33, 1152),      # 8 slabs, 33 tokens and more
-    (8192, 33, 256), (8224, 33, 256),      # 256 granules: eight waves or four
-    (16416, 48, 128), (16416, 49, 128),    # 48 tokens on the 128-row tiles; 49 .. 64 on the 32x32x32 loop
-    (64, 40, 896), (64, 40, 1024),         # 8 stages: split over K
-    (4096, 1024, 128), (4096, 1025, 128),  # 256 tiles of 128 x 128
-    (2048, 1024, 128), (2048, 1025, 128),  # 256 tiles of 128 x 64: a workgroup per CU
-    (1024, 1024, 4096), (1024, 896, 4096), (1024, 1024, 3968),  # 64 wide tiles, 32 stages: shares on the wide tile
-    (4096, 1024, 4096), (4096, 1025, 4096),                     # 256 wide tiles
-]
+# quantity at its limit and one step past it; and the kernels that the rules send them to (test_launch_routes.py), as the library
+# splits K and unsplit: "few" token groups and waves, "narrow" 16-token columns, a tile; "in" shares that a second launch adds up.
+EDGES = {
+    # 512 granules of rows: one workgroup per granule
+    (16384, 9, 128): ("few 1 4", "few 1 4"),
+    (16416, 9, 128): ("narrow 1", "narrow 1"),
+    # 12288 slabs, up to 32 tokens
+    (16384, 32, 3072): ("narrow 2, in 2", "few 1 4"),
+    (16384, 32, 3200): ("narrow 2, in 2", "narrow 2"),
+    # 4096 slabs, 33 tokens and more
+    (16384, 33, 1024): ("few 2 4", "narrow 3"),
+    (16384, 33, 1152): ("TileN, in 2", "narrow 3"),
+    # 64 tokens
+    (512, 64, 512): ("few 2 8", "few 2 8"),
+    (512, 65, 512): ("TileH", "TileH"),
+    # 15 slabs of a split launch, up to 32 tokens and under 96 granules
+    (256, 32, 1920): ("few 1 8", "few 1 8"),
+    (256, 32, 2048): ("few 1 8, in 8", "few 1 8"),
+    # 16 slabs from 96 granules on
+    (3040, 9, 2048): ("narrow 1, in 8", "few 1 8"),
+    (3072, 9, 2048): ("few 1 8", "few 1 8"),
+    (3072, 9, 2176): ("narrow 1, in 8", "few 1 8"),
+    # 8 slabs, 33 tokens and more
+    (256, 33, 1024): ("few 2 8", "few 2 8"),
+    (256, 33, 1152): ("few 2 8, in 4", "few 2 8"),
+    # 256 granules, up to 32 tokens: eight waves or four
+    (8192, 9, 128): ("few 1 8", "few 1 8"),
+    (8224, 9, 128): ("few 1 4", "few 1 4"),
+    # 256 granules, 33 tokens and more: one workgroup per granule
+    (8192, 33, 256): ("few 2 8", "few 2 8"),
+    (8224, 33, 256): ("narrow 3", "narrow 3"),
+    # 48 tokens on the 128-row tiles; 49 .. 64 on the 32x32x32 loop
+    (16416, 48, 128): ("narrow 3", "narrow 3"),
+    (16416, 49, 128): ("TileS", "TileS"),
+    # 8 stages: split over K (one launch either way)
+    (64, 40, 896): ("few 2 8", "few 2 8"),
+    (64, 40, 1024): ("few 2 8", "few 2 8"),
+    # 256 tiles of 128 x 128
+    (4096, 1024, 128): ("TileX", "TileX"),
+    (4096, 1025, 128): ("TileL", "TileL"),
+    # 256 tiles of 128 x 64
+    (2048, 1024, 128): ("TileS", "TileS"),
+    (2048, 1025, 128): ("TileX", "TileX"),
+    # 64 wide tiles, 32 stages: shares on the wide tile
+    (1024, 1024, 4096): ("TileN, in 4", "TileH"),
+    (1024, 896, 4096): ("TileN, in 2", "TileH"),
+    (1024, 1024, 3968): ("TileN, in 2", "TileH"),
+    # 256 wide tiles
+    (4096, 1024, 4096): ("TileX, in 2", "TileN"),
+    (4096, 1025, 4096): ("TileH", "TileH"),
+}
 
 
-@pytest.mark.parametrize("m,n,k", EDGES)
+@pytest.mark.parametrize("m,n,k", list(EDGES))
 def test_both_sides_of_every_launch_rule(ctx, oracle, m, n, k):
     """Either side of a rule gives the multi-token GEMV's result (another kernel, other sums: within 1e-6), in both layouts, added to
     what is there, and leaves the padding alone; split over K as the library does it, and unsplit."""
@@ -599,14 +636,19 @@ def test_the_gated_launch_starts_past_256_tiles(ctx, oracle, m, n, k):
     ws[0].free(), ws[1].free()
 
 
-# A launch with a last tile of 32 rows and of few tokens on each of the tiles that launch costs choose from.
-@pytest.mark.parametrize("m,n,k", [(96, 67, 256), (5472, 131, 1024), (5408, 643, 128), (4832, 1027, 512), (6176, 451, 128), (6944, 1669, 128)])
+# A launch with a last tile of 32 rows and of few tokens on each of the tiles that launch costs choose from, plain and with the gate.
+RAGGED_TILES = {(96, 67, 256): "TileH", (5472, 131, 1024): "TileN", (5408, 643, 128): "TileS", (4832, 1027, 512): "TileQ", (6176, 451, 128): "TileX",
+                (6944, 1669, 128): "TileL"}
+RAGGED_GATED_TILES = {(5472, 259, 128): "TileS", (6560, 259, 128): "TileQ", (6176, 451, 512): "TileX", (6752, 1031, 1024): "TileL"}
+
+
+@pytest.mark.parametrize("m,n,k", list(RAGGED_TILES))
 def test_ragged_launches_on_every_tile(ctx, oracle, m, n, k):
     """Partly filled tiles give the multi-token GEMV's result, in both layouts, added to what is there, and leave the padding alone."""
     test_both_sides_of_every_launch_rule(ctx, oracle, m, n, k)
 
 
-@pytest.mark.parametrize("m,n,k", [(5472, 259, 128), (6560, 259, 128), (6176, 451, 512), (6752, 1031, 1024)])
+@pytest.mark.parametrize("m,n,k", list(RAGGED_GATED_TILES))
 def test_ragged_gated_launches_on_every_tile(ctx, oracle, m, n, k):
     """The same of the launches with the gate in the epilogue, against the separate ones, bit for bit."""
     from wick_amd.lfm2 import Lfm2Ops

@@ -1,11 +1,14 @@
 """Which kernel a call runs on, at sizes on both sides of the rules that choose it: the library's host code against a pretended HIP
 runtime (tests/host/fake_hip.cpp), so that it is seen on the CPU."""
+import os
 import re
 
 import numpy as np
 import pytest
 
 import lfm2_synth
+import test_gpu_gemm as gemm
+from conftest import ROOT
 from lfm2_synth import Q4_0, Q8_0
 
 
@@ -25,6 +28,34 @@ def routes(host_faults):
         return kernels
 
     return run
+
+
+def short(kernels):
+    """The same as test_gpu_gemm.py names them."""
+    names = []
+    for k in kernels:
+        name, args = re.match(r"gemm_(\w+)_kernel<(.*)>$", k).groups()
+        args = args.split(", ")
+        names.append({"few": f"few {' '.join(args[3:])}", "narrow": f"narrow {args[-1]}", "tile": args[-1], "splitk_reduce": f"in {args[0]}"}[name])
+    return ", ".join(names)
+
+
+def test_the_sides_of_every_launch_rule_are_on_their_kernels(routes):
+    calls = [f"gemm {m} {n} {k} {splits}" for m, n, k in gemm.EDGES for splits in (0, 1)]
+    got = [short(k) for k in routes(*calls)]
+    assert dict(zip(gemm.EDGES, zip(got[::2], got[1::2]))) == gemm.EDGES
+
+
+def test_the_ragged_launches_are_on_every_tile(routes):
+    for tiles in (gemm.PROMPT_TILES, gemm.RAGGED_TILES):
+        for splits in (0, 1):
+            assert {s: short(k) for s, k in zip(tiles, routes(*(f"gemm {m} {n} {k} {splits}" for m, n, k in tiles)))} == tiles
+    gated = gemm.RAGGED_GATED_TILES
+    kernels = routes(*(f"gate_up {m} {n} {k}" for m, n, k in gated))
+    assert {s: short(k) for s, k in zip(gated, kernels)} == gated and all("<2, false, true, " in k for k, in kernels)
+    with open(os.path.join(ROOT, "wick_amd", "csrc", "gemm.hip")) as f:
+        plain, with_gate = (set(t.split(", ")) for t in re.findall(r"cheapest_tile<(Tile\w, [^>]*)>", f.read()))
+    assert plain == set(gemm.RAGGED_TILES.values()) and with_gate == set(gated.values())
 
 
 @pytest.mark.parametrize("dim,quads", [(32, 1), (1024, 1), (1056, 2), (2048, 2), (2080, 0), (2304, 0), (4096, 0), (8192, 0), (8224, 0)])
