@@ -772,6 +772,8 @@ __global__ __launch_bounds__(C::kThreads, DUMP ? 1 : C::kOcc) void gemm_tile_ker
         xsrc += SB * 32;
     };
     // token scales of a slab (block-major in memory) through registers, one float4 per token, threads 0 .. kTokens - 1
+    // (TileQ has not the registers: there the compiler parks the float4 in scratch, 20 bytes a lane, which is a wait for memory ahead of the
+    // stage's copies once per slab, on the waves that hold the scales)
     static_assert(C::kTokens <= C::kThreads, "a thread per token");
     const bool has_dx = threadIdx.x < (uint32_t)C::kTokens && a.xs;  // xs is null only for the parity hook, which never scales
     const uint8_t* dxsrc = reinterpret_cast<const uint8_t*>(a.xs + (size_t)tok0 * nb + (size_t)first * KB);
@@ -1451,8 +1453,10 @@ hipError_t launch_reduce(const GemmArgs& a, const Launch& L) {
 // per workgroup for filling, draining and storing it (and 3 us a launch, the same for all) -- plain launches first, those with the gate
 // in the epilogue second (0: not built).  Fitted to 130 launches (3072, 2048, 1024 x 1024, 1024 x 4608, 6144, 3072, 2048 x 2048, 2048 x 6912 and gate | up 4608 x 1024,
 // 6912 x 2048, each over 80 .. 2048 tokens, weights and activations of random bits: a launch that keeps the chip busy runs at the
-// power limit), which they meet to 5 % rms; the tile they choose is 0.3 % behind the best of the six.  A launch is workgroups on 256 CUs, kPerCu
-// at a time, and what the last round leaves idle is what separates the tiles: large ones do more per operand byte, small ones leave
+// power limit), which they meet to 5 % rms; the tile they choose is 0.3 % behind the best of the six.  Below the fit, over 115 launches of
+// 33 .. 96 tokens (14 shapes of 512 .. 16384 rows and 512 .. 8192 of K, split as the library does it): 5.4 % rms, 1.2 % behind the best, at worst
+// 8.5 % (8192 x 4096 over 56 in four shares: N where H is best, which cost 17 and 7 % more than they are given).  A launch is workgroups on 256
+// CUs, kPerCu at a time, and what the last round leaves idle is what separates the tiles: large ones do more per operand byte, small ones leave
 // less over, and a CU with a single workgroup on it wants that one's waves to be many.
 struct TileCost {
     float slab[4], fixed;
@@ -1469,7 +1473,7 @@ struct TileS : T32<2, 1, 2, 2, 4, 2> {  // 128 x 64, 4 waves of 64 x 32
     static constexpr int kPerCu = 2;
     static constexpr TileCost kCost[2] = {{{0.94f, 1.32f}, 1.25f}, {{0.99f, 1.37f}, 0.92f}};
 };
-struct TileQ : T32<2, 1, 2, 2, 2, 4> {  // the same with half a slab per stage: four of them on a CU
+struct TileQ : T32<2, 1, 2, 2, 2, 4> {  // the same with half a slab per stage: four of them on a CU (a wait per slab for token scales in scratch included)
     static constexpr int kPerCu = 4;
     static constexpr TileCost kCost[2] = {{{1.28f, 1.64f, 2.04f, 2.56f}, 1.32f}, {{1.31f, 1.66f, 2.03f, 2.61f}, 0.93f}};
 };
