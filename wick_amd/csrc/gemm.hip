@@ -619,7 +619,7 @@ __global__ __launch_bounds__(THREADS, 4) void gemm_mfma_kernel(GemmArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------
-// The tiles of a prompt: T32<RT, TT, WR, WT, SB> = WR x WT waves, each RT granules of 32 weight rows x TT groups of 32 tokens, on
+// The tiles of a prompt: T32<RT, TT, WR, WT, SB, ..> = WR x WT waves, each RT granules of 32 weight rows x TT groups of 32 tokens, on
 // v_mfma_i32_32x32x32_i8, SB blocks of K per stage.  Layout of a 32x32 result: lane l holds weight row n = l % 32 of its granule and
 // the 16 tokens m = 8 g + 4 (l / 32) + r, g = 0..3, r = 0..3 -- one row-scale pair per granule and 16 token scales per token group.
 //
@@ -637,11 +637,12 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 
 // WAVES: per SIMD, what the registers have to leave room for.  SCALE_FIRST: a result's 16 FMAs with the row scale go out ahead of its 16
 // with the token scales, in the result's registers, so that no FMA waits for the one before it: with two waves per SIMD the register-only
-// block loop runs at 1.52 instead of 1.32 POP/s (1.60 either way with four); smaller tiles have not the registers for it.
-template <int RT_, int TT_, int WR_, int WT_, int SB_, int WAVES, bool SCALE_FIRST = false>
+// block loop runs at 1.52 instead of 1.32 POP/s (1.60 either way with four); smaller tiles have not the registers for it.  COPIED_SCALES: how a
+// slab's token scales get into LDS, see load_dx.
+template <int RT_, int TT_, int WR_, int WT_, int SB_, int WAVES, bool SCALE_FIRST = false, bool COPIED_SCALES = false>
 struct T32 {
     static constexpr int RT = RT_, TT = TT_, WR = WR_, WT = WT_, SB = SB_, kOcc = WAVES;
-    static constexpr bool kScaleFirst = SCALE_FIRST;
+    static constexpr bool kScaleFirst = SCALE_FIRST, kCopiedScales = COPIED_SCALES;
     static constexpr int kWaves = WR * WT, kThreads = 64 * kWaves;
     static constexpr int kGranules = WR * RT, kRows = GR * kGranules, kTokens = 32 * WT * TT;
     static constexpr int kTiles = RT * TT;  // 32 x 32 results per wave and block
@@ -771,26 +772,37 @@ __global__ __launch_bounds__(C::kThreads, DUMP ? 1 : C::kOcc) void gemm_tile_ker
         for (int j = 0; j < kXPer; j++) tie(xoff[j]), copy_lds(xsrc + xoff[j], reinterpret_cast<uint8_t*>(&s.xt[0][0]) + 1024u * (kXPer * wave + j));
         xsrc += SB * 32;
     };
-    // token scales of a slab (block-major in memory) through registers, one float4 per token, threads 0 .. kTokens - 1
-    // (TileQ has not the registers: there the compiler parks the float4 in scratch, 20 bytes a lane, which is a wait for memory ahead of the
-    // stage's copies once per slab, on the waves that hold the scales)
-    static_assert(C::kTokens <= C::kThreads, "a thread per token");
-    const bool has_dx = threadIdx.x < (uint32_t)C::kTokens && a.xs;  // xs is null only for the parity hook, which never scales
+    // Token scales of a slab (token-major in memory), into block-major LDS with neighbours swapped (see the FMA that reads them).  Through registers, one
+    // float4 per token, threads 0 .. kTokens - 1, stored when the stage before the slab is done; or (copied) global -> LDS like the operands, a
+    // block's 64 tokens per wave: no registers, but a cache line per lane and block instead of per lane and slab.  TileQ, whose registers do
+    // not hold the float4 (the compiler parked it in scratch, and its waves waited for memory ahead of the next stage's copies), gains by the
+    // copies what the others lose: gated 4608 x 1024 over 555 tokens 26.0 -> 23.9 us, 3072 x 1024 over 2048 25.7 -> 23.7; TileX 62.7 -> 63.6
+    // (gated 4608 x 1024 over 2048), TileN 24.6 -> 26.0 and TileH 25.9 -> 26.6 (3072 x 1024 over 2048).
+    constexpr bool kCopied = C::kCopiedScales;
+    static_assert(kCopied ? KB * C::kTokens == C::kThreads && T > 1 : C::kTokens <= C::kThreads, "a block of 64 tokens per wave, or a thread per token");
+    const bool has_dx = (kCopied || threadIdx.x < (uint32_t)C::kTokens) && a.xs;  // xs is null only for the parity hook, which never scales
     const uint8_t* dxsrc = reinterpret_cast<const uint8_t*>(a.xs + (size_t)tok0 * nb + (size_t)first * KB);
-    uint32_t dxoff = min(threadIdx.x, a.n - 1u - tok0) * nb * (uint32_t)sizeof(float);
-    float4 dxr = make_float4(0.f, 0.f, 0.f, 0.f);
-    auto load_dx = [&] {
+    uint32_t dxoff = (min(kCopied ? lane ^ 1u : threadIdx.x, a.n - 1u - tok0) * nb + (kCopied ? wave : 0u)) * (uint32_t)sizeof(float);
+    [[maybe_unused]] float4 dxr = make_float4(0.f, 0.f, 0.f, 0.f);
+    auto load_dx = [&]([[maybe_unused]] uint32_t buf) {
         tie(dxoff);
-        if (has_dx) dxr = *reinterpret_cast<const float4*>(dxsrc + dxoff);
+        if (has_dx) {
+            if constexpr (kCopied)
+                __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(dxsrc + dxoff),
+                                                 (void __attribute__((address_space(3)))*)&sm.dxf[buf][wave][0], 4, 0, 0);
+            else dxr = *reinterpret_cast<const float4*>(dxsrc + dxoff);
+        }
         dxsrc += KB * sizeof(float);
     };
-    auto store_dx = [&](uint32_t buf) {
-        if (threadIdx.x < (uint32_t)C::kTokens) {
-            const uint32_t at = T == 1 ? threadIdx.x : threadIdx.x ^ 1u;  // neighbours swapped: see the FMA that reads them
-            sm.dxf[buf][0][at] = dxr.x;
-            sm.dxf[buf][1][at] = dxr.y;
-            sm.dxf[buf][2][at] = dxr.z;
-            sm.dxf[buf][3][at] = dxr.w;
+    auto store_dx = [&]([[maybe_unused]] uint32_t buf) {
+        if constexpr (!kCopied) {
+            if (threadIdx.x < (uint32_t)C::kTokens) {
+                const uint32_t at = T == 1 ? threadIdx.x : threadIdx.x ^ 1u;
+                sm.dxf[buf][0][at] = dxr.x;
+                sm.dxf[buf][1][at] = dxr.y;
+                sm.dxf[buf][2][at] = dxr.z;
+                sm.dxf[buf][3][at] = dxr.w;
+            }
         }
     };
 
@@ -962,14 +974,14 @@ __global__ __launch_bounds__(C::kThreads, DUMP ? 1 : C::kOcc) void gemm_tile_ker
 
     constexpr uint32_t HS = KB / SB;  // stages per slab
     const uint32_t stages = slabs * HS;
-    load_dx();
+    load_dx(0);
     copy_stage(0);
     store_dx(0);
     end_stage();
     for (uint32_t h = 0; h < stages; h++) {
         const uint32_t h1 = h + 1;
         const bool more = h1 < stages, new_slab = more && h1 % HS == 0;
-        if (new_slab) load_dx();
+        if (new_slab) load_dx((h1 / HS) & 1u);
         if (more) copy_stage(h1);
         compute_stage((first * HS + h) * SB);
         const uint32_t other = h & 1u ? 0u - kBuf : kBuf;  // to the other buffer
@@ -1455,7 +1467,9 @@ hipError_t launch_reduce(const GemmArgs& a, const Launch& L) {
 // 6912 x 2048, each over 80 .. 2048 tokens, weights and activations of random bits: a launch that keeps the chip busy runs at the
 // power limit), which they meet to 5 % rms; the tile they choose is 0.3 % behind the best of the six.  Below the fit, over 115 launches of
 // 33 .. 96 tokens (14 shapes of 512 .. 16384 rows and 512 .. 8192 of K, split as the library does it): 5.4 % rms, 1.2 % behind the best, at worst
-// 8.5 % (8192 x 4096 over 56 in four shares: N where H is best, which cost 17 and 7 % more than they are given).  A launch is workgroups on 256
+// 8.5 % (8192 x 4096 over 56 in four shares: N where H is best, which cost 17 and 7 % more than they are given).  TileQ's constants are what they were
+// times what copied token scales (load_dx) made of its launches: 0.85 .. 0.93 over 300 launches of 35 .. 4000 tokens, of which the tile chosen is now
+// 0.6 % (plain, 219) and 0.3 % (gated, 79) behind the best, 0.9 and 1.6 % before.  A launch is workgroups on 256
 // CUs, kPerCu at a time, and what the last round leaves idle is what separates the tiles: large ones do more per operand byte, small ones leave
 // less over, and a CU with a single workgroup on it wants that one's waves to be many.
 struct TileCost {
@@ -1473,9 +1487,9 @@ struct TileS : T32<2, 1, 2, 2, 4, 2> {  // 128 x 64, 4 waves of 64 x 32
     static constexpr int kPerCu = 2;
     static constexpr TileCost kCost[2] = {{{0.94f, 1.32f}, 1.25f}, {{0.99f, 1.37f}, 0.92f}};
 };
-struct TileQ : T32<2, 1, 2, 2, 2, 4> {  // the same with half a slab per stage: four of them on a CU (a wait per slab for token scales in scratch included)
+struct TileQ : T32<2, 1, 2, 2, 2, 4, false, true> {  // the same with half a slab per stage: four of them on a CU
     static constexpr int kPerCu = 4;
-    static constexpr TileCost kCost[2] = {{{1.28f, 1.64f, 2.04f, 2.56f}, 1.32f}, {{1.31f, 1.66f, 2.03f, 2.61f}, 0.93f}};
+    static constexpr TileCost kCost[2] = {{{1.12f, 1.40f, 1.87f, 2.36f}, 1.25f}, {{1.20f, 1.45f, 1.78f, 2.39f}, 0.97f}};
 };
 struct TileN : T32<1, 1, 4, 2, 4, 4> {  // 128 x 64, 8 waves of 32 x 32
     static constexpr int kPerCu = 2;
