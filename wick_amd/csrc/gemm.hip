@@ -9,7 +9,7 @@
 //
 // Three families of block loops:
 //   * gemm_tile_kernel, v_mfma_i32_32x32x32_i8: prompts, on the cheapest of six tiles for the launch (see T32 and TileL .. TileH);
-//   * gemm_few_kernel, the same instruction, 32 rows x all of up to 64 tokens: where latency is what a launch costs (few_applies);
+//   * gemm_few_kernel, v_mfma_i32_16x16x32_i8, 32 rows x all of up to 64 tokens: where latency is what a launch costs (few_applies);
 //   * gemm_narrow_kernel, v_mfma_i32_16x16x32_i8, 128 rows x 64 tokens: the other launches of up to 48 tokens, which skip the 16-token
 //     columns they do not have; gemm_mfma_kernel, the same shape on 128 x 128, on request (wick_rocm_set_gemm_mfma_shape).
 // The kernels are bound by the two scaling FMAs per result plus the matrix instructions, which a SIMD overlaps only in part, and by
@@ -55,6 +55,7 @@
 //     acc = fma(t, dx, acc), both plain v_fma_f32 (v_fma_mix_f32 with an f16 scale
 //     operand would save registers but issues at half the rate).
 #include <algorithm>
+#include <type_traits>
 
 #include "wick_rocm_device.h"
 #include "wick_rocm_internal.h"
@@ -1198,148 +1199,239 @@ __global__ __launch_bounds__(THREADS, 4) void gemm_narrow_kernel(GemmArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Few tokens (n <= 64: a chat turn, the tail of a prompt).  Such a launch is one latency after the other: with 128-row tiles a
-// 1024-row projection occupied 8 to 64 CUs, and every stage of K cost a barrier and the block loop of a lone workgroup.  Here a
-// workgroup takes ONE granule of 32 rows x all tokens (TG groups of 32), and K in rounds of one slab per wave and token group:
-//   * a wave multiplies its slab -- operands straight from memory into registers, a slab is in operand order already -- and leaves
-//     v = isum * dw of every (block, row, token) in LDS;
-//   * then every thread walks its elements through the round's blocks in order, acc = fma(v, dx, acc): the one part of a row's sum
-//     that is sequential is two LDS reads and an FMA per block instead of a whole block loop, and the bits are those of the tiles.
-// The next round's operands are requested before the walk.  Shares of K (split_k_factor) are walked one after the other and added up in
-// the same order as elsewhere, in the same workgroup: no scratch and no second launch.
-// Measured back to back, 23 tokens: 1024 x 1024 split in 4 6.7 -> 4.9 us, 2048 x 1024 (Q | K | V) 8.8 -> 4.9, 9216 x 1024 (gate | up)
-// 9.1 -> 6.5.
+// Few tokens (n <= 64: a chat turn, the tail of a prompt).  Such a launch is one latency after the other.  A workgroup takes ONE granule of
+// 32 rows x all tokens (TG groups of 32) of one share of K; a wave multiplies 16 rows x 16 tokens (or two such) with all of K in order, on
+// v_mfma_i32_16x16x32_i8, so that nothing is handed from wave to wave and the bits are those of the tiles.  The operands go global -> LDS
+// directly, R slabs deep: everything that fits is requested in one go when the launch starts, and a wave waits for a slab, not for memory.
+// Where a workgroup has more waves than tiles (32 tokens, eight waves) the other half of them sends the copies.
+//
+// What bounds it: a launch, a memory round trip, then each tile's chain of a slab (operands out of LDS, MFMA, four multiply-adds by the row
+// scale, four by the token scale: ~0.26 us with one wave per SIMD), and how fast the slabs come, 1.25 bytes a weight.  A 16 x 16 tile has four
+// results a lane: its token scales are read from LDS once per SLAB, 4 bytes a lane -- lane i of a row of 16 has that of block i / 4 and of
+// its row's token i % 4 -- and taken from there by the multiply-adds.  (Before, a wave multiplied slabs of its own on 32 x 32 tiles, left
+// isum * dw of every block in LDS, and all threads walked the blocks in order: half a megabyte through the LDS of a CU for gate | up of 1024
+// elements.)  Back to back, weights cold, us: 23 tokens 1024 x 1024 in 4 shares 4.0 -> 3.3, 1024 x 4608 in 8 5.4 -> 4.6, 2048 x 6912 in 8 8.0 -> 6.5,
+// 9216 x 1024 7.9 -> 6.1; 48 tokens 1024 x 1024 in 4 4.8 -> 3.5, 1024 x 4608 in 8 7.3 -> 5.1; gated 4608 x 1024 over 23 8.7 -> 6.5, 6912 x 2048 14.9 -> 10.4.
+// Tried and left: the ring deeper than R (8 slabs: 7.4 -> 8.9, the first slab waits behind the burst), shallower (3: 1 - 3 % faster up to
+// 8 slabs of K, 8 % slower at 16); a slab's operands in registers ahead of its turn, or a slab scaled under the next one's reads
+// (both 5 - 8 % slower: more code, and code that runs once has to be fetched).
+//
+// Shares of K (split_k_factor): side by side, a workgroup each, or walked one after the other and added up in the same order as elsewhere, in
+// the same workgroup: no scratch and no second launch.
 //
 // GATED: gate | up over few tokens with the SiLU gate and the down projection's quantizer behind it.  A workgroup takes a granule of gate
 // rows and the same one of up, half of the waves each; a granule is one Q8_0 block of every token, so the gated values are exchanged
 // through LDS and leave as blocks, element for element what the two projections and silu_mul_quantize_kernel compute.
+
+// sums[e] += x of lane 4 B + e of this lane's row of 16, times v[e].  One piece with its wait: see fmac_row_lanes.
+template <int B>
+__device__ __forceinline__ void fmac_row_lanes4(v4f& sums, float x, const v4f& v) {
+    float s0 = sums[0], s1 = sums[1], s2 = sums[2], s3 = sums[3];
+    asm("s_nop 1\n\t"
+        "v_fmac_f32_dpp %0, %4, %5 row_newbcast:%9 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %1, %4, %6 row_newbcast:%10 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %2, %4, %7 row_newbcast:%11 row_mask:0xf bank_mask:0xf\n\t"
+        "v_fmac_f32_dpp %3, %4, %8 row_newbcast:%12 row_mask:0xf bank_mask:0xf\n\t"
+        : "+&v"(s0), "+&v"(s1), "+&v"(s2), "+&v"(s3)
+        : "v"(x), "v"(v[0]), "v"(v[1]), "v"(v[2]), "v"(v[3]), "n"(4 * B), "n"(4 * B + 1), "n"(4 * B + 2), "n"(4 * B + 3));
+    sums[0] = s0, sums[1] = s1, sums[2] = s2, sums[3] = s3;
+}
+
+// The leading scalars repeat fields of `a` (p_more: w_up of a gated launch, else partial), so that the hardware preloads them into scalar registers at wave
+// launch (the build asks for that, -amdgpu-kernarg-preload-count): everything that the first copies need is there at the first instruction, and a
+// launch of 4 us does not begin with four scalar loads one after the other.  p_flags: log2 of the shares of K; kFewSide: they are side by
+// side; kFewMore: more weights than one.
+// (1024 x 1024 in 4 3.8 -> 3.5 us.)
+constexpr uint32_t kFewSide = 256, kFewMore = 512;
 template <int TYPE, bool DUMP, bool GATED, int TG, int WV>
-__global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(GemmArgs a) {
+__global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(const uint8_t* p_w, const int8_t* p_xq, const float* p_xs, const void* p_more, uint32_t p_n, uint32_t p_k,
+                                                              uint32_t p_row_tiles, uint32_t p_flags, GemmArgs a) {
     static_assert(!(GATED && DUMP), "the parity hook runs the plain launch");
-    constexpr int MS = GATED ? 2 : 1;                      // weights
-    constexpr int SL = WV / TG / MS, NB = SL * KB;         // slabs and blocks of a round
-    constexpr int EP = 16 * TG / WV, TPR = 32 * TG / EP;   // elements (consecutive tokens of a row) per thread and weight, threads per row
-    constexpr int kRow = 36;                               // floats of a row of 32 tokens: 16-byte aligned, rows spread over the banks
-    __shared__ __align__(16) float vs[MS][NB * TG][GR][kRow];
-    __shared__ __align__(16) float dxs[NB][32 * TG];
+    constexpr int MS = GATED ? 2 : 1;                                                   // weights
+    constexpr int TILES = MS * 4 * TG, MW = WV < TILES ? WV : TILES, TPW = TILES / MW;  // 16 x 16 tiles, waves that multiply, tiles of each
+    constexpr int CW = WV > TILES ? WV - TILES : WV;                                    // waves that copy: the others, or all
+    constexpr int kW = MS * kSlabChunks, kX = 4 * TG, kUnits = kW + kX + (DUMP ? 0 : 1), kPer = (kUnits + CW - 1) / CW;
+    // A slab's operands in LDS, a kilobyte per copy: the slab of each weight as it is in memory ([khalf][block][row] 16 bytes, [block][row] scale pairs),
+    // [token][16-byte chunk, swizzled], [token] {scales of the four blocks}.
+    constexpr uint32_t kStage = 1024 * (kW + kX + 1), kAtX = 1024 * kW, kAtDx = kAtX + 1024 * kX;
+    constexpr int R = 4;      // of them: more requested at once delay the first
+    constexpr int kRow = 36;  // (GATED) floats of a token's 32 gated values: 16-byte aligned, tokens spread over the banks
+    static_assert(kStage * R <= 80 * 1024, "two workgroups on a CU");
+    static_assert(!GATED || (WV * 8 >= 32 * TG && kStage * R >= sizeof(float) * 2 * 32 * TG * kRow), "eight threads and two rows of LDS per token");
+    __shared__ __align__(16) uint8_t sm[R * kStage];
     // shares of K: side by side, a workgroup each, into a.partial; or (no partial) one after the other in this one
-    const uint32_t ksplit = DUMP || GATED || a.ksplit < 2 ? 1u : a.ksplit;
-    const bool side = ksplit > 1 && a.partial;
-    const uint32_t shares = side ? 1u : ksplit, my_share = side ? blockIdx.x % ksplit : 0u;
-    uint32_t granule = side ? blockIdx.x / ksplit : blockIdx.x;  // within the launch's weights
-    if (granule >= a.row_tiles) return;                          // (grids are rounded up)
-    if constexpr (!GATED) select_weight(a, granule);
-    const uint32_t lane = threadIdx.x & 63u, l32 = lane & 31u, kh = lane >> 5;
+    const uint32_t shift = DUMP || GATED ? 0u : p_flags & 31u;
+    const bool side = !DUMP && !GATED && (p_flags & kFewSide);
+    const uint32_t my_share = side ? blockIdx.x & ((1u << shift) - 1u) : 0u;
+    uint32_t granule = side ? blockIdx.x >> shift : blockIdx.x;  // within the launch's weights
+    if (granule >= p_row_tiles) return;                          // (grids are rounded up)
+    a.w = p_w;
+    if (!GATED && (p_flags & kFewMore)) select_weight(a, granule);
+    const uint32_t lane = threadIdx.x & 63u, l16 = lane & 15u, kq = lane >> 4;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const uint32_t mat = wave / (WV / MS), sl = wave % (WV / MS) / TG, tg = wave % TG;
-    const uint32_t nb = a.k >> 5, all_slabs = nb / KB;
-    const uint32_t first = side ? my_share * all_slabs / ksplit : 0u;  // this workgroup's slabs; shares differ by at most one
-    const uint32_t slabs = side ? (my_share + 1u) * all_slabs / ksplit - first : all_slabs;
+    const uint32_t nb = p_k >> 5, all_slabs = nb / KB;
+    const uint32_t first = side ? my_share * all_slabs >> shift : 0u;  // this workgroup's slabs; shares differ by at most one
+    const uint32_t slabs = side ? ((my_share + 1u) * all_slabs >> shift) - first : all_slabs;
+    const uint32_t lds = lds_addr(sm);
 
-    struct Regs {
-        v4i w[KB], x[KB];
-        float2 dw[KB];
-        float4 dx;
-    };
-    const uint8_t* const slab0 = (GATED && mat ? a.w_up : a.w) + (((size_t)(granule >> 1) * all_slabs + first) * 2 + (granule & 1u)) * kSlab;
-    const int8_t* const xbase = a.xq + (size_t)min(32u * tg + l32, a.n - 1u) * a.k + (size_t)first * (32 * KB) + 16 * kh;
-    // token scales: thread t < 32 TG SL fetches the four of token t / SL and slab t % SL of the round
-    const uint32_t dtok = threadIdx.x / SL, dsl = threadIdx.x % SL;
-    const float* const sbase = DUMP ? nullptr : a.xs + (size_t)min(dtok, a.n - 1u) * nb + (size_t)first * KB;
-    const auto fetch = [&](uint32_t s0, Regs& r) {
-        const uint32_t s = s0 + sl;
-        if (s < slabs) {
-            const uint8_t* p = slab0 + (size_t)s * (2 * kSlab);
-#pragma unroll
-            for (int b = 0; b < KB; b++) {
-                r.w[b] = *reinterpret_cast<const v4i*>(p + 2048 * kh + 512 * b + 16 * l32);
-                r.x[b] = *reinterpret_cast<const v4i*>(xbase + (size_t)s * (32 * KB) + 32 * b);
-                r.dw[b] = *reinterpret_cast<const float2*>(p + kSlabWt + 256 * b + 8 * l32);
+    // ---- copies: the kilobytes of a stage dealt out over the copying waves, the same number to each (the last one more than once where they do not
+    // come out even), so that waiting for a stage is a count of those behind it ----
+    const bool copies = CW == WV || wave >= (uint32_t)MW;
+    const uint8_t* src[kPer];
+    uint32_t off[kPer], step[kPer], dst[kPer];
+    if (copies) {
+        const uint32_t cw = CW == WV ? wave : wave - MW;
+        const uint8_t* const slab0 = a.w + (((size_t)(granule >> 1) * all_slabs + first) * 2 + (granule & 1u)) * kSlab;
+        const size_t to_up = GATED ? static_cast<const uint8_t*>(p_more) - p_w - kSlab : 0;
+        const uint32_t t = lane >> 3, x0 = 16u * ((lane & 7u) ^ xt_swizzle(t));  // (eight tokens on: four on in the swizzle)
+        static_for<kPer>([&](auto j_) {
+            constexpr int j = decltype(j_)::value, lo = CW * j, hi = lo + CW - 1;  // the units that this one can be
+            const uint32_t u = min(cw + (uint32_t)lo, (uint32_t)kUnits - 1u);
+            dst[j] = lds + 1024u * u;
+            src[j] = slab0 + 1024u * u + (GATED && u >= (uint32_t)kSlabChunks ? to_up : 0), step[j] = 2 * kSlab, off[j] = 16u * lane;
+            if (hi >= kW && (lo >= kW || u >= (uint32_t)kW)) {
+                const uint32_t c = u - kW;
+                src[j] = reinterpret_cast<const uint8_t*>(p_xq) + first * (32u * KB), step[j] = 32 * KB;
+                off[j] = min(8u * c + t, p_n - 1u) * p_k + (x0 ^ (64u * (c & 1u)));
             }
-        }
-        if (!DUMP && threadIdx.x < 32u * TG * SL && s0 + dsl < slabs) r.dx = *reinterpret_cast<const float4*>(sbase + (s0 + dsl) * KB);
-    };
-
-    v16i cbias;
+            if (!DUMP && hi >= kW + kX && u >= (uint32_t)(kW + kX)) {
+                src[j] = reinterpret_cast<const uint8_t*>(p_xs) + first * (KB * sizeof(float)), step[j] = KB * sizeof(float);
+                off[j] = min(lane, p_n - 1u) * nb * (uint32_t)sizeof(float);
+            }
+            const uint64_t p = reinterpret_cast<uint64_t>(src[j]);  // (said again that it is the same for the wave: the compiler puts it in vector registers otherwise)
+            src[j] = reinterpret_cast<const uint8_t*>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)p) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(p >> 32)) << 32);
+            step[j] = (uint32_t)__builtin_amdgcn_readfirstlane((int)step[j]);
+        });
+    }
+    uint32_t at = 0;  // of the stage that is written
+    const auto copy_stage = [&] {
 #pragma unroll
-    for (int i = 0; i < 16; i++) cbias[i] = (int)kBiasBits;
+        for (int j = 0; j < kPer; j++) {
+            tie(off[j]);
+            __builtin_amdgcn_global_load_lds((const void __attribute__((address_space(1)))*)(src[j] + off[j]),
+                                             (void __attribute__((address_space(3)))*)(dst[j] + at), 16, 0, 0);
+            src[j] += step[j];
+        }
+        at = at == (R - 1) * kStage ? 0u : at + kStage;
+    };
+    if (copies)
+        for (uint32_t s = 0; s < R - 1u && s < slabs; s++) copy_stage();
+
+    // ---- this wave's tiles: 16 rows, TPW groups of 16 tokens ----
+    const uint32_t half = wave & 1u, mat = GATED ? (wave >> 1) & 1u : 0u, tg0 = (GATED ? wave >> 2 : wave >> 1) * TPW;
+    const bool multiplies = wave < (uint32_t)MW && 16u * tg0 < p_n;
+    uint32_t a_wt = lds + kSlab * mat + 2048u * (kq >> 1) + 16u * (16 * half + l16) + 8u * (kq & 1u);
+    uint32_t a_dx = lds + kAtDx + 16u * (16 * tg0 + 4 * kq + (l16 & 3u)) + 4u * (l16 >> 2);
+    uint32_t a_dws = lds + kSlab * mat + kSlabWt + 8u * (16 * half + l16);
+    uint32_t a_xt[KB];  // chunk 2 b + kq / 2 of this lane's token (the second tile's is 16 tokens on: the same swizzle)
+#pragma unroll
+    for (uint32_t b = 0; b < (uint32_t)KB; b++) a_xt[b] = lds + kAtX + 128u * (16 * tg0 + l16) + 16u * ((2 * b + (kq >> 1)) ^ xt_swizzle(l16)) + 8u * (kq & 1u);
+
+    v4i cbias;
+#pragma unroll
+    for (int i = 0; i < 4; i++) cbias[i] = (int)kBiasBits;
     asm volatile("" : "+v"(cbias));
-    const uint32_t row = threadIdx.x / TPR, tok0 = EP * (threadIdx.x % TPR);  // this thread's elements
-    float acc[MS][EP], total[EP];
+    v4f acc[TPW], total[TPW];
 #pragma unroll
-    for (int e = 0; e < EP; e++) {
-        total[e] = 0.0f;
+    for (int i = 0; i < TPW; i++) acc[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f}, total[i] = acc[i];
+    const bool walks = !DUMP && !GATED && shift != 0 && !side;
+    uint32_t share = 1, share_end = walks ? all_slabs >> shift : UINT32_MAX, stage = 0;
+    for (uint32_t s = 0; s < slabs; s++) {
+        if (copies) {  // slab s is there once no more copies are under way than those of the R - 2 slabs behind it
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 2) * kPer) : "memory");
+            if (s + (R - 2u) >= slabs) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (copies && s + (R - 1u) < slabs) copy_stage();  // where slab s - 1 was, which every wave has left
+        if (multiplies) {
+            if (__builtin_expect(s == share_end, 0)) {  // the next share of K starts
 #pragma unroll
-        for (int i = 0; i < MS; i++) acc[i][e] = 0.0f;
-    }
-    uint32_t share = 0, share_end = slabs / shares;
-
-    Regs r{};
-    fetch(0, r);
-    for (uint32_t s0 = 0; s0 < slabs; s0 += SL) {
-        if (s0 + sl < slabs) {
+                for (int i = 0; i < TPW; i++)
 #pragma unroll
-            for (int b = 0; b < KB; b++) {
-                const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(r.x[b], r.w[b], cbias, 0, 0, 0);
-                if constexpr (DUMP) {
+                    for (int r = 0; r < 4; r++) total[i][r] = share == 1 ? acc[i][r] : total[i][r] + acc[i][r], acc[i][r] = 0.0f;
+                share++;
+                share_end = share * all_slabs >> shift;
+            }
+            long w[KB], x[TPW][KB];
+            float2 dw[KB];
+            float dx[TPW];
+            v4i D[TPW][KB];
+            static_for<KB>([&](auto b_) {
+                constexpr int b = decltype(b_)::value;
+                lds_read8<512 * b>(a_wt, w[b]);
+                static_for<TPW>([&](auto i) { lds_read8<16 * 128 * decltype(i)::value>(a_xt[b], x[decltype(i)::value][b]); });
+            });
+            if constexpr (!DUMP) {
+                static_for<TPW>([&](auto i) { lds_read4<16 * 16 * decltype(i)::value>(a_dx, dx[decltype(i)::value]); });
+                static_for<KB>([&](auto b) { lds_read8<256 * decltype(b)::value>(a_dws, dw[decltype(b)::value]); });
+            }
+            constexpr int kScales = DUMP ? 0 : TPW + KB;
+            static_for<KB>([&](auto b_) {
+                constexpr int b = decltype(b_)::value, behind = (KB - 1 - b) * (1 + TPW) + kScales;
+                lds_arrived<(behind < 15 ? behind : 15)>(w[b]);
+                static_for<TPW>([&](auto i_) {
+                    constexpr int i = decltype(i_)::value;
+                    tie(x[i][b]);
+                    D[i][b] = __builtin_amdgcn_mfma_i32_16x16x32_i8(x[i][b], w[b], cbias, 0, 0, 0);
+                });
+            });
+            if constexpr (!DUMP) {
+                static_for<KB>([&](auto b_) {
+                    constexpr int b = decltype(b_)::value;
+                    lds_arrived<KB - 1 - b>(dw[b]);
+                    static_for<TPW>([&](auto i_) {
+                        constexpr int i = decltype(i_)::value;
+                        if constexpr (b == 0) tie(dx[i]);
+                        v4f t;
 #pragma unroll
-                    for (int e = 0; e < 16; e++) {
-                        const uint32_t rw = GR * granule + l32, t = 32u * tg + 4u * kh + 8u * (e >> 2) + (e & 3);
-                        if (rw < a.m && t < a.n) {
-                            int v = d[e] - (int)kBiasBits;
-                            if (TYPE == 2) v >>= 4;  // weights were stored x16; exact
-                            a.dots[((size_t)t * a.m + rw) * nb + (s0 + sl) * KB + b] = v;
+                        for (int r = 0; r < 4; r++) t[r] = __builtin_fmaf(__int_as_float(D[i][b][r]), dw[b].x, dw[b].y);
+                        fmac_row_lanes4<b>(acc[i], dx[i], t);
+                    });
+                });
+            } else {
+#pragma unroll
+                for (int i = 0; i < TPW; i++)
+#pragma unroll
+                    for (int b = 0; b < KB; b++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            const uint32_t rw = GR * granule + 16 * half + l16, t = 16 * (tg0 + i) + 4 * kq + r;
+                            if (rw < a.m && t < p_n) {
+                                int v = D[i][b][r] - (int)kBiasBits;
+                                if (TYPE == 2) v >>= 4;  // weights were stored x16; exact
+                                a.dots[((size_t)t * a.m + rw) * nb + s * KB + b] = v;
+                            }
                         }
-                    }
-                } else {
-#pragma unroll
-                    for (int g = 0; g < 4; g++) {
-                        v4f v;
-#pragma unroll
-                        for (int q = 0; q < 4; q++) v[q] = __builtin_fmaf(__int_as_float(d[4 * g + q]), r.dw[b].x, r.dw[b].y);
-                        *reinterpret_cast<v4f*>(&vs[mat][(sl * KB + b) * TG + tg][l32][8 * g + 4 * kh]) = v;
-                    }
-                }
             }
-        }
-        if constexpr (!DUMP) {
-            if (threadIdx.x < 32u * TG * SL) {
-                dxs[KB * dsl][dtok] = r.dx.x, dxs[KB * dsl + 1][dtok] = r.dx.y;
-                dxs[KB * dsl + 2][dtok] = r.dx.z, dxs[KB * dsl + 3][dtok] = r.dx.w;
-            }
-            __syncthreads();
-        }
-        if (s0 + SL < slabs) fetch(s0 + SL, r);
-        if constexpr (!DUMP) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this slab's reads are done
+            stage++;
+            const uint32_t next = (stage & (R - 1u)) == 0 ? 0u - (R - 1u) * kStage : kStage;
+            a_wt += next, a_dws += next, a_dx += next;
 #pragma unroll
-            for (uint32_t q = 0; q < (uint32_t)SL; q++) {
-                if (s0 + q < slabs) {
-                    if (!GATED && s0 + q == share_end) {  // the next share of K starts
-                        share++;
-                        share_end = (share + 1u) * slabs / shares;
-#pragma unroll
-                        for (int e = 0; e < EP; e++) total[e] = share == 1 ? acc[0][e] : total[e] + acc[0][e], acc[0][e] = 0.0f;
-                    }
-#pragma unroll
-                    for (int b = 0; b < KB; b++) {
-                        const float* const dx = &dxs[q * KB + b][tok0];
-#pragma unroll
-                        for (int i = 0; i < MS; i++) {
-                            const float* const v = &vs[i][(q * KB + b) * TG + tok0 / 32][row][tok0 % 32];
-#pragma unroll
-                            for (int e = 0; e < EP; e++) acc[i][e] = __builtin_fmaf(v[e], dx[e], acc[i][e]);
-                        }
-                    }
-                }
-            }
-            if (GATED || s0 + SL < slabs) __syncthreads();  // the planes are written again
+            for (int b = 0; b < KB; b++) a_xt[b] += next;
         }
     }
+    static_assert((R & (R - 1)) == 0, "stages are counted in a mask");
     if constexpr (GATED) {
-        static_assert(WV * 8 >= 32 * TG && sizeof(vs) >= sizeof(float) * 32 * TG * kRow, "eight threads and a row of LDS per token");
-        float* const h = &vs[0][0][0][0];  // [token][row]
+        // The waves of gate and of up have the same elements: each hands half of its own to the other and gates the rest.
+        __syncthreads();
+        float* const h = reinterpret_cast<float*>(sm);  // [token][row] of gate * up
+        float* const other = h + 32 * TG * kRow;        // [token][row] of what is handed over
+        const uint32_t el = kRow * (16 * tg0 + 4 * kq) + 16 * half + l16, mine = mat ? 2u : 0u;
 #pragma unroll
-        for (int e = 0; e < EP; e++) h[kRow * (tok0 + e) + row] = silu_mul(acc[0][e], acc[MS - 1][e]);
+        for (int i = 0; i < TPW; i++)
+#pragma unroll
+            for (uint32_t r = 0; r < 2; r++) other[el + kRow * (16 * i + 2 - mine + r)] = mat ? acc[i][r] : acc[i][2 + r];
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < TPW; i++)
+#pragma unroll
+            for (uint32_t r = 0; r < 2; r++) {
+                const float own = mat ? acc[i][2 + r] : acc[i][r], its = other[el + kRow * (16 * i + mine + r)];
+                h[el + kRow * (16 * i + mine + r)] = silu_mul(mat ? its : own, mat ? own : its);
+            }
         __syncthreads();
         const uint32_t tok = threadIdx.x >> 3, quad = threadIdx.x & 7u;
         if (tok < 32u * TG) {
@@ -1347,25 +1439,26 @@ __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(GemmArgs a) {
             float id;
             const float scale = q8_scale_and_inverse(group_max8(fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w)))), id);
             const uint32_t packed = q8_pack4(x.x, x.y, x.z, x.w, id);
-            if (tok < a.n) {
+            if (tok < p_n) {
                 *reinterpret_cast<uint32_t*>(a.q_out + (size_t)tok * a.m + GR * granule + 4u * quad) = packed;
                 if (quad == 0) a.s_out[(size_t)tok * (a.m >> 5) + granule] = scale;
             }
         }
     } else if constexpr (!DUMP) {
+        const uint32_t row = GR * granule + 16 * half + l16;
+        if (!multiplies || row >= a.m) return;
+        const size_t tok_step = side ? a.m : (a.y_row_major ? 1u : a.y_stride), row_step = side || !a.y_row_major ? 1u : a.y_stride;
+        const bool add = !side && a.accumulate;
+        float* y = (side ? static_cast<float*>(const_cast<void*>(p_more)) + (size_t)my_share * p_n * a.m : a.y) + row * row_step;
 #pragma unroll
-        for (int e = 0; e < EP; e++) {
-            const uint32_t rw = GR * granule + row, t = tok0 + e;
-            const float v = shares == 1 ? acc[0][e] : total[e] + acc[0][e];
-            if (rw < a.m && t < a.n) {
-                if (side) {
-                    a.partial[((size_t)my_share * a.n + t) * a.m + rw] = v;
-                    continue;
-                }
-                float* const y = a.y_row_major ? a.y + (size_t)rw * a.y_stride + t : a.y + (size_t)t * a.y_stride + rw;
-                *y = a.accumulate ? *y + v : v;
+        for (int i = 0; i < TPW; i++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const uint32_t t = 16 * (tg0 + i) + 4 * kq + r;
+                if (t >= p_n) continue;
+                const float v = walks ? total[i][r] + acc[i][r] : acc[i][r];
+                y[t * tok_step] = add ? y[t * tok_step] + v : v;
             }
-        }
     }
 }
 
@@ -1407,18 +1500,18 @@ bool narrow_tiles(uint64_t row_tiles, uint32_t n) { return n <= BN_NARROW || row
 
 // Launches of gemm_few_kernel: up to 64 tokens and few enough granules that latency and not the chip's throughput is what they cost
 // (every workgroup fetches all tokens' activations for its 32 rows; beyond, the 128-row tiles are the cheaper readers, and above 32
-// tokens, where a round of K is half as long, the 64-row ones from a second workgroup per CU on).  Tiles / here, us: 2048 x 1024 over 23
-// tokens 8.8 / 4.9, 1024 x 4608 29 / 14; 9216 x 1024 over 32 9.1 / 7.5, over 48 9.5 / 10.6; 65536 x 2048 over 16 27 / 40.
+// tokens the 64-row ones from a second workgroup per CU on: lines drawn for the kernel before this one, 9216 x 1024 over 48 9.5 / 10.6).  Tiles /
+// here, us: 2048 x 1024 over 23 tokens 8.8 / 4.9, 1024 x 4608 29 / 12.5; 9216 x 1024 over 32 9.1 / 6.5; 65536 x 2048 over 16 27 / 40.
 bool few_applies(uint64_t rows, uint32_t n, uint32_t k) {
     const uint64_t units = (rows + GR - 1) / GR, slabs = k / (KB * 32);
     return n <= 64 && units <= (n <= 32 ? 2 * kCus : kCus) && units * slabs <= (n <= 32 ? 12288u : 4096u);
 }
 
 // Shares of K side by side on the same kernel, a workgroup each: while the chip holds them all at once (one workgroup of eight waves per CU,
-// or two of four).  128-row or 64-row tiles / here, us: 1024 x 4608 in 8 over 23 tokens 6.7 / 4.7, over 48 6.9 / 6.3; 2048 x 6912 over 23 8.5 / 7.1,
-// over 37 8.7 / 9.9 (not taken); 2048 x 2048 over 23 4.8 / 4.3; 4096 x 4096 7.2 / 8.9 (not taken).
+// or two of four).  128-row or 64-row tiles / here, us: 1024 x 4608 in 8 over 23 tokens 6.7 / 4.6; 2048 x 6912 over 37 10.0 / 8.9, over 64 10.2 / 9.9;
+// 2048 x 4608 over 48 8.3 / 7.2; 1024 x 8192 over 64 10.0 / 6.8; past it, on the kernel before this one, 4096 x 4096 over 23 7.2 / 8.9.
 bool few_side_applies(uint64_t rows, uint32_t n, uint32_t shares) {
-    return n <= 64 && (rows + GR - 1) / GR * shares <= (n <= 32 ? 2 * kCus : kCus);
+    return n <= 64 && (rows + GR - 1) / GR * shares <= 2 * kCus;
 }
 
 // Shares of K one after the other in one launch of that kernel: ~0.3 us a slab up to 32 tokens, twice that above, against shares side by side and
@@ -1520,6 +1613,15 @@ hipError_t cheapest_tile(Cost&& cost, Go&& go) {
     return e;
 }
 
+// The few-token kernel with its leading scalars.
+template <typename Kernel>
+hipError_t launch_few(Kernel kernel, uint32_t grid, uint32_t threads, const GemmArgs& a, uint32_t shares, bool more, const Launch& L) {
+    const void* const p_more = a.w_up ? static_cast<const void*>(a.w_up) : a.partial;
+    const uint32_t shift = shares >= 8 ? 3u : (shares >= 4 ? 2u : shares >= 2 ? 1u : 0u);  // (split_k_factor makes 2, 4 or 8 shares)
+    return launch_kernel(L, kFamGemm, kernel, dim3(grid), dim3(threads), a.w, a.xq, a.xs, p_more, a.n, a.k, a.row_tiles,
+                         shift | (shift && a.partial ? kFewSide : 0u) | (more ? kFewMore : 0u), a);
+}
+
 // in_launch: the launch walks its shares of K itself (gemm_split_in_launch).  The parity hook comes with the product launch's share
 // count and in_launch, runs its kernel, and walks K whole.
 template <bool DUMP>
@@ -1546,7 +1648,9 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, bool in_launch, uint32
         if ((uint64_t)a.row_tiles * a.tok_tiles * shares > 0x7fffff00ull) return hipErrorInvalidValue;  // beyond a launch's grid
         // every XCD gets the same number of slots of the tile map; tile id = blockIdx.x / shares runs over all of them
         const uint32_t grid = (a.row_tiles * a.tok_tiles + 7u) / 8u * 8u * (whole ? 1u : shares);  // whole: a workgroup takes all shares of its rows
-        hipError_t e = launch_kernel(L, kFamGemm, kernel, dim3(grid), dim3(threads), a);
+        hipError_t e;
+        if constexpr (std::is_same<decltype(kernel), void (*)(GemmArgs)>::value) e = launch_kernel(L, kFamGemm, kernel, dim3(grid), dim3(threads), a);
+        else e = launch_few(kernel, grid, threads, a, shares, more != 0, L);
         if (e != hipSuccess || shares == 1 || defer_reduce || whole) return e;  // deferred: the caller's next kernel adds the shares up itself
         return launch_reduce(a, L);
     };
@@ -1659,20 +1763,21 @@ bool gemm_gated_applies(uint32_t m, uint32_t n, uint32_t k) {
 
 namespace {
 // The few-token form of the launch: one workgroup per granule and CU.
-bool gated_few_applies(uint32_t m, uint32_t n) { return n <= 32 && m / GR <= kCus; }
+bool gated_few_applies(uint32_t m, uint32_t n) { return n <= 64 && m / GR <= kCus; }
 
-// Where that form is the faster way.  Half of a workgroup's waves have a weight each, so that a round is half as many slabs of K as in the
-// projections alone (gemm_few_kernel as well where few_applies), on half as many workgroups: it saves a launch and the floats, once, and
-// loses time with every slab.  With a CU for every granule of both, 8 to 10 slabs of K; beyond, where the projections alone run on four
-// waves too, two to three times as many, fewer with more tokens to walk.  One launch / two, us, over 23 or 24 tokens:
-//   1024 x 512 5.0 / 6.2, x 1024 7.0 / 7.0, x 1536 8 % slower, x 2048 11.1 / 9.5, x 4096 21.0 / 15.6, x 8192 38.8 / 25.9
-//   2048 x 1024 7.0 / 7.2, x 1280 0.2 % slower, x 2048 12.1 / 10.5;  4096 x 1024 7 % faster, x 1280 4 %, x 1408 0.2 % slower, x 1792 6 %
-//   4608 x 1024 7.8 / 9.8, x 2048 12.4 / 13.3, x 3584 3 % faster, x 4096 1 % slower;  6912 x 2048 13.0 / 13.7, x 3584 0.2 % faster
-// and over 32: 4608 x 2816 0.5 % faster, x 3328 3 % slower, x 4096 6 %;  8192 x 2816 3 % faster.
-// Where the projections alone are more than few_applies takes, on the 128-row tiles, it always is: 6912 x 4096 24 / 34, 2048 x 16384 83 / 115.
+// Where that form is the faster way: it saves a launch and the floats (2.7 us together), once, and each weight has half of a workgroup's waves, so that
+// it loses time with every slab against the projections alone (gemm_few_kernel as well where few_applies).  One launch / the projections' alone,
+// us, over 24 tokens: 1024 x 512 4.3 / 3.9, x 1024 5.7 / 4.9, x 2048 9.0 / 7.4, x 4096 14.8 / 11.9; 2048 x 1024 6.2 / 5.6, x 2048 9.1 / 7.8; 4096 x 1024
+// 6.5 / 5.8, x 1792 8.8 / 7.6; 4608 x 1024 6.5 / 6.1, x 2048 9.7 / 9.4, x 4096 16.4 / 16.3; 6912 x 2048 10.5 / 10.4.  The lines up to 32 tokens were drawn for the
+// kernel before this one, on which a slab cost the gated launch more (8 to 10 slabs where the projections alone find a CU for every granule of
+// both, 28 or 22 beyond); they hold, with 1 us unclaimed around 16 slabs.  Above 32 tokens: over 40 1024 x 1536 9.7 / 6.8, 2048 x 1408 9.8 / 7.1,
+// 4096 x 1408 10.1 / 7.6; over 64 4096 x 1024 8.8 / 6.9; over 33 2048 x 2048 12.3 / 8.8.
+// Where the projections alone are more than few_applies takes, on the 128-row tiles, it always is: 6912 x 4096 over 24 17.5 / 33.7, 4608 x 1024 over 33
+// 8.4 / 11.1, 4608 x 4096 22.6 / 33.6.
 bool gated_few_faster(uint32_t m, uint32_t n, uint32_t k) {
     if (!few_applies(2 * (uint64_t)m, n, k)) return true;
     const uint32_t slabs = k / (KB * 32);
+    if (n > 32) return slabs <= 11;
     return 2 * m / GR <= kCus ? slabs <= 8 + m / 2048 : slabs <= (n <= 24 ? 28u : 22u);
 }
 
@@ -1681,8 +1786,7 @@ float gated_tile_cost(uint32_t m, uint32_t n, uint32_t k) { return tile_cost<C>(
 }  // namespace
 
 // Where the launch is expected to be faster than the two projections in one launch and the gate kernel behind it (2.7 us and the floats'
-// round trip).  In one launch / two, us: 4608 x 1024 over 9 .. 32 tokens 7.0 .. 7.8 / 9.5 .. 10.2, over 48 11.9 / 12.4, 128 12.2 / 13.1, 300 14.8 / 17.9;
-// 6912 x 2048 over 23 12.4 / 14.1, over 64 19.5 / 18.1 (not taken), 200 25.0 / 28.4.
+// round trip).  In one launch / two, us: 4608 x 1024 over 128 tokens 12.2 / 13.1, 300 14.8 / 17.9; 6912 x 2048 over 200 25.0 / 28.4.
 bool gemm_gated_faster(uint32_t m, uint32_t n, uint32_t k, const Launch& L) {
     if (gemm_gated_applies(m, n, k)) return true;
     if (L.gemm_mfma16 || m % GR != 0 || k % (KB * 32) != 0 || m == 0 || n == 0) return false;
@@ -1708,7 +1812,8 @@ hipError_t launch_gemm_mfma_gated(int /*type: the copies are the same for both*/
     a.tile_start[0] = a.tile_start[1] = UINT32_MAX;
     if (gated_few_applies(m, n)) {
         a.row_tiles = m / GR, a.tok_tiles = 1;
-        return launch_kernel(L, kFamGemm, gemm_few_kernel<2, false, true, 1, 8>, dim3(a.row_tiles), dim3(512), a);
+        if (n > 32) return launch_few(gemm_few_kernel<2, false, true, 2, 8>, a.row_tiles, 512, a, 1, false, L);
+        return launch_few(gemm_few_kernel<2, false, true, 1, 8>, a.row_tiles, 512, a, 1, false, L);
     }
     const auto tile = [&](auto cfg) {
         using C = decltype(cfg);
