@@ -107,6 +107,9 @@ struct GemmArgs {
     float* partial;
 };
 
+// (of a launch's leading scalars) More weights than one.
+constexpr uint32_t kMoreWeights = 512;
+
 // Makes `a` describe the weight that owns row tile `row_tile` and rebases the tile index to that weight.
 __device__ __forceinline__ void select_weight(GemmArgs& a, uint32_t& row_tile) {
     const bool second = row_tile >= a.tile_start[0], third = row_tile >= a.tile_start[1];
@@ -693,26 +696,28 @@ __device__ __forceinline__ void tie(V& v) {
 }
 
 // (DUMP, the parity hook: all registers that there are, which it would otherwise take from scratch, up to 840 bytes a lane.)
+// The leading scalars repeat fields of `a` (preloaded into scalar registers at wave launch, see gemm_few_kernel): what the first copies need.
 template <int TYPE, bool DUMP, bool GATED, typename C>
-__global__ __launch_bounds__(C::kThreads, DUMP ? 1 : C::kOcc) void gemm_tile_kernel(GemmArgs a) {
+__global__ __launch_bounds__(C::kThreads, DUMP ? 1 : C::kOcc) void gemm_tile_kernel(const uint8_t* p_w, const int8_t* p_xq, const float* p_xs, const uint8_t* p_w_up, uint32_t p_m,
+                                                                                   uint32_t p_n, uint32_t p_k, uint32_t p_row_tiles, uint32_t p_tok_tiles, uint32_t p_flags, GemmArgs a) {
+    a.w = p_w, a.xq = p_xq, a.xs = p_xs, a.w_up = p_w_up, a.m = p_m, a.n = p_n, a.k = p_k, a.row_tiles = p_row_tiles, a.tok_tiles = p_tok_tiles;
     constexpr int RT = C::RT, TT = C::TT, SB = C::SB, T = C::kTiles;
     __shared__ __align__(16) typename C::Smem sm;
     uint32_t row_tile, tok_tile;
     bool valid_tile;
     // K split (plain single-weight launches only): workgroup (tile, share) walks the slabs [first, first + slabs) of its tile
-    const uint32_t ksplit = DUMP || GATED || a.ksplit < 2 ? 1u : a.ksplit;
-    const uint32_t split = ksplit > 1 ? blockIdx.x % ksplit : 0u;
-    tile_of_block(ksplit > 1 ? blockIdx.x / ksplit : blockIdx.x, a.row_tiles, a.tok_tiles, row_tile, tok_tile, valid_tile);
+    const uint32_t shift = DUMP || GATED ? 0u : p_flags & 31u, ksplit = 1u << shift, split = blockIdx.x & (ksplit - 1u);
+    tile_of_block(blockIdx.x >> shift, a.row_tiles, a.tok_tiles, row_tile, tok_tile, valid_tile);
     if (!valid_tile) return;  // whole workgroup leaves together
-    if constexpr (!GATED) select_weight(a, row_tile);
+    if (!GATED && (p_flags & kMoreWeights)) select_weight(a, row_tile);
     const uint32_t row0 = row_tile * (GATED ? C::kRows / 2 : C::kRows);
     const uint32_t tok0 = tok_tile * C::kTokens;
     const uint32_t lane = threadIdx.x & 63u, l32 = lane & 31u, kh = lane >> 5;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t wr = wave / C::WT, wt = wave % C::WT;
     const uint32_t nb = a.k >> 5, all_slabs = nb / KB;
-    const uint32_t first = split * all_slabs / ksplit;  // shares differ by at most one slab, none is empty
-    const uint32_t slabs = (split + 1u) * all_slabs / ksplit - first;
+    const uint32_t first = split * all_slabs >> shift;  // shares differ by at most one slab, none is empty
+    const uint32_t slabs = ((split + 1u) * all_slabs >> shift) - first;
 
     // ---- the stage's copies: global -> LDS directly, 1 KB per wave instruction, uniform bases that move one stage on per copy round ----
     constexpr int kPairs = C::kGranules / 2, kXChunks = C::kTokens * 2 * SB / 64;
@@ -1240,9 +1245,9 @@ __device__ __forceinline__ void fmac_row_lanes4(v4f& sums, float x, const v4f& v
 // The leading scalars repeat fields of `a` (p_more: w_up of a gated launch, else partial), so that the hardware preloads them into scalar registers at wave
 // launch (the build asks for that, -amdgpu-kernarg-preload-count): everything that the first copies need is there at the first instruction, and a
 // launch of 4 us does not begin with four scalar loads one after the other.  p_flags: log2 of the shares of K; kFewSide: they are side by
-// side; kFewMore: more weights than one.
+// side; kMoreWeights: more weights than one.
 // (1024 x 1024 in 4 3.8 -> 3.5 us.)
-constexpr uint32_t kFewSide = 256, kFewMore = 512;
+constexpr uint32_t kFewSide = 256;
 template <int TYPE, bool DUMP, bool GATED, int TG, int WV>
 __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(const uint8_t* p_w, const int8_t* p_xq, const float* p_xs, const void* p_more, uint32_t p_n, uint32_t p_k,
                                                               uint32_t p_row_tiles, uint32_t p_flags, GemmArgs a) {
@@ -1266,7 +1271,7 @@ __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(const uint8_t* p_w
     uint32_t granule = side ? blockIdx.x >> shift : blockIdx.x;  // within the launch's weights
     if (granule >= p_row_tiles) return;                          // (grids are rounded up)
     a.w = p_w;
-    if (!GATED && (p_flags & kFewMore)) select_weight(a, granule);
+    if (!GATED && (p_flags & kMoreWeights)) select_weight(a, granule);
     const uint32_t lane = threadIdx.x & 63u, l16 = lane & 15u, kq = lane >> 4;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const uint32_t nb = p_k >> 5, all_slabs = nb / KB;
@@ -1613,13 +1618,21 @@ hipError_t cheapest_tile(Cost&& cost, Go&& go) {
     return e;
 }
 
-// The few-token kernel with its leading scalars.
+// A launch with the leading scalars of its kernel: none (the 16x16x32 kernels), a tile's, the few-token kernel's.
+using TileKernel = void (*)(const uint8_t*, const int8_t*, const float*, const uint8_t*, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, GemmArgs);
 template <typename Kernel>
-hipError_t launch_few(Kernel kernel, uint32_t grid, uint32_t threads, const GemmArgs& a, uint32_t shares, bool more, const Launch& L) {
-    const void* const p_more = a.w_up ? static_cast<const void*>(a.w_up) : a.partial;
+hipError_t enqueue(Kernel kernel, uint32_t grid, uint32_t threads, const GemmArgs& a, uint32_t shares, bool more, const Launch& L) {
+    const uint32_t flag = more ? kMoreWeights : 0u;
     const uint32_t shift = shares >= 8 ? 3u : (shares >= 4 ? 2u : shares >= 2 ? 1u : 0u);  // (split_k_factor makes 2, 4 or 8 shares)
-    return launch_kernel(L, kFamGemm, kernel, dim3(grid), dim3(threads), a.w, a.xq, a.xs, p_more, a.n, a.k, a.row_tiles,
-                         shift | (shift && a.partial ? kFewSide : 0u) | (more ? kFewMore : 0u), a);
+    if constexpr (std::is_same<Kernel, void (*)(GemmArgs)>::value) {
+        return launch_kernel(L, kFamGemm, kernel, dim3(grid), dim3(threads), a);
+    } else if constexpr (std::is_same<Kernel, TileKernel>::value) {
+        return launch_kernel(L, kFamGemm, kernel, dim3(grid), dim3(threads), a.w, a.xq, a.xs, a.w_up, a.m, a.n, a.k, a.row_tiles, a.tok_tiles, shift | flag, a);
+    } else {
+        const void* const p_more = a.w_up ? static_cast<const void*>(a.w_up) : a.partial;
+        return launch_kernel(L, kFamGemm, kernel, dim3(grid), dim3(threads), a.w, a.xq, a.xs, p_more, a.n, a.k, a.row_tiles,
+                             shift | (shift && a.partial ? kFewSide : 0u) | flag, a);
+    }
 }
 
 // in_launch: the launch walks its shares of K itself (gemm_split_in_launch).  The parity hook comes with the product launch's share
@@ -1648,9 +1661,7 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, bool in_launch, uint32
         if ((uint64_t)a.row_tiles * a.tok_tiles * shares > 0x7fffff00ull) return hipErrorInvalidValue;  // beyond a launch's grid
         // every XCD gets the same number of slots of the tile map; tile id = blockIdx.x / shares runs over all of them
         const uint32_t grid = (a.row_tiles * a.tok_tiles + 7u) / 8u * 8u * (whole ? 1u : shares);  // whole: a workgroup takes all shares of its rows
-        hipError_t e;
-        if constexpr (std::is_same<decltype(kernel), void (*)(GemmArgs)>::value) e = launch_kernel(L, kFamGemm, kernel, dim3(grid), dim3(threads), a);
-        else e = launch_few(kernel, grid, threads, a, shares, more != 0, L);
+        const hipError_t e = enqueue(kernel, grid, threads, a, shares, more != 0, L);
         if (e != hipSuccess || shares == 1 || defer_reduce || whole) return e;  // deferred: the caller's next kernel adds the shares up itself
         return launch_reduce(a, L);
     };
@@ -1812,14 +1823,14 @@ hipError_t launch_gemm_mfma_gated(int /*type: the copies are the same for both*/
     a.tile_start[0] = a.tile_start[1] = UINT32_MAX;
     if (gated_few_applies(m, n)) {
         a.row_tiles = m / GR, a.tok_tiles = 1;
-        if (n > 32) return launch_few(gemm_few_kernel<2, false, true, 2, 8>, a.row_tiles, 512, a, 1, false, L);
-        return launch_few(gemm_few_kernel<2, false, true, 1, 8>, a.row_tiles, 512, a, 1, false, L);
+        if (n > 32) return enqueue(gemm_few_kernel<2, false, true, 2, 8>, a.row_tiles, 512, a, 1, false, L);
+        return enqueue(gemm_few_kernel<2, false, true, 1, 8>, a.row_tiles, 512, a, 1, false, L);
     }
     const auto tile = [&](auto cfg) {
         using C = decltype(cfg);
         a.row_tiles = (m + C::kRows / 2 - 1) / (C::kRows / 2), a.tok_tiles = (n + C::kTokens - 1) / C::kTokens;
         if ((uint64_t)a.row_tiles * a.tok_tiles > 0x7fffff00ull) return hipErrorInvalidValue;
-        return launch_kernel(L, kFamGemm, gemm_tile_kernel<2, false, true, C>, dim3((a.row_tiles * a.tok_tiles + 7u) / 8u * 8u), dim3(C::kThreads), a);
+        return enqueue(gemm_tile_kernel<2, false, true, C>, (a.row_tiles * a.tok_tiles + 7u) / 8u * 8u, C::kThreads, a, 1, false, L);
     };
     return cheapest_tile<TileL, TileX, TileS, TileQ>([&](auto cfg) { return gated_tile_cost<decltype(cfg)>(m, n, k); }, tile);
 }
