@@ -1050,14 +1050,18 @@ __device__ __forceinline__ float exp_nonpos_hw(float x) { return __builtin_amdgc
 
 // KV = _Float16 (f16 caches): K and V are their own high halves and have no low halves, so the K_lo Q_hi and V_lo P_hi
 // products, their operand reads and the low planes' LDS writes drop out (8 of the 12 MFMAs per wave and tile remain).
-template <int HALVES, typename KV>
-__global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(const float* p_q, const void* p_k_cache, const void* p_v_cache, const uint32_t* p_pos, uint32_t pos0,
+// MOVERS: 512 more threads fetch, split and store the tiles, and the others only multiply.  A workgroup on a CU of its own is bound by its waves' chain of
+// a tile, ~2000 cycles with two waves per SIMD, and had the move of the next tile in it: 23 queries behind 700 positions 13.4 -> 11.8 us (f16 rows 10.1 ->
+// 9.1), 555 queries 14.4 -> 13.6, 808 behind 8192 (f16) 107 -> 102.  (256 threads: 13.2, 9.2, 15.1, 104.  A third tile in LDS, with the next tile's keys read
+// ahead of its barrier: 12.4, 9.8, 13.9, 109.)
+template <int HALVES, bool MOVERS, typename KV>
+__global__ __launch_bounds__(512 * HALVES + (MOVERS ? 512 : 0)) void attention_prefill_f16x3_kernel(const float* p_q, const void* p_k_cache, const void* p_v_cache, const uint32_t* p_pos, uint32_t pos0,
                                                                                 uint32_t n, uint32_t q_stride, uint32_t p_n_heads, uint32_t p_n_kv_heads, uint32_t p_max_seq,
                                                                                 AttentionArgs a, uint32_t out_stride, int8_t* q_out, float* s_out) {
     a.q = p_q, a.k_cache = p_k_cache, a.v_cache = p_v_cache, a.d_pos = p_pos, a.n_heads = p_n_heads, a.n_kv_heads = p_n_kv_heads, a.max_seq = p_max_seq;  // (preloaded)
     constexpr bool LO = std::is_same<KV, float>::value;  // the caches' values have low halves
     constexpr int PLANES = LO ? 2 : 1;                   // hi | lo
-    constexpr int HD = 64, KT = 64, NT = 512 * HALVES;
+    constexpr int HD = 64, KT = 64, NC = 512 * HALVES, NT = MOVERS ? 512 : NC;  // threads that multiply, threads that move tiles
     constexpr int LDH = 72;  // f16 per K row: 64 + 8 (144 bytes: 16-byte aligned rows, conflict-free 16-byte operand reads)
     constexpr int kPScale = 4096;
     // Two tiles: K [plane][key][LDH], V [plane][key][dim] with 16-byte piece p of a row at p ^ (key & 7), so that the 16 rows that a
@@ -1076,11 +1080,12 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(c
     const uint32_t tid = threadIdx.x, lane = tid & 63u, l16 = lane & 15u, g = lane >> 4;
     const uint32_t wave_id = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
     // (consecutive waves sit on different SIMDs: a block with few queries keeps as many of them busy as it can)
-    const uint32_t wave = (wave_id >> 1) & 3u, ksp = wave_id & 1u, half = wave_id >> 3;
+    const uint32_t wave = (wave_id >> 1) & 3u, ksp = wave_id & 1u, half = HALVES == 1 ? 0u : wave_id >> 3;
+    const bool moves = !MOVERS || wave_id >= NC / 64u, multiplies = !MOVERS || wave_id < NC / 64u;
     const uint32_t qb_long = qblocks - 1u - blockIdx.y;
     const uint32_t qb = half == 0 ? qb_long : blockIdx.y;
     const uint32_t j0 = qb * 64u;
-    const bool active = (half == 0 || qb != qb_long) && j0 + 16u * wave < n;  // the wave has queries
+    const bool active = multiplies && (half == 0 || qb != qb_long) && j0 + 16u * wave < n;  // the wave has queries
     const uint32_t base = a.d_pos ? *a.d_pos : pos0;
     const uint32_t kv_dim = a.n_kv_heads * HD;
     const KV* kbase = static_cast<const KV*>(a.k_cache) + (size_t)kvh * HD;
@@ -1094,7 +1099,7 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(c
 
     // this lane's query, dims 32 s + 8 g .. + 7 of slab s, scaled and split
     h8 qh[2], ql[2];
-    {
+    if (multiplies) {
         const float* qp = a.q + (size_t)jl * q_stride + (size_t)h * HD + 8u * g;
 #pragma unroll
         for (int s = 0; s < 2; s++) {
@@ -1118,7 +1123,8 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(c
     struct Regs {
         Piece k[NR], v[NR];  // (v unused where a thread moves one piece)
     };
-    const uint32_t piece = tid % PPR, row0 = tid / PPR % KT;
+    static_assert(kBoth > 1 || !MOVERS, "a thread's number among the movers does not matter");
+    const uint32_t piece = tid % PPR, row0 = (MOVERS ? tid - NC : tid) / PPR % KT;
     const bool moves_v = kBoth == 1 && 64u * wave_id >= (uint32_t)kPieces;
     // Rows past the last position any query sees repeat it (their weights are zero); tiles past the last one are never looked at.
     auto fetch = [&](uint32_t t0, Regs& r) {
@@ -1271,18 +1277,29 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(c
         __builtin_amdgcn_sched_barrier(0);
         request(then, r);
     };
-    request(0, r0);
-    request(KT, r1);
-    next_tile(tiles[0], r0, 2 * KT);
+    if (moves) {
+        request(0, r0);
+        request(KT, r1);
+        next_tile(tiles[0], r0, 2 * KT);
+    }
     __syncthreads();
     uint32_t t0 = 0;
-    for (; t0 + KT <= wg_last; t0 += 2 * KT) {  // (no way out in the middle: it would make the waits for one tile waits for both)
-        attend(tiles[0], t0);
-        next_tile(tiles[1], r1, t0 + 3 * KT);
-        __syncthreads();
-        attend(tiles[1], t0 + KT);
-        next_tile(tiles[0], r0, t0 + 4 * KT);
-        __syncthreads();
+    if (!MOVERS || multiplies) {
+        for (; t0 + KT <= wg_last; t0 += 2 * KT) {  // (no way out in the middle: it would make the waits for one tile waits for both)
+            attend(tiles[0], t0);
+            if constexpr (!MOVERS) next_tile(tiles[1], r1, t0 + 3 * KT);
+            __syncthreads();
+            attend(tiles[1], t0 + KT);
+            if constexpr (!MOVERS) next_tile(tiles[0], r0, t0 + 4 * KT);
+            __syncthreads();
+        }
+    } else {
+        for (; t0 + KT <= wg_last; t0 += 2 * KT) {  // the same barriers
+            next_tile(tiles[1], r1, t0 + 3 * KT);
+            __syncthreads();
+            next_tile(tiles[0], r0, t0 + 4 * KT);
+            __syncthreads();
+        }
     }
     if (t0 <= wg_last) attend(tiles[0], t0);
     __syncthreads();
@@ -1290,7 +1307,7 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(c
     {
         // the upper-key waves hand (maximum, weight sum, weighted values) to their partners through LDS
         float* xch = reinterpret_cast<float*>(smem) + (size_t)(half * 4u + wave) * kStates * 64u + lane;
-        if (ksp == 1) {
+        if (ksp == 1 && multiplies) {
             xch[0] = m_run, xch[64] = l_run;
 #pragma unroll
             for (int c = 0; c < 4; c++)
@@ -1298,7 +1315,7 @@ __global__ __launch_bounds__(512 * HALVES) void attention_prefill_f16x3_kernel(c
                 for (int r = 0; r < 4; r++) xch[(2 + 4 * c + r) * 64] = o[c][r];
         }
         __syncthreads();
-        if (ksp == 1) return;
+        if (ksp == 1 || !multiplies) return;
         const float m_b = xch[0], l_b = xch[64];
         const float m_all = fmaxf(m_run, m_b);
         const float fa = exp_nonpos_hw(m_run - m_all), fb = exp_nonpos_hw(m_b - m_all);
@@ -2040,9 +2057,9 @@ hipError_t launch_attention_prefill(const float* d_q, const void* d_k_cache, con
         return with_kv_type(kv_f16, [&](auto kv) {
             using KV = decltype(kv);
             if (n_heads * qblocks <= 256u)
-                return launch_kernel(L, kFamOther, attention_prefill_f16x3_kernel<1, KV>, dim3(n_heads, qblocks), dim3(512), a.q, a.k_cache, a.v_cache, a.d_pos, pos0, n,
+                return launch_kernel(L, kFamOther, attention_prefill_f16x3_kernel<1, true, KV>, dim3(n_heads, qblocks), dim3(1024), a.q, a.k_cache, a.v_cache, a.d_pos, pos0, n,
                                      q_stride, n_heads, n_kv_heads, max_seq, a, out_stride, d_q8, d_q8_scales);
-            return launch_kernel(L, kFamOther, attention_prefill_f16x3_kernel<2, KV>, dim3(n_heads, (qblocks + 1u) / 2u), dim3(1024), a.q, a.k_cache, a.v_cache, a.d_pos,
+            return launch_kernel(L, kFamOther, attention_prefill_f16x3_kernel<2, false, KV>, dim3(n_heads, (qblocks + 1u) / 2u), dim3(1024), a.q, a.k_cache, a.v_cache, a.d_pos,
                                  pos0, n, q_stride, n_heads, n_kv_heads, max_seq, a, out_stride, d_q8, d_q8_scales);
         });
     }
