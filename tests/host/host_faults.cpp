@@ -81,9 +81,9 @@ struct Gguf {
 struct Model {
     wick_rocm_ctx* ctx;
     wick_rocm_lfm2* m = nullptr;
-    Model(wick_rocm_ctx* c, const char* path) : ctx(c) {
+    Model(wick_rocm_ctx* c, const char* path, uint32_t context = 64) : ctx(c) {
         Gguf g(path);
-        if (wick_rocm_lfm2_load(c, g.g, 64, &m) != WICK_ROCM_OK) std::abort();
+        if (wick_rocm_lfm2_load(c, g.g, context, &m) != WICK_ROCM_OK) std::abort();
     }
     ~Model() { wick_rocm_lfm2_free(ctx, m); }
     operator wick_rocm_lfm2*() const { return m; }
@@ -316,7 +316,7 @@ void routes(int count, char** calls) {
             return w;
         };
         if (std::sscanf(calls[i], "prompt %511s %u", path, a) == 2) {
-            Model m(ctx, path);
+            Model m(ctx, path, a[0] > 64 ? a[0] : 64);
             const std::vector<uint32_t> tokens(a[0]);
             fake_hip::kernels();
             rc = wick_rocm_lfm2_forward_prefill(ctx, m, tokens.data(), a[0], 0, nullptr);

@@ -702,3 +702,25 @@ def test_the_gate_in_the_launch_over_all_magnitudes(ctx, oracle, dtype):
     assert all(np.array_equal(a, b) for a, b in zip(*out))
     for b in (d_q, d_s, d_g, d_u, d_oq, d_os, *ws):
         b.free()
+
+
+# m, n, k -> the kernels of a projection, split over K as the library does it and unsplit: several tiles of 32 or 64 tokens on the few-token kernel
+FEW_TILES = {
+    (1056, 97, 640): ("few 1 4", "few 1 4"),           # one token and one granule over
+    (2080, 81, 128): ("few 1 4", "few 1 4"),           # one slab
+    (544, 65, 512): ("few 1 4", "few 1 4"),            # past 512 x 512
+    (3584, 128, 256): ("few 1 4", "few 1 4"),          # 448 tiles of 32 tokens
+    (3584, 129, 256): ("few 2 8", "few 2 8"),
+    (8192, 128, 128): ("few 2 8", "few 2 8"),          # 512 of 64
+    (8224, 128, 128): ("TileS", "TileS"),
+    (1024, 832, 384): ("few 2 8", "few 2 8"),          # 832 tokens
+    (1024, 833, 384): ("TileH", "TileH"),
+    (1024, 76, 2048): ("few 1 4", "few 1 4"),          # 16 slabs in shares: in the launch
+    (1024, 74, 2048): ("few 2 8, in 8", "few 1 4"),    # or 512 side by side
+}
+
+
+@pytest.mark.parametrize("m,n,k", list(FEW_TILES))
+def test_few_token_tiles_side_by_side(ctx, oracle, m, n, k):
+    """More than 64 tokens on the few-token kernel give the multi-token GEMV's result, in both layouts, added to what is there, and leave the padding alone."""
+    test_both_sides_of_every_launch_rule(ctx, oracle, m, n, k)

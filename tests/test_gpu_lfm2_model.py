@@ -528,11 +528,12 @@ def test_a_prompt_is_the_same_on_either_block_loop(ctx, oracle, tmp_path, wtype)
 @pytest.mark.parametrize("hidden,inter", [(128, 1152), (640, 128), (1152, 640)])
 def test_short_prompts_at_the_edges_of_their_tiles(ctx, oracle, tmp_path, hidden, inter):
     """The few-token launches on both sides of their 16-token tiles, gate | up in one launch among them, over 1, 5 and 9 slabs of K (fewer than
-    their ring of stages holds, one more, and twice round): bit for bit the 16x16x32 kernels, which take none of them."""
-    model, _, _ = load(ctx, oracle, tmp_path, context=128, n_layers=2, hidden=hidden, inter=inter, n_heads=hidden // 64, kv_heads=(0, 2), vocab=256, embd_type=W.Q8_0)
-    tokens = np.random.default_rng(5).integers(0, 256, 64).astype(np.uint32)
+    their ring of stages holds, one more, and twice round), and over several tiles of 32 and 64 tokens: bit for bit the 16x16x32 kernels, which take
+    none of them."""
+    model, _, _ = load(ctx, oracle, tmp_path, context=512, n_layers=2, hidden=hidden, inter=inter, n_heads=hidden // 64, kv_heads=(0, 2), vocab=256, embd_type=W.Q8_0)
+    tokens = np.random.default_rng(5).integers(0, 256, 449).astype(np.uint32)
     try:
-        for n in (10, 15, 31, 34, 47, 63):
+        for n in (10, 15, 31, 34, 47, 63, 65, 97, 130, 449):
             got = []
             for shape in (32, 16):
                 ctx.set_gemm_mfma_shape(shape)

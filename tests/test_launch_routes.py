@@ -58,6 +58,12 @@ def test_the_ragged_launches_are_on_every_tile(routes):
     assert plain == set(gemm.RAGGED_TILES.values()) and with_gate == set(gated.values())
 
 
+def test_prompts_on_the_few_token_kernel(routes):
+    calls = [f"gemm {m} {n} {k} {splits}" for m, n, k in gemm.FEW_TILES for splits in (0, 1)]
+    got = [short(k) for k in routes(*calls)]
+    assert dict(zip(gemm.FEW_TILES, zip(got[::2], got[1::2]))) == gemm.FEW_TILES
+
+
 @pytest.mark.parametrize("dim,quads", [(32, 1), (1024, 1), (1056, 2), (2048, 2), (2080, 0), (2304, 0), (4096, 0), (8192, 0), (8224, 0)])
 def test_the_norm_keeps_short_rows_only(routes, dim, quads):
     """Rows past 2048 elements are read a second time: kept, they would leave the CU four workgroups."""
@@ -91,3 +97,23 @@ def test_few_tokens_take_the_gate_into_the_launch_while_k_is_short(routes, tmp_p
     kernels, = routes(f"prompt {path} {tokens}")
     assert ("gemm_few_kernel<2, false, true, 1, 8>" in kernels) == gated
     assert ("silu_mul_quantize_kernel" not in kernels) == gated or tokens == 33  # (33 tokens: the tiles' costs decide)
+
+
+@pytest.mark.parametrize("tokens,kernel", [(200, "few_kernel<2, false, false, 2, 8>"),  # 512 tiles of 64 tokens, four shares
+                                           (255, "few_kernel<2, false, false, 2, 8>"), (257, "few_kernel<2, false, false, 1, 4>"),  # 8 slabs, 256 x 1024 outputs
+                                           (512, "few_kernel<2, false, false, 2, 8>"), (513, "tile_kernel<2, false, false, TileN>")])
+def test_residual_projections_of_a_prompt(routes, tokens, kernel):
+    """Shares of K that the norm behind adds up: side by side on the few-token kernel, walked by it, on the tiles."""
+    assert routes(f"residual 1024 {tokens} 1024 8")[0][0] == f"gemm_{kernel}"
+
+
+@pytest.mark.parametrize("inter,tokens,kernel", [
+    (3584, 65, "few_kernel<2, false, true, 1, 8>"), (3584, 128, "few_kernel<2, false, true, 1, 8>"),  # 448 tiles of 32 tokens
+    (3584, 129, "few_kernel<2, false, true, 2, 8>"),
+    (4096, 160, "few_kernel<2, false, true, 2, 8>"), (4096, 161, "tile_kernel<2, false, true, TileS>"),  # 1280 of 16
+])
+def test_prompts_take_the_gate_into_the_few_token_kernel(routes, tmp_path, inter, tokens, kernel):
+    path = tmp_path / "model.gguf"
+    path.write_bytes(bytes(lfm2_synth.build(Zeros, n_layers=1, hidden=1024, inter=inter, n_heads=16, kv_heads=(0,), embd_type=Q8_0)[0]))
+    kernels, = routes(f"prompt {path} {tokens}")
+    assert f"gemm_{kernel}" in kernels and "silu_mul_quantize_kernel" not in kernels

@@ -9,7 +9,7 @@
 //
 // Three families of block loops:
 //   * gemm_tile_kernel, v_mfma_i32_32x32x32_i8: prompts, on the cheapest of six tiles for the launch (see T32 and TileL .. TileH);
-//   * gemm_few_kernel, v_mfma_i32_16x16x32_i8, 32 rows x all of up to 64 tokens: where latency is what a launch costs (few_applies);
+//   * gemm_few_kernel, v_mfma_i32_16x16x32_i8, 32 rows x up to 64 tokens: where latency is what a launch costs (few_applies, few_tokens_per_tile);
 //   * gemm_narrow_kernel, v_mfma_i32_16x16x32_i8, 128 rows x 64 tokens: the other launches of up to 48 tokens, which skip the 16-token
 //     columns they do not have; gemm_mfma_kernel, the same shape on 128 x 128, on request (wick_rocm_set_gemm_mfma_shape).
 // The kernels are bound by the two scaling FMAs per result plus the matrix instructions, which a SIMD overlaps only in part, and by
@@ -1204,8 +1204,8 @@ __global__ __launch_bounds__(THREADS, 4) void gemm_narrow_kernel(GemmArgs a) {
 }
 
 // ---------------------------------------------------------------------------------------
-// Few tokens (n <= 64: a chat turn, the tail of a prompt).  Such a launch is one latency after the other.  A workgroup takes ONE granule of
-// 32 rows x all tokens (TG groups of 32) of one share of K; a wave multiplies 16 rows x 16 tokens (or two such) with all of K in order, on
+// Few tokens (a chat turn, the tail of a prompt; up to a few hundred where the rows are few).  Such a launch is one latency after the other.  A workgroup
+// takes ONE granule of 32 rows x 32 TG tokens (blockIdx.y: which) of one share of K; a wave multiplies 16 rows x 16 tokens (or two such) with all of K in order, on
 // v_mfma_i32_16x16x32_i8, so that nothing is handed from wave to wave and the bits are those of the tiles.  The operands go global -> LDS
 // directly, R slabs deep: everything that fits is requested in one go when the launch starts, and a wave waits for a slab, not for memory.
 // Where a workgroup has more waves than tiles (32 tokens, eight waves) the other half of them sends the copies.
@@ -1278,6 +1278,7 @@ __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(const uint8_t* p_w
     const uint32_t first = side ? my_share * all_slabs >> shift : 0u;  // this workgroup's slabs; shares differ by at most one
     const uint32_t slabs = side ? ((my_share + 1u) * all_slabs >> shift) - first : all_slabs;
     const uint32_t lds = lds_addr(sm);
+    const uint32_t tok0 = 32u * TG * blockIdx.y, n_here = p_n - tok0;  // this workgroup's tokens
 
     // ---- copies: the kilobytes of a stage dealt out over the copying waves, the same number to each (the last one more than once where they do not
     // come out even), so that waiting for a stage is a count of those behind it ----
@@ -1296,12 +1297,12 @@ __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(const uint8_t* p_w
             src[j] = slab0 + 1024u * u + (GATED && u >= (uint32_t)kSlabChunks ? to_up : 0), step[j] = 2 * kSlab, off[j] = 16u * lane;
             if (hi >= kW && (lo >= kW || u >= (uint32_t)kW)) {
                 const uint32_t c = u - kW;
-                src[j] = reinterpret_cast<const uint8_t*>(p_xq) + first * (32u * KB), step[j] = 32 * KB;
-                off[j] = min(8u * c + t, p_n - 1u) * p_k + (x0 ^ (64u * (c & 1u)));
+                src[j] = reinterpret_cast<const uint8_t*>(p_xq) + (size_t)tok0 * p_k + first * (32u * KB), step[j] = 32 * KB;
+                off[j] = min(8u * c + t, n_here - 1u) * p_k + (x0 ^ (64u * (c & 1u)));
             }
             if (!DUMP && hi >= kW + kX && u >= (uint32_t)(kW + kX)) {
-                src[j] = reinterpret_cast<const uint8_t*>(p_xs) + first * (KB * sizeof(float)), step[j] = KB * sizeof(float);
-                off[j] = min(lane, p_n - 1u) * nb * (uint32_t)sizeof(float);
+                src[j] = reinterpret_cast<const uint8_t*>(p_xs) + ((size_t)tok0 * nb + first * KB) * sizeof(float), step[j] = KB * sizeof(float);
+                off[j] = min(lane, n_here - 1u) * nb * (uint32_t)sizeof(float);
             }
             const uint64_t p = reinterpret_cast<uint64_t>(src[j]);  // (said again that it is the same for the wave: the compiler puts it in vector registers otherwise)
             src[j] = reinterpret_cast<const uint8_t*>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)p) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(p >> 32)) << 32);
@@ -1324,7 +1325,7 @@ __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(const uint8_t* p_w
 
     // ---- this wave's tiles: 16 rows, TPW groups of 16 tokens ----
     const uint32_t half = wave & 1u, mat = GATED ? (wave >> 1) & 1u : 0u, tg0 = (GATED ? wave >> 2 : wave >> 1) * TPW;
-    const bool multiplies = wave < (uint32_t)MW && 16u * tg0 < p_n;
+    const bool multiplies = wave < (uint32_t)MW && 16u * tg0 < n_here;
     uint32_t a_wt = lds + kSlab * mat + 2048u * (kq >> 1) + 16u * (16 * half + l16) + 8u * (kq & 1u);
     uint32_t a_dx = lds + kAtDx + 16u * (16 * tg0 + 4 * kq + (l16 & 3u)) + 4u * (l16 >> 2);
     uint32_t a_dws = lds + kSlab * mat + kSlabWt + 8u * (16 * half + l16);
@@ -1403,10 +1404,10 @@ __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(const uint8_t* p_w
 #pragma unroll
                         for (int r = 0; r < 4; r++) {
                             const uint32_t rw = GR * granule + 16 * half + l16, t = 16 * (tg0 + i) + 4 * kq + r;
-                            if (rw < a.m && t < p_n) {
+                            if (rw < a.m && t < n_here) {
                                 int v = D[i][b][r] - (int)kBiasBits;
                                 if (TYPE == 2) v >>= 4;  // weights were stored x16; exact
-                                a.dots[((size_t)t * a.m + rw) * nb + s * KB + b] = v;
+                                a.dots[((size_t)(tok0 + t) * a.m + rw) * nb + s * KB + b] = v;
                             }
                         }
             }
@@ -1444,9 +1445,9 @@ __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(const uint8_t* p_w
             float id;
             const float scale = q8_scale_and_inverse(group_max8(fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w)))), id);
             const uint32_t packed = q8_pack4(x.x, x.y, x.z, x.w, id);
-            if (tok < p_n) {
-                *reinterpret_cast<uint32_t*>(a.q_out + (size_t)tok * a.m + GR * granule + 4u * quad) = packed;
-                if (quad == 0) a.s_out[(size_t)tok * (a.m >> 5) + granule] = scale;
+            if (tok < n_here) {
+                *reinterpret_cast<uint32_t*>(a.q_out + (size_t)(tok0 + tok) * a.m + GR * granule + 4u * quad) = packed;
+                if (quad == 0) a.s_out[(size_t)(tok0 + tok) * (a.m >> 5) + granule] = scale;
             }
         }
     } else if constexpr (!DUMP) {
@@ -1454,13 +1455,13 @@ __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(const uint8_t* p_w
         if (!multiplies || row >= a.m) return;
         const size_t tok_step = side ? a.m : (a.y_row_major ? 1u : a.y_stride), row_step = side || !a.y_row_major ? 1u : a.y_stride;
         const bool add = !side && a.accumulate;
-        float* y = (side ? static_cast<float*>(const_cast<void*>(p_more)) + (size_t)my_share * p_n * a.m : a.y) + row * row_step;
+        float* y = (side ? static_cast<float*>(const_cast<void*>(p_more)) + (size_t)my_share * p_n * a.m : a.y) + row * row_step + tok0 * tok_step;
 #pragma unroll
         for (int i = 0; i < TPW; i++)
 #pragma unroll
             for (int r = 0; r < 4; r++) {
                 const uint32_t t = 16 * (tg0 + i) + 4 * kq + r;
-                if (t >= p_n) continue;
+                if (t >= n_here) continue;
                 const float v = walks ? total[i][r] + acc[i][r] : acc[i][r];
                 y[t * tok_step] = add ? y[t * tok_step] + v : v;
             }
@@ -1519,6 +1520,22 @@ bool few_side_applies(uint64_t rows, uint32_t n, uint32_t shares) {
     return n <= 64 && (rows + GR - 1) / GR * shares <= 2 * kCus;
 }
 
+// More tokens on that kernel, side by side in tiles of 32 or 64 (0: not): while the chip holds all of the workgroups at once, each slab is a
+// quarter of a 32 x 32 tile's chain and three slabs of cold weights are under way, not one.  In tiles of 32 while they are 7/4 a CU at most (beyond,
+// the 64-token tile's half as many weight copies count for more), else of 64 up to two a CU (their LDS); past that the larger tiles do more per byte read
+// from LDS.  64-row or 128-row tiles / 32 / 64 tokens here, us:
+//   one share:  1024 x 1024 over 100 7.7 / 4.7 / 5.4, 300 7.8 / 5.5 / 5.6, 555 8.0 / 7.6 / 7.0, 1300 10.1 / 11.9 / 11.1; 2048 x 2048 over 160 15.3 / 8.2 / 8.9,
+//               256 15.3 / 11.0 / 9.7, 400 15.5 / 16.0 / 12.6, 555 15.9 / 19.5 / 17.9; 4608 x 1024 over 130 9.6 / 8.6 / 7.9, 256 11.0 / 12.3 / 11.5; 3072 x 2048 over 300 15.8 / 17.6 / 13.9
+//   in shares:  1024 x 1024 in 4 over 130 4.5 / 3.9 / 3.8, 300 5.5 / 5.6 / 6.0; 1024 x 4608 in 8 over 72 7.3 / 6.5 / 6.0, 130 8.4 / 8.4 / 8.7; 2048 x 6912 in 8 over 72 11.2 / 12.9 / 12.4
+// Up to 832 tokens: over more, few rows only fit and little is left to gain (1024 x 1024 over 808 8.3 / 7.6, over 1000 8.4 / 8.1; x 2048 over 1000 13.1 / 12.9).
+// Weights of up to 512 x 512 elements, smaller than any projection of a model, stay on the 64-row tile, whose edges small launches check.
+uint32_t few_tokens_per_tile(uint64_t rows, uint32_t n, uint32_t k, uint32_t shares) {
+    const uint64_t units = (rows + GR - 1) / GR * shares;
+    if (n <= 64 || n > 832 || rows * k <= 512u * 512u) return 0;
+    if (4 * units * ((n + 31) / 32) <= 7 * kCus) return 32;
+    return units * ((n + 63) / 64) <= 2 * kCus ? 64 : 0;
+}
+
 // Shares of K one after the other in one launch of that kernel: ~0.3 us a slab up to 32 tokens, twice that above, against shares side by side and
 // the launch that adds them up, or, with `deferrable`, the additions in the norm's kernel behind the projection.  With the norm, side by
 // side is the faster way wherever few_side_applies (1024 x 1024 in 4 over 23 tokens 3.5 and 0.4 more in the norm, here 4.7); beyond, and plain:
@@ -1527,8 +1544,18 @@ bool few_side_applies(uint64_t rows, uint32_t n, uint32_t shares) {
 //   plain, 40:              1024 x 1024 7.2 / 7.0, 4096 x 1024 8.2 / 7.1; 2048 x 2048 8.2 / 11.5
 //   with the norm, 24:      4096 x 2048 13.3 / 12.5; over 40 tokens 3072 x 1024 11.3 / 11.6, 4096 x 1024 12.9 / 12.3
 // Without room for shares side by side: all that needs none, the faster way or not.
+// Above 64 tokens, against shares on the 64-row or 128-row tiles: the walk costs 0.3 us a slab and the other way the sums' round trip through memory:
+//   plain:                  3072 x 1024 over 66 8.7 / 5.4, 130 10.0 / 6.2, 320 13.3 / 8.0; 1024 x 1024 over 512 11.3 / 6.1; 2048 x 2048 over 66 9.4 / 7.7, 256 13.6 / 9.5;
+//                           1024 x 3072 over 96 8.5 / 9.7, 160 10.3 / 9.8; 1024 x 4608 over 200 12.1 / 13.7, 256 13.8 / 13.7; 512 x 4096 over 400 11.7 / 12.2, 512 12.9 / 12.3
+//   with the norm, a prompt of the 350M shape, all of it: 220 tokens 839 / 840, 300 963 / 947, 420 1039 / 1016, 680 1388 / 1394; of the 1.2B shape's first six layers
+//                           (2048 x 2048): 200 550 / 559, 300 689 / 685, 400 742 / 734
 bool few_applies_split(uint64_t rows, uint32_t n, uint32_t k, uint32_t shares, bool deferrable, bool room) {
     const uint64_t units = (rows + GR - 1) / GR, slabs = k / (KB * 32), cost = n <= 32 ? 1u : 2u;
+    if (n > 64) {
+        if (!few_tokens_per_tile(rows, n, k, 1)) return false;
+        if (deferrable) return slabs <= 16 && n <= 512 && rows * n >= 32768 * slabs && !few_tokens_per_tile(rows, n, k, shares);
+        return slabs <= 8 + rows * n / 9500;
+    }
     if (n > 64 || units > 2 * kCus || units * slabs > (cost == 1 ? 12288u : 4096u) || slabs * cost > (cost == 1 && units < 96 ? 15u : 16u)) return false;
     if (deferrable && 12 * slabs * cost > 72 + units) return false;
     return !room || (few_applies(rows, n, k) && !(deferrable && few_side_applies(rows, n, shares)));
@@ -1630,7 +1657,7 @@ hipError_t enqueue(Kernel kernel, uint32_t grid, uint32_t threads, const GemmArg
         return launch_kernel(L, kFamGemm, kernel, dim3(grid), dim3(threads), a.w, a.xq, a.xs, a.w_up, a.m, a.n, a.k, a.row_tiles, a.tok_tiles, shift | flag, a);
     } else {
         const void* const p_more = a.w_up ? static_cast<const void*>(a.w_up) : a.partial;
-        return launch_kernel(L, kFamGemm, kernel, dim3(grid), dim3(threads), a.w, a.xq, a.xs, p_more, a.n, a.k, a.row_tiles,
+        return launch_kernel(L, kFamGemm, kernel, dim3(grid, a.tok_tiles), dim3(threads), a.w, a.xq, a.xs, p_more, a.n, a.k, a.row_tiles,
                              shift | (shift && a.partial ? kFewSide : 0u) | flag, a);
     }
 }
@@ -1659,8 +1686,8 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, bool in_launch, uint32
         a.tok_tiles = (a.n + tokens - 1) / tokens;
         const uint32_t shares = a.ksplit;
         if ((uint64_t)a.row_tiles * a.tok_tiles * shares > 0x7fffff00ull) return hipErrorInvalidValue;  // beyond a launch's grid
-        // every XCD gets the same number of slots of the tile map; tile id = blockIdx.x / shares runs over all of them
-        const uint32_t grid = (a.row_tiles * a.tok_tiles + 7u) / 8u * 8u * (whole ? 1u : shares);  // whole: a workgroup takes all shares of its rows
+        // every XCD gets the same number of slots of the tile map; tile id = blockIdx.x / shares runs over all of them (gemm_few_kernel: tokens in blockIdx.y)
+        const uint32_t grid = (a.row_tiles * (rows == GR ? 1u : a.tok_tiles) + 7u) / 8u * 8u * (whole ? 1u : shares);  // whole: a workgroup takes all shares of its rows
         const hipError_t e = enqueue(kernel, grid, threads, a, shares, more != 0, L);
         if (e != hipSuccess || shares == 1 || defer_reduce || whole) return e;  // deferred: the caller's next kernel adds the shares up itself
         return launch_reduce(a, L);
@@ -1673,7 +1700,8 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, bool in_launch, uint32
             if (q8) return go(gemm_tile_kernel<8, true, false, C>, C::kRows, C::kTokens, C::kThreads);
         return go(gemm_tile_kernel<2, DUMP, false, C>, C::kRows, C::kTokens, C::kThreads);
     };
-    const bool few = !L.gemm_mfma16 && (ksplit > 1 ? in_launch || few_side_applies(a.m, a.n, ksplit) : few_applies(GR * tile_rows(GR), a.n, a.k));
+    const uint32_t few_tiled = L.gemm_mfma16 ? 0 : few_tokens_per_tile(GR * tile_rows(GR), a.n, a.k, in_launch ? 1u : ksplit);
+    const bool few = !L.gemm_mfma16 && (few_tiled || (ksplit > 1 ? in_launch || few_side_applies(a.m, a.n, ksplit) : few_applies(GR * tile_rows(GR), a.n, a.k)));
     const bool narrow = !wide_split && narrow_tiles(tile_rows(BM), a.n);
     if (few) {
         // Eight waves and 151 KB of LDS while every CU gets one workgroup at most, else four and half of it.
@@ -1681,9 +1709,10 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, bool in_launch, uint32
         const auto waves = [&](auto tg, auto wv) {
             constexpr int TG = decltype(tg)::value, WV = decltype(wv)::value;
             if constexpr (DUMP)
-                if (q8) return go(gemm_few_kernel<8, true, false, TG, WV>, GR, 64, 64 * WV, whole);
-            return go(gemm_few_kernel<2, DUMP, false, TG, WV>, GR, 64, 64 * WV, whole);
+                if (q8) return go(gemm_few_kernel<8, true, false, TG, WV>, GR, 32 * TG, 64 * WV, whole);
+            return go(gemm_few_kernel<2, DUMP, false, TG, WV>, GR, 32 * TG, 64 * WV, whole);
         };
+        if (few_tiled) return few_tiled == 32 ? waves(Idx<1>{}, Idx<4>{}) : waves(Idx<2>{}, Idx<8>{});
         if (tile_rows(GR) * (whole ? 1u : ksplit) <= kCus) return a.n <= 32 ? waves(Idx<1>{}, Idx<8>{}) : waves(Idx<2>{}, Idx<8>{});
         return a.n <= 32 ? waves(Idx<1>{}, Idx<4>{}) : waves(Idx<2>{}, Idx<4>{});
     }
@@ -1773,8 +1802,16 @@ bool gemm_gated_applies(uint32_t m, uint32_t n, uint32_t k) {
 }
 
 namespace {
-// The few-token form of the launch: one workgroup per granule and CU.
-bool gated_few_applies(uint32_t m, uint32_t n) { return n <= 64 && m / GR <= kCus; }
+// The few-token form of the launch: one workgroup per granule and CU, and 32 or 64 tokens (0: not).  Above 64 tokens, workgroups side by
+// side in tiles of 32 up to 7/4 a CU, else of 64 up to five quarters of a CU's worth, tiles of 16 tokens that have any counted.  TileQ's kind / 32 / 64 tokens here, us:
+// 4608 x 1024 over 72 13.1 / 8.7 / 10.2, 100 13.0 / 11.8 / 12.1, 160 13.6 / 13.5 / 13.7; 2816 x 1024 over 130 13.0 / 8.6 / 10.2, 200 13.3 / 12.2 / 12.3, 300 13.4 / 14.6 / 13.8;
+// 6912 x 2048 over 72 23.0 / 20.5 / 20.4, 100 24.0 / 26.3 / 24.6; 1024 x 2048 over 400 20.3 / 12.9 / 13.2; 4096 x 4096 over 160 39.1 / 40.8 / 31.7, 256 42.5 / 49.6 / 43.2.
+uint32_t gated_few_tokens(uint32_t m, uint32_t n) {
+    const uint64_t units = m / GR;
+    if (n <= 64) return units > kCus ? 0 : (n <= 32 ? 32 : 64);
+    if (4 * units * ((n + 31) / 32) <= 7 * kCus) return 32;
+    return units * ((n + 15) / 16) <= 5 * kCus ? 64 : 0;
+}
 
 // Where that form is the faster way: it saves a launch and the floats (2.7 us together), once, and each weight has half of a workgroup's waves, so that
 // it loses time with every slab against the projections alone (gemm_few_kernel as well where few_applies).  One launch / the projections' alone,
@@ -1801,7 +1838,7 @@ float gated_tile_cost(uint32_t m, uint32_t n, uint32_t k) { return tile_cost<C>(
 bool gemm_gated_faster(uint32_t m, uint32_t n, uint32_t k, const Launch& L) {
     if (gemm_gated_applies(m, n, k)) return true;
     if (L.gemm_mfma16 || m % GR != 0 || k % (KB * 32) != 0 || m == 0 || n == 0) return false;
-    if (gated_few_applies(m, n)) return gated_few_faster(m, n, k);
+    if (gated_few_tokens(m, n)) return n > 64 || gated_few_faster(m, n, k);
     if (n <= 48 && (uint64_t)2 * m / GR > 2 * kCus) return false;  // the narrow kernel's
     const auto plain = [&](auto cfg) {
         using C = decltype(cfg);
@@ -1821,9 +1858,9 @@ hipError_t launch_gemm_mfma_gated(int /*type: the copies are the same for both*/
     a.w = d_w_gate, a.w_up = d_w_up, a.xq = d_q, a.xs = d_scales, a.q_out = d_out_q, a.s_out = d_out_scales;
     a.m = m, a.n = n, a.k = k;
     a.tile_start[0] = a.tile_start[1] = UINT32_MAX;
-    if (gated_few_applies(m, n)) {
-        a.row_tiles = m / GR, a.tok_tiles = 1;
-        if (n > 32) return enqueue(gemm_few_kernel<2, false, true, 2, 8>, a.row_tiles, 512, a, 1, false, L);
+    if (const uint32_t tokens = gated_few_tokens(m, n)) {
+        a.row_tiles = m / GR, a.tok_tiles = (n + tokens - 1) / tokens;
+        if (tokens == 64) return enqueue(gemm_few_kernel<2, false, true, 2, 8>, a.row_tiles, 512, a, 1, false, L);
         return enqueue(gemm_few_kernel<2, false, true, 1, 8>, a.row_tiles, 512, a, 1, false, L);
     }
     const auto tile = [&](auto cfg) {
