@@ -101,7 +101,7 @@ def test_few_tokens_take_the_gate_into_the_launch_while_k_is_short(routes, tmp_p
 
 @pytest.mark.parametrize("tokens,kernel", [(200, "few_kernel<2, false, false, 2, 8>"),  # 512 tiles of 64 tokens, four shares
                                            (255, "few_kernel<2, false, false, 2, 8>"), (257, "few_kernel<2, false, false, 1, 4>"),  # 8 slabs, 256 x 1024 outputs
-                                           (512, "few_kernel<2, false, false, 2, 8>"), (513, "tile_kernel<2, false, false, TileN>")])
+                                           (512, "few_kernel<2, false, false, 2, 8>"), (513, "tile_kernel<2, false, false, TileH>"), (1000, "tile_kernel<2, false, false, TileN>")])
 def test_residual_projections_of_a_prompt(routes, tokens, kernel):
     """Shares of K that the norm behind adds up: side by side on the few-token kernel, walked by it, on the tiles."""
     assert routes(f"residual 1024 {tokens} 1024 8")[0][0] == f"gemm_{kernel}"
