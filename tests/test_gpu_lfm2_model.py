@@ -543,3 +543,23 @@ def test_short_prompts_at_the_edges_of_their_tiles(ctx, oracle, tmp_path, hidden
     finally:
         ctx.set_gemm_mfma_shape(32)
         model.free()
+
+
+@pytest.mark.parametrize("embd_type,hidden", [(W.Q6_K, 1280), (W.Q4_0, 1152), (W.Q8_0, 1152)])
+def test_a_prompts_rows_are_the_embeddings(ctx, oracle, tmp_path, embd_type, hidden):
+    """Rows past the lookup's 1024 elements, tokens past its groups of four: bit for bit the prompt given as the oracle's rows."""
+    kw = dict(n_layers=1, hidden=hidden, inter=256, n_heads=hidden // 64, kv_heads=(2,), vocab=256, embd_type=embd_type)
+    model, _, _ = load(ctx, oracle, tmp_path, **kw)
+    dtype, _, wb = lfm2_synth.build(oracle, **kw)[2]["token_embd.weight"]
+    tokens = np.random.default_rng(7).integers(0, 256, 21).astype(np.uint32)
+    tokens[[0, -1]] = 255, 0
+    try:
+        for n in (3, 4, 21):
+            rows = np.stack([L.embed_row(dtype, wb, int(t), hidden) for t in tokens[:n]])
+            got = [model.forward_prefill(tokens[:n], 0).view(np.uint32)]
+            model.reset()
+            got.append(model.forward_prefill_from_embeddings(rows, 0).view(np.uint32))
+            model.reset()
+            assert np.array_equal(*got), f"{n} tokens"
+    finally:
+        model.free()

@@ -95,13 +95,52 @@ __global__ __launch_bounds__(256) void embed_row_kernel(const uint8_t* __restric
     for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < k; e += gridDim.x * blockDim.x) out[e] = dequant_element(w, type, row, k, e);
 }
 
-// The rows of a whole prompt: out[j][k] = row d_tokens[j] (blockIdx.y = j).
-__global__ __launch_bounds__(256) void embed_rows_kernel(const uint8_t* __restrict__ w, int type, uint32_t m, uint32_t k,
-                                                         const uint32_t* __restrict__ d_tokens, float* __restrict__ out) {
-    const uint32_t row = d_tokens[blockIdx.y];
-    if (row >= m) return;
-    float* o = out + (size_t)blockIdx.y * k;
-    for (uint32_t e = blockIdx.x * blockDim.x + threadIdx.x; e < k; e += gridDim.x * blockDim.x) o[e] = dequant_element(w, type, row, k, e);
+// The rows of a whole prompt: out[j][k] = row d_tokens[j].  The tokens are where the host wrote them, in its own memory, and a read over the bus is what the
+// launch waits for: a wave takes kEmbedRows tokens with one of them, a lane four elements of each, everything requested together.  Element
+// for element dequant_element.  (Before, a read over the bus per wave of
+// 64 elements, and now, us: 555 tokens x 1024 6.2 / 4.9, 808 6.8 / 5.6, 2002 x 2048 22.2 / 9.2.)
+constexpr uint32_t kEmbedRows = 4;
+template <int TYPE>
+__global__ __launch_bounds__(256) void embed_rows_kernel(const uint32_t* __restrict__ d_tokens, const uint8_t* __restrict__ w, float* __restrict__ out, uint32_t m,
+                                                         uint32_t k, uint32_t n) {
+    const uint32_t j0 = kEmbedRows * blockIdx.y, mine = d_tokens[min(j0 + (threadIdx.x & (kEmbedRows - 1u)), n - 1u)];
+    const uint32_t e = 4u * (blockIdx.x * 256u + threadIdx.x), ee = e < k ? e : 0u;
+    const auto two = [](const uint8_t* p) { return (uint32_t)*reinterpret_cast<const uint16_t*>(p); };  // (blocks are even numbers of bytes)
+    uint32_t row[kEmbedRows], lo[kEmbedRows][2], hi[kEmbedRows][2], d[kEmbedRows], sc[kEmbedRows];
+#pragma unroll
+    for (uint32_t i = 0; i < kEmbedRows; i++) {
+        row[i] = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)i);
+        const size_t r = row[i] < m ? row[i] : 0u;
+        if constexpr (TYPE == kTypeQ6_K) {
+            const uint8_t* const blk = w + (r * (k >> 8) + (ee >> 8)) * kQ6KBlockBytes;
+            const uint32_t q = ee & 255u, half = q >> 7, part = (q >> 5) & 3u, l = q & 31u;
+            const uint8_t *const ql = blk + 64u * half + 32u * (part & 1u) + l, *const qh = blk + 128u + 32u * half + l;
+            lo[i][0] = two(ql), lo[i][1] = two(ql + 2), hi[i][0] = two(qh), hi[i][1] = two(qh + 2), d[i] = two(blk + 208), sc[i] = blk[192 + (q >> 4)];
+        } else {
+            const uint8_t* const blk = w + (r * (k >> 5) + (ee >> 5)) * (TYPE == kTypeQ4_0 ? kQ4BlockBytes : kQ8BlockBytes);
+            const uint8_t* const qs = blk + 2 + (ee & (TYPE == kTypeQ4_0 ? 15u : 31u));
+            lo[i][0] = two(qs), lo[i][1] = two(qs + 2), d[i] = two(blk);
+        }
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kEmbedRows; i++) {
+        const float df = f16_bits_to_f32(d[i]);
+        float v[4];
+#pragma unroll
+        for (uint32_t b = 0; b < 4; b++) {
+            const uint32_t l = lo[i][b >> 1] >> (8u * (b & 1u)) & 255u;
+            if constexpr (TYPE == kTypeQ6_K) {
+                const uint32_t part = (ee >> 5) & 3u, h = hi[i][b >> 1] >> (8u * (b & 1u)) & 255u;
+                const int q = (int)((l >> (4u * (part >> 1)) & 15u) | (h >> (2u * part) & 3u) << 4) - 32;
+                v[b] = __fmul_rn(__fmul_rn(df, (float)(int)(int8_t)sc[i]), (float)q);
+            } else if constexpr (TYPE == kTypeQ4_0) {
+                v[b] = __fmul_rn((float)((int)((ee & 16u) ? l >> 4 : l & 15u) - 8), df);
+            } else {
+                v[b] = __fmul_rn((float)(int)(int8_t)l, df);
+            }
+        }
+        if (e < k && j0 + i < n && row[i] < m) *reinterpret_cast<float4*>(out + (size_t)(j0 + i) * k + e) = make_float4(v[0], v[1], v[2], v[3]);
+    }
 }
 
 // ---- RMSNorm ---------------------------------------------------------------------------
@@ -1988,8 +2027,10 @@ hipError_t launch_shortconv_step(const float* d_proj, float* d_buffer, const flo
 hipError_t launch_embed_rows(const uint8_t* d_w, int type, uint32_t m, uint32_t k, const uint32_t* d_tokens, uint32_t n, float* d_out,
                              const Launch& L) {
     if (n == 0) return hipSuccess;
-    const uint32_t blocks = (k + 255u) / 256u;
-    return launch_kernel(L, kFamOther, embed_rows_kernel, dim3(blocks < 16u ? blocks : 16u, n), dim3(256), d_w, type, m, k, d_tokens, d_out);
+    const auto go = [&](auto kernel) {
+        return launch_kernel(L, kFamOther, kernel, dim3((k + 1023u) / 1024u, (n + kEmbedRows - 1u) / kEmbedRows), dim3(256), d_tokens, d_w, d_out, m, k, n);
+    };
+    return type == kTypeQ6_K ? go(embed_rows_kernel<kTypeQ6_K>) : (type == kTypeQ4_0 ? go(embed_rows_kernel<kTypeQ4_0>) : go(embed_rows_kernel<kTypeQ8_0>));
 }
 
 hipError_t launch_shortconv_seq(const float* d_proj, float* d_buffer, const float* d_conv_w, float* d_out, uint32_t hidden,
