@@ -563,3 +563,18 @@ def test_a_prompts_rows_are_the_embeddings(ctx, oracle, tmp_path, embd_type, hid
             assert np.array_equal(*got), f"{n} tokens"
     finally:
         model.free()
+
+
+@pytest.mark.parametrize("kv_heads", [(2, 0), (0, 2)])
+def test_a_prompt_of_two_passes_is_the_two_prompts(ctx, oracle, tmp_path, kv_heads):
+    """A pass that is not the last stops at the last layer's state: the same state and logits as the two passes as prompts of their own."""
+    model, _, _ = load(ctx, oracle, tmp_path, context=2200, n_layers=2, hidden=128, inter=128, n_heads=2, kv_heads=kv_heads, vocab=256, embd_type=W.Q8_0)
+    tokens = np.random.default_rng(9).integers(0, 256, 2048 + 77).astype(np.uint32)
+    try:
+        got = [(model.forward_prefill(tokens, 0).view(np.uint32), model.snapshot_state(tokens.size))]
+        model.reset()
+        model.forward_prefill(tokens[:2048], 0)
+        got.append((model.forward_prefill(tokens[2048:], 2048).view(np.uint32), model.snapshot_state(tokens.size)))
+        assert all(np.array_equal(a, b) for a, b in zip(*got))
+    finally:
+        model.free()

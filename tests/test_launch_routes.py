@@ -114,6 +114,16 @@ def test_residual_projections_of_a_prompt(routes, tokens, kernel):
 ])
 def test_prompts_take_the_gate_into_the_few_token_kernel(routes, tmp_path, inter, tokens, kernel):
     path = tmp_path / "model.gguf"
-    path.write_bytes(bytes(lfm2_synth.build(Zeros, n_layers=1, hidden=1024, inter=inter, n_heads=16, kv_heads=(0,), embd_type=Q8_0)[0]))
+    path.write_bytes(bytes(lfm2_synth.build(Zeros, n_layers=2, hidden=1024, inter=inter, n_heads=16, kv_heads=(0, 0), embd_type=Q8_0)[0]))
     kernels, = routes(f"prompt {path} {tokens}")
     assert f"gemm_{kernel}" in kernels and "silu_mul_quantize_kernel" not in kernels
+
+
+def test_the_last_layer_is_for_the_last_token(routes, tmp_path):
+    """Past 64 tokens its feed-forward block is a product of one token, and a pass that is not the last one does without."""
+    path = tmp_path / "model.gguf"
+    path.write_bytes(bytes(lfm2_synth.build(Zeros, n_layers=1, hidden=1024, inter=1024, n_heads=16, kv_heads=(0,), embd_type=Q8_0)[0]))
+    short, long, passes = routes(f"prompt {path} 64", f"prompt {path} 65", f"prompt {path} 2113")
+    gated, one = "gemm_few_kernel<2, false, true, 2, 8>", "gemm_few_kernel<2, false, true, 1, 8>"
+    assert gated in short and one not in short and gated not in long and one in long
+    assert passes[-len(long) + 3:] == long[3:] and len(passes) < 2 * len(long) and passes.count(one) == 1

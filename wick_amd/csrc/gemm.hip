@@ -1782,6 +1782,18 @@ hipError_t launch_gemm_mfma(int type, const uint8_t* d_w, uint32_t m, uint32_t k
     return launch<false>(type, a, L, in_launch, 0, defer_reduce);
 }
 
+// One token of a launch over more.  A row's sum is fixed by the shares of K and by nothing else of the launch.
+hipError_t launch_gemm_mfma_row(const uint8_t* d_w, uint32_t m, uint32_t k, const int8_t* d_q, const float* d_scales, float* d_y, const Launch& L,
+                                uint32_t splits, float* d_partial) {
+    if (L.gemm_mfma16) return hipErrorInvalidValue;
+    GemmArgs a{};
+    a.w = d_w, a.xq = d_q, a.xs = d_scales, a.y = d_y;
+    a.m = m, a.n = 1, a.k = k, a.y_stride = m;
+    a.accumulate = 1;
+    if (splits > 1) a.ksplit = splits, a.partial = d_partial;
+    return launch<false>(kTypeQ4_0, a, L, splits > 1 && !d_partial);
+}
+
 // The same launch over up to three weights of one type and k that share the activations: outputs y[i] (same stride,
 // layout and accumulate flag), tiles of all weights in one tile list.
 hipError_t launch_gemm_mfma_multi(int type, const uint8_t* const* d_w, const uint32_t* m, uint32_t count, uint32_t k, const int8_t* d_q,

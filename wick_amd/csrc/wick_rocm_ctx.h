@@ -135,6 +135,9 @@ struct HostPiece {
 // Copies the pieces in stream order and waits (lock held, not capturing).  The device addresses are the library's own: they go
 // to a kernel unchecked.  api.hip.
 int copy_pieces(wick_rocm_ctx* ctx, const HostPiece* pieces, size_t count, bool to_host);
+// y += W x for one token of a batched product over n, to the bit (gemm_row_applies: where that product is the matrix cores'; lock held).
+bool gemm_row_applies(wick_rocm_ctx* ctx, const wick_rocm_weight* w, uint32_t n);
+int gemm_row(wick_rocm_ctx* ctx, const wick_rocm_weight* w, const int8_t* d_q, const float* d_s, uint32_t n, float* d_y);
 
 // Takes the context lock and makes its device current for the calling thread.
 struct Guard {
