@@ -1633,7 +1633,10 @@ float tile_cost(uint64_t row_tiles, uint32_t n, uint32_t k, uint32_t shares, boo
     // Shares of K whose second workgroup only some CUs have: the small tile gives way by what the others leave it of the caches (128-row / 64-row tile, us,
     // and workgroups a CU: 1024 x 4608 in 2 over 555 19.0 / 17.8 and 1.13, 700 19.4 / 18.6 and 1.38, 900 in 4 18.3 / 20.0; in 4 over 300 11.8 / 11.2 and 1.25,
     // 420 12.2 / 12.0 and 1.63, 480 12.4 / 12.4 and 1.88; 2048 x 6912 in 2 over 300 27.2 / 25.3 and 1.25, 360 27.9 / 28.6 and 1.5).
-    if (shares > 1 && C::kPerCu == 4 && per_cu == 2) per_slab *= 1.0f - 0.14f * (2.0f - (float)tiles / (float)kCus);
+    if (shares > 1 && C::kRows == 64 && per_cu == 2) per_slab *= 1.0f - 0.14f * (2.0f - (float)tiles / (float)kCus);
+    // Past the four that are on a CU at a time its many stores of shares count (TileQ / 64-row tile, us: 2048 x 6912 in 4 over 555 32.3 / 35.0, 620
+    // 35.2 / 37.2; in 2 over 1200 56.6 / 57.2).
+    if (shares > 1 && C::kRows == 64 && per_cu > 4) per_slab *= 1.06f;
     return per_slab * (float)k / (float)(KB * 32 * shares) + (float)per_cu * c.fixed;
 }
 // go(tile) for the one of them that cost(tile) is lowest for.
