@@ -525,7 +525,7 @@ def test_a_prompt_is_the_same_on_either_block_loop(ctx, oracle, tmp_path, wtype)
         model.free()
 
 
-@pytest.mark.parametrize("hidden,inter", [(128, 1152), (640, 128), (1152, 640)])
+@pytest.mark.parametrize("hidden,inter", [(128, 1152), (640, 128), (1152, 640), (128, 1952), (1152, 1152)])
 def test_short_prompts_at_the_edges_of_their_tiles(ctx, oracle, tmp_path, hidden, inter):
     """The few-token launches on both sides of their 16-token tiles, gate | up in one launch among them, over 1, 5 and 9 slabs of K (fewer than
     their ring of stages holds, one more, and twice round), and over several tiles of 32 and 64 tokens: bit for bit the 16x16x32 kernels, which take

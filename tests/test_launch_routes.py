@@ -107,14 +107,15 @@ def test_residual_projections_of_a_prompt(routes, tokens, kernel):
     assert routes(f"residual 1024 {tokens} 1024 8")[0][0] == f"gemm_{kernel}"
 
 
-@pytest.mark.parametrize("inter,tokens,kernel", [
-    (3584, 65, "few_kernel<2, false, true, 1, 8>"), (3584, 128, "few_kernel<2, false, true, 1, 8>"),  # 448 tiles of 32 tokens
-    (3584, 129, "few_kernel<2, false, true, 2, 8>"),
-    (4096, 160, "few_kernel<2, false, true, 2, 8>"), (4096, 161, "tile_kernel<2, false, true, TileS>"),  # 1280 of 16
+@pytest.mark.parametrize("hidden,inter,tokens,kernel", [
+    (1024, 3584, 65, "few_kernel<2, false, true, 1, 8>"), (1024, 3584, 128, "few_kernel<2, false, true, 1, 8>"),  # 448 tiles of 32 tokens
+    (1024, 2048, 280, "few_kernel<2, false, true, 2, 8>"), (1024, 2048, 281, "tile_kernel<2, false, true, TileN>"),  # 256 of 64
+    (1024, 4096, 256, "tile_kernel<2, false, true, TileN>"), (1024, 4096, 257, "tile_kernel<2, false, true, TileS>"),  # 256 tiles of 64 rows
+    (2048, 4096, 160, "few_kernel<2, false, true, 2, 8>"), (2048, 4096, 161, "tile_kernel<2, false, true, TileN>"),  # 1280 of 16 tokens
 ])
-def test_prompts_take_the_gate_into_the_few_token_kernel(routes, tmp_path, inter, tokens, kernel):
+def test_prompts_take_the_gate_into_the_few_token_kernel(routes, tmp_path, hidden, inter, tokens, kernel):
     path = tmp_path / "model.gguf"
-    path.write_bytes(bytes(lfm2_synth.build(Zeros, n_layers=2, hidden=1024, inter=inter, n_heads=16, kv_heads=(0, 0), embd_type=Q8_0)[0]))
+    path.write_bytes(bytes(lfm2_synth.build(Zeros, n_layers=2, hidden=hidden, inter=inter, n_heads=hidden // 64, kv_heads=(0, 0), embd_type=Q8_0)[0]))
     kernels, = routes(f"prompt {path} {tokens}")
     assert f"gemm_{kernel}" in kernels and "silu_mul_quantize_kernel" not in kernels
 

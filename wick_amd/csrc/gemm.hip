@@ -823,8 +823,8 @@ __global__ __launch_bounds__(C::kThreads, DUMP ? 1 : C::kOcc) void gemm_tile_ker
     asm volatile("" : "+v"(cbias));  // keep it in registers (left alone, the compiler rebuilds it before every MFMA)
 
     // This lane's LDS bases; everything else of an address is an immediate.
-    // (granule rt of a wave: its RT consecutive ones of the tile, or its RT / 2 of gate and the same RT / 2 of up)
-    constexpr int kOwn = GATED ? RT / 2 : RT;
+    // (granule rt of a wave: its RT consecutive ones of the tile, or its RT / 2 of gate and the same RT / 2 of up; RT == 1: one of either)
+    constexpr int kOwn = GATED && RT > 1 ? RT / 2 : RT;
     uint32_t a_wt = lds_addr(&sm.st[0].wt[kOwn * wr][kh][0][l32]);
     uint32_t a_dws = lds_addr(&sm.st[0].dws[kOwn * wr][0][l32]);
     // token scales: the first of the lane's four groups of four, or (T == 1) the lane of every 16 that holds the scale of their result e reads
@@ -1000,7 +1000,49 @@ __global__ __launch_bounds__(C::kThreads, DUMP ? 1 : C::kOcc) void gemm_tile_ker
         end_stage();
     }
 
-    if constexpr (GATED) {
+    if constexpr (GATED && RT == 1) {
+        // The same as below where a wave has a granule of gate or of up: it takes sixteen tokens of both, hands the other wave the other sixteen and
+        // quantizes its own.
+        constexpr int kRow = 36;
+        static_assert(C::WR == 4 && TT == 1 && sizeof(sm) >= sizeof(float) * (8 * 64 + 16 * kRow) * C::kWaves, "gate waves, then up waves");
+        float* const ex = reinterpret_cast<float*>(&sm);  // [wave][8][lane]
+        float* const h = ex + 8 * 64 * C::kWaves + 16 * kRow * wave;
+        const bool up = wr >= 2u;
+#pragma unroll
+        for (int e = 0; e < 8; e++) ex[64 * (8 * wave + e) + lane] = up ? acc[0][0][e] : acc[0][0][8 + e];
+        __syncthreads();
+        float g[8], u[8], v[8], far = 0.0f, small = 1.0f;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const float its = ex[64 * (8 * (wave ^ (2u * C::WT)) + e) + lane];
+            g[e] = up ? its : acc[0][0][e], u[e] = up ? acc[0][0][8 + e] : its;
+            v[e] = silu_mul_near(g[e], u[e], far, small);
+        }
+        if (__builtin_amdgcn_ballot_w64(!silu_mul_was_near(far, small)) != 0) {
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] = silu_mul(g[e], u[e]);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) h[kRow * (4 * kh + 8 * (e >> 2) + (e & 3)) + l32] = v[e];
+        const uint32_t rbase = row0 + 32u * (wr & 1u), tok = tok0 + 32 * wt + (up ? 16u : 0u) + (lane >> 3), mine = lane & 1u;
+        if (rbase < a.m) {
+            float4 x[2];
+            float amax[2], id;
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                x[i] = *reinterpret_cast<const float4*>(&h[kRow * (8u * i + (lane >> 3)) + 4u * (lane & 7u)]);
+                amax[i] = group_max8(fmaxf(fmaxf(fabsf(x[i].x), fabsf(x[i].y)), fmaxf(fabsf(x[i].z), fabsf(x[i].w))));
+            }
+            const float scale = q8_scale_and_inverse(mine ? amax[1] : amax[0], id);
+            if ((lane & 7u) < 2u && tok + 8u * mine < a.n) a.s_out[(size_t)(tok + 8u * mine) * (a.m >> 5) + (rbase >> 5)] = scale;
+            static_for<2>([&](auto i_) {
+                constexpr int i = decltype(i_)::value;
+                const float idi = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(id), 0x55 * i, 0xf, 0xf, false));
+                const uint32_t packed = q8_pack4(x[i].x, x[i].y, x[i].z, x[i].w, idi);
+                if (tok + 8u * i < a.n) *reinterpret_cast<uint32_t*>(a.q_out + (size_t)(tok + 8u * i) * a.m + rbase + 4u * (lane & 7u)) = packed;
+            });
+        }
+    } else if constexpr (GATED) {
         // silu(gate) * up and the Q8_0 quantizer, element for element what silu_mul_quantize_kernel computes from the two float
         // results: granules 0 .. RT / 2 - 1 of the wave are gate rows, the others the same rows of up, 32 rows = one Q8_0 block of a
         // token.  The gated values go through a wave-private piece of LDS (the stages are done with), so that eight lanes own a block
@@ -1618,7 +1660,7 @@ struct TileQ : T32<2, 1, 2, 2, 2, 4, false, true> {  // the same with half a sla
 };
 struct TileN : T32<1, 1, 4, 2, 4, 4> {  // 128 x 64, 8 waves of 32 x 32
     static constexpr int kPerCu = 2;
-    static constexpr TileCost kCost[2] = {{{0.70f, 1.25f}, 1.53f}, {}};
+    static constexpr TileCost kCost[2] = {{{0.70f, 1.25f}, 1.53f}, {{0.94f, 1.45f}, 0.9f}};  // (with the gate: see gated_tile_n)
 };
 struct TileH : T32<1, 1, 2, 2, 4, 4> {  // 64 x 64, 4 waves of 32 x 32
     static constexpr int kPerCu = 4;
@@ -1822,15 +1864,21 @@ bool gemm_gated_applies(uint32_t m, uint32_t n, uint32_t k) {
 
 namespace {
 // The few-token form of the launch: one workgroup per granule and CU, and 32 or 64 tokens (0: not).  Above 64 tokens, workgroups side by
-// side in tiles of 32 up to 7/4 a CU, else of 64 up to five quarters of a CU's worth, tiles of 16 tokens that have any counted.  TileQ's kind / 32 / 64 tokens here, us:
-// 4608 x 1024 over 72 13.1 / 8.7 / 10.2, 100 13.0 / 11.8 / 12.1, 160 13.6 / 13.5 / 13.7; 2816 x 1024 over 130 13.0 / 8.6 / 10.2, 200 13.3 / 12.2 / 12.3, 300 13.4 / 14.6 / 13.8;
-// 6912 x 2048 over 72 23.0 / 20.5 / 20.4, 100 24.0 / 26.3 / 24.6; 1024 x 2048 over 400 20.3 / 12.9 / 13.2; 4096 x 4096 over 160 39.1 / 40.8 / 31.7, 256 42.5 / 49.6 / 43.2.
-uint32_t gated_few_tokens(uint32_t m, uint32_t n) {
+// side in tiles of 32 up to 7/4 a CU, else of 64 while every workgroup of more than 24 tokens has a CU, or from 16 slabs on up to five quarters of a CU's worth, tiles of 16
+// tokens that have any counted.  TileQ's kind / 32 / 64 tokens here, us: 4608 x 1024 over 72 13.1 / 8.7 / 10.2, 2816 x 1024 over 130 13.0 / 8.6 / 10.2;
+// 2048 x 1024 over 256 13.0 / 9.0 / 9.2; over 280 13.0 / - / 10.7 and TileN below 11.3; 6912 x 2048 over 72 23.0 / 20.5 / 20.4; 1024 x 2048 over 400 20.3 / 12.9 / 13.2; 4096 x 4096 over 160 39.1 / 40.8 / 31.7.
+uint32_t gated_few_tokens(uint32_t m, uint32_t n, uint32_t k) {
     const uint64_t units = m / GR;
     if (n <= 64) return units > kCus ? 0 : (n <= 32 ? 32 : 64);
     if (4 * units * ((n + 31) / 32) <= 7 * kCus) return 32;
-    return units * ((n + 15) / 16) <= 5 * kCus ? 64 : 0;
+    if (units * ((n + 39) / 64) <= kCus) return 64;
+    return k >= 16 * KB * 32 && units * ((n + 15) / 16) <= 5 * kCus ? 64 : 0;
 }
+
+// TileN with the gate: past those, while every workgroup has a CU, whose eight waves make shorter slabs of it than four do.  The cheapest of the
+// other tiles or 64 tokens above / here, us: 4608 x 1024 over 128 12.5 / 11.7, 160 13.4 / 11.8, 200 (288 workgroups) 15.9 / 16.4; 6912 x 2048 over 100 22.7 / 20.8, 160
+// (324) 28.6 / 28.6; 2816 x 1024 over 300 13.3 / 11.6; 2048 x 1024 over 400 13.3 / 11.4; 4096 x 4096 over 200 41.3 / 36.6, 300 (320) 48.8 / 49.5.
+bool gated_tile_n(uint32_t m, uint32_t n) { return n > 64 && (uint64_t)((m + 63) / 64) * ((n + 63) / 64) <= kCus; }
 
 // Where that form is the faster way: it saves a launch and the floats (2.7 us together), once, and each weight has half of a workgroup's waves, so that
 // it loses time with every slab against the projections alone (gemm_few_kernel as well where few_applies).  One launch / the projections' alone,
@@ -1857,14 +1905,15 @@ float gated_tile_cost(uint32_t m, uint32_t n, uint32_t k) { return tile_cost<C>(
 bool gemm_gated_faster(uint32_t m, uint32_t n, uint32_t k, const Launch& L) {
     if (gemm_gated_applies(m, n, k)) return true;
     if (L.gemm_mfma16 || m % GR != 0 || k % (KB * 32) != 0 || m == 0 || n == 0) return false;
-    if (gated_few_tokens(m, n)) return n > 64 || gated_few_faster(m, n, k);
+    if (gated_few_tokens(m, n, k)) return n > 64 || gated_few_faster(m, n, k);
     if (n <= 48 && (uint64_t)2 * m / GR > 2 * kCus) return false;  // the narrow kernel's
     const auto plain = [&](auto cfg) {
         using C = decltype(cfg);
         return tile_cost<C>(2 * (uint64_t)((m + C::kRows - 1) / C::kRows), n, k, 1);
     };
     const float separate = std::min({plain(TileL{}), plain(TileX{}), plain(TileS{}), plain(TileQ{}), plain(TileN{}), plain(TileH{})});
-    const float gated = std::min({gated_tile_cost<TileL>(m, n, k), gated_tile_cost<TileX>(m, n, k), gated_tile_cost<TileS>(m, n, k), gated_tile_cost<TileQ>(m, n, k)});
+    float gated = std::min({gated_tile_cost<TileL>(m, n, k), gated_tile_cost<TileX>(m, n, k), gated_tile_cost<TileS>(m, n, k), gated_tile_cost<TileQ>(m, n, k)});
+    if (gated_tile_n(m, n)) gated = std::min(gated, gated_tile_cost<TileN>(m, n, k));
     return !few_applies(2 * (uint64_t)m, n, k) && gated < separate + 2.7f + (float)n * (float)m * 3e-6f;
 }
 
@@ -1877,7 +1926,7 @@ hipError_t launch_gemm_mfma_gated(int /*type: the copies are the same for both*/
     a.w = d_w_gate, a.w_up = d_w_up, a.xq = d_q, a.xs = d_scales, a.q_out = d_out_q, a.s_out = d_out_scales;
     a.m = m, a.n = n, a.k = k;
     a.tile_start[0] = a.tile_start[1] = UINT32_MAX;
-    if (const uint32_t tokens = gated_few_tokens(m, n)) {
+    if (const uint32_t tokens = gated_few_tokens(m, n, k)) {
         a.row_tiles = m / GR, a.tok_tiles = (n + tokens - 1) / tokens;
         if (tokens == 64) return enqueue(gemm_few_kernel<2, false, true, 2, 8>, a.row_tiles, 512, a, 1, false, L);
         return enqueue(gemm_few_kernel<2, false, true, 1, 8>, a.row_tiles, 512, a, 1, false, L);
@@ -1888,6 +1937,7 @@ hipError_t launch_gemm_mfma_gated(int /*type: the copies are the same for both*/
         if ((uint64_t)a.row_tiles * a.tok_tiles > 0x7fffff00ull) return hipErrorInvalidValue;
         return enqueue(gemm_tile_kernel<2, false, true, C>, (a.row_tiles * a.tok_tiles + 7u) / 8u * 8u, C::kThreads, a, 1, false, L);
     };
+    if (gated_tile_n(m, n)) return tile(TileN{});
     return cheapest_tile<TileL, TileX, TileS, TileQ>([&](auto cfg) { return gated_tile_cost<decltype(cfg)>(m, n, k); }, tile);
 }
 
