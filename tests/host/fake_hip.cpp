@@ -81,12 +81,16 @@ void enqueue(std::function<void()> f) {
     if (!st().capturing) st().queue.push_back(std::move(f));
 }
 
-hipError_t launch(const void* f, void** args, hipStream_t stream) {
+hipError_t launch(const void* f, dim3 grid, void** args, hipStream_t stream) {
     Lock lk;
     if (reinterpret_cast<uintptr_t>(stream) != (uintptr_t)current + 1) fake_hip::other_device++;
     if (due(st().launch_fails)) return done(hipErrorLaunchFailure);
     fake_hip::launches++;
     st().enqueued.push_back(st().kernels[f]);
+    if (st().kernels[f].find("rmsnorm_quantize_kernel") != std::string::npos) {  // (x, shares, their stride, weight, quants, scales, dim, ..)
+        const size_t elements = (size_t)grid.x * *static_cast<uint32_t*>(args[6]);
+        if (!covers(*static_cast<void**>(args[4]), elements) || !covers(*static_cast<void**>(args[5]), elements / 32 * sizeof(float))) fake_hip::out_of_range++;
+    }
     if (st().kernels[f].find("stage_copy_kernel") == std::string::npos) {
         enqueue([] {});
         return hipSuccess;
@@ -175,8 +179,8 @@ hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shared, hi
     *grid = config.grid, *block = config.block, *shared = config.shared, *stream = config.stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t s) { return launch(f, args, s); }
-hipError_t hipExtLaunchKernel(const void* f, dim3, dim3, void** args, size_t, hipStream_t s, hipEvent_t, hipEvent_t, int) { return launch(f, args, s); }
+hipError_t hipLaunchKernel(const void* f, dim3 grid, dim3, void** args, size_t, hipStream_t s) { return launch(f, grid, args, s); }
+hipError_t hipExtLaunchKernel(const void* f, dim3 grid, dim3, void** args, size_t, hipStream_t s, hipEvent_t, hipEvent_t, int) { return launch(f, grid, args, s); }
 
 hipError_t hipGetDeviceCount(int* n) {
     *n = 2;

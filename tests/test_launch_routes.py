@@ -128,3 +128,12 @@ def test_the_last_layer_is_for_the_last_token(routes, tmp_path):
     gated, one = "gemm_few_kernel<2, false, true, 2, 8>", "gemm_few_kernel<2, false, true, 1, 8>"
     assert gated in short and one not in short and gated not in long and one in long
     assert passes[-len(long) + 3:] == long[3:] and len(passes) < 2 * len(long) and passes.count(one) == 1
+
+
+def test_the_last_token_has_room_for_its_norm(routes, tmp_path):
+    """A row of hidden elements longer than all gated rows of the prompt together: the norm in front of the last token's feed-forward block
+    stays in its buffers (the pretended runtime looks)."""
+    path = tmp_path / "model.gguf"
+    path.write_bytes(bytes(lfm2_synth.build(Zeros, n_layers=1, hidden=8448, inter=128, n_heads=132, kv_heads=(2,), embd_type=Q8_0)[0]))
+    kernels, = routes(f"prompt {path} 65")
+    assert "gemm_few_kernel<2, false, true, 1, 8>" in kernels

@@ -553,11 +553,12 @@ int ensure_prefill_buffers(wick_rocm_ctx* ctx, wick_rocm_lfm2* m) {
     const wick_rocm_lfm2_config& c = m->cfg;
     const size_t P = c.max_seq_len < kPrefillChunk ? c.max_seq_len : kPrefillChunk;
     const size_t hs = c.hidden_size, inter = c.intermediate_size, hd = hs / c.n_heads, wide = hs > inter ? hs : inter;
+    const size_t q2 = P * inter > hs ? P * inter : hs;  // gated rows of every token, or the last token's norm (last_token)
     int rc;
     if ((rc = alloc_t(ctx, m, P * hs, &m->pX)) || (rc = alloc_t(ctx, m, P * 3 * hs, &m->pA)) ||
         (rc = alloc_t(ctx, m, P * hs, &m->pG)) || (rc = alloc_t(ctx, m, P * inter, &m->pGate)) || (rc = alloc_t(ctx, m, P * inter, &m->pUp)) ||
         (rc = alloc_t(ctx, m, P * wide, &m->pQ)) || (rc = alloc_t(ctx, m, P * (wide / 32), &m->pS)) ||
-        (rc = alloc_t(ctx, m, P * inter, &m->pQ2)) || (rc = alloc_t(ctx, m, P * (inter / 32), &m->pS2)) ||
+        (rc = alloc_t(ctx, m, q2, &m->pQ2)) || (rc = alloc_t(ctx, m, q2 / 32, &m->pS2)) ||
         (rc = alloc_t(ctx, m, attention_prefill_scratch_floats((uint32_t)P, c.n_heads, (uint32_t)hd), &m->pAttn)))
         return rc;
     // room for the K shares of a split projection, once: no prompt then regrows the context's scratch (a regrow waits for the
