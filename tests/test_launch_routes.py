@@ -137,3 +137,13 @@ def test_the_last_token_has_room_for_its_norm(routes, tmp_path):
     path.write_bytes(bytes(lfm2_synth.build(Zeros, n_layers=1, hidden=8448, inter=128, n_heads=132, kv_heads=(2,), embd_type=Q8_0)[0]))
     kernels, = routes(f"prompt {path} 65")
     assert "gemm_few_kernel<2, false, true, 1, 8>" in kernels
+
+
+def test_arguments_in_front_of_a_struct_are_no_pointers(host_faults, tmp_path):
+    """The fields that a kernel takes once more, to have them in registers when it starts: numbers, which the runtime does not look up at every launch."""
+    path = tmp_path / "model.gguf"
+    path.write_bytes(bytes(lfm2_synth.build(Zeros, n_layers=2, hidden=1024, inter=4608, n_heads=16, kv_heads=(0, 2), embd_type=Q8_0)[0]))
+    out = host_faults("routes", *(f"prompt {path} {n}" for n in (23, 128, 555)))
+    found = re.findall(r"(gemm_few|gemm_tile|qk_norm_rope_tokens64|attention_prefill_f16x3)_kernel<.*>\((.*?)(?:wick_rocm::\(anonymous namespace\)::)?\w+Args", out)
+    assert {name for name, _ in found} == {"gemm_few", "gemm_tile", "qk_norm_rope_tokens64", "attention_prefill_f16x3"}
+    assert [(name, args) for name, args in found if "*" in args or "unsigned int" not in args] == []

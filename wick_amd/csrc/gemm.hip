@@ -698,9 +698,10 @@ __device__ __forceinline__ void tie(V& v) {
 // (DUMP, the parity hook: all registers that there are, which it would otherwise take from scratch, up to 840 bytes a lane.)
 // The leading scalars repeat fields of `a` (preloaded into scalar registers at wave launch, see gemm_few_kernel): what the first copies need.
 template <int TYPE, bool DUMP, bool GATED, typename C>
-__global__ __launch_bounds__(C::kThreads, DUMP ? 1 : C::kOcc) void gemm_tile_kernel(const uint8_t* p_w, const int8_t* p_xq, const float* p_xs, const uint8_t* p_w_up, uint32_t p_m,
+__global__ __launch_bounds__(C::kThreads, DUMP ? 1 : C::kOcc) void gemm_tile_kernel(Address p_w, Address p_xq, Address p_xs, Address p_w_up, uint32_t p_m,
                                                                                    uint32_t p_n, uint32_t p_k, uint32_t p_row_tiles, uint32_t p_tok_tiles, uint32_t p_flags, GemmArgs a) {
-    a.w = p_w, a.xq = p_xq, a.xs = p_xs, a.w_up = p_w_up, a.m = p_m, a.n = p_n, a.k = p_k, a.row_tiles = p_row_tiles, a.tok_tiles = p_tok_tiles;
+    a.w = in_global<const uint8_t>(p_w), a.xq = in_global<const int8_t>(p_xq), a.xs = in_global<const float>(p_xs), a.w_up = in_global<const uint8_t>(p_w_up);
+    a.m = p_m, a.n = p_n, a.k = p_k, a.row_tiles = p_row_tiles, a.tok_tiles = p_tok_tiles;
     constexpr int RT = C::RT, TT = C::TT, SB = C::SB, T = C::kTiles;
     __shared__ __align__(16) typename C::Smem sm;
     uint32_t row_tile, tok_tile;
@@ -1291,8 +1292,8 @@ __device__ __forceinline__ void fmac_row_lanes4(v4f& sums, float x, const v4f& v
 // (1024 x 1024 in 4 3.8 -> 3.5 us.)
 constexpr uint32_t kFewSide = 256;
 template <int TYPE, bool DUMP, bool GATED, int TG, int WV>
-__global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(const uint8_t* p_w, const int8_t* p_xq, const float* p_xs, const void* p_more, uint32_t p_n, uint32_t p_k,
-                                                              uint32_t p_row_tiles, uint32_t p_flags, GemmArgs a) {
+__global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(Address p_w, Address p_xq, Address p_xs, Address p_more, uint32_t p_n, uint32_t p_k, uint32_t p_row_tiles,
+                                                              uint32_t p_flags, GemmArgs a) {
     static_assert(!(GATED && DUMP), "the parity hook runs the plain launch");
     constexpr int MS = GATED ? 2 : 1;                                                   // weights
     constexpr int TILES = MS * 4 * TG, MW = WV < TILES ? WV : TILES, TPW = TILES / MW;  // 16 x 16 tiles, waves that multiply, tiles of each
@@ -1312,7 +1313,7 @@ __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(const uint8_t* p_w
     const uint32_t my_share = side ? blockIdx.x & ((1u << shift) - 1u) : 0u;
     uint32_t granule = side ? blockIdx.x >> shift : blockIdx.x;  // within the launch's weights
     if (granule >= p_row_tiles) return;                          // (grids are rounded up)
-    a.w = p_w;
+    a.w = in_global<const uint8_t>(p_w);
     if (!GATED && (p_flags & kMoreWeights)) select_weight(a, granule);
     const uint32_t lane = threadIdx.x & 63u, l16 = lane & 15u, kq = lane >> 4;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -1330,7 +1331,7 @@ __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(const uint8_t* p_w
     if (copies) {
         const uint32_t cw = CW == WV ? wave : wave - MW;
         const uint8_t* const slab0 = a.w + (((size_t)(granule >> 1) * all_slabs + first) * 2 + (granule & 1u)) * kSlab;
-        const size_t to_up = GATED ? static_cast<const uint8_t*>(p_more) - p_w - kSlab : 0;
+        const size_t to_up = GATED ? p_more - p_w - kSlab : 0;
         const uint32_t t = lane >> 3, x0 = 16u * ((lane & 7u) ^ xt_swizzle(t));  // (eight tokens on: four on in the swizzle)
         static_for<kPer>([&](auto j_) {
             constexpr int j = decltype(j_)::value, lo = CW * j, hi = lo + CW - 1;  // the units that this one can be
@@ -1339,11 +1340,11 @@ __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(const uint8_t* p_w
             src[j] = slab0 + 1024u * u + (GATED && u >= (uint32_t)kSlabChunks ? to_up : 0), step[j] = 2 * kSlab, off[j] = 16u * lane;
             if (hi >= kW && (lo >= kW || u >= (uint32_t)kW)) {
                 const uint32_t c = u - kW;
-                src[j] = reinterpret_cast<const uint8_t*>(p_xq) + (size_t)tok0 * p_k + first * (32u * KB), step[j] = 32 * KB;
+                src[j] = in_global<const uint8_t>(p_xq) + (size_t)tok0 * p_k + first * (32u * KB), step[j] = 32 * KB;
                 off[j] = min(8u * c + t, n_here - 1u) * p_k + (x0 ^ (64u * (c & 1u)));
             }
             if (!DUMP && hi >= kW + kX && u >= (uint32_t)(kW + kX)) {
-                src[j] = reinterpret_cast<const uint8_t*>(p_xs) + ((size_t)tok0 * nb + first * KB) * sizeof(float), step[j] = KB * sizeof(float);
+                src[j] = in_global<const uint8_t>(p_xs) + ((size_t)tok0 * nb + first * KB) * sizeof(float), step[j] = KB * sizeof(float);
                 off[j] = min(lane, n_here - 1u) * nb * (uint32_t)sizeof(float);
             }
             const uint64_t p = reinterpret_cast<uint64_t>(src[j]);  // (said again that it is the same for the wave: the compiler puts it in vector registers otherwise)
@@ -1497,7 +1498,7 @@ __global__ __launch_bounds__(64 * WV, 2) void gemm_few_kernel(const uint8_t* p_w
         if (!multiplies || row >= a.m) return;
         const size_t tok_step = side ? a.m : (a.y_row_major ? 1u : a.y_stride), row_step = side || !a.y_row_major ? 1u : a.y_stride;
         const bool add = !side && a.accumulate;
-        float* y = (side ? static_cast<float*>(const_cast<void*>(p_more)) + (size_t)my_share * p_n * a.m : a.y) + row * row_step + tok0 * tok_step;
+        float* y = (side ? in_global<float>(p_more) + (size_t)my_share * p_n * a.m : a.y) + row * row_step + tok0 * tok_step;
 #pragma unroll
         for (int i = 0; i < TPW; i++)
 #pragma unroll
@@ -1695,7 +1696,7 @@ hipError_t cheapest_tile(Cost&& cost, Go&& go) {
 }
 
 // A launch with the leading scalars of its kernel: none (the 16x16x32 kernels), a tile's, the few-token kernel's.
-using TileKernel = void (*)(const uint8_t*, const int8_t*, const float*, const uint8_t*, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, GemmArgs);
+using TileKernel = void (*)(Address, Address, Address, Address, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, GemmArgs);
 template <typename Kernel>
 hipError_t enqueue(Kernel kernel, uint32_t grid, uint32_t threads, const GemmArgs& a, uint32_t shares, bool more, const Launch& L) {
     const uint32_t flag = more ? kMoreWeights : 0u;
@@ -1703,10 +1704,11 @@ hipError_t enqueue(Kernel kernel, uint32_t grid, uint32_t threads, const GemmArg
     if constexpr (std::is_same<Kernel, void (*)(GemmArgs)>::value) {
         return launch_kernel(L, kFamGemm, kernel, dim3(grid), dim3(threads), a);
     } else if constexpr (std::is_same<Kernel, TileKernel>::value) {
-        return launch_kernel(L, kFamGemm, kernel, dim3(grid), dim3(threads), a.w, a.xq, a.xs, a.w_up, a.m, a.n, a.k, a.row_tiles, a.tok_tiles, shift | flag, a);
+        return launch_kernel(L, kFamGemm, kernel, dim3(grid), dim3(threads), address(a.w), address(a.xq), address(a.xs), address(a.w_up), a.m, a.n, a.k,
+                             a.row_tiles, a.tok_tiles, shift | flag, a);
     } else {
-        const void* const p_more = a.w_up ? static_cast<const void*>(a.w_up) : a.partial;
-        return launch_kernel(L, kFamGemm, kernel, dim3(grid, a.tok_tiles), dim3(threads), a.w, a.xq, a.xs, p_more, a.n, a.k, a.row_tiles,
+        const Address p_more = a.w_up ? address(a.w_up) : address(a.partial);
+        return launch_kernel(L, kFamGemm, kernel, dim3(grid, a.tok_tiles), dim3(threads), address(a.w), address(a.xq), address(a.xs), p_more, a.n, a.k, a.row_tiles,
                              shift | (shift && a.partial ? kFewSide : 0u) | flag, a);
     }
 }

@@ -71,10 +71,10 @@ __device__ __forceinline__ void read_run(const uint8_t* slot, uint32_t off, uint
 // every wave redoes the vector (k floats from the L2), which costs less than that launch.
 // (The leading parameters repeat fields of `a`, p_x = xf or xq: the hardware preloads them into scalar registers at wave launch, see gemv_pairs_kernel.)
 template <int LPR, bool DUMP, bool FUSED = false>
-__global__ __launch_bounds__(64) void gemv_q6k_kernel(const void* p_x, const uint8_t* p_w, const float* p_norm_w, uint32_t p_m, uint32_t p_k, uint32_t p_rows_per_wave, Q6kArgs a) {
-    a.w = p_w, a.norm_w = p_norm_w, a.m = p_m, a.k = p_k, a.rows_per_wave = p_rows_per_wave;
-    if constexpr (FUSED) a.xf = static_cast<const float*>(p_x);
-    else a.xq = static_cast<const int8_t*>(p_x);
+__global__ __launch_bounds__(64) void gemv_q6k_kernel(Address p_x, Address p_w, Address p_norm_w, uint32_t p_m, uint32_t p_k, uint32_t p_rows_per_wave, Q6kArgs a) {
+    a.w = in_global<const uint8_t>(p_w), a.norm_w = in_global<const float>(p_norm_w), a.m = p_m, a.k = p_k, a.rows_per_wave = p_rows_per_wave;
+    if constexpr (FUSED) a.xf = in_global<const float>(p_x);
+    else a.xq = in_global<const int8_t>(p_x);
     static_assert(!(DUMP && FUSED), "the parity hook runs on pre-quantized activations");
     constexpr int RPW = 64 / LPR;  // rows per pass
     constexpr int PIECES = (15 + RPW * LPR * kHalfBytes + 15) / 16;  // upper bound of 16-byte pieces per span
@@ -288,8 +288,8 @@ uint32_t plan_lpr(uint32_t m, int num_cus, uint32_t& rows_per_wave, uint32_t wav
 template <int LPR, bool DUMP, bool FUSED>
 hipError_t launch_lpr(Q6kArgs& a, int num_cus, const Launch& L) {
     const uint32_t waves = plan_lpr<LPR>(a.m, num_cus, a.rows_per_wave, FUSED ? kFusedWavesPerCu : 12u);
-    return launch_kernel(L, kFamGemv, gemv_q6k_kernel<LPR, DUMP, FUSED>, dim3(waves), dim3(64), FUSED ? static_cast<const void*>(a.xf) : a.xq, a.w, a.norm_w,
-                         a.m, a.k, a.rows_per_wave, a);
+    return launch_kernel(L, kFamGemv, gemv_q6k_kernel<LPR, DUMP, FUSED>, dim3(waves), dim3(64), FUSED ? address(a.xf) : address(a.xq), address(a.w),
+                         address(a.norm_w), a.m, a.k, a.rows_per_wave, a);
 }
 
 template <typename F>

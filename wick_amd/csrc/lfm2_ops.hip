@@ -270,9 +270,10 @@ __global__ __launch_bounds__(256) void qk_norm_rope_tokens_kernel(QkNormRopeArgs
 // took 11.7 us for 2048 tokens of 16 + 8 heads on f16 rows, 17.4 for 2002 of 32 + 8 on f32 rows.
 constexpr uint32_t kRopeTokens = 2;
 template <typename KV>  // (leading parameters: fields of `a`, preloaded)
-__global__ __launch_bounds__(256) void qk_norm_rope_tokens64_kernel(float* p_q, float* p_k, const float* p_v, const float* p_q_norm, const float* p_k_norm, uint32_t p_q_stride,
+__global__ __launch_bounds__(256) void qk_norm_rope_tokens64_kernel(Address p_q, Address p_k, Address p_v, Address p_q_norm, Address p_k_norm, uint32_t p_q_stride,
                                                                     uint32_t p_kv_stride, uint32_t p_n_heads, uint32_t n, QkNormRopeArgs a) {
-    a.q = p_q, a.k = p_k, a.v = p_v, a.q_norm = p_q_norm, a.k_norm = p_k_norm, a.q_stride = p_q_stride, a.kv_stride = p_kv_stride, a.n_heads = p_n_heads;
+    a.q = in_global<float>(p_q), a.k = in_global<float>(p_k), a.v = in_global<const float>(p_v), a.q_norm = in_global<const float>(p_q_norm);
+    a.k_norm = in_global<const float>(p_k_norm), a.q_stride = p_q_stride, a.kv_stride = p_kv_stride, a.n_heads = p_n_heads;
     constexpr uint32_t HD = 64, HB = 3;
     __shared__ __align__(16) float sn_tab[kRopeTokens][HD / 2], cs_tab[kRopeTokens][HD / 2];
     const uint32_t l16 = threadIdx.x & 15u, sub = (threadIdx.x >> 4) & 3u;
@@ -746,9 +747,10 @@ struct KvQuad {
 
 // (The leading parameters repeat fields of `f`: the hardware preloads them into scalar registers at wave launch, see gemv_pairs_kernel.)
 template <int HD, typename KV, int NH>
-__global__ __launch_bounds__(256) void attention_layer_kernel(const uint32_t* p_pos, const float* p_q_raw, const float* p_k_raw, const float* p_v, const float* p_q_norm,
-                                                              const float2* p_rope, uint32_t splits, uint32_t p_max_seq, AttentionLayerArgs f) {
-    f.at.d_pos = p_pos, f.q_raw = p_q_raw, f.k_raw = p_k_raw, f.v = p_v, f.q_norm = p_q_norm, f.rope = p_rope, f.at.max_seq = p_max_seq;
+__global__ __launch_bounds__(256) void attention_layer_kernel(Address p_pos, Address p_q_raw, Address p_k_raw, Address p_v, Address p_q_norm, Address p_rope, uint32_t splits,
+                                                              uint32_t p_max_seq, AttentionLayerArgs f) {
+    f.at.d_pos = in_global<const uint32_t>(p_pos), f.q_raw = in_global<const float>(p_q_raw), f.k_raw = in_global<const float>(p_k_raw);
+    f.v = in_global<const float>(p_v), f.q_norm = in_global<const float>(p_q_norm), f.rope = in_global<const float2>(p_rope), f.at.max_seq = p_max_seq;
     constexpr uint32_t LR = HD / 4, RPP = 256 / LR, KROWS = kAttnChunk / RPP;  // lanes per key row, rows per pass, key rows per thread
     constexpr uint32_t VG = 256 / HD, VROWS = kAttnChunk / VG;                  // position groups of the value sum, rows of each
     using NR = NormRope<HD>;
@@ -1094,10 +1096,11 @@ __device__ __forceinline__ float exp_nonpos_hw(float x) { return __builtin_amdgc
 // 9.1), 555 queries 14.4 -> 13.6, 808 behind 8192 (f16) 107 -> 102.  (256 threads: 13.2, 9.2, 15.1, 104.  A third tile in LDS, with the next tile's keys read
 // ahead of its barrier: 12.4, 9.8, 13.9, 109.)
 template <int HALVES, bool MOVERS, typename KV>
-__global__ __launch_bounds__(512 * HALVES + (MOVERS ? 512 : 0)) void attention_prefill_f16x3_kernel(const float* p_q, const void* p_k_cache, const void* p_v_cache, const uint32_t* p_pos, uint32_t pos0,
+__global__ __launch_bounds__(512 * HALVES + (MOVERS ? 512 : 0)) void attention_prefill_f16x3_kernel(Address p_q, Address p_k_cache, Address p_v_cache, Address p_pos, uint32_t pos0,
                                                                                 uint32_t n, uint32_t q_stride, uint32_t p_n_heads, uint32_t p_n_kv_heads, uint32_t p_max_seq,
                                                                                 AttentionArgs a, uint32_t out_stride, int8_t* q_out, float* s_out) {
-    a.q = p_q, a.k_cache = p_k_cache, a.v_cache = p_v_cache, a.d_pos = p_pos, a.n_heads = p_n_heads, a.n_kv_heads = p_n_kv_heads, a.max_seq = p_max_seq;  // (preloaded)
+    a.q = in_global<const float>(p_q), a.k_cache = in_global<const uint8_t>(p_k_cache), a.v_cache = in_global<const uint8_t>(p_v_cache);  // (preloaded)
+    a.d_pos = in_global<const uint32_t>(p_pos), a.n_heads = p_n_heads, a.n_kv_heads = p_n_kv_heads, a.max_seq = p_max_seq;
     constexpr bool LO = std::is_same<KV, float>::value;  // the caches' values have low halves
     constexpr int PLANES = LO ? 2 : 1;                   // hi | lo
     constexpr int HD = 64, KT = 64, NC = 512 * HALVES, NT = MOVERS ? 512 : NC;  // threads that multiply, threads that move tiles
@@ -1886,8 +1889,8 @@ hipError_t launch_qk_norm_rope(float* d_q, float* d_k, const float* d_v, const f
         const uintptr_t floats = (uintptr_t)d_q | (uintptr_t)d_k | (uintptr_t)d_v | (uintptr_t)d_q_norm | (uintptr_t)d_k_norm;
         const uintptr_t rows = (uintptr_t)d_k_cache | (uintptr_t)d_v_cache;
         if (n_tokens > 1 && head_dim == 64 && floats % 16u == 0 && rows % (4u * sizeof(KV)) == 0 && q_stride % 4u == 0 && kv_stride % 4u == 0)
-            return launch_kernel(L, kFamOther, qk_norm_rope_tokens64_kernel<KV>, dim3((n_tokens + kRopeTokens - 1) / kRopeTokens), dim3(256), a.q, a.k, a.v,
-                                 a.q_norm, a.k_norm, a.q_stride, a.kv_stride, a.n_heads, n_tokens, a);
+            return launch_kernel(L, kFamOther, qk_norm_rope_tokens64_kernel<KV>, dim3((n_tokens + kRopeTokens - 1) / kRopeTokens), dim3(256), address(a.q),
+                                 address(a.k), address(a.v), address(a.q_norm), address(a.k_norm), a.q_stride, a.kv_stride, a.n_heads, n_tokens, a);
         if (n_tokens > 1 && head_dim / 2 <= kRopeTableMax) return launch_kernel(L, kFamOther, qk_norm_rope_tokens_kernel<KV>, dim3(n_tokens), dim3(256), a);
         return launch_kernel(L, kFamOther, qk_norm_rope_kernel<KV>, dim3(n_heads + n_kv_heads, n_tokens), dim3(64), a);
     });
@@ -1983,8 +1986,8 @@ hipError_t launch_attention_layer(const float* d_q, const float* d_k, const floa
         const auto go = [&](auto nh) {
             constexpr int NH = decltype(nh)::value;
             return with_kv_type(kv_f16, [&](auto kv) {
-                return launch_kernel(L, kFamOther, attention_layer_kernel<HD, decltype(kv), NH>, dim3(n_heads / NH * splits), block, f.at.d_pos, f.q_raw, f.k_raw, f.v,
-                                     f.q_norm, f.rope, splits, max_seq, f);
+                return launch_kernel(L, kFamOther, attention_layer_kernel<HD, decltype(kv), NH>, dim3(n_heads / NH * splits), block, address(f.at.d_pos), address(f.q_raw),
+                                     address(f.k_raw), address(f.v), address(f.q_norm), address(f.rope), splits, max_seq, f);
             });
         };
         // As many query heads per workgroup as share a KV head and as their accumulators leave registers for.  One head each is as
@@ -2098,10 +2101,10 @@ hipError_t launch_attention_prefill(const float* d_q, const void* d_k_cache, con
         return with_kv_type(kv_f16, [&](auto kv) {
             using KV = decltype(kv);
             if (n_heads * qblocks <= 256u)
-                return launch_kernel(L, kFamOther, attention_prefill_f16x3_kernel<1, true, KV>, dim3(n_heads, qblocks), dim3(1024), a.q, a.k_cache, a.v_cache, a.d_pos, pos0, n,
-                                     q_stride, n_heads, n_kv_heads, max_seq, a, out_stride, d_q8, d_q8_scales);
-            return launch_kernel(L, kFamOther, attention_prefill_f16x3_kernel<2, false, KV>, dim3(n_heads, (qblocks + 1u) / 2u), dim3(1024), a.q, a.k_cache, a.v_cache, a.d_pos,
-                                 pos0, n, q_stride, n_heads, n_kv_heads, max_seq, a, out_stride, d_q8, d_q8_scales);
+                return launch_kernel(L, kFamOther, attention_prefill_f16x3_kernel<1, true, KV>, dim3(n_heads, qblocks), dim3(1024), address(a.q), address(a.k_cache),
+                                     address(a.v_cache), address(a.d_pos), pos0, n, q_stride, n_heads, n_kv_heads, max_seq, a, out_stride, d_q8, d_q8_scales);
+            return launch_kernel(L, kFamOther, attention_prefill_f16x3_kernel<2, false, KV>, dim3(n_heads, (qblocks + 1u) / 2u), dim3(1024), address(a.q),
+                                 address(a.k_cache), address(a.v_cache), address(a.d_pos), pos0, n, q_stride, n_heads, n_kv_heads, max_seq, a, out_stride, d_q8, d_q8_scales);
         });
     }
     const dim3 grid(n_heads, (n + 7u) / 8u), block(256);

@@ -6,6 +6,16 @@
 
 namespace wick_rocm {
 
+// A device address as a kernel argument of its own.  The runtime looks up every argument that is a pointer among its allocations when
+// the kernel is enqueued, 0.025 us each in a loop of one launch, more among others; numbers and structs it only copies.  Four pointers
+// a launch / numbers: a prompt of 23 tokens behind 700 on the 350M shape, 121 launches, 655 / 623 us, of 100 tokens 709 / 700.
+typedef uint64_t Address;
+inline Address address(const void* p) { return reinterpret_cast<uint64_t>(p); }
+template <typename T>
+__device__ __forceinline__ T* in_global(Address a) {
+    return (T*)(T __attribute__((address_space(1)))*)a;
+}
+
 // f16 bit pattern -> f32 (v_cvt_f32_f16; exact, subnormals kept).
 __device__ __forceinline__ float f16_bits_to_f32(uint32_t bits) {
     uint16_t b = (uint16_t)bits;
