@@ -225,15 +225,10 @@ bool gemm_row_applies(wick_rocm_ctx* ctx, const wick_rocm_weight* w, uint32_t n)
 }
 
 int gemm_row(wick_rocm_ctx* ctx, const wick_rocm_weight* w, const int8_t* d_q, const float* d_s, uint32_t n, float* d_y) {
-    uint32_t splits = ctx->gemm_max_splits > 1 ? gemm_split_k(w->m, n, w->k, ctx->gemm_max_splits) : 1u;
-    if (splits > 1 && ctx->capturing && (size_t)splits * n * w->m > ctx->scratch_f_cap &&  // (without that room the product is unsplit, see gemm_locked)
-        !gemm_split_in_launch(w->m, n, w->k, ctx->gemm_max_splits, ctx->launch(), false, false))
-        splits = 1;
-    const size_t floats = splits > 1 ? (size_t)splits * w->m : 0;
-    const bool room = !ctx->capturing || floats <= ctx->scratch_f_cap;
-    if (room)
-        if (int rc = ensure_scratch(ctx, 0, 0, floats)) return rc;
-    const hipError_t e = launch_gemm_mfma_row(static_cast<const uint8_t*>(w->d_gemm), w->m, w->k, d_q, d_s, d_y, ctx->launch(), splits, room ? ctx->scratch_f : nullptr);
+    const uint32_t splits = ctx->gemm_max_splits > 1 ? gemm_split_k(w->m, n, w->k, ctx->gemm_max_splits) : 1u;
+    // (Prompts only, which end with a wait: never part of a graph that is launched.)
+    if (int rc = ensure_scratch(ctx, 0, 0, splits > 1 ? (size_t)splits * w->m : 0)) return rc;
+    const hipError_t e = launch_gemm_mfma_row(static_cast<const uint8_t*>(w->d_gemm), w->m, w->k, d_q, d_s, d_y, ctx->launch(), splits, ctx->scratch_f);
     return e == hipSuccess ? WICK_ROCM_OK : fail_hip(ctx, e, "gemm launch");
 }
 

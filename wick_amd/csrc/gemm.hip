@@ -1599,7 +1599,7 @@ bool few_applies_split(uint64_t rows, uint32_t n, uint32_t k, uint32_t shares, b
         if (deferrable) return slabs <= 16 && n <= 512 && rows * n >= 32768 * slabs && !few_tokens_per_tile(rows, n, k, shares);
         return slabs <= 8 + rows * n / 9500;
     }
-    if (n > 64 || units > 2 * kCus || units * slabs > (cost == 1 ? 12288u : 4096u) || slabs * cost > (cost == 1 && units < 96 ? 15u : 16u)) return false;
+    if (units > 2 * kCus || units * slabs > (cost == 1 ? 12288u : 4096u) || slabs * cost > (cost == 1 && units < 96 ? 15u : 16u)) return false;
     if (deferrable && 12 * slabs * cost > 72 + units) return false;
     return !room || (few_applies(rows, n, k) && !(deferrable && few_side_applies(rows, n, shares)));
 }
@@ -1661,7 +1661,7 @@ struct TileQ : T32<2, 1, 2, 2, 2, 4, false, true> {  // the same with half a sla
 };
 struct TileN : T32<1, 1, 4, 2, 4, 4> {  // 128 x 64, 8 waves of 32 x 32
     static constexpr int kPerCu = 2;
-    static constexpr TileCost kCost[2] = {{{0.70f, 1.25f}, 1.53f}, {{0.94f, 1.45f}, 0.9f}};  // (with the gate: see gated_tile_n)
+    static constexpr TileCost kCost[2] = {{{0.70f, 1.25f}, 1.53f}, {{0.94f}, 0.9f}};  // (with the gate: one on a CU, see gated_tile_n)
 };
 struct TileH : T32<1, 1, 2, 2, 4, 4> {  // 64 x 64, 4 waves of 32 x 32
     static constexpr int kPerCu = 4;
@@ -1832,13 +1832,13 @@ hipError_t launch_gemm_mfma(int type, const uint8_t* d_w, uint32_t m, uint32_t k
 // One token of a launch over more.  A row's sum is fixed by the shares of K and by nothing else of the launch.
 hipError_t launch_gemm_mfma_row(const uint8_t* d_w, uint32_t m, uint32_t k, const int8_t* d_q, const float* d_scales, float* d_y, const Launch& L,
                                 uint32_t splits, float* d_partial) {
-    if (L.gemm_mfma16) return hipErrorInvalidValue;
+    if (L.gemm_mfma16 || (splits > 1 && !d_partial)) return hipErrorInvalidValue;
     GemmArgs a{};
     a.w = d_w, a.xq = d_q, a.xs = d_scales, a.y = d_y;
     a.m = m, a.n = 1, a.k = k, a.y_stride = m;
     a.accumulate = 1;
     if (splits > 1) a.ksplit = splits, a.partial = d_partial;
-    return launch<false>(kTypeQ4_0, a, L, splits > 1 && !d_partial);
+    return launch<false>(kTypeQ4_0, a, L, false);
 }
 
 // The same launch over up to three weights of one type and k that share the activations: outputs y[i] (same stride,

@@ -157,7 +157,7 @@ uint32_t gemm_split_k(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits);
 // deferrable: the caller's next kernel would add the shares up.  (With deferrable: a part of what there is without.)  room: there is scratch for
 // shares side by side that the call may use; some launches are faster with it that can do without.
 bool gemm_split_in_launch(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits, const Launch& L, bool deferrable, bool room);
-// y += W x for one token of a launch over more, to the bit (not on the 16x16x32 loop): splits: that launch's; d_partial: splits * m floats, or null.
+// y += W x for one token of a launch over more, to the bit (not on the 16x16x32 loop): splits: that launch's; d_partial: splits * m floats.
 hipError_t launch_gemm_mfma_row(const uint8_t* d_w, uint32_t m, uint32_t k, const int8_t* d_q, const float* d_scales, float* d_y, const Launch& L,
                                 uint32_t splits, float* d_partial);
 hipError_t launch_gemm_mfma_multi(int type, const uint8_t* const* d_w, const uint32_t* m, uint32_t count, uint32_t k, const int8_t* d_q,
