@@ -55,7 +55,8 @@ def test_the_ragged_launches_are_on_every_tile(routes):
     assert {s: short(k) for s, k in zip(gated, kernels)} == gated and all("<2, false, true, " in k for k, in kernels)
     with open(os.path.join(ROOT, "wick_amd", "csrc", "gemm.hip")) as f:
         plain, with_gate = (set(t.split(", ")) for t in re.findall(r"cheapest_tile<(Tile\w, [^>]*)>", f.read()))
-    assert plain == set(gemm.RAGGED_TILES.values()) and with_gate == set(gated.values())
+    # (TileN with the gate is for fewer workgroups than the public launch takes: prompts reach it, see below)
+    assert plain == set(gemm.RAGGED_TILES.values()) and with_gate == set(gated.values()) | {"TileN"}
 
 
 def test_prompts_on_the_few_token_kernel(routes):

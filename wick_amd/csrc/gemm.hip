@@ -55,6 +55,7 @@
 //     acc = fma(t, dx, acc), both plain v_fma_f32 (v_fma_mix_f32 with an f16 scale
 //     operand would save registers but issues at half the rate).
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "wick_rocm_device.h"
@@ -1877,8 +1878,8 @@ uint32_t gated_few_tokens(uint32_t m, uint32_t n, uint32_t k) {
     return k >= 16 * KB * 32 && units * ((n + 15) / 16) <= 5 * kCus ? 64 : 0;
 }
 
-// TileN with the gate: past those, while every workgroup has a CU, whose eight waves make shorter slabs of it than four do.  The cheapest of the
-// other tiles or 64 tokens above / here, us: 4608 x 1024 over 128 12.5 / 11.7, 160 13.4 / 11.8, 200 (288 workgroups) 15.9 / 16.4; 6912 x 2048 over 100 22.7 / 20.8, 160
+// TileN with the gate: past those, while every workgroup has a CU, whose eight waves make shorter slabs of it than four do (its cost is that of one a
+// CU, and lower there than the other tiles').  The cheapest of the other tiles or 64 tokens above / here, us: 4608 x 1024 over 128 12.5 / 11.7, 160 13.4 / 11.8, 200 (288 workgroups) 15.9 / 16.4; 6912 x 2048 over 100 22.7 / 20.8, 160
 // (324) 28.6 / 28.6; 2816 x 1024 over 300 13.3 / 11.6; 2048 x 1024 over 400 13.3 / 11.4; 4096 x 4096 over 200 41.3 / 36.6, 300 (320) 48.8 / 49.5.
 bool gated_tile_n(uint32_t m, uint32_t n) { return n > 64 && (uint64_t)((m + 63) / 64) * ((n + 63) / 64) <= kCus; }
 
@@ -1899,7 +1900,10 @@ bool gated_few_faster(uint32_t m, uint32_t n, uint32_t k) {
 }
 
 template <typename C>
-float gated_tile_cost(uint32_t m, uint32_t n, uint32_t k) { return tile_cost<C>((m + C::kRows / 2 - 1) / (C::kRows / 2), n, k, 1, true); }
+float gated_tile_cost(uint32_t m, uint32_t n, uint32_t k) {
+    if (std::is_same<C, TileN>::value && !gated_tile_n(m, n)) return INFINITY;
+    return tile_cost<C>((m + C::kRows / 2 - 1) / (C::kRows / 2), n, k, 1, true);
+}
 }  // namespace
 
 // Where the launch is expected to be faster than the two projections in one launch and the gate kernel behind it (2.7 us and the floats'
@@ -1914,8 +1918,8 @@ bool gemm_gated_faster(uint32_t m, uint32_t n, uint32_t k, const Launch& L) {
         return tile_cost<C>(2 * (uint64_t)((m + C::kRows - 1) / C::kRows), n, k, 1);
     };
     const float separate = std::min({plain(TileL{}), plain(TileX{}), plain(TileS{}), plain(TileQ{}), plain(TileN{}), plain(TileH{})});
-    float gated = std::min({gated_tile_cost<TileL>(m, n, k), gated_tile_cost<TileX>(m, n, k), gated_tile_cost<TileS>(m, n, k), gated_tile_cost<TileQ>(m, n, k)});
-    if (gated_tile_n(m, n)) gated = std::min(gated, gated_tile_cost<TileN>(m, n, k));
+    const float gated = std::min({gated_tile_cost<TileL>(m, n, k), gated_tile_cost<TileX>(m, n, k), gated_tile_cost<TileS>(m, n, k), gated_tile_cost<TileQ>(m, n, k),
+                                  gated_tile_cost<TileN>(m, n, k)});
     return !few_applies(2 * (uint64_t)m, n, k) && gated < separate + 2.7f + (float)n * (float)m * 3e-6f;
 }
 
@@ -1939,8 +1943,7 @@ hipError_t launch_gemm_mfma_gated(int /*type: the copies are the same for both*/
         if ((uint64_t)a.row_tiles * a.tok_tiles > 0x7fffff00ull) return hipErrorInvalidValue;
         return enqueue(gemm_tile_kernel<2, false, true, C>, (a.row_tiles * a.tok_tiles + 7u) / 8u * 8u, C::kThreads, a, 1, false, L);
     };
-    if (gated_tile_n(m, n)) return tile(TileN{});
-    return cheapest_tile<TileL, TileX, TileS, TileQ>([&](auto cfg) { return gated_tile_cost<decltype(cfg)>(m, n, k); }, tile);
+    return cheapest_tile<TileL, TileX, TileS, TileQ, TileN>([&](auto cfg) { return gated_tile_cost<decltype(cfg)>(m, n, k); }, tile);
 }
 
 // Parity hook through the matrix-core path: the same loads, unpack, LDS layout and
