@@ -531,7 +531,8 @@ EDGES = {
     (16384, 33, 1152): ("TileN, in 2", "narrow 3"),
     # 64 tokens
     (512, 64, 512): ("few 2 8", "few 2 8"),
-    (512, 65, 512): ("TileH", "TileH"),
+    (512, 65, 512): ("few 1 4", "few 1 4"),
+    (512, 833, 512): ("TileH", "TileH"),
     # 15 slabs of a split launch, up to 32 tokens and under 96 granules
     (256, 32, 1920): ("few 1 8", "few 1 8"),
     (256, 32, 2048): ("few 1 8, in 8", "few 1 8"),
@@ -576,7 +577,7 @@ def test_both_sides_of_every_launch_rule(ctx, oracle, m, n, k):
     what is there, and leaves the padding alone; split over K as the library does it, and unsplit."""
     dtype = W.Q4_0 if (m + n + k) % 2 == 0 else W.Q8_0
     rows = 256 if m % 256 == 0 else 32  # of the weight, repeated: making 16384 of them takes the oracle seconds
-    wb = np.tile(oracle.synth_weight(dtype, rows, k, 7, 0.02).reshape(rows, -1), (m // rows, 1))
+    wb = np.tile(oracle.synth_weight(dtype, rows, k, 7, 0.02).reshape(rows, -1), (-(-m // rows), 1))[:m]
     s, q = oracle.quantize_q8_0_batch(oracle.fill_normal(5, 1.0, n * k), n, k)
     w, d_q, d_s = ctx.upload_weight(wb, dtype, m, k), ctx.to_device(q), ctx.to_device(s)
     old = oracle.fill_normal(6, 1.0, (n + 3) * (m + 5))
@@ -637,7 +638,7 @@ def test_the_gated_launch_starts_past_256_tiles(ctx, oracle, m, n, k):
 
 
 # A launch with a last tile of 32 rows and of few tokens on each of the tiles that launch costs choose from, plain and with the gate.
-RAGGED_TILES = {(96, 67, 256): "TileH", (5472, 131, 1024): "TileN", (5408, 643, 128): "TileS", (4832, 1027, 512): "TileQ", (6176, 451, 128): "TileX",
+RAGGED_TILES = {(31, 961, 384): "TileH", (65, 895, 128): "TileH", (96, 835, 256): "TileH", (5472, 131, 1024): "TileN", (5408, 643, 128): "TileS", (4832, 1027, 512): "TileQ", (6176, 451, 128): "TileX",
                 (6944, 1669, 128): "TileL"}
 RAGGED_GATED_TILES = {(5472, 259, 128): "TileS", (6560, 259, 128): "TileQ", (6176, 451, 512): "TileX", (6752, 1031, 1024): "TileL"}
 
@@ -708,7 +709,10 @@ def test_the_gate_in_the_launch_over_all_magnitudes(ctx, oracle, dtype):
 FEW_TILES = {
     (1056, 97, 640): ("few 1 4", "few 1 4"),           # one token and one granule over
     (2080, 81, 128): ("few 1 4", "few 1 4"),           # one slab
-    (544, 65, 512): ("few 1 4", "few 1 4"),            # past 512 x 512
+    (544, 65, 512): ("few 1 4", "few 1 4"),            # 512 x 512 and a granule
+    (96, 67, 256): ("few 1 4", "few 1 4"),
+    (31, 832, 128): ("few 1 4", "few 1 4"),            # less than a granule, one slab
+    (33, 200, 4096): ("few 1 4, in 8", "few 1 4"),     # few rows in shares
     (3584, 128, 256): ("few 1 4", "few 1 4"),          # 448 tiles of 32 tokens
     (3584, 129, 256): ("few 2 8", "few 2 8"),
     (8192, 128, 128): ("few 2 8", "few 2 8"),          # 512 of 64

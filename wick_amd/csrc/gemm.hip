@@ -1572,10 +1572,11 @@ bool few_side_applies(uint64_t rows, uint32_t n, uint32_t shares) {
 //               256 15.3 / 11.0 / 9.7, 400 15.5 / 16.0 / 12.6, 555 15.9 / 19.5 / 17.9; 4608 x 1024 over 130 9.6 / 8.6 / 7.9, 256 11.0 / 12.3 / 11.5; 3072 x 2048 over 300 15.8 / 17.6 / 13.9
 //   in shares:  1024 x 1024 in 4 over 130 4.5 / 3.9 / 3.8, 300 5.5 / 5.6 / 6.0; 1024 x 4608 in 8 over 72 7.3 / 6.5 / 6.0, 130 8.4 / 8.4 / 8.7; 2048 x 6912 in 8 over 72 11.2 / 12.9 / 12.4
 // Up to 832 tokens: over more, few rows only fit and little is left to gain (1024 x 1024 over 808 8.3 / 7.6, over 1000 8.4 / 8.1; x 2048 over 1000 13.1 / 12.9).
-// Weights of up to 512 x 512 elements, smaller than any projection of a model, stay on the 64-row tile, whose edges small launches check.
-uint32_t few_tokens_per_tile(uint64_t rows, uint32_t n, uint32_t k, uint32_t shares) {
+// Small weights gain the same: in a graph 512 x 512 over 65 5.0 / 3.2, over 832 5.5 / 3.9; 1024 x 256 over 400 4.1 / 3.2; 32 x 128 over 66 3.1 / 2.1; and
+// back to back, in shares and with their addition or walked, 512 x 512 over 400 5.2 / 3.9, 64 x 4096 over 200 7.4 / 6.5, 128 x 2048 over 100 6.4 / 6.5.
+uint32_t few_tokens_per_tile(uint64_t rows, uint32_t n, uint32_t shares) {
     const uint64_t units = (rows + GR - 1) / GR * shares;
-    if (n <= 64 || n > 832 || rows * k <= 512u * 512u) return 0;
+    if (n <= 64 || n > 832) return 0;
     if (4 * units * ((n + 31) / 32) <= 7 * kCus) return 32;
     return units * ((n + 63) / 64) <= 2 * kCus ? 64 : 0;
 }
@@ -1596,8 +1597,8 @@ uint32_t few_tokens_per_tile(uint64_t rows, uint32_t n, uint32_t k, uint32_t sha
 bool few_applies_split(uint64_t rows, uint32_t n, uint32_t k, uint32_t shares, bool deferrable, bool room) {
     const uint64_t units = (rows + GR - 1) / GR, slabs = k / (KB * 32), cost = n <= 32 ? 1u : 2u;
     if (n > 64) {
-        if (!few_tokens_per_tile(rows, n, k, 1)) return false;
-        if (deferrable) return slabs <= 16 && n <= 512 && rows * n >= 32768 * slabs && !few_tokens_per_tile(rows, n, k, shares);
+        if (!few_tokens_per_tile(rows, n, 1)) return false;
+        if (deferrable) return slabs <= 16 && n <= 512 && rows * n >= 32768 * slabs && !few_tokens_per_tile(rows, n, shares);
         return slabs <= 8 + rows * n / 9500;
     }
     if (units > 2 * kCus || units * slabs > (cost == 1 ? 12288u : 4096u) || slabs * cost > (cost == 1 && units < 96 ? 15u : 16u)) return false;
@@ -1752,7 +1753,7 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, bool in_launch, uint32
             if (q8) return go(gemm_tile_kernel<8, true, false, C>, C::kRows, C::kTokens, C::kThreads);
         return go(gemm_tile_kernel<2, DUMP, false, C>, C::kRows, C::kTokens, C::kThreads);
     };
-    const uint32_t few_tiled = L.gemm_mfma16 ? 0 : few_tokens_per_tile(GR * tile_rows(GR), a.n, a.k, in_launch ? 1u : ksplit);
+    const uint32_t few_tiled = L.gemm_mfma16 ? 0 : few_tokens_per_tile(GR * tile_rows(GR), a.n, in_launch ? 1u : ksplit);
     const bool few = !L.gemm_mfma16 && (few_tiled || (ksplit > 1 ? in_launch || few_side_applies(a.m, a.n, ksplit) : few_applies(GR * tile_rows(GR), a.n, a.k)));
     const bool narrow = !wide_split && narrow_tiles(tile_rows(BM), a.n);
     if (few) {
