@@ -9,7 +9,7 @@ F32, Q4_0, Q8_0, Q6_K = 0, 2, 8, 14
 
 
 def build(oracle, n_layers=4, hidden=256, inter=512, n_heads=4, kv_heads=(0, 2, 0, 4), vocab=320, kernel=3, rope_theta=1_000_000.0,
-          eps=1e-5, wtype=Q4_0, embd_type=Q6_K, seed=1, context_length=None, sigma=0.08, mixed_qkv=False):
+          eps=1e-5, wtype=Q4_0, embd_type=Q6_K, seed=1, context_length=None, sigma=0.08, mixed_qkv=False, gate_sigma=None):
     """Returns (gguf image bytes, cfg dict for the oracle, {name: (ggml_type, dims, array)})."""
     assert len(kv_heads) == n_layers
     rng = np.random.default_rng(seed)
@@ -17,9 +17,9 @@ def build(oracle, n_layers=4, hidden=256, inter=512, n_heads=4, kv_heads=(0, 2, 
     tensors = {}
     counter = [seed * 1000]
 
-    def quant(name, m, k, t):
+    def quant(name, m, k, t, sd=sigma):
         counter[0] += 1
-        tensors[name] = (t, [k, m], oracle.synth_weight(t, m, k, counter[0], sigma))
+        tensors[name] = (t, [k, m], oracle.synth_weight(t, m, k, counter[0], sd))
 
     def f32(name, dims, center=1.0, spread=0.2):
         n = int(np.prod(dims))
@@ -42,7 +42,7 @@ def build(oracle, n_layers=4, hidden=256, inter=512, n_heads=4, kv_heads=(0, 2, 
             quant(p + "shortconv.in_proj.weight", 3 * hidden, hidden, wtype)
             quant(p + "shortconv.out_proj.weight", hidden, hidden, wtype)
             f32(p + "shortconv.conv.weight", [kernel, hidden], center=0.0, spread=0.5)
-        quant(p + "ffn_gate.weight", inter, hidden, wtype)
+        quant(p + "ffn_gate.weight", inter, hidden, wtype, gate_sigma or sigma)
         quant(p + "ffn_up.weight", inter, hidden, wtype)
         quant(p + "ffn_down.weight", hidden, inter, wtype)
     meta = [

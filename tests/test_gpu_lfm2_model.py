@@ -545,6 +545,45 @@ def test_short_prompts_at_the_edges_of_their_tiles(ctx, oracle, tmp_path, hidden
         model.free()
 
 
+def on_either_block_loop(ctx, model, tokens):
+    """The logits and the state behind a prompt, bit for bit the same on the 16x16x32 kernels, which run every layer for all tokens, the gate in a
+    launch of its own."""
+    got = []
+    try:
+        for shape in (32, 16):
+            ctx.set_gemm_mfma_shape(shape)
+            model.reset()
+            got.append((model.forward_prefill(tokens, 0).view(np.uint32), model.snapshot_state(tokens.size)))
+    finally:
+        ctx.set_gemm_mfma_shape(32)
+    assert all(np.array_equal(a, b) for a, b in zip(*got)), f"{tokens.size} tokens"
+    return got[0][0].view(np.float32)
+
+
+@pytest.mark.parametrize("gate_sigma", [0.08, 0.45, 8.0])
+def test_gates_of_all_sizes_on_the_tile_of_eight_waves(ctx, oracle, tmp_path, gate_sigma):
+    """Gate | up of 1952 rows over 449 tokens and five slabs of K, gates of 25 gate_sigma: a launch whose silu takes gates below 41 in a shorter way, for a
+    wave's 1024 of them together; all of them inside, a few outside in some waves, most outside in all."""
+    model, _, _ = load(ctx, oracle, tmp_path, context=512, n_layers=2, hidden=640, inter=1952, n_heads=10, kv_heads=(0, 2), vocab=256, embd_type=W.Q8_0, gate_sigma=gate_sigma)
+    try:
+        assert np.isfinite(on_either_block_loop(ctx, model, np.random.default_rng(11).integers(0, 256, 449).astype(np.uint32))).all()
+    finally:
+        model.free()
+
+
+@pytest.mark.parametrize("kv_heads", [(2, 0), (0, 2)])
+def test_the_last_token_alone_is_the_whole_layer(ctx, oracle, tmp_path, kv_heads):
+    """The last layer's feed-forward block as products of one token, behind a convolution and behind attention, with the K shares of the products over
+    all tokens: none of 4 slabs, eight of 32 (up to 128 tokens), four of 32 from 64 tiles of 128 x 128 on."""
+    model, _, _ = load(ctx, oracle, tmp_path, context=2048, n_layers=2, hidden=512, inter=4096, n_heads=8, kv_heads=kv_heads, vocab=256, embd_type=W.Q8_0)
+    tokens = np.random.default_rng(13).integers(0, 256, 2000).astype(np.uint32)
+    try:
+        for n in (65, 128, 2000):
+            on_either_block_loop(ctx, model, tokens[:n])
+    finally:
+        model.free()
+
+
 @pytest.mark.parametrize("embd_type,hidden", [(W.Q6_K, 1280), (W.Q4_0, 1152), (W.Q8_0, 1152)])
 def test_a_prompts_rows_are_the_embeddings(ctx, oracle, tmp_path, embd_type, hidden):
     """Rows past the lookup's 1024 elements, tokens past its groups of four: bit for bit the prompt given as the oracle's rows."""

@@ -89,15 +89,18 @@ class Zeros:
     (4128, 2816, 25, True), (4128, 2944, 25, False),   # 22
     (8192, 3200, 32, True),                            # 512 x 25 slabs: the projections alone are the 128-row tiles'
     (8224, 1024, 23, False),                           # 257 granules
-    (4608, 1024, 32, True), (4608, 1024, 33, False),   # 32 tokens
+    (4608, 1024, 32, True), (4608, 1024, 33, True),    # 32 tokens
+    (2048, 1408, 33, True), (2048, 1536, 33, False),   # 11 slabs above them
+    (4096, 1408, 64, True), (4096, 1536, 64, False),
+    (4128, 1536, 64, True),                            # past 256 granules of both
 ])
 def test_few_tokens_take_the_gate_into_the_launch_while_k_is_short(routes, tmp_path, inter, hidden, tokens, gated):
-    """A prompt's gate | up over up to 32 tokens: one launch, or the projections and the gate behind them."""
+    """A prompt's gate | up over up to 64 tokens: one launch, or the projections and the gate behind them."""
     path = tmp_path / "model.gguf"
     path.write_bytes(bytes(lfm2_synth.build(Zeros, n_layers=1, hidden=hidden, inter=inter, n_heads=hidden // 64, kv_heads=(0,), embd_type=Q8_0)[0]))
     kernels, = routes(f"prompt {path} {tokens}")
-    assert ("gemm_few_kernel<2, false, true, 1, 8>" in kernels) == gated
-    assert ("silu_mul_quantize_kernel" not in kernels) == gated or tokens == 33  # (33 tokens: the tiles' costs decide)
+    assert (f"gemm_few_kernel<2, false, true, {1 if tokens <= 32 else 2}, 8>" in kernels) == gated
+    assert ("silu_mul_quantize_kernel" not in kernels) == gated
 
 
 @pytest.mark.parametrize("tokens,kernel", [(200, "few_kernel<2, false, false, 2, 8>"),  # 512 tiles of 64 tokens, four shares
@@ -112,6 +115,7 @@ def test_residual_projections_of_a_prompt(routes, tokens, kernel):
     (1024, 3584, 65, "few_kernel<2, false, true, 1, 8>"), (1024, 3584, 128, "few_kernel<2, false, true, 1, 8>"),  # 448 tiles of 32 tokens
     (1024, 2048, 280, "few_kernel<2, false, true, 2, 8>"), (1024, 2048, 281, "tile_kernel<2, false, true, TileN>"),  # 256 of 64
     (1024, 4096, 256, "tile_kernel<2, false, true, TileN>"), (1024, 4096, 257, "tile_kernel<2, false, true, TileS>"),  # 256 tiles of 64 rows
+    (640, 1952, 449, "tile_kernel<2, false, true, TileN>"),  # 5 slabs
     (2048, 4096, 160, "few_kernel<2, false, true, 2, 8>"), (2048, 4096, 161, "tile_kernel<2, false, true, TileN>"),  # 1280 of 16 tokens
 ])
 def test_prompts_take_the_gate_into_the_few_token_kernel(routes, tmp_path, hidden, inter, tokens, kernel):
