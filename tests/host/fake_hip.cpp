@@ -25,7 +25,7 @@ struct State {  // (in a function: kernels are registered by other files' static
     std::map<const void*, std::string> kernels;
     std::map<const void*, void*> symbols;
     std::deque<std::function<void()>> queue;
-    std::vector<std::string> enqueued;  // kernels, mangled
+    std::vector<std::pair<std::string, dim3>> enqueued;  // kernels, mangled, and their grids
     bool capturing = false;
     long launch_fails = 0, copy_fails = 0;
     bool pinned_fails = false;
@@ -86,7 +86,7 @@ hipError_t launch(const void* f, dim3 grid, void** args, hipStream_t stream) {
     if (reinterpret_cast<uintptr_t>(stream) != (uintptr_t)current + 1) fake_hip::other_device++;
     if (due(st().launch_fails)) return done(hipErrorLaunchFailure);
     fake_hip::launches++;
-    st().enqueued.push_back(st().kernels[f]);
+    st().enqueued.push_back({st().kernels[f], grid});
     if (st().kernels[f].find("rmsnorm_quantize_kernel") != std::string::npos) {  // (x, shares, their stride, weight, quants, scales, dim, ..)
         const size_t elements = (size_t)grid.x * *static_cast<uint32_t*>(args[6]);
         if (!covers(*static_cast<void**>(args[4]), elements) || !covers(*static_cast<void**>(args[5]), elements / 32 * sizeof(float))) fake_hip::out_of_range++;
@@ -140,9 +140,9 @@ size_t allocations() {
 std::vector<std::string> kernels() {
     Lock lk;
     std::vector<std::string> names;
-    for (const std::string& mangled : st().enqueued) {
+    for (const auto& [mangled, grid] : st().enqueued) {
         char* const plain = abi::__cxa_demangle(mangled.c_str(), nullptr, nullptr, nullptr);
-        names.push_back(plain ? plain : mangled);
+        names.push_back((plain ? plain : mangled) + (" (" + std::to_string(grid.x) + " x " + std::to_string(grid.y) + ")"));
         std::free(plain);
     }
     st().enqueued.clear();

@@ -15,7 +15,7 @@ extern long other_device;  // kernels on a stream of another GPU than the callin
 extern long out_of_range;  // accesses of the copy kernel outside every allocation (they are left out), and outputs of the norm + quantizer
 size_t pending();          // enqueued and not done
 size_t allocations();      // device allocations that are not freed
-std::vector<std::string> kernels();  // names of the kernels enqueued since the last call of this, with their template arguments
+std::vector<std::string> kernels();  // names of the kernels enqueued since the last call of this, with their template arguments and grids, "(x x y)"
 void fail_launch(long n);  // the n-th kernel launch from now fails (n = 1: the next one; 0: none)
 void fail_copy(long n);    // the same for hipMemcpyAsync
 void fail_pinned(bool on); // no pinned memory is to be had

@@ -14,14 +14,14 @@ from lfm2_synth import Q4_0, Q8_0
 
 @pytest.fixture(scope="session")
 def routes(host_faults):
-    """(calls) -> the kernels of each, e.g. "gemm_tile_kernel<2, false, false, TileX>"."""
-    def run(*calls):
+    """(calls) -> the kernels of each, e.g. "gemm_tile_kernel<2, false, false, TileX>"; with grids=True, the kernels' grids."""
+    def run(*calls, grids=False):
         out = host_faults("routes", *calls)
         out = re.sub(r"wick_rocm::|\(anonymous namespace\)::", "", out)
         kernels = []
         for line in out.splitlines():
             if line.startswith("\t"):
-                kernels[-1].append(re.sub(r"^void |\(.*$", "", line.strip()))
+                kernels[-1].append(tuple(map(int, re.search(r" \((\d+) x (\d+)\)$", line).groups())) if grids else re.sub(r"^void |\(.*$", "", line.strip()))
             else:
                 kernels.append([])
         assert len(kernels) == len(calls), out
@@ -63,6 +63,17 @@ def test_prompts_on_the_few_token_kernel(routes):
     calls = [f"gemm {m} {n} {k} {splits}" for m, n, k in gemm.FEW_TILES for splits in (0, 1)]
     got = [short(k) for k in routes(*calls)]
     assert dict(zip(gemm.FEW_TILES, zip(got[::2], got[1::2]))) == gemm.FEW_TILES
+
+
+@pytest.mark.parametrize("m,n,k,even", [(1056, 832, 1024, False), (1312, 768, 1024, False), (1568, 300, 2048, False), (5408, 130, 2688, False),
+                                        (1024, 832, 384, True), (2208, 200, 1024, True), (544, 300, 1024, True), (7712, 128, 1024, True)])
+def test_few_token_tiles_are_even_over_the_xcds(routes, m, n, k, even):
+    """Workgroup i of a launch goes to XCD i % 8.  A granule's token tiles share an XCD unless that takes one of its 32 CUs another workgroup."""
+    (x, y), = routes(f"gemm {m} {n} {k} 1", grids=True)[0]
+    granules = -(-m // 32)
+    on = [sum(i + x * j & 7 == xcd for i in range(granules) for j in range(y)) for xcd in range(8)]
+    assert x in (granules, -(-granules // 8) * 8) and (x % 8 == 0) == even
+    assert -(-max(on) // 32) == -(-(-(-granules * y // 8)) // 32)
 
 
 @pytest.mark.parametrize("dim,quads", [(32, 1), (1024, 1), (1056, 2), (2048, 2), (2080, 0), (2304, 0), (4096, 0), (8192, 0), (8224, 0)])

@@ -1581,6 +1581,18 @@ uint32_t few_tokens_per_tile(uint64_t rows, uint32_t n, uint32_t shares) {
     return units * ((n + 63) / 64) <= 2 * kCus ? 64 : 0;
 }
 
+// Workgroups of such a launch per token tile (blockIdx.y).  Rounded up to whole rounds over the XCDs, a granule's token tiles are all on one, which
+// reads its weights once; but with a last round that is not full the first XCDs have more of them, and where that is another workgroup for their
+// 32 CUs, the launch waits for those: there the token tiles go round the XCDs one after the other.  Tiles of other kernels / rounded / not, us:
+// 1312 x 1024 over 768 8.2 / 10.3 / 7.8, 1056 x 1024 over 832 8.0 / 9.9 / 7.6, 5408 x 2688 over 130 19.5 / 18.0 / 14.9, 1568 x 2048 over 300 13.8 / 10.2 / 8.9;
+// as many either way: 2208 x 1024 over 200 8.4 / 6.2 / 6.5, 7712 x 1024 over 128 9.8 / 9.0 / 9.3, 544 x 1024 over 300 7.7 / 4.7 / 4.8.
+uint32_t few_grid(uint32_t granules, uint32_t shares, uint32_t tok_tiles) {
+    const auto per_cu = [](uint32_t on_an_xcd) { return (on_an_xcd + kCus / 8 - 1) / (kCus / 8); };
+    const uint32_t n = granules * shares;
+    const bool uneven = per_cu((n + 7) / 8 * tok_tiles) > per_cu((n * tok_tiles + 7) / 8);
+    return uneven ? n : (granules + 7) / 8 * 8 * shares;
+}
+
 // Shares of K one after the other in one launch of that kernel: ~0.3 us a slab up to 32 tokens, twice that above, against shares side by side and
 // the launch that adds them up, or, with `deferrable`, the additions in the norm's kernel behind the projection.  With the norm, side by
 // side is the faster way wherever few_side_applies (1024 x 1024 in 4 over 23 tokens 3.5 and 0.4 more in the norm, here 4.7); beyond, and plain:
@@ -1739,8 +1751,9 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, bool in_launch, uint32
         a.tok_tiles = (a.n + tokens - 1) / tokens;
         const uint32_t shares = a.ksplit;
         if ((uint64_t)a.row_tiles * a.tok_tiles * shares > 0x7fffff00ull) return hipErrorInvalidValue;  // beyond a launch's grid
-        // every XCD gets the same number of slots of the tile map; tile id = blockIdx.x / shares runs over all of them (gemm_few_kernel: tokens in blockIdx.y)
-        const uint32_t grid = (a.row_tiles * (rows == GR ? 1u : a.tok_tiles) + 7u) / 8u * 8u * (whole ? 1u : shares);  // whole: a workgroup takes all shares of its rows
+        // every XCD gets the same number of slots of the tile map; tile id = blockIdx.x / shares runs over all of them
+        const uint32_t side = whole ? 1u : shares;  // whole: a workgroup takes all shares of its rows
+        const uint32_t grid = rows == GR ? few_grid(a.row_tiles, side, a.tok_tiles) : (a.row_tiles * a.tok_tiles + 7u) / 8u * 8u * side;
         const hipError_t e = enqueue(kernel, grid, threads, a, shares, more != 0, L);
         if (e != hipSuccess || shares == 1 || defer_reduce || whole) return e;  // deferred: the caller's next kernel adds the shares up itself
         return launch_reduce(a, L);
