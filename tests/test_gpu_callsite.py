@@ -379,3 +379,28 @@ def test_a_graph_of_a_short_residual_projection_needs_no_scratch(oracle):
         ctx.close()
     for other in got[1:]:
         assert all(np.array_equal(a, b) for a, b in zip(got[0], other))
+
+
+def test_captured_shares_of_a_long_prompt_with_and_without_scratch(oracle):
+    """48 slabs over 832 tokens: side by side where there is room, in a capture too; without room a capture walks them in the launch.  The same bits."""
+    m, n, k = 512, 832, 6144
+    s, q = oracle.quantize_q8_0_batch(oracle.fill_normal(4, 1.0, n * k), n, k)
+    wb, got = oracle.synth_weight(W.Q4_0, m, k, 13), []
+    for room in (True, False):
+        ctx = W.RocmContext(0)
+        w, d_s, d_q, d_y = ctx.upload_weight(wb, W.Q4_0, m, k), ctx.to_device(s), ctx.to_device(q), ctx.alloc(n * m * 4)
+        if room:
+            ctx.gemm_preq(w, d_s, d_q, n, d_y)
+            got.append(d_y.download(np.uint32, n * m))
+        ctx.graph_begin()
+        ctx.gemm_preq(w, d_s, d_q, n, d_y)
+        g = ctx.graph_end()
+        for _ in range(2):
+            d_y.upload(np.zeros(n * m, np.float32))
+            ctx.graph_launch(g)
+            got.append(d_y.download(np.uint32, n * m))
+        ctx.graph_destroy(g)
+        for b in (w, d_s, d_q, d_y):
+            b.free()
+        ctx.close()
+    assert all(np.array_equal(got[0], other) for other in got[1:])
