@@ -718,6 +718,7 @@ FEW_TILES = {
     (8192, 128, 128): ("few 2 8", "few 2 8"),          # 512 of 64
     (8224, 128, 128): ("TileS", "TileS"),
     (1056, 831, 384): ("few 2 8", "few 2 8"),          # 33 granules, not rounded up
+    (160, 635, 3968): ("few 2 8, in 8", "few 1 4"),    # 40 workgroups of shares, all with work
     (1024, 832, 384): ("few 2 8", "few 2 8"),          # 832 tokens
     (1024, 833, 384): ("TileH", "TileH"),
     (1024, 76, 2048): ("few 1 4", "few 1 4"),          # 16 slabs in shares: in the launch

@@ -76,6 +76,13 @@ def test_few_token_tiles_are_even_over_the_xcds(routes, m, n, k, even):
     assert -(-max(on) // 32) == -(-(-(-granules * y // 8)) // 32)
 
 
+@pytest.mark.parametrize("m,n,k,shares", [(1344, 163, 7040, 4), (192, 635, 3968, 8), (32, 100, 2048, 8), (512, 200, 4608, 8)])
+def test_shares_leave_no_granules_of_workgroups_without_work(routes, m, n, k, shares):
+    call = f"gemm {m} {n} {k} 8"
+    assert routes(call) == [["gemm_few_kernel<2, false, false, %s>" % ("1, 4" if m == 32 else "2, 8"), f"gemm_splitk_reduce_kernel<{shares}>"]]
+    assert routes(call, grids=True)[0][0][0] == -(-(-(-m // 32) * shares) // 8) * 8
+
+
 @pytest.mark.parametrize("dim,quads", [(32, 1), (1024, 1), (1056, 2), (2048, 2), (2080, 0), (2304, 0), (4096, 0), (8192, 0), (8224, 0)])
 def test_the_norm_keeps_short_rows_only(routes, dim, quads):
     """Rows past 2048 elements are read a second time: kept, they would leave the CU four workgroups."""

@@ -1586,11 +1586,13 @@ uint32_t few_tokens_per_tile(uint64_t rows, uint32_t n, uint32_t shares) {
 // 32 CUs, the launch waits for those: there the token tiles go round the XCDs one after the other.  Tiles of other kernels / rounded / not, us:
 // 1312 x 1024 over 768 8.2 / 10.3 / 7.8, 1056 x 1024 over 832 8.0 / 9.9 / 7.6, 5408 x 2688 over 130 19.5 / 18.0 / 14.9, 1568 x 2048 over 300 13.8 / 10.2 / 8.9;
 // as many either way: 2208 x 1024 over 200 8.4 / 6.2 / 6.5, 7712 x 1024 over 128 9.8 / 9.0 / 9.3, 544 x 1024 over 300 7.7 / 4.7 / 4.8.
+// Shares are rounded up together, not eight granules of each: a workgroup without work still takes its turn on a CU.  Tiles of other kernels / eight granules /
+// here, with the addition: 1344 x 7040 in 4 over 163 16.5 / 18.0 / 14.2, 192 x 3968 in 8 over 635 9.4 / 10.7 / 9.2, 544 x 7040 in 4 over 405 16.8 / 18.0 / 14.3.
 uint32_t few_grid(uint32_t granules, uint32_t shares, uint32_t tok_tiles) {
     const auto per_cu = [](uint32_t on_an_xcd) { return (on_an_xcd + kCus / 8 - 1) / (kCus / 8); };
     const uint32_t n = granules * shares;
     const bool uneven = per_cu((n + 7) / 8 * tok_tiles) > per_cu((n * tok_tiles + 7) / 8);
-    return uneven ? n : (granules + 7) / 8 * 8 * shares;
+    return uneven ? n : (n + 7) / 8 * 8;
 }
 
 // Shares of K one after the other in one launch of that kernel: ~0.3 us a slab up to 32 tokens, twice that above, against shares side by side and
