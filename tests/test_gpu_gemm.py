@@ -723,9 +723,10 @@ FEW_TILES = {
     (1024, 833, 384): ("TileH", "TileH"),
     (1024, 76, 2048): ("few 1 4", "few 1 4"),          # 16 slabs in shares: in the launch
     (1024, 74, 2048): ("few 2 8, in 8", "few 1 4"),    # or 512 side by side
-    (1024, 340, 5632): ("few 1 4", "few 1 4"), (1024, 340, 5760): ("TileN, in 4", "few 1 4"),  # 44 slabs walked
-    (512, 832, 3072): ("few 1 4", "few 1 4"), (512, 832, 3200): ("few 1 4", "few 1 4"),        # 24; 832 x 3200 and
-    (512, 832, 4096): ("few 1 4", "few 1 4"), (512, 832, 4224): ("TileN, in 4", "few 1 4"),    # 832 x 4224 activations
+    (1024, 334, 3328): ("few 1 4", "few 1 4"), (1024, 334, 3456): ("TileH, in 4", "few 1 4"),  # 26 slabs walked in tiles of 32
+    (1600, 448, 5376): ("few 2 8", "few 2 8"), (1600, 448, 5504): ("TileH, in 2", "few 2 8"),  # 42 in tiles of 64
+    (3072, 96, 3840): ("few 1 4", "few 1 4"), (3072, 97, 3840): ("TileH, in 4", "few 1 4"),    # or over 96 tokens
+    (256, 330, 2048): ("few 1 4", "few 1 4"), (256, 300, 2048): ("few 2 8, in 8", "few 1 4"),  # 16 slabs, 256 x 301 results
 }
 
 

@@ -1606,19 +1606,21 @@ uint32_t few_grid(uint32_t granules, uint32_t shares, uint32_t tok_tiles) {
 // Above 64 tokens, against shares on the 64-row or 128-row tiles: the walk costs 0.3 us a slab and the other way the sums' round trip through memory:
 //   plain:                  3072 x 1024 over 66 8.7 / 5.4, 130 10.0 / 6.2, 320 13.3 / 8.0; 1024 x 1024 over 512 11.3 / 6.1; 2048 x 2048 over 66 9.4 / 7.7, 256 13.6 / 9.5;
 //                           1024 x 3072 over 96 8.5 / 9.7, 160 10.3 / 9.8; 1024 x 4608 over 200 12.1 / 13.7, 256 13.8 / 13.7; 512 x 4096 over 400 11.7 / 12.2, 512 12.9 / 12.3
-//   plain, longer rows:     640 x 7296 over 761 25.4 / 35.8; 512 x 6144 over 832 18.3 / 23.8; 544 x 5376 over 374 13.6 / 14.7; 3872 x 7296 over 214 32.2 / 36.9; 1024 x 6144
-//                           over 400 18.7 / 20.5; 1216 x 5248 over 519 24.7 / 22.6; 1600 x 5504 over 435 25.0 / 23.8; 512 x 4608 over 832 15.7 / 17.1, over 600 14.3 / 13.8
-//                           -- up to 44 slabs, and past 24 while the activations leave an XCD's 4 MB of L2 room for weights (113 launches of 20 to
-//                           64 slabs: at worst 5 % slower than shares side by side, 736 x 3328 over 564 13.4 / 14.0, and 0.3 % behind the better one on average)
+//   plain, longer rows, weights cold; warm and with the quantizer: 640 x 7296 over 761 25.4 / 35.8 (warm); 512 x 6144 over 832 18.3 / 23.8 (cold); 4128 x 4352 over 82
+//                           19.3 / 16.5; 20.9 / 15.5.  In tiles of 32 tokens 512 x 3072 over 832 13.2 / 10.9; 18.5 / 19.0, 1024 x 4608 over 400 16.0 / 15.0; 19.3 / 20.9, 768 x
+//                           4352 over 566 15.0 / 13.7; 19.2 / 21.6.  Of 64 1216 x 5248 over 519 24.2 / 22.0; 28.0 / 27.4, 1024 x 6144 over 800 27.9 / 28.2; 31.1 / 34.1.
+//                           (A walk is a chain of slabs, behind which cold weights hide; warm ones shorten what it is compared with.  The lines are where neither
+//                           loses what the other gains: 190 launches of 16 to 64 slabs.)
 //   with the norm, a prompt of the 350M shape, all of it: 220 tokens 839 / 840, 300 963 / 947, 420 1039 / 1016, 680 1388 / 1394; of the 1.2B shape's first six layers
 //                           (2048 x 2048): 200 550 / 559, 300 689 / 685, 400 742 / 734
 bool few_applies_split(uint64_t rows, uint32_t n, uint32_t k, uint32_t shares, bool deferrable, bool room) {
     const uint64_t units = (rows + GR - 1) / GR, slabs = k / (KB * 32), cost = n <= 32 ? 1u : 2u;
     if (n > 64) {
-        if (!few_tokens_per_tile(rows, n, 1)) return false;
+        const uint32_t tokens = few_tokens_per_tile(rows, n, 1);
+        if (!tokens) return false;
         if (deferrable) return slabs <= 16 && n <= 512 && rows * n >= 32768 * slabs && !few_tokens_per_tile(rows, n, shares);
-        if (room && slabs > 24 && (slabs > 44 || (uint64_t)n * k > 3500000u)) return false;
-        return slabs <= 8 + rows * n / 9500;
+        if (!room) return slabs <= 9 + rows * n / 9500;  // (all that walks with room, at least)
+        return slabs <= 9 + rows * n / 11000 && slabs <= (tokens == 64 || n <= 96 ? 42u : 26u);
     }
     if (units > 2 * kCus || units * slabs > (cost == 1 ? 12288u : 4096u) || slabs * cost > (cost == 1 && units < 96 ? 15u : 16u)) return false;
     if (deferrable && 12 * slabs * cost > 72 + units) return false;
