@@ -532,7 +532,7 @@ EDGES = {
     # 64 tokens
     (512, 64, 512): ("few 2 8", "few 2 8"),
     (512, 65, 512): ("few 1 4", "few 1 4"),
-    (512, 833, 512): ("TileH", "TileH"),
+    (512, 2049, 512): ("TileN", "TileN"),
     # 15 slabs of a split launch, up to 32 tokens and under 96 granules
     (256, 32, 1920): ("few 1 8", "few 1 8"),
     (256, 32, 2048): ("few 1 8, in 8", "few 1 8"),
@@ -562,9 +562,9 @@ EDGES = {
     (2048, 1024, 128): ("TileS", "TileS"),
     (2048, 1025, 128): ("TileX", "TileX"),
     # 64 wide tiles, 32 stages: shares on the wide tile
-    (1024, 1024, 4096): ("TileN, in 4", "TileH"),
-    (1024, 896, 4096): ("TileN, in 2", "TileH"),
-    (1024, 1024, 3968): ("TileN, in 2", "TileH"),
+    (1024, 1024, 4096): ("TileN, in 4", "few 2 8"),
+    (1024, 896, 4096): ("TileN, in 2", "few 2 8"),
+    (1024, 1024, 3968): ("TileN, in 2", "few 2 8"),
     # 256 wide tiles
     (4096, 1024, 4096): ("TileX, in 2", "TileN"),
     (4096, 1025, 4096): ("TileH", "TileH"),
@@ -638,7 +638,7 @@ def test_the_gated_launch_starts_past_256_tiles(ctx, oracle, m, n, k):
 
 
 # A launch with a last tile of 32 rows and of few tokens on each of the tiles that launch costs choose from, plain and with the gate.
-RAGGED_TILES = {(31, 961, 384): "TileH", (65, 895, 128): "TileH", (96, 835, 256): "TileH", (5472, 131, 1024): "TileN", (5408, 643, 128): "TileS", (4832, 1027, 512): "TileQ", (6176, 451, 128): "TileX",
+RAGGED_TILES = {(31, 2081, 384): "TileH", (65, 2111, 128): "TileH", (96, 2051, 256): "TileH", (5472, 131, 1024): "TileN", (5408, 643, 128): "TileS", (4832, 1027, 512): "TileQ", (6176, 451, 128): "TileX",
                 (6944, 1669, 128): "TileL"}
 RAGGED_GATED_TILES = {(5472, 259, 128): "TileS", (6560, 259, 128): "TileQ", (6176, 451, 512): "TileX", (6752, 1031, 1024): "TileL"}
 
@@ -720,7 +720,10 @@ FEW_TILES = {
     (1056, 831, 384): ("few 2 8", "few 2 8"),          # 33 granules, not rounded up
     (160, 635, 3968): ("few 2 8, in 8", "few 1 4"),    # 40 workgroups of shares, all with work
     (1024, 832, 384): ("few 2 8", "few 2 8"),          # 832 tokens
-    (1024, 833, 384): ("TileH", "TileH"),
+    (1024, 833, 384): ("few 2 8", "few 2 8"),
+    (512, 2048, 384): ("few 2 8", "few 2 8"), (480, 2049, 384): ("TileN", "TileN"),
+    (512, 1024, 2304): ("few 2 8", "few 2 8"), (512, 1025, 2304): ("TileH, in 2", "few 2 8"),  # 18 slabs walked up to 1024 tokens
+    (1024, 768, 4608): ("few 2 8", "few 2 8"), (1024, 769, 4608): ("TileN, in 2", "few 2 8"),  # 36 up to 768
     (1024, 76, 2048): ("few 1 4", "few 1 4"),          # 16 slabs in shares: in the launch
     (1024, 74, 2048): ("few 2 8, in 8", "few 1 4"),    # or 512 side by side
     (1024, 334, 3328): ("few 1 4", "few 1 4"), (1024, 334, 3456): ("TileH, in 4", "few 1 4"),  # 26 slabs walked in tiles of 32

@@ -1571,12 +1571,13 @@ bool few_side_applies(uint64_t rows, uint32_t n, uint32_t shares) {
 //   one share:  1024 x 1024 over 100 7.7 / 4.7 / 5.4, 300 7.8 / 5.5 / 5.6, 555 8.0 / 7.6 / 7.0, 1300 10.1 / 11.9 / 11.1; 2048 x 2048 over 160 15.3 / 8.2 / 8.9,
 //               256 15.3 / 11.0 / 9.7, 400 15.5 / 16.0 / 12.6, 555 15.9 / 19.5 / 17.9; 4608 x 1024 over 130 9.6 / 8.6 / 7.9, 256 11.0 / 12.3 / 11.5; 3072 x 2048 over 300 15.8 / 17.6 / 13.9
 //   in shares:  1024 x 1024 in 4 over 130 4.5 / 3.9 / 3.8, 300 5.5 / 5.6 / 6.0; 1024 x 4608 in 8 over 72 7.3 / 6.5 / 6.0, 130 8.4 / 8.4 / 8.7; 2048 x 6912 in 8 over 72 11.2 / 12.9 / 12.4
-// Up to 832 tokens: over more, few rows only fit and little is left to gain (1024 x 1024 over 808 8.3 / 7.6, over 1000 8.4 / 8.1; x 2048 over 1000 13.1 / 12.9).
+// Up to 2048 tokens, where the few granules that are left re-read activations that an XCD's L2 no longer holds: 1024 x 1024 over 1000 8.1 / 7.5, 256 x 512 over
+// 1220 5.5 / 3.8, over 2211 5.6 / 4.7, 704 x 3072 over 1459 19.3 / 18.0, 512 x 2048 over 2048 12.7 / 12.6; 256 x 2048 over 3000 12.4 / 13.3, over 4000 12.7 / 14.7.
 // Small weights gain the same: in a graph 512 x 512 over 65 5.0 / 3.2, over 832 5.5 / 3.9; 1024 x 256 over 400 4.1 / 3.2; 32 x 128 over 66 3.1 / 2.1; and
 // back to back, in shares and with their addition or walked, 512 x 512 over 400 5.2 / 3.9, 64 x 4096 over 200 7.4 / 6.5, 128 x 2048 over 100 6.4 / 6.5.
 uint32_t few_tokens_per_tile(uint64_t rows, uint32_t n, uint32_t shares) {
     const uint64_t units = (rows + GR - 1) / GR * shares;
-    if (n <= 64 || n > 832) return 0;
+    if (n <= 64 || n > 2048) return 0;
     if (4 * units * ((n + 31) / 32) <= 7 * kCus) return 32;
     return units * ((n + 63) / 64) <= 2 * kCus ? 64 : 0;
 }
@@ -1609,6 +1610,8 @@ uint32_t few_grid(uint32_t granules, uint32_t shares, uint32_t tok_tiles) {
 //   plain, longer rows, weights cold; warm and with the quantizer: 640 x 7296 over 761 25.4 / 35.8 (warm); 512 x 6144 over 832 18.3 / 23.8 (cold); 4128 x 4352 over 82
 //                           19.3 / 16.5; 20.9 / 15.5.  In tiles of 32 tokens 512 x 3072 over 832 13.2 / 10.9; 18.5 / 19.0, 1024 x 4608 over 400 16.0 / 15.0; 19.3 / 20.9, 768 x
 //                           4352 over 566 15.0 / 13.7; 19.2 / 21.6.  Of 64 1216 x 5248 over 519 24.2 / 22.0; 28.0 / 27.4, 1024 x 6144 over 800 27.9 / 28.2; 31.1 / 34.1.
+//                           Over more tokens, cold; warm: 1024 x 3584 over 887 21.1 / 17.4; 25.3 / 23.5, 512 x 5120 over 1144 22.1 / 26.0; 28.3 / 33.1, 256 x 2560 over 1651
+//                           12.6 / 12.2; 18.1 / 19.1, 544 x 2176 over 1100 14.0 / 10.8; 19.3 / 17.2.
 //                           (A walk is a chain of slabs, behind which cold weights hide; warm ones shorten what it is compared with.  The lines are where neither
 //                           loses what the other gains: 190 launches of 16 to 64 slabs.)
 //   with the norm, a prompt of the 350M shape, all of it: 220 tokens 839 / 840, 300 963 / 947, 420 1039 / 1016, 680 1388 / 1394; of the 1.2B shape's first six layers
@@ -1620,7 +1623,7 @@ bool few_applies_split(uint64_t rows, uint32_t n, uint32_t k, uint32_t shares, b
         if (!tokens) return false;
         if (deferrable) return slabs <= 16 && n <= 512 && rows * n >= 32768 * slabs && !few_tokens_per_tile(rows, n, shares);
         if (!room) return slabs <= 9 + rows * n / 9500;  // (all that walks with room, at least)
-        return slabs <= 9 + rows * n / 11000 && slabs <= (tokens == 64 || n <= 96 ? 42u : 26u);
+        return slabs <= 9 + rows * n / 11000 && slabs <= (n > 1024 ? 17u : (n <= 768 && tokens == 64) || n <= 96 ? 42u : 26u);
     }
     if (units > 2 * kCus || units * slabs > (cost == 1 ? 12288u : 4096u) || slabs * cost > (cost == 1 && units < 96 ? 15u : 16u)) return false;
     if (deferrable && 12 * slabs * cost > 72 + units) return false;
