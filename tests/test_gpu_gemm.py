@@ -524,8 +524,8 @@ EDGES = {
     (16384, 9, 128): ("few 1 4", "few 1 4"),
     (16416, 9, 128): ("narrow 1", "narrow 1"),
     # 12288 slabs, up to 32 tokens
-    (16384, 32, 3072): ("narrow 2, in 2", "few 1 4"),
-    (16384, 32, 3200): ("narrow 2, in 2", "narrow 2"),
+    (16384, 32, 3072): ("few 1 4, in 2", "few 1 4"),
+    (16384, 32, 3200): ("few 1 4, in 2", "narrow 2"),
     # 4096 slabs, 33 tokens and more
     (16384, 33, 1024): ("few 2 4", "narrow 3"),
     (16384, 33, 1152): ("TileN, in 2", "narrow 3"),
@@ -537,9 +537,12 @@ EDGES = {
     (256, 32, 1920): ("few 1 8", "few 1 8"),
     (256, 32, 2048): ("few 1 8, in 8", "few 1 8"),
     # 16 slabs from 96 granules on
-    (3040, 9, 2048): ("narrow 1, in 8", "few 1 8"),
+    (3040, 9, 2048): ("few 1 4, in 8", "few 1 8"),
     (3072, 9, 2048): ("few 1 8", "few 1 8"),
-    (3072, 9, 2176): ("narrow 1, in 8", "few 1 8"),
+    (3072, 9, 2176): ("few 1 4, in 8", "few 1 8"),
+    # shares past two workgroups a CU: up to 32 tokens
+    (4096, 32, 4096): ("few 1 4, in 8", "few 1 8"),
+    (4096, 33, 4096): ("TileN, in 8", "few 2 8"),
     # 8 slabs, 33 tokens and more
     (256, 33, 1024): ("few 2 8", "few 2 8"),
     (256, 33, 1152): ("few 2 8, in 4", "few 2 8"),

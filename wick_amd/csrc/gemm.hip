@@ -1557,11 +1557,12 @@ bool few_applies(uint64_t rows, uint32_t n, uint32_t k) {
     return n <= 64 && units <= (n <= 32 ? 2 * kCus : kCus) && units * slabs <= (n <= 32 ? 12288u : 4096u);
 }
 
-// Shares of K side by side on the same kernel, a workgroup each: while the chip holds them all at once (one workgroup of eight waves per CU,
-// or two of four).  128-row or 64-row tiles / here, us: 1024 x 4608 in 8 over 23 tokens 6.7 / 4.6; 2048 x 6912 over 37 10.0 / 8.9, over 64 10.2 / 9.9;
-// 2048 x 4608 over 48 8.3 / 7.2; 1024 x 8192 over 64 10.0 / 6.8; past it, on the kernel before this one, 4096 x 4096 over 23 7.2 / 8.9.
+// Shares of K side by side on the same kernel, a workgroup each.  Above 32 tokens while the chip holds them all at once, two workgroups a CU; up to 32
+// always (there are four a CU at most).  128-row or 64-row tiles / here with the addition, us: 1024 x 4608 in 8 over 23 tokens 6.7 / 4.6; 2048 x 6912 over 37
+// 10.0 / 8.9, over 64 12.6 / 12.2; 2048 x 4096 over 48 10.5 / 10.2; past two a CU, over 23 2560 x 4096 9.7 / 9.2, 4096 x 4096 11.4 / 10.5, 8192 x 2048 11.1 / 10.2, 16384 x 2048
+// 14.6 / 12.9, over 32 4096 x 2048 9.4 / 9.2, 16384 x 3072 18.4 / 17.6; over 48 2560 x 4096 10.9 / 11.8, 4096 x 4096 12.8 / 14.1, 6144 x 2048 11.7 / 12.3.
 bool few_side_applies(uint64_t rows, uint32_t n, uint32_t shares) {
-    return n <= 64 && (rows + GR - 1) / GR * shares <= 2 * kCus;
+    return n <= 32 || (n <= 64 && (rows + GR - 1) / GR * shares <= 2 * kCus);
 }
 
 // More tokens on that kernel, side by side in tiles of 32 or 64 (0: not): while the chip holds all of the workgroups at once, each slab is a
@@ -1598,7 +1599,7 @@ uint32_t few_grid(uint32_t granules, uint32_t shares, uint32_t tok_tiles) {
 
 // Shares of K one after the other in one launch of that kernel: ~0.3 us a slab up to 32 tokens, twice that above, against shares side by side and
 // the launch that adds them up, or, with `deferrable`, the additions in the norm's kernel behind the projection.  With the norm, side by
-// side is the faster way wherever few_side_applies (1024 x 1024 in 4 over 23 tokens 3.5 and 0.4 more in the norm, here 4.7); beyond, and plain:
+// side is the faster way up to two workgroups a CU (1024 x 1024 in 4 over 23 tokens 3.5 and 0.4 more in the norm, here 4.7); beyond, and plain:
 //   plain, 9 tokens:        1024 x 1024 6.3 / 4.5, x 1792 7.5 / 6.5, x 2048 (8 shares, not 4) 6.7 / 7.1; 4096 x 2048 7.0 / 7.3
 //   plain, 24:              1024 x 1024 6.6 / 4.9, x 1792 8.0 / 6.8, x 2048 7.0 / 7.4; 3072 x 2048 7.6 / 7.5, 4096 x 2048 8.5 / 7.5
 //   plain, 40:              1024 x 1024 7.2 / 7.0, 4096 x 1024 8.2 / 7.1; 2048 x 2048 8.2 / 11.5
@@ -1627,7 +1628,7 @@ bool few_applies_split(uint64_t rows, uint32_t n, uint32_t k, uint32_t shares, b
     }
     if (units > 2 * kCus || units * slabs > (cost == 1 ? 12288u : 4096u) || slabs * cost > (cost == 1 && units < 96 ? 15u : 16u)) return false;
     if (deferrable && 12 * slabs * cost > 72 + units) return false;
-    return !room || (few_applies(rows, n, k) && !(deferrable && few_side_applies(rows, n, shares)));
+    return !room || (few_applies(rows, n, k) && !(deferrable && units * shares <= 2 * kCus));
 }
 
 uint32_t split_k_factor(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits) {
