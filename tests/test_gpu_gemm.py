@@ -522,13 +522,20 @@ def test_one_token_accumulates_into_a_column(ctx, oracle, dtype, layout, ms, k):
 EDGES = {
     # 512 granules of rows: one workgroup per granule
     (16384, 9, 128): ("few 1 4", "few 1 4"),
-    (16416, 9, 128): ("narrow 1", "narrow 1"),
-    # 12288 slabs, up to 32 tokens
+    (16416, 9, 128): ("few 1 4", "few 1 4"),
+    # 1024 granules, up to 32 tokens; 768 past 16 slabs of K
+    (32768, 9, 128): ("few 1 4", "few 1 4"),
+    (32800, 9, 128): ("narrow 1", "narrow 1"),
+    (32800, 32, 128): ("narrow 2", "narrow 2"),
+    (24608, 17, 2048): ("few 1 4", "few 1 4"),
+    (24576, 17, 2176): ("few 1 4", "few 1 4"),
+    (24608, 17, 2176): ("narrow 2", "narrow 2"),
+    # two shares of 512 granules, up to 32 tokens
     (16384, 32, 3072): ("few 1 4, in 2", "few 1 4"),
-    (16384, 32, 3200): ("few 1 4, in 2", "narrow 2"),
-    # 4096 slabs, 33 tokens and more
-    (16384, 33, 1024): ("few 2 4", "narrow 3"),
-    (16384, 33, 1152): ("TileN, in 2", "narrow 3"),
+    (16384, 32, 3200): ("few 1 4, in 2", "few 1 4"),
+    # 8 slabs of 512 granules walked, 9 in shares, 33 tokens and more
+    (16384, 33, 1024): ("few 2 8", "few 2 8"),
+    (16384, 33, 1152): ("TileN, in 2", "few 2 8"),
     # 64 tokens
     (512, 64, 512): ("few 2 8", "few 2 8"),
     (512, 65, 512): ("few 1 4", "few 1 4"),
@@ -549,9 +556,9 @@ EDGES = {
     # 256 granules, up to 32 tokens: eight waves or four
     (8192, 9, 128): ("few 1 8", "few 1 8"),
     (8224, 9, 128): ("few 1 4", "few 1 4"),
-    # 256 granules, 33 tokens and more: one workgroup per granule
+    # 256 granules, 33 tokens and more: one workgroup a CU, or two; 512 below
     (8192, 33, 256): ("few 2 8", "few 2 8"),
-    (8224, 33, 256): ("narrow 3", "narrow 3"),
+    (8224, 33, 256): ("few 2 8", "few 2 8"),
     # 48 tokens on the 128-row tiles; 49 .. 64 on the 32x32x32 loop
     (16416, 48, 128): ("narrow 3", "narrow 3"),
     (16416, 49, 128): ("TileS", "TileS"),

@@ -1548,13 +1548,17 @@ uint32_t wide_split_factor(uint32_t m, uint32_t n, uint32_t k, uint32_t max_spli
 // Launches of few 128 x 128 tiles (at most one per CU): the ones that may be split over K.
 bool narrow_tiles(uint64_t row_tiles, uint32_t n) { return n <= BN_NARROW || row_tiles * ((n + BN - 1) / BN) <= kCus; }
 
-// Launches of gemm_few_kernel: up to 64 tokens and few enough granules that latency and not the chip's throughput is what they cost
-// (every workgroup fetches all tokens' activations for its 32 rows; beyond, the 128-row tiles are the cheaper readers, and above 32
-// tokens the 64-row ones from a second workgroup per CU on: lines drawn for the kernel before this one, 9216 x 1024 over 48 9.5 / 10.6).  Tiles /
-// here, us: 2048 x 1024 over 23 tokens 8.8 / 4.9, 1024 x 4608 29 / 12.5; 9216 x 1024 over 32 9.1 / 6.5; 65536 x 2048 over 16 27 / 40.
+// Launches of gemm_few_kernel: up to 64 tokens and few enough granules that latency and not the chip's throughput is what they cost (every workgroup
+// fetches all tokens' activations for its 32 rows; beyond, the 128-row tiles are the cheaper readers).  Above 32 tokens up to the two workgroups a CU
+// that it holds at once, up to 32 to three, or four over shorter rows.  Tiles / here, us, weights cold, in a graph:
+//   up to 32:  1024 x 4608 over 23 29 / 12.5; 16384 x 1024 10.9 / 6.6, x 3072 24.7 / 13.2, x 4096 over 32 32.9 / 19.3; 8192 x 8192 59.2 / 21.6; 24576 x 1024 11.6 / 8.6, x 4096 over
+//              32 34.5 / 28.1; 32768 x 1024 12.8 / 10.5, x 2048 20.8 / 18.3, x 4096 over 32 36.5 / 37.2; 40960 x 2048 over 32 24.1 / 24.2; 65536 x 1024 17.7 / 18.2, x 2048 over 16 29.3 / 31.9
+//   above:     8192 x 1024 over 40 10.8 / 6.1, x 8192 over 64 52.6 / 29.5; 9216 x 1024 over 48 10.6 / 7.4; 16384 x 1024 over 33 11.3 / 7.7, x 2048 over 64 16.9 / 15.3, x 4096 29.9 / 27.2;
+//              18432 x 1024 over 64 11.3 / 12.0, 20480 x 2048 18.8 / 19.8, 24576 x 1024 over 48 12.0 / 12.5
 bool few_applies(uint64_t rows, uint32_t n, uint32_t k) {
-    const uint64_t units = (rows + GR - 1) / GR, slabs = k / (KB * 32);
-    return n <= 64 && units <= (n <= 32 ? 2 * kCus : kCus) && units * slabs <= (n <= 32 ? 12288u : 4096u);
+    const uint64_t units = (rows + GR - 1) / GR;
+    if (n > 32) return n <= 64 && units <= 2 * kCus;
+    return units <= (k <= 16 * KB * 32 ? 4 : 3) * kCus;
 }
 
 // Shares of K side by side on the same kernel, a workgroup each.  Above 32 tokens while the chip holds them all at once, two workgroups a CU; up to 32
@@ -1602,7 +1606,7 @@ uint32_t few_grid(uint32_t granules, uint32_t shares, uint32_t tok_tiles) {
 // side is the faster way up to two workgroups a CU (1024 x 1024 in 4 over 23 tokens 3.5 and 0.4 more in the norm, here 4.7); beyond, and plain:
 //   plain, 9 tokens:        1024 x 1024 6.3 / 4.5, x 1792 7.5 / 6.5, x 2048 (8 shares, not 4) 6.7 / 7.1; 4096 x 2048 7.0 / 7.3
 //   plain, 24:              1024 x 1024 6.6 / 4.9, x 1792 8.0 / 6.8, x 2048 7.0 / 7.4; 3072 x 2048 7.6 / 7.5, 4096 x 2048 8.5 / 7.5
-//   plain, 40:              1024 x 1024 7.2 / 7.0, 4096 x 1024 8.2 / 7.1; 2048 x 2048 8.2 / 11.5
+//   plain, 40:              1024 x 1024 7.2 / 7.0, 4096 x 1024 8.2 / 7.1, 9216 x 1024 over 48 10.8 / 7.6, 16384 x 1024 over 33 12.5 / 7.6, over 64 14.8 / 9.2; 2048 x 2048 8.2 / 11.5
 //   with the norm, 24:      4096 x 2048 13.3 / 12.5; over 40 tokens 3072 x 1024 11.3 / 11.6, 4096 x 1024 12.9 / 12.3
 // Without room for shares side by side: all that needs none, the faster way or not.
 // Above 64 tokens, against shares on the 64-row or 128-row tiles: the walk costs 0.3 us a slab and the other way the sums' round trip through memory:
@@ -1626,9 +1630,9 @@ bool few_applies_split(uint64_t rows, uint32_t n, uint32_t k, uint32_t shares, b
         if (!room) return slabs <= 9 + rows * n / 9500;  // (all that walks with room, at least)
         return slabs <= 9 + rows * n / 11000 && slabs <= (n > 1024 ? 17u : (n <= 768 && tokens == 64) || n <= 96 ? 42u : 26u);
     }
-    if (units > 2 * kCus || units * slabs > (cost == 1 ? 12288u : 4096u) || slabs * cost > (cost == 1 && units < 96 ? 15u : 16u)) return false;
+    if (units > 2 * kCus || slabs * cost > (cost == 1 && units < 96 ? 15u : 16u)) return false;
     if (deferrable && 12 * slabs * cost > 72 + units) return false;
-    return !room || (few_applies(rows, n, k) && !(deferrable && units * shares <= 2 * kCus));
+    return !room || !(deferrable && units * shares <= 2 * kCus);
 }
 
 uint32_t split_k_factor(uint32_t m, uint32_t n, uint32_t k, uint32_t max_splits) {
@@ -1783,7 +1787,9 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, bool in_launch, uint32
     const bool few = !L.gemm_mfma16 && (few_tiled || (ksplit > 1 ? in_launch || few_side_applies(a.m, a.n, ksplit) : few_applies(GR * tile_rows(GR), a.n, a.k)));
     const bool narrow = !wide_split && narrow_tiles(tile_rows(BM), a.n);
     if (few) {
-        // Eight waves and 151 KB of LDS while every CU gets one workgroup at most, else four and half of it.
+        // 32 tokens, 40 KB of LDS: four waves, a 16 x 16 tile each, that also copy, or, while every CU gets one workgroup at most, four more that copy for
+        // them: as fast in a graph (8192 x 1024 over 23 5.3 / 5.4 us, x 3072 10.0 / 9.9), past it 1 - 5 % slower (16384 x 1024 6.6 / 6.9).  64 tokens, 56 KB: eight
+        // tiles, a wave each (four waves with two tiles each / eight: 8192 x 1024 over 48 6.4 / 6.2, 16384 x 1024 over 40 8.5 / 8.0, 2048 x 6912 in 8 over 48 11.2 / 10.8).
         const bool whole = DUMP || ksplit == 1 || in_launch;
         const auto waves = [&](auto tg, auto wv) {
             constexpr int TG = decltype(tg)::value, WV = decltype(wv)::value;
@@ -1792,8 +1798,8 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, bool in_launch, uint32
             return go(gemm_few_kernel<2, DUMP, false, TG, WV>, GR, 32 * TG, 64 * WV, whole);
         };
         if (few_tiled) return few_tiled == 32 ? waves(Idx<1>{}, Idx<4>{}) : waves(Idx<2>{}, Idx<8>{});
-        if (tile_rows(GR) * (whole ? 1u : ksplit) <= kCus) return a.n <= 32 ? waves(Idx<1>{}, Idx<8>{}) : waves(Idx<2>{}, Idx<8>{});
-        return a.n <= 32 ? waves(Idx<1>{}, Idx<4>{}) : waves(Idx<2>{}, Idx<4>{});
+        if (a.n > 32) return waves(Idx<2>{}, Idx<8>{});
+        return tile_rows(GR) * (whole ? 1u : ksplit) <= kCus ? waves(Idx<1>{}, Idx<8>{}) : waves(Idx<1>{}, Idx<4>{});
     }
     if (narrow && (a.n <= (ksplit > 1 ? 32u : 48u) || L.gemm_mfma16)) {
         // a launch of at most 16 / 32 / 48 tokens computes one / two / three of the tile's four 16-token MFMA tiles (the parity
@@ -1920,8 +1926,9 @@ bool gated_tile_n(uint32_t m, uint32_t n) { return n > 64 && (uint64_t)((m + 63)
 // Where the projections alone are more than few_applies takes, on the 128-row tiles, it always is: 6912 x 4096 over 24 17.5 / 33.7, 4608 x 1024 over 33
 // 8.4 / 11.1, 4608 x 4096 22.6 / 33.6.
 bool gated_few_faster(uint32_t m, uint32_t n, uint32_t k) {
-    if (!few_applies(2 * (uint64_t)m, n, k)) return true;
     const uint32_t slabs = k / (KB * 32);
+    const uint64_t units = 2 * (uint64_t)m / GR;
+    if (units > (n <= 32 ? 2 * kCus : kCus) || units * slabs > (n <= 32 ? 12288u : 4096u)) return true;
     if (n > 32) return slabs <= 11;
     return 2 * m / GR <= kCus ? slabs <= 8 + m / 2048 : slabs <= (n <= 24 ? 28u : 22u);
 }
@@ -1939,7 +1946,7 @@ bool gemm_gated_faster(uint32_t m, uint32_t n, uint32_t k, const Launch& L) {
     if (gemm_gated_applies(m, n, k)) return true;
     if (L.gemm_mfma16 || m % GR != 0 || k % (KB * 32) != 0 || m == 0 || n == 0) return false;
     if (gated_few_tokens(m, n, k)) return n > 64 || gated_few_faster(m, n, k);
-    if (n <= 48 && (uint64_t)2 * m / GR > 2 * kCus) return false;  // the narrow kernel's
+    if (n <= 48 && (uint64_t)2 * m / GR > 2 * kCus) return false;  // the few-token kernel's or the narrow one's
     const auto plain = [&](auto cfg) {
         using C = decltype(cfg);
         return tile_cost<C>(2 * (uint64_t)((m + C::kRows - 1) / C::kRows), n, k, 1);
