@@ -99,13 +99,11 @@ class Zeros:
 
 
 @pytest.mark.parametrize("inter,hidden,tokens,gated", [
-    (1024, 1024, 23, True), (1024, 1152, 23, False),   # 8 slabs of K
-    (2048, 1152, 32, True), (2048, 1280, 32, False),   # 9
-    (4096, 1280, 9, True), (4096, 1408, 9, False),     # 10: 128 workgroups against 256
-    (4128, 1408, 9, True),                             # past 256 granules of both
-    (4128, 3584, 24, True), (4128, 3712, 24, False),   # 28 slabs
-    (4128, 2816, 25, True), (4128, 2944, 25, False),   # 22
-    (8192, 3200, 32, True),                            # 512 x 25 slabs: the projections alone are the 128-row tiles'
+    (1024, 1024, 23, True), (1024, 1152, 23, True),
+    (2048, 1280, 32, True), (3040, 2816, 32, True), (3040, 2944, 32, False),  # 22 slabs of K
+    (3072, 2944, 24, True), (4096, 4096, 9, True), (4096, 4224, 9, False),    # 32 from 3072 rows on
+    (4128, 4224, 24, True), (4128, 2944, 25, True),    # past 256 granules of both
+    (8192, 3200, 32, True),                            # 512
     (8224, 1024, 23, False),                           # 257 granules
     (4608, 1024, 32, True), (4608, 1024, 33, True),    # 32 tokens
     (2048, 1408, 33, True), (2048, 1536, 33, False),   # 11 slabs above them

@@ -1917,20 +1917,18 @@ uint32_t gated_few_tokens(uint32_t m, uint32_t n, uint32_t k) {
 bool gated_tile_n(uint32_t m, uint32_t n) { return n > 64 && (uint64_t)((m + 63) / 64) * ((n + 63) / 64) <= kCus; }
 
 // Where that form is the faster way: it saves a launch and the floats (2.7 us together), once, and each weight has half of a workgroup's waves, so that
-// it loses time with every slab against the projections alone (gemm_few_kernel as well where few_applies).  One launch / the projections' alone,
-// us, over 24 tokens: 1024 x 512 4.3 / 3.9, x 1024 5.7 / 4.9, x 2048 9.0 / 7.4, x 4096 14.8 / 11.9; 2048 x 1024 6.2 / 5.6, x 2048 9.1 / 7.8; 4096 x 1024
-// 6.5 / 5.8, x 1792 8.8 / 7.6; 4608 x 1024 6.5 / 6.1, x 2048 9.7 / 9.4, x 4096 16.4 / 16.3; 6912 x 2048 10.5 / 10.4.  The lines up to 32 tokens were drawn for the
-// kernel before this one, on which a slab cost the gated launch more (8 to 10 slabs where the projections alone find a CU for every granule of
-// both, 28 or 22 beyond); they hold, with 1 us unclaimed around 16 slabs.  Above 32 tokens: over 40 1024 x 1536 9.7 / 6.8, 2048 x 1408 9.8 / 7.1,
-// 4096 x 1408 10.1 / 7.6; over 64 4096 x 1024 8.8 / 6.9; over 33 2048 x 2048 12.3 / 8.8.
-// Where the projections alone are more than few_applies takes, on the 128-row tiles, it always is: 6912 x 4096 over 24 17.5 / 33.7, 4608 x 1024 over 33
-// 8.4 / 11.1, 4608 x 4096 22.6 / 33.6.
+// it loses time with every slab against the projections alone, which run on gemm_few_kernel too.  us a layer that a prompt gains (+) or loses by it,
+// hidden x feed-forward size:
+//   up to 32 tokens, a CU for every granule of both: 1024 x 1024 over 9 3.3, over 24 2.5, 1280 x 2048 1.5, 2048 x 1024 1.2, x 2048 1.0, x 4096 1.1, 2560 x 2048 0.8, 2816 x 2048 0.6;
+//                     3072 x 1024 0.2, x 2048 -0.2, x 3584 0.8, 4096 x 1024 -0.3, x 2048 -0.9, x 3072 0.3, x 4096 0.7; 6144 x 2048 -1.6, x 4096 -0.4, 8192 x 4096 -1.5
+//   more granules:    1024 x 4608 over 24 1.9, 2048 x 6912 2.5, 4096 x 4608 3.7, over 32 5.1, 6144 x 6912 over 24 6.6, 8192 x 8192 5.7
+//   above 32:         1280 x 4096 over 40 0.1, 1536 x 4096 -0.2, x 2048 -0.5, 2048 x 1024 -1.4, x 3584 -0.8, over 64 -0.9
+//   more granules:    1024 x 4608 over 40 2.3, 2048 x 4608 1.9, over 64 4.1, x 8192 over 48 3.5, 4096 x 4608 over 64 6.7, 8192 x 8192 over 64 12.7
 bool gated_few_faster(uint32_t m, uint32_t n, uint32_t k) {
     const uint32_t slabs = k / (KB * 32);
-    const uint64_t units = 2 * (uint64_t)m / GR;
-    if (units > (n <= 32 ? 2 * kCus : kCus) || units * slabs > (n <= 32 ? 12288u : 4096u)) return true;
+    if (2 * m / GR > kCus) return true;
     if (n > 32) return slabs <= 11;
-    return 2 * m / GR <= kCus ? slabs <= 8 + m / 2048 : slabs <= (n <= 24 ? 28u : 22u);
+    return slabs <= 22 || (m >= 3072 && slabs <= 32);
 }
 
 template <typename C>
