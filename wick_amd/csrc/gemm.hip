@@ -9,9 +9,10 @@
 //
 // Three families of block loops:
 //   * gemm_tile_kernel, v_mfma_i32_32x32x32_i8: prompts, on the cheapest of six tiles for the launch (see T32 and TileL .. TileH);
-//   * gemm_few_kernel, v_mfma_i32_16x16x32_i8, 32 rows x up to 64 tokens: where latency is what a launch costs (few_applies, few_tokens_per_tile);
-//   * gemm_narrow_kernel, v_mfma_i32_16x16x32_i8, 128 rows x 64 tokens: the other launches of up to 48 tokens, which skip the 16-token
-//     columns they do not have; gemm_mfma_kernel, the same shape on 128 x 128, on request (wick_rocm_set_gemm_mfma_shape).
+//   * gemm_few_kernel, v_mfma_i32_16x16x32_i8, 32 rows x 32 or 64 tokens, several such tiles side by side past 64 tokens: where latency is what a
+//     launch costs (few_applies, few_side_applies, few_tokens_per_tile);
+//   * gemm_narrow_kernel, v_mfma_i32_16x16x32_i8, 128 rows x 64 tokens: the other unsplit launches of up to 48 tokens (many rows), which skip the
+//     16-token columns they do not have; gemm_mfma_kernel, the same shape on 128 x 128, on request (wick_rocm_set_gemm_mfma_shape).
 // The kernels are bound by the two scaling FMAs per result plus the matrix instructions, which a SIMD overlaps only in part, and by
 // feeding both from LDS.  A wave issues a vector-ALU instruction only every ~4.7 cycles while a SIMD retires one every ~2.3, so two
 // waves per SIMD at least, four where a wave has one result buffer.
@@ -1801,10 +1802,10 @@ hipError_t launch(int type, GemmArgs& a, const Launch& L, bool in_launch, uint32
         if (a.n > 32) return waves(Idx<2>{}, Idx<8>{});
         return tile_rows(GR) * (whole ? 1u : ksplit) <= kCus ? waves(Idx<1>{}, Idx<8>{}) : waves(Idx<1>{}, Idx<4>{});
     }
-    if (narrow && (a.n <= (ksplit > 1 ? 32u : 48u) || L.gemm_mfma16)) {
+    if (narrow && ((ksplit == 1 && a.n <= 48) || L.gemm_mfma16)) {
         // a launch of at most 16 / 32 / 48 tokens computes one / two / three of the tile's four 16-token MFMA tiles (the parity
         // hook: all four).  These launches are bound by their block loop, not by memory: 65536 x 16 x 2048 40 -> 34 us.
-        // (33 .. 48 tokens in shares of K: the 64-row tile.  2048 x 6912 in 8 over 37 9.6 / 8.7 us.)
+        // (Shares of K over as many: gemm_few_kernel above, or the tiles.)
         if constexpr (!DUMP) {
             if (a.n <= 16) return go(gemm_narrow_kernel<2, false, 1>, BM, BN_NARROW, THREADS);
             if (a.n <= 32) return go(gemm_narrow_kernel<2, false, 2>, BM, BN_NARROW, THREADS);
